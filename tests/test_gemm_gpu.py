@@ -88,6 +88,56 @@ def test_fused_epilogues_small_m_long_k(ttmi, oracle, dt):
     assert max_abs(host(C), base + rounded(bias, dt) + rounded(res, dt)) <= GEMM_TOL[dt] * 3
 
 
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (33, 72, 128), (65, 200, 192), (127, 520, 768), (700, 1544, 256), (1400, 3072, 768),
+                                   (2000, 768, 768), (2560, 776, 320), (2500, 3072, 192), (260, 768, 3072)])
+def test_ring_kernel_epilogues_on_ragged_tiles(ttmi, oracle, dt, M, N, K):
+    """The deep-ring tiles behind bias, bias + residual, bias + ReLU and fp32 output: fewer K steps than ring stages, rows and
+    columns past the last whole tile of every width, whole and K-sliced products.  Rows past M stay untouched."""
+    import ctypes
+    if K * (4 if dt == "f32" else 2) % 128:
+        pytest.skip("K is no whole number of 128-byte steps")
+    rng = np.random.default_rng(M + N + K)
+    A, W = _ab(rng, M, N, K, 1)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    dA, dW, db, dres = dev(A, dt), dev(W, dt), dev(bias, dt), dev(res, dt)
+    base = oracle.matmul(rounded(A, dt), rounded(W, dt), True) + rounded(bias, dt)
+    for epi, args, want in ((capi.EPI_BIAS, _epi(bias=db), base), (capi.EPI_BIAS_ACT, _epi(bias=db, act=capi.ACT_RELU), np.maximum(base, 0)),
+                            (capi.EPI_BIAS_RESIDUAL, _epi(bias=db, residual=dres), base + rounded(res, dt)),
+                            (capi.EPI_F32_OUT, _epi(bias=db), base)):
+        C = torch.full((M + 40, N), -7.0, dtype=torch.float32 if epi == capi.EPI_F32_OUT else dA.dtype, device="cuda")
+        ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(dW), ptr(C), M, N, K, K, K, N, epi, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+        assert max_abs(host(C[:M]), want) <= GEMM_TOL[dt] * 3
+        assert torch.all(C[M:] == -7.0)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("v_transposed", [False, True])
+@pytest.mark.parametrize("B,S,h", [(1, 1, 12), (3, 5, 12), (1, 37, 16), (9, 31, 12), (7, 130, 12), (2, 387, 16)])
+def test_ring_kernel_head_split(ttmi, oracle, dt, v_transposed, B, S, h):
+    """The same tiles behind the QKV projection: sequences shorter than a group of rows and off its grid, V row-major and
+    transposed (four or eight rows a store), hidden sizes whose V third starts inside and on a wavefront's columns."""
+    import ctypes
+    d, H = 64, h * 64
+    rng = np.random.default_rng(S + h)
+    A, W = _ab(rng, B * S, 3 * H, H, 1)
+    bias = rng.standard_normal(3 * H).astype(np.float32)
+    dA, dW, db = dev(A, dt), dev(W, dt), dev(bias, dt)
+    pitch = (S + 7) // 8 * 8 if v_transposed else 0
+    q, k = (torch.full((B, h, S, d), float("nan"), dtype=dA.dtype, device="cuda") for _ in range(2))
+    v = torch.full((B, h, d, pitch) if v_transposed else (B, h, S, d), 7.0, dtype=dA.dtype, device="cuda")
+    args = _epi(bias=db, q=q, k=k, v=v, seq=S, heads=h, head_dim=d, v_seq_pitch=pitch)
+    ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(dW), None, B * S, 3 * H, H, H, H, 3 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args),
+                            TTMI_DTYPES[dt], stream()))
+    want = oracle.split_add_bias_transpose(oracle.matmul(rounded(A, dt), rounded(W, dt), True), rounded(bias, dt), B, S, h, d)
+    got_v = host(v)
+    if v_transposed:
+        assert np.all(got_v[..., S:] == 7.0)
+        got_v = got_v[..., :S].transpose(0, 1, 3, 2)
+    for got, w in zip((host(q), host(k), got_v), want):
+        assert max_abs(got, w) <= GEMM_TOL[dt] * 2
+
+
 @pytest.fixture(params=["3 A stages", "2 A stages"])
 def large_tile_forced(request, ttmi):
     """Switch TTMI_LARGE_TILE = 1 sends every eligible problem to the one-wavefront-per-SIMD kernel whatever its

@@ -341,6 +341,31 @@ struct EpiQkvSplit {
       v[(((int64_t)bj * heads + head) * dim + i) * v_pitch + (pr - bj * seq)] = from_float<T>(val[j]);
     }
   }
+  // The same for four rows (one 8-byte store): the form for wavefronts that own a single 16-row block.
+  __device__ __forceinline__ void store_col4(int m, int m_limit, int n, const float (&val)[4]) const {
+    const uint32_t rem = (uint32_t)(n - 2 * hidden);
+    const uint32_t prow = PAD ? (uint32_t)token_rows[m] : (uint32_t)m;
+    const uint32_t b = div_seq.div(prow);
+    const uint32_t s = prow - b * seq;
+    T* row = v + (int64_t)rem * v_pitch;
+    const int64_t per_batch = (int64_t)hidden * v_pitch;
+    bool fast = m + 4 <= m_limit && s + 4 <= (uint32_t)seq;
+    if (PAD && fast) fast = (uint32_t)token_rows[m + 3] == prow + 3;
+    if (fast) {
+      Vec<T, 4> o;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o.v[j] = from_float<T>(val[j]);
+      store_vec_unaligned<T, 4>(row + b * per_batch + s, o);
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (m + j >= m_limit) break;
+      const uint32_t pr = PAD ? (uint32_t)token_rows[m + j] : (uint32_t)(m + j);
+      const uint32_t bj = div_seq.div(pr);
+      row[bj * per_batch + (pr - bj * seq)] = from_float<T>(val[j]);
+    }
+  }
   __device__ __forceinline__ int64_t vt_hop() const { return (int64_t)hidden * v_pitch - seq; }
   __device__ __forceinline__ T* dest(uint32_t b, uint32_t s, uint32_t n) const {
     const uint32_t w = div_hidden.div(n);
@@ -1288,8 +1313,8 @@ __global__ __launch_bounds__(WM * WN * kWave) void gemm_fast_kernel(const GemmAr
 // Dry run: while a thread has a string installed here, the launchers below write the name of the kernel variant
 // they would launch (tile, wavefronts, K split) into it and launch nothing.  ttmi_gemm_describe uses it, so the
 // answer comes from the very code path that picks the kernel.
-static thread_local std::string* tl_describe = nullptr;
-static bool describe_only(const char* family, int waves, int bm, int bn, int splits = 1) {
+inline thread_local std::string* tl_describe = nullptr;
+inline bool describe_only(const char* family, int waves, int bm, int bn, int splits = 1) {
   if (tl_describe == nullptr) return false;
   *tl_describe = std::string(family) + std::to_string(waves) + "w_" + std::to_string(bm) + "x" + std::to_string(bn);
   if (splits > 1) *tl_describe += "_splitk" + std::to_string(splits);
@@ -1299,9 +1324,9 @@ static bool describe_only(const char* family, int waves, int bm, int bn, int spl
 // A dequantising epilogue that was asked for per-workgroup maxima gets them only from a launch whose workgroups fit
 // the slots; otherwise the request is dropped and the caller told (tl_absmax_written stays 0), and it finds the
 // maximum with a pass of its own.
-static thread_local int tl_absmax_written = 0;
+inline thread_local int tl_absmax_written = 0;
 template <typename Epi>
-static bool absmax_grid_ok(const Epi& epi, unsigned grid_x, int batch) {
+inline bool absmax_grid_ok(const Epi& epi, unsigned grid_x, int batch) {
   if constexpr (Dequantises<Epi>::value) {
     if (epi.absmax_slots() == nullptr) return true;
     if (grid_x > (unsigned)kAbsmaxSlots || batch != 1) return false;
@@ -1310,13 +1335,13 @@ static bool absmax_grid_ok(const Epi& epi, unsigned grid_x, int batch) {
   return true;
 }
 template <typename Epi>
-static Epi without_absmax(Epi epi) {
+inline Epi without_absmax(Epi epi) {
   if constexpr (std::is_same<Epi, EpiDequant>::value) epi.absmax = nullptr;
   return epi;
 }
 
 // Kernels that use more than 64 KB of dynamic LDS need the limit raised once per kernel and device.
-static int allow_large_lds(const void* kern, int bytes) {
+inline int allow_large_lds(const void* kern, int bytes) {
   static std::mutex mu;
   static std::set<std::pair<const void*, int>> done;
   int dev = 0;
@@ -1329,7 +1354,7 @@ static int allow_large_lds(const void* kern, int bytes) {
 }
 
 template <typename T, int BM, int BN, int WM, int WN, bool B_KN, bool ALIGNED, typename Epi>
-static int launch_config(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
+inline int launch_config(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
   constexpr int NT = WM * WN * kWave;
   constexpr int LDS = 2 * (BM + BN) * kRowBytes;
   if (describe_only("reg", WM * WN, BM, BN)) return 0;
@@ -1349,9 +1374,9 @@ static int launch_config(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
   return launch_status("gemm_kernel");
 }
 
-static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-static int compute_units() {
+inline int compute_units() {
   static int cus = [] {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
@@ -1362,7 +1387,7 @@ static int compute_units() {
 }
 
 template <typename T, int BM, int BN, int WM, int WN, typename Epi, int NS = 2>
-static int launch_fast(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
+inline int launch_fast(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
   constexpr int NT = WM * WN * kWave;
   constexpr int LDS = fast_lds_bytes<BM, BN, WM, WN, NS>();
   static_assert(LDS <= kLdsPerCu, "tile does not fit in LDS");
@@ -1397,9 +1422,9 @@ struct FixedWorkspace {
   float* ptr = nullptr;
   size_t bytes = 0;
 };
-static thread_local FixedWorkspace tl_fixed_workspace;
+inline thread_local FixedWorkspace tl_fixed_workspace;
 
-static int splitk_workspace(size_t bytes, hipStream_t s, float** out) {
+inline int splitk_workspace(size_t bytes, hipStream_t s, float** out) {
   *out = nullptr;
   if (tl_fixed_workspace.ptr != nullptr) {
     if (bytes > tl_fixed_workspace.bytes)
@@ -1441,7 +1466,7 @@ static int splitk_workspace(size_t bytes, hipStream_t s, float** out) {
 // this chip), which a problem that already has a hundred tiles of 16-bit operands does not win back:
 // 128 x 3072 x 768 in fp16 runs 1.3 us faster unsplit, with its epilogue in the GEMM; in fp32 (twice
 // the K steps, a quarter of the matrix rate) the same problem is 15 us faster split.
-static int pick_splits(int64_t m, int64_t n, int64_t ksteps, int64_t batch, size_t elem_size) {
+inline int pick_splits(int64_t m, int64_t n, int64_t ksteps, int64_t batch, size_t elem_size) {
   const int64_t tiles = ceil_div(m, 64) * ceil_div(n, 64);
   const int64_t most_tiles = elem_size <= 2 ? 64 : 128;
   if (batch != 1 || tiles > most_tiles || ksteps < 8) return 1;
@@ -1452,23 +1477,23 @@ static int pick_splits(int64_t m, int64_t n, int64_t ksteps, int64_t batch, size
 // the 64 x 64 tiles, for A/B timing).
 constexpr int kWaveDepth = 4;  // K steps a wavefront keeps in flight: 32 loads of 16 bytes per lane
 template <typename T>
-static bool wave_kernel_ok(const GemmArgs& g, int batch, bool aligned) {
+inline bool wave_kernel_ok(const GemmArgs& g, int batch, bool aligned) {
   if (sizeof(T) != 2 || !aligned || batch != 1 || g.m > 128 || g.k % (kRowBytes / (int)sizeof(T)) != 0) return false;
   return kernel_switch(kSwitchWaveKernel) != 0;
 }
 // K slices for it: up to two wavefronts per CU, at least four K steps per slice.
-static int wave_splits(int64_t m, int64_t n, int64_t ksteps) {
+inline int wave_splits(int64_t m, int64_t n, int64_t ksteps) {
   const int64_t tiles = ceil_div(m, 32) * ceil_div(n, 32);
   return (int)std::max<int64_t>(1, std::min<int64_t>({2 * (int64_t)compute_units() / tiles, ksteps / 4, 16}));
 }
-static void wave_grid(GemmArgs& g, unsigned* grid_x) {
+inline void wave_grid(GemmArgs& g, unsigned* grid_x) {
   g.tiles_m = (g.m + 31) / 32;
   g.tiles_n = (g.n + 31) / 32;
   const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
   *grid_x = tiles >= kXcdRemapMinTiles ? (unsigned)(ceil_div(tiles, kNumXcd) * kNumXcd) : (unsigned)tiles;
 }
 template <typename T, typename Epi>
-static int launch_wave(GemmArgs g, const Epi& epi, hipStream_t s) {
+inline int launch_wave(GemmArgs g, const Epi& epi, hipStream_t s) {
   if constexpr (sizeof(T) == 2) {
     if (describe_only("wave", 1, 32, 32)) return 0;
     unsigned grid_x = 0;
@@ -1480,7 +1505,7 @@ static int launch_wave(GemmArgs g, const Epi& epi, hipStream_t s) {
 
 // `reduce(ws, slices, vec, stream)` launches the kernel that sums the slices and applies the epilogue.
 template <typename T, typename Reduce>
-static int launch_splitk(GemmArgs g, int splits, int64_t ksteps, int bk, hipStream_t s, const Reduce& reduce) {
+inline int launch_splitk(GemmArgs g, int splits, int64_t ksteps, int bk, hipStream_t s, const Reduce& reduce) {
   constexpr int kTile = 64, kWaveTile = 32;  // tile edge of the LDS-tiled and of the one-wavefront form
   const bool wave = wave_kernel_ok<T>(g, 1, true);  // callers come here with aligned operands and one problem
   if (wave) splits = std::max(2, wave_splits(g.m, g.n, ksteps));
@@ -1518,7 +1543,7 @@ static int launch_splitk(GemmArgs g, int splits, int64_t ksteps, int bk, hipStre
 // Split-K on the DMA kernel with 128x128 tiles, for mid-size problems whose tiles do not fill the chip
 // (M = 2560, N = 768, K = 3072: 120 tiles, 48 K steps each).
 template <typename T, typename Reduce>
-static int launch_fast_splitk(GemmArgs g, int splits, int64_t ksteps, int bk, hipStream_t s, const Reduce& reduce) {
+inline int launch_fast_splitk(GemmArgs g, int splits, int64_t ksteps, int bk, hipStream_t s, const Reduce& reduce) {
   constexpr int kTile = 128;
   g.k_chunk = (int)ceil_div(ksteps, splits) * bk;
   const int used = (int)ceil_div(g.k, g.k_chunk);  // slices that actually hold part of K: what is launched
@@ -1573,7 +1598,7 @@ struct TileConfig {
 constexpr TileConfig kTileConfigs[] = {
     {256, 256, 1, 1.00f}, {256, 192, 1, 0.93f}, {256, 128, 1, 0.82f}, {128, 128, 2, 0.62f}, {64, 64, 4, 0.30f}};
 
-static double tile_cost(const TileConfig& c, int64_t m, int64_t n, int64_t batch) {
+inline double tile_cost(const TileConfig& c, int64_t m, int64_t n, int64_t batch) {
   const int64_t tiles = ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch;
   const int64_t slots = (int64_t)compute_units() * c.per_cu;
   const int64_t full = tiles / slots, rem = tiles % slots;
@@ -1586,13 +1611,13 @@ static double tile_cost(const TileConfig& c, int64_t m, int64_t n, int64_t batch
 // little: efficiencies fitted to a sweep of M = 800 ... 16384 by N, K = 768 / 3072 (4000 x 768 x 3072: 175 us on
 // 64 x 64 tiles, three per CU, against 233 us on 128 x 128, one on three CUs of four).
 constexpr float kTileEff32[] = {0.88f, 0.85f, 0.82f, 0.78f, 0.74f};
-static double tile_cost32(int i, int64_t m, int64_t n, int64_t batch) {
+inline double tile_cost32(int i, int64_t m, int64_t n, int64_t batch) {
   const TileConfig& c = kTileConfigs[i];
   const int64_t tiles = ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch;
   return (double)ceil_div(tiles, compute_units()) * c.bm * c.bn / kTileEff32[i];
 }
 
-static int pick_tile(int64_t m, int64_t n, int64_t batch, double* cost_out = nullptr, size_t elem_size = 2) {
+inline int pick_tile(int64_t m, int64_t n, int64_t batch, double* cost_out = nullptr, size_t elem_size = 2) {
   int best = 0;
   double best_cost = 1e300;
   for (int i = 0; i < (int)(sizeof(kTileConfigs) / sizeof(kTileConfigs[0])); ++i) {
@@ -1611,6 +1636,8 @@ static int pick_tile(int64_t m, int64_t n, int64_t batch, double* cost_out = nul
 template <typename T, typename Epi, typename Enable = void>
 struct LargeTileKernel {
   static bool wanted(const GemmArgs&, const Epi&, int, bool) { return false; }
+  static bool eligible(const GemmArgs&, const Epi&) { return false; }
+  static double us(const GemmArgs&, const Epi&) { return 1e300; }
   static int launch(const GemmArgs&, const Epi&, hipStream_t) { return 0; }
 };
 
@@ -1621,7 +1648,7 @@ struct SplitPlan {
   int splits;
 };
 template <typename T>
-static SplitPlan plan_split(int64_t m, int64_t n, int64_t k, int64_t batch, bool aligned) {
+inline SplitPlan plan_split(int64_t m, int64_t n, int64_t k, int64_t batch, bool aligned) {
   constexpr int BK = kRowBytes / sizeof(T);
   if (!aligned || k % BK != 0 || batch != 1) return {SplitKind::kNone, 1};
   const int64_t ksteps = k / BK;
@@ -1665,47 +1692,58 @@ static SplitPlan plan_split(int64_t m, int64_t n, int64_t k, int64_t batch, bool
   return {SplitKind::kNone, 1};
 }
 
+// The deep-ring kernel of gemm_ring.h and its selection; declared here for launch_gemm.
+template <typename T, typename Epi>
+struct RingKernel;
+
+// A plain product C = alpha A op(B) + beta C.  (What the encoder's fused products run on is picked by RingKernel.)
+template <typename T, typename Epi>
+inline int launch_plain(const GemmArgs& g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
+  constexpr int BK = kRowBytes / sizeof(T);
+  auto tiles = [&](int bm, int bn) { return (int64_t)ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch; };
+  if (LargeTileKernel<T, Epi>::wanted(g, epi, batch, aligned)) return LargeTileKernel<T, Epi>::launch(g, epi, s);
+  switch (pick_tile(g.m, g.n, batch, nullptr, sizeof(T))) {
+    case 0: return launch_fast<T, 256, 256, 2, 4, Epi>(g, epi, batch, s);
+    case 1: return launch_fast<T, 256, 192, 4, 2, Epi>(g, epi, batch, s);
+    case 2: return launch_fast<T, 256, 128, 4, 2, Epi>(g, epi, batch, s);
+    case 3: {
+      const SplitPlan plan = plan_split<T>(g.m, g.n, g.k, batch, aligned);
+      if (plan.kind == SplitKind::kDmaTiles)
+        return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
+      // 128 x 128 tiles on at most half the CUs and a K too short to cut: 128 x 64 tiles put twice as many CUs
+      // to work (2560 x 768 x 768: 240 tiles in one round, 9 us against 11)
+      if (batch == 1 && tiles(128, 128) <= compute_units() / 2 && tiles(128, 64) <= compute_units())
+        return launch_fast<T, 128, 64, 2, 2, Epi, 4>(g, epi, batch, s);
+      return launch_fast<T, 128, 128, 2, 2, Epi>(g, epi, batch, s);
+    }
+    // small problems are latency-bound: the register-staged kernel hides the global latency
+    // of a one-step prefetch better than the DMA path does with a tiny tile
+    default: {
+      const SplitPlan plan = plan_split<T>(g.m, g.n, g.k, batch, aligned);
+      if (plan.kind == SplitKind::kSmallTiles)
+        return launch_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
+      if (plan.kind == SplitKind::kDmaTiles)
+        return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
+      if (wave_kernel_ok<T>(g, batch, aligned)) return launch_wave<T>(g, epi, s);
+      return launch_config<T, 64, 64, 2, 2, false, true, Epi>(g, epi, batch, s);
+    }
+  }
+}
+
+template <typename Epi>
+struct IsPlain : std::false_type {};
+template <typename T>
+struct IsPlain<EpiAlphaBeta<T>> : std::true_type {};
+
 template <typename T, bool B_KN, typename Epi>
-static int launch_gemm(GemmArgs g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
+inline int launch_gemm(GemmArgs g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
   if (g.m <= 0 || g.n <= 0 || batch <= 0) return 0;
   TTMI_REQUIRE(g.k > 0, "K must be positive");
   auto tiles = [&](int bm, int bn) { return (int64_t)ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch; };
   if (!B_KN) {
-    constexpr int BK = kRowBytes / sizeof(T);
-    if (aligned && g.k % BK == 0) {
-      bool column_pass = false;
-      if constexpr (HasColumnPass<Epi>::value) column_pass = epi.v_pitch > 0;
-      if (LargeTileKernel<T, Epi>::wanted(g, epi, batch, aligned)) return LargeTileKernel<T, Epi>::launch(g, epi, s);
-      switch (pick_tile(g.m, g.n, batch, nullptr, sizeof(T))) {
-        case 0: return launch_fast<T, 256, 256, 2, 4, Epi>(g, epi, batch, s);
-        case 1: return launch_fast<T, 256, 192, 4, 2, Epi>(g, epi, batch, s);
-        case 2: return launch_fast<T, 256, 128, 4, 2, Epi>(g, epi, batch, s);
-        case 3: {
-          if constexpr (std::is_same<typename Epi::Acc, float>::value) {
-            const SplitPlan plan = column_pass ? SplitPlan{SplitKind::kNone, 1} : plan_split<T>(g.m, g.n, g.k, batch, aligned);
-            if (plan.kind == SplitKind::kDmaTiles)
-              return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-          }
-          // 128 x 128 tiles on at most half the CUs and a K too short to cut: 128 x 64 tiles put twice as many CUs
-          // to work (2560 x 768 x 768: 240 tiles in one round, 9 us against 11)
-          if (batch == 1 && tiles(128, 128) <= compute_units() / 2 && tiles(128, 64) <= compute_units())
-            return launch_fast<T, 128, 64, 2, 2, Epi, 4>(g, epi, batch, s);
-          return launch_fast<T, 128, 128, 2, 2, Epi>(g, epi, batch, s);
-        }
-        // small problems are latency-bound: the register-staged kernel hides the global latency
-        // of a one-step prefetch better than the DMA path does with a tiny tile
-        default: {
-          if constexpr (std::is_same<typename Epi::Acc, float>::value) {
-            const SplitPlan plan = column_pass ? SplitPlan{SplitKind::kNone, 1} : plan_split<T>(g.m, g.n, g.k, batch, aligned);
-            if (plan.kind == SplitKind::kSmallTiles)
-              return launch_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-            if (plan.kind == SplitKind::kDmaTiles)
-              return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-            if (wave_kernel_ok<T>(g, batch, aligned)) return launch_wave<T>(g, epi, s);
-          }
-          return launch_config<T, 64, 64, 2, 2, false, true, Epi>(g, epi, batch, s);
-        }
-      }
+    if (aligned && g.k % (kRowBytes / (int)sizeof(T)) == 0) {
+      if constexpr (IsPlain<Epi>::value) return launch_plain<T>(g, epi, batch, aligned, s);
+      else if (RingKernel<T, Epi>::ok(g, epi, batch)) return RingKernel<T, Epi>::launch(g, epi, s);
     }
     if (aligned) {
       if (tiles(128, 128) >= 200) return launch_config<T, 128, 128, 2, 2, false, true, Epi>(g, epi, batch, s);
@@ -1719,33 +1757,6 @@ static int launch_gemm(GemmArgs g, const Epi& epi, int batch, bool aligned, hipS
     }
     return launch_config<T, 64, 64, 2, 2, true, false, Epi>(g, epi, batch, s);
   }
-}
-
-template <typename T>
-static int gemm_alpha_beta(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda,
-                           int64_t ldb, int64_t ldc, int inner, int64_t a_outer, int64_t a_inner,
-                           int64_t b_outer, int64_t b_inner, int64_t c_outer, int64_t c_inner, int64_t batch,
-                           int trans_b, float alpha, float beta, hipStream_t s) {
-  TTMI_REQUIRE(m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension too large");
-  GemmArgs g{};
-  g.a = (const char*)a;
-  g.b = (const char*)b;
-  g.m = (int)m; g.n = (int)n; g.k = (int)k;
-  g.lda = lda; g.ldb = ldb;
-  g.inner = inner;
-  g.a_outer = a_outer; g.a_inner = a_inner; g.b_outer = b_outer; g.b_inner = b_inner;
-  constexpr int KPC = 16 / sizeof(T);
-  const bool c_vec = aligned16(c) && ldc % KPC == 0 && c_outer % KPC == 0 && c_inner % KPC == 0;
-  EpiAlphaBeta<T> epi{(T*)c, ldc, c_outer, c_inner, inner, alpha, beta, c_vec};
-  auto mult = [](int64_t v) { return v % KPC == 0; };
-  bool aligned = aligned16(a) && aligned16(b) && mult(lda) && mult(ldb) && mult(a_outer) && mult(a_inner) &&
-                 mult(b_outer) && mult(b_inner);
-  if (trans_b) {
-    aligned = aligned && mult(k);
-    return launch_gemm<T, false>(g, epi, (int)batch, aligned, s);
-  }
-  aligned = aligned && mult(k) && mult(n);
-  return launch_gemm<T, true>(g, epi, (int)batch, aligned, s);
 }
 
 }  // namespace ttmi

@@ -1,0 +1,605 @@
+// Mid-size GEMM kernel for gfx950: small tiles in an LDS ring of three or four K steps, whose loads are spread evenly
+// between the matrix instructions.
+//
+//   C[M,N] = epilogue(A[M,K] * B[N,K]^T)   (both operands K-contiguous and 16-byte aligned, K a multiple of 128 bytes)
+//
+// What bounds a product of some hundred to a few thousand rows is neither memory nor the matrix pipe.  A CU fetches
+// 115 GB/s from L2 (one 1 KB `global -> LDS` load per 18 cycles), and the older kernels of gemm_impl.h issue the loads of
+// a K step in one burst behind its barrier: a wavefront that waits at the full load queue issues no matrix instruction, so
+// the two times add up (a 128 x 128 step: 580 + 510 cycles).  Here a load goes out every few matrix instructions over the
+// whole step, half of them behind the step's barrier and half in front of the next one's, and the two overlap: a step of
+// 128 x 64 takes 0.25 us instead of 0.35, of 128 x 192 0.44 against a matrix time of 0.35.
+// The other half of such a launch is what a workgroup spends outside its K loop, so everything there is short: eight
+// wavefronts where the tile has room for them (a lone wavefront per SIMD issues dependent instructions every eight cycles),
+// destinations as column part + row part, 16-byte stores straight from the accumulator layout (epilogue of a 128 x 192 tile
+// 4.7 -> 1.3 us).  Steps past the last one are requested from a buffer of size 0: they return at once, the loop needs no
+// tail and its wait counters stay constants.
+// Measured, fp16, us per launch before / after: 2000 x 2304 x 768 16.7 / 12.5, 2000 x 768 x 768 8.3 / 6.2, 2000 x 3072 x 768
+// 16.5 / 12.5, 2000 x 768 x 3072 24.4 (four K slices) / 14.0, 387 x 2304 x 768 8.9 / 5.7; fp32: 87 / 63, 33 / 23, 100 / 74,
+// 93 / 77.
+#pragma once
+
+#include "gemm_impl.h"
+#include "gemm_w4.h"
+
+namespace ttmi {
+
+// One 16 x 16 block of the output per 64 bytes of K, accumulator pinned to the AGPR half (see MmaBlock in gemm_w4.h).
+// PARTS instructions per 16-byte chunk: the fp32 instruction takes one of the chunk's four values at a time.
+template <typename T>
+struct RingMma;
+template <>
+struct RingMma<f16> {
+  using Acc = floatx4;
+  static constexpr int PARTS = 1;
+  static __device__ __forceinline__ void run(const Chunk& a, const Chunk& b, Acc& c, int) { MmaBlock<f16, 16>::run(a, b, c); }
+};
+template <>
+struct RingMma<bf16> {
+  using Acc = floatx4;
+  static constexpr int PARTS = 1;
+  static __device__ __forceinline__ void run(const Chunk& a, const Chunk& b, Acc& c, int) { MmaBlock<bf16, 16>::run(a, b, c); }
+};
+template <>
+struct RingMma<int8_t> {
+  using Acc = intx4;
+  static constexpr int PARTS = 1;
+  static __device__ __forceinline__ void run(const Chunk& a, const Chunk& b, Acc& c, int) {
+    asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(c) : "v"(__builtin_bit_cast(intx4, a)), "v"(__builtin_bit_cast(intx4, b)));
+  }
+};
+template <>
+struct RingMma<float> {
+  using Acc = floatx4;
+  static constexpr int PARTS = 4;
+  static __device__ __forceinline__ void run(const Chunk& a, const Chunk& b, Acc& c, int part) {
+    asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(c) : "v"(a.w[part]), "v"(b.w[part]));
+  }
+};
+
+// Where an epilogue's output goes, as column part + row part (`split`), and what finishes a value; the epilogues this does
+// not cover store through their store8().
+template <typename Epi>
+struct RingDest {
+  using Elem = float;
+  static constexpr bool split = false;
+};
+template <typename Epi>
+struct AddsResidual : std::false_type {};
+template <typename T, int ACT, bool HAS_ACT>
+struct AddsResidual<EpiBias<T, ACT, HAS_ACT, true>> : std::true_type {};
+template <typename T>
+struct RingDest<EpiAlphaBeta<T>> {  // one problem, beta == 0 (see ring_ok)
+  using Elem = T;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ T* column(const EpiAlphaBeta<T>& e, int, int n) { return e.c + n; }
+  static __device__ __forceinline__ int64_t row(const EpiAlphaBeta<T>& e, int m) { return (int64_t)m * e.ldc; }
+  static __device__ __forceinline__ float finish(const EpiAlphaBeta<T>& e, float x) { return x * e.alpha; }
+};
+template <typename T, int ACT, bool HAS_ACT, bool HAS_RES>
+struct RingDest<EpiBias<T, ACT, HAS_ACT, HAS_RES>> {
+  using Epi = EpiBias<T, ACT, HAS_ACT, HAS_RES>;
+  using Elem = T;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ T* column(const Epi& e, int, int n) { return e.c + n; }
+  static __device__ __forceinline__ int64_t row(const Epi& e, int m) { return (int64_t)m * e.ldc; }
+  static __device__ __forceinline__ float finish(const Epi& e, float x) { return e.finish(x); }
+};
+template <typename T>
+struct RingDest<EpiF32<T>> {
+  using Elem = float;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ float* column(const EpiF32<T>& e, int, int n) { return e.c + n; }
+  static __device__ __forceinline__ int64_t row(const EpiF32<T>& e, int m) { return (int64_t)m * e.ldc; }
+  static __device__ __forceinline__ float finish(const EpiF32<T>&, float x) { return x; }
+};
+template <>
+struct RingDest<EpiPartial> {
+  using Elem = float;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ float* column(const EpiPartial& e, int z, int n) { return e.ws + (int64_t)z * e.mn + n; }
+  static __device__ __forceinline__ int64_t row(const EpiPartial& e, int m) { return (int64_t)m * e.ldn; }
+  static __device__ __forceinline__ float finish(const EpiPartial&, float x) { return x; }
+};
+template <typename T, bool PAD>
+struct RingDest<EpiQkvSplit<T, PAD>> {
+  using Elem = T;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ T* column(const EpiQkvSplit<T, PAD>& e, int, int n) { return e.col_part((uint32_t)n); }
+  static __device__ __forceinline__ int64_t row(const EpiQkvSplit<T, PAD>& e, int m) { return e.row_part(m); }
+  static __device__ __forceinline__ float finish(const EpiQkvSplit<T, PAD>&, float x) { return x; }
+};
+
+template <>
+struct RingDest<EpiDequant> {
+  using Elem = float;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ float* column(const EpiDequant& e, int, int n) { return e.c + n; }
+  static __device__ __forceinline__ int64_t row(const EpiDequant& e, int m) { return (int64_t)m * e.ldc; }
+  static __device__ __forceinline__ float finish(const EpiDequant&, int x) { return __builtin_bit_cast(float, x); }
+};
+template <>
+struct RingDest<EpiDequantQkvSplit> {
+  using Elem = float;
+  static constexpr bool split = true;
+  static __device__ __forceinline__ float* column(const EpiDequantQkvSplit& e, int, int n) { return e.split.col_part((uint32_t)n); }
+  static __device__ __forceinline__ int64_t row(const EpiDequantQkvSplit& e, int m) { return e.split.row_part(m); }
+  static __device__ __forceinline__ float finish(const EpiDequantQkvSplit&, int x) { return __builtin_bit_cast(float, x); }
+};
+
+template <int BM, int BN, int NS>
+constexpr int ring_lds_bytes() { return NS * (BM + BN) * kRowBytes; }
+
+// A workgroup of WM x WN wavefronts owns one BM x BN tile (and, with g.k_chunk, one K slice of it).  LDS: NS stages of
+// [A rows | B rows], 128 bytes of K per row, XOR-swizzled as in gemm_w4.h.
+// K step s: multiply its first half while its second half is read and the rest of step s - 1 + NS is requested; wait until
+// step s + 1 has landed (the NS - 2 younger steps stay in flight) and everyone has read step s; multiply the second half
+// while the first half of step s + 1 is read and the first loads of step s + NS go into the stage just freed.
+template <typename T, int BM, int BN, int WM, int WN, int NS, typename Epi>
+__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const GemmArgs g, const Epi epi) {
+  constexpr int NW = WM * WN;
+  constexpr int RB = BM / WM / 16, CB = BN / WN / 16;  // 16 x 16 blocks per wavefront
+  constexpr int A_BYTES = BM * kRowBytes, B_BYTES = BN * kRowBytes, STAGE = A_BYTES + B_BYTES;
+  constexpr int A_LOADS = BM / 8 / NW, B_LOADS = BN / 8 / NW, LOADS = A_LOADS + B_LOADS;
+  constexpr int L1 = LOADS / 2, L0 = LOADS - L1;  // loads issued behind the barrier of a step / in the next step's first half
+  constexpr int YOUNGER = (NS - 2) * LOADS;       // loads that may be in flight at a step's barrier
+  static_assert(BM / 8 % NW == 0 && BN / 8 % NW == 0, "tile rows must split evenly over the wavefronts");
+  static_assert(CB % 2 == 0, "blocks are stored in pairs");
+  static_assert(NS >= 2 && YOUNGER < 64, "vmcnt is a six-bit counter");
+  using MB = RingMma<T>;
+  using Acc = typename MB::Acc;
+  using AccScalar = typename Epi::Acc;
+
+  extern __shared__ __align__(16) char smem[];
+
+  const int tiles = g.tiles_m * g.tiles_n;
+  const bool remap = tiles >= kXcdRemapMinTiles;
+  const int per_xcd = (tiles + kNumXcd - 1) / kNumXcd;
+  const int logical = remap ? (int)(blockIdx.x % kNumXcd) * per_xcd + (int)(blockIdx.x / kNumXcd) : (int)blockIdx.x;
+  if (logical >= tiles) {
+    if constexpr (Dequantises<Epi>::value)
+      if (epi.absmax_slots() != nullptr && threadIdx.x == 0) epi.absmax_slots()[blockIdx.x] = 0.f;
+    return;
+  }
+  int tile_m, tile_n;
+  tile_coords(logical, g.tiles_m, g.tiles_n, tile_m, tile_n);
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wm0 = (wave / WN) * (BM / WM), wn0 = (wave % WN) * (BN / WN);
+  const int lrow = lane & 15, lgrp = lane >> 4;
+  const int a_row0 = (wm0 + lrow) * kRowBytes, b_row0 = A_BYTES + (wn0 + lrow) * kRowBytes;
+  const int swz = (lrow >> 1) & 7;
+  int kdim = g.k, z_epi = 0;
+  uint32_t k_lo = 0;  // bytes
+  if (g.k_chunk > 0) {
+    const int lo = (int)blockIdx.y * g.k_chunk;
+    kdim = min(g.k_chunk, g.k - lo);
+    k_lo = (uint32_t)lo * (uint32_t)sizeof(T);
+    z_epi = (int)blockIdx.y;
+  }
+  const int ksteps = kdim / (kRowBytes / (int)sizeof(T));
+
+  // ---- load cursor: per-lane offsets of this wavefront's rows (rows past the edge repeat the last one)
+  const uint32_t lda_bytes = (uint32_t)(g.lda * (int64_t)sizeof(T)), ldb_bytes = (uint32_t)(g.ldb * (int64_t)sizeof(T));
+  uint32_t voff[LOADS];
+  {
+    const int sub = lane >> 3, p = lane & 7;
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i) {
+      const int row = (wave * A_LOADS + i) * 8 + sub;
+      voff[i] = (uint32_t)min(m0 + row, g.m - 1) * lda_bytes + ((p ^ ((row >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < B_LOADS; ++i) {
+      const int row = (wave * B_LOADS + i) * 8 + sub;
+      voff[A_LOADS + i] = (uint32_t)min(n0 + row, g.n - 1) * ldb_bytes + ((p ^ ((row >> 1) & 7)) << 4);
+    }
+  }
+  int dma_step = 0, dma_stage = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((address_space(3))) char lds_char;
+  lds_char* lds0 = reinterpret_cast<lds_char*>(reinterpret_cast<uintptr_t>(smem));
+  const int a_size = (int)((int64_t)g.m * lda_bytes), b_size = (int)((int64_t)g.n * ldb_bytes);
+  auto issue_one = [&](int i) __attribute__((always_inline)) {
+    const bool live = dma_step < ksteps;
+    if (i < A_LOADS) {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.a), 0, live ? a_size : 0, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds0 + dma_stage + (wave * A_LOADS + i) * 1024, 16, voff[i], k_lo + dma_step * kRowBytes, 0, 0);
+    } else {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.b), 0, live ? b_size : 0, 0x00020000);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds0 + dma_stage + A_BYTES + (wave * B_LOADS + i - A_LOADS) * 1024, 16, voff[i], k_lo + dma_step * kRowBytes, 0, 0);
+    }
+  };
+#else
+  auto issue_one = [&](int) {};
+#endif
+  auto advance = [&]() __attribute__((always_inline)) {
+    ++dma_step;
+    dma_stage = dma_stage == (NS - 1) * STAGE ? 0 : dma_stage + STAGE;
+  };
+
+  Chunk fa[2][RB], fb[2][CB];
+  Acc acc[RB][CB];
+  constexpr int READS = RB + CB, BLOCKS = RB * CB, MMAS = BLOCKS * MB::PARTS;
+  constexpr int RPM = (READS + MMAS - 1) / MMAS;  // reads per matrix instruction
+  // LO, NL: the loads of the cursor's step issued here, evenly spread over the matrix instructions
+  auto substep = [&](auto swap_tag, auto cur_tag, auto sub_tag, auto lo_tag, auto nl_tag, int rd) __attribute__((always_inline)) {
+    constexpr bool SWAP = decltype(swap_tag)::value;
+    constexpr int CUR = decltype(cur_tag)::value, SUB = decltype(sub_tag)::value, LO = decltype(lo_tag)::value, NL = decltype(nl_tag)::value;
+    const int off = ((SUB * 4 + lgrp) ^ swz) << 4;
+    const int a_at = a_row0 + off + rd, b_at = b_row0 + off + rd;
+#pragma unroll
+    for (int m = 0; m < MMAS; ++m) {
+      const int part = m / BLOCKS, blk = m % BLOCKS, i = blk / CB, j = blk % CB;  // (a block's parts apart: they form a chain)
+      if constexpr (SWAP) MB::run(fb[CUR][j], fa[CUR][i], acc[i][j], part);
+      else MB::run(fa[CUR][i], fb[CUR][j], acc[i][j], part);
+      // the fragments of the next half step, read as early as one per instruction allows
+#pragma unroll
+      for (int r = m * RPM; r < (m + 1) * RPM && r < READS; ++r) {
+        if (r < RB) fa[CUR ^ 1][r] = *reinterpret_cast<const Chunk*>(smem + a_at + r * 16 * kRowBytes);
+        else fb[CUR ^ 1][r - RB] = *reinterpret_cast<const Chunk*>(smem + b_at + (r - RB) * 16 * kRowBytes);
+      }
+#pragma unroll
+      for (int l = m * NL / MMAS; l < (m + 1) * NL / MMAS; ++l) issue_one(LO + l);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // ---- prologue: NS - 1 steps and the first part of one more are requested, the first step has landed
+#pragma unroll
+  for (int st = 0; st < NS - 1; ++st) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) issue_one(i);
+    advance();
+  }
+#pragma unroll
+  for (int i = 0; i < L1; ++i) issue_one(i);
+
+  const auto* bias = epi.bias_ptr();
+  using BiasT = typename std::remove_cv<typename std::remove_pointer<decltype(bias)>::type>::type;
+  BiasVec<BiasT> bv[CB / 2];
+  auto unit_chunk = [&](int p) __attribute__((always_inline)) { return 2 * (2 * p + (lgrp & 1)) + (lgrp >> 1); };
+
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][j][e] = 0;
+      asm volatile("" : "+a"(acc[i][j]));
+    }
+  asm volatile("s_nop 7");  // (the matrix instructions are inline asm: no hazard is seen between them and the zeroing)
+  dma_landed_barrier_but<(NS - 2) * LOADS + L1>();
+  {
+    const int off = (lgrp ^ swz) << 4;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) fa[0][i] = *reinterpret_cast<const Chunk*>(smem + (a_row0 + off) + i * 16 * kRowBytes);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) fb[0][j] = *reinterpret_cast<const Chunk*>(smem + (b_row0 + off) + j * 16 * kRowBytes);
+  }
+  auto k_loop = [&](auto swap_tag) __attribute__((always_inline)) {
+    int rd = 0;
+#pragma unroll 1
+    for (int s = 0; s < ksteps; ++s) {
+      substep(swap_tag, template_int<0>{}, template_int<1>{}, template_int<L1>{}, template_int<L0>{}, rd);
+      advance();
+      __builtin_amdgcn_sched_barrier(0);
+      dma_landed_barrier_but<YOUNGER>();
+      __builtin_amdgcn_sched_barrier(0);
+      rd = rd == (NS - 1) * STAGE ? 0 : rd + STAGE;
+      substep(swap_tag, template_int<1>{}, template_int<0>{}, template_int<0>{}, template_int<L1>{}, rd);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15");
+  };
+
+  float amax = 0.f;
+  bool swap = true;
+  if constexpr (HasColumnPass<Epi>::value) swap = !(epi.column_pass() && n0 + wn0 >= epi.first_column_of_pass());
+  if (swap) {
+    if constexpr (!Dequantises<Epi>::value) {
+#pragma unroll
+      for (int p = 0; p < CB / 2; ++p) bv[p].load(bias, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8), g.b);
+    }
+    k_loop(std::true_type{});
+    // Destination of a unit = a part that depends on its columns + a part that depends on its row, each found once.
+    typename RingDest<Epi>::Elem* col_at[CB / 2];
+    int64_t row_at[RB];
+    if constexpr (RingDest<Epi>::split) {
+#pragma unroll
+      for (int p = 0; p < CB / 2; ++p) col_at[p] = RingDest<Epi>::column(epi, z_epi, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8));
+#pragma unroll
+      for (int i = 0; i < RB; ++i) row_at[i] = RingDest<Epi>::row(epi, min(m0 + wm0 + i * 16 + lrow, g.m - 1));
+    }
+#pragma unroll
+    for (int p = 0; p < CB / 2; ++p) {
+      const int n = n0 + wn0 + unit_chunk(p) * 8;
+      float wide[8], scale[8];
+      float act_scale = 0.f;
+      if constexpr (Dequantises<Epi>::value) {
+        const int nc = min(n, g.n - 8);
+        act_scale = epi.act_scale[0];
+        load_row8<float>(epi.w_scale + nc, scale);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wide[e] = 0.f;
+        if (epi.has_bias()) load_row8<float>(bias + nc, wide);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wide[e] = 0.f;
+        if (bias != nullptr) bv[p].widen(wide);
+      }
+#pragma unroll
+      for (int i = 0; i < RB; ++i) {
+        AccScalar out[8];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          auto a = acc_read(acc[i][2 * p][e]), b = acc_read(acc[i][2 * p + 1][e]);
+          pair_swap<16>(a, b);
+          out[e] = a;
+          out[4 + e] = b;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if constexpr (Dequantises<Epi>::value) {
+            const float r = epi.activate(dequantise(out[e], act_scale, scale[e], wide[e], epi.has_bias()));
+            amax = fmaxf(amax, fabsf(r));
+            out[e] = __builtin_bit_cast(AccScalar, r);
+          } else {
+            out[e] += (AccScalar)wide[e];
+          }
+        }
+        const int m = m0 + wm0 + i * 16 + lrow;
+        if (m < g.m && n < g.n) {
+          if constexpr (RingDest<Epi>::split) {
+            float fin[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) fin[e] = RingDest<Epi>::finish(epi, out[e]);
+            if constexpr (AddsResidual<Epi>::value) {
+              float res[8];
+              load_row8(epi.residual + (col_at[p] - epi.c) + row_at[i], res);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) fin[e] += res[e];
+            }
+            store_row8(col_at[p] + row_at[i], fin);
+          } else {
+            epi.store8(z_epi, m, n, out, 8);
+          }
+        }
+      }
+    }
+  } else {
+    if constexpr (HasColumnPass<Epi>::value) {
+      float bj[CB];
+      load_bias_columns_stride<CB, 16>(epi, n0 + wn0 + lrow, g.n, bj);
+      k_loop(std::false_type{});
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const int n = n0 + wn0 + j * 16 + lrow;
+        if constexpr (RB % 2 == 0) {
+#pragma unroll
+          for (int p = 0; p < RB / 2; ++p) {
+            float out[8];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float a = acc_read(acc[2 * p][j][e]), b = acc_read(acc[2 * p + 1][j][e]);
+              pair_swap<16>(a, b);
+              out[e] = a + bj[j];
+              out[4 + e] = b + bj[j];
+            }
+            const int m = m0 + wm0 + unit_chunk(p) * 8;
+            if (m < g.m && n < g.n) epi.store_col8(m, g.m, n, out);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < RB; ++i) {
+            float out[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = acc_read(acc[i][j][e]) + bj[j];
+            const int m = m0 + wm0 + i * 16 + lgrp * 4;
+            if (m < g.m && n < g.n) epi.store_col4(m, g.m, n, out);
+          }
+        }
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // the loads past the last step have returned before the LDS is given back
+  publish_absmax(epi, amax, reinterpret_cast<float*>(smem), NW * kWave);
+}
+
+template <typename T, int BM, int BN, int WM, int WN, int NS, typename Epi>
+inline int launch_ring(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
+  constexpr int LDS = ring_lds_bytes<BM, BN, NS>();
+  static_assert(LDS <= kLdsPerCu, "tile does not fit in LDS");
+  if (describe_only("dma", WM * WN, BM, BN, slices)) return 0;
+  g.tiles_m = (g.m + BM - 1) / BM;
+  g.tiles_n = (g.n + BN - 1) / BN;
+  const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n;
+  TTMI_REQUIRE(tiles < (1ll << 30), "GEMM grid too large");
+  const unsigned grid_x = tiles >= kXcdRemapMinTiles ? (unsigned)(ceil_div(tiles, kNumXcd) * kNumXcd) : (unsigned)tiles;
+  if (!absmax_grid_ok(epi, grid_x, 1)) return launch_ring<T, BM, BN, WM, WN, NS>(g, without_absmax(epi), slices, s);
+  auto kern = gemm_ring_kernel<T, BM, BN, WM, WN, NS, Epi>;
+  if (LDS > 64 * 1024) {
+    const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
+    if (rc != 0) return rc;
+  }
+  hipLaunchKernelGGL(kern, dim3(grid_x, (unsigned)slices), dim3(WM * WN * kWave), LDS, s, g, epi);
+  return launch_status("gemm_ring_kernel");
+}
+
+// ------------------------------------------------------------------------ selection -----
+// Tiles and the time model that picks one, in microseconds.  With q = workgroups per CU (rounded up) and R = how many of
+// them are resident there at once,
+//   time = first + again * (q - 1) + K steps * max(lone * ceil(q / R), shared * q):
+// `first` and `again` are what a workgroup costs beyond its K loop (launch, first operands, epilogue), `lone` a K step of
+// a workgroup that waits for its own latencies, `shared` one on a CU whose matrix pipe or operand path is full.  The
+// numbers are least-squares fits to launches of M = 72 ... 16384 rows by the four encoder products of hidden 768 and
+// 1024 (fp16, fp32, int8); over those the tile the model picks is 0.3 % (fp32: 2.5 %) slower than the best one.
+struct RingTile {
+  int bm, bn, wave_cols, resident;
+  float first, again, lone, shared;
+};
+// X(BM, BN, WM, WN, stages, resident, first, again, lone, shared)
+#define TTMI_RING_TILES_16(X)                                \
+  X(32, 64, 2, 2, 4, 3, 2.90f, 0.27f, 0.152f, 0.128f)        \
+  X(64, 64, 4, 2, 4, 2, 3.10f, 0.65f, 0.177f, 0.177f)        \
+  X(64, 96, 4, 1, 4, 2, 3.27f, 1.15f, 0.188f, 0.212f)        \
+  X(128, 64, 2, 2, 4, 1, 3.19f, 2.17f, 0.252f, 0.252f)       \
+  X(128, 96, 4, 1, 3, 1, 3.58f, 2.66f, 0.325f, 0.326f)       \
+  X(128, 128, 4, 2, 3, 1, 3.74f, 4.03f, 0.374f, 0.373f)      \
+  X(128, 192, 4, 2, 3, 1, 4.88f, 6.69f, 0.464f, 0.461f)      \
+  X(256, 128, 4, 2, 3, 1, 5.36f, 8.33f, 0.576f, 0.571f)
+#define TTMI_RING_TILES_32(X)                                \
+  X(32, 64, 2, 2, 3, 4, 1.58f, 0.66f, 0.727f, 0.257f)        \
+  X(64, 64, 4, 2, 4, 2, 5.87f, 0.00f, 0.289f, 0.540f)        \
+  X(64, 64, 2, 2, 3, 3, 10.1f, 0.00f, 0.350f, 0.509f)        \
+  X(64, 96, 4, 1, 3, 2, 9.93f, 0.00f, 0.170f, 0.777f)        \
+  X(64, 128, 4, 2, 3, 2, 4.34f, 0.00f, 0.281f, 0.957f)       \
+  X(128, 192, 4, 2, 3, 1, 7.27f, 7.53f, 2.620f, 2.619f)
+#define TTMI_RING_TILES_8(X)                                 \
+  X(32, 64, 2, 2, 4, 3, 3.55f, 0.74f, 0.141f, 0.120f)        \
+  X(64, 64, 4, 2, 4, 2, 4.06f, 1.59f, 0.173f, 0.173f)        \
+  X(64, 96, 4, 1, 4, 2, 5.47f, 2.29f, 0.203f, 0.214f)        \
+  X(128, 64, 2, 2, 4, 1, 5.08f, 4.03f, 0.258f, 0.258f)       \
+  X(64, 192, 4, 2, 3, 1, 6.02f, 5.34f, 0.379f, 0.377f)       \
+  X(128, 128, 4, 2, 3, 1, 6.55f, 6.98f, 0.376f, 0.376f)      \
+  X(128, 192, 4, 2, 3, 1, 8.73f, 10.6f, 0.465f, 0.465f)
+
+#define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
+template <size_t ELEM>
+struct RingTiles;
+template <>
+struct RingTiles<2> {
+  static constexpr RingTile k[] = {TTMI_RING_TILES_16(TTMI_RING_ROW)};
+};
+template <>
+struct RingTiles<4> {
+  static constexpr RingTile k[] = {TTMI_RING_TILES_32(TTMI_RING_ROW)};
+};
+template <>
+struct RingTiles<1> {
+  static constexpr RingTile k[] = {TTMI_RING_TILES_8(TTMI_RING_ROW)};
+};
+#undef TTMI_RING_ROW
+
+enum class RingUse { kWhole, kSliced, kLayerNorm };  // never cut along K / cut where it pays / slices summed by the LayerNorm
+struct RingPlan {
+  int tile = -1, slices = 1;
+  int64_t rounds = 0;  // workgroups per CU, rounded up
+  double us = 1e300;
+};
+
+// column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V)
+template <typename T>
+inline RingPlan pick_ring(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit = 0) {
+  RingPlan best;
+  int index = 0;
+  for (const RingTile& t : RingTiles<sizeof(T)>::k) {
+    const int i = index++;
+    if (column_limit > 0 && column_limit % t.wave_cols != 0) continue;
+    const int most = use == RingUse::kWhole ? 1 : (int)std::min<int64_t>(16, std::max<int64_t>(1, ksteps / 4));
+    for (int slices = 1; slices <= most; ++slices) {
+      if (slices > 1 && slices * m * n * 4 > (32ll << 20)) break;
+      const int64_t q = ceil_div(ceil_div(m, t.bm) * ceil_div(n, t.bn) * slices, compute_units());
+      double us = t.first + t.again * (q - 1) + ceil_div(ksteps, slices) * std::max<double>(t.lone * ceil_div(q, t.resident), t.shared * q);
+      // partial products: written and read once more, and a launch of their own where no LayerNorm follows
+      if (slices > 1 || use == RingUse::kLayerNorm) us += slices * m * n * 4 / 4e6;
+      if (slices > 1 && use == RingUse::kSliced) us += 4.0;
+      if (us < best.us) best = RingPlan{i, slices, q, us};
+    }
+  }
+  return best;
+}
+
+template <typename T>
+inline bool ring_operands_ok(const GemmArgs& g) {  // 32-bit buffer offsets, columns in groups of eight
+  const int64_t limit = (int64_t)1 << 31;
+  return g.n % 8 == 0 && (int64_t)g.m * g.lda * (int64_t)sizeof(T) < limit && (int64_t)g.n * g.ldb * (int64_t)sizeof(T) < limit;
+}
+
+template <typename T, typename Epi>
+inline int launch_ring_tile(int tile, const GemmArgs& g, const Epi& epi, int slices, hipStream_t s) {
+  int index = 0;
+#define TTMI_RING_TRY(BM, BN, WM, WN, NS, R, F, A, L, S) \
+  if (tile == index++) return launch_ring<T, BM, BN, WM, WN, NS>(g, epi, slices, s);
+  if constexpr (sizeof(T) == 2) { TTMI_RING_TILES_16(TTMI_RING_TRY) }
+  if constexpr (sizeof(T) == 4) { TTMI_RING_TILES_32(TTMI_RING_TRY) }
+  if constexpr (sizeof(T) == 1) { TTMI_RING_TILES_8(TTMI_RING_TRY) }
+#undef TTMI_RING_TRY
+  return fail(TTMI_EINVAL, "no such tile");
+}
+
+// The product in `plan.slices` K slices: fp32 partial products in the split-K workspace, summed by `reduce(ws, slices, vec, stream)`.
+template <typename T, typename Reduce>
+inline int launch_ring_slices(GemmArgs g, const RingPlan& plan, hipStream_t s, const Reduce& reduce) {
+  constexpr int BK = kRowBytes / (int)sizeof(T);
+  g.k_chunk = (int)ceil_div(g.k / BK, plan.slices) * BK;
+  const int used = (int)ceil_div(g.k, g.k_chunk);
+  float* ws = nullptr;
+  if (tl_describe == nullptr) {
+    const int rc = splitk_workspace((size_t)used * g.m * g.n * sizeof(float), s, &ws);
+    if (rc != 0) return rc;
+  }
+  const EpiPartial part{ws, (int64_t)g.m * g.n, g.n, true};
+  const int rc = launch_ring_tile<T>(plan.tile, g, part, used, s);
+  if (rc != 0 || tl_describe != nullptr) return rc;
+  reduce(ws, used, true, s);
+  return launch_status("gemm_ring_slices");
+}
+
+template <typename Epi>
+inline bool epilogue_vec(const Epi& epi) {
+  if constexpr (std::is_same<Epi, EpiDequantQkvSplit>::value) return epi.split.vec && aligned16(epi.w_scale) && aligned16(epi.split.bias);
+  else if constexpr (std::is_same<Epi, EpiDequant>::value) return epi.vec && aligned16(epi.w_scale) && aligned16(epi.bias);
+  else return epi.vec;
+}
+template <typename Epi>
+struct IsGelu : std::false_type {};
+template <typename T>
+struct IsGelu<EpiBias<T, TTMI_ACT_GELU, true, false>> : std::true_type {};
+
+// Selection for the products with an epilogue: this kernel, or for large problems the persistent tiles of gemm_w4.h
+// (16-bit types) and of gemm_fast_kernel (int8), whose epilogues run under the next tile's first loads.
+template <typename T, typename Epi>
+struct RingKernel {
+  static int64_t column_limit(const Epi& epi) {
+    if constexpr (HasColumnPass<Epi>::value) return epi.v_pitch > 0 ? 2 * (int64_t)epi.hidden : 0;
+    else return 0;
+  }
+  static RingPlan plan(const GemmArgs& g, const Epi& epi) {
+    // a cut needs an epilogue that the reduction kernel can apply to rows of eight columns
+    constexpr bool cut = std::is_same<typename Epi::Acc, float>::value;
+    const RingUse use = cut && column_limit(epi) == 0 ? RingUse::kSliced : RingUse::kWhole;
+    return pick_ring<T>(g.m, g.n, g.k / (kRowBytes / (int)sizeof(T)), use, column_limit(epi));
+  }
+  static bool ok(const GemmArgs& g, const Epi& epi, int batch) {
+    return batch == 1 && g.k_chunk == 0 && ring_operands_ok<T>(g) && epilogue_vec(epi) && plan(g, epi).tile >= 0;
+  }
+  static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) {
+    constexpr int BK = kRowBytes / (int)sizeof(T);
+    // (65 to 128 rows with GELU: one 32 x 32 tile per wavefront, W and A straight from L2)
+    if constexpr (IsGelu<Epi>::value && sizeof(T) == 2)
+      if (g.m > 64 && wave_kernel_ok<T>(g, 1, true)) return launch_wave<T>(g, epi, s);
+    const RingPlan p = plan(g, epi);
+    if constexpr (sizeof(T) == 2) {
+      const int force = kernel_switch(kSwitchLargeTile);
+      // More than one workgroup per CU: long enough a launch that the chip runs at its power limit, under which the small
+      // tiles' extra LDS and L2 traffic costs clock (16384 x 1024 x 4096: 123 us against 106 although the unthrottled
+      // model has it 20 % ahead).
+      const double margin = p.rounds > 1 ? 1.3 : 1.0;
+      if (force != 0 && LargeTileKernel<T, Epi>::eligible(g, epi) && (force == 1 || LargeTileKernel<T, Epi>::us(g, epi) < margin * p.us))
+        return LargeTileKernel<T, Epi>::launch(g, epi, s);
+    }
+    if constexpr (sizeof(T) == 1) {
+      auto us = [&](int bn, double first, double again, double step) {
+        return first + ceil_div(ceil_div(g.m, 256) * ceil_div(g.n, bn), compute_units()) * (again + g.k / BK * step);
+      };
+      const double us192 = us(192, 2.8, 11.3, 1.224), us256 = us(256, 2.6, 6.8, 2.761);
+      if (std::min(us192, us256) < p.us)
+        return us192 < us256 ? launch_fast<T, 256, 192, 4, 2, Epi>(g, epi, 1, s) : launch_fast<T, 256, 256, 2, 4, Epi>(g, epi, 1, s);
+    }
+    if constexpr (std::is_same<typename Epi::Acc, float>::value)
+      if (p.slices > 1) return launch_ring_slices<T>(g, p, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
+    return launch_ring_tile<T>(p.tile, g, epi, 1, s);
+  }
+};
+
+}  // namespace ttmi

@@ -1,0 +1,181 @@
+// The entry points of the GEMM family for one element type.  gemm_<type>.hip instantiates them, so that the element
+// types compile side by side; gemm.hip holds the C ABI.
+#pragma once
+
+#include "gemm_ring.h"
+
+namespace ttmi {
+
+template <typename T>
+int gemm_alpha_beta(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda,
+                           int64_t ldb, int64_t ldc, int inner, int64_t a_outer, int64_t a_inner,
+                           int64_t b_outer, int64_t b_inner, int64_t c_outer, int64_t c_inner, int64_t batch,
+                           int trans_b, float alpha, float beta, hipStream_t s) {
+  TTMI_REQUIRE(m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension too large");
+  GemmArgs g{};
+  g.a = (const char*)a;
+  g.b = (const char*)b;
+  g.m = (int)m; g.n = (int)n; g.k = (int)k;
+  g.lda = lda; g.ldb = ldb;
+  g.inner = inner;
+  g.a_outer = a_outer; g.a_inner = a_inner; g.b_outer = b_outer; g.b_inner = b_inner;
+  constexpr int KPC = 16 / sizeof(T);
+  const bool c_vec = aligned16(c) && ldc % KPC == 0 && c_outer % KPC == 0 && c_inner % KPC == 0;
+  EpiAlphaBeta<T> epi{(T*)c, ldc, c_outer, c_inner, inner, alpha, beta, c_vec};
+  auto mult = [](int64_t v) { return v % KPC == 0; };
+  bool aligned = aligned16(a) && aligned16(b) && mult(lda) && mult(ldb) && mult(a_outer) && mult(a_inner) &&
+                 mult(b_outer) && mult(b_inner);
+  if (trans_b) {
+    aligned = aligned && mult(k);
+    return launch_gemm<T, false>(g, epi, (int)batch, aligned, s);
+  }
+  aligned = aligned && mult(k) && mult(n);
+  return launch_gemm<T, true>(g, epi, (int)batch, aligned, s);
+}
+
+
+template <typename T>
+int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, hipStream_t s) {
+  const int64_t m = g.m, n = g.n, k = g.k, lda = g.lda, ldb = g.ldb;
+  const void *a = g.a, *b = g.b;
+  constexpr int KPC = 16 / sizeof(T);
+  const bool aligned = aligned16(a) && aligned16(b) && lda % KPC == 0 && ldb % KPC == 0 && k % KPC == 0;
+  const bool c_vec = aligned16(c) && ldc % KPC == 0 && aligned16(args->bias) && aligned16(args->residual);
+  const bool qkv_vec = aligned16(args->q) && aligned16(args->k) && aligned16(args->v) && aligned16(args->bias) &&
+                       args->head_dim % 8 == 0;
+  switch (epilogue) {
+    case TTMI_EPI_BIAS: {
+      TTMI_REQUIRE(c && args->bias && ldc >= n, "BIAS epilogue needs c and bias");
+      EpiBias<T, 0, false, false> epi{(T*)c, (const T*)args->bias, nullptr, ldc, c_vec};
+      return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+    }
+    case TTMI_EPI_BIAS_ACT: {
+      TTMI_REQUIRE(c && args->bias && ldc >= n, "BIAS_ACT epilogue needs c and bias");
+      if (args->act == TTMI_ACT_GELU) {
+        EpiBias<T, TTMI_ACT_GELU, true, false> epi{(T*)c, (const T*)args->bias, nullptr, ldc, c_vec};
+        return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+      } else if (args->act == TTMI_ACT_TANH) {
+        EpiBias<T, TTMI_ACT_TANH, true, false> epi{(T*)c, (const T*)args->bias, nullptr, ldc, c_vec};
+        return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+      } else if (args->act == TTMI_ACT_RELU) {
+        EpiBias<T, TTMI_ACT_RELU, true, false> epi{(T*)c, (const T*)args->bias, nullptr, ldc, c_vec};
+        return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+      }
+      return fail(TTMI_EINVAL, "unknown activation");
+    }
+    case TTMI_EPI_F32_OUT: {
+      TTMI_REQUIRE(c && ldc >= n, "F32_OUT epilogue needs c");
+      EpiF32<T> epi{(float*)c, (const T*)args->bias, ldc, aligned16(c) && ldc % 4 == 0 && aligned16(args->bias)};
+      return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+    }
+    case TTMI_EPI_BIAS_RESIDUAL: {
+      TTMI_REQUIRE(c && args->bias && args->residual && ldc >= n, "BIAS_RESIDUAL epilogue needs c, bias, residual");
+      EpiBias<T, 0, false, true> epi{(T*)c, (const T*)args->bias, (const T*)args->residual, ldc, c_vec};
+      return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+    }
+    case TTMI_EPI_QKV_SPLIT:
+    case TTMI_EPI_QKV_SPLIT_PAD: {
+      const bool pad = epilogue == TTMI_EPI_QKV_SPLIT_PAD;
+      TTMI_REQUIRE(args->seq > 0 && args->heads > 0 && args->head_dim > 0, "QKV epilogue needs seq/heads/head_dim");
+      const bool single = n == args->heads * args->head_dim;  // one projection: only q is written
+      TTMI_REQUIRE(single || n == 3 * args->heads * args->head_dim, "N must be heads*head_dim or 3*heads*head_dim");
+      TTMI_REQUIRE(args->q && args->bias && (single || (args->k && args->v)), "QKV epilogue needs q, k, v, bias");
+      TTMI_REQUIRE(!single || args->v_seq_pitch == 0, "v_seq_pitch needs the three-way split");
+      if (pad) TTMI_REQUIRE(args->token_rows != nullptr && args->batch > 0, "padded QKV epilogue needs token_rows and batch");
+      else TTMI_REQUIRE(m % args->seq == 0, "M must be a multiple of seq");
+      const int hidden = (int)(args->heads * args->head_dim);
+      const int64_t vp = args->v_seq_pitch;
+      TTMI_REQUIRE(vp == 0 || (vp >= args->seq && vp % 8 == 0 && vp < (1ll << 31) && hidden % 8 == 0),
+                   "v_seq_pitch must be 0 or a multiple of 8 that is >= seq (hidden a multiple of 8)");
+      if (pad) {
+        EpiQkvSplit<T, true> epi{(T*)args->q, (T*)args->k, (T*)args->v, (const T*)args->bias, args->token_rows,
+                                 (int)args->seq, (int)args->heads, (int)args->head_dim, hidden,
+                                 FastDiv((uint32_t)args->seq), FastDiv((uint32_t)hidden), FastDiv((uint32_t)args->head_dim), qkv_vec, (int)vp};
+        return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+      }
+      EpiQkvSplit<T, false> epi{(T*)args->q, (T*)args->k, (T*)args->v, (const T*)args->bias, nullptr,
+                                (int)args->seq, (int)args->heads, (int)args->head_dim, hidden,
+                                FastDiv((uint32_t)args->seq), FastDiv((uint32_t)hidden), FastDiv((uint32_t)args->head_dim), qkv_vec, (int)vp};
+      return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+    }
+    default:
+      return fail(TTMI_EINVAL, "unknown epilogue");
+  }
+}
+
+// Product + AddBiasLayerNorm.  The product reaches the normalisation in fp32 where it is short of rows or long in K
+// (`fp32_product`: few rows make the extra bytes free, a long sum loses most to a 16-bit rounding), as K slices or
+// whole, summed by the kernel that normalises; else it passes through `out` in the storage type.
+template <typename T>
+int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
+                               const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
+                               int64_t k, float eps, int dtype, hipStream_t s) {
+  constexpr int KPC = 16 / sizeof(T), BK = kRowBytes / sizeof(T);
+  const bool aligned = aligned16(a) && aligned16(w) && k % KPC == 0;
+  auto aligned_rows = [&](const void* p, size_t elem) { return (reinterpret_cast<uintptr_t>(p) % (4 * elem)) == 0; };
+  const bool rows_ok = n % 4 == 0 && n <= 4096 && aligned_rows(out, sizeof(T)) && aligned_rows(bias, sizeof(T)) &&
+                       aligned_rows(gamma, sizeof(T)) && aligned_rows(beta, sizeof(T)) &&
+                       (residual_f32 != nullptr ? aligned16(residual_f32) && aligned16(out_f32) : aligned_rows(residual, sizeof(T)));
+  GemmArgs g{};
+  g.a = (const char*)a;
+  g.b = (const char*)w;
+  g.m = (int)m; g.n = (int)n; g.k = (int)k;
+  g.lda = k; g.ldb = k;
+  g.inner = 1;
+  auto reduce = [&](const float* ws, int slices, bool, hipStream_t st) {
+    auto launch = [&](auto iters) {
+      hipLaunchKernelGGL((splitk_reduce_layer_norm_kernel<T, decltype(iters)::value>), dim3((unsigned)m), dim3(256), 0, st, ws,
+                         slices, (int)m, (int)n, (const T*)bias, (const T*)residual, residual_f32, (const T*)gamma,
+                         (const T*)beta, (T*)out, out_f32, eps);
+    };
+    if (n <= 1024) launch(std::integral_constant<int, 1>{});
+    else if (n <= 2048) launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 4>{});
+  };
+  if constexpr (sizeof(T) == 2) {
+    int slices = rows_ok ? w4_splitk_slices<T>(g, aligned) : 0;
+    // (an optimisation of a product that also runs whole: where the caller has fixed the workspace and the partial
+    // products do not fit it, nothing is refused)
+    if (slices > 1 && tl_fixed_workspace.ptr != nullptr &&
+        (size_t)slices * (size_t)m * (size_t)n * sizeof(float) > tl_fixed_workspace.bytes)
+      slices = 0;
+    if (slices > 1) return launch_w4_splitk<T>(g, slices, s, reduce);
+  }
+  const bool ring = aligned && k % BK == 0 && ring_operands_ok<T>(g);
+  if (!ring && rows_ok) {  // widths that are no multiple of eight
+    const SplitPlan plan = plan_split<T>(m, n, k, 1, aligned);
+    if (plan.kind == SplitKind::kDmaTiles) return launch_fast_splitk<T>(g, plan.splits, k / BK, BK, s, reduce);
+    if (plan.kind == SplitKind::kSmallTiles) return launch_splitk<T>(g, plan.splits, k / BK, BK, s, reduce);
+  }
+  const bool fp32_product = m <= 384 || (k >= 2 * n && m * n * 4 <= (20ll << 20));
+  if (ring && rows_ok && fp32_product) {
+    const RingPlan plan = pick_ring<T>(m, n, k / BK, RingUse::kLayerNorm);
+    return launch_ring_slices<T>(g, plan, s, reduce);
+  }
+  // With an fp32 residual stream and room for it, the product stays in fp32 too: the GEMM stores its accumulators to
+  // out_f32 and the LayerNorm pass reads them there.
+  if (residual_f32 != nullptr && out_f32 != residual_f32 && dtype != TTMI_F32) {
+    EpiF32<T> epi{out_f32, nullptr, n, aligned16(out_f32) && n % 4 == 0};
+    const int rc = launch_gemm<T, false>(g, epi, 1, aligned, s);
+    if (rc != 0) return rc;
+    return ttmi_add_bias_layer_norm_product32(out, residual_f32, bias, gamma, beta, out_f32, m, n, eps, dtype, s);
+  }
+  // (EpiBias without a bias: the plain product, through the selection of the fused ones)
+  EpiBias<T, 0, false, false> epi{(T*)out, nullptr, nullptr, n, aligned16(out) && n % KPC == 0};
+  const int rc = launch_gemm<T, false>(g, epi, 1, aligned, s);
+  if (rc != 0) return rc;
+  if (residual_f32 != nullptr)
+    return ttmi_add_bias_layer_norm_residual32(out, residual_f32, bias, gamma, beta, out_f32, m, n, eps, dtype, s);
+  return ttmi_add_bias_layer_norm(out, residual, bias, gamma, beta, m, n, eps, dtype, s);
+}
+
+#define TTMI_INSTANTIATE_GEMM(T)                                                                                            \
+  template int gemm_alpha_beta<T>(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, \
+                                  int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, float, float,           \
+                                  hipStream_t);                                                                               \
+  template int gemm_fused_typed<T>(const GemmArgs&, void*, int64_t, int, const ttmi_epilogue_args*, hipStream_t);             \
+  template int gemm_bias_layer_norm_typed<T>(const void*, const void*, void*, const void*, const float*, const void*,         \
+                                             const void*, const void*, float*, int64_t, int64_t, int64_t, float, int,         \
+                                             hipStream_t);
+
+}  // namespace ttmi

@@ -945,7 +945,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
 // Whether a problem may take this kernel: 16-bit type, one problem, aligned operands, an even number of K steps,
 // columns in groups of eight, operands below 2 GiB (32-bit buffer offsets).
 template <typename T>
-static bool w4_eligible(const GemmArgs& g, int batch, bool aligned) {
+inline bool w4_eligible(const GemmArgs& g, int batch, bool aligned) {
   if (sizeof(T) != 2 || batch != 1 || !aligned || g.k_chunk != 0) return false;
   constexpr int BK = kRowBytes / (int)sizeof(T);
   if (g.k % (2 * BK) != 0 || g.n % 8 != 0) return false;
@@ -954,7 +954,7 @@ static bool w4_eligible(const GemmArgs& g, int batch, bool aligned) {
 }
 // The output of a linear epilogue is addressed with 32-bit offsets as well.
 template <typename T>
-static bool w4_output_fits(const GemmArgs& g, int64_t ldc) {
+inline bool w4_output_fits(const GemmArgs& g, int64_t ldc) {
   return (int64_t)g.m * ldc * (int64_t)sizeof(T) < ((int64_t)1 << 31);
 }
 
@@ -965,7 +965,7 @@ template <int BN, typename Epi>
 constexpr bool w4_three_stages_fit() { return (BN == 192 && !HasColumnPass<Epi>::value) || StoresF32<Epi>::value; }
 
 template <typename T, int BN, typename Epi, int AS = 2, bool DIRECT = false>
-static int launch_w4(GemmArgs g, const Epi& epi, hipStream_t s, int split_col = 0) {
+inline int launch_w4(GemmArgs g, const Epi& epi, hipStream_t s, int split_col = 0) {
   if constexpr (AS == 2 && !DIRECT && w4_three_stages_fit<BN, Epi>()) {
     if (kernel_switch(kSwitchW4AStages) != 2) return launch_w4<T, BN, Epi, 3>(g, epi, s, split_col);
   }
@@ -1008,7 +1008,7 @@ constexpr TileConfig kW4Tile256{256, 256, 1, 1.10f};
 // TTMI_LARGE_TILE=0 keeps every problem on the 8-wavefront kernels, =1 sends every eligible problem here whatever
 // the cost model says (for A/B timing and for tests of small and ragged shapes); unset: the cost model decides.
 template <typename T, typename Epi>
-static bool w4_wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned) {
+inline bool w4_wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned) {
   if (!epi.vec || !w4_eligible<T>(g, batch, aligned)) return false;
   const int force = kernel_switch(kSwitchLargeTile);
   if (force == 0) return false;
@@ -1019,9 +1019,20 @@ static bool w4_wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned
                                              : tile_cost(kW4Tile192, g.m, g.n, batch);
   return mine < other;
 }
+// Time model for the selection among the products with an epilogue (see gemm_ring.h), in microseconds: fits to the launches
+// of 3200 ... 16384 rows, one persistent workgroup per CU.
+inline double w4_us(int bn, int64_t m, int64_t tiles_n, int64_t ksteps) {
+  const int64_t per_cu = ceil_div(ceil_div(m, 256) * tiles_n, compute_units());
+  return bn == 256 ? 3.8 + per_cu * (4.1 + ksteps * 1.449) : 4.2 + per_cu * (4.3 + ksteps * 1.090);
+}
+template <typename T>
+inline double w4_linear_us(const GemmArgs& g) {
+  const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T));
+  return std::min(w4_us(192, g.m, ceil_div(g.n, 192), ksteps), w4_us(256, g.m, ceil_div(g.n, 256), ksteps));
+}
 // Which of the two tile widths a linear epilogue takes.
 template <typename T, typename Epi>
-static int launch_w4_linear(const GemmArgs& g, const Epi& epi, hipStream_t s) {
+inline int launch_w4_linear(const GemmArgs& g, const Epi& epi, hipStream_t s) {
   if (tile_cost(kW4Tile256, g.m, g.n, 1) < tile_cost(kW4Tile192, g.m, g.n, 1)) return launch_w4<T, 256>(g, epi, s);
   return launch_w4<T, 192>(g, epi, s);
 }
@@ -1032,30 +1043,22 @@ static int launch_w4_linear(const GemmArgs& g, const Epi& epi, hipStream_t s) {
 // 6275 x 768 x 3072), where whole tiles are too few for the CUs whatever their size: 100 tiles of 256 x 192 with 48 K
 // steps each become 200 items of 24 steps.  Every slice has the same, even number of K steps.
 template <typename T>
-static bool w4_splitk_ok(const GemmArgs& g, int splits, bool aligned) {
+inline bool w4_splitk_ok(const GemmArgs& g, int splits, bool aligned) {
   constexpr int BK = kRowBytes / (int)sizeof(T);
   return splits > 1 && w4_eligible<T>(g, 1, aligned) && g.k % (splits * 2 * BK) == 0 && g.n % 8 == 0 &&
          (int64_t)splits * g.m * g.n * 4 < ((int64_t)1 << 31);
 }
-// How many K slices such a product gets on this kernel (0 or 1 = it is not taken).  Switch TTMI_W4_SPLITK: 0 = never,
-// n >= 2 = n slices for every product that can be cut that way.
+// How many K slices such a product gets on this kernel: none by itself (the tiles of gemm_ring.h fill the chip at those
+// sizes: 6275 x 768 x 3072 in 32 against 41 us), n under switch TTMI_W4_SPLITK = n for every product that can be cut.
 template <typename T>
-static int w4_splitk_slices(const GemmArgs& g, bool aligned) {
+inline int w4_splitk_slices(const GemmArgs& g, bool aligned) {
   const int force = kernel_switch(kSwitchW4SplitK);
   if (force == 0 || kernel_switch(kSwitchLargeTile) == 0) return 0;
   if (force >= 2) return w4_splitk_ok<T>(g, force, aligned) ? force : 0;
-  // Two slices where they turn 0.35-0.5 rounds of whole tiles into 0.7-1 round of items and K is long enough to
-  // pay for the fp32 partial products (measured, LayerNorm included: 6275 x 768 x 3072 54 -> 46 us; at 4924 and at
-  // 10000 rows, where the 8-wavefront kernels' own tiles fill the chip better, level, and not taken).
-  constexpr int BK = kRowBytes / (int)sizeof(T);
-  if (g.k / BK < 32 || !w4_splitk_ok<T>(g, 2, aligned)) return 0;
-  const bool wide = tile_cost(kW4Tile256, g.m, g.n, 2) < tile_cost(kW4Tile192, g.m, g.n, 2);  // as launch_w4_splitk picks
-  const int64_t tiles = ceil_div(g.m, 256) * ceil_div(g.n, wide ? 256 : 192);
-  const int64_t cus = compute_units();
-  return (2 * tiles <= cus && 2 * tiles * 10 > cus * 7) ? 2 : 0;
+  return 0;
 }
 template <typename T, typename Reduce>
-static int launch_w4_splitk(GemmArgs g, int splits, hipStream_t s, const Reduce& reduce) {
+inline int launch_w4_splitk(GemmArgs g, int splits, hipStream_t s, const Reduce& reduce) {
   float* ws = nullptr;
   if (tl_describe == nullptr) {
     const int rc = splitk_workspace((size_t)splits * g.m * g.n * sizeof(float), s, &ws);
@@ -1076,9 +1079,8 @@ static int launch_w4_splitk(GemmArgs g, int splits, hipStream_t s, const Reduce&
 template <typename T, int ACT, bool HAS_ACT>
 struct LargeTileKernel<T, EpiBias<T, ACT, HAS_ACT, false>, typename std::enable_if<sizeof(T) == 2>::type> {
   using Epi = EpiBias<T, ACT, HAS_ACT, false>;
-  static bool wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned) {
-    return w4_output_fits<T>(g, epi.ldc) && w4_wanted<T>(g, epi, batch, aligned);
-  }
+  static bool eligible(const GemmArgs& g, const Epi& epi) { return epi.vec && w4_output_fits<T>(g, epi.ldc) && w4_eligible<T>(g, 1, true); }
+  static double us(const GemmArgs& g, const Epi&) { return w4_linear_us<T>(g); }
   static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) { return launch_w4_linear<T>(g, epi, s); }
 };
 // Bias + head split of a dense (not packed) batch.  With V kept transposed the tiles of the V third run unswapped, so
@@ -1091,30 +1093,24 @@ struct LargeTileKernel<T, EpiQkvSplit<T, false>, typename std::enable_if<sizeof(
   static bool split_run(const GemmArgs& g, const Epi& epi) {
     return epi.v_pitch > 0 && g.n == 3 * epi.hidden && (2 * epi.hidden) % 192 != 0;
   }
-  // cost of the 192-wide tiles with the tile columns the two runs really have (one or two of them ragged)
-  static double cost192(const GemmArgs& g, const Epi& epi, int batch) {
+  // (with the tile columns the two runs really have, one or two of them ragged)
+  static double us192(const GemmArgs& g, const Epi& epi) {
     const int64_t columns = split_run(g, epi) ? ceil_div(2 * epi.hidden, 192) + ceil_div(epi.hidden, 192) : ceil_div(g.n, 192);
-    return tile_cost(kW4Tile192, g.m, columns * 192, batch);
+    return w4_us(192, g.m, columns, g.k / (kRowBytes / (int)sizeof(T)));
   }
   // the 256-wide tile serves widths it divides, V third included; its head-split epilogue spills some registers, so
   // it is rated a little below the 256-wide tile of the row-major epilogues
-  static constexpr TileConfig kTile256{256, 256, 1, 1.07f};
-  static bool fits256(const GemmArgs& g, const Epi& epi) { return g.n % 256 == 0 && (epi.v_pitch == 0 || (2 * epi.hidden) % 256 == 0); }
-  static double cost(const GemmArgs& g, const Epi& epi, int batch) {
-    return std::min(cost192(g, epi, batch), fits256(g, epi) ? tile_cost(kTile256, g.m, g.n, batch) : 1e300);
+  static double us256(const GemmArgs& g, const Epi& epi) {
+    if (g.n % 256 != 0 || (epi.v_pitch > 0 && (2 * epi.hidden) % 256 != 0)) return 1e300;
+    return 1.03 * w4_us(256, g.m, g.n / 256, g.k / (kRowBytes / (int)sizeof(T)));
   }
-  static bool wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned) {
-    if (!epi.vec || !w4_eligible<T>(g, batch, aligned)) return false;
+  static bool eligible(const GemmArgs& g, const Epi& epi) {
+    if (!epi.vec || !w4_eligible<T>(g, 1, true)) return false;
     // eight rows of a transposed V lie in at most two sequences: what the kernel's element-wise store assumes
     // (and steps from one sequence to the next with a 32-bit element offset)
-    if (epi.v_pitch > 0 && (epi.seq < 8 || (int64_t)epi.hidden * epi.v_pitch >= (1ll << 31))) return false;
-    const int force = kernel_switch(kSwitchLargeTile);
-    if (force == 0) return false;
-    if (force == 1) return true;
-    double other = 0;
-    (void)pick_tile(g.m, g.n, batch, &other);
-    return cost(g, epi, batch) < other;
+    return epi.v_pitch == 0 || (epi.seq >= 8 && (int64_t)epi.hidden * epi.v_pitch < (1ll << 31));
   }
+  static double us(const GemmArgs& g, const Epi& epi) { return std::min(us192(g, epi), us256(g, epi)); }
   // Q, K (and a row-major V) leave straight from the accumulator layout when every 16-row block lies in one sequence and
   // every 32-column group in one head, and a destination tensor stays below 2 GiB (32-bit buffer offsets).
   static bool direct_ok(const GemmArgs& g, const Epi& epi) {
@@ -1123,7 +1119,7 @@ struct LargeTileKernel<T, EpiQkvSplit<T, false>, typename std::enable_if<sizeof(
   }
   static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) {
     const bool direct = direct_ok(g, epi);
-    if (fits256(g, epi) && tile_cost(kTile256, g.m, g.n, 1) < cost192(g, epi, 1))
+    if (us256(g, epi) < us192(g, epi))
       return direct ? launch_w4<T, 256, Epi, 2, true>(g, epi, s) : launch_w4<T, 256>(g, epi, s);
     const int split_col = split_run(g, epi) ? 2 * epi.hidden : 0;
     return direct ? launch_w4<T, 192, Epi, 2, true>(g, epi, s, split_col) : launch_w4<T, 192>(g, epi, s, split_col);
@@ -1133,7 +1129,8 @@ struct LargeTileKernel<T, EpiQkvSplit<T, false>, typename std::enable_if<sizeof(
 template <typename T>
 struct LargeTileKernel<T, EpiF32<T>, typename std::enable_if<sizeof(T) == 2>::type> {
   using Epi = EpiF32<T>;
-  static bool wanted(const GemmArgs& g, const Epi& epi, int batch, bool aligned) { return w4_wanted<T>(g, epi, batch, aligned); }
+  static bool eligible(const GemmArgs& g, const Epi& epi) { return epi.vec && w4_eligible<T>(g, 1, true); }
+  static double us(const GemmArgs& g, const Epi&) { return w4_linear_us<T>(g); }
   static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) {
     if (tile_cost(kW4Tile256, g.m, g.n, 1) < tile_cost(kW4Tile192, g.m, g.n, 1)) return launch_w4<T, 256>(g, epi, s);
     return launch_w4<T, 192>(g, epi, s);
