@@ -127,6 +127,15 @@ struct RingDest<EpiDequantQkvSplit> {
   static __device__ __forceinline__ float finish(const EpiDequantQkvSplit&, int x) { return __builtin_bit_cast(float, x); }
 };
 
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(const F& f, std::integer_sequence<int, I...>) {
+  (f(template_int<I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(const F& f) {  // f(0), ..., f(N - 1) with compile-time arguments
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
 template <int BM, int BN, int NS>
 constexpr int ring_lds_bytes() { return NS * (BM + BN) * kRowBytes; }
 
@@ -222,27 +231,43 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
   Acc acc[RB][CB];
   constexpr int READS = RB + CB, BLOCKS = RB * CB, MMAS = BLOCKS * MB::PARTS;
   constexpr int RPM = (READS + MMAS - 1) / MMAS;  // reads per matrix instruction
+  // Fragment reads are written as instructions: in front of an LDS read that it knows of, the compiler waits for EVERY
+  // global -> LDS load in flight (vmcnt(0) in each half step), which empties the ring.  They are ordered by hand: behind a
+  // barrier that their stage has passed, and landed() before the first use names every register they wrote.
+  auto read_a = [&](Chunk& dst, uint32_t at, auto i) __attribute__((always_inline)) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(reinterpret_cast<Quad&>(dst)) : "v"(at), "n"(decltype(i)::value * 16 * kRowBytes) : "memory");
+  };
+  const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>(smem);  // low half of a generic LDS address = LDS offset
+  auto landed = [&](Chunk (&a)[RB], Chunk (&b)[CB]) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < RB; ++i) asm volatile("" : "+v"(reinterpret_cast<Quad&>(a[i])));
+#pragma unroll
+    for (int j = 0; j < CB; ++j) asm volatile("" : "+v"(reinterpret_cast<Quad&>(b[j])));
+  };
   // LO, NL: the loads of the cursor's step issued here, evenly spread over the matrix instructions
   auto substep = [&](auto swap_tag, auto cur_tag, auto sub_tag, auto lo_tag, auto nl_tag, int rd) __attribute__((always_inline)) {
     constexpr bool SWAP = decltype(swap_tag)::value;
     constexpr int CUR = decltype(cur_tag)::value, SUB = decltype(sub_tag)::value, LO = decltype(lo_tag)::value, NL = decltype(nl_tag)::value;
-    const int off = ((SUB * 4 + lgrp) ^ swz) << 4;
-    const int a_at = a_row0 + off + rd, b_at = b_row0 + off + rd;
-#pragma unroll
-    for (int m = 0; m < MMAS; ++m) {
-      const int part = m / BLOCKS, blk = m % BLOCKS, i = blk / CB, j = blk % CB;  // (a block's parts apart: they form a chain)
+    const uint32_t off = (uint32_t)(((SUB * 4 + lgrp) ^ swz) << 4) + (uint32_t)rd + lds_base;
+    const uint32_t a_at = a_row0 + off, b_at = b_row0 + off;
+    static_for<MMAS>([&](auto m_tag) __attribute__((always_inline)) {
+      constexpr int m = decltype(m_tag)::value;
+      constexpr int part = m / BLOCKS, blk = m % BLOCKS, i = blk / CB, j = blk % CB;  // (a block's parts apart: they form a chain)
       if constexpr (SWAP) MB::run(fb[CUR][j], fa[CUR][i], acc[i][j], part);
       else MB::run(fa[CUR][i], fb[CUR][j], acc[i][j], part);
       // the fragments of the next half step, read as early as one per instruction allows
-#pragma unroll
-      for (int r = m * RPM; r < (m + 1) * RPM && r < READS; ++r) {
-        if (r < RB) fa[CUR ^ 1][r] = *reinterpret_cast<const Chunk*>(smem + a_at + r * 16 * kRowBytes);
-        else fb[CUR ^ 1][r - RB] = *reinterpret_cast<const Chunk*>(smem + b_at + (r - RB) * 16 * kRowBytes);
-      }
+      static_for<RPM>([&](auto r_tag) __attribute__((always_inline)) {
+        constexpr int r = m * RPM + decltype(r_tag)::value;
+        if constexpr (r < RB) read_a(fa[CUR ^ 1][r], a_at, template_int<r>{});
+        else if constexpr (r < READS) read_a(fb[CUR ^ 1][r - RB], b_at, template_int<r - RB>{});
+      });
 #pragma unroll
       for (int l = m * NL / MMAS; l < (m + 1) * NL / MMAS; ++l) issue_one(LO + l);
       __builtin_amdgcn_sched_barrier(0);
-    }
+    });
+    landed(fa[CUR ^ 1], fb[CUR ^ 1]);
+    __builtin_amdgcn_sched_barrier(0);
   };
 
   // ---- prologue: NS - 1 steps and the first part of one more are requested, the first step has landed
@@ -271,11 +296,10 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
   asm volatile("s_nop 7");  // (the matrix instructions are inline asm: no hazard is seen between them and the zeroing)
   dma_landed_barrier_but<(NS - 2) * LOADS + L1>();
   {
-    const int off = (lgrp ^ swz) << 4;
-#pragma unroll
-    for (int i = 0; i < RB; ++i) fa[0][i] = *reinterpret_cast<const Chunk*>(smem + (a_row0 + off) + i * 16 * kRowBytes);
-#pragma unroll
-    for (int j = 0; j < CB; ++j) fb[0][j] = *reinterpret_cast<const Chunk*>(smem + (b_row0 + off) + j * 16 * kRowBytes);
+    const uint32_t off = (uint32_t)((lgrp ^ swz) << 4) + lds_base;
+    static_for<RB>([&](auto i) __attribute__((always_inline)) { read_a(fa[0][decltype(i)::value], a_row0 + off, i); });
+    static_for<CB>([&](auto j) __attribute__((always_inline)) { read_a(fb[0][decltype(j)::value], b_row0 + off, j); });
+    landed(fa[0], fb[0]);
   }
   auto k_loop = [&](auto swap_tag) __attribute__((always_inline)) {
     int rd = 0;
@@ -448,12 +472,13 @@ struct RingTile {
   X(128, 192, 4, 2, 3, 1, 4.88f, 6.69f, 0.464f, 0.461f)      \
   X(256, 128, 4, 2, 3, 1, 5.36f, 8.33f, 0.576f, 0.571f)
 #define TTMI_RING_TILES_32(X)                                \
-  X(32, 64, 2, 2, 3, 4, 1.58f, 0.66f, 0.727f, 0.257f)        \
-  X(64, 64, 4, 2, 4, 2, 5.87f, 0.00f, 0.289f, 0.540f)        \
-  X(64, 64, 2, 2, 3, 3, 10.1f, 0.00f, 0.350f, 0.509f)        \
-  X(64, 96, 4, 1, 3, 2, 9.93f, 0.00f, 0.170f, 0.777f)        \
-  X(64, 128, 4, 2, 3, 2, 4.34f, 0.00f, 0.281f, 0.957f)       \
-  X(128, 192, 4, 2, 3, 1, 7.27f, 7.53f, 2.620f, 2.619f)
+  X(32, 64, 2, 2, 4, 3, 3.40f, 0.11f, 0.215f, 0.263f)        \
+  X(64, 64, 2, 2, 3, 3, 3.83f, 0.22f, 0.332f, 0.499f)        \
+  X(64, 64, 4, 2, 4, 2, 4.58f, 0.82f, 0.126f, 0.480f)        \
+  X(64, 96, 4, 1, 3, 2, 4.90f, 1.32f, 0.680f, 0.671f)        \
+  X(64, 128, 4, 2, 3, 2, 5.03f, 0.97f, 0.272f, 0.907f)       \
+  X(64, 192, 4, 2, 3, 1, 4.43f, 7.73f, 1.399f, 1.392f)       \
+  X(128, 192, 4, 2, 3, 1, 6.53f, 10.7f, 2.684f, 2.683f)
 #define TTMI_RING_TILES_8(X)                                 \
   X(32, 64, 2, 2, 4, 3, 3.55f, 0.74f, 0.141f, 0.120f)        \
   X(64, 64, 4, 2, 4, 2, 4.06f, 1.59f, 0.173f, 0.173f)        \
