@@ -61,7 +61,9 @@ TTMI_API const char* ttmi_last_error(void);
  * knob).  Names and values:
  *   "TTMI_LARGE_TILE"       1 = every eligible 16-bit product on the one-wavefront-per-SIMD GEMM kernel, 0 = none;
  *   "TTMI_WAVE_KERNEL"      0 = products of at most 128 rows stay on the LDS-tiled kernels;
- *   "TTMI_ATTENTION_WAVES"  4 / 8 = wavefronts per workgroup of the one-kernel attention;
+ *   "TTMI_ATTENTION_WAVES"  4 / 8 = wavefronts per workgroup of the one-kernel attention; 1 = its form whose
+ *                           wavefronts share the keys of a head, where that form exists (dense 16-bit batches with V
+ *                           transposed; fp32);
  *   "TTMI_STATIC_SCRATCH_LIMIT"  bytes of its buffer ttmi_gemm_bias_layer_norm_static admits (to test its refusal);
  *   "TTMI_W4_A_STAGES"      2 = the one-wavefront-per-SIMD GEMM kernel keeps two LDS stages for the A operand
  *                           where it would take three;

@@ -805,6 +805,29 @@ def test_fused_attention_fp32_vs_unfused_oracle(ttmi, oracle, attention_waves, B
     assert float(slots.max()) == float(out.abs().max())
 
 
+@pytest.mark.parametrize("dt,v_transposed", [("f16", True), ("bf16", True), ("f32", True), ("f32", False)])
+@pytest.mark.parametrize("S", [1, 31, 33, 129, 256, 257, 545])
+def test_attention_with_split_keys(ttmi, oracle, dt, v_transposed, S):
+    """The form whose wavefronts share the keys of a head (forced): fewer blocks of keys than wavefronts, the change from four
+    to eight of them past 256 keys, ragged last blocks with NaN in the pad columns of V^T."""
+    rng = np.random.default_rng(S)
+    B, h, d = 2, 2, 64
+    Q, K, V = (rng.standard_normal((B, h, S, d), np.float32) for _ in range(3))
+    mask = np.zeros((B, 1, 1, S), np.float32)
+    mask[0, ..., S // 2 + 1:] = -10000.0
+    dV, pitch = _v_operand(V, dt, v_transposed)
+    out = torch.full((B, S, h * d), 9.0, dtype=dV.dtype, device="cuda")
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", 1))
+    try:
+        ok(ttmi.ttmi_fused_attention(ptr(dev(Q, dt)), ptr(dev(K, dt)), ptr(dV), ptr(dev(mask)), ptr(out), None, B, h, S, d, pitch,
+                                     0.125, TTMI_DTYPES[dt], stream()))
+    finally:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+    prob = oracle.apply_mask_and_softmax(oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125), mask, 1.0, True)
+    want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, S, h * d)
+    assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
+
+
 def test_fused_attention_absmax_reports_no_slots_where_it_leaves_none(ttmi):
     """16-bit types, packed batches and launches with more workgroups than slots: the output as always, 0 slots
     reported, the slots untouched."""

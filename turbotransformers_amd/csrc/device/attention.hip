@@ -366,6 +366,11 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
                         int64_t batch, int64_t heads, int64_t seq, int64_t v_seq_pitch, float scale, int nw, float* absmax,
                         hipStream_t s);
 
+// attention_split.hip: the keys of a head split over the wavefronts of a workgroup
+bool split_attention_takes(int dtype, bool packed, bool v_transposed);
+int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch,
+                    int64_t heads, int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s);
+
 // absmax / slots_written: see ttmi_fused_attention_absmax; both null for the plain entry point
 static int fused_attention_impl(const void* q, const void* k, const void* v, const float* mask, void* out,
                                 const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
@@ -393,9 +398,25 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }();
   const bool fits_four = seq <= 128 || 8 * ceil_div(seq, 256) >= 5 * ceil_div(seq, 128);
   int nw = (fits_four || ceil_div(seq, 128) * batch * heads < (int64_t)cus) ? 4 : 8;
-  // TTMI_ATTENTION_WAVES=4 / 8 overrides the choice (A/B timing, and tests of the eight-wavefront form on small shapes)
+  // TTMI_ATTENTION_WAVES=4 / 8 (1: keys split over the wavefronts) overrides the choice (A/B timing, and tests of one form
+  // on the shapes of another)
   const int force = kernel_switch(kSwitchAttentionWaves);
   if (force == 4 || force == 8) nw = force;
+  // Few sequences: a workgroup per 32 queries, its wavefronts sharing the keys (attention_split.hip).  It re-reads K and V
+  // per 32 queries, so it wins while its workgroups fit the CUs at once: 16-bit, us split / four wavefronts, 12 heads:
+  // 1 x 128: 4.3 / 4.7, 1 x 387: 7.0 / 10.6, 4 x 128 (192 workgroups): 4.5 / 4.8, 8 x 128 (384): 6.5 / 5.0; one tile of
+  // keys is a draw.  fp32 is bound by the matrix pipes and gains further on: 1 x 128: 6.3 / 12.7, 2 x 512 (384): 32 / 42,
+  // 8 x 128 (384): 12.3 / 13.4, 16 x 128 (768): 18.8 / 13.9; and always below 33 keys, where a tile of 64 is half padding.
+  const int64_t split_wgs = ceil_div(seq, 32) * batch * heads;
+  const bool split_wins = dtype == TTMI_F32 ? 2 * split_wgs <= 3 * (int64_t)cus || seq <= 32 : seq > 64 && split_wgs <= (int64_t)cus;
+  const bool split = force == 1 || (force != 4 && force != 8 && split_wins);
+  if (split && split_attention_takes(dtype, cu_seqlens != nullptr, v_seq_pitch > 0)) {
+    const bool leave_maxima = absmax != nullptr && cu_seqlens == nullptr && split_wgs <= TTMI_ABSMAX_SLOTS;
+    const int rc = split_attention(q, k, v, mask, out, cu_seqlens, batch, heads, seq, v_seq_pitch, scale, dtype,
+                                   leave_maxima ? absmax : nullptr, (hipStream_t)stream);
+    if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
+    return rc;
+  }
   const dim3 grid((unsigned)ceil_div(seq, nw * 32), (unsigned)(batch * heads));
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;

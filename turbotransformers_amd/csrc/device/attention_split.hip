@@ -1,0 +1,335 @@
+// Fused self-attention for head_dim 64 where there are few sequences: the keys of a head are split over the wavefronts of a
+// workgroup.  Same formulas and matrix instructions as attention.hip (fp16 / bf16) and attention_f32.hip, which describe
+// them; what differs is the split of the work.
+//
+// Those kernels give a wavefront 32 queries and ALL keys of the head, staged through LDS and shared by the four or eight
+// wavefronts of the workgroup: the fewest bytes per query, but one sequence of 128 tokens is then 12 workgroups on 256 CUs,
+// each a serial chain of key tiles (fp32: 13.7 us, of which the matrix pipes need 0.4).  Here a workgroup owns 32 queries,
+// its NW wavefronts take every NW-th block of 32 keys, and each keeps its own running maximum, sum and output block; K and
+// V fragments come straight from global memory in the layout of the matrix instruction (a 16-byte piece of a K row or of a
+// V^T row per lane; fp32 with V row-major: one float per lane, 32 lanes on one row), the next block's while this one is
+// multiplied, so the K loop has neither LDS nor barriers.  At the end the NW partial results meet in LDS and are combined
+// with the weights 2^(m_w - max m).
+// One sequence, 12 heads, us per launch before / after: fp16 387 tokens 10.6 / 7.0, fp32 128 tokens 12.7 / 6.3 (1.5 of each
+// is the launch, 1 the first loads; fp32 then runs 64 matrix instructions of 64 cycles in a chain per block of keys).
+#include <type_traits>
+
+#include "common.h"
+
+namespace ttmi {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
+
+constexpr int kD = 64;            // head dim
+constexpr int kQ = 32, kKeys = 32;  // queries per workgroup, keys per block
+constexpr float kNegBig = -1.0e30f;
+
+// D = A B + C over one 16-byte piece of both operands
+template <typename T>
+__device__ __forceinline__ floatx16 mma(const u32x4& a, const u32x4& b, floatx16 c) {
+  if constexpr (std::is_same<T, f16>::value) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  } else if constexpr (std::is_same<T, bf16>::value) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[j]), __builtin_bit_cast(float, (uint32_t)b[j]), c, 0, 0, 0);
+    return c;
+  }
+}
+
+// Two probabilities rounded to T, and acc + both of them as rounded (the values the second product consumes).
+template <typename T>
+__device__ __forceinline__ uint32_t pack_probabilities(float lo, float hi, float& sum) {
+  if constexpr (std::is_same<T, f16>::value) {
+    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, halfx2));
+    sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(halfx2, p), halfx2{(_Float16)1.0f, (_Float16)1.0f}, sum, false);
+    return p;
+  } else {
+    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
+    sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), bf16x2{(__bf16)1.0f, (__bf16)1.0f}, sum, false);
+    return p;
+  }
+}
+
+// VT: V is [B,h,d,v_pitch]; otherwise [B,h,S,d] (fp32 only).  PACKED: q,k,v padded to seq, lengths and output rows from cu.
+template <typename T, bool VT, bool PACKED, int NW>
+__global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
+                                                                  const T* __restrict__ v, const float* __restrict__ mask,
+                                                                  T* __restrict__ out, const int32_t* __restrict__ cu, int heads,
+                                                                  int seq, int v_pitch, float scale_log2e, float inv_scale,
+                                                                  float* __restrict__ absmax) {
+  static_assert(VT || sizeof(T) == 4, "row-major V: fp32");
+  constexpr int KPC = 16 / (int)sizeof(T);   // elements per 16-byte piece
+  constexpr int PIECES = kD / KPC / 2;       // pieces of a row per lane: 4 (16-bit), 8 (fp32)
+  constexpr int VPIECES = 4 * (int)sizeof(T) / 2;  // pieces of V per lane and block: two halves of d, 32 keys
+  constexpr int PITCH = kD + 4;
+  __shared__ __align__(16) float part[NW][kQ][PITCH];
+  __shared__ float stat[2][NW][kQ];  // m and l of every wavefront's share
+  __shared__ float red[NW];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  const int bh = blockIdx.y, b = bh / heads, head = bh - b * heads;
+  const int q0 = blockIdx.x * kQ;
+  int kv_len = seq, out_row0 = b * seq;
+  if (PACKED) {
+    kv_len = cu[b + 1] - cu[b];
+    out_row0 = cu[b];
+    if (q0 >= kv_len) return;  // whole workgroup is padding
+  }
+  const T* qb = q + (int64_t)bh * seq * kD;
+  const T* kb = k + (int64_t)bh * seq * kD;
+  const T* vb = v + (int64_t)bh * kD * (VT ? v_pitch : seq);
+  const float* mb = mask != nullptr ? mask + (int64_t)b * seq : nullptr;
+
+  u32x4 qf[PIECES];
+  {
+    const T* row = qb + (int64_t)min(q0 + lrow, kv_len - 1) * kD + lhalf * KPC;  // rows past the end repeat the last one
+#pragma unroll
+    for (int kk = 0; kk < PIECES; ++kk) qf[kk] = *reinterpret_cast<const u32x4*>(row + 2 * kk * KPC);
+  }
+
+  struct Block {
+    u32x4 kf[PIECES];
+    u32x4 vf[VPIECES];
+    float mk;  // of key lrow
+  };
+  const int blocks = (kv_len + kKeys - 1) / kKeys;
+  // Keys past the end repeat valid ones; they carry a mask of -1e30, so their probability is 0.
+  auto load = [&](int blk, Block& x) __attribute__((always_inline)) {
+    const int key0 = blk * kKeys;
+    const T* row = kb + (int64_t)min(key0 + lrow, kv_len - 1) * kD + lhalf * KPC;
+#pragma unroll
+    for (int kk = 0; kk < PIECES; ++kk) x.kf[kk] = *reinterpret_cast<const u32x4*>(row + 2 * kk * KPC);
+    x.mk = mb != nullptr ? mb[min(key0 + lrow, kv_len - 1)] : 0.f;
+    if constexpr (sizeof(T) == 2) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          const T* vr = vb + (int64_t)(t * 32 + lrow) * v_pitch;
+          const int c = key0 + 16 * kk + 4 * lhalf;
+          const u32x2 lo = *reinterpret_cast<const u32x2*>(vr + min(c, v_pitch - 4)), hi = *reinterpret_cast<const u32x2*>(vr + min(c + 8, v_pitch - 4));
+          x.vf[2 * t + kk] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+    } else if constexpr (VT) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          x.vf[4 * t + g] = *reinterpret_cast<const u32x4*>(vb + (int64_t)(t * 32 + lrow) * v_pitch + min(key0 + 8 * g + 4 * lhalf, v_pitch - 4));
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const T* vr = vb + (int64_t)min(key0 + 8 * g + 4 * lhalf + i, kv_len - 1) * kD + lrow;
+#pragma unroll
+          for (int t = 0; t < 2; ++t) x.vf[4 * t + g][i] = __builtin_bit_cast(uint32_t, (float)vr[t * 32]);
+        }
+    }
+  };
+
+  floatx16 ot[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) ot[t][e] = 0.f;
+  float m_run = kNegBig, l_run = 0.f;
+
+  auto compute = [&](int blk, Block& x) __attribute__((always_inline)) {
+    const int key0 = blk * kKeys;
+    const bool ragged = key0 + kKeys > kv_len;  // uniform
+    // scores start from mask / scale of their key: [mask | 0] . [1 | 1], exact in fp32
+    floatx16 st;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) st[e] = 0.f;
+    {
+      const float mk = key0 + lrow < kv_len ? x.mk * inv_scale : kNegBig;
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(lhalf == 0 ? mk : 0.f, 1.f, st, 0, 0, 0);
+    }
+    if (VT && ragged) {  // V^T past the last key may hold anything: 0 * NaN would reach the output
+#pragma unroll
+      for (int p = 0; p < VPIECES; ++p)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          if constexpr (sizeof(T) == 2) {
+            const int key = key0 + 16 * (p & 1) + 8 * (w >> 1) + 4 * lhalf + 2 * (w & 1);
+            if (key >= kv_len) x.vf[p][w] = 0u;
+            else if (key + 1 >= kv_len) x.vf[p][w] &= 0xffffu;
+          } else {
+            if (key0 + 8 * (p & 3) + 4 * lhalf + w >= kv_len) x.vf[p][w] = 0u;
+          }
+        }
+    }
+#pragma unroll
+    for (int kk = 0; kk < PIECES; ++kk) st = mma<T>(x.kf[kk], qf[kk], st);
+    float mx = st[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
+      mx = fmaxf(__builtin_bit_cast(float, sw[0]), __builtin_bit_cast(float, sw[1]));
+    }
+    const float m_new = fmaxf(m_run, mx);
+    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
+    const float neg_m = -m_run * scale_log2e;
+    float psum = 0.f;
+    if constexpr (sizeof(T) == 2) {
+      u32x4 pf[2];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w], scale_log2e, neg_m));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w + 1], scale_log2e, neg_m));
+        pf[w >> 2][w & 3] = pack_probabilities<T>(p0, p1, psum);
+      }
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) ot[t] = mma<T>(x.vf[2 * t + kk], pf[kk], ot[t]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        st[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[e], scale_log2e, neg_m));
+        psum += st[e];
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        u32x4 pf;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pf[i] = __builtin_bit_cast(uint32_t, (float)st[4 * g + i]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) ot[t] = mma<T>(x.vf[4 * t + g], pf, ot[t]);
+      }
+    }
+    l_run = l_run * alpha + psum;
+  };
+
+  {
+    Block x, y;
+    int blk = wave;
+    if (blk < blocks) load(blk, x);
+    while (blk < blocks) {
+      if (blk + NW < blocks) load(blk + NW, y);
+      compute(blk, x);
+      blk += NW;
+      if (blk >= blocks) break;
+      if (blk + NW < blocks) load(blk + NW, x);
+      compute(blk, y);
+      blk += NW;
+    }
+  }
+
+  // ---- the wavefronts' shares meet: ot[t][4g+i] = O[query lrow][d = 32t + 8g + 4*lhalf + i]
+  l_run += __shfl_xor(l_run, 32, kWave);
+  if (lhalf == 0) {
+    stat[0][wave][lrow] = m_run;
+    stat[1][wave][lrow] = l_run;
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<floatx4*>(&part[wave][lrow][t * 32 + 8 * g + 4 * lhalf]) =
+          floatx4{ot[t][4 * g], ot[t][4 * g + 1], ot[t][4 * g + 2], ot[t][4 * g + 3]};
+  __syncthreads();
+  constexpr int EPT = kQ * kD / (NW * 64);  // output elements per thread: 8 or 4
+  const int qi = tid / (kD / EPT), d0 = (tid % (kD / EPT)) * EPT;
+  float m = kNegBig;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m = fmaxf(m, stat[0][w][qi]);
+  float l = 0.f, o[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) o[e] = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    const float f = __builtin_amdgcn_exp2f((stat[0][w][qi] - m) * scale_log2e);  // a share without keys: 2^-huge = 0
+    l += f * stat[1][w][qi];
+#pragma unroll
+    for (int e = 0; e < EPT; e += 4) {
+      const floatx4 p = *reinterpret_cast<const floatx4*>(&part[w][qi][d0 + e]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[e + j] += f * p[j];
+    }
+  }
+  const float inv = 1.0f / l;
+  float amax = 0.f;
+  if (q0 + qi < kv_len) {
+    T* dst = out + ((int64_t)out_row0 + q0 + qi) * (heads * kD) + head * kD + d0;
+    Vec<T, EPT> r;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+      const float x = o[e] * inv;
+      r.v[e] = from_float<T>(x);
+      amax = fmaxf(amax, fabsf(x));
+    }
+    if constexpr (sizeof(Vec<T, EPT>) <= 16) {
+      store_vec<T, EPT>(dst, r);
+    } else {
+#pragma unroll
+      for (int e = 0; e < EPT; e += 4) *reinterpret_cast<floatx4*>(dst + e) = floatx4{(float)r.v[e], (float)r.v[e + 1], (float)r.v[e + 2], (float)r.v[e + 3]};
+    }
+  }
+  // Optional (dense fp32 batches): max|out| of this workgroup to its slot, as in attention_f32.hip.
+  if (absmax != nullptr) {
+    amax = group_max<kWave>(amax);
+    if (lane == 0) red[wave] = amax;
+    __syncthreads();
+    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), wgs = (int)(gridDim.x * gridDim.y);
+    if (tid == 0) {
+      float mx = red[0];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) mx = fmaxf(mx, red[w]);
+      absmax[wg] = mx;
+    }
+    if (wg == 0)
+      for (int i = wgs + tid; i < TTMI_ABSMAX_SLOTS; i += NW * 64) absmax[i] = 0.f;
+  }
+}
+
+template <typename T, bool VT, bool PACKED>
+int launch(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch, int64_t heads,
+           int64_t seq, int64_t v_pitch, float scale, float* absmax, hipStream_t s) {
+  const dim3 grid((unsigned)ceil_div(seq, kQ), (unsigned)(batch * heads));
+  const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
+  // eight wavefronts where four would each have more than two blocks of keys
+#define TTMI_SPLIT_ATTENTION(NW)                                                                                              \
+  hipLaunchKernelGGL((split_attention_kernel<T, VT, PACKED, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
+                     mask, (T*)out, cu, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax)
+  if (seq > 4 * 2 * kKeys) TTMI_SPLIT_ATTENTION(8);
+  else TTMI_SPLIT_ATTENTION(4);
+#undef TTMI_SPLIT_ATTENTION
+  return launch_status("split_attention_kernel");
+}
+
+}  // namespace
+
+bool split_attention_takes(int dtype, bool packed, bool v_transposed) { return dtype == TTMI_F32 ? !(packed && v_transposed) : v_transposed && !packed; }
+
+// Arguments were checked by ttmi_fused_attention; absmax needs seq / 32 * batch * heads workgroups to fit the slots.
+int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch,
+                    int64_t heads, int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s) {
+  if (dtype == TTMI_F16) return launch<f16, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, nullptr, s);
+  if (dtype == TTMI_BF16) return launch<bf16, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, nullptr, s);
+  if (v_pitch > 0) return launch<float, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
+  if (cu != nullptr) return launch<float, false, true>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
+  return launch<float, false, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
+}
+
+}  // namespace ttmi
