@@ -62,8 +62,7 @@ TTMI_API const char* ttmi_last_error(void);
  *   "TTMI_LARGE_TILE"       1 = every eligible 16-bit product on the one-wavefront-per-SIMD GEMM kernel, 0 = none;
  *   "TTMI_WAVE_KERNEL"      0 = products of at most 128 rows stay on the LDS-tiled kernels;
  *   "TTMI_ATTENTION_WAVES"  4 / 8 = wavefronts per workgroup of the one-kernel attention; 1 = its form whose
- *                           wavefronts share the keys of a head, where that form exists (dense 16-bit batches with V
- *                           transposed; fp32);
+ *                           wavefronts share the keys of a head, where that form exists (dense batches with V transposed);
  *   "TTMI_STATIC_SCRATCH_LIMIT"  bytes of its buffer ttmi_gemm_bias_layer_norm_static admits (to test its refusal);
  *   "TTMI_W4_A_STAGES"      2 = the one-wavefront-per-SIMD GEMM kernel keeps two LDS stages for the A operand
  *                           where it would take three;
@@ -118,6 +117,10 @@ TTMI_API int ttmi_check_async(void);
  * In place on out[m,n]: mean = sum/n, var = sumsq/n - mean^2, out = beta + gamma*(x-mean)/sqrt(var+eps). */
 TTMI_API int ttmi_layer_norm(void* out, const void* gamma, const void* beta, int64_t m, int64_t n,
                              float eps, int dtype, void* stream);
+/* The same from `input` (which must not overlap `out`): the copy in front of a pre-LayerNorm
+ * (layers/multi_headed_attention.cpp:66-80) is not a pass of its own. */
+TTMI_API int ttmi_layer_norm_from(void* out, const void* input, const void* gamma, const void* beta, int64_t m, int64_t n,
+                                  float eps, int dtype, void* stream);
 
 /* kernels::AddBiasLayerNorm  (layers/kernels/layer_norm.cpp:99-180, CPU branch :130-164).
  * out = LN(out + input + bias), in place on out. */
@@ -327,6 +330,19 @@ TTMI_API int ttmi_gemm_batched_heads(const void* a, const void* b, void* c, int6
 TTMI_API int ttmi_fused_attention(const void* q, const void* k, const void* v, const float* mask, void* out,
                                   const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq,
                                   int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype, void* stream);
+
+/* Attention that returns its probabilities, for head_dim 64: P = softmax(scale * Q K^T + mask), out = P V with
+ * K = [k_past | k] and V = [v_past | v] along the sequence.  q is [B,h,F,64]; k_past, v_past [B,h,past,64] (NULL with
+ * past = 0), k, v [B,h,keys-past,64]; `mask` is an additive fp32 [B,keys], or [B,F,keys] with mask_per_query, or NULL;
+ * probs is [B,h,F,keys], out [B,F,h*64].  k_out, v_out (both or none, overlapping nothing else) receive the grown cache
+ * [B,h,keys,64].  Replaces the concatenation with the layer cache, the cache's copy and the four-kernel attention chain
+ * (layers/multi_headed_attention.cpp:205-229, :323-354).  keys <= TTMI_PROBS_MAX_KEYS; every tensor but probs and mask
+ * is 16-byte aligned. */
+#define TTMI_PROBS_MAX_KEYS 512
+TTMI_API int ttmi_attention_with_probs(const void* q, const void* k_past, const void* v_past, int64_t past, const void* k,
+                                       const void* v, void* k_out, void* v_out, const float* mask, int mask_per_query,
+                                       void* probs, void* out, int64_t batch, int64_t heads, int64_t queries, int64_t keys,
+                                       int64_t head_dim, float scale, int dtype, void* stream);
 
 /* Arguments of the fused epilogues; unused members are NULL / 0. */
 typedef struct ttmi_epilogue_args {

@@ -805,9 +805,9 @@ def test_fused_attention_fp32_vs_unfused_oracle(ttmi, oracle, attention_waves, B
     assert float(slots.max()) == float(out.abs().max())
 
 
-@pytest.mark.parametrize("dt,v_transposed", [("f16", True), ("bf16", True), ("f32", True), ("f32", False)])
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("S", [1, 31, 33, 129, 256, 257, 545])
-def test_attention_with_split_keys(ttmi, oracle, dt, v_transposed, S):
+def test_attention_with_split_keys(ttmi, oracle, dt, S):
     """The form whose wavefronts share the keys of a head (forced): fewer blocks of keys than wavefronts, the change from four
     to eight of them past 256 keys, ragged last blocks with NaN in the pad columns of V^T."""
     rng = np.random.default_rng(S)
@@ -815,7 +815,7 @@ def test_attention_with_split_keys(ttmi, oracle, dt, v_transposed, S):
     Q, K, V = (rng.standard_normal((B, h, S, d), np.float32) for _ in range(3))
     mask = np.zeros((B, 1, 1, S), np.float32)
     mask[0, ..., S // 2 + 1:] = -10000.0
-    dV, pitch = _v_operand(V, dt, v_transposed)
+    dV, pitch = _v_operand(V, dt, True)
     out = torch.full((B, S, h * d), 9.0, dtype=dV.dtype, device="cuda")
     ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", 1))
     try:
@@ -825,6 +825,35 @@ def test_attention_with_split_keys(ttmi, oracle, dt, v_transposed, S):
         ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
     prob = oracle.apply_mask_and_softmax(oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125), mask, 1.0, True)
     want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, S, h * d)
+    assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("F,past,fresh,per_query", [(1, 0, 1, False), (33, 0, 33, True), (1, 40, 1, False), (1, 127, 1, True),
+                                                    (5, 124, 5, True), (64, 0, 256, False), (2, 255, 2, True), (31, 300, 212, False)])
+def test_attention_with_probs(ttmi, oracle, dt, F, past, fresh, per_query):
+    """Attention that returns its probabilities and grows the cache: [past | new] keys around the block of 32 and the limits
+    of its three forms (128, 256, 512 keys), masks per key and per query, against the oracle's chain."""
+    rng = np.random.default_rng(F + past + fresh)
+    B, h, d, T = 2, 3, 64, past + fresh
+    Q = rng.standard_normal((B, h, F, d), np.float32)
+    K, V = (rng.standard_normal((B, h, T, d), np.float32) for _ in range(2))
+    mask = np.where(rng.random((B, F if per_query else 1, T)) < 0.3, -1e18, 0.0).astype(np.float32)
+    mask[..., 0] = 0.0
+    dQ, dK, dV = dev(Q, dt), dev(K, dt), dev(V, dt)
+    split = lambda x: (x[:, :, :past].contiguous(), x[:, :, past:].contiguous())
+    (kp, kn), (vp, vn) = split(dK), split(dV)
+    probs = torch.full((B, h, F, T), 9.0, dtype=dQ.dtype, device="cuda")
+    out = torch.full((B, F, h * d), 9.0, dtype=dQ.dtype, device="cuda")
+    kg, vg = torch.zeros_like(dK), torch.zeros_like(dV)
+    ok(ttmi.ttmi_attention_with_probs(ptr(dQ), ptr(kp) if past else None, ptr(vp) if past else None, past, ptr(kn), ptr(vn), ptr(kg),
+                                      ptr(vg), ptr(dev(mask)), int(per_query), ptr(probs), ptr(out), B, h, F, T, d, 0.125,
+                                      TTMI_DTYPES[dt], stream()))
+    assert torch.equal(kg, dK) and torch.equal(vg, dV)
+    score = oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125)
+    prob = oracle.apply_mask_and_softmax(score, mask.reshape(B, 1, -1, T), 1.0, not per_query)
+    want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, F, h * d)
+    assert max_abs(host(probs), prob) <= (2e-6 if dt == "f32" else GEMM_TOL[dt])
     assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
 
 

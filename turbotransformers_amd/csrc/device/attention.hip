@@ -128,8 +128,8 @@ __device__ __forceinline__ void attention_tile(const char* kt, const char* vt, c
     {
       // the other half-wavefront holds the remaining 16 keys of this query: exchange through
       // v_permlane32_swap (two VALU instructions) instead of an LDS permute and its wait
-      const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
-      mx = fmaxf(__builtin_bit_cast(float, sw[0]), __builtin_bit_cast(float, sw[1]));
+      const LanePair sw = swap_halves(mx);
+      mx = fmaxf(sw.a, sw.b);
     }
     // Lazy running maximum: the reference point m_run only moves when some query of the
     // wavefront would otherwise see exp2 arguments above kSlack (fp16: probabilities up to 2^kSlack are
@@ -367,9 +367,8 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
                         hipStream_t s);
 
 // attention_split.hip: the keys of a head split over the wavefronts of a workgroup
-bool split_attention_takes(int dtype, bool packed, bool v_transposed);
-int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch,
-                    int64_t heads, int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s);
+int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s);
 
 // absmax / slots_written: see ttmi_fused_attention_absmax; both null for the plain entry point
 static int fused_attention_impl(const void* q, const void* k, const void* v, const float* mask, void* out,
@@ -407,12 +406,14 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   // 1 x 128: 4.3 / 4.7, 1 x 387: 7.0 / 10.6, 4 x 128 (192 workgroups): 4.5 / 4.8, 8 x 128 (384): 6.5 / 5.0; one tile of
   // keys is a draw.  fp32 is bound by the matrix pipes and gains further on: 1 x 128: 6.3 / 12.7, 2 x 512 (384): 32 / 42,
   // 8 x 128 (384): 12.3 / 13.4, 16 x 128 (768): 18.8 / 13.9; and always below 33 keys, where a tile of 64 is half padding.
+  // (Dense batches with V transposed.  The quantised layers, whose rounding to 8 bits turns sums in another order into
+  // whole steps, keep V row-major and with it the order of the other kernel.)
   const int64_t split_wgs = ceil_div(seq, 32) * batch * heads;
   const bool split_wins = dtype == TTMI_F32 ? 2 * split_wgs <= 3 * (int64_t)cus || seq <= 32 : seq > 64 && split_wgs <= (int64_t)cus;
   const bool split = force == 1 || (force != 4 && force != 8 && split_wins);
-  if (split && split_attention_takes(dtype, cu_seqlens != nullptr, v_seq_pitch > 0)) {
-    const bool leave_maxima = absmax != nullptr && cu_seqlens == nullptr && split_wgs <= TTMI_ABSMAX_SLOTS;
-    const int rc = split_attention(q, k, v, mask, out, cu_seqlens, batch, heads, seq, v_seq_pitch, scale, dtype,
+  if (split && cu_seqlens == nullptr && v_seq_pitch > 0) {
+    const bool leave_maxima = absmax != nullptr && dtype == TTMI_F32 && split_wgs <= TTMI_ABSMAX_SLOTS;
+    const int rc = split_attention(q, k, v, mask, out, batch, heads, seq, v_seq_pitch, scale, dtype,
                                    leave_maxima ? absmax : nullptr, (hipStream_t)stream);
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;

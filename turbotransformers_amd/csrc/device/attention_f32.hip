@@ -177,8 +177,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
       for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
       {
         // the other half-wavefront holds the remaining 16 keys of this query
-        const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
-        mx = fmaxf(__builtin_bit_cast(float, sw[0]), __builtin_bit_cast(float, sw[1]));
+        const LanePair sw = swap_halves(mx);
+        // Any reference point near the maximum does: the sums are rounded relative to their own size.  The half that holds
+        // the first keys gives it unless the other one's exponentials would leave the fp32 range (2^64 leaves 2^63 to sum).
+        mx = (sw.b - sw.a) * scale_log2e > 64.f ? sw.b : sw.a;
       }
       if (__any(mx > m_run)) {
         const float m_new = fmaxf(m_run, mx);

@@ -7,8 +7,7 @@
 // each a serial chain of key tiles (fp32: 13.7 us, of which the matrix pipes need 0.4).  Here a workgroup owns 32 queries,
 // its NW wavefronts take every NW-th block of 32 keys, and each keeps its own running maximum, sum and output block; K and
 // V fragments come straight from global memory in the layout of the matrix instruction (a 16-byte piece of a K row or of a
-// V^T row per lane; fp32 with V row-major: one float per lane, 32 lanes on one row), the next block's while this one is
-// multiplied, so the K loop has neither LDS nor barriers.  At the end the NW partial results meet in LDS and are combined
+// V^T row per lane), the next block's while this one is multiplied, so the K loop has neither LDS nor barriers.  At the end the NW partial results meet in LDS and are combined
 // with the weights 2^(m_w - max m).
 // One sequence, 12 heads, us per launch before / after: fp16 387 tokens 10.6 / 7.0, fp32 128 tokens 12.7 / 6.3 (1.5 of each
 // is the launch, 1 the first loads; fp32 then runs 64 matrix instructions of 64 cycles in a chain per block of keys).
@@ -62,14 +61,12 @@ __device__ __forceinline__ uint32_t pack_probabilities(float lo, float hi, float
   }
 }
 
-// VT: V is [B,h,d,v_pitch]; otherwise [B,h,S,d] (fp32 only).  PACKED: q,k,v padded to seq, lengths and output rows from cu.
-template <typename T, bool VT, bool PACKED, int NW>
+// V is [B,h,d,v_pitch]
+template <typename T, int NW>
 __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                   const T* __restrict__ v, const float* __restrict__ mask,
-                                                                  T* __restrict__ out, const int32_t* __restrict__ cu, int heads,
-                                                                  int seq, int v_pitch, float scale_log2e, float inv_scale,
+                                                                  T* __restrict__ out, int heads, int seq, int v_pitch, float scale_log2e, float inv_scale,
                                                                   float* __restrict__ absmax) {
-  static_assert(VT || sizeof(T) == 4, "row-major V: fp32");
   constexpr int KPC = 16 / (int)sizeof(T);   // elements per 16-byte piece
   constexpr int PIECES = kD / KPC / 2;       // pieces of a row per lane: 4 (16-bit), 8 (fp32)
   constexpr int VPIECES = 4 * (int)sizeof(T) / 2;  // pieces of V per lane and block: two halves of d, 32 keys
@@ -78,24 +75,18 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   __shared__ float stat[2][NW][kQ];  // m and l of every wavefront's share
   __shared__ float red[NW];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int bh = blockIdx.y, b = bh / heads, head = bh - b * heads;
   const int q0 = blockIdx.x * kQ;
-  int kv_len = seq, out_row0 = b * seq;
-  if (PACKED) {
-    kv_len = cu[b + 1] - cu[b];
-    out_row0 = cu[b];
-    if (q0 >= kv_len) return;  // whole workgroup is padding
-  }
   const T* qb = q + (int64_t)bh * seq * kD;
   const T* kb = k + (int64_t)bh * seq * kD;
-  const T* vb = v + (int64_t)bh * kD * (VT ? v_pitch : seq);
+  const T* vb = v + (int64_t)bh * kD * v_pitch;
   const float* mb = mask != nullptr ? mask + (int64_t)b * seq : nullptr;
 
   u32x4 qf[PIECES];
   {
-    const T* row = qb + (int64_t)min(q0 + lrow, kv_len - 1) * kD + lhalf * KPC;  // rows past the end repeat the last one
+    const T* row = qb + (int64_t)min(q0 + lrow, seq - 1) * kD + lhalf * KPC;  // rows past the end repeat the last one
 #pragma unroll
     for (int kk = 0; kk < PIECES; ++kk) qf[kk] = *reinterpret_cast<const u32x4*>(row + 2 * kk * KPC);
   }
@@ -105,14 +96,14 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     u32x4 vf[VPIECES];
     float mk;  // of key lrow
   };
-  const int blocks = (kv_len + kKeys - 1) / kKeys;
+  const int blocks = (seq + kKeys - 1) / kKeys;
   // Keys past the end repeat valid ones; they carry a mask of -1e30, so their probability is 0.
   auto load = [&](int blk, Block& x) __attribute__((always_inline)) {
     const int key0 = blk * kKeys;
-    const T* row = kb + (int64_t)min(key0 + lrow, kv_len - 1) * kD + lhalf * KPC;
+    const T* row = kb + (int64_t)min(key0 + lrow, seq - 1) * kD + lhalf * KPC;
 #pragma unroll
     for (int kk = 0; kk < PIECES; ++kk) x.kf[kk] = *reinterpret_cast<const u32x4*>(row + 2 * kk * KPC);
-    x.mk = mb != nullptr ? mb[min(key0 + lrow, kv_len - 1)] : 0.f;
+    x.mk = mb != nullptr ? mb[min(key0 + lrow, seq - 1)] : 0.f;
     if constexpr (sizeof(T) == 2) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -123,21 +114,12 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
           const u32x2 lo = *reinterpret_cast<const u32x2*>(vr + min(c, v_pitch - 4)), hi = *reinterpret_cast<const u32x2*>(vr + min(c + 8, v_pitch - 4));
           x.vf[2 * t + kk] = u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
-    } else if constexpr (VT) {
+    } else {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           x.vf[4 * t + g] = *reinterpret_cast<const u32x4*>(vb + (int64_t)(t * 32 + lrow) * v_pitch + min(key0 + 8 * g + 4 * lhalf, v_pitch - 4));
-    } else {
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const T* vr = vb + (int64_t)min(key0 + 8 * g + 4 * lhalf + i, kv_len - 1) * kD + lrow;
-#pragma unroll
-          for (int t = 0; t < 2; ++t) x.vf[4 * t + g][i] = __builtin_bit_cast(uint32_t, (float)vr[t * 32]);
-        }
     }
   };
 
@@ -150,26 +132,26 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 
   auto compute = [&](int blk, Block& x) __attribute__((always_inline)) {
     const int key0 = blk * kKeys;
-    const bool ragged = key0 + kKeys > kv_len;  // uniform
+    const bool ragged = key0 + kKeys > seq;  // uniform
     // scores start from mask / scale of their key: [mask | 0] . [1 | 1], exact in fp32
     floatx16 st;
 #pragma unroll
     for (int e = 0; e < 16; ++e) st[e] = 0.f;
     {
-      const float mk = key0 + lrow < kv_len ? x.mk * inv_scale : kNegBig;
+      const float mk = key0 + lrow < seq ? x.mk * inv_scale : kNegBig;
       st = __builtin_amdgcn_mfma_f32_32x32x2f32(lhalf == 0 ? mk : 0.f, 1.f, st, 0, 0, 0);
     }
-    if (VT && ragged) {  // V^T past the last key may hold anything: 0 * NaN would reach the output
+    if (ragged) {  // V^T past the last key may hold anything: 0 * NaN would reach the output
 #pragma unroll
       for (int p = 0; p < VPIECES; ++p)
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           if constexpr (sizeof(T) == 2) {
             const int key = key0 + 16 * (p & 1) + 8 * (w >> 1) + 4 * lhalf + 2 * (w & 1);
-            if (key >= kv_len) x.vf[p][w] = 0u;
-            else if (key + 1 >= kv_len) x.vf[p][w] &= 0xffffu;
+            if (key >= seq) x.vf[p][w] = 0u;
+            else if (key + 1 >= seq) x.vf[p][w] &= 0xffffu;
           } else {
-            if (key0 + 8 * (p & 3) + 4 * lhalf + w >= kv_len) x.vf[p][w] = 0u;
+            if (key0 + 8 * (p & 3) + 4 * lhalf + w >= seq) x.vf[p][w] = 0u;
           }
         }
     }
@@ -179,8 +161,8 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 #pragma unroll
     for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
     {
-      const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
-      mx = fmaxf(__builtin_bit_cast(float, sw[0]), __builtin_bit_cast(float, sw[1]));
+      const LanePair sw = swap_halves(mx);
+      mx = fmaxf(sw.a, sw.b);
     }
     const float m_new = fmaxf(m_run, mx);
     const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
@@ -270,8 +252,8 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   }
   const float inv = 1.0f / l;
   float amax = 0.f;
-  if (q0 + qi < kv_len) {
-    T* dst = out + ((int64_t)out_row0 + q0 + qi) * (heads * kD) + head * kD + d0;
+  if (q0 + qi < seq) {
+    T* dst = out + ((int64_t)b * seq + q0 + qi) * (heads * kD) + head * kD + d0;
     Vec<T, EPT> r;
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
@@ -303,15 +285,15 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   }
 }
 
-template <typename T, bool VT, bool PACKED>
-int launch(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch, int64_t heads,
+template <typename T>
+int launch(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
            int64_t seq, int64_t v_pitch, float scale, float* absmax, hipStream_t s) {
   const dim3 grid((unsigned)ceil_div(seq, kQ), (unsigned)(batch * heads));
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   // eight wavefronts where four would each have more than two blocks of keys
 #define TTMI_SPLIT_ATTENTION(NW)                                                                                              \
-  hipLaunchKernelGGL((split_attention_kernel<T, VT, PACKED, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
-                     mask, (T*)out, cu, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax)
+  hipLaunchKernelGGL((split_attention_kernel<T, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
+                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax)
   if (seq > 4 * 2 * kKeys) TTMI_SPLIT_ATTENTION(8);
   else TTMI_SPLIT_ATTENTION(4);
 #undef TTMI_SPLIT_ATTENTION
@@ -320,16 +302,12 @@ int launch(const void* q, const void* k, const void* v, const float* mask, void*
 
 }  // namespace
 
-bool split_attention_takes(int dtype, bool packed, bool v_transposed) { return dtype == TTMI_F32 ? !(packed && v_transposed) : v_transposed && !packed; }
-
-// Arguments were checked by ttmi_fused_attention; absmax needs seq / 32 * batch * heads workgroups to fit the slots.
-int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, const int32_t* cu, int64_t batch,
-                    int64_t heads, int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s) {
-  if (dtype == TTMI_F16) return launch<f16, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, nullptr, s);
-  if (dtype == TTMI_BF16) return launch<bf16, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, nullptr, s);
-  if (v_pitch > 0) return launch<float, true, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
-  if (cu != nullptr) return launch<float, false, true>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
-  return launch<float, false, false>(q, k, v, mask, out, cu, batch, heads, seq, v_pitch, scale, absmax, s);
+// Arguments were checked by ttmi_fused_attention; absmax (fp32) needs seq / 32 * batch * heads workgroups to fit the slots.
+int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s) {
+  if (dtype == TTMI_F16) return launch<f16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, s);
+  if (dtype == TTMI_BF16) return launch<bf16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, s);
+  return launch<float>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, absmax, s);
 }
 
 }  // namespace ttmi

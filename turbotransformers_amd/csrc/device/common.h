@@ -77,18 +77,56 @@ __device__ __forceinline__ void store_vec_unaligned(T* p, const Vec<T, N>& x) {
   reinterpret_cast<UnalignedVec<T, N>*>(p)->x = x;
 }
 
-// ---- wave64 reductions over groups of G lanes (G power of two <= 64) -------------------
-template <int G>
-__device__ __forceinline__ float group_sum(float v) {
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+// ---- wave64 reductions over groups of G lanes (G power of two, 4 <= G <= 64) ------------
+// Partners come through data-parallel-primitive moves and the row swaps, a few cycles each, where a __shfl_xor is a trip
+// through the LDS unit (~100 cycles, six in a chain: the larger part of a LayerNorm over a few rows).  The order is that
+// of the butterfly over G/2, ..., 2, 1: once lanes that differ by 16 and 8 agree, rotating a row of 16 by 4, 2 or 1 meets
+// the same values as the exclusive or.  (The quantised layers round what follows to 8 bits, so a sum in another order
+// would move their results by whole steps.)
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// A value of both half-wavefronts (both halves of every pair of 16-lane rows) in every lane.  The elements of the result are
+// copied before the bit cast: the compiler takes element 0 where it casts an element of a vector in place.
+struct LanePair {
+  float a, b;
+};
+__device__ __forceinline__ LanePair swap_halves(float v) {
+  const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a = sw[0], b = sw[1];
+  return {__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
+}
+__device__ __forceinline__ LanePair swap_rows(float v) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, v), false, false);
+  const unsigned a = sw[0], b = sw[1];
+  return {__builtin_bit_cast(float, a), __builtin_bit_cast(float, b)};
+}
+template <int G, typename Op>
+__device__ __forceinline__ float group_reduce(float v, Op op) {
+  static_assert(G == 4 || G == 8 || G == 16 || G == 32 || G == 64, "group of 4 to 64 lanes");
+  if constexpr (G >= 64) {
+    const LanePair p = swap_halves(v);
+    v = op(p.a, p.b);
+  }
+  if constexpr (G >= 32) {
+    const LanePair p = swap_rows(v);
+    v = op(p.a, p.b);
+  }
+  if constexpr (G >= 16) v = op(v, dpp_move<0x128>(v));  // row_ror:8
+  if constexpr (G >= 16) v = op(v, dpp_move<0x124>(v));  // row_ror:4
+  else if constexpr (G >= 8) v = op(v, __shfl_xor(v, 4, kWave));
+  v = op(v, dpp_move<0x4E>(v));  // quad_perm [2,3,0,1]
+  v = op(v, dpp_move<0xB1>(v));  // quad_perm [1,0,3,2]
   return v;
 }
 template <int G>
+__device__ __forceinline__ float group_sum(float v) {
+  return group_reduce<G>(v, [](float a, float b) { return a + b; });
+}
+template <int G>
 __device__ __forceinline__ float group_max(float v) {
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, kWave));
-  return v;
+  return group_reduce<G>(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // tanh-form GELU exactly as the reference states it, written through the logistic identity

@@ -1003,26 +1003,41 @@ __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const flo
   const int64_t mn = (int64_t)m * n;
   float x[ITERS][4];
   float sum = 0.f, sumsq = 0.f;
+  // A row is a few KB: the kernel is a chain of waits, so everything the row needs is requested before the first use
+  // (gamma and beta in front of the reduction, the slices four at a time).
+  Vec<T, 4> gm[ITERS], bt[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * 256 + threadIdx.x) * 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[it][j] = 0.f;
     if (col < n) {
+      const Vec<T, 4> b = load_vec<T, 4>(bias + col);
+      float4 r32;
+      Vec<T, 4> r16;
+      if (residual32 != nullptr) r32 = *reinterpret_cast<const float4*>(residual32 + (int64_t)row * n + col);
+      else r16 = load_vec<T, 4>(residual + (int64_t)row * n + col);
+      gm[it] = load_vec<T, 4>(gamma + col);
+      bt[it] = load_vec<T, 4>(beta + col);
       const float* p = ws + (int64_t)row * n + col;
-      for (int sidx = 0; sidx < splits; ++sidx) {
+      int sidx = 0;
+      for (; sidx + 4 <= splits; sidx += 4) {
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const float4*>(p + (sidx + u) * mn);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[it][0] += v[u].x, x[it][1] += v[u].y, x[it][2] += v[u].z, x[it][3] += v[u].w;
+      }
+      for (; sidx < splits; ++sidx) {
         const float4 v = *reinterpret_cast<const float4*>(p + sidx * mn);
         x[it][0] += v.x; x[it][1] += v.y; x[it][2] += v.z; x[it][3] += v.w;
       }
-      const Vec<T, 4> b = load_vec<T, 4>(bias + col);
       float r[4];
       if (residual32 != nullptr) {
-        const float4 v = *reinterpret_cast<const float4*>(residual32 + (int64_t)row * n + col);
-        r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
+        r[0] = r32.x; r[1] = r32.y; r[2] = r32.z; r[3] = r32.w;
       } else {
-        const Vec<T, 4> v = load_vec<T, 4>(residual + (int64_t)row * n + col);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r[j] = to_float(v.v[j]);
+        for (int j = 0; j < 4; ++j) r[j] = to_float(r16.v[j]);
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -1048,12 +1063,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const flo
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * 256 + threadIdx.x) * 4;
     if (col < n) {
-      const Vec<T, 4> gm = load_vec<T, 4>(gamma + col), bt = load_vec<T, 4>(beta + col);
       Vec<T, 4> o;
       float y[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        y[j] = to_float(bt.v[j]) + to_float(gm.v[j]) * rstd * (x[it][j] - mean);
+        y[j] = to_float(bt[it].v[j]) + to_float(gm[it].v[j]) * rstd * (x[it][j] - mean);
         o.v[j] = from_float<T>(y[j]);
       }
       store_vec<T, 4>(out + (int64_t)row * n + col, o);

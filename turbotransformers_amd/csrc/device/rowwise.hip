@@ -34,16 +34,21 @@ __global__ __launch_bounds__(kBlock) void layer_norm_rows(T* __restrict__ out, c
   const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / G;
   const bool row_ok = row < m;
   T* orow = out + row * n;
-  const T* irow = (ADD && !RES32) ? input + row * n : nullptr;
+  const T* irow = !RES32 && input != nullptr ? input + row * n : orow;  // without ADD: the source, null = in place
 
   float x[ITERS][VEC];
   float sum = 0.f, sumsq = 0.f;
+  // gamma and beta are requested with the row: behind the reduction their latency would come on top, which is a fifth of
+  // the kernel where a few rows leave nothing else to run meanwhile
+  Vec<T, VEC> g[ITERS], bt[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * G + lane) * VEC;
     if (row_ok && col < n) {
+      g[it] = load_vec<T, VEC>(gamma + col);
+      bt[it] = load_vec<T, VEC>(beta + col);
       Vec<T, VEC> o;
-      if (RES32 != 2) o = load_vec<T, VEC>(orow + col);
+      if (RES32 != 2) o = load_vec<T, VEC>((ADD ? orow : irow) + col);
       if (ADD && RES32 == 2) {
         Vec<T, VEC> b = load_vec<T, VEC>(bias + col);
 #pragma unroll
@@ -81,13 +86,11 @@ __global__ __launch_bounds__(kBlock) void layer_norm_rows(T* __restrict__ out, c
   for (int it = 0; it < ITERS; ++it) {
     const int col = (it * G + lane) * VEC;
     if (row_ok && col < n) {
-      Vec<T, VEC> g = load_vec<T, VEC>(gamma + col);
-      Vec<T, VEC> b = load_vec<T, VEC>(beta + col);
       Vec<T, VEC> o;
       float y[VEC];
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
-        y[j] = to_float(b.v[j]) + to_float(g.v[j]) * rstd * (x[it][j] - mean);
+        y[j] = to_float(bt[it].v[j]) + to_float(g[it].v[j]) * rstd * (x[it][j] - mean);
         if (RES32) asm volatile("" : "+v"(y[j]));  // out is the rounding of the fp32 value, not of the exact multiply-add
       }
       // (the stores in loops of their own: an asm statement between two stores keeps them from being merged)
@@ -129,11 +132,11 @@ __global__ __launch_bounds__(kBlock) void layer_norm_block(T* __restrict__ out, 
   __shared__ float red[2][kBlock / kWave];
   const int64_t row = blockIdx.x;
   T* orow = out + row * n;
-  const T* irow = (ADD && !RES32) ? input + row * n : nullptr;
+  const T* irow = !RES32 && input != nullptr ? input + row * n : orow;
   const float* rrow = RES32 ? res32 + row * n : nullptr;
   float sum = 0.f, sumsq = 0.f;
   for (int c = threadIdx.x; c < n; c += kBlock) {
-    float x = RES32 == 2 ? out32[row * n + c] : to_float(orow[c]);
+    float x = RES32 == 2 ? out32[row * n + c] : to_float((ADD ? orow : irow)[c]);
     if (ADD) x = x + (RES32 ? rrow[c] : to_float(irow[c])) + to_float(bias[c]);
     sum += x;
     sumsq += x * x;
@@ -156,7 +159,7 @@ __global__ __launch_bounds__(kBlock) void layer_norm_block(T* __restrict__ out, 
   const float var = fmaxf(sumsq / (float)n - mean * mean, 0.f);  // cancellation on a near-constant row must not go negative
   const float rstd = 1.0f / sqrtf(var + eps);
   for (int c = threadIdx.x; c < n; c += kBlock) {
-    float x = RES32 == 2 ? out32[row * n + c] : to_float(orow[c]);
+    float x = RES32 == 2 ? out32[row * n + c] : to_float((ADD ? orow : irow)[c]);
     if (ADD) x = x + (RES32 ? rrow[c] : to_float(irow[c])) + to_float(bias[c]);
     float y = to_float(beta[c]) + to_float(gamma[c]) * rstd * (x - mean);
     // the 16-bit output is the rounding of the fp32 one: keep the compiler from folding the conversion into the
@@ -188,7 +191,7 @@ static int layer_norm_dispatch(T* out, const T* input, const T* bias, const T* g
   constexpr int VEC = 16 / sizeof(T);
   auto aligned16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const bool vec_ok = (n % VEC == 0) && aligned16(out) && aligned16(gamma) && aligned16(beta) &&
-                      (!ADD || ((RES32 || aligned16(input)) && aligned16(bias)));
+                      (RES32 || aligned16(input)) && (!ADD || aligned16(bias));
   if (vec_ok) {
     const int64_t nv = n / VEC;  // 16-byte vectors per row
     // Pick the group width G so that nv = G * ITERS with as little idle lane time as possible.
@@ -425,6 +428,15 @@ int ttmi_layer_norm(void* out, const void* gamma, const void* beta, int64_t m, i
   TTMI_DISPATCH_FLOAT(dtype, T, return (layer_norm_dispatch<T, false>((T*)out, nullptr, nullptr, (const T*)gamma,
                                                                        (const T*)beta, m, n, eps,
                                                                        (hipStream_t)stream)));
+  return 0;
+}
+
+int ttmi_layer_norm_from(void* out, const void* input, const void* gamma, const void* beta, int64_t m, int64_t n, float eps,
+                         int dtype, void* stream) {
+  TTMI_REQUIRE(out && input && gamma && beta && out != input, "null tensor, or in place");
+  TTMI_REQUIRE(m >= 0 && n >= 0 && n < (1ll << 31), "bad shape");
+  TTMI_DISPATCH_FLOAT(dtype, T, return (layer_norm_dispatch<T, false>((T*)out, (const T*)input, nullptr, (const T*)gamma,
+                                                                       (const T*)beta, m, n, eps, (hipStream_t)stream)));
   return 0;
 }
 

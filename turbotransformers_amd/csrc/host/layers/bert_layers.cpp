@@ -172,8 +172,7 @@ void PositionwiseFeedForward::operator()(const Tensor& input_tensor, Tensor* out
   const DLDeviceType dev = input_tensor.device_type();
   const int id = input_tensor.device_id();
   normed_.ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/LayerNorm/Reshape");
-  core::CopyBytes(normed_.mutable_raw(), dev, input_tensor.raw(), dev, (size_t)input_tensor.numel() * input_tensor.element_size());
-  kernels::LayerNorm<float>(layer_norm_weight_, layer_norm_bias_, &normed_, 1e-12f);
+  kernels::LayerNormFrom(input_tensor, layer_norm_weight_, layer_norm_bias_, &normed_, 1e-12f);
   hidden_.ReshapeAs(input_tensor.dtype(), {m, d_ff}, dev, id, "FFN/gemm0/Reshape");
   GemmBiasAct(normed_, packed1_.Get(dense_weight_1_, is_trans_weight), d_ff, dense_bias_1_, TTMI_ACT_RELU, &hidden_);
   output->ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/Reshape");

@@ -181,6 +181,17 @@ void LayerNorm(const Tensor& gamma, const Tensor& beta, Tensor* out_tensor, T ep
 }
 template void LayerNorm<float>(const Tensor&, const Tensor&, Tensor*, float, const std::string);
 
+void LayerNormFrom(const Tensor& input, const Tensor& gamma, const Tensor& beta, Tensor* out_tensor, float eps) {
+  RequireGpu(*out_tensor, "LayerNorm");
+  const int64_t n = out_tensor->shape(-1), m = out_tensor->numel() / n;
+  TT_ENFORCE_EQ(input.numel(), m * n, "LayerNorm: input and output differ in size");
+  TT_ENFORCE_EQ(gamma.numel(), n, "LayerNorm gamma size mismatch");
+  TT_ENFORCE_EQ(beta.numel(), n, "LayerNorm beta size mismatch");
+  RequireSameDType(input, *out_tensor, "LayerNorm");
+  TT_DEVICE_CALL(ttmi_layer_norm_from(out_tensor->mutable_raw(), input.raw(), gamma.raw(), beta.raw(), m, n, eps,
+                                      DeviceDType(*out_tensor), Stream()));
+}
+
 template <typename T>
 void AddBiasLayerNorm(const Tensor& input_tensor, const Tensor& bias_tensor, const Tensor& gamma_tensor,
                       const Tensor& beta_tensor, Tensor* out_tensor, T eps, const std::string) {

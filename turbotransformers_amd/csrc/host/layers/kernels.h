@@ -55,6 +55,9 @@ void ApplyMaskAndSoftmax(core::Tensor* inout, const core::Tensor& att_mask, floa
 template <typename T>
 void LayerNorm(const core::Tensor& gamma, const core::Tensor& beta, core::Tensor* out_tensor, T eps = 1e-12,
                const std::string name = "LayerNorm");
+// out = LayerNorm(input), out of place
+void LayerNormFrom(const core::Tensor& input, const core::Tensor& gamma, const core::Tensor& beta, core::Tensor* out_tensor,
+                   float eps);
 template <typename T>
 void AddBiasLayerNorm(const core::Tensor& input_tensor, const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor,
                       const core::Tensor& beta_tensor, core::Tensor* out_tensor, T eps = 1e-12,

@@ -35,7 +35,7 @@ void BertAttention::EnforceShapeAndType() const {
 }
 
 bool MultiHeadedAttention::UseFusedCore(const Tensor& attention_mask, const Tensor* att_score, int64_t head_dim, int dtype,
-                                        int64_t batch, int64_t seq, int64_t heads) {
+                                        int64_t batch, int64_t seq, int64_t heads, bool v_transposed) {
   bool mask_is_key_mask = true;
   if (!attention_mask.is_null()) {
     mask_is_key_mask = attention_mask.n_dim() == 2 || (attention_mask.n_dim() == 3 && attention_mask.shape(1) == 1) ||
@@ -47,9 +47,16 @@ bool MultiHeadedAttention::UseFusedCore(const Tensor& attention_mask, const Tens
     // three launches of the chain (18 us) when the sequence is short or when there are wavefronts for half the SIMDs
     // (1024 on this chip).  (batch, seq: of the padded tensors when the batch is a packed one)
     const int64_t wave_blocks = batch * heads * ((seq + 31) / 32);
-    dtype_ok = seq <= 128 || wave_blocks >= 512;
+    // With V transposed, few long sequences take the form that splits the keys (1 x 512: 18 against 34 us).
+    dtype_ok = v_transposed || seq <= 128 || wave_blocks >= 512;
   }
   return att_score == nullptr && head_dim == 64 && dtype_ok && mask_is_key_mask;
+}
+
+bool MultiHeadedAttention::UseProbsCore(int64_t head_dim, int64_t keys, std::initializer_list<const Tensor*> tensors) const {
+  bool aligned = true;
+  for (const Tensor* t : tensors) aligned = aligned && reinterpret_cast<uintptr_t>(t->raw()) % 16 == 0;
+  return head_dim == 64 && keys > 0 && keys <= TTMI_PROBS_MAX_KEYS && aligned;
 }
 
 static int64_t RoundUp8(int64_t n) { return (n + 7) / 8 * 8; }
@@ -58,7 +65,8 @@ static int64_t RoundUp8(int64_t n) { return (n + 7) / 8 * 8; }
 void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tensor& attention_mask, Tensor* output,
                                          Tensor* att_score, int64_t batch, int64_t seq, int64_t key_seq, const Tensor& k,
                                          const Tensor& v, const std::vector<int64_t>* seq_list, bool fused_core, int64_t v_pitch,
-                                         bool post_layernorm, bool post_add_input, bool is_trans_weight) const {
+                                         bool post_layernorm, bool post_add_input, bool is_trans_weight,
+                                         const CacheGrowth* grow) const {
   const int dt = kernels::DeviceDType(query_tensor);
   const DLDeviceType dev = query_tensor.device_type();
   const int dev_id = query_tensor.device_id();
@@ -87,6 +95,23 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   // and when a key/value cache has been prepended)
   const int64_t F = seq, T = key_seq;
   score->ReshapeAs(query_tensor.dtype(), {batch, heads, F, T}, dev, dev_id, "batch_gemm3/Reshape");
+  // One kernel for the chain below: 8 hypotheses x 100 keys 4.5 against 14.8 us (fp16), 64 x 64 queries x 256 keys 32
+  // against 42; with thousands of workgroups the chain's larger tiles win (32 x 512 x 512: 212 against 201 us).
+  const int64_t workgroups = batch * heads * ((F + 31) / 32);
+  if (grow != nullptr || (seq_list == nullptr && batch * heads < 65536 && workgroups <= 4096 && UseProbsCore(d, T, {&k, &v}))) {
+    const float* mask = nullptr;
+    bool per_query = false;
+    if (!attention_mask.is_null()) {
+      per_query = !(attention_mask.n_dim() == 2 || (attention_mask.n_dim() == 3 && attention_mask.shape(1) == 1) ||
+                    (attention_mask.n_dim() == 4 && attention_mask.shape(2) == 1));
+      mask = attention_mask.data<float>();
+      TT_ENFORCE_EQ(attention_mask.numel(), per_query ? batch * F * T : batch * T, "attention mask has the wrong size");
+    }
+    TT_DEVICE_CALL(ttmi_attention_with_probs(
+        q_.raw(), grow ? grow->k_past->raw() : nullptr, grow ? grow->v_past->raw() : nullptr, grow ? grow->k_past->shape(2) : 0,
+        k.raw(), v.raw(), grow ? grow->k_grown->mutable_raw() : nullptr, grow ? grow->v_grown->mutable_raw() : nullptr, mask,
+        per_query ? 1 : 0, score->mutable_raw(), ctx_.mutable_raw(), batch, heads, F, T, d, scaler, dt, Stream()));
+  } else {
   // batch_gemm3: score[b,h] = scaler * q[b,h] k[b,h]^T   (multi_headed_attention.cpp:328-330)
   TT_DEVICE_CALL(ttmi_gemm_strided_batched(q_.raw(), k.raw(), score->mutable_raw(), F, T, d, d, d, T, F * d, T * d, F * T,
                                            batch * heads, 1, scaler, 0.f, dt, Stream()));
@@ -105,6 +130,7 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
                                              seq * d, seq * d, batch * heads, 0, 1.f, 0.f, dt, Stream()));
     kernels::TransposeForScorePad(&ctx_, padded, *seq_list);
   }
+  }  // chain
   }  // unfused core
 
   output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
@@ -186,8 +212,7 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
   if (pre_layernorm) {  // :66-80, :190-199 -- eps is 1e-6 there
     TT_ENFORCE(!layernorm_gamma_.is_null() && !layernorm_beta_.is_null(), "pre_layernorm needs LayerNorm parameters");
     ln_query_.ReshapeAs(query_tensor.dtype(), {batch, seq, hidden}, dev, dev_id, "self/layernorm/Reshape");
-    core::CopyBytes(ln_query_.mutable_raw(), dev, query_tensor.raw(), dev, (size_t)query_tensor.numel() * query_tensor.element_size());
-    kernels::LayerNorm<float>(layernorm_gamma_, layernorm_beta_, &ln_query_, 1e-6f);
+    kernels::LayerNormFrom(query_tensor, layernorm_gamma_, layernorm_beta_, &ln_query_, 1e-6f);
     q_in = &ln_query_;
   }
 
@@ -195,25 +220,47 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
   const Tensor* v_used = &v_;
   int64_t v_pitch = 0;
   bool fused_core = false;
+  // What a call adds to the layer cache is computed into fresh tensors and moved there: no copy.
+  auto fresh = [&](int64_t len, const char* name) {
+    Tensor t(nullptr);
+    t.ReshapeAs(query_tensor.dtype(), {batch, heads, len, d}, dev, dev_id, name);
+    return t;
+  };
+  auto move_to_cache = [&](const char* key, Tensor& t) -> const Tensor* {
+    auto it = layer_cache.find(key);
+    TT_ENFORCE(it != layer_cache.end() && it->second != nullptr, "layer_cache has no entry %s", key);
+    *it->second = std::move(t);
+    return it->second;
+  };
+  Tensor k_cache(nullptr), v_cache(nullptr);
+  CacheGrowth growth{};
   if (is_self) {
     MultiHeadedAttention::EnforceShapeAndType();
     // with the fused core V is kept transposed, [B,h,d,pitch]: its tiles are then plain copies.
     // A key/value cache needs the row-major layout (it is appended along the sequence).
-    // (fp32 with up to 192 rows keeps V row-major: that QKV projection is cut along K, which the transposed-V
-    // epilogue cannot be, and the fp32 kernel takes either layout)
-    const bool fused_self = layer_cache.empty() && UseFusedCore(attention_mask, att_score, d, dt, batch, seq, heads);
-    if (fused_self && !(dt == TTMI_F32 && batch * seq <= 192)) v_pitch = RoundUp8(seq);
+    const bool fused_self = layer_cache.empty() && UseFusedCore(attention_mask, att_score, d, dt, batch, seq, heads, true);
+    if (fused_self) v_pitch = RoundUp8(seq);
     fused_core = fused_self;
     q_.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/q/Reshape");
+    const bool past_k = CacheHas(layer_cache, "self_keys"), past_v = CacheHas(layer_cache, "self_values");
+    Tensor* k_new = &k_;  // where the projection puts keys and values
+    Tensor* v_new = &v_;
+    if (!layer_cache.empty() && !past_k && !past_v) {
+      k_cache = fresh(seq, "self/self_key/Reshape");
+      v_cache = fresh(seq, "self/self_value/Reshape");
+      k_new = &k_cache;
+      v_new = &v_cache;
+    } else {
     k_.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/k/Reshape");
     if (v_pitch > 0) v_.ReshapeAs(query_tensor.dtype(), {batch, heads, d, v_pitch}, dev, dev_id, "self/v/Reshape");
     else v_.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/v/Reshape");
+    }
     // gemm012_fused + SplitAddBiasTransposeForScore in one launch (:199-203)
     ttmi_epilogue_args args{};
     args.bias = qkv_bias_.raw();
     args.q = q_.mutable_raw();
-    args.k = k_.mutable_raw();
-    args.v = v_.mutable_raw();
+    args.k = k_new->mutable_raw();
+    args.v = v_new->mutable_raw();
     args.seq = seq;
     args.heads = heads;
     args.head_dim = d;
@@ -229,9 +276,22 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
       TT_DEVICE_CALL(ttmi_concat(past.raw(), cur->raw(), grown->mutable_raw(), batch * heads, past_len * d, seq * d, dt, Stream()));
       std::swap(*cur, *grown);
     };
-    prepend("self_keys", &k_, &k_grown_, "self/keys/Concat");
-    prepend("self_values", &v_, &v_grown_, "self/values/Concat");
-    if (!layer_cache.empty()) {
+    if (k_new == &k_cache) {
+      k_used = move_to_cache("self_keys", k_cache);
+      v_used = move_to_cache("self_values", v_cache);
+    } else if (past_k && past_v && batch * heads < 65536 && layer_cache.at("self_keys")->shape(2) > 0 &&
+               layer_cache.at("self_keys")->shape(2) == layer_cache.at("self_values")->shape(2) &&
+               UseProbsCore(d, layer_cache.at("self_keys")->shape(2) + seq, {layer_cache.at("self_keys"), layer_cache.at("self_values")})) {
+      // the attention core reads [past | new] in place and writes the grown cache on the way
+      const int64_t total = layer_cache.at("self_keys")->shape(2) + seq;
+      k_cache = fresh(total, "self/self_key/Reshape");
+      v_cache = fresh(total, "self/self_value/Reshape");
+      growth = CacheGrowth{layer_cache.at("self_keys"), layer_cache.at("self_values"), &k_cache, &v_cache};
+    } else {
+      prepend("self_keys", &k_, &k_grown_, "self/keys/Concat");
+      prepend("self_values", &v_, &v_grown_, "self/values/Concat");
+    }
+    if (!layer_cache.empty() && k_used == &k_ && growth.k_grown == nullptr) {
       StoreInCache(layer_cache, "self_keys", k_, "self/self_key/Reshape");
       StoreInCache(layer_cache, "self_values", v_, "self/self_value/Reshape");
     }
@@ -253,19 +313,25 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
                  "key and value must be [batch_size, key_seq_len, hidden_size]");
       TT_ENFORCE(core::SameDataType(key_tensor.dtype(), query_tensor.dtype()) && core::SameDataType(value_tensor.dtype(), query_tensor.dtype()),
                  "key, value and query must share one element type");
-      ProjectToHeads(key_tensor, k_packed_.Get(k_weight_, is_trans_weight), k_bias_, heads, &k_, "context/keys/AddBiasTransposeForScore/Reshape");
-      ProjectToHeads(value_tensor, v_packed_.Get(v_weight_, is_trans_weight), v_bias_, heads, &v_, "context/values/AddBiasTransposeForScore/Reshape");
-      if (!layer_cache.empty()) {  // :128-150
-        StoreInCache(layer_cache, "memory_keys", k_, "context/keys/AddBiasTransposeForScore/Reshape");
-        StoreInCache(layer_cache, "memory_values", v_, "context/values/AddBiasTransposeForScore/Reshape");
+      const bool keep = !layer_cache.empty();  // :128-150
+      ProjectToHeads(key_tensor, k_packed_.Get(k_weight_, is_trans_weight), k_bias_, heads, keep ? &k_cache : &k_, "context/keys/AddBiasTransposeForScore/Reshape");
+      ProjectToHeads(value_tensor, v_packed_.Get(v_weight_, is_trans_weight), v_bias_, heads, keep ? &v_cache : &v_, "context/values/AddBiasTransposeForScore/Reshape");
+      if (keep) {
+        k_used = move_to_cache("memory_keys", k_cache);
+        v_used = move_to_cache("memory_values", v_cache);
       }
     }
   }
-  const int64_t key_seq = fused_core ? seq : k_used->shape(2);
-  TT_ENFORCE_EQ(fused_core ? seq : v_used->shape(2), key_seq, "keys and values differ in length");
+  const bool growing = growth.k_grown != nullptr;
+  const int64_t key_seq = fused_core ? seq : growing ? k_cache.shape(2) : k_used->shape(2);
+  TT_ENFORCE_EQ(fused_core ? seq : growing ? v_cache.shape(2) : v_used->shape(2), key_seq, "keys and values differ in length");
 
   AttentionTail(query_tensor, attention_mask, output, att_score, batch, seq, key_seq, *k_used, *v_used, nullptr, fused_core, v_pitch,
-                post_layernorm, post_add_input, is_trans_weight);
+                post_layernorm, post_add_input, is_trans_weight, growing ? &growth : nullptr);
+  if (growing) {
+    move_to_cache("self_keys", k_cache);
+    move_to_cache("self_values", v_cache);
+  }
 }
 
 void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attention_mask, Tensor* output, Tensor* attn,

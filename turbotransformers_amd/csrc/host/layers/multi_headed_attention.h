@@ -17,6 +17,7 @@
 //   AddBiasLayerNorm(out, input) in place                             (AddBiasLayerNorm)
 #pragma once
 
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -62,19 +63,28 @@ class MultiHeadedAttention {
 
   // The whole attention core runs as one kernel when nobody asks for the probabilities
   // (head size 64, additive key mask broadcast over the query rows).
-  // batch, seq, heads: the shape of a dense batch (fp32 takes the fused kernel only for those, and only where it pays)
+  // batch, seq, heads: the shape of a dense batch (fp32 takes the fused kernel only for those, and only where it pays:
+  // everywhere if the caller keeps V transposed)
   static bool UseFusedCore(const core::Tensor& attention_mask, const core::Tensor* att_score, int64_t head_dim, int dtype,
-                           int64_t batch = 0, int64_t seq = 0, int64_t heads = 0);
+                           int64_t batch = 0, int64_t seq = 0, int64_t heads = 0, bool v_transposed = false);
 
  protected:
+  // A key/value cache that the attention core extends: [past | new] along the sequence into the grown tensors.
+  struct CacheGrowth {
+    const core::Tensor *k_past, *v_past;
+    core::Tensor *k_grown, *v_grown;
+  };
+  // The one-kernel core that also returns the probabilities (head size 64, up to TTMI_PROBS_MAX_KEYS keys).
+  bool UseProbsCore(int64_t head_dim, int64_t keys, std::initializer_list<const core::Tensor*> tensors) const;
+
   // Everything after q/k/v exist, shared by the dense and the smart-batch layers.
   // `fused_core`: the one-kernel attention core runs; `v_pitch` > 0: v holds V transposed, [B,h,d,v_pitch].
-  // `seq` query positions against `key_seq` key positions held in k / v ([B,h,key_seq,d]).
+  // `seq` query positions against `key_seq` key positions held in k / v ([B,h,key_seq,d]); with `grow` the first of them
+  // are in its past tensors instead, and k / v hold the rest.
   void AttentionTail(const core::Tensor& query_tensor, const core::Tensor& attention_mask, core::Tensor* output,
                      core::Tensor* att_score, int64_t batch, int64_t seq, int64_t key_seq, const core::Tensor& k,
                      const core::Tensor& v, const std::vector<int64_t>* seq_list, bool fused_core, int64_t v_pitch,
-                     bool post_layernorm,
-                     bool post_add_input, bool is_trans_weight) const;
+                     bool post_layernorm, bool post_add_input, bool is_trans_weight, const CacheGrowth* grow = nullptr) const;
 
   core::Tensor k_weight_, k_bias_, v_weight_, v_bias_, q_weight_, q_bias_;
   core::Tensor dense_weight_, dense_bias_, qkv_weight_, qkv_bias_;

@@ -34,8 +34,10 @@ class MultiHeadedAttention(cxx.MultiHeadedAttention):
         if layer_cache is not None:
             for k, v in layer_cache.items():
                 cache[k] = try_convert(v) if v is not None else cxx.Tensor.create_empty()
-        super().__call__(try_convert(key_tensor), try_convert(value_tensor), try_convert(query_tensor),
-                         try_convert(create_empty_if_none(mask)), attn_type, output, attn, cache, pre_layernorm,
+        query = try_convert(query_tensor)
+        key = query if key_tensor is query_tensor else try_convert(key_tensor)
+        value = key if value_tensor is key_tensor else try_convert(value_tensor)
+        super().__call__(key, value, query, try_convert(create_empty_if_none(mask)), attn_type, output, attn, cache, pre_layernorm,
                          post_layernorm, post_add_input, is_trans_weight)
         if layer_cache is not None:
             for k, v in cache.items():

@@ -2,11 +2,15 @@
 import enum
 from typing import Optional
 
+import torch
 import torch.utils.dlpack as dlpack
 
 from .. import cxx
 
 __all__ = ['ReturnType', 'convert_returns_as_type']
+
+
+_capsule_to_torch = getattr(torch._C, '_from_dlpack', dlpack.from_dlpack)  # a capsule needs no protocol negotiation
 
 
 class ReturnType(enum.Enum):
@@ -21,12 +25,10 @@ def convert_returns_as_type(tensor, rtype: Optional[ReturnType]):
     device, so an error a kernel reported (an embedding id out of range, whose row is NaN in the result) is raised
     by the next `cxx.synchronize()`.  NUMPY copies to the host, which waits for the device anyway, and raises
     such an error itself."""
-    if rtype is None:
-        rtype = ReturnType.TORCH
+    if rtype is None or rtype is ReturnType.TORCH:
+        return _capsule_to_torch(tensor.to_dlpack())
     if rtype == ReturnType.turbo_transformers:
         return tensor
-    if rtype == ReturnType.TORCH:
-        return dlpack.from_dlpack(tensor.to_dlpack())
     if rtype == ReturnType.NUMPY:
         t = dlpack.from_dlpack(tensor.to_dlpack())
         host = t.float().cpu().numpy()

@@ -12,12 +12,18 @@ __all__ = ['try_convert', 'convert2tt_tensor', 'to_param_dict_convert_tt', 'to_p
 
 AnyTensor = Union[cxx.Tensor, torch.Tensor]
 
+# (looked up once: a decoder step converts about a hundred tensors)
+_to_dlpack = dlpack.to_dlpack
+_from_dlpack = cxx.Tensor.from_dlpack
+_create_empty = cxx.Tensor.create_empty
+_raw_stream = getattr(torch._C, '_cuda_getCurrentRawStream', None)  # absent from builds without a device
+
 
 def convert2tt_tensor(t: torch.Tensor):
     """Zero-copy alias of a torch tensor; the cxx.Tensor keeps the torch storage alive."""
     if not t.is_contiguous():
         t = t.contiguous()
-    return cxx.Tensor.from_dlpack(dlpack.to_dlpack(t.detach()))
+    return _from_dlpack(_to_dlpack(t.detach() if t.requires_grad else t))
 
 
 def try_convert(t, device: Optional[torch.device] = None):
@@ -38,13 +44,16 @@ def to_param_dict(torch_module: torch.nn.Module):
 
 
 def create_empty_if_none(output):
-    return output if output is not None else cxx.Tensor.create_empty()
+    return output if output is not None else _create_empty()
 
 
 def use_current_stream():
     """Enqueue the kernels of the following calls on torch's current stream, so they are ordered
     after whatever torch has queued on the inputs."""
-    cxx.set_stream(torch.cuda.current_stream().cuda_stream)
+    if _raw_stream is not None and torch.cuda.is_initialized():
+        cxx.set_stream(_raw_stream(torch.cuda.current_device()))  # a tenth of the cost of a Stream object
+    else:
+        cxx.set_stream(torch.cuda.current_stream().cuda_stream)
 
 
 def weight_in_out(linear_weight: torch.Tensor) -> torch.Tensor:
