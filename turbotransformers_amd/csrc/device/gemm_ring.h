@@ -495,7 +495,8 @@ struct RingTile {
   X(128, 64, 2, 2, 4, 1, 5.08f, 4.03f, 0.258f, 0.258f)       \
   X(64, 192, 4, 2, 3, 1, 6.02f, 5.34f, 0.379f, 0.377f)       \
   X(128, 128, 4, 2, 3, 1, 6.55f, 6.98f, 0.376f, 0.376f)      \
-  X(128, 192, 4, 2, 3, 1, 8.73f, 10.6f, 0.465f, 0.465f)
+  X(128, 192, 4, 2, 3, 1, 8.73f, 10.6f, 0.465f, 0.465f)      \
+  X(256, 128, 4, 2, 3, 1, 11.0f, 10.9f, 0.594f, 0.594f)
 
 #define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
 template <size_t ELEM>
