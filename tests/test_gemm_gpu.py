@@ -112,6 +112,28 @@ def test_ring_kernel_epilogues_on_ragged_tiles(ttmi, oracle, dt, M, N, K):
 
 
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("M,N,steps", [(1, 8, 1), (16, 24, 16), (17, 776, 17), (33, 768, 24), (32, 3072, 12), (10, 768, 33), (64, 136, 96),
+                                       (160, 768, 12)])
+def test_few_row_kernel_epilogues(ttmi, oracle, dt, M, N, steps):
+    """The form for few rows (sixteen wavefronts divide K): shares of no, one, two and more K steps of 128 bytes, one and two blocks
+    of rows, ragged rows and columns, every epilogue.  Rows past M stay untouched."""
+    import ctypes
+    K = steps * (32 if dt == "f32" else 64)
+    rng = np.random.default_rng(M + N + K)
+    A, W = _ab(rng, M, N, K, 1)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    dA, dW, db, dres = dev(A, dt), dev(W, dt), dev(bias, dt), dev(res, dt)
+    base = oracle.matmul(rounded(A, dt), rounded(W, dt), True) + rounded(bias, dt)
+    for epi, args, want in ((capi.EPI_BIAS, _epi(bias=db), base), (capi.EPI_BIAS_ACT, _epi(bias=db, act=capi.ACT_RELU), np.maximum(base, 0)),
+                            (capi.EPI_BIAS_RESIDUAL, _epi(bias=db, residual=dres), base + rounded(res, dt)),
+                            (capi.EPI_F32_OUT, _epi(bias=db), base)):
+        C = torch.full((M + 40, N), -7.0, dtype=torch.float32 if epi == capi.EPI_F32_OUT else dA.dtype, device="cuda")
+        ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(dW), ptr(C), M, N, K, K, K, N, epi, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+        assert max_abs(host(C[:M]), want) <= GEMM_TOL[dt] * 3
+        assert torch.all(C[M:] == -7.0)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("v_transposed", [False, True])
 @pytest.mark.parametrize("B,S,h", [(1, 1, 12), (3, 5, 12), (1, 37, 16), (9, 31, 12), (7, 130, 12), (2, 387, 16)])
 def test_ring_kernel_head_split(ttmi, oracle, dt, v_transposed, B, S, h):

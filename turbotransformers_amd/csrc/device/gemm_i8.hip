@@ -1,5 +1,5 @@
 // int8 products: the plain int32 one and those with the dequantisation in their epilogue.
-#include "gemm_ring.h"
+#include "gemm_select.h"
 
 using namespace ttmi;
 
