@@ -375,6 +375,14 @@ TTMI_API int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, i
                              int64_t lda, int64_t ldb, int64_t ldc, int epilogue,
                              const ttmi_epilogue_args* args, int dtype, void* stream);
 
+/* ttmi_gemm_fused on LayerNorm(x): x [m,k], w [n,k] and normed [m,k] are contiguous.  One launch for a few rows with the
+ * QKV_SPLIT and the BIAS_ACT (ReLU) epilogue; otherwise ttmi_layer_norm_from into `normed` (scratch of the caller, which must
+ * not overlap x) and the product from there.  What `normed` holds afterwards is unspecified.
+ * (The pre-LayerNorm of layers/multi_headed_attention.cpp:66-80, :190-199 and of layers/positionwise_ffn.cpp.) */
+TTMI_API int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const void* beta, float eps, void* normed,
+                                        const void* w, void* c, int64_t m, int64_t n, int64_t k, int64_t ldc, int epilogue,
+                                        const ttmi_epilogue_args* args, int dtype, void* stream);
+
 /* Which kernel variant ttmi_gemm (epilogue TTMI_EPI_NONE, args NULL) or ttmi_gemm_fused would launch for an
  * aligned, densely packed product of this shape, as text: family (reg = register-staged, dma = global->LDS DMA,
  * dma_agpr = DMA with accumulators in AGPRs, dma3_agpr = the same with a third LDS stage for the A operand, wave = one wavefront per tile with its operand fragments straight from

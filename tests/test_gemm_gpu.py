@@ -929,3 +929,35 @@ def test_fused_attention_packed_batch(ttmi, oracle, attention_waves, dt, v_trans
     ctx = oracle.batch_matmul(prob, rounded(V, dt), False)
     want = oracle.transpose_for_score_pad(ctx, lens).reshape(total, h * d)
     assert max_abs(host(out), want) <= GEMM_TOL[dt] * 2
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("M,h,steps", [(1, 1, 1), (16, 1, 16), (17, 12, 12), (33, 3, 17), (8, 12, 24), (31, 4, 32), (40, 2, 33)])
+def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps):
+    """LayerNorm on the rows' way into the form for few rows (and, past its sizes, in a launch of its own): one and two steps of K
+    per wavefront, one and two blocks of rows, ragged tiles; ReLU and head-split epilogues; a row of equal values."""
+    import ctypes
+    N, K = 64 * h, steps * (32 if dt == "f32" else 64)
+    rng = np.random.default_rng(M + N + K)
+    X, W = rng.standard_normal((M, K)).astype(np.float32), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    X[M // 2] = 3.0
+    gamma, beta = 1 + 0.1 * rng.standard_normal(K).astype(np.float32), 0.1 * rng.standard_normal(K).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    dX, dW, dg, dbeta, db = dev(X, dt), dev(W, dt), dev(gamma, dt), dev(beta, dt), dev(bias, dt)
+    x = rounded(X, dt).astype(np.float64)
+    ln = (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-6) * rounded(gamma, dt) + rounded(beta, dt)
+    base = ln @ rounded(W, dt).astype(np.float64).T + rounded(bias, dt)
+    normed = torch.empty_like(dX)
+    C = torch.full((M + 40, N), -7.0, dtype=dX.dtype, device="cuda")
+    args = _epi(bias=db, act=capi.ACT_RELU)
+    ok(ttmi.ttmi_layer_norm_gemm_fused(ptr(dX), ptr(dg), ptr(dbeta), ctypes.c_float(1e-6), ptr(normed), ptr(dW), ptr(C), M, N, K, N, capi.EPI_BIAS_ACT,
+                                       ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+    # |LN| and the rows of W are of size 1, so the rounding of LN to the type is one more rounding of the kind GEMM_TOL holds
+    assert max_abs(host(C[:M]), np.maximum(base, 0)) <= GEMM_TOL[dt] * 3
+    assert torch.all(C[M:] == -7.0)
+    q = torch.full((M + 1, h, 1, 64), -7.0, dtype=dX.dtype, device="cuda")
+    args = _epi(bias=db, q=q, seq=1, heads=h, head_dim=64)
+    ok(ttmi.ttmi_layer_norm_gemm_fused(ptr(dX), ptr(dg), ptr(dbeta), ctypes.c_float(1e-6), ptr(normed), ptr(dW), None, M, N, K, N, capi.EPI_QKV_SPLIT,
+                                       ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+    assert max_abs(host(q[:M]).reshape(M, N), base) <= GEMM_TOL[dt] * 3
+    assert torch.all(q[M:] == -7.0)

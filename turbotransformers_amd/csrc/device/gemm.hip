@@ -12,7 +12,11 @@ int gemm_alpha_beta(const void* a, const void* b, void* c, int64_t m, int64_t n,
                     int inner, int64_t a_outer, int64_t a_inner, int64_t b_outer, int64_t b_inner, int64_t c_outer,
                     int64_t c_inner, int64_t batch, int trans_b, float alpha, float beta, hipStream_t s);
 template <typename T>
-int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, hipStream_t s);
+int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, hipStream_t s,
+                     const NormRows<T>* norm);
+template <typename T>
+int gemm_norm_fused_typed(const GemmArgs& g, const void* gamma, const void* beta, float eps, void* c, int64_t ldc, int epilogue,
+                          const ttmi_epilogue_args* args, hipStream_t s);
 template <typename T>
 int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
@@ -111,8 +115,27 @@ int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, int64_t n,
   g.m = (int)m; g.n = (int)n; g.k = (int)k;
   g.lda = lda; g.ldb = ldb;
   g.inner = 1;
-  TTMI_DISPATCH_FLOAT(dtype, T, return gemm_fused_typed<T>(g, c, ldc, epilogue, args, (hipStream_t)stream));
+  TTMI_DISPATCH_FLOAT(dtype, T, return gemm_fused_typed<T>(g, c, ldc, epilogue, args, (hipStream_t)stream, nullptr));
   return 0;
+}
+
+int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const void* beta, float eps, void* normed, const void* w, void* c,
+                               int64_t m, int64_t n, int64_t k, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, int dtype,
+                               void* stream) {
+  TTMI_REQUIRE(x && gamma && beta && normed && w && args && normed != x, "null tensor, or in place");
+  TTMI_REQUIRE(m >= 0 && n >= 0 && k >= 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension out of range");
+  GemmArgs g{};
+  g.a = (const char*)x;
+  g.b = (const char*)w;
+  g.m = (int)m; g.n = (int)n; g.k = (int)k;
+  g.lda = k; g.ldb = k;
+  g.inner = 1;
+  int rc = kNormNotTaken;
+  TTMI_DISPATCH_FLOAT(dtype, T, rc = gemm_norm_fused_typed<T>(g, gamma, beta, eps, c, ldc, epilogue, args, (hipStream_t)stream));
+  if (rc != kNormNotTaken) return rc;
+  rc = ttmi_layer_norm_from(normed, x, gamma, beta, m, k, eps, dtype, stream);
+  if (rc != 0) return rc;
+  return ttmi_gemm_fused(normed, w, c, m, n, k, k, k, ldc, epilogue, args, dtype, stream);
 }
 
 int ttmi_gemm_describe(int64_t m, int64_t n, int64_t k, int epilogue, const ttmi_epilogue_args* args, int dtype, char* out,

@@ -11,6 +11,11 @@
 // (Straight from memory to registers is slower: the 64 bytes of K that a matrix instruction takes of a row are half a
 // cache line, and a CU then fetches 43 GB/s instead of 115.)
 // Narrow tiles spread the weights over many CUs; every row tile reads them again.
+//
+// LayerNorm in front (NormRows): every workgroup normalises the rows of its tile itself, a row per wavefront, while its first
+// weights are on their way, and keeps them in LDS for the whole of K.  The rows are a few KB that L2 serves, so the repeated
+// work hides under the wait for the weights; a launch of its own and the gap in front of the next one are gone.
+// Six decoder layers, fp16, 8 x 1 tokens, 41 keys: 67 launches and 343 us a step before, 49 and 264 after.
 #pragma once
 
 #include "gemm_ring.h"
@@ -36,6 +41,14 @@ __device__ __forceinline__ void flat_mma(const Chunk& a, const Chunk& b, typenam
 #endif
 }
 
+// What becomes of the rows of A on their way in.
+struct PlainRows {};
+template <typename T>
+struct NormRows {  // beta + gamma * (x - mean) / sqrt(var + eps), rounded to T as a tensor of its own would be
+  const T *gamma, *beta;
+  float eps;
+};
+
 constexpr int kFlatWaves = 16;
 constexpr int kFlatPitch = 20;  // words of a row of a partial tile: 16-byte aligned, four rows apart on other banks
 template <int MB>
@@ -44,11 +57,13 @@ template <int MB>
 constexpr int flat_partial_bytes() { return kFlatWaves * MB * 16 * kFlatPitch * 4; }
 
 // MB: blocks of 16 rows.  D: LDS stages per wavefront (steps of 128 bytes of K; one suffices for a share of one step).
-// LDS: the stages of the wavefronts that have a share; afterwards one partial tile per wavefront.
-template <typename T, int MB, int D, typename Epi>
-__global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const GemmArgs g, const Epi epi) {
-  constexpr int NW = kFlatWaves, PITCH = kFlatPitch, STAGE = flat_stage_bytes<MB>();
-  constexpr int LOADS = 2 * (MB + 1);  // 1 KB loads of a step: eight rows each
+// LDS: (normalised rows: a block of MB * 16 rows x 128 bytes per step of K, then) the stages of the wavefronts that have a
+// share; afterwards one partial tile per wavefront.
+template <typename T, int MB, int D, typename Epi, typename Rows = PlainRows>
+__global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const GemmArgs g, const Epi epi, const Rows rows) {
+  constexpr bool NORM = !std::is_same<Rows, PlainRows>::value;
+  constexpr int NW = kFlatWaves, PITCH = kFlatPitch, STAGE = NORM ? flat_stage_bytes<0>() : flat_stage_bytes<MB>();
+  constexpr int A_LOADS = NORM ? 0 : 2 * MB, LOADS = A_LOADS + 2;  // 1 KB loads of a step: eight rows each
   using Acc = typename RingMma<T>::Acc;
   using AccScalar = typename Epi::Acc;
   extern __shared__ __align__(16) char smem[];
@@ -94,12 +109,12 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
     const int sub = lane >> 3, c = lane & 7;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const int row = i * 8 + sub;  // of the stage: MB * 16 rows of A, 16 of B
-      const uint32_t at = i < 2 * MB ? (uint32_t)min(m0 + row, g.m - 1) * lda_bytes : (uint32_t)min(n0 + row - MB * 16, g.n - 1) * ldb_bytes;
+      const int row = i * 8 + sub;  // of the stage: (MB * 16 rows of A,) 16 of B
+      const uint32_t at = i < A_LOADS ? (uint32_t)min(m0 + row, g.m - 1) * lda_bytes : (uint32_t)min(n0 + row - A_LOADS * 8, g.n - 1) * ldb_bytes;
       voff[i] = at + ((c ^ ((row >> 1) & 7)) << 4);
     }
   }
-  const int stage0 = wave * (D * STAGE);
+  const int stage0 = (NORM ? steps * (MB * 16 * kRowBytes) : 0) + wave * (D * STAGE);
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lds0 = reinterpret_cast<lds_char*>(reinterpret_cast<uintptr_t>(smem));
@@ -110,11 +125,28 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
     const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.b), 0, live ? b_size : 0, 0x00020000);
 #pragma unroll
     for (int i = 0; i < LOADS; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 2 * MB ? ra : rb, lds0 + stage0 + stage * STAGE + i * 1024, 16, voff[i], k_lo + s * kRowBytes, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < A_LOADS ? ra : rb, lds0 + stage0 + stage * STAGE + i * 1024, 16, voff[i], k_lo + s * kRowBytes, 0, 0);
   };
 #else
   auto load = [&](int, int) {};
 #endif
+
+  // ---- rows to normalise: a wavefront takes every sixteenth, 16 bytes per lane and turn (K is at most 16 * D steps)
+  constexpr int KPC = 16 / (int)sizeof(T), TURNS = NORM ? 2 * D : 1, ROWS = NORM ? MB : 1;
+  Vec<T, KPC> xr[ROWS][TURNS], gm[TURNS], bt[TURNS];
+  if constexpr (NORM) {
+#pragma unroll
+    for (int t = 0; t < TURNS; ++t) {
+      const int col = (t * kWave + lane) * KPC;
+      if (col < kdim) {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+          xr[i][t] = load_vec<T, KPC>(reinterpret_cast<const T*>(g.a) + min(m0 + wave + i * NW, g.m - 1) * g.lda + col);
+        gm[t] = load_vec<T, KPC>(rows.gamma + col);
+        bt[t] = load_vec<T, KPC>(rows.beta + col);
+      }
+    }
+  }
 
   // ---- the thread's piece of the output: eight columns of one row
   const bool stores = tid < MB * 32;
@@ -151,10 +183,44 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[i][e] = 0;
   if (busy) {
-    const uint32_t lds_base = (uint32_t)reinterpret_cast<uintptr_t>(smem) + stage0;
-    const int swz = (lrow >> 1) & 7;
 #pragma unroll
     for (int d = 0; d < D; ++d) load(s_lo + d, d);
+  }
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      float x[TURNS][KPC], sum = 0.f, sumsq = 0.f;
+#pragma unroll
+      for (int t = 0; t < TURNS; ++t)
+        if ((t * kWave + lane) * KPC < kdim)
+#pragma unroll
+          for (int j = 0; j < KPC; ++j) {
+            x[t][j] = to_float(xr[i][t].v[j]);
+            sum += x[t][j];
+            sumsq += x[t][j] * x[t][j];
+          }
+      sum = group_sum<kWave>(sum);
+      sumsq = group_sum<kWave>(sumsq);
+      const float mean = sum / (float)kdim;
+      const float var = fmaxf(sumsq / (float)kdim - mean * mean, 0.f);  // as in layer_norm_rows
+      const float rstd = 1.0f / sqrtf(var + rows.eps);
+      const int row = wave + i * NW;
+#pragma unroll
+      for (int t = 0; t < TURNS; ++t) {
+        const int piece = t * kWave + lane;  // of the row: step piece / 8, chunk piece % 8, at the swizzled place
+        if (piece * KPC < kdim) {
+          Vec<T, KPC> o;
+#pragma unroll
+          for (int j = 0; j < KPC; ++j) o.v[j] = from_float<T>(to_float(bt[t].v[j]) + to_float(gm[t].v[j]) * rstd * (x[t][j] - mean));
+          store_vec<T, KPC>(reinterpret_cast<T*>(smem + (piece >> 3) * (MB * 16 * kRowBytes) + row * kRowBytes + (((piece & 7) ^ ((row >> 1) & 7)) << 4)), o);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (busy) {
+    const uint32_t lds_rows = (uint32_t)reinterpret_cast<uintptr_t>(smem), lds_base = lds_rows + stage0;
+    const int swz = (lrow >> 1) & 7;
     int stage = 0;
 #pragma unroll 1
     for (int s = s_lo; s < s_hi; ++s) {
@@ -163,11 +229,12 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((D - 1) * LOADS) : "memory");
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const uint32_t at = lds_base + stage * STAGE + lrow * kRowBytes + (((h * 4 + lgrp) ^ swz) << 4);
+        const uint32_t in_row = lrow * kRowBytes + (((h * 4 + lgrp) ^ swz) << 4);
+        const uint32_t at = lds_base + stage * STAGE + in_row, at_a = NORM ? lds_rows + s * (MB * 16 * kRowBytes) + in_row : at;
 #pragma unroll
         for (int i = 0; i < MB; ++i)
-          asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(reinterpret_cast<Quad&>(fa[h][i])) : "v"(at), "n"(i * 16 * kRowBytes) : "memory");
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(reinterpret_cast<Quad&>(fb[h])) : "v"(at), "n"(MB * 16 * kRowBytes) : "memory");
+          asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(reinterpret_cast<Quad&>(fa[h][i])) : "v"(at_a), "n"(i * 16 * kRowBytes) : "memory");
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(reinterpret_cast<Quad&>(fb[h])) : "v"(at), "n"(A_LOADS * 8 * kRowBytes) : "memory");
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
@@ -241,8 +308,8 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
   publish_absmax(epi, amax, reinterpret_cast<float*>(smem), NW * kWave);
 }
 
-template <typename T, int MB, int D, typename Epi>
-inline int launch_flat_tile(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
+template <typename T, int MB, int D, typename Epi, typename Rows = PlainRows>
+inline int launch_flat_tile(GemmArgs g, const Epi& epi, int slices, hipStream_t s, const Rows& rows = Rows{}) {
   if (describe_only("dma", kFlatWaves, MB * 16, 16, slices)) return 0;
   g.tiles_m = (g.m + MB * 16 - 1) / (MB * 16);
   g.tiles_n = (g.n + 15) / 16;
@@ -250,18 +317,22 @@ inline int launch_flat_tile(GemmArgs g, const Epi& epi, int slices, hipStream_t 
   const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n * slices;
   TTMI_REQUIRE(tiles < (1ll << 30), "GEMM grid too large");
   const unsigned grid_x = tiles >= kXcdRemapMinTiles ? (unsigned)(ceil_div(tiles, kNumXcd) * kNumXcd) : (unsigned)tiles;
-  if (!absmax_grid_ok(epi, grid_x, 1)) return launch_flat_tile<T, MB, D>(g, without_absmax(epi), slices, s);
+  if (!absmax_grid_ok(epi, grid_x, 1)) return launch_flat_tile<T, MB, D>(g, without_absmax(epi), slices, s, rows);
   const int64_t steps = (g.k_chunk > 0 ? g.k_chunk : g.k) * (int64_t)sizeof(T) / kRowBytes;
   const int64_t share = ceil_div(steps, kFlatWaves);
-  const int lds = std::max((int)ceil_div(steps, share) * D * flat_stage_bytes<MB>(), flat_partial_bytes<MB>());
-  auto kern = gemm_flat_kernel<T, MB, D, Epi>;
+  constexpr bool norm = !std::is_same<Rows, PlainRows>::value;
+  if (norm) TTMI_REQUIRE(g.k_chunk == 0 && steps <= kFlatWaves * D, "rows to normalise come whole");
+  const int64_t stages = norm ? steps * MB * 16 * kRowBytes + ceil_div(steps, share) * D * flat_stage_bytes<0>()
+                              : ceil_div(steps, share) * D * flat_stage_bytes<MB>();
+  const int lds = (int)std::max<int64_t>(stages, flat_partial_bytes<MB>());
+  auto kern = gemm_flat_kernel<T, MB, D, Epi, Rows>;
   static_assert(kFlatWaves * 2 * flat_stage_bytes<1>() <= kLdsPerCu, "stages exceed the LDS");
   TTMI_REQUIRE(lds <= kLdsPerCu, "stages exceed the LDS");
   if (lds > 64 * 1024) {
     const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), kLdsPerCu);
     if (rc != 0) return rc;
   }
-  hipLaunchKernelGGL(kern, dim3(grid_x), dim3(kFlatWaves * kWave), lds, s, g, epi);
+  hipLaunchKernelGGL(kern, dim3(grid_x), dim3(kFlatWaves * kWave), lds, s, g, epi, rows);
   return launch_status("gemm_flat_kernel");
 }
 
@@ -289,6 +360,28 @@ inline int launch_flat(const GemmArgs& g, const Epi& epi, int slices, hipStream_
   const bool one = steps <= kFlatWaves;
   if (g.m <= 16 || !flat_fits<2>(steps)) return one ? launch_flat_tile<T, 1, 1>(g, epi, slices, s) : launch_flat_tile<T, 1, 2>(g, epi, slices, s);
   return one ? launch_flat_tile<T, 2, 1>(g, epi, slices, s) : launch_flat_tile<T, 2, 2>(g, epi, slices, s);
+}
+
+// The same with LayerNorm in front, for rows of at most two steps per wavefront (2048 16-bit or 1024 fp32 values).
+// The line is that of the product alone: one workgroup per CU, so that nobody normalises a row twice.  (A LayerNorm launch
+// of 8 x 768 is 2.9 us on the GPU and 3.5 on the host.)
+template <typename T, int MB>
+inline bool flat_norm_fits(int64_t steps) {
+  const int64_t share = ceil_div(steps, kFlatWaves);
+  return share <= 2 && steps * MB * 16 * kRowBytes + ceil_div(steps, share) * share * flat_stage_bytes<0>() <= kLdsPerCu;
+}
+template <typename T>
+inline bool flat_norm_wins(const GemmArgs& g) {
+  const int64_t steps = g.k * (int64_t)sizeof(T) / kRowBytes;
+  const int64_t rows = g.m <= 16 || !flat_norm_fits<T, 2>(steps) ? 16 : 32;
+  return flat_norm_fits<T, 1>(steps) && ceil_div(g.m, rows) * ceil_div(g.n, 16) <= compute_units();
+}
+template <typename T, typename Epi>
+inline int launch_flat_norm(const GemmArgs& g, const Epi& epi, const NormRows<T>& rows, hipStream_t s) {
+  const int64_t steps = g.k * (int64_t)sizeof(T) / kRowBytes;
+  const bool one = steps <= kFlatWaves;
+  if (g.m <= 16 || !flat_norm_fits<T, 2>(steps)) return one ? launch_flat_tile<T, 1, 1>(g, epi, 1, s, rows) : launch_flat_tile<T, 1, 2>(g, epi, 1, s, rows);
+  return one ? launch_flat_tile<T, 2, 1>(g, epi, 1, s, rows) : launch_flat_tile<T, 2, 2>(g, epi, 1, s, rows);
 }
 
 }  // namespace ttmi

@@ -1707,6 +1707,11 @@ inline SplitPlan plan_split(int64_t m, int64_t n, int64_t k, int64_t batch, bool
   return {SplitKind::kNone, 1};
 }
 
+// LayerNorm in front of a product (gemm_flat.h) and, not an error, that it takes a launch of its own.
+template <typename T>
+struct NormRows;
+constexpr int kNormNotTaken = 1;
+
 // The deep-ring kernel of gemm_ring.h and its selection; declared here for launch_gemm.
 template <typename T, typename Epi>
 struct RingKernel;

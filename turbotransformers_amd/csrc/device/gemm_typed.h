@@ -34,15 +34,23 @@ int gemm_alpha_beta(const void* a, const void* b, void* c, int64_t m, int64_t n,
 }
 
 
+template <typename T, bool PAD>
+inline EpiQkvSplit<T, PAD> qkv_epilogue(const ttmi_epilogue_args* args) {
+  const int hidden = (int)(args->heads * args->head_dim);
+  const bool vec = aligned16(args->q) && aligned16(args->k) && aligned16(args->v) && aligned16(args->bias) && args->head_dim % 8 == 0;
+  return {(T*)args->q, (T*)args->k, (T*)args->v, (const T*)args->bias, PAD ? args->token_rows : nullptr, (int)args->seq,
+          (int)args->heads, (int)args->head_dim, hidden, FastDiv((uint32_t)args->seq), FastDiv((uint32_t)hidden),
+          FastDiv((uint32_t)args->head_dim), vec, (int)args->v_seq_pitch};
+}
+
+// `norm`: A's rows are to be normalised on their way in (gemm_norm_fused_typed has checked that they can be).
 template <typename T>
-int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, hipStream_t s) {
+int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, hipStream_t s, const NormRows<T>* norm) {
   const int64_t m = g.m, n = g.n, k = g.k, lda = g.lda, ldb = g.ldb;
   const void *a = g.a, *b = g.b;
   constexpr int KPC = 16 / sizeof(T);
   const bool aligned = aligned16(a) && aligned16(b) && lda % KPC == 0 && ldb % KPC == 0 && k % KPC == 0;
   const bool c_vec = aligned16(c) && ldc % KPC == 0 && aligned16(args->bias) && aligned16(args->residual);
-  const bool qkv_vec = aligned16(args->q) && aligned16(args->k) && aligned16(args->v) && aligned16(args->bias) &&
-                       args->head_dim % 8 == 0;
   switch (epilogue) {
     case TTMI_EPI_BIAS: {
       TTMI_REQUIRE(c && args->bias && ldc >= n, "BIAS epilogue needs c and bias");
@@ -59,6 +67,8 @@ int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, cons
         return (launch_gemm<T, false>(g, epi, 1, aligned, s));
       } else if (args->act == TTMI_ACT_RELU) {
         EpiBias<T, TTMI_ACT_RELU, true, false> epi{(T*)c, (const T*)args->bias, nullptr, ldc, c_vec};
+        if (norm != nullptr && c_vec) return launch_flat_norm<T>(g, epi, *norm, s);
+        if (norm != nullptr) return kNormNotTaken;
         return (launch_gemm<T, false>(g, epi, 1, aligned, s));
       }
       return fail(TTMI_EINVAL, "unknown activation");
@@ -88,19 +98,31 @@ int gemm_fused_typed(const GemmArgs& g, void* c, int64_t ldc, int epilogue, cons
       TTMI_REQUIRE(vp == 0 || (vp >= args->seq && vp % 8 == 0 && vp < (1ll << 31) && hidden % 8 == 0),
                    "v_seq_pitch must be 0 or a multiple of 8 that is >= seq (hidden a multiple of 8)");
       if (pad) {
-        EpiQkvSplit<T, true> epi{(T*)args->q, (T*)args->k, (T*)args->v, (const T*)args->bias, args->token_rows,
-                                 (int)args->seq, (int)args->heads, (int)args->head_dim, hidden,
-                                 FastDiv((uint32_t)args->seq), FastDiv((uint32_t)hidden), FastDiv((uint32_t)args->head_dim), qkv_vec, (int)vp};
-        return (launch_gemm<T, false>(g, epi, 1, aligned, s));
+        return (launch_gemm<T, false>(g, qkv_epilogue<T, true>(args), 1, aligned, s));
       }
-      EpiQkvSplit<T, false> epi{(T*)args->q, (T*)args->k, (T*)args->v, (const T*)args->bias, nullptr,
-                                (int)args->seq, (int)args->heads, (int)args->head_dim, hidden,
-                                FastDiv((uint32_t)args->seq), FastDiv((uint32_t)hidden), FastDiv((uint32_t)args->head_dim), qkv_vec, (int)vp};
+      const EpiQkvSplit<T, false> epi = qkv_epilogue<T, false>(args);
+      if (norm != nullptr && epi.vec) return launch_flat_norm<T>(g, epi, *norm, s);
+      if (norm != nullptr) return kNormNotTaken;
       return (launch_gemm<T, false>(g, epi, 1, aligned, s));
     }
     default:
       return fail(TTMI_EINVAL, "unknown epilogue");
   }
+}
+
+// LayerNorm(x) in front of a product with an epilogue.  One launch where the form for few rows takes the product and its
+// epilogue (the bias and ReLU of a feed-forward layer, the head split): two are a wait more each and 3 to 4 us of host time.
+// 0: done.  kNormNotTaken: the two launches it is.
+template <typename T>
+int gemm_norm_fused_typed(const GemmArgs& g, const void* gamma, const void* beta, float eps, void* c, int64_t ldc, int epilogue,
+                          const ttmi_epilogue_args* args, hipStream_t s) {
+  const bool known = epilogue == TTMI_EPI_QKV_SPLIT || (epilogue == TTMI_EPI_BIAS_ACT && args->act == TTMI_ACT_RELU);
+  if (!known || g.m == 0 || g.n == 0 || g.k * (int)sizeof(T) % kRowBytes != 0 || g.k == 0 || !aligned16(g.a) || !aligned16(g.b) ||
+      g.lda * (int64_t)sizeof(T) % 16 != 0 || g.ldb * (int64_t)sizeof(T) % 16 != 0 || !aligned16(gamma) || !aligned16(beta) ||
+      !ring_operands_ok<T>(g) || !flat_norm_wins<T>(g))
+    return kNormNotTaken;
+  const NormRows<T> rows{(const T*)gamma, (const T*)beta, eps};
+  return gemm_fused_typed<T>(g, c, ldc, epilogue, args, s, &rows);
 }
 
 // Product + AddBiasLayerNorm.  The product reaches the normalisation in fp32 where it is short of rows or long in K
@@ -186,7 +208,10 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
   template int gemm_alpha_beta<T>(const void*, const void*, void*, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, \
                                   int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, float, float,           \
                                   hipStream_t);                                                                               \
-  template int gemm_fused_typed<T>(const GemmArgs&, void*, int64_t, int, const ttmi_epilogue_args*, hipStream_t);             \
+  template int gemm_fused_typed<T>(const GemmArgs&, void*, int64_t, int, const ttmi_epilogue_args*, hipStream_t,              \
+                                   const NormRows<T>*);                                                                       \
+  template int gemm_norm_fused_typed<T>(const GemmArgs&, const void*, const void*, float, void*, int64_t, int,                \
+                                        const ttmi_epilogue_args*, hipStream_t);                                              \
   template int gemm_bias_layer_norm_typed<T>(const void*, const void*, void*, const void*, const float*, const void*,         \
                                              const void*, const void*, float*, int64_t, int64_t, int64_t, float, int,         \
                                              hipStream_t);

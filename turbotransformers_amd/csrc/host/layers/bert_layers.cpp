@@ -171,10 +171,12 @@ void PositionwiseFeedForward::operator()(const Tensor& input_tensor, Tensor* out
   const int64_t m = input_tensor.numel() / model_dim;
   const DLDeviceType dev = input_tensor.device_type();
   const int id = input_tensor.device_id();
-  normed_.ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/LayerNorm/Reshape");
-  kernels::LayerNormFrom(input_tensor, layer_norm_weight_, layer_norm_bias_, &normed_, 1e-12f);
   hidden_.ReshapeAs(input_tensor.dtype(), {m, d_ff}, dev, id, "FFN/gemm0/Reshape");
-  GemmBiasAct(normed_, packed1_.Get(dense_weight_1_, is_trans_weight), d_ff, dense_bias_1_, TTMI_ACT_RELU, &hidden_);
+  ttmi_epilogue_args up{};
+  up.bias = dense_bias_1_.raw();
+  up.act = TTMI_ACT_RELU;
+  kernels::LayerNormGemm(input_tensor, layer_norm_weight_, layer_norm_bias_, 1e-12f, &normed_,
+                         packed1_.Get(dense_weight_1_, is_trans_weight), &hidden_, d_ff, TTMI_EPI_BIAS_ACT, up);
   output->ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/Reshape");
   // gemm1 + AddInputBias in one launch
   ttmi_epilogue_args args{};

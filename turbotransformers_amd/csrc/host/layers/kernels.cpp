@@ -181,15 +181,16 @@ void LayerNorm(const Tensor& gamma, const Tensor& beta, Tensor* out_tensor, T ep
 }
 template void LayerNorm<float>(const Tensor&, const Tensor&, Tensor*, float, const std::string);
 
-void LayerNormFrom(const Tensor& input, const Tensor& gamma, const Tensor& beta, Tensor* out_tensor, float eps) {
-  RequireGpu(*out_tensor, "LayerNorm");
-  const int64_t n = out_tensor->shape(-1), m = out_tensor->numel() / n;
-  TT_ENFORCE_EQ(input.numel(), m * n, "LayerNorm: input and output differ in size");
-  TT_ENFORCE_EQ(gamma.numel(), n, "LayerNorm gamma size mismatch");
-  TT_ENFORCE_EQ(beta.numel(), n, "LayerNorm beta size mismatch");
-  RequireSameDType(input, *out_tensor, "LayerNorm");
-  TT_DEVICE_CALL(ttmi_layer_norm_from(out_tensor->mutable_raw(), input.raw(), gamma.raw(), beta.raw(), m, n, eps,
-                                      DeviceDType(*out_tensor), Stream()));
+void LayerNormGemm(const Tensor& input, const Tensor& gamma, const Tensor& beta, float eps, Tensor* normed, const void* w_nk,
+                   Tensor* out, int64_t n, int epilogue, const ttmi_epilogue_args& args) {
+  RequireGpu(input, "LayerNorm");
+  const int64_t k = input.shape(-1), m = input.numel() / k;
+  TT_ENFORCE_EQ(gamma.numel(), k, "LayerNorm gamma size mismatch");
+  TT_ENFORCE_EQ(beta.numel(), k, "LayerNorm beta size mismatch");
+  normed->ReshapeAs(input.dtype(), {m, k}, input.device_type(), input.device_id(), "LayerNorm/Reshape");
+  TT_DEVICE_CALL(ttmi_layer_norm_gemm_fused(input.raw(), gamma.raw(), beta.raw(), eps, normed->mutable_raw(), w_nk,
+                                            out != nullptr ? out->mutable_raw() : nullptr, m, n, k, n, epilogue, &args,
+                                            DeviceDType(input), Stream()));
 }
 
 template <typename T>

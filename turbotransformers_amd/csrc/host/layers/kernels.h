@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "core/tensor.h"
+#include "ttmi.h"
 
 namespace turbo_transformers {
 namespace layers {
@@ -55,9 +56,9 @@ void ApplyMaskAndSoftmax(core::Tensor* inout, const core::Tensor& att_mask, floa
 template <typename T>
 void LayerNorm(const core::Tensor& gamma, const core::Tensor& beta, core::Tensor* out_tensor, T eps = 1e-12,
                const std::string name = "LayerNorm");
-// out = LayerNorm(input), out of place
-void LayerNormFrom(const core::Tensor& input, const core::Tensor& gamma, const core::Tensor& beta, core::Tensor* out_tensor,
-                   float eps);
+// ttmi_gemm_fused on LayerNorm(input), weights [n,k]; `normed` is scratch.  out may be null (QKV_SPLIT).
+void LayerNormGemm(const core::Tensor& input, const core::Tensor& gamma, const core::Tensor& beta, float eps, core::Tensor* normed,
+                   const void* w_nk, core::Tensor* out, int64_t n, int epilogue, const ttmi_epilogue_args& args);
 template <typename T>
 void AddBiasLayerNorm(const core::Tensor& input_tensor, const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor,
                       const core::Tensor& beta_tensor, core::Tensor* out_tensor, T eps = 1e-12,

@@ -208,13 +208,17 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
                "layer_cache[%s] must be [batch, heads, len, head_dim]", kv.first.c_str());
   }
 
-  const Tensor* q_in = &query_tensor;
-  if (pre_layernorm) {  // :66-80, :190-199 -- eps is 1e-6 there
-    TT_ENFORCE(!layernorm_gamma_.is_null() && !layernorm_beta_.is_null(), "pre_layernorm needs LayerNorm parameters");
-    ln_query_.ReshapeAs(query_tensor.dtype(), {batch, seq, hidden}, dev, dev_id, "self/layernorm/Reshape");
-    kernels::LayerNormFrom(query_tensor, layernorm_gamma_, layernorm_beta_, &ln_query_, 1e-6f);
-    q_in = &ln_query_;
-  }
+  if (pre_layernorm) TT_ENFORCE(!layernorm_gamma_.is_null() && !layernorm_beta_.is_null(), "pre_layernorm needs LayerNorm parameters");
+  // a projection of the query, with LayerNorm in front where asked for (:66-80, :190-199 -- eps is 1e-6 there)
+  auto project_query = [&](const void* packed_w, int64_t n, const ttmi_epilogue_args& args) {
+    if (pre_layernorm) {
+      kernels::LayerNormGemm(query_tensor, layernorm_gamma_, layernorm_beta_, 1e-6f, &ln_query_, packed_w, nullptr, n,
+                             TTMI_EPI_QKV_SPLIT, args);
+    } else {
+      TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), packed_w, nullptr, batch * seq, n, hidden, hidden, hidden, n,
+                                     TTMI_EPI_QKV_SPLIT, &args, dt, Stream()));
+    }
+  };
 
   const Tensor* k_used = &k_;
   const Tensor* v_used = &v_;
@@ -265,8 +269,7 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
     args.heads = heads;
     args.head_dim = d;
     args.v_seq_pitch = v_pitch;
-    TT_DEVICE_CALL(ttmi_gemm_fused(q_in->raw(), qkv_packed_.Get(qkv_weight_, is_trans_weight), nullptr, batch * seq, 3 * hidden,
-                                   hidden, hidden, hidden, 3 * hidden, TTMI_EPI_QKV_SPLIT, &args, dt, Stream()));
+    project_query(qkv_packed_.Get(qkv_weight_, is_trans_weight), 3 * hidden, args);
     // decoder self attention: earlier keys/values come first (:205-214), the grown tensors go back (:216-229)
     auto prepend = [&](const char* key, Tensor* cur, Tensor* grown, const char* name) {
       if (!CacheHas(layer_cache, key)) return;
@@ -298,7 +301,14 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
   } else {
     TT_ENFORCE(!q_weight_.is_null() && !k_weight_.is_null() && !v_weight_.is_null() && !q_bias_.is_null() && !k_bias_.is_null() &&
                    !v_bias_.is_null(), "context attention needs the separate q/k/v weights and biases");
-    ProjectToHeads(*q_in, q_packed_.Get(q_weight_, is_trans_weight), q_bias_, heads, &q_, "context/AddBiasTransposeForScore/q_out2/Reshape");
+    q_.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "context/AddBiasTransposeForScore/q_out2/Reshape");
+    ttmi_epilogue_args args{};
+    args.bias = q_bias_.raw();
+    args.q = q_.mutable_raw();
+    args.seq = seq;
+    args.heads = heads;
+    args.head_dim = d;
+    project_query(q_packed_.Get(q_weight_, is_trans_weight), hidden, args);
     if (CacheHas(layer_cache, "memory_keys") && CacheHas(layer_cache, "memory_values")) {
       // the encoder memory was projected at an earlier step (:90-105); used in place, no copy
       k_used = layer_cache.at("memory_keys");
