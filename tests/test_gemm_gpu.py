@@ -931,6 +931,32 @@ def test_fused_attention_packed_batch(ttmi, oracle, attention_waves, dt, v_trans
     assert max_abs(host(out), want) <= GEMM_TOL[dt] * 2
 
 
+@pytest.mark.parametrize("dt", ["f16", "f32"])
+@pytest.mark.parametrize("B,h,longest", [(64, 5, 40), (65, 4, 300), (130, 3, 7), (22, 12, 260)])
+def test_packed_attention_of_many_sequences(ttmi, dt, B, h, longest):
+    """More workgroups than CUs start in the order of the lengths: equal lengths, empty sequences, one more than the 64 that are
+    ordered together, one and several blocks of queries.  Every sequence against fp64."""
+    rng = np.random.default_rng(B)
+    d, lens = 64, rng.integers(0, longest + 1, B)
+    lens[rng.integers(B)] = longest
+    lens[:5] = lens[5]
+    Q, K, V = (rng.standard_normal((B, h, longest, d), np.float32) for _ in range(3))
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    out = torch.full((int(cu[-1]), h * d), 9.0, dtype=dev(Q[:1], dt).dtype, device="cuda")
+    dQ, dK, dV, dcu = dev(Q, dt), dev(K, dt), dev(V, dt), dev(cu)
+    ok(ttmi.ttmi_fused_attention(ptr(dQ), ptr(dK), ptr(dV), None, ptr(out), ptr(dcu), B, h, longest, d, 0, 0.125, TTMI_DTYPES[dt],
+                                 stream()))
+    got = host(out)
+    Q, K, V = (rounded(x, dt).astype(np.float64) for x in (Q, K, V))
+    for b, n in enumerate(lens):
+        if n == 0:
+            continue
+        score = Q[b, :, :n] @ K[b, :, :n].transpose(0, 2, 1) * 0.125
+        prob = np.exp(score - score.max(-1, keepdims=True))
+        want = (prob / prob.sum(-1, keepdims=True)) @ V[b, :, :n]
+        assert max_abs(got[cu[b]:cu[b + 1]], want.transpose(1, 0, 2).reshape(n, h * d)) <= GEMM_TOL[dt] * 2
+
+
 @pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("M,h,steps", [(1, 1, 1), (16, 1, 16), (17, 12, 12), (33, 3, 17), (8, 12, 24), (31, 4, 32), (40, 2, 33)])
 def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps):

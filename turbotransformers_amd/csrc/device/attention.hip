@@ -217,14 +217,24 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, lhalf = lane >> 5;
-  const int bh = blockIdx.y, b = bh / heads, head = bh - b * heads;
-  const int q0 = blockIdx.x * kBQ + wave * 32;
+  // A packed batch: one row of workgroups, sequence by sequence and there block by block, all heads of a block side by side
+  // (the workgroups of an XCD are then a mixture of first and last blocks).  See longest_first().
+  int b = blockIdx.y / heads, head = blockIdx.y - b * heads, block = blockIdx.x;
+  if (PACKED) {
+    const int blocks = (seq + kBQ - 1) / kBQ;
+    b = blockIdx.x / (blocks * heads);
+    block = (blockIdx.x - b * (blocks * heads)) / heads;
+    head = blockIdx.x - (b * blocks + block) * heads;
+    if (gridDim.x > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, gridDim.x / (blocks * heads), b, seq));
+  }
+  const int bh = b * heads + head;
+  const int q0 = block * kBQ + wave * 32;
 
   int kv_len = seq, out_row0 = b * seq;
   if (PACKED) {
     kv_len = cu[b + 1] - cu[b];
     out_row0 = cu[b];
-    if ((int)blockIdx.x * kBQ >= kv_len) return;  // whole workgroup is padding
+    if (block * kBQ >= kv_len) return;  // whole workgroup is padding
   }
   const int q_len = kv_len;  // self attention: as many queries as keys
 
@@ -418,7 +428,11 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;
   }
-  const dim3 grid((unsigned)ceil_div(seq, nw * 32), (unsigned)(batch * heads));
+  dim3 grid((unsigned)ceil_div(seq, nw * 32), (unsigned)(batch * heads));
+  if (cu_seqlens != nullptr) {  // one row of workgroups, see the kernel
+    TTMI_REQUIRE((int64_t)grid.x * grid.y < (1ll << 31), "attention grid too large");
+    grid = dim3(grid.x * grid.y);
+  }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == TTMI_F32) {
