@@ -262,6 +262,10 @@ TTMI_API int ttmi_fill_f32(float* data, int64_t n, float value, void* stream);
 TTMI_API int ttmi_sequence_rows_i64(int64_t* data, int64_t rows, int64_t cols, void* stream);
 /* dst[i] = -10000 * (1 - src[i]) */
 TTMI_API int ttmi_mask_transform(const int64_t* src, float* dst, int64_t n, void* stream);
+/* PrepareBertMasks (layers/prepare_bert_masks.cpp) in one launch: positions[r, c] = c, zeros = 0 and ones = 1 over rows x cols,
+ * each unless NULL; ext[i] = -10000 * (1 - mask[i]) for i < mask_size, or of a mask of rows x cols ones where mask is NULL. */
+TTMI_API int ttmi_prepare_masks(const int64_t* mask, int64_t* ones, int64_t* positions, int64_t* zeros, float* ext, int64_t rows,
+                                int64_t cols, int64_t mask_size, void* stream);
 
 /* kernels::SeqPool  (layers/kernels/seq_pool.cpp:124-155): in[B,S,H] -> out[B,H];
  * pool_type 0 = max, 1 = mean, 2 = first, 3 = last (layers/types.h PoolType order). */

@@ -292,6 +292,27 @@ def test_bert_embedding_fused(ttmi, oracle, dt, hidden):
     assert max_abs(host(out), want) <= {"f32": 5e-5, "f16": 3e-2, "bf16": 2.5e-1}[dt]
 
 
+@pytest.mark.parametrize("B,S", [(1, 1), (3, 85), (2, 128), (40, 300)])
+@pytest.mark.parametrize("given", [True, False])
+def test_prepare_masks_in_one_launch(ttmi, oracle, B, S, given):
+    """Every output, and each left alone that is not asked for; a mask of another size than the batch; one and many workgroups."""
+    mask = np.random.default_rng(B + S).integers(0, 2, (B, S)) if given else None
+    ones, pos, zeros = (torch.full((B * S + 1,), 7, dtype=torch.int64, device="cuda") for _ in range(3))
+    ext = torch.full((B * S + 1,), 7.0, device="cuda")
+    dmask = dev(mask) if given else None
+    ok(ttmi.ttmi_prepare_masks(ptr(dmask) if given else None, None if given else ptr(ones), ptr(pos), ptr(zeros), ptr(ext), B, S, B * S,
+                               stream()))
+    want_mask, want_type, want_pos, want_ext = oracle.prepare_bert_masks(B, S, att_mask=mask) if given else oracle.prepare_bert_masks(B, S)
+    for got, want in ((pos, want_pos), (zeros, want_type), (ext, want_ext)) + (() if given else ((ones, want_mask),)):
+        assert np.array_equal(host(got[:-1]), np.asarray(want).reshape(-1)) and float(got[-1]) == 7
+    if given:
+        assert torch.all(ones == 7)
+        other = torch.full((B * S + 4,), 7.0, device="cuda")
+        ok(ttmi.ttmi_prepare_masks(ptr(torch.zeros(B * S + 3, dtype=torch.int64, device="cuda")), None, None, None, ptr(other), B, S,
+                                   B * S + 3, stream()))
+        assert torch.all(other[:-1] == -10000.0) and float(other[-1]) == 7
+
+
 def test_prepare_bert_masks_helpers(ttmi, oracle):
     B, S = 3, 17
     rng = np.random.default_rng(0)

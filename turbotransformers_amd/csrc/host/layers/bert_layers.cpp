@@ -124,21 +124,14 @@ void PrepareBertMasks::operator()(const Tensor& inputs, Tensor* att_mask, Tensor
   const int64_t B = inputs.shape(0), S = inputs.shape(1);
   const DLDeviceType dev = inputs.device_type();
   const int id = inputs.device_id();
-  if (position_ids->is_null()) {
-    auto* p = position_ids->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/possitionids/Reshape");
-    kernels::common::Sequence(p, B, S, dev);
-  }
-  if (seq_type->is_null()) {
-    auto* p = seq_type->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/seqids/Reshape");
-    kernels::common::Fill<int64_t>(p, B * S, 0, dev);
-  }
-  if (att_mask->is_null()) {
-    auto* p = att_mask->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/attmask/Reshape");
-    kernels::common::Fill<int64_t>(p, B * S, 1, dev);
-  }
+  int64_t *positions = nullptr, *zeros = nullptr, *ones = nullptr;
+  if (position_ids->is_null()) positions = position_ids->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/possitionids/Reshape");
+  if (seq_type->is_null()) zeros = seq_type->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/seqids/Reshape");
+  if (att_mask->is_null()) ones = att_mask->Reshape<int64_t>({B, S}, dev, id, "PrepareBertMasks/attmask/Reshape");
   auto* ext = extended_attention_mask->Reshape<float>({att_mask->shape(0), 1, 1, att_mask->shape(1)}, dev, id,
                                                       "PrepareBertMasks/extendedattnmask/Reshape");
-  kernels::common::Transform(att_mask->mutableData<int64_t>(), ext, att_mask->numel(), dev);
+  TT_DEVICE_CALL(ttmi_prepare_masks(ones != nullptr ? nullptr : att_mask->data<int64_t>(), ones, positions, zeros, ext, B, S,
+                                    att_mask->numel(), Stream()));
 }
 
 // -------------------------------------------------------------------------- pooling -----
