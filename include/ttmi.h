@@ -356,7 +356,8 @@ typedef struct ttmi_epilogue_args {
   void* q; void* k; void* v; /* outputs [B,h,S,d]                   (QKV_SPLIT[_PAD])        */
   int64_t seq;               /* S (or max_seq for the padded form)                          */
   int64_t heads;             /* h                                                           */
-  int64_t head_dim;          /* d; N must equal 3*h*d, or h*d: then only q is written -- MatMul +
+  int64_t head_dim;          /* d; N must equal 3*h*d; 2*h*d: q and k are written, two projections of
+                                the same rows; or h*d: only q is written -- MatMul +
                                 AddBiasTransposeForScore of one projection
                                 (layers/multi_headed_attention.cpp:73-88)                   */
   const int32_t* token_rows; /* device [M]: packed token -> b*max_seq+s (QKV_SPLIT_PAD)      */

@@ -578,6 +578,27 @@ def test_fused_single_projection_to_heads(ttmi, oracle, dt, B, S, h, d):
 
 
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("B,S,h,d", [(1, 1, 2, 64), (2, 11, 3, 64), (8, 100, 12, 64), (33, 200, 12, 64), (2, 5, 3, 20)])
+def test_fused_two_projections_to_heads(ttmi, oracle, dt, B, S, h, d):
+    """Keys and values of one memory: N = 2*h*d, q and k are written, nothing past them."""
+    import ctypes
+    rng = np.random.default_rng(S * 7 + h)
+    H = h * d
+    A, W = _ab(rng, B * S, 2 * H, H, 1)
+    bias = rng.standard_normal(2 * H).astype(np.float32)
+    dA, dW, db = dev(A, dt), dev(W, dt), dev(bias, dt)
+    q, k = (torch.full((B + 1, h, S, d), -7.0, dtype=dA.dtype, device="cuda") for _ in range(2))
+    args = _epi(bias=db, q=q, k=k, seq=S, heads=h, head_dim=d)
+    ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(dW), None, B * S, 2 * H, H, H, H, 2 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args),
+                            TTMI_DTYPES[dt], stream()))
+    proj = oracle.matmul(rounded(A, dt), rounded(W, dt), True)
+    for got, part in ((q, slice(0, H)), (k, slice(H, 2 * H))):
+        want = oracle.add_bias_transpose_for_score(np.ascontiguousarray(proj[:, part]), rounded(bias, dt)[part], B, S, h, d)
+        assert max_abs(host(got[:B]), want) <= GEMM_TOL[dt] * 2
+        assert torch.all(got[B] == -7.0)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("v_transposed", [False, True])
 @pytest.mark.parametrize("lens", [[9, 30, 1, 17], [64, 8, 200, 16, 33]])
 def test_fused_qkv_split_pad(ttmi, oracle, dt, lens, v_transposed):

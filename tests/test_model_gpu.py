@@ -805,6 +805,28 @@ def test_multi_headed_attention_context_memory_cache(tt, oracle):
     assert np.isfinite(host(out2)).all()
 
 
+@pytest.mark.parametrize("T", [1, 9, 130])
+def test_multi_headed_attention_one_memory_for_keys_and_values(tt, T):
+    """Keys and values of the same tensor take one product, of two tensors two: the same cache and output, also after the bias
+    was changed in place."""
+    B, F, H, h = 3, 2, 256, 4
+    mod, ln, layer = _make_mha(tt, h, H, seed=11)
+    g = torch.Generator().manual_seed(T)
+    memory, query = torch.randn(B, T, H, generator=g).cuda(), torch.randn(B, F, H, generator=g).cuda()
+    for _ in range(2):
+        results = []
+        for value in (memory, memory.clone()):
+            cache = {"memory_keys": None, "memory_values": None, "self_keys": None, "self_values": None}
+            out, _ = layer(memory, value, query, layer_cache=cache, attn_type="context")
+            results.append([host(t).copy() for t in (out, cache["memory_keys"], cache["memory_values"])])
+        for one, two in zip(*results):
+            assert max_abs(one, two) < 2e-5  # fp32 sums of 256 products in another order
+        with torch.no_grad():
+            for p in mod.parameters():
+                if p.dim() == 1:
+                    p.add_(0.25)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_multi_headed_attention_half_precision(tt, oracle, dtype):
     B, F, T, H, h = 2, 16, 24, 256, 4

@@ -91,9 +91,9 @@ class MultiHeadedAttention {
   core::Tensor layernorm_gamma_, layernorm_beta_;
   int64_t num_attention_heads_;
 
-  PackedWeight qkv_packed_, dense_packed_, q_packed_, k_packed_, v_packed_;
+  PackedWeight qkv_packed_, dense_packed_, q_packed_, k_packed_, v_packed_, kv_packed_;
   // Per-call intermediates, reused across calls (Reshape keeps a buffer that is large enough).
-  mutable core::Tensor q_, k_, v_, k_grown_, v_grown_, ctx_, score_scratch_, ln_query_;
+  mutable core::Tensor q_, k_, v_, k_grown_, v_grown_, kv_bias_, ctx_, score_scratch_, ln_query_;
   mutable std::mutex mutex_;  // the layer keeps per-call state, like the reference (…attention.cpp:32,272)
 };
 
