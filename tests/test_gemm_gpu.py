@@ -953,7 +953,7 @@ def test_fused_attention_packed_batch(ttmi, oracle, attention_waves, dt, v_trans
 
 
 @pytest.mark.parametrize("dt", ["f16", "f32"])
-@pytest.mark.parametrize("B,h,longest", [(64, 5, 40), (65, 4, 300), (130, 3, 7), (22, 12, 260)])
+@pytest.mark.parametrize("B,h,longest", [(64, 5, 140), (65, 4, 300), (130, 3, 129), (22, 12, 260), (90, 4, 128)])
 def test_packed_attention_of_many_sequences(ttmi, dt, B, h, longest):
     """More workgroups than CUs start in the order of the lengths: equal lengths, empty sequences, one more than the 64 that are
     ordered together, one and several blocks of queries.  Every sequence against fp64."""

@@ -217,16 +217,12 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 31, lhalf = lane >> 5;
-  // A packed batch: one row of workgroups, sequence by sequence and there block by block, all heads of a block side by side
-  // (the workgroups of an XCD are then a mixture of first and last blocks).  See longest_first().
-  int b = blockIdx.y / heads, head = blockIdx.y - b * heads, block = blockIdx.x;
-  if (PACKED) {
-    const int blocks = (seq + kBQ - 1) / kBQ;
-    b = blockIdx.x / (blocks * heads);
-    block = (blockIdx.x - b * (blocks * heads)) / heads;
-    head = blockIdx.x - (b * blocks + block) * heads;
-    if (gridDim.x > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, gridDim.x / (blocks * heads), b, seq));
-  }
+  // A packed batch: sequence by sequence (y) and there block by block, all heads of a block side by side (x; the workgroups of
+  // an XCD are then a mixture of first and last blocks).  See longest_first().
+  const int major = (PACKED ? blockIdx.x : blockIdx.y) / heads, head = (PACKED ? blockIdx.x : blockIdx.y) - major * heads;
+  const int block = PACKED ? major : blockIdx.x;
+  int b = PACKED ? blockIdx.y : major;
+  if (PACKED && seq > kOrderMinLength && gridDim.x * gridDim.y > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, gridDim.y, b, seq));
   const int bh = b * heads + head;
   const int q0 = block * kBQ + wave * 32;
 
@@ -429,9 +425,9 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
     return rc;
   }
   dim3 grid((unsigned)ceil_div(seq, nw * 32), (unsigned)(batch * heads));
-  if (cu_seqlens != nullptr) {  // one row of workgroups, see the kernel
+  if (cu_seqlens != nullptr) {  // blocks and heads in one row, see the kernel
     TTMI_REQUIRE((int64_t)grid.x * grid.y < (1ll << 31), "attention grid too large");
-    grid = dim3(grid.x * grid.y);
+    grid = dim3((unsigned)(grid.x * heads), (unsigned)batch);
   }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;

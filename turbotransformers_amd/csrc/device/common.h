@@ -133,8 +133,10 @@ __device__ __forceinline__ float group_max(float v) {
 // and those of a batch of ordinary size are all resident at once, so what a CU gets besides its first workgroup is given by
 // that order: with the lengths in the caller's order some get two long ones, others none.  us per attention launch, 12 heads,
 // as given / longest first: 20 requests of 5 to 500 tokens fp16 23.8 / 20.4, fp32 146 / 105; 32 of 20 to 512 fp16 32.6 / 26.1;
-// 32 of 5 to 200 fp16 11.2 / 9.5.  Where every workgroup has a CU of its own there is nothing to gain and 0.4 us to lose.
+// 32 of 5 to 200 fp16 11.2 / 9.5.  Where every workgroup has a CU of its own, or none has more than
+// two tiles of keys, there is nothing to gain and 0.35 us to lose (fp16, 30 requests of 5 to 60 tokens).
 constexpr unsigned kOrderMinWorkgroups = 256;
+constexpr int kOrderMinLength = 128;
 // The sequence of a packed batch that comes `rank`-th when they are ordered by length, longest first (ties: by index).  Lane i
 // holds the length of sequence i; the length of that rank is found bit by bit, which takes a ballot per bit of `longest` (an
 // upper bound of the lengths).  Batches of more than 64 sequences are ordered 64 at a time.  `rank` is uniform.
