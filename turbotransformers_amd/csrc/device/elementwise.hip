@@ -271,7 +271,7 @@ __global__ void mask_transform_kernel(const int64_t* src, float* dst, int64_t n)
   for (; i < n; i += stride) dst[i] = -10000.0f * (float)(1 - src[i]);  // common.cpp:80
 }
 // What PrepareBertMasks makes of a batch, each where wanted, in one launch: a forward of a few tokens is as long as its
-// launches, and four of them for a few KB are four waits (fp32 1 x 128: 611 us per forward before, 606 after; 10 tokens fp16 336, 332).
+// launches, and four of them for a few KB are four waits (fp32 1 x 128 with FFN1 in one launch: 611 us per forward before, 606 after; 10 tokens fp16 336, 332).
 __global__ void prepare_masks_kernel(const int64_t* src, int64_t* ones, int64_t* positions, int64_t* zeros, float* ext, int64_t n,
                                      int64_t ext_n, int64_t cols) {
   int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;

@@ -515,7 +515,7 @@ struct RingTiles<1> {
 };
 #undef TTMI_RING_ROW
 
-enum class RingUse { kWhole, kSliced, kLayerNorm };  // never cut along K / cut where it pays / slices summed by the LayerNorm
+enum class RingUse { kWhole, kSliced, kCut, kLayerNorm };  // never cut along K / cut where it pays / always cut / slices summed by the LayerNorm
 struct RingPlan {
   int tile = -1, slices = 1;
   int64_t rounds = 0;  // workgroups per CU, rounded up
@@ -531,13 +531,13 @@ inline RingPlan pick_ring(int64_t m, int64_t n, int64_t ksteps, RingUse use, int
     const int i = index++;
     if (column_limit > 0 && column_limit % t.wave_cols != 0) continue;
     const int most = use == RingUse::kWhole ? 1 : (int)std::min<int64_t>(16, std::max<int64_t>(1, ksteps / 4));
-    for (int slices = 1; slices <= most; ++slices) {
+    for (int slices = use == RingUse::kCut ? 2 : 1; slices <= most; ++slices) {
       if (slices > 1 && slices * m * n * 4 > (32ll << 20)) break;
       const int64_t q = ceil_div(ceil_div(m, t.bm) * ceil_div(n, t.bn) * slices, compute_units());
       double us = t.first + t.again * (q - 1) + ceil_div(ksteps, slices) * std::max<double>(t.lone * ceil_div(q, t.resident), t.shared * q);
       // partial products: written and read once more, and a launch of their own where no LayerNorm follows
       if (slices > 1 || use == RingUse::kLayerNorm) us += slices * m * n * 4 / 4e6;
-      if (slices > 1 && use == RingUse::kSliced) us += 4.0;
+      if (slices > 1 && use != RingUse::kLayerNorm) us += 4.0;
       if (us < best.us) best = RingPlan{i, slices, q, us};
     }
   }
