@@ -323,6 +323,7 @@ TTMI_API int ttmi_gemm_batched_heads(const void* a, const void* b, void* c, int6
 /* Self-attention core in one kernel, for head_dim 64 and fp16/bf16/fp32:
  *   out[b, s, head*64 + :] = softmax(scale * q[b,head,s,:] k[b,head]^T + mask[b,:]) v[b,head]
  * q,k,v are [B,h,S,64]; `mask` is an additive fp32 [B,S] key mask or NULL; `out` is [B,S,h*64].
+ * A sequence that a finite mask covers wholly (the lowest float included) is the mean of its values.
  * It replaces BatchMatMul + ApplyMaskAndSoftmax + BatchMatMul + TransposeForScore
  * (layers/multi_headed_attention.cpp:323-354) when the [B,h,S,S] probabilities are not an
  * output: the score tensor never reaches HBM.  With `cu_seqlens` (device int32 [B+1]) q,k,v are

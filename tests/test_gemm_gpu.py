@@ -871,6 +871,40 @@ def test_attention_with_split_keys(ttmi, oracle, dt, S):
     assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
 
 
+LOWEST = float(np.finfo(np.float32).min)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("form,v_transposed", [(-1, False), (-1, True), (8, False), (8, True), (1, True)])
+@pytest.mark.parametrize("S", [1, 33, 70, 200, 300])
+def test_attention_masks_far_from_zero(ttmi, oracle, dt, form, v_transposed, S):
+    """Additive masks of the lowest float, of -inf and of ordinary large sizes: a wholly masked sequence is the mean of V
+    (its scores vanish against the mask), a partly masked one is not changed by its masked keys, wherever the first
+    unmasked key lies.  Every form of the one-kernel attention."""
+    rng = np.random.default_rng(S)
+    h, d = 2, 64
+    rows = [np.full(S, x) for x in (LOWEST, -1e9, -1e11, -1e20, -1e37)]   # wholly masked
+    rows += [np.where(np.arange(S) < S - 1, x, 0.0) for x in (LOWEST, -np.inf, -1e11)]      # only the last key is seen
+    rows += [np.where(np.arange(S) >= (S + 1) // 2, x, 0.0) for x in (LOWEST, -np.inf)]
+    rows += [np.where(np.arange(S) % 2 == 1, -np.inf, LOWEST), np.where(np.arange(S) == S // 2, 1e12, 0.0)]
+    mask = np.stack(rows).astype(np.float32)
+    B = len(rows)
+    Q, K, V = (rng.standard_normal((B, h, S, d), np.float32) for _ in range(3))
+    dV, pitch = _v_operand(V, dt, v_transposed)
+    out = torch.full((B, S, h * d), 9.0, dtype=dV.dtype, device="cuda")
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", form))
+    try:
+        ok(ttmi.ttmi_fused_attention(ptr(dev(Q, dt)), ptr(dev(K, dt)), ptr(dV), ptr(dev(mask)), ptr(out), None, B, h, S, d, pitch,
+                                     0.125, TTMI_DTYPES[dt], stream()))
+    finally:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+    score = oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125)
+    prob = oracle.apply_mask_and_softmax(score, mask.reshape(B, 1, 1, S), 1.0, True)
+    assert max_abs(prob[0], np.full_like(prob[0], 1.0 / S)) < 1e-6
+    want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, S, h * d)
+    assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("F,past,fresh,per_query", [(1, 0, 1, False), (33, 0, 33, True), (1, 40, 1, False), (1, 127, 1, True),
                                                     (5, 124, 5, True), (64, 0, 256, False), (2, 255, 2, True), (31, 300, 212, False)])

@@ -52,6 +52,21 @@ def test_bert_embeddings_vs_huggingface(tt):
     assert max_abs(host(got), host(want)) < 1e-5  # bert_embedding_test.py:76-77
 
 
+@pytest.mark.parametrize("B,S", [(2, 200), (3, 40), (1, 129), (20, 130)])
+def test_bert_attention_with_a_wholly_masked_sequence(tt, oracle, B, S):
+    """The caller's own mask of the lowest float over one whole batch entry: its context is the mean of V on every route
+    (dense fp32 batches of all sizes take a one-kernel attention), not 0 / 0."""
+    model, cfg = _hf_bert(1)
+    layer = model.encoder.layer[0]
+    attn = tt.BertAttention.from_torch(layer.attention)
+    x = torch.rand(B, S, cfg.hidden_size, device="cuda")
+    ext = torch.zeros(B, 1, 1, S, device="cuda")
+    ext[0] = torch.finfo(torch.float32).min
+    want, _ = oracle.bert_attention(host(x), host(ext), oracle_layer_weights({k: v.detach().cpu().numpy() for k, v in layer.named_parameters()}),
+                                    cfg.num_attention_heads)
+    assert max_abs(host(attn(x, ext)[0]), want) < 1e-4
+
+
 @pytest.mark.parametrize("B,S", [(1, 10), (2, 40), (4, 128)])
 def test_bert_attention_vs_huggingface(tt, B, S):
     model, cfg = _hf_bert(1, seed=B)

@@ -26,7 +26,7 @@
 // scale*log2(e) is applied inside the exp2 argument, so no separate scale/mask pass exists.
 #include <cstdlib>
 
-#include "common.h"
+#include "attention_common.h"
 
 namespace ttmi {
 
@@ -86,7 +86,6 @@ __device__ __forceinline__ float add_pair<bf16>(uint32_t p, float acc) {
 
 constexpr int kD = 64;          // head dim
 constexpr int kBKV = 64;        // keys per LDS tile
-constexpr float kNegBig = -1.0e30f;
 // log2 of the largest probability tolerated before the running maximum is moved.  bf16 keeps the
 // exact maximum: with 8 mantissa bits a dominant probability of exactly 1.0 is worth keeping exact.
 template <typename T>
@@ -145,7 +144,7 @@ __device__ __forceinline__ void attention_tile(const char* kt, const char* vt, c
 #pragma unroll
         for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
     }
-    const float neg_m = -m_run * scale_log2e;
+    const float neg_m = relative_scores(st, m_run, scale_log2e);
     Chunk16 pf[2];
     float psum = 0.f;
 #pragma unroll
@@ -254,11 +253,11 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int e = 0; e < 16; ++e) ot[t][e] = 0.f;
-  float m_run = kNegBig, l_run = 0.f;
+  float m_run = -kFarthestScore, l_run = 0.f;
 
   // K/V tiles are register-staged: the global loads of tile t+1 are issued before the MFMAs of
   // tile t and written to the other LDS stage afterwards, so their latency hides behind compute.
-  // Loads past the last key are clamped to valid memory: such keys carry a -1e30 mask, so a
+  // Loads past the last key are clamped to valid memory: such keys carry a mask of -inf, so a
   // duplicated K row is harmless; V^T columns past the last key may be uninitialised memory and
   // are zeroed on the way to LDS (0 * NaN would poison the output).
   // (Named vector registers, not arrays: an array captured by the two lambdas ends up in scratch.)
@@ -286,8 +285,8 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
     }
     if (tid < kBKV) {
       const int key = key0 + tid;
-      const float mv = mask ? mask[(int64_t)b * seq + min(key, kv_len - 1)] * inv_scale : 0.f;
-      mreg = key < kv_len ? mv : kNegBig;
+      const float mv = mask ? mask_in_scores(mask[(int64_t)b * seq + min(key, kv_len - 1)], inv_scale) : 0.f;
+      mreg = key < kv_len ? mv : -__builtin_inff();
     }
   };
   auto put_vt = [&](u32x4 x, int tile, int stage, int drow, int ch) {

@@ -24,7 +24,7 @@
 #include <mutex>
 #include <set>
 
-#include "common.h"
+#include "attention_common.h"
 
 namespace ttmi {
 
@@ -36,7 +36,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
 constexpr int kD = 64;           // head dim
 constexpr int kBKV = 64;         // keys per LDS tile
 constexpr int kRow = 256;        // bytes of a K row (64 floats) and of a V^T row (64 keys)
-constexpr float kNegBig = -1.0e30f;
 
 // four K indices of both operands, one per instruction
 __device__ __forceinline__ floatx16 mma4(const floatx4& a, const floatx4& b, floatx16 c) {
@@ -106,7 +105,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int e = 0; e < 16; ++e) ot[t][e] = 0.f;
-  float m_run = kNegBig, l_run = 0.f;
+  float m_run = -kFarthestScore, l_run = 0.f;
 
   // tile staging: thread -> (row r0 + 64*NW/16*p, chunk ch); global -> registers one tile ahead -> LDS
   constexpr int kRowsPerPass = NW * 64 / 16;
@@ -129,8 +128,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     }                                                                                                               \
     if (tid < kBKV) {                                                                                               \
       const int key_ = key0_ + tid;                                                                                 \
-      const float mv_ = mask ? mask[(int64_t)b * seq + min(key_, kv_len - 1)] * inv_scale : 0.f;                    \
-      mreg = key_ < kv_len ? mv_ : kNegBig;                                                                         \
+      const float mv_ = mask ? mask_in_scores(mask[(int64_t)b * seq + min(key_, kv_len - 1)], inv_scale) : 0.f;     \
+      mreg = key_ < kv_len ? mv_ : -__builtin_inff();                                                               \
     }                                                                                                               \
   } while (0)
 
@@ -198,7 +197,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
           for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
       }
-      const float neg_m = -m_run * scale_log2e;
+      const float neg_m = relative_scores(st, m_run, scale_log2e);
       float psum = 0.f;
 #pragma unroll
       for (int e = 0; e < 16; ++e) {

@@ -13,7 +13,7 @@
 // is the launch, 1 the first loads; fp32 then runs 64 matrix instructions of 64 cycles in a chain per block of keys).
 #include <type_traits>
 
-#include "common.h"
+#include "attention_common.h"
 
 namespace ttmi {
 namespace {
@@ -30,7 +30,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
 
 constexpr int kD = 64;            // head dim
 constexpr int kQ = 32, kKeys = 32;  // queries per workgroup, keys per block
-constexpr float kNegBig = -1.0e30f;
 
 // D = A B + C over one 16-byte piece of both operands
 template <typename T>
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     float mk;  // of key lrow
   };
   const int blocks = (seq + kKeys - 1) / kKeys;
-  // Keys past the end repeat valid ones; they carry a mask of -1e30, so their probability is 0.
+  // Keys past the end repeat valid ones; they carry a mask of -inf, so their probability is 0.
   auto load = [&](int blk, Block& x) __attribute__((always_inline)) {
     const int key0 = blk * kKeys;
     const T* row = kb + (int64_t)min(key0 + lrow, seq - 1) * kD + lhalf * KPC;
@@ -128,7 +127,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   for (int t = 0; t < 2; ++t)
 #pragma unroll
     for (int e = 0; e < 16; ++e) ot[t][e] = 0.f;
-  float m_run = kNegBig, l_run = 0.f;
+  float m_run = -kFarthestScore, l_run = 0.f;
 
   auto compute = [&](int blk, Block& x) __attribute__((always_inline)) {
     const int key0 = blk * kKeys;
@@ -138,7 +137,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 #pragma unroll
     for (int e = 0; e < 16; ++e) st[e] = 0.f;
     {
-      const float mk = key0 + lrow < seq ? x.mk * inv_scale : kNegBig;
+      const float mk = key0 + lrow < seq ? mask_in_scores(x.mk, inv_scale) : -__builtin_inff();
       st = __builtin_amdgcn_mfma_f32_32x32x2f32(lhalf == 0 ? mk : 0.f, 1.f, st, 0, 0, 0);
     }
     if (ragged) {  // V^T past the last key may hold anything: 0 * NaN would reach the output
@@ -171,7 +170,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
-    const float neg_m = -m_run * scale_log2e;
+    const float neg_m = relative_scores(st, m_run, scale_log2e);
     float psum = 0.f;
     if constexpr (sizeof(T) == 2) {
       u32x4 pf[2];
@@ -233,7 +232,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   __syncthreads();
   constexpr int EPT = kQ * kD / (NW * 64);  // output elements per thread: 8 or 4
   const int qi = tid / (kD / EPT), d0 = (tid % (kD / EPT)) * EPT;
-  float m = kNegBig;
+  float m = -kFarthestScore;
 #pragma unroll
   for (int w = 0; w < NW; ++w) m = fmaxf(m, stat[0][w][qi]);
   float l = 0.f, o[EPT];
@@ -241,7 +240,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   for (int e = 0; e < EPT; ++e) o[e] = 0.f;
 #pragma unroll
   for (int w = 0; w < NW; ++w) {
-    const float f = __builtin_amdgcn_exp2f((stat[0][w][qi] - m) * scale_log2e);  // a share without keys: 2^-huge = 0
+    const float f = __builtin_amdgcn_exp2f((stat[0][w][qi] - m) * scale_log2e);  // a share without keys has no sum
     l += f * stat[1][w][qi];
 #pragma unroll
     for (int e = 0; e < EPT; e += 4) {
