@@ -320,3 +320,29 @@ def test_fp32_products_pick_tiles_by_rounds_over_the_compute_units():
     assert variant(1600, 768, 768, capi.F32) == "reg4w_64x64"          # K too short for the cut to pay
     assert variant(32768, 3072, 768, capi.F32) == "dma8w_256x256"
     assert variant(128, 768, 3072, capi.F32) == "reg4w_64x64_splitk10"  # one short sequence: as before
+
+
+def test_fused_products_off_the_ring_keep_the_kernels_for_their_size():
+    """Widths that are no multiple of eight (vocabulary- and class-sized heads), operands of 2 GiB and more and heads that no
+    16-byte store fits are refused by the ring tiles; they then run on the DMA tiles, the wavefront kernel or K slices that
+    their size calls for, not all on the register-staged tiles."""
+    import ctypes
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+
+    def variant(m, n, k, dt, epi=capi.EPI_BIAS, args=None):
+        capi.check(lib.ttmi_gemm_describe(m, n, k, epi, ctypes.byref(args or capi.EpilogueArgs()), dt, buf, 64))
+        return buf.value.decode()
+
+    for dt in (capi.F16, capi.BF16):
+        assert variant(8192, 30522, 768, dt) == "dma8w_256x256"
+        assert variant(600000, 768, 3072, dt) == "dma8w_256x256"
+        assert variant(1000, 772, 3072, dt) == "dma4w_128x64"
+        assert variant(200, 772, 3072, dt).startswith("reg4w_64x64_splitk")
+        assert variant(128, 772, 3072, dt) == "wave1w_32x32"
+        assert variant(10, 2, 768, dt) == "wave1w_32x32"
+    assert variant(128, 772, 3072, capi.F32).startswith("reg4w_64x64_splitk")
+    assert variant(8192, 30522, 768, capi.F32).startswith("dma8w")
+    heads = capi.EpilogueArgs()
+    heads.seq, heads.heads, heads.head_dim = 128, 12, 20
+    assert variant(64 * 128, 720, 256, capi.F16, capi.EPI_QKV_SPLIT, heads).startswith("dma")

@@ -112,6 +112,29 @@ def test_ring_kernel_epilogues_on_ragged_tiles(ttmi, oracle, dt, M, N, K):
 
 
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("M,N,K,offset", [(10, 2, 768, 0), (128, 772, 3072, 0), (300, 1541, 768, 0), (2560, 772, 3072, 0), (9000, 1002, 256, 0),
+                                          (40, 768, 1536, 1), (128, 3072, 768, 1), (2000, 768, 1024, 1), (8200, 768, 256, 1)])
+def test_fused_products_that_the_ring_tiles_refuse(ttmi, dt, M, N, K, offset):
+    """Widths that are no multiple of eight, and biases, residuals and outputs off the 16-byte grid: few rows, the wavefront
+    kernel, K slices, the DMA tiles of every size.  Rows past M stay untouched."""
+    import ctypes
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    off = lambda t: torch.cat([t.new_full((offset,), -7.0), t.flatten()])[offset:].view(t.shape)
+    A, W = rand(M, K).to(TORCH_DTYPES[dt]), (rand(N, K) / K ** 0.5).to(TORCH_DTYPES[dt])
+    bias, res = off(rand(N).to(A.dtype)), off(rand(M, N).to(A.dtype))
+    base = (A.double() @ W.double().T + bias.double())
+    for epi, args, want in ((capi.EPI_BIAS, _epi(bias=bias), base), (capi.EPI_BIAS_ACT, _epi(bias=bias, act=capi.ACT_RELU), base.relu()),
+                            (capi.EPI_BIAS_ACT, _epi(bias=bias, act=capi.ACT_GELU), torch.nn.functional.gelu(base, approximate="tanh")),
+                            (capi.EPI_BIAS_RESIDUAL, _epi(bias=bias, residual=res), base + res.double()),
+                            (capi.EPI_F32_OUT, _epi(bias=bias), base)):
+        C = off(torch.full((M + 40, N), -7.0, dtype=torch.float32 if epi == capi.EPI_F32_OUT else A.dtype, device="cuda"))
+        ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(W), ptr(C), M, N, K, K, K, N, epi, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+        assert float((C[:M].double() - want).abs().max()) <= GEMM_TOL[dt] * 3
+        assert torch.all(C[M:] == -7.0)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("M,N,steps", [(1, 8, 1), (16, 24, 16), (17, 776, 17), (33, 768, 24), (32, 3072, 12), (10, 768, 33), (64, 136, 96),
                                        (160, 768, 12)])
 def test_few_row_kernel_epilogues(ttmi, oracle, dt, M, N, steps):

@@ -1716,44 +1716,64 @@ constexpr int kNormNotTaken = 1;
 template <typename T, typename Epi>
 struct RingKernel;
 
-// A plain product C = alpha A op(B) + beta C.  (What the encoder's fused products run on is picked by RingKernel.)
-template <typename T, typename Epi>
-inline int launch_plain(const GemmArgs& g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
-  constexpr int BK = kRowBytes / sizeof(T);
-  auto tiles = [&](int bm, int bn) { return (int64_t)ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch; };
-  if (LargeTileKernel<T, Epi>::wanted(g, epi, batch, aligned)) return LargeTileKernel<T, Epi>::launch(g, epi, s);
-  switch (pick_tile(g.m, g.n, batch, nullptr, sizeof(T))) {
-    case 0: return launch_fast<T, 256, 256, 2, 4, Epi>(g, epi, batch, s);
-    case 1: return launch_fast<T, 256, 192, 4, 2, Epi>(g, epi, batch, s);
-    case 2: return launch_fast<T, 256, 128, 4, 2, Epi>(g, epi, batch, s);
-    case 3: {
-      const SplitPlan plan = plan_split<T>(g.m, g.n, g.k, batch, aligned);
-      if (plan.kind == SplitKind::kDmaTiles)
-        return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-      // 128 x 128 tiles on at most half the CUs and a K too short to cut: 128 x 64 tiles put twice as many CUs
-      // to work (2560 x 768 x 768: 240 tiles in one round, 9 us against 11)
-      if (batch == 1 && tiles(128, 128) <= compute_units() / 2 && tiles(128, 64) <= compute_units())
-        return launch_fast<T, 128, 64, 2, 2, Epi, 4>(g, epi, batch, s);
-      return launch_fast<T, 128, 128, 2, 2, Epi>(g, epi, batch, s);
-    }
-    // small problems are latency-bound: the register-staged kernel hides the global latency
-    // of a one-step prefetch better than the DMA path does with a tiny tile
-    default: {
-      const SplitPlan plan = plan_split<T>(g.m, g.n, g.k, batch, aligned);
-      if (plan.kind == SplitKind::kSmallTiles)
-        return launch_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-      if (plan.kind == SplitKind::kDmaTiles)
-        return launch_fast_splitk<T>(g, plan.splits, g.k / BK, BK, s, ReduceWithEpilogue<Epi>{epi, g.m, g.n});
-      if (wave_kernel_ok<T>(g, batch, aligned)) return launch_wave<T>(g, epi, s);
-      return launch_config<T, 64, 64, 2, 2, false, true, Epi>(g, epi, batch, s);
-    }
-  }
-}
-
 template <typename Epi>
 struct IsPlain : std::false_type {};
 template <typename T>
 struct IsPlain<EpiAlphaBeta<T>> : std::true_type {};
+
+// The tiles of this file and K slices on them, for aligned operands with whole K steps: plain products C = alpha A op(B) + beta C,
+// and the products with an epilogue that the ring tiles refuse (see RingKernel::ok): widths that are no multiple of eight, as
+// vocabulary- and class-sized heads have, operands of 2 GiB and more, destinations off the 16-byte grid.
+// us, on the register-staged tiles alone / here: fp16 8192 x 30522 x 768 797 / 717, 6000 x 1540 x 3072 122 / 77, 1000 x 772 x
+// 3072 24.8 / 21.3, 128 x 772 x 768 9.3 / 6.6, 10 x 2 x 768 6.6 / 4.3; fp32 128 x 772 x 3072 68 / 26, 2560 x 1540 x 768 103 / 59.
+template <typename T, typename Epi>
+inline int launch_tiles(const GemmArgs& g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
+  constexpr int BK = kRowBytes / sizeof(T);
+  // Where a 16-bit product with an epilogue lies between two forms, other lines than the plain products' (sweep of M = 10 ... 8192,
+  // N = 2 ... 3076, K = 256 ... 8192).  A cut costs a launch that applies the epilogue; us, whole / cut:
+  //   up to 128 rows it pays past 48 steps of K (128 x 772: 10.5 / 15.0 at 24, 21.7 / 20.2 at 64);
+  //   more rows on small tiles from 32 steps (200 x 772: 9.1 / 11.9 at 12, 14.2 / 15.6 at 24, 23.9 / 16.7 at 48), up to eight
+  //   columns from 24 (700 x 2: 10.9 / 9.1);
+  //   128 x 128 tiles past 64 steps, up to eight columns from 32.  Shorter, they run whole as 128 x 64 tiles with four stages
+  //   (1600 x 772: 22 / 30 at 48, 384 x 772: 45 / 31 at 128; at 16 steps 64 x 64 tiles win, 2560 x 100: 9.7 / 10.9).
+  // Whole 128 x 128 tiles for less than 200 CUs lose to 64 x 64 (2560 x 772 x 3072: fp16 39 / 36, int8 24 / 20).
+  constexpr bool fused16 = !IsPlain<Epi>::value && sizeof(T) == 2;
+  auto tiles = [&](int bm, int bn) { return (int64_t)ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch; };
+  const int ksteps = g.k / BK;
+  if constexpr (IsPlain<Epi>::value)
+    if (LargeTileKernel<T, Epi>::wanted(g, epi, batch, aligned)) return LargeTileKernel<T, Epi>::launch(g, epi, s);
+  const int tile = pick_tile(g.m, g.n, batch, nullptr, sizeof(T));
+  if (tile == 0) return launch_fast<T, 256, 256, 2, 4, Epi>(g, epi, batch, s);
+  if (tile == 1) return launch_fast<T, 256, 192, 4, 2, Epi>(g, epi, batch, s);
+  if (tile == 2) return launch_fast<T, 256, 128, 4, 2, Epi>(g, epi, batch, s);
+  // 128 x 128 tiles on at most half the CUs and a K too short to cut: 128 x 64 tiles put twice as many CUs
+  // to work (2560 x 768 x 768: 240 tiles in one round, 9 us against 11)
+  bool narrower = tile == 3 && batch == 1 && tiles(128, 128) <= compute_units() / 2 && tiles(128, 64) <= compute_units();
+  // (the reduction over K slices sums floats and applies an epilogue to rows: no int8, no transposed V)
+  if constexpr (std::is_same<typename Epi::Acc, float>::value) {
+    bool column_pass = false;
+    if constexpr (HasColumnPass<Epi>::value) column_pass = epi.v_pitch > 0;
+    SplitPlan plan = column_pass ? SplitPlan{SplitKind::kNone, 1} : plan_split<T>(g.m, g.n, g.k, batch, aligned);
+    if (fused16 && plan.kind != SplitKind::kNone) {
+      const bool dma = plan.kind == SplitKind::kDmaTiles;
+      const bool pays = g.m <= 128 ? ksteps > 48 : g.n <= 8 ? ksteps >= (dma ? 32 : 24) : dma ? ksteps > 64 : ksteps >= 32;
+      if (!pays) {
+        narrower = dma && ksteps >= (g.n > 32 ? 24 : 32);
+        plan.kind = SplitKind::kNone;
+      }
+    }
+    const ReduceWithEpilogue<Epi> reduce{epi, g.m, g.n};
+    if (plan.kind == SplitKind::kSmallTiles) return launch_splitk<T>(g, plan.splits, ksteps, BK, s, reduce);
+    if (plan.kind == SplitKind::kDmaTiles) return launch_fast_splitk<T>(g, plan.splits, ksteps, BK, s, reduce);
+  }
+  if (narrower) return launch_fast<T, 128, 64, 2, 2, Epi, 4>(g, epi, batch, s);
+  if (tile == 3 && (IsPlain<Epi>::value || sizeof(T) == 4 || tiles(128, 128) >= 200)) return launch_fast<T, 128, 128, 2, 2, Epi>(g, epi, batch, s);
+  // small problems are latency-bound: the register-staged kernel hides the global latency
+  // of a one-step prefetch better than the DMA path does with a tiny tile
+  if constexpr (std::is_same<typename Epi::Acc, float>::value)
+    if (wave_kernel_ok<T>(g, batch, aligned)) return launch_wave<T>(g, epi, s);
+  return launch_config<T, 64, 64, 2, 2, false, true, Epi>(g, epi, batch, s);
+}
 
 template <typename T, bool B_KN, typename Epi>
 inline int launch_gemm(GemmArgs g, const Epi& epi, int batch, bool aligned, hipStream_t s) {
@@ -1762,8 +1782,9 @@ inline int launch_gemm(GemmArgs g, const Epi& epi, int batch, bool aligned, hipS
   auto tiles = [&](int bm, int bn) { return (int64_t)ceil_div(g.m, bm) * ceil_div(g.n, bn) * batch; };
   if (!B_KN) {
     if (aligned && g.k % (kRowBytes / (int)sizeof(T)) == 0) {
-      if constexpr (IsPlain<Epi>::value) return launch_plain<T>(g, epi, batch, aligned, s);
-      else if (RingKernel<T, Epi>::ok(g, epi, batch)) return RingKernel<T, Epi>::launch(g, epi, s);
+      if constexpr (!IsPlain<Epi>::value)
+        if (RingKernel<T, Epi>::ok(g, epi, batch)) return RingKernel<T, Epi>::launch(g, epi, s);
+      return launch_tiles<T>(g, epi, batch, aligned, s);
     }
     if (aligned) {
       if (tiles(128, 128) >= 200) return launch_config<T, 128, 128, 2, 2, false, true, Epi>(g, epi, batch, s);
