@@ -148,8 +148,8 @@ TTMI_API int ttmi_add_bias_layer_norm_product32(void* out, const float* residual
 /* The dense projection and AddBiasLayerNorm that close both halves of an encoder layer, as one call:
  *   out[m,n] = LN(a[m,k] . w[n,k]^T + bias + residual)
  * (BertOutput, layers/bert_output.cpp:41-60; the attention output, layers/multi_headed_attention.cpp:359-371;
- * the reference issues MatMul then AddBiasLayerNorm).  Small problems, where the product is cut along K to
- * fill the chip, normalise inside the kernel that sums the K slices; larger ones run ttmi_gemm followed by
+ * the reference issues MatMul then AddBiasLayerNorm).  Small and mid-size problems hold the product in fp32, whole or in
+ * K slices, and normalise inside the kernel that sums the slices; larger ones run the product followed by
  * ttmi_add_bias_layer_norm.  Either `residual` (same dtype as out) or the pair residual_f32 / out_f32 (the
  * fp32 residual stream of ttmi_add_bias_layer_norm_residual32, which may alias each other) is given; the
  * unused ones are NULL.  With the fp32 pair and out_f32 != residual_f32, 16-bit products of large problems are kept
@@ -167,16 +167,15 @@ TTMI_API int ttmi_gemm_bias_layer_norm(const void* a, const void* w, void* out, 
  * arguments, same kernels and bit-identical results; the fp32 partial tiles of a product that is cut along K
  * live in a buffer of TTMI_STATIC_SCRATCH_BYTES that is part of the library's device image (every GPU the
  * library runs on holds it until the process ends) instead of the per-stream workspace ttmi_gemm_bias_layer_norm
- * allocates on first use.  The call reaches no hipMalloc / hipFree.  A problem whose K slices need more than
- * that buffer (slices * m * n * 4 bytes; the largest the encoder configurations produce is m = 2560, n = 768,
- * k = 3072 in three slices, 23.6 MB) is refused with TTMI_EINVAL; problems large enough to run unsplit need no
- * scratch and are accepted at any size.  One exception to "the same kernels": a product of a few thousand rows that
- * ttmi_gemm_bias_layer_norm cuts in two on its large-tile kernel (an optimisation of a product that also runs whole;
- * 6275 x 768 x 3072 is one) is cut here only if its partial products fit the buffer, and runs whole otherwise, with
- * the 16-bit rounding of the product in front of the LayerNorm that large problems have.  The first call on a device resolves the buffer's address and sets kernel
- * attributes, so make one call outside a graph capture before capturing calls.  Nothing has to be cleared between calls (every partial tile that is read
- * has been written by the same call), but all calls on one GPU share the buffer: calls that overlap in time
- * on one GPU (different streams or threads) race. */
+ * allocates on first use.  The call reaches no hipMalloc / hipFree.  Sizes and slices are
+ * chosen so that the partial tiles (slices * m * n * 4 bytes) always fit; with a smaller size admitted (switch
+ * "TTMI_STATIC_SCRATCH_LIMIT") a problem whose K slices do not fit is refused with TTMI_EINVAL, and a product of more
+ * than 384 rows that is held in fp32 for its precision alone (2048 x 1024 x 1024 and 8192 x 768 x 3072 are two) is
+ * rounded to the 16-bit type in front of the LayerNorm instead, as the product of a larger problem is.  Problems large
+ * enough to run unsplit need no scratch and are accepted at any size.  The first call on a device resolves the
+ * buffer's address and sets kernel attributes, so make one call outside a graph capture before capturing calls.
+ * Nothing has to be cleared between calls (every partial tile that is read has been written by the same call), but all
+ * calls on one GPU share the buffer: calls that overlap in time on one GPU (different streams or threads) race. */
 #define TTMI_STATIC_SCRATCH_BYTES (32u << 20)
 TTMI_API int ttmi_gemm_bias_layer_norm_static(const void* a, const void* w, void* out, const void* residual,
                                               const float* residual_f32, const void* bias, const void* gamma,

@@ -414,6 +414,31 @@ def test_gemm_bias_layer_norm_k_slices_on_the_large_tile_kernel(ttmi, oracle, dt
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("M,N,K,most", [(384, 768, 768, 7), (512, 512, 512, 9), (385, 1024, 1024, 7), (2048, 1024, 1024, 7), (6827, 768, 3072, 3),
+                                        (10752, 768, 3072, 3), (5121, 1024, 4096, 3), (8192, 1024, 4096, 3)])
+def test_product_in_front_of_a_layer_norm_is_held_in_fp32(ttmi, dt, static, M, N, K, most):
+    """The product reaches AddBiasLayerNorm unrounded up to the sizes of fp32_product_expected in gemm_typed.h: the residual is minus
+    the product rounded to 16 bits, so that what is normalised is that rounding, which a 16-bit product would not have.
+    Whole numbers throughout (products below 2^16 and 2^24): the sum in front of the LayerNorm is exact."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A, W = (torch.randint(0, most + 1, shape, generator=g, device="cuda").to(TORCH_DTYPES[dt]) for shape in ((M, K), (N, K)))
+    product = A.float() @ W.float().T
+    assert float(product.max()) < 65504 and torch.equal(product, product.round())
+    residual = (-product).to(TORCH_DTYPES[dt])
+    zero, one = torch.zeros(N, dtype=A.dtype, device="cuda"), torch.ones(N, dtype=A.dtype, device="cuda")
+    out = torch.full((M + 8, N), -7.0, dtype=A.dtype, device="cuda")
+    fn = ttmi.ttmi_gemm_bias_layer_norm_static if static else ttmi.ttmi_gemm_bias_layer_norm
+    ok(fn(ptr(A), ptr(W), ptr(out), ptr(residual), None, ptr(zero), ptr(one), ptr(zero), None, M, N, K, 1e-12, TTMI_DTYPES[dt], stream()))
+    x = (product + residual.float()).double()
+    want = (x - x.mean(1, keepdim=True)) / (x.var(1, unbiased=False, keepdim=True) + 1e-12).sqrt()
+    assert float(x.abs().max()) >= 1
+    # one rounding to 16 bits of values of up to about 4, and fp32 sums of squares of numbers of one or two digits
+    assert float((out[:M].double() - want).abs().max()) <= GEMM_TOL[dt]
+    assert torch.all(out[M:] == -7.0)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("forced", [False, True])
 @pytest.mark.parametrize("M,N,K,with_bias", [(300, 200, 256, True), (4100, 1024, 1024, False), (2560, 768, 3072, True),
                                              (8192, 768, 768, True), (777, 776, 384, False), (128, 768, 3072, True)])

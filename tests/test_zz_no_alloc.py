@@ -114,6 +114,30 @@ def test_static_scratch_refuses_what_does_not_fit(ttmi):
     _both(ttmi, "f16", M, N, K, seed=8)
 
 
+def test_static_scratch_holds_the_product_only_where_it_fits(ttmi):
+    """2048 x 1024 x 1024: the product in front of the LayerNorm is held in fp32 (8 MiB); with 1 MiB admitted the call is not
+    refused but rounds it to 16 bits on its way: one more rounding of values below 8."""
+    M, N, K = 2048, 1024, 1024
+    _both(ttmi, "f16", M, N, K, seed=13)
+    rng = np.random.default_rng(14)
+    dA, dW = dev(rng.standard_normal((M, K)).astype(np.float32), "f16"), dev((rng.standard_normal((N, K)) / 32).astype(np.float32), "f16")
+    dres = dev(rng.standard_normal((M, N)).astype(np.float32), "f16")
+    one, zero = dev(np.ones(N, np.float32), "f16"), dev(np.zeros(N, np.float32), "f16")
+    outs = []
+    try:
+        for limit in (-1, 1 << 20):
+            ok(ttmi.ttmi_set_kernel_switch(b"TTMI_STATIC_SCRATCH_LIMIT", limit))
+            outs.append(torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda"))
+            ok(ttmi.ttmi_gemm_bias_layer_norm_static(ptr(dA), ptr(dW), ptr(outs[-1]), ptr(dres), None, ptr(zero), ptr(one), ptr(zero), None,
+                                                     M, N, K, 1e-12, TTMI_DTYPES["f16"], stream()))
+    finally:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_STATIC_SCRATCH_LIMIT", -1))
+    torch.cuda.synchronize()
+    assert not torch.equal(outs[0], outs[1])
+    # half an ulp of a product below 8 (0.004 / 2) over the row's deviation of about 1.4, and an ulp of the result
+    assert float((outs[0].float() - outs[1].float()).abs().max()) < 8e-3
+
+
 def test_static_scratch_call_under_graph_capture(ttmi):
     """What the entry point is for: a call recorded into a HIP graph (after one eager call, which resolves the
     buffer's address and sets the kernel attributes).  The graph is replayed three times with eager work and

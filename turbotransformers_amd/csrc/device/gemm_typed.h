@@ -126,9 +126,21 @@ int gemm_norm_fused_typed(const GemmArgs& g, const void* gamma, const void* beta
   return gemm_fused_typed<T>(g, c, ldc, epilogue, args, s, &rows);
 }
 
-// Product + AddBiasLayerNorm.  The product reaches the normalisation in fp32 where it is short of rows or long in K
-// (`fp32_product`: few rows make the extra bytes free, a long sum loses most to a 16-bit rounding), as K slices or
-// whole, summed by the kernel that normalises; else it passes through `out` in the storage type.
+// Where the product in front of a LayerNorm is held in fp32 although nothing else asks for it (RingUse::kLayerNorm: whole or
+// in K slices, summed by the kernel that normalises).  Elsewhere a 16-bit product is rounded on its way through `out`.
+// Few rows make the extra bytes free, and a long sum loses most to the rounding.
+inline bool fp32_product_pays(int64_t m, int64_t n, int64_t k) { return m <= 384 || (k >= 2 * n && m * n * 4 <= (20ll << 20)); }
+// ... and where the tiles leave so many CUs idle over so long a K that such products have always been cut along K, which
+// holds them: rounded, they would lose precision that callers had.  It costs an fp32 copy of the product; us, fp16, rounded /
+// held: 512 x 512 x 512 7.6 / 7.3, 1024 x 1024 x 1024 10.3 / 12.1, 2048 x 1024 x 1024 13.2 / 17.2, 8192 x 768 x 3072 44.9 /
+// 50.6, 10752 x 768 x 3072 55.1 / 62.0, 8192 x 1024 x 4096 66.5 / 74.5 (cut, as they were: 7.9, 16.5, 22.5, 53.4, 67.2, 76.9).
+inline bool fp32_product_expected(int64_t m, int64_t n, int64_t k) {
+  auto tiles = [&](int edge) { return ceil_div(m, edge) * ceil_div(n, edge); };
+  const int64_t cus = compute_units();
+  return (k >= 512 && tiles(64) <= cus / 4) || (k >= 1024 && tiles(128) <= cus / 2) || (k >= 2048 && tiles(256) <= cus / 2);
+}
+
+// Product + AddBiasLayerNorm.
 template <typename T>
 int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
@@ -170,14 +182,21 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
     if (plan.kind == SplitKind::kDmaTiles) return launch_fast_splitk<T>(g, plan.splits, k / BK, BK, s, reduce);
     if (plan.kind == SplitKind::kSmallTiles) return launch_splitk<T>(g, plan.splits, k / BK, BK, s, reduce);
   }
-  const bool fp32_product = m <= 384 || (k >= 2 * n && m * n * 4 <= (20ll << 20));
-  if (ring && rows_ok && fp32_product) {
+  // with an fp32 residual stream and room for it the product stays in fp32 without a workspace
+  const bool product_in_out32 = sizeof(T) == 2 && residual_f32 != nullptr && out_f32 != residual_f32;
+  const bool pays = fp32_product_pays(m, n, k);
+  if (ring && rows_ok && (pays || (sizeof(T) == 2 && !product_in_out32 && fp32_product_expected(m, n, k)))) {
     // Few rows: one slice; more of K is cheaper cut (10 x 768 x 3072 in twelve slices 3.8 us, whole 5.4), and so is fp32
     // (128 x 768 x 768 in five slices 5.7 us, whole 6.6).
-    if (sizeof(T) == 2 && flat_wins<T>(g, 32)) {
+    const bool flat = sizeof(T) == 2 && flat_wins<T>(g, 32);
+    const RingPlan plan = flat ? RingPlan{} : pick_ring<T>(m, n, k / BK, RingUse::kLayerNorm);
+    const size_t bytes = (size_t)plan.slices * (size_t)m * (size_t)n * sizeof(float);
+    // (where the caller has fixed the workspace and the copy does not fit it, the product is rounded and not refused)
+    if (pays || tl_fixed_workspace.ptr == nullptr || bytes <= tl_fixed_workspace.bytes) {
+      if (!flat) return launch_ring_slices<T>(g, plan, s, reduce);
       float* ws = nullptr;
       if (tl_describe == nullptr) {
-        const int rc = splitk_workspace((size_t)m * n * sizeof(float), s, &ws);
+        const int rc = splitk_workspace(bytes, s, &ws);
         if (rc != 0) return rc;
       }
       const int rc = launch_flat<T>(g, EpiPartial{ws, m * n, n, true}, 1, s);
@@ -185,12 +204,8 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
       reduce(ws, 1, true, s);
       return launch_status("gemm_flat_layer_norm");
     }
-    const RingPlan plan = pick_ring<T>(m, n, k / BK, RingUse::kLayerNorm);
-    return launch_ring_slices<T>(g, plan, s, reduce);
   }
-  // With an fp32 residual stream and room for it, the product stays in fp32 too: the GEMM stores its accumulators to
-  // out_f32 and the LayerNorm pass reads them there.
-  if (residual_f32 != nullptr && out_f32 != residual_f32 && dtype != TTMI_F32) {
+  if (product_in_out32) {  // the GEMM stores its accumulators to out_f32 and the LayerNorm pass reads them there
     EpiF32<T> epi{out_f32, nullptr, n, aligned16(out_f32) && n % 4 == 0};
     const int rc = launch_gemm<T, false>(g, epi, 1, aligned, s);
     if (rc != 0) return rc;
