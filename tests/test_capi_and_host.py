@@ -346,3 +346,24 @@ def test_fused_products_off_the_ring_keep_the_kernels_for_their_size():
     heads = capi.EpilogueArgs()
     heads.seq, heads.heads, heads.head_dim = 128, 12, 20
     assert variant(64 * 128, 720, 256, capi.F16, capi.EPI_QKV_SPLIT, heads).startswith("dma")
+
+
+def test_gelu_products_of_65_to_128_rows_leave_the_ring_only_for_one_short_sequence():
+    """The wavefront kernel (16-bit, whole) and the cut along K (fp32) are kept for the widths of an intermediate Linear over
+    one short sequence; long K, few columns and wide outputs take the ring tiles, which the wavefront kernel trails by up to
+    four times there."""
+    import ctypes
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+    args = capi.EpilogueArgs()
+    args.act = capi.ACT_GELU
+
+    def variant(m, n, k, dt):
+        capi.check(lib.ttmi_gemm_describe(m, n, k, capi.EPI_BIAS_ACT, ctypes.byref(args), dt, buf, 64))
+        return buf.value.decode()
+
+    for dt in (capi.F16, capi.BF16):
+        for m, n, k in ((128, 16384, 4096), (128, 8192, 2048), (128, 768, 3072), (100, 768, 768), (128, 256, 1024)):
+            assert variant(m, n, k, dt).startswith("dma"), (m, n, k)
+    for m, n, k in ((128, 8192, 512), (128, 16384, 4096)):
+        assert "_splitk" not in variant(m, n, k, capi.F32), (m, n, k)

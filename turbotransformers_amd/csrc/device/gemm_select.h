@@ -24,14 +24,21 @@ struct RingKernel {
     if constexpr (HasColumnPass<Epi>::value) return epi.v_pitch > 0 ? 2 * (int64_t)epi.hidden : 0;
     else return 0;
   }
+  // 65 to 128 rows with GELU of a width and K for which ttmi_gemm_describe has always named one form: fp32 cut along K (eight
+  // steps or more, up to 128 tiles of 64 x 64), 16-bit whole on the wavefront kernel (short of sixteen steps, more than 64
+  // tiles).  Neither is the fastest since the ring tiles.  us, kept / ring: fp32 128 x 3072 x 768 14.8 / 9.5, 128 x 4096 x
+  // 1024 16.7 / 11.9, 128 x 2048 x 512 9.5 / 7.2; fp16 128 x 3072 x 768 8.4 / 5.0, 72 x 3072 x 768 8.3 / 5.1.  Outside these
+  // lines they would cost up to four times the ring's time (fp16 128 x 16384 x 4096 114 / 30, fp32 128 x 8192 x 512 18.1 / 11.4).
+  static bool keeps_named_form(const GemmArgs& g) {
+    const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T)), tiles = ceil_div(g.m, 64) * ceil_div(g.n, 64);
+    return g.m > 64 && g.m <= 128 && (sizeof(T) == 4 ? ksteps >= 8 && tiles <= 128 : ksteps < 16 && tiles > 64);
+  }
   static RingPlan plan(const GemmArgs& g, const Epi& epi) {
     // a cut needs an epilogue that the reduction kernel can apply to rows of eight columns
     constexpr bool cut = std::is_same<typename Epi::Acc, float>::value;
     RingUse use = cut && column_limit(epi) == 0 ? RingUse::kSliced : RingUse::kWhole;
-    // 65 to 128 fp32 rows with GELU stay cut along K: the cut is what ttmi_gemm_describe has always named for this product.
-    // It is not the faster form since the ring tiles: 128 x 3072 x 768 whole 11.6 us traced, four slices 10.9 + 4.7.
     if constexpr (IsGelu<Epi>::value && sizeof(T) == 4)
-      if (g.m > 64 && g.m <= 128 && g.k / (kRowBytes / (int)sizeof(T)) >= 8) use = RingUse::kCut;
+      if (keeps_named_form(g)) use = RingUse::kCut;
     return pick_ring<T>(g.m, g.n, g.k / (kRowBytes / (int)sizeof(T)), use, column_limit(epi));
   }
   static bool ok(const GemmArgs& g, const Epi& epi, int batch) {
@@ -39,9 +46,8 @@ struct RingKernel {
   }
   static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) {
     constexpr int BK = kRowBytes / (int)sizeof(T);
-    // (65 to 128 rows with GELU: one 32 x 32 tile per wavefront, W and A straight from L2)
     if constexpr (IsGelu<Epi>::value && sizeof(T) == 2)
-      if (g.m > 64 && wave_kernel_ok<T>(g, 1, true)) return launch_wave<T>(g, epi, s);
+      if (keeps_named_form(g) && wave_kernel_ok<T>(g, 1, true)) return launch_wave<T>(g, epi, s);
     if (flat_wins<T>(g, 96)) return launch_flat<T>(g, epi, 1, s);
     const RingPlan p = plan(g, epi);
     if constexpr (sizeof(T) == 2) {
