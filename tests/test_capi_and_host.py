@@ -367,3 +367,26 @@ def test_gelu_products_of_65_to_128_rows_leave_the_ring_only_for_one_short_seque
             assert variant(m, n, k, dt).startswith("dma"), (m, n, k)
     for m, n, k in ((128, 8192, 512), (128, 16384, 4096)):
         assert "_splitk" not in variant(m, n, k, capi.F32), (m, n, k)
+
+
+def test_picking_a_tile_costs_less_than_a_microsecond():
+    """The selection of a ring tile and its K slices runs on the host in front of every launch, and the small cases are bound by
+    the host.  Through ttmi_gemm_describe, whose own cost a plain product of the same size shares: 16 slices of at most eight
+    tiles at some 3 ns each are 0.4 us; twice that is allowed (a plain search of all of them, run twice, takes 2.5 us more)."""
+    import ctypes
+    import time
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+    args = ctypes.byref(capi.EpilogueArgs())
+
+    def best_us(m, n, k, dt, epi):
+        best = 1e9
+        for _ in range(60):
+            start = time.perf_counter()
+            for _ in range(200):
+                lib.ttmi_gemm_describe(m, n, k, epi, args, dt, buf, 64)
+            best = min(best, (time.perf_counter() - start) / 200 * 1e6)
+        return best
+
+    for m, n, k, dt in ((128, 768, 3072, capi.F32), (896, 768, 3072, capi.F32), (8, 768, 3072, capi.F16), (128, 768, 3072, capi.F16)):
+        assert best_us(m, n, k, dt, capi.EPI_BIAS) < best_us(m, n, k, dt, capi.EPI_NONE) + 0.8, (m, n, k, dt)

@@ -42,7 +42,7 @@ struct RingKernel {
     return pick_ring<T>(g.m, g.n, g.k / (kRowBytes / (int)sizeof(T)), use, column_limit(epi));
   }
   static bool ok(const GemmArgs& g, const Epi& epi, int batch) {
-    return batch == 1 && g.k_chunk == 0 && ring_operands_ok<T>(g) && epilogue_vec(epi) && plan(g, epi).tile >= 0;
+    return batch == 1 && g.k_chunk == 0 && ring_operands_ok<T>(g) && epilogue_vec(epi) && column_limit(epi) % kRingColumns == 0;
   }
   static int launch(const GemmArgs& g, const Epi& epi, hipStream_t s) {
     constexpr int BK = kRowBytes / (int)sizeof(T);
