@@ -953,6 +953,36 @@ def test_attention_masks_far_from_zero(ttmi, oracle, dt, form, v_transposed, S):
     assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
 
 
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("form,v_transposed", [(-1, False), (-1, True), (8, True), (1, True)])
+@pytest.mark.parametrize("S", [33, 200])
+def test_attention_keeps_nans_where_they_belong(ttmi, dt, form, v_transposed, S):
+    """A NaN in a query makes the row of that query and head NaN, one in a key or in the mask of a key the head or the sequence,
+    and nothing else, on every form of the one-kernel attention."""
+    rng = np.random.default_rng(S)
+    B, h, d = 3, 2, 64
+    Q, K, V = (rng.standard_normal((B, h, S, d), np.float32) for _ in range(3))
+    mask = np.zeros((B, S), np.float32)
+    Q[0, 0, S // 2, 7] = np.nan
+    K[1, 1, S - 1, 50] = np.nan
+    mask[2, 3] = np.nan
+    dV, pitch = _v_operand(V, dt, v_transposed)
+    out = torch.full((B, S, h * d), 9.0, dtype=dV.dtype, device="cuda")
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", form))
+    try:
+        ok(ttmi.ttmi_fused_attention(ptr(dev(Q, dt)), ptr(dev(K, dt)), ptr(dV), ptr(dev(mask)), ptr(out), None, B, h, S, d, pitch,
+                                     0.125, TTMI_DTYPES[dt], stream()))
+    finally:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+    q, k, v = (rounded(x, dt).astype(np.float64) for x in (Q, K, V))
+    p = np.exp(q @ k.transpose(0, 1, 3, 2) * 0.125 + mask[:, None, None, :])
+    want = ((p / p.sum(-1, keepdims=True)) @ v).transpose(0, 2, 1, 3).reshape(B, S, h * d)
+    got = host(out)
+    assert np.isnan(want).sum() == d + S * d + S * h * d
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert max_abs(got[~np.isnan(want)], want[~np.isnan(want)]) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("F,past,fresh,per_query", [(1, 0, 1, False), (33, 0, 33, True), (1, 40, 1, False), (1, 127, 1, True),
                                                     (5, 124, 5, True), (64, 0, 256, False), (2, 255, 2, True), (31, 300, 212, False)])

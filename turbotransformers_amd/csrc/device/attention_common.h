@@ -2,8 +2,6 @@
 // from zero.
 #pragma once
 
-#include <cfloat>
-
 #include "common.h"
 
 namespace ttmi {
@@ -14,15 +12,19 @@ namespace ttmi {
 // of such a row 0 and the row 0 / 0), and keys past the end carry -inf, below any mask.  A mask of -inf stays -inf.
 constexpr float kFarthestScore = 0x1p127f;  // the running maximum starts at its negative
 __device__ __forceinline__ float mask_in_scores(float mask, float inv_scale) {
-  const float x = mask * inv_scale;
-  return fabsf(mask) <= FLT_MAX ? fminf(fmaxf(x, -kFarthestScore), kFarthestScore) : x;
+  // A NaN has to stay one, but attention.hip is compiled as if there were none: the bits are tested, out of the compiler's sight.
+  uint32_t bits = __builtin_bit_cast(uint32_t, mask);
+  asm("" : "+v"(bits));
+  const float x = fminf(fmaxf(mask * inv_scale, -kFarthestScore), kFarthestScore);
+  return __builtin_bit_cast(float, (bits & 0x7f800000u) != 0x7f800000u ? __builtin_bit_cast(uint32_t, x) : bits);
 }
 
 // m * c is rounded.  The error is the same for all keys of a row and cancels in the division by the row's sum, but from
 // |m * c| = 2^30 on it is 64 and more: the probabilities of a row masked with -1e10 would be 0 or infinite.  Beyond 2^12
 // (error 2^-13; no row with an unmasked key comes near) the maximum is subtracted from the scores first, exactly.
-// The test is three instructions per 32 keys: us per launch without / with it, 12 heads, fp16 64 x 512 tokens 83.8 / 83.0, 8 x
-// 256 7.6 / 7.7, 1 x 387 6.8 / 6.8, fp32 1 x 128 6.5 / 6.5, 20 x 100 14.8 / 14.8, 16 x 512 147.2 / 148.1.
+// The test is three instructions per 32 keys: us per launch without / with it, 12 heads, fp16 64 x 512 tokens 82.9 / 83.0, 8 x
+// 256 7.5 / 7.7, 1 x 387 6.6 / 6.6, 20 packed requests 19.3 / 19.3, 32 of them 23.9 / 24.1, fp32 1 x 128 6.5 / 6.5, 20 x 100 14.8 /
+// 14.8, 16 x 512 146.2 / 147.2.  (Joined to the test for a maximum that moves it costs registers: 7.5 / 7.8, 20 requests 19.7.)
 template <typename Scores>
 __device__ __forceinline__ float relative_scores(Scores& st, float m_run, float scale_log2e) {
   const float neg_m = -m_run * scale_log2e;
