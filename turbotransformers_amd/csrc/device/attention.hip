@@ -30,13 +30,6 @@
 
 namespace ttmi {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
-
 struct __attribute__((may_alias)) alignas(16) Chunk16 {
   uint32_t w[4];
 };
@@ -44,47 +37,6 @@ struct __attribute__((may_alias)) alignas(8) Chunk8 {
   uint32_t w[2];
 };
 
-template <typename T>
-__device__ __forceinline__ floatx16 mma16(const Chunk16& a, const Chunk16& b, floatx16 c);
-template <>
-__device__ __forceinline__ floatx16 mma16<f16>(const Chunk16& a, const Chunk16& b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
-}
-template <>
-__device__ __forceinline__ floatx16 mma16<bf16>(const Chunk16& a, const Chunk16& b, floatx16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// Two floats -> one packed register (round to nearest even): v_cvt_pk_{f16,bf16}_f32.
-template <typename T>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi);
-template <>
-__device__ __forceinline__ uint32_t pack2<f16>(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, halfx2));
-}
-template <>
-__device__ __forceinline__ uint32_t pack2<bf16>(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
-}
-
-// acc + lo + hi of a packed pair (v_dot2c_f32_*): the softmax denominator is summed from the
-// ROUNDED probabilities, the same values the P.V MFMA consumes.
-template <typename T>
-__device__ __forceinline__ float add_pair(uint32_t p, float acc);
-template <>
-__device__ __forceinline__ float add_pair<f16>(uint32_t p, float acc) {
-  return __builtin_amdgcn_fdot2(__builtin_bit_cast(halfx2, p), halfx2{(_Float16)1.0f, (_Float16)1.0f}, acc, false);
-}
-template <>
-__device__ __forceinline__ float add_pair<bf16>(uint32_t p, float acc) {
-  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), bf16x2{(__bf16)1.0f, (__bf16)1.0f}, acc, false);
-}
-
-constexpr int kD = 64;          // head dim
 constexpr int kBKV = 64;        // keys per LDS tile
 // log2 of the largest probability tolerated before the running maximum is moved.  bf16 keeps the
 // exact maximum: with 8 mantissa bits a dominant probability of exactly 1.0 is worth keeping exact.
@@ -119,7 +71,7 @@ __device__ __forceinline__ void attention_tile(const char* kt, const char* vt, c
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const Chunk16 kf = *reinterpret_cast<const Chunk16*>(kt + sk * 128 + k_off[kk]);
-      st = mma16<T>(kf, qf[kk], st);
+      st = mma32<T>(kf, qf[kk], st);
     }
     float mx = st[0];
 #pragma unroll
@@ -161,7 +113,7 @@ __device__ __forceinline__ void attention_tile(const char* kt, const char* vt, c
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const Chunk16 vf = *reinterpret_cast<const Chunk16*>(vt + t * 32 * 128 + k_off[2 * sub + kk]);
-        ot[t] = mma16<T>(vf, pf[kk], ot[t]);
+        ot[t] = mma32<T>(vf, pf[kk], ot[t]);
       }
   }
 }

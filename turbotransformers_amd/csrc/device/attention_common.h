@@ -1,10 +1,56 @@
-// What the one-kernel attention forms (attention.hip, attention_f32.hip, attention_split.hip) share: masks and scores far
-// from zero.
+// What the one-kernel attention forms share: vector types, the matrix instruction over a 16-byte piece of both operands, pairs
+// of 16-bit probabilities, and masks and scores far from zero.
 #pragma once
+
+#include <type_traits>
 
 #include "common.h"
 
 namespace ttmi {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
+
+constexpr int kD = 64;  // head dim
+
+// D = A B + C over one 16-byte piece of both operands: eight K indices per half-wavefront in one instruction (16-bit types), or
+// four, one per instruction (fp32)
+template <typename T, typename Piece>
+__device__ __forceinline__ floatx16 mma32(const Piece& a, const Piece& b, floatx16 c) {
+  static_assert(sizeof(Piece) == 16, "a 16-byte piece");
+  if constexpr (std::is_same<T, f16>::value) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  } else if constexpr (std::is_same<T, bf16>::value) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  } else {
+    const floatx4 x = __builtin_bit_cast(floatx4, a), y = __builtin_bit_cast(floatx4, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_32x32x2f32(x[j], y[j], c, 0, 0, 0);
+    return c;
+  }
+}
+
+// Two floats -> one packed register (round to nearest even): v_cvt_pk_{f16,bf16}_f32.
+template <typename T>
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  if constexpr (std::is_same<T, f16>::value) return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, halfx2));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
+}
+// acc + lo + hi of a packed pair (v_dot2c_f32_*): the softmax denominator is summed from the ROUNDED probabilities, the same
+// values the second product consumes.
+template <typename T>
+__device__ __forceinline__ float add_pair(uint32_t p, float acc) {
+  if constexpr (std::is_same<T, f16>::value)
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(halfx2, p), halfx2{(_Float16)1.0f, (_Float16)1.0f}, acc, false);
+  else return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), bf16x2{(__bf16)1.0f, (__bf16)1.0f}, acc, false);
+}
 
 // Scores are kept in raw units: q . k + mask / scale, and a probability is 2^(s * c - m * c) with c = scale * log2(e), one
 // multiply-add, m the running maximum.  A wholly masked row is the mean of V, as a softmax over mask + score gives it, so

@@ -30,19 +30,8 @@ namespace ttmi {
 
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
-
-constexpr int kD = 64;           // head dim
 constexpr int kBKV = 64;         // keys per LDS tile
 constexpr int kRow = 256;        // bytes of a K row (64 floats) and of a V^T row (64 keys)
-
-// four K indices of both operands, one per instruction
-__device__ __forceinline__ floatx16 mma4(const floatx4& a, const floatx4& b, floatx16 c) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], c, 0, 0, 0);
-  return c;
-}
 
 // 16-byte chunk `chunk` of row `row` of a tile with 256-byte rows: the 16 lanes the LDS serves together read one chunk
 // column of 16 different rows, so the chunk index is XORed with the row
@@ -175,7 +164,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) {
         const floatx4 kf = *reinterpret_cast<const floatx4*>(kt + tile_off(sk + lrow, 2 * kk + lhalf));
-        st = mma4(kf, qf[kk], st);
+        st = mma32<float>(kf, qf[kk], st);
       }
       float mx = st[0];
 #pragma unroll
@@ -211,7 +200,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           const floatx4 vf = *reinterpret_cast<const floatx4*>(vt + tile_off(t * 32 + lrow, sk / 4 + 2 * g + lhalf));
-          ot[t] = mma4(vf, pf, ot[t]);
+          ot[t] = mma32<float>(vf, pf, ot[t]);
         }
       }
     }

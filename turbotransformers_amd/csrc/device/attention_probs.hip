@@ -14,45 +14,13 @@
 // needs is requested before the first product.  V is row-major (a cache grows along the sequence): fp32 fragments are read
 // one float per lane, 16-bit rows go through LDS, where a lane picks its column.
 // Keys past 32 * NW * NB do not fit: the launcher takes the form for up to 128, 256 and 512 keys.
-#include <type_traits>
-
-#include "common.h"
+#include "attention_common.h"
 
 namespace ttmi {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
-
-constexpr int kD = 64;
 constexpr int kQ = 32, kKeys = 32;  // queries per workgroup, keys per block
 constexpr int kPitch = kD + 4;      // floats of a row of a partial output in LDS
-
-template <typename T>
-__device__ __forceinline__ floatx16 mma(const u32x4& a, const u32x4& b, floatx16 c) {
-  if constexpr (std::is_same<T, f16>::value) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
-  } else if constexpr (std::is_same<T, bf16>::value) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      c = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[j]), __builtin_bit_cast(float, (uint32_t)b[j]), c, 0, 0, 0);
-    return c;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  if constexpr (std::is_same<T, f16>::value) return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, halfx2));
-  else return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
-}
 
 struct ProbsArgs {
   const void *q, *k_past, *v_past, *k, *v;
@@ -144,7 +112,7 @@ __global__ __launch_bounds__(NW * 64) void attention_probs_kernel(const ProbsArg
 #pragma unroll
     for (int e = 0; e < 16; ++e) st[n][e] = 0.f;
 #pragma unroll
-    for (int kk = 0; kk < PIECES; ++kk) st[n] = mma<T>(kf[n][kk], qf[kk], st[n]);
+    for (int kk = 0; kk < PIECES; ++kk) st[n] = mma32<T>(kf[n][kk], qf[kk], st[n]);
 #pragma unroll
     for (int g = 0; g < 4; ++g)
 #pragma unroll
@@ -273,7 +241,7 @@ __global__ __launch_bounds__(NW * 64) void attention_probs_kernel(const ProbsArg
             const uint16_t* e = reinterpret_cast<const uint16_t*>(rows) + (16 * kk + 4 * lhalf + 8 * (w >> 1) + 2 * (w & 1)) * VP + t * 32 + lrow;
             a[w] = (uint32_t)e[0] | (uint32_t)e[VP] << 16;
           }
-          ot[t] = mma<T>(a, pf[kk], ot[t]);
+          ot[t] = mma32<T>(a, pf[kk], ot[t]);
         }
     } else {
 #pragma unroll
@@ -282,7 +250,7 @@ __global__ __launch_bounds__(NW * 64) void attention_probs_kernel(const ProbsArg
 #pragma unroll
         for (int i = 0; i < 4; ++i) pf[i] = __builtin_bit_cast(uint32_t, (float)st[n][4 * g + i]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) ot[t] = mma<T>(vf[n][4 * t + g], pf, ot[t]);
+        for (int t = 0; t < 2; ++t) ot[t] = mma32<T>(vf[n][4 * t + g], pf, ot[t]);
       }
     }
   }

@@ -11,54 +11,12 @@
 // with the weights 2^(m_w - max m).
 // One sequence, 12 heads, us per launch before / after: fp16 387 tokens 10.6 / 7.0, fp32 128 tokens 12.7 / 6.3 (1.5 of each
 // is the launch, 1 the first loads; fp32 then runs 64 matrix instructions of 64 cycles in a chain per block of keys).
-#include <type_traits>
-
 #include "attention_common.h"
 
 namespace ttmi {
 namespace {
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef float floatx4 __attribute__((ext_vector_type(4), may_alias));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
-
-constexpr int kD = 64;            // head dim
 constexpr int kQ = 32, kKeys = 32;  // queries per workgroup, keys per block
-
-// D = A B + C over one 16-byte piece of both operands
-template <typename T>
-__device__ __forceinline__ floatx16 mma(const u32x4& a, const u32x4& b, floatx16 c) {
-  if constexpr (std::is_same<T, f16>::value) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
-  } else if constexpr (std::is_same<T, bf16>::value) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      c = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)a[j]), __builtin_bit_cast(float, (uint32_t)b[j]), c, 0, 0, 0);
-    return c;
-  }
-}
-
-// Two probabilities rounded to T, and acc + both of them as rounded (the values the second product consumes).
-template <typename T>
-__device__ __forceinline__ uint32_t pack_probabilities(float lo, float hi, float& sum) {
-  if constexpr (std::is_same<T, f16>::value) {
-    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, halfx2));
-    sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(halfx2, p), halfx2{(_Float16)1.0f, (_Float16)1.0f}, sum, false);
-    return p;
-  } else {
-    const uint32_t p = __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
-    sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, p), bf16x2{(__bf16)1.0f, (__bf16)1.0f}, sum, false);
-    return p;
-  }
-}
 
 // V is [B,h,d,v_pitch]
 template <typename T, int NW>
@@ -155,7 +113,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
         }
     }
 #pragma unroll
-    for (int kk = 0; kk < PIECES; ++kk) st = mma<T>(x.kf[kk], qf[kk], st);
+    for (int kk = 0; kk < PIECES; ++kk) st = mma32<T>(x.kf[kk], qf[kk], st);
     float mx = st[0];
 #pragma unroll
     for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
@@ -178,12 +136,14 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
       for (int w = 0; w < 8; ++w) {
         const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w], scale_log2e, neg_m));
         const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w + 1], scale_log2e, neg_m));
-        pf[w >> 2][w & 3] = pack_probabilities<T>(p0, p1, psum);
+        const uint32_t pair = pack2<T>(p0, p1);
+        pf[w >> 2][w & 3] = pair;
+        psum = add_pair<T>(pair, psum);
       }
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) ot[t] = mma<T>(x.vf[2 * t + kk], pf[kk], ot[t]);
+        for (int t = 0; t < 2; ++t) ot[t] = mma32<T>(x.vf[2 * t + kk], pf[kk], ot[t]);
     } else {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -196,7 +156,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 #pragma unroll
         for (int i = 0; i < 4; ++i) pf[i] = __builtin_bit_cast(uint32_t, (float)st[4 * g + i]);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) ot[t] = mma<T>(x.vf[4 * t + g], pf, ot[t]);
+        for (int t = 0; t < 2; ++t) ot[t] = mma32<T>(x.vf[4 * t + g], pf, ot[t]);
       }
     }
     l_run = l_run * alpha + psum;
