@@ -68,14 +68,6 @@ template <typename Epi>
 struct AddsResidual : std::false_type {};
 template <typename T, int ACT, bool HAS_ACT>
 struct AddsResidual<EpiBias<T, ACT, HAS_ACT, true>> : std::true_type {};
-template <typename T>
-struct RingDest<EpiAlphaBeta<T>> {  // one problem, beta == 0 (see ring_ok)
-  using Elem = T;
-  static constexpr bool split = true;
-  static __device__ __forceinline__ T* column(const EpiAlphaBeta<T>& e, int, int n) { return e.c + n; }
-  static __device__ __forceinline__ int64_t row(const EpiAlphaBeta<T>& e, int m) { return (int64_t)m * e.ldc; }
-  static __device__ __forceinline__ float finish(const EpiAlphaBeta<T>& e, float x) { return x * e.alpha; }
-};
 template <typename T, int ACT, bool HAS_ACT, bool HAS_RES>
 struct RingDest<EpiBias<T, ACT, HAS_ACT, HAS_RES>> {
   using Epi = EpiBias<T, ACT, HAS_ACT, HAS_RES>;
