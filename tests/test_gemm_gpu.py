@@ -785,6 +785,23 @@ def test_gemm_i8_dequant_leaves_the_maxima_for_the_next_quantisation(ttmi, M, N,
     assert torch.equal(q1, q2) and torch.equal(s1[:2], s2[:2])
 
 
+@pytest.mark.parametrize("exponent", [-125, -119, -110, -104, -96, -95, 0, 100])
+def test_quantisation_rounds_as_the_division_does(ttmi, exponent):
+    """rint(x / scale) at the floats around every half-integer, for scales next to powers of two of all sizes: the shared
+    reciprocal must not be used where its remainder would be a subnormal number."""
+    halves = np.arange(127, dtype=np.float32) + np.float32(0.5)
+    for mantissa in (1, 2, 3, 4096, (1 << 23) - 1):
+        scale = np.array([((127 + exponent) << 23) | mantissa], np.uint32).view(np.float32)
+        near = (halves * scale).view(np.uint32)[:, None] + np.arange(-2, 3).astype(np.uint32)
+        x = np.concatenate([np.float32(127) * scale, near.reshape(-1).view(np.float32), -near.reshape(-1).view(np.float32)])
+        scale = x[0] / np.float32(127)
+        want = np.clip(np.rint(x / scale), -127, 127).astype(np.int8)
+        q, found = torch.zeros(x.size, dtype=torch.int8, device="cuda"), torch.zeros(capi.QUANT_SCALE_FLOATS, device="cuda")
+        ok(ttmi.ttmi_quantize_rows_i8(ptr(dev(x)), ptr(q), ptr(found), 1, x.size, stream()))
+        assert host(found)[0] == scale
+        assert np.array_equal(host(q), want)
+
+
 def test_int8_linear_pipeline(ttmi, oracle):
     """quantize -> int8 GEMM -> dequant+bias, against the oracle's statement of the same scheme."""
     rng = np.random.default_rng(3)
