@@ -214,7 +214,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   // are zeroed on the way to LDS (0 * NaN would poison the output).
   // (Named vector registers, not arrays: an array captured by the two lambdas ends up in scratch.)
   u32x4 kreg0{}, kreg1{}, vreg0{}, vreg1{};
-  float mreg = 0.f;
+  uint32_t mreg = 0;
   auto load_regs = [&](int tile) {
     const int key0 = tile * kBKV;
     const int ch = tid & 7, r0 = tid >> 3;  // chunk and row of this lane's first 16-byte piece; second (four wavefronts): row + 32
@@ -235,11 +235,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
       vreg0 = *reinterpret_cast<const u32x4*>(vb + (int64_t)key * kD + dch * 8);
       if (kPieces == 2) vreg1 = *reinterpret_cast<const u32x4*>(vb + (int64_t)key * kD + (dch + 4) * 8);
     }
-    if (tid < kBKV) {
-      const int key = key0 + tid;
-      const float mv = mask ? mask_in_scores(mask[(int64_t)b * seq + min(key, kv_len - 1)], inv_scale) : 0.f;
-      mreg = key < kv_len ? mv : -__builtin_inff();
-    }
+    if (tid < kBKV && mask) mreg = load_mask(mask + (int64_t)b * seq + min(key0 + tid, kv_len - 1));
   };
   auto put_vt = [&](u32x4 x, int tile, int stage, int drow, int ch) {
     if (tile * kBKV + kBKV > kv_len) {  // only the last tile: zero the keys past the end
@@ -278,7 +274,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
       scatter_v(vreg0, stage, tid >> 6);
       if (kPieces == 2) scatter_v(vreg1, stage, (tid >> 6) + 4);
     }
-    if (tid < kBKV) mask_lds(stage)[tid] = mreg;
+    if (tid < kBKV) mask_lds(stage)[tid] = tile * kBKV + tid < kv_len ? mask_in_scores(mreg, inv_scale) : -__builtin_inff();
   };
 
   // One 64-key tile from LDS stage STAGE (a compile-time constant so every LDS address is a

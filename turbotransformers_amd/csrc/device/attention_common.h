@@ -57,20 +57,20 @@ __device__ __forceinline__ float add_pair(uint32_t p, float acc) {
 // the mask of a valid key stays finite however low it is (the lowest float over the scale would be -inf, every probability
 // of such a row 0 and the row 0 / 0), and keys past the end carry -inf, below any mask.  A mask of -inf stays -inf.
 constexpr float kFarthestScore = 0x1p127f;  // the running maximum starts at its negative
-__device__ __forceinline__ float mask_in_scores(float mask, float inv_scale) {
-  // A NaN has to stay one, but attention.hip is compiled as if there were none: the bits are tested, out of the compiler's sight.
-  uint32_t bits = __builtin_bit_cast(uint32_t, mask);
-  asm("" : "+v"(bits));
-  const float x = fminf(fmaxf(mask * inv_scale, -kFarthestScore), kFarthestScore);
-  return __builtin_bit_cast(float, (bits & 0x7f800000u) != 0x7f800000u ? __builtin_bit_cast(uint32_t, x) : bits);
+// The mask is loaded as bits: a NaN has to stay one, but attention.hip is compiled as if there were none.  It is converted where it
+// is used, not where it is requested: the conversion waits for its load, and with it for the older ones of the tile.  us per launch,
+// 12 heads, converted at the request / where used: fp16 4 x 400 tokens 12.2 / 10.9, 8 x 256 7.6 / 7.4, fp32 4 x 400 40.6 / 37.8.
+__device__ __forceinline__ float mask_in_scores(uint32_t mask, float inv_scale) {
+  const float x = fminf(fmaxf(__builtin_bit_cast(float, mask) * inv_scale, -kFarthestScore), kFarthestScore);
+  return __builtin_bit_cast(float, (mask & 0x7f800000u) != 0x7f800000u ? __builtin_bit_cast(uint32_t, x) : mask);
 }
+__device__ __forceinline__ uint32_t load_mask(const float* mask) { return *reinterpret_cast<const __attribute__((may_alias)) uint32_t*>(mask); }
 
 // m * c is rounded.  The error is the same for all keys of a row and cancels in the division by the row's sum, but from
 // |m * c| = 2^30 on it is 64 and more: the probabilities of a row masked with -1e10 would be 0 or infinite.  Beyond 2^12
 // (error 2^-13; no row with an unmasked key comes near) the maximum is subtracted from the scores first, exactly.
-// The test is three instructions per 32 keys: us per launch without / with it, 12 heads, fp16 64 x 512 tokens 82.9 / 83.0, 8 x
-// 256 7.5 / 7.7, 1 x 387 6.6 / 6.6, 20 packed requests 19.3 / 19.3, 32 of them 23.9 / 24.1, fp32 1 x 128 6.5 / 6.5, 20 x 100 14.8 /
-// 14.8, 16 x 512 146.2 / 147.2.  (Joined to the test for a maximum that moves it costs registers: 7.5 / 7.8, 20 requests 19.7.)
+// The test is three instructions per 32 keys, 1 to 2 % of a launch: fp16 1 x 400 tokens 6.6 / 6.8, 32 packed requests 23.8 / 24.0,
+// fp32 16 x 512 146.1 / 146.6.  (Joined to the test for a maximum that moves it costs registers: 8 x 256 7.8 against 7.6.)
 template <typename Scores>
 __device__ __forceinline__ float relative_scores(Scores& st, float m_run, float scale_log2e) {
   const float neg_m = -m_run * scale_log2e;

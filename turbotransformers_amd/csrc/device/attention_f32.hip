@@ -100,7 +100,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   constexpr int kRowsPerPass = NW * 64 / 16;
   const int ch = tid & 15, r0 = tid >> 4;
   floatx4 kreg[kPieces], vreg[kPieces];
-  float mreg = 0.f;
+  uint32_t mreg = 0;
 
 #define TTMI_FA32_LOAD(tile_)                                                                                      \
   do {                                                                                                              \
@@ -115,11 +115,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         vreg[p] = *reinterpret_cast<const floatx4*>(vb + (int64_t)min(key0_ + r_, kv_len - 1) * kD + ch * 4);       \
       }                                                                                                             \
     }                                                                                                               \
-    if (tid < kBKV) {                                                                                               \
-      const int key_ = key0_ + tid;                                                                                 \
-      const float mv_ = mask ? mask_in_scores(mask[(int64_t)b * seq + min(key_, kv_len - 1)], inv_scale) : 0.f;     \
-      mreg = key_ < kv_len ? mv_ : -__builtin_inff();                                                               \
-    }                                                                                                               \
+    if (tid < kBKV && mask) mreg = load_mask(mask + (int64_t)b * seq + min(key0_ + tid, kv_len - 1));               \
   } while (0)
 
 #define TTMI_FA32_STORE(tile_, stage_)                                                                             \
@@ -142,7 +138,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
           *reinterpret_cast<float*>(vt_ + tile_off(ch * 4 + w, r_ >> 2) + (r_ & 3) * 4) = live_ ? x_[w] : 0.f;      \
       }                                                                                                             \
     }                                                                                                               \
-    if (tid < kBKV) reinterpret_cast<float*>(smem + 4 * kTile)[(stage_) * kBKV + tid] = mreg;                       \
+    if (tid < kBKV)                                                                                                 \
+      reinterpret_cast<float*>(smem + 4 * kTile)[(stage_) * kBKV + tid] =                                           \
+          (tile_) * kBKV + tid < kv_len ? mask_in_scores(mreg, inv_scale) : -__builtin_inff();                      \
   } while (0)
 
   // One 64-key tile from LDS stage STAGE.  m_run is kept in raw score units; p = exp2(s*c - m*c), c = scale*log2(e).

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   struct Block {
     u32x4 kf[PIECES];
     u32x4 vf[VPIECES];
-    float mk;  // of key lrow
+    uint32_t mk;  // of key lrow
   };
   const int blocks = (seq + kKeys - 1) / kKeys;
   // Keys past the end repeat valid ones; they carry a mask of -inf, so their probability is 0.
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     const T* row = kb + (int64_t)min(key0 + lrow, seq - 1) * kD + lhalf * KPC;
 #pragma unroll
     for (int kk = 0; kk < PIECES; ++kk) x.kf[kk] = *reinterpret_cast<const u32x4*>(row + 2 * kk * KPC);
-    x.mk = mb != nullptr ? mb[min(key0 + lrow, seq - 1)] : 0.f;
+    x.mk = mb != nullptr ? load_mask(mb + min(key0 + lrow, seq - 1)) : 0u;
     if constexpr (sizeof(T) == 2) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -98,20 +98,6 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
       const float mk = key0 + lrow < seq ? mask_in_scores(x.mk, inv_scale) : -__builtin_inff();
       st = __builtin_amdgcn_mfma_f32_32x32x2f32(lhalf == 0 ? mk : 0.f, 1.f, st, 0, 0, 0);
     }
-    if (ragged) {  // V^T past the last key may hold anything: 0 * NaN would reach the output
-#pragma unroll
-      for (int p = 0; p < VPIECES; ++p)
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-          if constexpr (sizeof(T) == 2) {
-            const int key = key0 + 16 * (p & 1) + 8 * (w >> 1) + 4 * lhalf + 2 * (w & 1);
-            if (key >= seq) x.vf[p][w] = 0u;
-            else if (key + 1 >= seq) x.vf[p][w] &= 0xffffu;
-          } else {
-            if (key0 + 8 * (p & 3) + 4 * lhalf + w >= seq) x.vf[p][w] = 0u;
-          }
-        }
-    }
 #pragma unroll
     for (int kk = 0; kk < PIECES; ++kk) st = mma32<T>(x.kf[kk], qf[kk], st);
     float mx = st[0];
@@ -129,6 +115,22 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 #pragma unroll
       for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
     const float neg_m = relative_scores(st, m_run, scale_log2e);
+    // V^T past the last key may hold anything: 0 * NaN would reach the output.  (Here and not in front of the first product, which
+    // would then wait for V.)
+    if (ragged) {
+#pragma unroll
+      for (int p = 0; p < VPIECES; ++p)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          if constexpr (sizeof(T) == 2) {
+            const int key = key0 + 16 * (p & 1) + 8 * (w >> 1) + 4 * lhalf + 2 * (w & 1);
+            if (key >= seq) x.vf[p][w] = 0u;
+            else if (key + 1 >= seq) x.vf[p][w] &= 0xffffu;
+          } else {
+            if (key0 + 8 * (p & 3) + 4 * lhalf + w >= seq) x.vf[p][w] = 0u;
+          }
+        }
+    }
     float psum = 0.f;
     if constexpr (sizeof(T) == 2) {
       u32x4 pf[2];
