@@ -375,10 +375,11 @@ def test_gemm_bias_layer_norm_fp32_residual(ttmi, oracle, dt, M, N, K):
                                                         (1300, 1000, 1024, 4, True), (520, 200, 256, 2, False)])
 def test_gemm_bias_layer_norm_k_slices_on_the_large_tile_kernel(ttmi, oracle, dt, M, N, K, slices, fp32_residual):
     """The projection in front of a LayerNorm cut along K on the one-wavefront-per-SIMD kernel: (slice, tile) work
-    items, fp32 partial products, summed and normalised by the reduction kernel.  Once where the library chooses that
-    path by itself (the second FFN product of a 6275-token batch: 100 tiles for 256 CUs), and forced onto small and
-    ragged shapes with 2, 3 and 4 slices (switch TTMI_W4_SPLITK).  Against the oracle, and against the same call with
-    the path switched off: both sum fp32 partial sums of the same products, in another order."""
+    items, fp32 partial products, summed and normalised by the reduction kernel.  Forced onto small and ragged shapes
+    with 2, 3 and 4 slices (switch TTMI_W4_SPLITK: the library takes this path by itself for no size), and left to the
+    library's choice for the second FFN product of a 6275-token batch, which the ring tiles hold in fp32.  Against the
+    oracle, and against the same call with the path switched off: both sum fp32 partial sums of the same products, in
+    another order."""
     rng = np.random.default_rng(M + N + K)
     A, W = _ab(rng, M, N, K, 1)
     res = rng.standard_normal((M, N)).astype(np.float32)
@@ -1022,6 +1023,30 @@ def test_attention_with_probs(ttmi, oracle, dt, F, past, fresh, per_query):
                                       ptr(vg), ptr(dev(mask)), int(per_query), ptr(probs), ptr(out), B, h, F, T, d, 0.125,
                                       TTMI_DTYPES[dt], stream()))
     assert torch.equal(kg, dK) and torch.equal(vg, dV)
+    score = oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125)
+    prob = oracle.apply_mask_and_softmax(score, mask.reshape(B, 1, -1, T), 1.0, not per_query)
+    want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, F, h * d)
+    assert max_abs(host(probs), prob) <= (2e-6 if dt == "f32" else GEMM_TOL[dt])
+    assert max_abs(host(out), want) <= (5e-5 if dt == "f32" else GEMM_TOL[dt] * 2)
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("F,past,fresh,per_query", [(1, 40, 1, False), (33, 0, 70, True), (5, 195, 5, True), (2, 298, 2, False)])
+def test_attention_with_probs_masks_far_from_zero(ttmi, oracle, dt, F, past, fresh, per_query):
+    """The lowest float over a whole row (uniform probabilities), over all keys but one, and -inf: the three forms of the kernel."""
+    rng = np.random.default_rng(F + past + fresh)
+    h, d, T = 2, 64, past + fresh
+    rows = [np.full(T, LOWEST), np.full(T, -1e11), np.where(np.arange(T) == T - 1, 0.0, LOWEST), np.where(np.arange(T) < T // 2, -np.inf, 0.0)]
+    B = len(rows)
+    mask = np.repeat(np.stack(rows).astype(np.float32)[:, None], F if per_query else 1, axis=1)
+    Q = rng.standard_normal((B, h, F, d), np.float32)
+    K, V = (rng.standard_normal((B, h, T, d), np.float32) for _ in range(2))
+    dQ, dK, dV = dev(Q, dt), dev(K, dt), dev(V, dt)
+    (kp, kn), (vp, vn) = ((x[:, :, :past].contiguous(), x[:, :, past:].contiguous()) for x in (dK, dV))
+    probs = torch.full((B, h, F, T), 9.0, dtype=dQ.dtype, device="cuda")
+    out = torch.full((B, F, h * d), 9.0, dtype=dQ.dtype, device="cuda")
+    ok(ttmi.ttmi_attention_with_probs(ptr(dQ), ptr(kp) if past else None, ptr(vp) if past else None, past, ptr(kn), ptr(vn), None, None,
+                                      ptr(dev(mask)), int(per_query), ptr(probs), ptr(out), B, h, F, T, d, 0.125, TTMI_DTYPES[dt], stream()))
     score = oracle.batch_matmul(rounded(Q, dt), rounded(K, dt), True, 0.125)
     prob = oracle.apply_mask_and_softmax(score, mask.reshape(B, 1, -1, T), 1.0, not per_query)
     want = oracle.transpose_for_score(oracle.batch_matmul(prob, rounded(V, dt), False)).reshape(B, F, h * d)

@@ -42,9 +42,8 @@ def _both(ttmi, dt, M, N, K, seed, fp32_residual=False):
 
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
 def test_static_scratch_matches_allocating_entry_point_twice_in_a_row(ttmi, dt):
-    """Two calls in a row on the same scratch, the second smaller: a split-K shape on the DMA tiles
-    (M = 2560: three slices, 23.6 MB of partial tiles), then one short sequence (M = 128, a few slices of the
-    one-wavefront-per-tile kernel)."""
+    """Two calls in a row on the same scratch, the second smaller: 2560 rows, whose product is held in fp32 (7.9 MB) on
+    the ring tiles, then one short sequence (M = 128, a few K slices)."""
     _both(ttmi, dt, 2560, 768, 3072, seed=1)
     _both(ttmi, dt, 128, 768, 3072, seed=2)
     _both(ttmi, dt, 100, 768, 768, seed=3)
@@ -64,11 +63,11 @@ def test_static_scratch_unsplit_problems_need_no_scratch(ttmi):
 
 
 def test_static_scratch_and_the_two_slices_of_the_large_tile_kernel(ttmi):
-    """A product of a few thousand rows that the allocating entry point cuts in two on its large-tile kernel: where the
-    two fp32 partial products fit the static buffer (5000 x 768: 30.7 MB) both entry points run the same kernels and
-    agree bit for bit; where they do not (6275 x 768: 38.6 MB) the static form is not refused but runs the product
-    whole, so the two differ by the rounding of the 16-bit product in front of the LayerNorm and no more."""
-    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_W4_SPLITK", 2))  # by itself the library takes two slices from about 5700 rows on
+    """A product of a few thousand rows cut in two on the large-tile kernel (by the switch; by itself the library cuts none
+    there): the two fp32 partial products of 5000 x 768 fit the static buffer (30.7 MB), and both entry points run the same
+    kernels and agree bit for bit.  6275 x 768 as the library runs it, whole and in fp32 on the ring tiles (19.3 MB): the two
+    entry points agree as closely as the rounding of a 16-bit product would allow."""
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_W4_SPLITK", 2))
     try:
         _both(ttmi, "f16", 5000, 768, 3072, seed=11)
     finally:
@@ -91,8 +90,8 @@ def test_static_scratch_and_the_two_slices_of_the_large_tile_kernel(ttmi):
 
 
 def test_static_scratch_refuses_what_does_not_fit(ttmi):
-    """With the admitted size lowered to 1 MiB the K slices of 2560 x 768 x 3072 (23.6 MB of partial tiles) no longer
-    fit: the call is refused with TTMI_EINVAL and a message that names both sizes, nothing is launched and `out`
+    """With the admitted size lowered to 1 MiB the fp32 product of 2560 x 768 x 3072 (7.9 MB) no longer
+    fits: the call is refused with TTMI_EINVAL and a message that names both sizes, nothing is launched and `out`
     keeps its contents; the allocating entry point and a later call with the limit lifted are unaffected."""
     M, N, K = 2560, 768, 3072
     rng = np.random.default_rng(7)
