@@ -60,14 +60,14 @@ TTMI_API const char* ttmi_last_error(void);
  * launchers would not pick for them.  No counterpart in the reference (cuBLAS and the CUDA kernels have no such
  * knob).  Names and values:
  *   "TTMI_LARGE_TILE"       1 = every eligible 16-bit product on the one-wavefront-per-SIMD GEMM kernel, 0 = none;
- *   "TTMI_WAVE_KERNEL"      0 = products of at most 128 rows stay on the LDS-tiled kernels;
+ *   "TTMI_WAVE_KERNEL"      0 = products of at most 128 rows that would take the wavefront kernel stay on the others;
  *   "TTMI_ATTENTION_WAVES"  4 / 8 = wavefronts per workgroup of the one-kernel attention; 1 = its form whose
  *                           wavefronts share the keys of a head, where that form exists (dense batches with V transposed);
  *   "TTMI_STATIC_SCRATCH_LIMIT"  bytes of its buffer ttmi_gemm_bias_layer_norm_static admits (to test its refusal);
  *   "TTMI_W4_A_STAGES"      2 = the one-wavefront-per-SIMD GEMM kernel keeps two LDS stages for the A operand
  *                           where it would take three;
- *   "TTMI_W4_SPLITK"        0 = ttmi_gemm_bias_layer_norm never cuts a product along K on that kernel, n >= 2 = n
- *                           slices for every product that can be cut that way;
+ *   "TTMI_W4_SPLITK"        n >= 2 = ttmi_gemm_bias_layer_norm cuts every product that allows it into n K slices on that
+ *                           kernel, 0 = never (the launcher by itself cuts none there);
  *   -1 = the launcher decides (the default).
  * Each switch starts from the environment variable of the same name, which is read once, at the first launch or
  * the first call of this function; later changes of the environment are not seen. */
@@ -389,9 +389,12 @@ TTMI_API int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const 
                                         const ttmi_epilogue_args* args, int dtype, void* stream);
 
 /* Which kernel variant ttmi_gemm (epilogue TTMI_EPI_NONE, args NULL) or ttmi_gemm_fused would launch for an
- * aligned, densely packed product of this shape, as text: family (reg = register-staged, dma = global->LDS DMA,
- * dma_agpr = DMA with accumulators in AGPRs, dma3_agpr = the same with a third LDS stage for the A operand, wave = one wavefront per tile with its operand fragments straight from
- * global memory), wavefronts per workgroup, tile, K split; e.g. "dma8w_256x256", "wave1w_32x32_splitk3".
+ * aligned, densely packed product of this shape, as text: family (reg = register-staged; dma = any kernel that fills
+ * LDS by global->LDS DMA, the ring tiles, the form for few rows (16 wavefronts, tiles 16 columns wide) and the older
+ * tiles alike; dma_agpr = the one-wavefront-per-SIMD kernel, accumulators in AGPRs, dma3_agpr = the same with a third
+ * LDS stage for the A operand; wave = one wavefront per tile with its operand fragments straight from global memory),
+ * wavefronts per workgroup, tile, K split; e.g. "dma8w_256x256", "wave1w_32x32_splitk3".  The name does not tell ring
+ * and older tiles of one size apart.
  * Nothing is launched.  No counterpart in the reference (cuBLAS picks its kernels out of sight); measurement
  * scripts use it to tie recorded per-kernel figures to the variant they were recorded on.  For the QKV epilogues
  * `args` supplies seq / heads / head_dim / v_seq_pitch (and batch); pointers in it are ignored. */

@@ -1488,8 +1488,9 @@ inline int pick_splits(int64_t m, int64_t n, int64_t ksteps, int64_t batch, size
   return (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)compute_units() / tiles, ksteps / 4, 16}));
 }
 
-// The wavefront kernel takes 16-bit problems of at most 128 rows on the [N,K] path (TTMI_WAVE_KERNEL=0 keeps them on
-// the 64 x 64 tiles, for A/B timing).
+// The wavefront kernel takes 16-bit problems of at most 128 rows on the [N,K] path: plain products, what the ring tiles refuse,
+// and the GELU products that keep their form (RingKernel::keeps_named_form).  TTMI_WAVE_KERNEL=0 keeps them off it, for A/B
+// timing.
 constexpr int kWaveDepth = 4;  // K steps a wavefront keeps in flight: 32 loads of 16 bytes per lane
 template <typename T>
 inline bool wave_kernel_ok(const GemmArgs& g, int batch, bool aligned) {
