@@ -439,6 +439,43 @@ def test_product_in_front_of_a_layer_norm_is_held_in_fp32(ttmi, dt, static, M, N
     assert torch.all(out[M:] == -7.0)
 
 
+def test_captured_product_survives_larger_ones_on_its_stream(ttmi):
+    """The workspace of a stream does not move: a product in K slices is captured, then the same stream runs the largest
+    product that is held in fp32 (32 MiB of workspace), and every replay still equals the eager result."""
+    M, N, K = 128, 768, 3072
+    g = torch.Generator(device="cuda").manual_seed(0)
+    new = lambda *shape: torch.randn(shape, generator=g, device="cuda").half()
+    A, W, res, bias, gamma, beta = new(M, K), new(N, K) / 55, new(M, N), new(N), new(N), new(N)
+    big = [new(8192, 4096), new(1024, 4096) / 64, new(8192, 1024), new(1024), new(1024), new(1024)]
+    out, want, big_out = torch.zeros_like(res), torch.zeros_like(res), torch.zeros_like(big[2])
+    side = torch.cuda.Stream()
+
+    def call(dst, ops, m, n, k):
+        a, w, r, b, ga, be = ops
+        ok(ttmi.ttmi_gemm_bias_layer_norm(ptr(a), ptr(w), ptr(dst), ptr(r), None, ptr(b), ptr(ga), ptr(be), None, m, n, k, 1e-12,
+                                          TTMI_DTYPES["f16"], stream()))
+
+    small = (A, W, res, bias, gamma, beta)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(out, small, M, N, K)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        call(out, small, M, N, K)
+    for turn in range(3):
+        A.copy_(new(M, K))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            call(big_out, big, 8192, 1024, 4096)
+            call(want, small, M, N, K)
+        torch.cuda.synchronize()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert not torch.isnan(want).any() and torch.equal(out, want), "replay %d" % turn
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("forced", [False, True])
 @pytest.mark.parametrize("M,N,K,with_bias", [(300, 200, 256, True), (4100, 1024, 1024, False), (2560, 768, 3072, True),

@@ -1427,8 +1427,10 @@ inline int launch_fast(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
   return launch_status("gemm_fast_kernel");
 }
 
-// Workspace of the split-K path: one buffer per stream, grown on demand, kept for the life of
-// the process (work on one stream is ordered, so consecutive GEMMs can share it).
+// Workspace of the split-K path: one buffer per stream, kept for the life of the process (work on one stream is ordered, so
+// consecutive GEMMs can share it).  It is allocated in the size of the static buffer, which no selection exceeds by itself, so
+// it never moves: a graph that was captured with it stays valid whatever sizes the stream sees later.  (Only slices forced
+// through a kernel switch can outgrow it.)
 //
 // A caller that must not allocate (ttmi_gemm_bias_layer_norm_static) installs a fixed buffer for
 // the duration of its call on its thread; then that buffer is handed out, or the request is
@@ -1463,7 +1465,7 @@ inline int splitk_workspace(size_t bytes, hipStream_t s, float** out) {
       (void)hipFree(slot.ptr);
       slot = Slot{};
     }
-    const size_t want = std::max(bytes, (size_t)8 << 20);
+    const size_t want = std::max(bytes, (size_t)TTMI_STATIC_SCRATCH_BYTES);
     void* p = nullptr;
     if (hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
