@@ -30,7 +30,7 @@ extern "C" {
 
 #define TTMI_API __attribute__((visibility("default")))
 
-enum ttmi_dtype { TTMI_F32 = 0, TTMI_F16 = 1, TTMI_BF16 = 2, TTMI_I8 = 3, TTMI_I32 = 4, TTMI_I64 = 5 };
+enum ttmi_dtype { TTMI_F32 = 0, TTMI_F16 = 1, TTMI_BF16 = 2, TTMI_I8 = 3, TTMI_I32 = 4, TTMI_I64 = 5, TTMI_F32_PACKED = 6 };
 enum ttmi_act { TTMI_ACT_NONE = -1, TTMI_ACT_GELU = 0, TTMI_ACT_TANH = 1, TTMI_ACT_RELU = 2 };
 enum ttmi_memcpy_kind { TTMI_H2D = 0, TTMI_D2H = 1, TTMI_D2D = 2 };
 enum ttmi_status {
@@ -365,6 +365,16 @@ typedef struct ttmi_epilogue_args {
   int64_t v_seq_pitch;       /* 0: v is [B,h,S,d]; > 0: v is written transposed as
                                 [B,h,d,v_seq_pitch] (multiple of 8, >= seq)  (QKV_SPLIT*)    */
 } ttmi_epilogue_args;
+
+/* Weights of fp32 products, laid out once for the kernels that form fp32 products on the 16-bit matrix instructions: n rows of k
+ * floats (k a multiple of TTMI_PACKED_WEIGHT_K), written by the caller, and behind them what ttmi_split_weights computes from
+ * them, TTMI_PACKED_WEIGHT_FLOATS(n, k) floats in all, 16-byte aligned.  ttmi_gemm_fused, ttmi_layer_norm_gemm_fused,
+ * ttmi_gemm_bias_layer_norm[_static] and ttmi_gemm_describe take them as their weight with dtype TTMI_F32_PACKED (ldb = k);
+ * everything else about such a call is as with TTMI_F32.  Infinities, NaNs and rows of any magnitude are allowed: what the halves
+ * do not hold is computed from the fp32 rows.  No counterpart in the reference (cuBLAS takes its weights as they are). */
+#define TTMI_PACKED_WEIGHT_K 32
+#define TTMI_PACKED_WEIGHT_FLOATS(n, k) (2 * (n) * (k) + (n))
+TTMI_API int ttmi_split_weights(void* packed, int64_t n, int64_t k, void* stream);
 
 /* MatMul with the following memory-bound op folded into the store of the accumulators:
  *   BIAS_ACT       = MatMul + AddBiasAct            (layers/bert_intermediate.cpp:43-46)

@@ -1199,3 +1199,115 @@ def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps)
                                        ctypes.byref(args), TTMI_DTYPES[dt], stream()))
     assert max_abs(host(q[:M]).reshape(M, N), base) <= GEMM_TOL[dt] * 3
     assert torch.all(q[M:] == -7.0)
+
+
+def _packed(ttmi, W):
+    """fp32 weights [N, K] as ttmi_split_weights lays them out."""
+    N, K = W.shape
+    p = torch.full((2 * N * K + N, ), float("nan"), device="cuda")
+    p[:N * K] = W.flatten()
+    ok(ttmi.ttmi_split_weights(ptr(p), N, K, stream()))
+    return p
+
+
+def _split_error_bound(A, W):
+    """Per element.  Halves of 11 bits leave 2^-22 of a value and drop the product of the low ones (2^-22): 3 * 2^-22 of sum |a b|.
+    The sums: one rounding (2^-24) per 32 products of each kind, of partial sums no larger than sum |a b|."""
+    absolute = A.double().abs() @ W.double().abs().T
+    return absolute * (3 * 2.0**-22 + (A.shape[1] / 32 + 8) * 2.0**-23)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 8, 32), (40, 72, 64), (100, 776, 96), (129, 2304, 768), (264, 768, 3072), (387, 3072, 768),
+                                   (1000, 1536, 160), (1999, 768, 768), (2000, 3072, 128), (2500, 2304, 768), (8200, 520, 256)])
+def test_packed_weights(ttmi, M, N, K):
+    """fp32 products on the 16-bit matrix instructions: every tile, ragged rows and columns, one to many K steps, K slices, every
+    epilogue; rows past M stay untouched.  No further from 64 bits than the fp32 instruction is."""
+    import ctypes
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    A, W, bias, res = rand(M, K), rand(N, K) * 0.02, rand(N), rand(M, N)
+    P, base = _packed(ttmi, W), A.double() @ W.double().T
+    bound = _split_error_bound(A, W) + 2.0**-22 * (1 + bias.abs() + res.abs()).double()
+    error = {}
+    for name, epi, args, want in (("bias", capi.EPI_BIAS, _epi(bias=bias), base + bias.double()),
+                                  ("relu", capi.EPI_BIAS_ACT, _epi(bias=bias, act=capi.ACT_RELU), (base + bias.double()).relu()),
+                                  ("residual", capi.EPI_BIAS_RESIDUAL, _epi(bias=bias, residual=res), base + bias.double() + res.double()),
+                                  ("f32", capi.EPI_F32_OUT, _epi(), base)):
+        for weight, dt in ((P, capi.F32_PACKED), (W, capi.F32)):
+            C = torch.full((M + 40, N), -7.0, device="cuda")
+            ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(weight), ptr(C), M, N, K, K, K, N, epi, ctypes.byref(args), dt, stream()))
+            assert torch.all(C[M:] == -7.0)
+            error[name, dt] = (C[:M].double() - want).norm()
+            if dt == capi.F32_PACKED:
+                assert bool(((C[:M].double() - want).abs() <= bound).all()), name
+    if K >= 96:
+        assert float(error["f32", capi.F32_PACKED]) <= float(error["f32", capi.F32])
+    if N <= 4096:
+        one, zero, out, out2 = torch.ones(N, device="cuda"), torch.zeros(N, device="cuda"), torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+        x = base + res.double() + bias.double()
+        want = torch.nn.functional.layer_norm(x, (N, ), eps=1e-5)
+        for fn, dst in ((ttmi.ttmi_gemm_bias_layer_norm, out), (ttmi.ttmi_gemm_bias_layer_norm_static, out2)):
+            ok(fn(ptr(A), ptr(P), ptr(dst), ptr(res), None, ptr(bias), ptr(one), ptr(zero), None, M, N, K, 1e-5, capi.F32_PACKED, stream()))
+        assert torch.equal(out, out2)
+        assert float((out.double() - want).abs().max()) <= LN_TOL["f32"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("v_transposed", [False, True])
+@pytest.mark.parametrize("B,S,h", [(7, 5, 12), (1, 37, 16), (9, 31, 12), (7, 130, 12), (2, 387, 16), (20, 100, 12)])
+def test_packed_weights_head_split(ttmi, v_transposed, B, S, h):
+    """The QKV projection: row by row and through the column pass of a transposed V (sequences off every grid)."""
+    import ctypes
+    d, H = 64, h * 64
+    g = torch.Generator(device="cuda").manual_seed(S + h)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    A, W, bias = rand(B * S, H), rand(3 * H, H) * 0.02, rand(3 * H)
+    pitch = (S + 7) // 8 * 8 if v_transposed else 0
+    q, k = (torch.full((B, h, S, d), float("nan"), device="cuda") for _ in range(2))
+    v = torch.full((B, h, d, pitch) if v_transposed else (B, h, S, d), 7.0, device="cuda")
+    args = _epi(bias=bias, q=q, k=k, v=v, seq=S, heads=h, head_dim=d, v_seq_pitch=pitch)
+    ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, W)), None, B * S, 3 * H, H, H, H, 3 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args),
+                            capi.F32_PACKED, stream()))
+    split = lambda x: x.view(B, S, 3, h, d).permute(2, 0, 3, 1, 4)
+    want = split(A.double() @ W.double().T + bias.double())
+    bound = split(_split_error_bound(A, W) + 2.0**-22 * (1 + bias.abs()).double())
+    if v_transposed:
+        assert torch.all(v[..., S:] == 7.0)
+        v = v[..., :S].transpose(2, 3)
+    for i, got in enumerate((q, k, v)):
+        assert bool(((got.double() - want[i]).abs() <= bound[i]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(70, 136, 96), (300, 768, 768), (2000, 768, 768)])
+def test_packed_weights_outside_the_window(ttmi, M, N, K):
+    """Rows of either operand whose largest value the halves do not hold (tiny, huge, zero, infinite, NaN) come out as the fp32
+    instruction gives them: to fp32 accuracy of the row, infinities and NaNs where they belong."""
+    import ctypes
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A, W = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 0.02
+    A[3] *= 1e-9
+    A[17] *= 1e6
+    A[18] = 0
+    A[40] *= 2.0**-12
+    A[33, :5] = torch.tensor([5e4, -3e5, 1.0, 1e-6, 0.0], device="cuda")
+    W[7] *= 1e-12
+    W[8] = 0
+    W[50] *= 1e8
+    want = A.double() @ W.double().T
+    bound = (A.double().abs() @ W.double().abs().T) * (K + 8) * 2.0**-24 + 1e-37
+    C = torch.empty(M, N, device="cuda")
+
+    def run(A, W):
+        C.fill_(7.0)
+        ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, W)), ptr(C), M, N, K, K, K, N, capi.EPI_F32_OUT, ctypes.byref(_epi()), capi.F32_PACKED, stream()))
+        return C.double()
+
+    assert bool(((run(A, W) - want).abs() <= bound).all())
+    A[20, 2], A[21, 3], A[60, 9], W[70, 4] = float("inf"), float("-inf"), float("nan"), float("inf")
+    want = A.double() @ W.double().T
+    got = run(A, W)
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
+    assert bool(((got - want).abs() <= bound)[finite].all())

@@ -3,6 +3,7 @@
 #include <cstring>
 
 #include "gemm_impl.h"
+#include "split_f32.h"
 
 namespace ttmi {
 
@@ -18,7 +19,7 @@ template <typename T>
 int gemm_norm_fused_typed(const GemmArgs& g, const void* gamma, const void* beta, float eps, void* c, int64_t ldc, int epilogue,
                           const ttmi_epilogue_args* args, hipStream_t s);
 template <typename T>
-int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
+int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* out, const void* residual, const float* residual_f32,
                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
                                int64_t k, float eps, int dtype, hipStream_t s);
 
@@ -48,6 +49,40 @@ static int static_scratch(float** out) {
   return 0;
 }
 
+// TTMI_F32_PACKED: fp32 with packed weights.
+static int packed_operand(int* dtype, int64_t k, int64_t ldb, bool* packed) {
+  *packed = *dtype == TTMI_F32_PACKED;
+  if (*packed) {
+    TTMI_REQUIRE(k % TTMI_PACKED_WEIGHT_K == 0 && ldb == k, "packed weights are contiguous rows of whole groups of K");
+    *dtype = TTMI_F32;
+  }
+  return 0;
+}
+
+// The halves of packed weights (split_f32.h) behind their fp32 rows, and per row whether its largest value is outside the window
+// in which they hold it.  Once per weight: one workgroup per row, 16 bytes of it per thread and turn.
+static __global__ __launch_bounds__(256) void split_weights_kernel(float* __restrict__ packed, int n, int k) {
+  __shared__ float part[256 / kWave];
+  const int row = blockIdx.x;
+  const float* src = packed + (int64_t)row * k;
+  char* dst = reinterpret_cast<char*>(packed + (int64_t)n * k + (int64_t)row * k);
+  float largest = 0.f;
+  for (int col = threadIdx.x * 4; col < k; col += 1024) {
+    const float4 x = *reinterpret_cast<const float4*>(src + col);
+    const uint2 hi = make_uint2(split_hi(x.x, x.y), split_hi(x.z, x.w));
+    char* group = dst + (col / TTMI_PACKED_WEIGHT_K) * (TTMI_PACKED_WEIGHT_K * 4) + (col % TTMI_PACKED_WEIGHT_K) * 2;
+    *reinterpret_cast<uint2*>(group) = hi;
+    *reinterpret_cast<uint2*>(group + TTMI_PACKED_WEIGHT_K * 2) = make_uint2(split_lo(hi.x, x.x, x.y), split_lo(hi.y, x.z, x.w));
+    split_max(largest, x.x, x.y);
+    split_max(largest, x.z, x.w);
+  }
+  largest = group_max<kWave>(largest);
+  if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = largest;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    reinterpret_cast<int*>(packed + 2 * (int64_t)n * k)[row] = split_outside(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+}
+
 static int gemm_bias_layer_norm_impl(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
                               const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
                               int64_t k, float eps, int dtype, void* stream) {
@@ -59,7 +94,10 @@ static int gemm_bias_layer_norm_impl(const void* a, const void* w, void* out, co
   TTMI_REQUIRE(m >= 0 && n >= 0 && m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension out of range");
   if (m == 0 || n == 0) return 0;
   TTMI_REQUIRE(k > 0, "K must be positive");
-  TTMI_DISPATCH_FLOAT(dtype, T, return gemm_bias_layer_norm_typed<T>(a, w, out, residual, residual_f32, bias, gamma, beta, out_f32, m,
+  bool packed = false;
+  const int rc = packed_operand(&dtype, k, k, &packed);
+  if (rc != 0) return rc;
+  TTMI_DISPATCH_FLOAT(dtype, T, return gemm_bias_layer_norm_typed<T>(a, w, packed, out, residual, residual_f32, bias, gamma, beta, out_f32, m,
                                                                      n, k, eps, dtype, (hipStream_t)stream));
   return 0;
 }
@@ -109,12 +147,16 @@ int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, int64_t n,
   TTMI_REQUIRE(a && b && args, "null argument");
   TTMI_REQUIRE(m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension too large");
   TTMI_REQUIRE(lda >= k && ldb >= k, "leading dimension too small");
+  bool packed = false;
+  const int rc = packed_operand(&dtype, k, ldb, &packed);
+  if (rc != 0) return rc;
   GemmArgs g{};
   g.a = (const char*)a;
   g.b = (const char*)b;
   g.m = (int)m; g.n = (int)n; g.k = (int)k;
   g.lda = lda; g.ldb = ldb;
   g.inner = 1;
+  if (packed) use_packed_weights(g);
   TTMI_DISPATCH_FLOAT(dtype, T, return gemm_fused_typed<T>(g, c, ldc, epilogue, args, (hipStream_t)stream, nullptr));
   return 0;
 }
@@ -130,12 +172,23 @@ int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const void* bet
   g.m = (int)m; g.n = (int)n; g.k = (int)k;
   g.lda = k; g.ldb = k;
   g.inner = 1;
-  int rc = kNormNotTaken;
-  TTMI_DISPATCH_FLOAT(dtype, T, rc = gemm_norm_fused_typed<T>(g, gamma, beta, eps, c, ldc, epilogue, args, (hipStream_t)stream));
+  bool packed = false;
+  int base = dtype, rc = packed_operand(&base, k, k, &packed);
+  if (rc != 0) return rc;
+  rc = kNormNotTaken;
+  TTMI_DISPATCH_FLOAT(base, T, rc = gemm_norm_fused_typed<T>(g, gamma, beta, eps, c, ldc, epilogue, args, (hipStream_t)stream));
   if (rc != kNormNotTaken) return rc;
-  rc = ttmi_layer_norm_from(normed, x, gamma, beta, m, k, eps, dtype, stream);
+  rc = ttmi_layer_norm_from(normed, x, gamma, beta, m, k, eps, base, stream);
   if (rc != 0) return rc;
   return ttmi_gemm_fused(normed, w, c, m, n, k, k, k, ldc, epilogue, args, dtype, stream);
+}
+
+int ttmi_split_weights(void* packed, int64_t n, int64_t k, void* stream) {
+  TTMI_REQUIRE(packed != nullptr && aligned16(packed), "packed weights must be 16-byte aligned");
+  TTMI_REQUIRE(n >= 0 && k >= 0 && n < (1ll << 31) && k < (1ll << 31) && k % TTMI_PACKED_WEIGHT_K == 0, "weight size");
+  if (n == 0 || k == 0) return 0;
+  hipLaunchKernelGGL(split_weights_kernel, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream, (float*)packed, (int)n, (int)k);
+  return launch_status("split_weights_kernel");
 }
 
 int ttmi_gemm_describe(int64_t m, int64_t n, int64_t k, int epilogue, const ttmi_epilogue_args* args, int dtype, char* out,

@@ -18,7 +18,7 @@
 // Six decoder layers, fp16, 8 x 1 tokens, 41 keys: 67 launches and 343 us a step before, 49 and 264 after.
 #pragma once
 
-#include "gemm_ring.h"
+#include "gemm_split.h"
 
 namespace ttmi {
 

@@ -140,7 +140,14 @@ struct GemmArgs {
   // One-wavefront-per-SIMD kernel only: a column at which a new run of tiles starts (0 = none).  Tile columns
   // [0, split_tiles) cover [0, split_col), the last of them ragged; the tiles after them start at split_col again.
   int split_col, split_tiles;
+  // fp32 products with packed weights (gemm_split.h): b is their fp32 part, these the halves and the per-row flags; else null
+  const char* b_split;
+  const int* b_outside;
 };
+inline void use_packed_weights(GemmArgs& g) {
+  g.b_split = g.b + (int64_t)g.n * g.k * 4;
+  g.b_outside = reinterpret_cast<const int*>(g.b + (int64_t)g.n * g.k * 8);
+}
 
 // ------------------------------------------------------------------------ epilogues -----
 // After the K loop each wavefront transposes its accumulators through LDS so that a lane holds

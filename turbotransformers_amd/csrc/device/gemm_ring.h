@@ -490,7 +490,19 @@ struct RingTile {
   X(128, 192, 4, 2, 3, 1, 8.73f, 10.6f, 0.465f, 0.465f)      \
   X(256, 128, 4, 2, 3, 1, 11.0f, 10.9f, 0.594f, 0.594f)
 
+// X(BM, BN, WM, WN, A steps in registers, B stages, resident, first, again, lone, shared): fp32 with packed weights (gemm_split.h).
+// Fits of the same kind (M = 40 ... 10240, hidden 768 and 1024; the tile the model picks is 0.14 % slower than the best one).
+#define TTMI_SPLIT_TILES(X)                                     \
+  X(32, 64, 2, 2, 4, 6, 2, 3.43f, 1.13f, 0.252f, 0.167f)        \
+  X(64, 64, 4, 2, 4, 6, 2, 3.74f, 1.81f, 0.313f, 0.250f)        \
+  X(64, 128, 2, 4, 4, 6, 1, 4.29f, 5.50f, 0.397f, 0.397f)       \
+  X(64, 192, 4, 2, 2, 4, 1, 5.33f, 8.27f, 0.512f, 0.512f)       \
+  X(64, 256, 2, 4, 2, 4, 1, 5.66f, 10.4f, 0.608f, 0.607f)       \
+  X(128, 128, 4, 2, 2, 4, 1, 5.94f, 10.5f, 0.571f, 0.571f)      \
+  X(128, 192, 4, 2, 2, 4, 1, 7.84f, 16.2f, 0.718f, 0.718f)
+
 #define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
+#define TTMI_SPLIT_ROW(BM, BN, WM, WN, DA, SB, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
 template <size_t ELEM>
 struct RingTiles;
 template <>
@@ -505,7 +517,11 @@ template <>
 struct RingTiles<1> {
   static constexpr RingTile k[] = {TTMI_RING_TILES_8(TTMI_RING_ROW)};
 };
+struct SplitTiles {
+  static constexpr RingTile k[] = {TTMI_SPLIT_TILES(TTMI_SPLIT_ROW)};
+};
 #undef TTMI_RING_ROW
+#undef TTMI_SPLIT_ROW
 
 enum class RingUse { kWhole, kSliced, kCut, kLayerNorm };  // never cut along K / cut where it pays / always cut / slices summed by the LayerNorm
 struct RingPlan {
@@ -516,10 +532,10 @@ struct RingPlan {
 
 // column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V)
 constexpr int kRingColumns = 32;  // the narrowest wavefront's: a limit that is no multiple of it suits no tile
-template <typename T>
+template <typename Tiles>
 constexpr bool ring_columns_ok() {
   bool narrowest = false;
-  for (const RingTile& t : RingTiles<sizeof(T)>::k) {
+  for (const RingTile& t : Tiles::k) {
     if (t.wave_cols % kRingColumns != 0) return false;
     narrowest = narrowest || t.wave_cols == kRingColumns;
   }
@@ -530,9 +546,9 @@ constexpr bool ring_columns_ok() {
 // number of slices can win any more (the partial products so far, and K shared evenly by all CUs, already take longer).
 // Host time, ns, with a plain loop / so: fp32 128 x 768 x 3072 2070 / 260, fp16 8 x 768 x 3072 2310 / 190, 2000 x 768 x 3072
 // 730 / 110, whole 145 / 80.
-template <typename T>
-inline RingPlan pick_ring(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit = 0) {
-  static_assert(ring_columns_ok<T>(), "kRingColumns");
+template <typename Tiles>
+inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit) {
+  static_assert(ring_columns_ok<Tiles>(), "kRingColumns");
   constexpr uint32_t kMostSlices = 16;
   constexpr uint64_t kMostTiles = 1u << 27;  // (launch_ring refuses such grids: 32-bit arithmetic suffices)
   const uint32_t cus = (uint32_t)compute_units(), rows = (uint32_t)m, cols = (uint32_t)n, steps = (uint32_t)ksteps;
@@ -544,7 +560,7 @@ inline RingPlan pick_ring(int64_t m, int64_t n, int64_t ksteps, RingUse use, int
   for (uint32_t s = 1; s <= most; ++s) share[s] = (steps + s - 1) / s;
   RingPlan best;
   int index = 0;
-  for (const RingTile& t : RingTiles<sizeof(T)>::k) {
+  for (const RingTile& t : Tiles::k) {
     const int i = index++;
     if (column_limit > 0 && column_limit % t.wave_cols != 0) continue;
     const uint32_t tiles = (uint32_t)std::min<uint64_t>((uint64_t)((rows + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn), kMostTiles);
@@ -565,6 +581,13 @@ inline RingPlan pick_ring(int64_t m, int64_t n, int64_t ksteps, RingUse use, int
   }
   return best;
 }
+template <typename T>
+inline RingPlan pick_ring(const GemmArgs& g, RingUse use, int64_t column_limit = 0) {
+  const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T));
+  if constexpr (sizeof(T) == 4)
+    if (g.b_split != nullptr) return pick_tile_of<SplitTiles>(g.m, g.n, ksteps, use, column_limit);
+  return pick_tile_of<RingTiles<sizeof(T)>>(g.m, g.n, ksteps, use, column_limit);
+}
 
 template <typename T>
 inline bool ring_operands_ok(const GemmArgs& g) {  // 32-bit buffer offsets, columns in groups of eight
@@ -572,9 +595,21 @@ inline bool ring_operands_ok(const GemmArgs& g) {  // 32-bit buffer offsets, col
   return g.n % 8 == 0 && (int64_t)g.m * g.lda * (int64_t)sizeof(T) < limit && (int64_t)g.n * g.ldb * (int64_t)sizeof(T) < limit;
 }
 
+template <int BM, int BN, int WM, int WN, int DA, int SB, typename Epi>
+int launch_split(GemmArgs g, const Epi& epi, int slices, hipStream_t s);  // gemm_split.h
+
 template <typename T, typename Epi>
 inline int launch_ring_tile(int tile, const GemmArgs& g, const Epi& epi, int slices, hipStream_t s) {
   int index = 0;
+  if constexpr (sizeof(T) == 4) {
+    if (g.b_split != nullptr) {
+#define TTMI_SPLIT_TRY(BM, BN, WM, WN, DA, SB, R, F, A, L, S) \
+  if (tile == index++) return launch_split<BM, BN, WM, WN, DA, SB>(g, epi, slices, s);
+      TTMI_SPLIT_TILES(TTMI_SPLIT_TRY)
+#undef TTMI_SPLIT_TRY
+      return fail(TTMI_EINVAL, "no such tile");
+    }
+  }
 #define TTMI_RING_TRY(BM, BN, WM, WN, NS, R, F, A, L, S) \
   if (tile == index++) return launch_ring<T, BM, BN, WM, WN, NS>(g, epi, slices, s);
   if constexpr (sizeof(T) == 2) { TTMI_RING_TILES_16(TTMI_RING_TRY) }

@@ -1,4 +1,5 @@
-// Selection for the products with an epilogue: few rows (gemm_flat.h), mid-size (gemm_ring.h), or for large problems the
+// Selection for the products with an epilogue: few rows (gemm_flat.h), mid-size (gemm_ring.h), fp32 with packed weights
+// (gemm_split.h), or for large problems the
 // persistent tiles of gemm_w4.h (16-bit types) and of gemm_fast_kernel (int8).
 #pragma once
 
@@ -38,8 +39,8 @@ struct RingKernel {
     constexpr bool cut = std::is_same<typename Epi::Acc, float>::value;
     RingUse use = cut && column_limit(epi) == 0 ? RingUse::kSliced : RingUse::kWhole;
     if constexpr (IsGelu<Epi>::value && sizeof(T) == 4)
-      if (keeps_named_form(g)) use = RingUse::kCut;
-    return pick_ring<T>(g.m, g.n, g.k / (kRowBytes / (int)sizeof(T)), use, column_limit(epi));
+      if (g.b_split == nullptr && keeps_named_form(g)) use = RingUse::kCut;
+    return pick_ring<T>(g, use, column_limit(epi));
   }
   static bool ok(const GemmArgs& g, const Epi& epi, int batch) {
     return batch == 1 && g.k_chunk == 0 && ring_operands_ok<T>(g) && epilogue_vec(epi) && column_limit(epi) % kRingColumns == 0;

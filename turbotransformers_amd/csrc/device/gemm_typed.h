@@ -142,7 +142,7 @@ inline bool fp32_product_expected(int64_t m, int64_t n, int64_t k) {
 
 // Product + AddBiasLayerNorm.
 template <typename T>
-int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
+int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* out, const void* residual, const float* residual_f32,
                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
                                int64_t k, float eps, int dtype, hipStream_t s) {
   constexpr int KPC = 16 / sizeof(T), BK = kRowBytes / sizeof(T);
@@ -157,6 +157,7 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
   g.m = (int)m; g.n = (int)n; g.k = (int)k;
   g.lda = k; g.ldb = k;
   g.inner = 1;
+  if (packed) use_packed_weights(g);
   auto reduce = [&](const float* ws, int slices, bool, hipStream_t st) {
     auto launch = [&](auto iters) {
       hipLaunchKernelGGL((splitk_reduce_layer_norm_kernel<T, decltype(iters)::value>), dim3((unsigned)m), dim3(256), 0, st, ws,
@@ -189,7 +190,7 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
     // Few rows: one slice; more of K is cheaper cut (10 x 768 x 3072 in twelve slices 3.8 us, whole 5.4), and so is fp32
     // (128 x 768 x 768 in five slices 5.7 us, whole 6.6).
     const bool flat = sizeof(T) == 2 && flat_wins<T>(g, 32);
-    const RingPlan plan = flat ? RingPlan{} : pick_ring<T>(m, n, k / BK, RingUse::kLayerNorm);
+    const RingPlan plan = flat ? RingPlan{} : pick_ring<T>(g, RingUse::kLayerNorm);
     const size_t bytes = (size_t)plan.slices * (size_t)m * (size_t)n * sizeof(float);
     // (where the caller has fixed the workspace and the copy does not fit it, the product is rounded and not refused)
     if (pays || tl_fixed_workspace.ptr == nullptr || bytes <= tl_fixed_workspace.bytes) {
@@ -228,7 +229,7 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, void* out, const vo
                                    const NormRows<T>*);                                                                       \
   template int gemm_norm_fused_typed<T>(const GemmArgs&, const void*, const void*, float, void*, int64_t, int,                \
                                         const ttmi_epilogue_args*, hipStream_t);                                              \
-  template int gemm_bias_layer_norm_typed<T>(const void*, const void*, void*, const void*, const float*, const void*,         \
+  template int gemm_bias_layer_norm_typed<T>(const void*, const void*, bool, void*, const void*, const float*, const void*,         \
                                              const void*, const void*, float*, int64_t, int64_t, int64_t, float, int,         \
                                              hipStream_t);
 

@@ -48,16 +48,16 @@ void BERTEmbedding::operator()(const Tensor& input_ids, const Tensor& position_i
 }
 
 // ------------------------------------------------------------------------------ FFN -----
-static void GemmBiasAct(const Tensor& in, const void* w_nk, int64_t n, const Tensor& bias, int act, Tensor* out) {
+static void GemmBiasAct(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& bias, int act, Tensor* out) {
   const int64_t k = in.shape(-1), m = in.numel() / k;
   ttmi_epilogue_args args{};
   args.bias = bias.raw();
   args.act = act;
-  TT_DEVICE_CALL(ttmi_gemm_fused(in.raw(), w_nk, out->mutable_raw(), m, n, k, k, k, n, TTMI_EPI_BIAS_ACT, &args,
-                                 kernels::DeviceDType(in), Stream()));
+  TT_DEVICE_CALL(ttmi_gemm_fused(in.raw(), w_nk.data, out->mutable_raw(), m, n, k, k, k, n, TTMI_EPI_BIAS_ACT, &args,
+                                 w_nk.DTypeFor(kernels::DeviceDType(in)), Stream()));
 }
 
-static void GemmThenAddBiasLayerNorm(const Tensor& in, const void* w_nk, int64_t n, const Tensor& bias, const Tensor& residual,
+static void GemmThenAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& bias, const Tensor& residual,
                                      const Tensor& gamma, const Tensor& beta, Tensor* out) {
   kernels::GemmAddBiasLayerNorm(in, w_nk, n, residual, bias, gamma, beta, out, 1e-12f);
 }
@@ -175,9 +175,9 @@ void PositionwiseFeedForward::operator()(const Tensor& input_tensor, Tensor* out
   ttmi_epilogue_args args{};
   args.bias = dense_bias_2_.raw();
   args.residual = input_tensor.raw();
-  TT_DEVICE_CALL(ttmi_gemm_fused(hidden_.raw(), packed2_.Get(dense_weight_2_, is_trans_weight), output->mutable_raw(), m, model_dim,
-                                 d_ff, d_ff, d_ff, model_dim, TTMI_EPI_BIAS_RESIDUAL, &args, kernels::DeviceDType(input_tensor),
-                                 Stream()));
+  const WeightRef w2 = packed2_.Get(dense_weight_2_, is_trans_weight);
+  TT_DEVICE_CALL(ttmi_gemm_fused(hidden_.raw(), w2.data, output->mutable_raw(), m, model_dim, d_ff, d_ff, d_ff, model_dim,
+                                 TTMI_EPI_BIAS_RESIDUAL, &args, w2.DTypeFor(kernels::DeviceDType(input_tensor)), Stream()));
 }
 
 void DistrillFFN::operator()(const Tensor& input_tensor, Tensor* output, bool is_trans_weight) const {
@@ -211,8 +211,9 @@ void LinearBias::operator()(const Tensor& input_tensor, Tensor* output_tensor) c
                            input_tensor.device_id(), "LinearBias/Reshape");
   ttmi_epilogue_args args{};
   args.bias = bias_.raw();
-  TT_DEVICE_CALL(ttmi_gemm_fused(input_tensor.raw(), packed_.Get(weight_, false), output_tensor->mutable_raw(), m, n, k, k, k,
-                                 n, TTMI_EPI_BIAS, &args, kernels::DeviceDType(input_tensor), Stream()));
+  const WeightRef w = packed_.Get(weight_, false);
+  TT_DEVICE_CALL(ttmi_gemm_fused(input_tensor.raw(), w.data, output_tensor->mutable_raw(), m, n, k, k, k, n, TTMI_EPI_BIAS, &args,
+                                 w.DTypeFor(kernels::DeviceDType(input_tensor)), Stream()));
 }
 
 // ----------------------------------------------------------------- stand-alone epilogues

@@ -181,16 +181,16 @@ void LayerNorm(const Tensor& gamma, const Tensor& beta, Tensor* out_tensor, T ep
 }
 template void LayerNorm<float>(const Tensor&, const Tensor&, Tensor*, float, const std::string);
 
-void LayerNormGemm(const Tensor& input, const Tensor& gamma, const Tensor& beta, float eps, Tensor* normed, const void* w_nk,
+void LayerNormGemm(const Tensor& input, const Tensor& gamma, const Tensor& beta, float eps, Tensor* normed, const WeightRef& w_nk,
                    Tensor* out, int64_t n, int epilogue, const ttmi_epilogue_args& args) {
   RequireGpu(input, "LayerNorm");
   const int64_t k = input.shape(-1), m = input.numel() / k;
   TT_ENFORCE_EQ(gamma.numel(), k, "LayerNorm gamma size mismatch");
   TT_ENFORCE_EQ(beta.numel(), k, "LayerNorm beta size mismatch");
   normed->ReshapeAs(input.dtype(), {m, k}, input.device_type(), input.device_id(), "LayerNorm/Reshape");
-  TT_DEVICE_CALL(ttmi_layer_norm_gemm_fused(input.raw(), gamma.raw(), beta.raw(), eps, normed->mutable_raw(), w_nk,
+  TT_DEVICE_CALL(ttmi_layer_norm_gemm_fused(input.raw(), gamma.raw(), beta.raw(), eps, normed->mutable_raw(), w_nk.data,
                                             out != nullptr ? out->mutable_raw() : nullptr, m, n, k, n, epilogue, &args,
-                                            DeviceDType(input), Stream()));
+                                            w_nk.DTypeFor(DeviceDType(input)), Stream()));
 }
 
 template <typename T>
@@ -261,7 +261,7 @@ void AddBiasLayerNormResidual(const Tensor& input_tensor, const Tensor& bias_ten
                                                      DeviceDType(*out_tensor), Stream()));
 }
 
-void GemmAddBiasLayerNorm(const Tensor& in, const void* w_nk, int64_t n, const Tensor& residual, const Tensor& bias_tensor,
+void GemmAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& residual, const Tensor& bias_tensor,
                           const Tensor& gamma_tensor, const Tensor& beta_tensor, Tensor* out_tensor, float eps) {
   RequireGpu(*out_tensor, "AddBiasLayerNorm");
   const int64_t k = in.shape(-1), m = in.numel() / k;
@@ -270,9 +270,9 @@ void GemmAddBiasLayerNorm(const Tensor& in, const void* w_nk, int64_t n, const T
   TT_ENFORCE_EQ(n, bias_tensor.shape(0), "AddBiasLayerNorm input_tensor.shape(-1) should be the same as bias_tensor.shape(0)");
   TT_ENFORCE_EQ(residual.numel(), m * n, "The shape of the input_tensor and out_tensor is not equal.");
   TT_ENFORCE_EQ(out_tensor->numel(), m * n, "The shape of the input_tensor and out_tensor is not equal.");
-  const int dt = DeviceDType(*out_tensor);
+  const int dt = w_nk.DTypeFor(DeviceDType(*out_tensor));
   if (!KeepsFp32Residual(*out_tensor)) {
-    TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk, out_tensor->mutable_raw(), residual.raw(), nullptr, bias_tensor.raw(),
+    TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk.data, out_tensor->mutable_raw(), residual.raw(), nullptr, bias_tensor.raw(),
                                              gamma_tensor.raw(), beta_tensor.raw(), nullptr, m, n, k, eps, dt, Stream()));
     return;
   }
@@ -286,7 +286,7 @@ void GemmAddBiasLayerNorm(const Tensor& in, const void* w_nk, int64_t n, const T
     residual32 = p;
   }
   Tensor* out32 = out_tensor->EnsureShadow();
-  TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk, out_tensor->mutable_raw(), nullptr, residual32, bias_tensor.raw(),
+  TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk.data, out_tensor->mutable_raw(), nullptr, residual32, bias_tensor.raw(),
                                            gamma_tensor.raw(), beta_tensor.raw(), out32->mutableData<float>(), m, n, k, eps, dt,
                                            Stream()));
 }

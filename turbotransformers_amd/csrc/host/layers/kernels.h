@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "core/tensor.h"
+#include "layers/packed_weight.h"
 #include "ttmi.h"
 
 namespace turbo_transformers {
@@ -58,7 +59,7 @@ void LayerNorm(const core::Tensor& gamma, const core::Tensor& beta, core::Tensor
                const std::string name = "LayerNorm");
 // ttmi_gemm_fused on LayerNorm(input), weights [n,k]; `normed` is scratch.  out may be null (QKV_SPLIT).
 void LayerNormGemm(const core::Tensor& input, const core::Tensor& gamma, const core::Tensor& beta, float eps, core::Tensor* normed,
-                   const void* w_nk, core::Tensor* out, int64_t n, int epilogue, const ttmi_epilogue_args& args);
+                   const WeightRef& w_nk, core::Tensor* out, int64_t n, int epilogue, const ttmi_epilogue_args& args);
 template <typename T>
 void AddBiasLayerNorm(const core::Tensor& input_tensor, const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor,
                       const core::Tensor& beta_tensor, core::Tensor* out_tensor, T eps = 1e-12,
@@ -94,7 +95,7 @@ void AddBiasLayerNormWithAbsmax(const core::Tensor& input_tensor, const core::Te
 bool KeepsFp32Residual(const core::Tensor& t);  // true for bfloat16 tensors
 // out = AddBiasLayerNorm(in . w^T, residual) with the same treatment of the residual; `w_nk` is the
 // [n, k] weight on the device, `out_tensor` already has its [.., n] shape.
-void GemmAddBiasLayerNorm(const core::Tensor& in, const void* w_nk, int64_t n, const core::Tensor& residual,
+void GemmAddBiasLayerNorm(const core::Tensor& in, const WeightRef& w_nk, int64_t n, const core::Tensor& residual,
                           const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor, const core::Tensor& beta_tensor,
                           core::Tensor* out_tensor, float eps = 1e-12f);
 

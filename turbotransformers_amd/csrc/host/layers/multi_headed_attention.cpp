@@ -134,7 +134,7 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   }  // unfused core
 
   output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
-  const void* wo = dense_packed_.Get(dense_weight_, is_trans_weight);
+  const WeightRef wo = dense_packed_.Get(dense_weight_, is_trans_weight);
   if (!post_add_input && post_layernorm) {
     // gemm5 then AddBiasLayerNorm(query, bias, gamma, beta, out), eps 1e-12 (:359-371)
     kernels::GemmAddBiasLayerNorm(ctx_, wo, hidden, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
@@ -142,14 +142,14 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
     ttmi_epilogue_args args{};
     args.bias = dense_bias_.raw();
     args.residual = post_add_input ? query_tensor.raw() : nullptr;
-    TT_DEVICE_CALL(ttmi_gemm_fused(ctx_.raw(), wo, output->mutable_raw(), tokens, hidden, hidden, hidden, hidden, hidden,
-                                   post_add_input ? TTMI_EPI_BIAS_RESIDUAL : TTMI_EPI_BIAS, &args, dt, Stream()));
+    TT_DEVICE_CALL(ttmi_gemm_fused(ctx_.raw(), wo.data, output->mutable_raw(), tokens, hidden, hidden, hidden, hidden, hidden,
+                                   post_add_input ? TTMI_EPI_BIAS_RESIDUAL : TTMI_EPI_BIAS, &args, wo.DTypeFor(dt), Stream()));
   }
 }
 
 // One projection followed by AddBiasTransposeForScore, as one GEMM: x[B,S,H] W + b -> [B,h,S,d]
 // (multi_headed_attention.cpp:73-88, :107-150).
-static void ProjectToHeads(const Tensor& x, const void* packed_w, const Tensor& bias, int64_t heads, Tensor* out,
+static void ProjectToHeads(const Tensor& x, const WeightRef& packed_w, const Tensor& bias, int64_t heads, Tensor* out,
                            const char* name) {
   const int64_t batch = x.shape(0), seq = x.shape(1), hidden = x.shape(2), d = hidden / heads;
   out->ReshapeAs(x.dtype(), {batch, heads, seq, d}, x.device_type(), x.device_id(), name);
@@ -159,8 +159,8 @@ static void ProjectToHeads(const Tensor& x, const void* packed_w, const Tensor& 
   args.seq = seq;
   args.heads = heads;
   args.head_dim = d;
-  TT_DEVICE_CALL(ttmi_gemm_fused(x.raw(), packed_w, nullptr, batch * seq, hidden, hidden, hidden, hidden, hidden,
-                                 TTMI_EPI_QKV_SPLIT, &args, kernels::DeviceDType(x), Stream()));
+  TT_DEVICE_CALL(ttmi_gemm_fused(x.raw(), packed_w.data, nullptr, batch * seq, hidden, hidden, hidden, hidden, hidden,
+                                 TTMI_EPI_QKV_SPLIT, &args, packed_w.DTypeFor(kernels::DeviceDType(x)), Stream()));
 }
 
 static bool CacheHas(const std::unordered_map<std::string, Tensor*>& cache, const char* key) {
@@ -210,13 +210,13 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
 
   if (pre_layernorm) TT_ENFORCE(!layernorm_gamma_.is_null() && !layernorm_beta_.is_null(), "pre_layernorm needs LayerNorm parameters");
   // a projection of the query, with LayerNorm in front where asked for (:66-80, :190-199 -- eps is 1e-6 there)
-  auto project_query = [&](const void* packed_w, int64_t n, const ttmi_epilogue_args& args) {
+  auto project_query = [&](const WeightRef& packed_w, int64_t n, const ttmi_epilogue_args& args) {
     if (pre_layernorm) {
       kernels::LayerNormGemm(query_tensor, layernorm_gamma_, layernorm_beta_, 1e-6f, &ln_query_, packed_w, nullptr, n,
                              TTMI_EPI_QKV_SPLIT, args);
     } else {
-      TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), packed_w, nullptr, batch * seq, n, hidden, hidden, hidden, n,
-                                     TTMI_EPI_QKV_SPLIT, &args, dt, Stream()));
+      TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), packed_w.data, nullptr, batch * seq, n, hidden, hidden, hidden, n,
+                                     TTMI_EPI_QKV_SPLIT, &args, packed_w.DTypeFor(dt), Stream()));
     }
   };
 
@@ -343,8 +343,9 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
         kv.seq = len;
         kv.heads = heads;
         kv.head_dim = d;
-        TT_DEVICE_CALL(ttmi_gemm_fused(key_tensor.raw(), kv_packed_.GetPair(k_weight_, v_weight_), nullptr, batch * len, 2 * hidden,
-                                       hidden, hidden, hidden, 2 * hidden, TTMI_EPI_QKV_SPLIT, &kv, dt, Stream()));
+        const WeightRef both = kv_packed_.GetPair(k_weight_, v_weight_);
+        TT_DEVICE_CALL(ttmi_gemm_fused(key_tensor.raw(), both.data, nullptr, batch * len, 2 * hidden, hidden, hidden, hidden,
+                                       2 * hidden, TTMI_EPI_QKV_SPLIT, &kv, both.DTypeFor(dt), Stream()));
       } else {
         ProjectToHeads(key_tensor, k_packed_.Get(k_weight_, is_trans_weight), k_bias_, heads, k_out, "context/keys/AddBiasTransposeForScore/Reshape");
         ProjectToHeads(value_tensor, v_packed_.Get(v_weight_, is_trans_weight), v_bias_, heads, v_out, "context/values/AddBiasTransposeForScore/Reshape");
@@ -431,8 +432,9 @@ void MultiHeadedAttentionSmartBatch::operator()(const Tensor& key_tensor, const 
   args.head_dim = d;
   args.token_rows = plan.token_rows;
   args.batch = batch;
-  TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), qkv_packed_.Get(qkv_weight_, is_trans_weight), nullptr, plan.total,
-                                 3 * hidden, hidden, hidden, hidden, 3 * hidden, TTMI_EPI_QKV_SPLIT_PAD, &args, dt, Stream()));
+  const WeightRef wqkv = qkv_packed_.Get(qkv_weight_, is_trans_weight);
+  TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), wqkv.data, nullptr, plan.total, 3 * hidden, hidden, hidden, hidden, 3 * hidden,
+                                 TTMI_EPI_QKV_SPLIT_PAD, &args, wqkv.DTypeFor(dt), Stream()));
 
   AttentionTail(query_tensor, attention_mask, output, att_score, batch, max_seq, max_seq, k_, v_, &query_seq_len_list, fused_core, 0,
                 post_layernorm, post_add_input, is_trans_weight);

@@ -7,39 +7,46 @@
 namespace turbo_transformers {
 namespace layers {
 
-const void* PackedWeight::Get(const core::Tensor& w, bool is_trans_weight) const {
-  TT_ENFORCE_EQ(w.n_dim(), (size_t)2, "weights must be 2-D");
-  kernels::RequireGpu(w, "weight");
-  if (is_trans_weight) return w.raw();
-  std::lock_guard<std::mutex> lock(mutex_);
-  if (source_ != w.raw() || packed_.is_null()) {
-    const int64_t K = w.shape(0), N = w.shape(1);
-    packed_.ReshapeAs(w.dtype(), {N, K}, w.device_type(), w.device_id(), "PackedWeight");
-    TT_DEVICE_CALL(ttmi_transpose_2d(w.raw(), packed_.mutable_raw(), K, N, core::ToDeviceDType(w.dtype()),
-                                     core::DeviceContext::GetInstance().stream()));
-    source_ = w.raw();
+WeightRef PackedWeight::Pack(std::initializer_list<const core::Tensor*> parts) const {
+  const core::Tensor& w = **parts.begin();
+  const int64_t K = w.shape(0), N = w.shape(1), rows = N * (int64_t)parts.size();
+  const int dtype = core::ToDeviceDType(w.dtype());
+  void* stream = core::DeviceContext::GetInstance().stream();
+  const bool split = dtype == TTMI_F32 && K > 0 && K % TTMI_PACKED_WEIGHT_K == 0;
+  if (split) packed_.ReshapeAs(w.dtype(), {TTMI_PACKED_WEIGHT_FLOATS(rows, K)}, w.device_type(), w.device_id(), "PackedWeight");
+  else packed_.ReshapeAs(w.dtype(), {rows, K}, w.device_type(), w.device_id(), "PackedWeight");
+  char* at = static_cast<char*>(packed_.mutable_raw());
+  for (const core::Tensor* part : parts) {
+    TT_DEVICE_CALL(ttmi_transpose_2d(part->raw(), at, K, N, dtype, stream));
+    at += (size_t)(K * N) * w.element_size();
   }
-  return packed_.raw();
+  if (split) TT_DEVICE_CALL(ttmi_split_weights(packed_.mutable_raw(), rows, K, stream));
+  dtype_ = split ? TTMI_F32_PACKED : dtype;
+  return {packed_.raw(), dtype_};
 }
 
-const void* PackedWeight::GetPair(const core::Tensor& w, const core::Tensor& v) const {
+WeightRef PackedWeight::Get(const core::Tensor& w, bool is_trans_weight) const {
+  TT_ENFORCE_EQ(w.n_dim(), (size_t)2, "weights must be 2-D");
+  kernels::RequireGpu(w, "weight");
+  if (is_trans_weight) return {w.raw(), core::ToDeviceDType(w.dtype())};
+  std::lock_guard<std::mutex> lock(mutex_);
+  if (source_ == w.raw() && !packed_.is_null()) return {packed_.raw(), dtype_};
+  const WeightRef ref = Pack({&w});
+  source_ = w.raw();
+  return ref;
+}
+
+WeightRef PackedWeight::GetPair(const core::Tensor& w, const core::Tensor& v) const {
   TT_ENFORCE(w.n_dim() == 2 && v.n_dim() == 2 && w.shape(0) == v.shape(0) && w.shape(1) == v.shape(1), "a pair of weights has one shape");
   TT_ENFORCE(core::SameDataType(w.dtype(), v.dtype()), "a pair of weights has one element type");
   kernels::RequireGpu(w, "weight");
   kernels::RequireGpu(v, "weight");
   std::lock_guard<std::mutex> lock(mutex_);
-  if (source_ != w.raw() || second_source_ != v.raw() || packed_.is_null()) {
-    const int64_t K = w.shape(0), N = w.shape(1);
-    packed_.ReshapeAs(w.dtype(), {2 * N, K}, w.device_type(), w.device_id(), "PackedWeight");
-    char* half = static_cast<char*>(packed_.mutable_raw());
-    for (const core::Tensor* t : {&w, &v}) {
-      TT_DEVICE_CALL(ttmi_transpose_2d(t->raw(), half, K, N, core::ToDeviceDType(w.dtype()), core::DeviceContext::GetInstance().stream()));
-      half += (size_t)(K * N) * w.element_size();
-    }
-    source_ = w.raw();
-    second_source_ = v.raw();
-  }
-  return packed_.raw();
+  if (source_ == w.raw() && second_source_ == v.raw() && !packed_.is_null()) return {packed_.raw(), dtype_};
+  const WeightRef ref = Pack({&w, &v});
+  source_ = w.raw();
+  second_source_ = v.raw();
+  return ref;
 }
 
 }  // namespace layers
