@@ -173,7 +173,7 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
       load_row8<float>(epi.w_scale + n, scale);
     }
     if constexpr (AddsResidual<Epi>::value) load_row8(epi.residual + (int64_t)m * epi.ldc + n, res);
-    if constexpr (RingDest<Epi>::split) dest = RingDest<Epi>::column(epi, z_epi, n) + RingDest<Epi>::row(epi, m);
+    dest = RingDest<Epi>::column(epi, z_epi, n) + RingDest<Epi>::row(epi, m);
   }
   if (column_piece && bias != nullptr) column_bias = to_float(bias[n0 + (tid & 15)]);
 
@@ -282,13 +282,13 @@ __global__ __launch_bounds__(kFlatWaves * kWave) void gemm_flat_kernel(const Gem
         v[e] += (AccScalar)wide[e];
       }
     }
-    if constexpr (RingDest<Epi>::split) {
+    if constexpr (std::is_same<Epi, EpiInt32>::value) {
+      epi.store8(z_epi, m, n, v, 8);
+    } else {
       float fin[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) fin[e] = RingDest<Epi>::finish(epi, v[e]) + res[e];
       store_row8(dest, fin);
-    } else {
-      epi.store8(z_epi, m, n, v, 8);
     }
   }
   if constexpr (HasColumnPass<Epi>::value) {

@@ -57,13 +57,9 @@ struct RingMma<float> {
   }
 };
 
-// Where an epilogue's output goes, as column part + row part (`split`), and what finishes a value; the epilogues this does
-// not cover store through their store8().
+// Where an epilogue's output goes, as column part + row part, and what finishes a value.
 template <typename Epi>
-struct RingDest {
-  using Elem = float;
-  static constexpr bool split = false;
-};
+struct RingDest;
 template <typename Epi>
 struct AddsResidual : std::false_type {};
 template <typename T, int ACT, bool HAS_ACT>
@@ -72,7 +68,6 @@ template <typename T, int ACT, bool HAS_ACT, bool HAS_RES>
 struct RingDest<EpiBias<T, ACT, HAS_ACT, HAS_RES>> {
   using Epi = EpiBias<T, ACT, HAS_ACT, HAS_RES>;
   using Elem = T;
-  static constexpr bool split = true;
   static __device__ __forceinline__ T* column(const Epi& e, int, int n) { return e.c + n; }
   static __device__ __forceinline__ int64_t row(const Epi& e, int m) { return (int64_t)m * e.ldc; }
   static __device__ __forceinline__ float finish(const Epi& e, float x) { return e.finish(x); }
@@ -80,7 +75,6 @@ struct RingDest<EpiBias<T, ACT, HAS_ACT, HAS_RES>> {
 template <typename T>
 struct RingDest<EpiF32<T>> {
   using Elem = float;
-  static constexpr bool split = true;
   static __device__ __forceinline__ float* column(const EpiF32<T>& e, int, int n) { return e.c + n; }
   static __device__ __forceinline__ int64_t row(const EpiF32<T>& e, int m) { return (int64_t)m * e.ldc; }
   static __device__ __forceinline__ float finish(const EpiF32<T>&, float x) { return x; }
@@ -88,7 +82,6 @@ struct RingDest<EpiF32<T>> {
 template <>
 struct RingDest<EpiPartial> {
   using Elem = float;
-  static constexpr bool split = true;
   static __device__ __forceinline__ float* column(const EpiPartial& e, int z, int n) { return e.ws + (int64_t)z * e.mn + n; }
   static __device__ __forceinline__ int64_t row(const EpiPartial& e, int m) { return (int64_t)m * e.ldn; }
   static __device__ __forceinline__ float finish(const EpiPartial&, float x) { return x; }
@@ -96,16 +89,20 @@ struct RingDest<EpiPartial> {
 template <typename T, bool PAD>
 struct RingDest<EpiQkvSplit<T, PAD>> {
   using Elem = T;
-  static constexpr bool split = true;
   static __device__ __forceinline__ T* column(const EpiQkvSplit<T, PAD>& e, int, int n) { return e.col_part((uint32_t)n); }
   static __device__ __forceinline__ int64_t row(const EpiQkvSplit<T, PAD>& e, int m) { return e.row_part(m); }
   static __device__ __forceinline__ float finish(const EpiQkvSplit<T, PAD>&, float x) { return x; }
 };
 
 template <>
+struct RingDest<EpiInt32> {
+  using Elem = int32_t;
+  static __device__ __forceinline__ int32_t* column(const EpiInt32& e, int, int n) { return e.c + n; }
+  static __device__ __forceinline__ int64_t row(const EpiInt32& e, int m) { return (int64_t)m * e.ldc; }
+};
+template <>
 struct RingDest<EpiDequant> {
   using Elem = float;
-  static constexpr bool split = true;
   static __device__ __forceinline__ float* column(const EpiDequant& e, int, int n) { return e.c + n; }
   static __device__ __forceinline__ int64_t row(const EpiDequant& e, int m) { return (int64_t)m * e.ldc; }
   static __device__ __forceinline__ float finish(const EpiDequant&, int x) { return __builtin_bit_cast(float, x); }
@@ -113,7 +110,6 @@ struct RingDest<EpiDequant> {
 template <>
 struct RingDest<EpiDequantQkvSplit> {
   using Elem = float;
-  static constexpr bool split = true;
   static __device__ __forceinline__ float* column(const EpiDequantQkvSplit& e, int, int n) { return e.split.col_part((uint32_t)n); }
   static __device__ __forceinline__ int64_t row(const EpiDequantQkvSplit& e, int m) { return e.split.row_part(m); }
   static __device__ __forceinline__ float finish(const EpiDequantQkvSplit&, int x) { return __builtin_bit_cast(float, x); }
@@ -126,6 +122,71 @@ __device__ __forceinline__ void static_for_impl(const F& f, std::integer_sequenc
 template <int N, typename F>
 __device__ __forceinline__ void static_for(const F& f) {  // f(0), ..., f(N - 1) with compile-time arguments
   static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Rows of 32-bit results (operands swapped: of block (i, j) a lane owns four columns of a row): 16 bytes a store straight from the
+// accumulators, the four lanes of a row side by side.  (Eight columns a lane, as 16-bit results are stored, are two stores that
+// each touch every other 16 bytes of a row: BERT base, us a pass, so / here: int8 20 x 128 tokens 1341 / 1314, fp32 20 x 100 1756 / 1722.)
+// What a lane needs of its columns, requested before the K loop.
+template <typename BT, int CB, bool SCALE>
+struct ColumnQuads {
+  Vec<BT, 4> bias[CB];
+  float4 scale[SCALE ? CB : 1];
+  bool present;
+  // `fallback`: as in BiasVec
+  __device__ __forceinline__ void load(const BT* b, const float* w_scale, int n_first, int n, int lgrp, const void* fallback) {
+    present = b != nullptr;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const int col = min(n_first + j * 16 + lgrp * 4, n - 4);
+      bias[j] = load_vec<BT, 4>(present ? b + col : static_cast<const BT*>(fallback));
+      if constexpr (SCALE) scale[j] = *reinterpret_cast<const float4*>(w_scale + col);
+    }
+  }
+};
+// read(i, j, e): element e of the lane's part of block (i, j).
+template <int RB, int CB, typename Epi, typename Quads, typename Read>
+__device__ __forceinline__ void store_rows32(const GemmArgs& g, const Epi& epi, const Quads& quads, int z_epi, int m_first, int n_first, int lrow, int lgrp,
+                                             float& amax, const Read& read) {
+  using Dest = RingDest<Epi>;
+  using Elem = typename Dest::Elem;
+  float act_scale = 0.f;
+  if constexpr (Dequantises<Epi>::value) act_scale = epi.act_scale[0];
+  int64_t row_at[RB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i) row_at[i] = Dest::row(epi, min(m_first + i * 16 + lrow, g.m - 1));
+#pragma unroll
+  for (int j = 0; j < CB; ++j) {
+    const int n = n_first + j * 16 + lgrp * 4;  // (N is a multiple of eight: the four columns are all inside, or none)
+    Elem* const col = Dest::column(epi, z_epi, min(n, g.n - 4));
+    float wide[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) wide[e] = quads.present ? to_float(quads.bias[j].v[e]) : 0.f;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      Vec<Elem, 4> out;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (Dequantises<Epi>::value) {
+          const float scale[4] = {quads.scale[j].x, quads.scale[j].y, quads.scale[j].z, quads.scale[j].w};
+          out.v[e] = epi.activate(dequantise(read(i, j, e), act_scale, scale[e], wide[e], quads.present));
+          amax = fmaxf(amax, fabsf(out.v[e]));
+        } else if constexpr (std::is_same<Elem, int32_t>::value) {
+          out.v[e] = read(i, j, e);
+        } else {
+          out.v[e] = Dest::finish(epi, read(i, j, e) + wide[e]);
+        }
+      }
+      if (m_first + i * 16 + lrow < g.m && n < g.n) {
+        if constexpr (AddsResidual<Epi>::value) {
+          const Vec<Elem, 4> res = load_vec<Elem, 4>(epi.residual + (col - epi.c) + row_at[i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) out.v[e] += res.v[e];
+        }
+        store_vec<Elem, 4>(col + row_at[i], out);
+      }
+    }
+  }
 }
 
 template <int BM, int BN, int NS>
@@ -149,7 +210,6 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
   static_assert(NS >= 2 && YOUNGER < 64, "vmcnt is a six-bit counter");
   using MB = RingMma<T>;
   using Acc = typename MB::Acc;
-  using AccScalar = typename Epi::Acc;
 
   extern __shared__ __align__(16) char smem[];
 
@@ -319,64 +379,51 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
   float amax = 0.f;
   bool swap = true;
   if constexpr (HasColumnPass<Epi>::value) swap = !(epi.column_pass() && n0 + wn0 >= epi.first_column_of_pass());
+  using Dest = RingDest<Epi>;
   if (swap) {
-    if constexpr (!Dequantises<Epi>::value) {
+    if constexpr (sizeof(typename Dest::Elem) == 4) {
+      ColumnQuads<BiasT, CB, Dequantises<Epi>::value> quads;
+      const float* w_scale = nullptr;
+      if constexpr (Dequantises<Epi>::value) w_scale = epi.w_scale;
+      quads.load(bias, w_scale, n0 + wn0, g.n, lgrp, g.b);
+      k_loop(std::true_type{});
+      store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax,
+                           [&](int i, int j, int e) __attribute__((always_inline)) { return acc_read(acc[i][j][e]); });
+    } else {
 #pragma unroll
       for (int p = 0; p < CB / 2; ++p) bv[p].load(bias, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8), g.b);
-    }
-    k_loop(std::true_type{});
-    // Destination of a unit = a part that depends on its columns + a part that depends on its row, each found once.
-    typename RingDest<Epi>::Elem* col_at[CB / 2];
-    int64_t row_at[RB];
-    if constexpr (RingDest<Epi>::split) {
+      k_loop(std::true_type{});
+      // Destination of a unit = a part that depends on its columns + a part that depends on its row, each found once.
+      typename Dest::Elem* col_at[CB / 2];
+      int64_t row_at[RB];
 #pragma unroll
-      for (int p = 0; p < CB / 2; ++p) col_at[p] = RingDest<Epi>::column(epi, z_epi, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8));
+      for (int p = 0; p < CB / 2; ++p) col_at[p] = Dest::column(epi, z_epi, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8));
 #pragma unroll
-      for (int i = 0; i < RB; ++i) row_at[i] = RingDest<Epi>::row(epi, min(m0 + wm0 + i * 16 + lrow, g.m - 1));
-    }
+      for (int i = 0; i < RB; ++i) row_at[i] = Dest::row(epi, min(m0 + wm0 + i * 16 + lrow, g.m - 1));
 #pragma unroll
-    for (int p = 0; p < CB / 2; ++p) {
-      const int n = n0 + wn0 + unit_chunk(p) * 8;
-      float wide[8], scale[8];
-      float act_scale = 0.f;
-      if constexpr (Dequantises<Epi>::value) {
-        const int nc = min(n, g.n - 8);
-        act_scale = epi.act_scale[0];
-        load_row8<float>(epi.w_scale + nc, scale);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) wide[e] = 0.f;
-        if (epi.has_bias()) load_row8<float>(bias + nc, wide);
-      } else {
+      for (int p = 0; p < CB / 2; ++p) {
+        const int n = n0 + wn0 + unit_chunk(p) * 8;
+        float wide[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) wide[e] = 0.f;
         if (bias != nullptr) bv[p].widen(wide);
-      }
 #pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        AccScalar out[8];
+        for (int i = 0; i < RB; ++i) {
+          float out[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          auto a = acc_read(acc[i][2 * p][e]), b = acc_read(acc[i][2 * p + 1][e]);
-          pair_swap<16>(a, b);
-          out[e] = a;
-          out[4 + e] = b;
-        }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          if constexpr (Dequantises<Epi>::value) {
-            const float r = epi.activate(dequantise(out[e], act_scale, scale[e], wide[e], epi.has_bias()));
-            amax = fmaxf(amax, fabsf(r));
-            out[e] = __builtin_bit_cast(AccScalar, r);
-          } else {
-            out[e] += (AccScalar)wide[e];
+          for (int e = 0; e < 4; ++e) {
+            auto a = acc_read(acc[i][2 * p][e]), b = acc_read(acc[i][2 * p + 1][e]);
+            pair_swap<16>(a, b);
+            out[e] = a;
+            out[4 + e] = b;
           }
-        }
-        const int m = m0 + wm0 + i * 16 + lrow;
-        if (m < g.m && n < g.n) {
-          if constexpr (RingDest<Epi>::split) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) out[e] += wide[e];
+          const int m = m0 + wm0 + i * 16 + lrow;
+          if (m < g.m && n < g.n) {
             float fin[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) fin[e] = RingDest<Epi>::finish(epi, out[e]);
+            for (int e = 0; e < 8; ++e) fin[e] = Dest::finish(epi, out[e]);
             if constexpr (AddsResidual<Epi>::value) {
               float res[8];
               load_row8(epi.residual + (col_at[p] - epi.c) + row_at[i], res);
@@ -384,8 +431,6 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
               for (int e = 0; e < 8; ++e) fin[e] += res[e];
             }
             store_row8(col_at[p] + row_at[i], fin);
-          } else {
-            epi.store8(z_epi, m, n, out, 8);
           }
         }
       }

@@ -214,9 +214,6 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
     for (int i = 0; i < B_LOADS; ++i) request_b(i, step, B_BASE + step * B_STAGE);
   });
 
-  const float* bias = epi.bias_ptr();
-  BiasVec<float> bv[CB / 2];
-
   auto clear = [&] {
 #pragma unroll
     for (int i = 0; i < RB; ++i)
@@ -315,50 +312,14 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
     return __builtin_fmaf(acc_read(cross[i][j][e]), 1.f / kSplitScale, acc_read(acc[i][j][e]));
   };
   auto unit_chunk = [&](int p) __attribute__((always_inline)) { return 2 * (2 * p + (lgrp & 1)) + (lgrp >> 1); };
-  using Dest = RingDest<Epi>;
   bool swap = true;
   if constexpr (HasColumnPass<Epi>::value) swap = !(epi.column_pass() && n0 + wn0 >= epi.first_column_of_pass());
   if (swap) {
-#pragma unroll
-    for (int p = 0; p < CB / 2; ++p) bv[p].load(bias, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8), g.b);
+    float amax = 0.f;
+    ColumnQuads<float, CB, false> quads;
+    quads.load(epi.bias_ptr(), nullptr, n0 + wn0, g.n, lgrp, g.b);
     k_loop(std::true_type{});
-    // (destinations as in gemm_ring_kernel)
-    float* col_at[CB / 2];
-    int64_t row_at[RB];
-#pragma unroll
-    for (int p = 0; p < CB / 2; ++p) col_at[p] = Dest::column(epi, z_epi, min(n0 + wn0 + unit_chunk(p) * 8, g.n - 8));
-#pragma unroll
-    for (int i = 0; i < RB; ++i) row_at[i] = Dest::row(epi, min(m0 + wm0 + i * 16 + lrow, g.m - 1));
-#pragma unroll
-    for (int p = 0; p < CB / 2; ++p) {
-      const int n = n0 + wn0 + unit_chunk(p) * 8;
-      float wide[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) wide[e] = 0.f;
-      if (bias != nullptr) bv[p].widen(wide);
-#pragma unroll
-      for (int i = 0; i < RB; ++i) {
-        float out[8];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float a = read(i, 2 * p, e), b = read(i, 2 * p + 1, e);
-          pair_swap<16>(a, b);
-          out[e] = a;
-          out[4 + e] = b;
-        }
-        if (m0 + wm0 + i * 16 + lrow < g.m && n < g.n) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) out[e] = Dest::finish(epi, out[e] + wide[e]);
-          if constexpr (AddsResidual<Epi>::value) {
-            float res[8];
-            load_row8(epi.residual + (col_at[p] - epi.c) + row_at[i], res);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) out[e] += res[e];
-          }
-          store_row8(col_at[p] + row_at[i], out);
-        }
-      }
-    }
+    store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax, read);
   } else {
     if constexpr (HasColumnPass<Epi>::value) {
       float bj[CB];
