@@ -1201,6 +1201,94 @@ def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps)
     assert torch.all(q[M:] == -7.0)
 
 
+def _attention64(Q, K, V, mask, scale=0.125):
+    s = Q.double() @ K.double().transpose(2, 3) * scale
+    return torch.softmax(s if mask is None else s + mask.double()[:, None, None, :], -1) @ V.double()
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("lens", [[1], [63, 64, 65, 3], [129, 100], [40, 300, 7], [545]])
+@pytest.mark.parametrize("form", ["dense", "packed", "packed, V transposed"])
+def test_fused_attention_fp32_in_halves(ttmi, waves, lens, form):
+    """fp32 attention on the 16-bit matrix instructions, against 64 bits: lengths around the tiles of 64 keys, masks, both layouts of V
+    (NaN behind the last key).  No further off than the fp32 instruction, which a dense batch with row-major V runs on."""
+    B, h, S, d = len(lens), 2, max(lens), 64
+    g = torch.Generator(device="cuda").manual_seed(S + waves)
+    Q, K, V = (torch.randn(B, h, S, d, generator=g, device="cuda") for _ in range(3))
+    pitch, packed = (S + 7) // 8 * 8, form != "dense"
+    Vt = torch.full((B, h, d, pitch), float("nan"), device="cuda")
+    Vt[..., :S] = V.transpose(2, 3)
+    if packed:
+        for b, n in enumerate(lens):
+            K[b, :, n:], V[b, :, n:], Vt[b, :, :, n:] = float("nan"), float("nan"), float("nan")
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    mask = torch.where(torch.rand(B, S, generator=g, device="cuda") < 0.2, -1e4, 0.0)
+
+    def run(v, v_pitch, cu):
+        out = torch.full((sum(lens) if cu is not None else B * S, h * d), 9.0, device="cuda")
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", waves))
+        ok(ttmi.ttmi_fused_attention(ptr(Q), ptr(K), ptr(v), ptr(mask), ptr(out), ptr(cu), B, h, S, d, v_pitch, 0.125, capi.F32, stream()))
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+        if cu is None:
+            return list(out.view(B, S, h, d).permute(0, 2, 1, 3).double())
+        return [out[cu[b]:cu[b + 1]].view(-1, h, d).permute(1, 0, 2).double() for b in range(B)]
+
+    lengths = lens if packed else [S] * B
+    want = [_attention64(Q[b:b + 1, :, :n], K[b:b + 1, :, :n], V[b:b + 1, :, :n], mask[b:b + 1, :n])[0] for b, n in enumerate(lengths)]
+    got = run(V if form == "packed" else Vt, 0 if form == "packed" else pitch, cu if packed else None)
+    # scores up to 8 of 64 products each (3 * 2^-22 of sum |q k| / 8 <= 20), as a relative error of a probability, and as much again
+    # for sums and exp2: 2^-16 of the largest value
+    for a, w in zip(got, want):
+        assert float((a - w).abs().max()) <= 2.0**-16 * float(w.abs().max())
+    if not packed and S > 32:
+        fp32 = run(V, 0, None)
+        error = lambda x: sum(float(((a - w)**2).sum()) for a, w in zip(x, want))**0.5
+        assert error(got) <= error(fp32), (error(got), error(fp32))
+
+
+@pytest.mark.parametrize("what", ["large Q", "large K", "infinite K", "large V", "infinite V", "tiny column of V", "zero column of V", "NaN"])
+@pytest.mark.parametrize("v_transposed,packed", [(True, False), (False, True), (True, True)])
+def test_fused_attention_fp32_outside_the_window(ttmi, what, v_transposed, packed):
+    """Values that fp16 halves do not hold: the workgroups that meet one compute on the fp32 instruction, the others as before."""
+    B, h, S, d = 2, 2, 150, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    Q, K, V = (torch.randn(B, h, S, d, generator=g, device="cuda") for _ in range(3))
+    if what == "large Q":
+        Q[0, 0, 140] *= 1e5
+    elif what == "large K":
+        K[0, 1, 70] *= 3e3
+    elif what == "infinite K":
+        K[0, 1, 70, 5] = float("inf")
+    elif what == "large V":
+        V[1, 0] *= 1e6
+    elif what == "infinite V":
+        V[1, 0, 149, 7] = float("-inf")
+    elif what == "tiny column of V":
+        V[1, 1, :, 9] *= 1e-9
+    elif what == "zero column of V":
+        V[1, 1, :, 9] = 0
+    else:
+        V[0, 0, 3, 3] = float("nan")
+    pitch = (S + 7) // 8 * 8
+    v = V
+    if v_transposed:
+        v = torch.full((B, h, d, pitch), float("nan"), device="cuda")
+        v[..., :S] = V.transpose(2, 3)
+    cu = torch.tensor([0, S, 2 * S], dtype=torch.int32, device="cuda") if packed else None
+    out = torch.full((B * S, h * d), 9.0, device="cuda")
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", 4))
+    ok(ttmi.ttmi_fused_attention(ptr(Q), ptr(K), ptr(v), None, ptr(out), ptr(cu), B, h, S, d, pitch if v_transposed else 0, 0.125, capi.F32, stream()))
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+    got, want = out.view(B, S, h, d).permute(0, 2, 1, 3).double(), _attention64(Q, K, V, None)
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(got), finite) and torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
+    # relative to the column that a value averages; scores of up to 1e5 are themselves rounded by 2^-8
+    column = torch.where(torch.isfinite(V), V.abs(), 0).amax(2, keepdim=True).double()
+    bound = 2.0**-6 if what in ("large Q", "large K") else 2.0**-15
+    assert bool(((got - want).abs() <= bound * column + 1e-30)[finite].all())
+
+
 def _packed(ttmi, W):
     """fp32 weights [N, K] as ttmi_split_weights lays them out."""
     N, K = W.shape

@@ -350,6 +350,11 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }();
   const bool fits_four = seq <= 128 || 8 * ceil_div(seq, 256) >= 5 * ceil_div(seq, 128);
   int nw = (fits_four || ceil_div(seq, 128) * batch * heads < (int64_t)cus) ? 4 : 8;
+  // fp32 in halves: splitting K and V on their way into LDS is half of a short sequence's work, and eight wavefronts share it even
+  // where four have no queries, as long as every workgroup has a CU of its own (us, four / eight: 20 x 100 tokens 12.0 / 10.0,
+  // 8 x 40 8.0 / 6.6, 8 packed of up to 84 9.8 / 8.5; 32 x 100, 384 workgroups, 16.3 / 18.6).
+  const bool halves = dtype == TTMI_F32 && (v_seq_pitch > 0 || cu_seqlens != nullptr);
+  if (halves && seq <= 128 && batch * heads <= (int64_t)cus) nw = 8;
   // TTMI_ATTENTION_WAVES=4 / 8 (1: keys split over the wavefronts) overrides the choice (A/B timing, and tests of one form
   // on the shapes of another)
   const int force = kernel_switch(kSwitchAttentionWaves);
@@ -357,12 +362,12 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   // Few sequences: a workgroup per 32 queries, its wavefronts sharing the keys (attention_split.hip).  It re-reads K and V
   // per 32 queries, so it wins while its workgroups fit the CUs at once: 16-bit, us split / four wavefronts, 12 heads:
   // 1 x 128: 4.3 / 4.7, 1 x 387: 7.0 / 10.6, 4 x 128 (192 workgroups): 4.5 / 4.8, 8 x 128 (384): 6.5 / 5.0; one tile of
-  // keys is a draw.  fp32 is bound by the matrix pipes and gains further on: 1 x 128: 6.3 / 12.7, 2 x 512 (384): 32 / 42,
-  // 8 x 128 (384): 12.3 / 13.4, 16 x 128 (768): 18.8 / 13.9; and always below 33 keys, where a tile of 64 is half padding.
+  // keys is a draw.  fp32, split / the better of four and eight: 1 x 128 6.5 / 8.7, 4 x 128 (192) 6.8 / 9.0, 2 x 256 (192) 10.9 / 15.6,
+  // 3 x 256 (288) 20.2 / 15.6, 8 x 128 (384) 12.2 / 9.2; and always below 33 keys, where a tile of 64 is half padding.
   // (Dense batches with V transposed.  The quantised layers, whose rounding to 8 bits turns sums in another order into
   // whole steps, keep V row-major and with it the order of the other kernel.)
   const int64_t split_wgs = ceil_div(seq, 32) * batch * heads;
-  const bool split_wins = dtype == TTMI_F32 ? 2 * split_wgs <= 3 * (int64_t)cus || seq <= 32 : seq > 64 && split_wgs <= (int64_t)cus;
+  const bool split_wins = dtype == TTMI_F32 ? split_wgs <= (int64_t)cus || seq <= 32 : seq > 64 && split_wgs <= (int64_t)cus;
   const bool split = force == 1 || (force != 4 && force != 8 && split_wins);
   if (split && cu_seqlens == nullptr && v_seq_pitch > 0) {
     const bool leave_maxima = absmax != nullptr && dtype == TTMI_F32 && split_wgs <= TTMI_ABSMAX_SLOTS;

@@ -3,18 +3,22 @@
 // batch_gemm4 -> TransposeForScore chain of layers/multi_headed_attention.cpp:323-354 when the caller does not ask for
 // the probabilities: the [B,h,S,S] scores, written and read twice by that chain, never reach HBM.
 //
-// Same formulation as the 16-bit kernel, on v_mfma_f32_32x32x2_f32: scores are computed TRANSPOSED,
+// Same formulation as the 16-bit kernel.  Scores are computed TRANSPOSED,
 //     St[key, query] = K_tile[key, :] . Q[query, :]      (A = K from LDS, B = Q from registers)
 // so a lane holds one query column and 16 key rows of a 32-key sub-tile; the online-softmax statistics are lane-local
-// plus one exchange between the half-wavefronts.  A 32x32x2 instruction takes K index 0 from lanes 0-31 and K index 1
-// from lanes 32-63, and which two indices of the long dimension a given instruction pairs is free as long as both
-// operands agree.  Accumulator register 4g+i of a lane in half h is key 8g + 4h + i: pairing keys (8g+i, 8g+4+i)
-// in instruction (g, i) makes the probabilities, still in the accumulator registers, the B operand of
+// plus one exchange between the half-wavefronts, and the probabilities, still in the accumulator registers, are the B operand of
 //     Ot[d, query] += Vt[d, keys] . Pt[keys, query]      (A = V^T from LDS, B = P from registers)
-// with A read as the 16-byte chunk (2g+h) of a V^T row: four keys, one per instruction.  The first product pairs the
-// head dimension the same way (chunk 2kk+h of a K row and of a Q row).  Everything stays fp32; exp is exp2 with
-// scale*log2(e) folded into the argument, the additive mask (divided by the scale) seeds the score accumulators, the
-// running maximum is exact.  The matrix pipe bounds the kernel (4*S*64 FLOP per query and head at 157 TFLOP/s).
+// with the keys that a lane holds given to it in V^T as well.  exp is exp2 with scale*log2(e) folded into the argument, the
+// additive mask (divided by the scale) seeds the score accumulators.
+// Both products run on v_mfma_f32_32x32x16_f16, three instructions for one, with Q, K, V and the probabilities split in fp16 halves
+// (split_f32.h): K and V once per workgroup on their way into LDS, the others in registers.  A sub-tile is 24 instructions of 32
+// cycles where the fp32 instruction needs 64 of 64, and what bounds the kernel is then the arithmetic around them.  Scores
+// have an absolute error, so Q and K only need an upper limit; a column of V has the window of split_f32.h.  A workgroup that
+// meets a value outside starts again on v_mfma_f32_32x32x2_f32: there an instruction takes K index 0 from lanes 0-31 and K index 1
+// from lanes 32-63, and accumulator register 4g+i of a lane in half h is key 8g + 4h + i, so keys (8g+i, 8g+4+i) are paired in
+// instruction (g, i), A is the 16-byte chunk (2g+h) of a V^T row, and the head dimension is paired the same way.
+// us per launch, 12 heads, fp32 instruction / halves: 20 x 100 tokens 13.6 / 10.0, 8 x 256 23.4 / 16.9, 20 x 300 74 / 43, 20 x 512 148 / 72;
+// packed, 20 requests of 5 to 500 tokens 100 / 47.
 //
 // V may be given transposed ([B,h,d,pitch], as the QKV epilogue writes it with v_seq_pitch: its tiles are then copied)
 // or row-major ([B,h,S,d]: a thread scatters its four values of a key into four V^T rows).  With cu_seqlens q,k,v are
@@ -25,6 +29,7 @@
 #include <set>
 
 #include "attention_common.h"
+#include "split_f32.h"
 
 namespace ttmi {
 
@@ -33,9 +38,14 @@ namespace {
 constexpr int kBKV = 64;         // keys per LDS tile
 constexpr int kRow = 256;        // bytes of a K row (64 floats) and of a V^T row (64 keys)
 
-// 16-byte chunk `chunk` of row `row` of a tile with 256-byte rows: the 16 lanes the LDS serves together read one chunk
-// column of 16 different rows, so the chunk index is XORed with the row
-__device__ __forceinline__ int tile_off(int row, int chunk) { return row * kRow + ((chunk ^ (row & 15)) << 4); }
+// 16-byte chunk `chunk` of row `row` of a tile with 256-byte rows.  The 16 lanes that the LDS serves together read one chunk
+// column of 16 rows (0-3, 12-15, 20-27 of 32, or the others), and the scatter of a row-major V writes to every fourth row:
+// for both the chunk index is XORed with 16 different values.
+__device__ __forceinline__ int tile_off(int row, int chunk) { return row * kRow + ((chunk ^ (((row >> 2) ^ (row << 2)) & 15)) << 4); }
+// Where the halves of keys 4 c ... 4 c + 3 lie in a V^T row: the keys that a lane multiplies at once (registers 8 kk ... 8 kk + 7 of
+// its scores: keys 4 h + i and 8 + 4 h + i of 16) are one 16-byte chunk.
+__device__ __forceinline__ int vt_chunk(int c) { return 2 * (c >> 2) + (c & 1); }
+__device__ __forceinline__ int vt_half(int c) { return (c >> 1) & 1; }
 
 template <int NW>
 constexpr int lds_bytes() {
@@ -43,15 +53,292 @@ constexpr int lds_bytes() {
   return tiles > outb ? tiles : outb;
 }
 
-template <int NW, bool VT, bool PACKED>
+// The scores and the weighted sum of one wavefront's 32 queries (ot: not yet divided by the row sums, of which l_run holds this
+// half-wavefront's share).  SPLIT: on the 16-bit matrix instructions, everything in halves (split_f32.h); the answer is whether
+// a value does not fit them, the same for the whole workgroup.  Otherwise on the fp32 instruction.
+template <int NW, bool VT, bool SPLIT>
+__device__ __forceinline__ bool attend(char* const smem, const float* __restrict__ qb, const float* __restrict__ kb, const float* __restrict__ vb,
+                                       const float* __restrict__ mask, int q0, int kv_len, int v_pitch, float scale_log2e, float inv_scale,
+                                       floatx16 (&ot)[2], float& l_run) {
+  constexpr int kPieces = 1024 / (NW * 64);  // 16-byte pieces of a K (V^T) tile per thread: 64 rows of 16
+  constexpr int kTile = kBKV * kRow;         // 16 KB
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  const int q_len = kv_len;  // self attention: as many queries as keys
+
+  // Q fragments: B operand of the first product.  fp32: chunk 2kk+lhalf of the lane's query row; halves: eight values of the
+  // head dimension, hi and lo.
+  u32x4 qf[8];
+  float largest = 0.f;  // of Q and K: only their upper limit counts, since a score's error is absolute
+  {
+    const int qi = q0 + lrow;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      floatx4 x[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int c = SPLIT ? 4 * kk + 2 * lhalf + j : 4 * kk + 2 * j + lhalf;
+        if (qi < q_len) x[j] = *reinterpret_cast<const floatx4*>(qb + (int64_t)qi * kD + c * 4);
+        else x[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const float a = x[w >> 1][2 * (w & 1)], b = x[w >> 1][2 * (w & 1) + 1];
+          qf[2 * kk][w] = split_hi(a, b);
+          qf[2 * kk + 1][w] = split_lo(qf[2 * kk][w], a, b);
+          split_max(largest, a, b);
+        }
+      } else {
+        qf[2 * kk] = __builtin_bit_cast(u32x4, x[0]);
+        qf[2 * kk + 1] = __builtin_bit_cast(u32x4, x[1]);
+      }
+    }
+  }
+
+  floatx16 oc[2];  // SPLIT: the products of a hi and a lo, 2^16 times too large
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) ot[t][e] = 0.f, oc[t][e] = 0.f;
+  float m_run = -kFarthestScore;
+  l_run = 0.f;
+
+  // tile staging: thread -> chunk ch of rows r0 + 64*NW/16*p; global -> registers one tile ahead -> LDS.  (Of a row-major V a
+  // thread takes neighbouring keys, whose halves are written together.)
+  constexpr int kRowsPerPass = NW * 64 / 16;
+  const int ch = tid & 15, r0 = tid >> 4;
+  auto v_key = [&](int p) __attribute__((always_inline)) { return SPLIT ? (p >> 1) * (2 * kRowsPerPass) + 2 * r0 + (p & 1) : r0 + p * kRowsPerPass; };
+  floatx4 kreg[kPieces], vreg[kPieces];
+  float v_largest[VT ? kPieces : 4];  // of a V^T row
+#pragma unroll
+  for (int i = 0; i < (VT ? kPieces : 4); ++i) v_largest[i] = 0.f;
+  uint32_t mreg = 0;
+
+  auto load_tile = [&](int tile) __attribute__((always_inline)) {
+    const int key0 = tile * kBKV;
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+      const int r = r0 + p * kRowsPerPass;
+      kreg[p] = *reinterpret_cast<const floatx4*>(kb + (int64_t)min(key0 + r, kv_len - 1) * kD + ch * 4);
+      if constexpr (VT)  // row r of V^T, keys 4ch.. of the tile
+        vreg[p] = *reinterpret_cast<const floatx4*>(vb + (int64_t)r * v_pitch + min(key0 + ch * 4, v_pitch - 4));
+      else  // a key of the tile, head dimensions 4ch..
+        vreg[p] = *reinterpret_cast<const floatx4*>(vb + (int64_t)min(key0 + v_key(p), kv_len - 1) * kD + ch * 4);
+    }
+    if (tid < kBKV && mask != nullptr) mreg = load_mask(mask + min(key0 + tid, kv_len - 1));
+  };
+  auto store_tile = [&](int tile, int stage) __attribute__((always_inline)) {
+    char* const kt = smem + stage * kTile;
+    char* const vt = smem + 2 * kTile + stage * kTile;
+    const int nv = kv_len - (tile * kBKV + ch * 4);  // valid keys in this thread's V^T chunk
+#pragma unroll
+    for (int p = 0; p < kPieces; ++p) {
+      const int r = r0 + p * kRowsPerPass;
+      const floatx4 kx = kreg[p];
+      floatx4 x = vreg[p];
+      if constexpr (VT) {
+        if (nv < 4) {  // only in the last tile: keys past the end may hold anything, zero them
+#pragma unroll
+          for (int w = 0; w < 4; ++w)
+            if (w >= nv) x[w] = 0.f;
+        }
+      } else if (tile * kBKV + v_key(p) >= kv_len) {
+        x = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+      if constexpr (SPLIT) {
+        const uint2 kh = make_uint2(split_hi(kx[0], kx[1]), split_hi(kx[2], kx[3]));
+        char* const at = kt + tile_off(r, ch >> 1) + (ch & 1) * 8;
+        *reinterpret_cast<uint2*>(at) = kh;
+        *reinterpret_cast<uint2*>(kt + (tile_off(r, (ch >> 1) ^ 8) + (ch & 1) * 8)) = make_uint2(split_lo(kh.x, kx[0], kx[1]), split_lo(kh.y, kx[2], kx[3]));
+        split_max(largest, kx[0], kx[1]);
+        split_max(largest, kx[2], kx[3]);
+        if constexpr (VT) {
+          const uint2 vh = make_uint2(split_hi(x[0], x[1]), split_hi(x[2], x[3]));
+          *reinterpret_cast<uint2*>(vt + tile_off(r, vt_chunk(ch)) + vt_half(ch) * 8) = vh;
+          *reinterpret_cast<uint2*>(vt + tile_off(r, vt_chunk(ch) ^ 8) + vt_half(ch) * 8) = make_uint2(split_lo(vh.x, x[0], x[1]), split_lo(vh.y, x[2], x[3]));
+          split_max(v_largest[p], x[0], x[1]);
+          split_max(v_largest[p], x[2], x[3]);
+        } else if (p % 2 == 1) {  // V^T[d = 4ch + w][two keys]
+          floatx4 y = vreg[p - 1];
+          if (tile * kBKV + v_key(p - 1) >= kv_len) y = floatx4{0.f, 0.f, 0.f, 0.f};
+          const int key = v_key(p - 1), c = key >> 2;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const uint32_t h = split_hi(y[w], x[w]);
+            char* const row = vt + vt_half(c) * 8 + (key & 2) * 2;
+            *reinterpret_cast<uint32_t*>(row + tile_off(ch * 4 + w, vt_chunk(c))) = h;
+            *reinterpret_cast<uint32_t*>(row + tile_off(ch * 4 + w, vt_chunk(c) ^ 8)) = split_lo(h, y[w], x[w]);
+            split_max(v_largest[w], y[w], x[w]);
+          }
+        }
+      } else {
+        *reinterpret_cast<floatx4*>(kt + tile_off(r, ch)) = kx;
+        if constexpr (VT) {
+          *reinterpret_cast<floatx4*>(vt + tile_off(r, ch)) = x;
+        } else {  // V^T[d = 4ch + w][key r]: float r % 4 of chunk r / 4 of row d
+#pragma unroll
+          for (int w = 0; w < 4; ++w) *reinterpret_cast<float*>(vt + tile_off(ch * 4 + w, r >> 2) + (r & 3) * 4) = x[w];
+        }
+      }
+    }
+    if (tid < kBKV)
+      reinterpret_cast<float*>(smem + 4 * kTile)[stage * kBKV + tid] =
+          tile * kBKV + tid < kv_len ? mask_in_scores(mreg, inv_scale) : -__builtin_inff();
+  };
+
+  // One 64-key tile from LDS stage STAGE.  m_run is kept in raw score units; p = exp2(s*c - m*c), c = scale*log2(e).
+  auto compute_tile = [&](auto stage_c) {
+    constexpr int STAGE = decltype(stage_c)::value;
+    const char* kt = smem + STAGE * kTile;
+    const char* vt = smem + 2 * kTile + STAGE * kTile;
+    const float* mk = reinterpret_cast<const float*>(smem + 4 * kTile) + STAGE * kBKV;
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {  // two 32-key sub-tiles
+      const int sk = sub * 32;
+      // st[4g+i] = score of (key sk + 8g + 4*lhalf + i, query lrow), seeded with mask/scale
+      floatx16 st;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 mv = *reinterpret_cast<const float4*>(mk + sk + 8 * g + 4 * lhalf);
+        st[4 * g] = mv.x, st[4 * g + 1] = mv.y, st[4 * g + 2] = mv.z, st[4 * g + 3] = mv.w;
+      }
+      if constexpr (SPLIT) {
+        floatx16 sc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          const u32x4 kh = *reinterpret_cast<const u32x4*>(kt + tile_off(sk + lrow, 2 * kk + lhalf));
+          const u32x4 kl = *reinterpret_cast<const u32x4*>(kt + tile_off(sk + lrow, (2 * kk + lhalf) ^ 8));
+          sc = mma32<f16>(kh, qf[2 * kk + 1], sc);
+          st = mma32<f16>(kh, qf[2 * kk], st);
+          sc = mma32<f16>(kl, qf[2 * kk], sc);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) st[e] = __builtin_fmaf(sc[e], 1.f / kSplitScale, st[e]);
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) {
+          const floatx4 kf = *reinterpret_cast<const floatx4*>(kt + tile_off(sk + lrow, 2 * kk + lhalf));
+          st = mma32<float>(kf, __builtin_bit_cast(floatx4, qf[kk]), st);
+        }
+      }
+      float mx = st[0];
+#pragma unroll
+      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
+      {
+        // the other half-wavefront holds the remaining 16 keys of this query
+        const LanePair sw = swap_halves(mx);
+        // fp32: any reference point near the maximum does, since the sums are rounded relative to their own size.  The half that holds
+        // the first keys gives it unless the other one's exponentials would leave the fp32 range (2^64 leaves 2^63 to sum).
+        // Halves: the maximum itself, so that no probability exceeds 1.
+        if constexpr (SPLIT) mx = fmaxf(sw.a, sw.b);
+        else mx = (sw.b - sw.a) * scale_log2e > 64.f ? sw.b : sw.a;
+      }
+      if (__any(mx > m_run)) {
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            ot[t][e] *= alpha;
+            if constexpr (SPLIT) oc[t][e] *= alpha;
+          }
+      }
+      const float neg_m = relative_scores(st, m_run, scale_log2e);
+      float psum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        st[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[e], scale_log2e, neg_m));
+        psum += st[e];
+      }
+      l_run += psum;
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4 ph, pl;
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            const float a = st[8 * kk + 2 * w], b = st[8 * kk + 2 * w + 1];
+            ph[w] = split_hi(a, b);
+            pl[w] = split_lo(ph[w], a, b);
+          }
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const int c = 2 * (sk / 16 + kk) + lhalf;
+            const u32x4 vh = *reinterpret_cast<const u32x4*>(vt + tile_off(t * 32 + lrow, c));
+            const u32x4 vl = *reinterpret_cast<const u32x4*>(vt + tile_off(t * 32 + lrow, c ^ 8));
+            oc[t] = mma32<f16>(vh, pl, oc[t]);
+            ot[t] = mma32<f16>(vh, ph, ot[t]);
+            oc[t] = mma32<f16>(vl, ph, oc[t]);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const floatx4 pf{st[4 * g], st[4 * g + 1], st[4 * g + 2], st[4 * g + 3]};
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const floatx4 vf = *reinterpret_cast<const floatx4*>(vt + tile_off(t * 32 + lrow, sk / 4 + 2 * g + lhalf));
+            ot[t] = mma32<float>(vf, pf, ot[t]);
+          }
+        }
+      }
+    }
+  };
+
+  const int tiles = (kv_len + kBKV - 1) / kBKV;
+  const bool wave_active = q0 < q_len;
+  load_tile(0);
+  store_tile(0, 0);
+  __syncthreads();
+  for (int tile = 0; tile < tiles; tile += 2) {
+    if (tile + 1 < tiles) load_tile(tile + 1);
+    if (wave_active) compute_tile(std::integral_constant<int, 0>{});
+    if (tile + 1 < tiles) store_tile(tile + 1, 1);
+    __syncthreads();
+    if (tile + 1 >= tiles) break;
+    if (tile + 2 < tiles) load_tile(tile + 2);
+    if (wave_active) compute_tile(std::integral_constant<int, 1>{});
+    if (tile + 2 < tiles) store_tile(tile + 2, 0);
+    __syncthreads();
+  }
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ot[t][e] = __builtin_fmaf(oc[t][e], 1.f / kSplitScale, ot[t][e]);
+    bool outside = largest >= kSplitLargest;
+    if constexpr (VT) {
+#pragma unroll
+      for (int p = 0; p < kPieces; ++p) outside = outside || split_outside(group_max<16>(v_largest[p]));
+    } else {  // (the tiles have been read: the front of LDS holds the maxima of every four keys' share)
+      float* const part = reinterpret_cast<float*>(smem);
+#pragma unroll
+      for (int w = 0; w < 4; ++w) part[r0 * kD + ch * 4 + w] = v_largest[w];
+      __syncthreads();
+      if (tid < kD) {
+        float top = 0.f;
+        for (int r = 0; r < kRowsPerPass; ++r) top = fmaxf(top, part[r * kD + tid]);
+        outside = outside || split_outside(top);
+      }
+    }
+    return __syncthreads_or(outside) != 0;
+  }
+  return false;
+}
+
+template <int NW, bool VT, bool PACKED, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void fused_attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ mask,
     float* __restrict__ out, const int32_t* __restrict__ cu, int heads, int seq, int v_pitch, float scale_log2e,
     float inv_scale, float* __restrict__ absmax) {
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
-  constexpr int kBQ = NW * 32;               // queries per workgroup
-  constexpr int kPieces = 1024 / (NW * 64);  // 16-byte pieces of a K (V^T) tile per thread: 64 rows of 16
-  constexpr int kTile = kBKV * kRow;         // 16 KB
+  constexpr int kBQ = NW * 32;  // queries per workgroup
   // dynamic LDS (lds_bytes<NW>(), more than the 64 KB a kernel gets without asking):
   // [2 x K tile | 2 x V^T tile | 2 x mask]; the front is reused for the output tile
   extern __shared__ __align__(16) char smem[];
@@ -77,151 +364,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   const float* qb = q + (int64_t)bh * seq * kD;
   const float* kb = k + (int64_t)bh * seq * kD;
   const float* vb = v + (int64_t)bh * kD * (VT ? v_pitch : seq);
-
-  // Q fragments: B operand of the first product, chunk 2kk+lhalf of the lane's query row
-  floatx4 qf[8];
-  {
-    const int qi = q0 + lrow;
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      if (qi < q_len) qf[kk] = *reinterpret_cast<const floatx4*>(qb + (int64_t)qi * kD + (2 * kk + lhalf) * 4);
-      else qf[kk] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-
+  const float* mb = mask != nullptr ? mask + (int64_t)b * seq : nullptr;
   floatx16 ot[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) ot[t][e] = 0.f;
-  float m_run = -kFarthestScore, l_run = 0.f;
-
-  // tile staging: thread -> (row r0 + 64*NW/16*p, chunk ch); global -> registers one tile ahead -> LDS
-  constexpr int kRowsPerPass = NW * 64 / 16;
-  const int ch = tid & 15, r0 = tid >> 4;
-  floatx4 kreg[kPieces], vreg[kPieces];
-  uint32_t mreg = 0;
-
-#define TTMI_FA32_LOAD(tile_)                                                                                      \
-  do {                                                                                                              \
-    const int key0_ = (tile_) * kBKV;                                                                               \
-    _Pragma("unroll") for (int p = 0; p < kPieces; ++p) {                                                           \
-      const int r_ = r0 + p * kRowsPerPass;                                                                         \
-      kreg[p] = *reinterpret_cast<const floatx4*>(kb + (int64_t)min(key0_ + r_, kv_len - 1) * kD + ch * 4);         \
-      if (VT) { /* row r_ of V^T, keys 4ch.. of the tile */                                                         \
-        const int ks_ = min(key0_ + ch * 4, v_pitch - 4);                                                           \
-        vreg[p] = *reinterpret_cast<const floatx4*>(vb + (int64_t)r_ * v_pitch + ks_);                              \
-      } else { /* key r_ of the tile, head dimensions 4ch.. */                                                      \
-        vreg[p] = *reinterpret_cast<const floatx4*>(vb + (int64_t)min(key0_ + r_, kv_len - 1) * kD + ch * 4);       \
-      }                                                                                                             \
-    }                                                                                                               \
-    if (tid < kBKV && mask) mreg = load_mask(mask + (int64_t)b * seq + min(key0_ + tid, kv_len - 1));               \
-  } while (0)
-
-#define TTMI_FA32_STORE(tile_, stage_)                                                                             \
-  do {                                                                                                              \
-    char* const kt_ = smem + (stage_) * kTile;                                                                      \
-    char* const vt_ = smem + 2 * kTile + (stage_) * kTile;                                                          \
-    const int nv_ = kv_len - ((tile_) * kBKV + ch * 4); /* valid keys in this thread's V^T chunk */                 \
-    _Pragma("unroll") for (int p = 0; p < kPieces; ++p) {                                                           \
-      const int r_ = r0 + p * kRowsPerPass;                                                                         \
-      *reinterpret_cast<floatx4*>(kt_ + tile_off(r_, ch)) = kreg[p];                                                \
-      floatx4 x_ = vreg[p];                                                                                         \
-      if (VT) {                                                                                                     \
-        if (nv_ < 4) { /* only in the last tile: keys past the end may hold anything, zero them */                  \
-          _Pragma("unroll") for (int w = 0; w < 4; ++w) if (w >= nv_) x_[w] = 0.f;                                  \
-        }                                                                                                           \
-        *reinterpret_cast<floatx4*>(vt_ + tile_off(r_, ch)) = x_;                                                   \
-      } else { /* V^T[d = 4ch + w][key r_]: float r_ % 4 of chunk r_ / 4 of row d; keys past the end are zero */    \
-        const bool live_ = (tile_) * kBKV + r_ < kv_len;                                                            \
-        _Pragma("unroll") for (int w = 0; w < 4; ++w)                                                               \
-          *reinterpret_cast<float*>(vt_ + tile_off(ch * 4 + w, r_ >> 2) + (r_ & 3) * 4) = live_ ? x_[w] : 0.f;      \
-      }                                                                                                             \
-    }                                                                                                               \
-    if (tid < kBKV)                                                                                                 \
-      reinterpret_cast<float*>(smem + 4 * kTile)[(stage_) * kBKV + tid] =                                           \
-          (tile_) * kBKV + tid < kv_len ? mask_in_scores(mreg, inv_scale) : -__builtin_inff();                      \
-  } while (0)
-
-  // One 64-key tile from LDS stage STAGE.  m_run is kept in raw score units; p = exp2(s*c - m*c), c = scale*log2(e).
-  auto compute_tile = [&](auto stage_c) {
-    constexpr int STAGE = decltype(stage_c)::value;
-    const char* kt = smem + STAGE * kTile;
-    const char* vt = smem + 2 * kTile + STAGE * kTile;
-    const float* mk = reinterpret_cast<const float*>(smem + 4 * kTile) + STAGE * kBKV;
-#pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {  // two 32-key sub-tiles
-      const int sk = sub * 32;
-      // st[4g+i] = score of (key sk + 8g + 4*lhalf + i, query lrow), seeded with mask/scale
-      floatx16 st;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float4 mv = *reinterpret_cast<const float4*>(mk + sk + 8 * g + 4 * lhalf);
-        st[4 * g] = mv.x, st[4 * g + 1] = mv.y, st[4 * g + 2] = mv.z, st[4 * g + 3] = mv.w;
-      }
-#pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
-        const floatx4 kf = *reinterpret_cast<const floatx4*>(kt + tile_off(sk + lrow, 2 * kk + lhalf));
-        st = mma32<float>(kf, qf[kk], st);
-      }
-      float mx = st[0];
-#pragma unroll
-      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, st[e]);
-      {
-        // the other half-wavefront holds the remaining 16 keys of this query
-        const LanePair sw = swap_halves(mx);
-        // Any reference point near the maximum does: the sums are rounded relative to their own size.  The half that holds
-        // the first keys gives it unless the other one's exponentials would leave the fp32 range (2^64 leaves 2^63 to sum).
-        mx = (sw.b - sw.a) * scale_log2e > 64.f ? sw.b : sw.a;
-      }
-      if (__any(mx > m_run)) {
-        const float m_new = fmaxf(m_run, mx);
-        const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * scale_log2e);
-        m_run = m_new;
-        l_run *= alpha;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) ot[t][e] *= alpha;
-      }
-      const float neg_m = relative_scores(st, m_run, scale_log2e);
-      float psum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        st[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[e], scale_log2e, neg_m));
-        psum += st[e];
-      }
-      l_run += psum;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const floatx4 pf{st[4 * g], st[4 * g + 1], st[4 * g + 2], st[4 * g + 3]};
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const floatx4 vf = *reinterpret_cast<const floatx4*>(vt + tile_off(t * 32 + lrow, sk / 4 + 2 * g + lhalf));
-          ot[t] = mma32<float>(vf, pf, ot[t]);
-        }
-      }
-    }
-  };
-
-  const int tiles = (kv_len + kBKV - 1) / kBKV;
-  const bool wave_active = q0 < q_len;
-  TTMI_FA32_LOAD(0);
-  TTMI_FA32_STORE(0, 0);
-  __syncthreads();
-  for (int tile = 0; tile < tiles; tile += 2) {
-    if (tile + 1 < tiles) TTMI_FA32_LOAD(tile + 1);
-    if (wave_active) compute_tile(std::integral_constant<int, 0>{});
-    if (tile + 1 < tiles) TTMI_FA32_STORE(tile + 1, 1);
-    __syncthreads();
-    if (tile + 1 >= tiles) break;
-    if (tile + 2 < tiles) TTMI_FA32_LOAD(tile + 2);
-    if (wave_active) compute_tile(std::integral_constant<int, 1>{});
-    if (tile + 2 < tiles) TTMI_FA32_STORE(tile + 2, 0);
-    __syncthreads();
-  }
-#undef TTMI_FA32_LOAD
-#undef TTMI_FA32_STORE
+  float l_run;
+  bool again = true;
+  if constexpr (SPLIT) again = attend<NW, VT, true>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, ot, l_run);
+  if (again) attend<NW, VT, false>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, ot, l_run);
 
   // normalise and write: ot[t][4g+i] = O[query lrow][d = 32t + 8g + 4*lhalf + i]
   const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
@@ -299,14 +447,19 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
   };
   const bool vt = v_seq_pitch > 0, packed = cu != nullptr;
   int rc = 0;
-#define TTMI_FA32_CASE(NW, VT, PACKED) rc = launch(&fused_attention_f32_kernel<NW, VT, PACKED>, NW * 64, lds_bytes<NW>())
-  if (nw == 8) {
-    if (vt) { if (packed) TTMI_FA32_CASE(8, true, true); else TTMI_FA32_CASE(8, true, false); }
-    else { if (packed) TTMI_FA32_CASE(8, false, true); else TTMI_FA32_CASE(8, false, false); }
-  } else {
-    if (vt) { if (packed) TTMI_FA32_CASE(4, true, true); else TTMI_FA32_CASE(4, true, false); }
-    else { if (packed) TTMI_FA32_CASE(4, false, true); else TTMI_FA32_CASE(4, false, false); }
-  }
+#define TTMI_FA32_CASE(NW, VT, PACKED, SPLIT) rc = launch(&fused_attention_f32_kernel<NW, VT, PACKED, SPLIT>, NW * 64, lds_bytes<NW>())
+#define TTMI_FA32_WAVES(VT, PACKED, SPLIT)          \
+  do {                                              \
+    if (nw == 8) TTMI_FA32_CASE(8, VT, PACKED, SPLIT); \
+    else TTMI_FA32_CASE(4, VT, PACKED, SPLIT);         \
+  } while (0)
+  // A dense batch with V row-major is what the quantised layers pass: they round the result to 8 bits, which turns a difference in
+  // the last bit into a whole step, so it keeps the fp32 instruction.
+  if (vt && packed) TTMI_FA32_WAVES(true, true, true);
+  else if (vt) TTMI_FA32_WAVES(true, false, true);
+  else if (packed) TTMI_FA32_WAVES(false, true, true);
+  else TTMI_FA32_WAVES(false, false, false);
+#undef TTMI_FA32_WAVES
 #undef TTMI_FA32_CASE
   if (rc != 0) return rc;
   return launch_status("fused_attention_f32_kernel");
