@@ -1306,11 +1306,11 @@ def _split_error_bound(A, W):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(33, 8, 32), (40, 72, 64), (100, 776, 96), (129, 2304, 768), (264, 768, 3072), (387, 3072, 768),
+@pytest.mark.parametrize("M,N,K", [(33, 8, 32), (40, 72, 64), (100, 776, 96), (100, 776, 416), (129, 2304, 544), (300, 1024, 1056), (129, 2304, 768), (264, 768, 3072), (387, 3072, 768),
                                    (1000, 1536, 160), (1999, 768, 768), (2000, 3072, 128), (2500, 2304, 768), (8200, 520, 256)])
 def test_packed_weights(ttmi, M, N, K):
-    """fp32 products on the 16-bit matrix instructions: every tile, ragged rows and columns, one to many K steps, K slices, every
-    epilogue; rows past M stay untouched.  No further from 64 bits than the fp32 instruction is."""
+    """fp32 products on the 16-bit matrix instructions: every tile, ragged rows and columns, one to many K steps, shares
+    of them that differ by group of wavefronts, K slices, every epilogue; rows past M stay untouched.  No further from 64 bits than the fp32 instruction is."""
     import ctypes
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")

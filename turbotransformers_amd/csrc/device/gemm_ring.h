@@ -535,19 +535,22 @@ struct RingTile {
   X(128, 192, 4, 2, 3, 1, 8.73f, 10.6f, 0.465f, 0.465f)      \
   X(256, 128, 4, 2, 3, 1, 11.0f, 10.9f, 0.594f, 0.594f)
 
-// X(BM, BN, WM, WN, A steps in registers, B stages, resident, first, again, lone, shared): fp32 with packed weights (gemm_split.h).
-// Fits of the same kind (M = 40 ... 10240, hidden 768 and 1024; the tile the model picks is 0.14 % slower than the best one).
-#define TTMI_SPLIT_TILES(X)                                     \
-  X(32, 64, 2, 2, 4, 6, 2, 3.43f, 1.13f, 0.252f, 0.167f)        \
-  X(64, 64, 4, 2, 4, 6, 2, 3.74f, 1.81f, 0.313f, 0.250f)        \
-  X(64, 128, 2, 4, 4, 6, 1, 4.29f, 5.50f, 0.397f, 0.397f)       \
-  X(64, 192, 4, 2, 2, 4, 1, 5.33f, 8.27f, 0.512f, 0.512f)       \
-  X(64, 256, 2, 4, 2, 4, 1, 5.66f, 10.4f, 0.608f, 0.607f)       \
-  X(128, 128, 4, 2, 2, 4, 1, 5.94f, 10.5f, 0.571f, 0.571f)      \
-  X(128, 192, 4, 2, 2, 4, 1, 7.84f, 16.2f, 0.718f, 0.718f)
+// X(BM, BN, WM, WN, K groups, A steps in registers, B stages, resident, first, again, lone, shared): fp32 with packed weights
+// (gemm_split.h).  Fits of the same kind (M = 40 ... 10240, K = 256 ... 3072; the tile the model picks is 0.1 % slower than the best one).
+#define TTMI_SPLIT_TILES(X)                                        \
+  X(32, 32, 2, 1, 4, 4, 5, 1, 4.80f, 3.23f, 0.100f, 0.100f)        \
+  X(32, 64, 2, 2, 1, 4, 6, 2, 3.02f, 1.19f, 0.260f, 0.161f)        \
+  X(32, 64, 2, 2, 3, 2, 4, 1, 4.55f, 3.18f, 0.154f, 0.154f)        \
+  X(64, 64, 4, 2, 1, 4, 6, 2, 3.97f, 1.59f, 0.298f, 0.246f)        \
+  X(64, 64, 2, 2, 2, 2, 4, 1, 4.69f, 3.90f, 0.233f, 0.234f)        \
+  X(64, 128, 2, 4, 1, 4, 6, 1, 4.47f, 4.90f, 0.390f, 0.389f)       \
+  X(64, 192, 4, 2, 1, 2, 4, 1, 4.96f, 7.32f, 0.508f, 0.509f)       \
+  X(64, 256, 2, 4, 1, 2, 4, 1, 5.62f, 9.16f, 0.603f, 0.603f)       \
+  X(128, 128, 4, 2, 1, 2, 4, 1, 5.71f, 9.31f, 0.573f, 0.573f)      \
+  X(128, 192, 4, 2, 1, 2, 4, 1, 7.29f, 13.8f, 0.738f, 0.738f)
 
 #define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
-#define TTMI_SPLIT_ROW(BM, BN, WM, WN, DA, SB, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
+#define TTMI_SPLIT_ROW(BM, BN, WM, WN, KG, DA, SB, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
 template <size_t ELEM>
 struct RingTiles;
 template <>
@@ -640,7 +643,7 @@ inline bool ring_operands_ok(const GemmArgs& g) {  // 32-bit buffer offsets, col
   return g.n % 8 == 0 && (int64_t)g.m * g.lda * (int64_t)sizeof(T) < limit && (int64_t)g.n * g.ldb * (int64_t)sizeof(T) < limit;
 }
 
-template <int BM, int BN, int WM, int WN, int DA, int SB, typename Epi>
+template <int BM, int BN, int WM, int WN, int KG, int DA, int SB, typename Epi>
 int launch_split(GemmArgs g, const Epi& epi, int slices, hipStream_t s);  // gemm_split.h
 
 template <typename T, typename Epi>
@@ -648,8 +651,8 @@ inline int launch_ring_tile(int tile, const GemmArgs& g, const Epi& epi, int sli
   int index = 0;
   if constexpr (sizeof(T) == 4) {
     if (g.b_split != nullptr) {
-#define TTMI_SPLIT_TRY(BM, BN, WM, WN, DA, SB, R, F, A, L, S) \
-  if (tile == index++) return launch_split<BM, BN, WM, WN, DA, SB>(g, epi, slices, s);
+#define TTMI_SPLIT_TRY(BM, BN, WM, WN, KG, DA, SB, R, F, A, L, S) \
+  if (tile == index++) return launch_split<BM, BN, WM, WN, KG, DA, SB>(g, epi, slices, s);
       TTMI_SPLIT_TILES(TTMI_SPLIT_TRY)
 #undef TTMI_SPLIT_TRY
       return fail(TTMI_EINVAL, "no such tile");

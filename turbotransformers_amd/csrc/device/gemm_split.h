@@ -6,7 +6,7 @@
 // What bounds it: up to some hundred rows the instructions of a step (below), then the matrix pipe: 128 x 192 tiles take 0.77 us a step
 // against 0.55 of matrix time, and 10240 x 3072 x 768 runs at 0.98 PFLOP/s of 16-bit products, where fp16 tiles run.
 // us per launch, fp32 ring tiles / here: 2000 x 2304 x 768 56 / 27, 2000 x 768 x 768 22.4 / 14.4, 2000 x 3072 x 768 (GELU) 73 / 31,
-// 264 x 3072 x 768 16.5 / 12.4, 128 x 2304 x 768 9.9 / 9.4, 10240 x 768 x 3072 335 / 141.
+// 264 x 3072 x 768 16.5 / 10.9, 128 x 2304 x 768 9.9 / 8.0, 10240 x 768 x 3072 335 / 141.
 #pragma once
 
 #include "gemm_ring.h"
@@ -30,9 +30,12 @@ constexpr int split_lds_bytes() { return (kSplitStagesA * BM + SB * BN) * kRowBy
 // s + SB - 1 are on their way into LDS without passing a register.  All of it goes out between the matrix instructions: a wavefront
 // issues an instruction every eight cycles, so what a step costs besides its matrix time is the number of its instructions
 // (B split on the way in as well, 2000 x 3072 x 768: 35.7 us; fragments split by each wavefront behind LDS would be more still).
-template <int BM, int BN, int WM, int WN, int DA, int SB, typename Epi>
-__global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const GemmArgs g, const Epi epi) {
-  constexpr int NW = WM * WN, NT = NW * kWave, ROWS = NT / 8;  // a thread loads 16 bytes of A, eight threads a row
+// KG > 1: as many such groups of wavefronts share a tile, each with its part of the K steps and stages of its own, and meet in LDS at
+// the end.  Where the tiles are fewer than the CUs a step is a chain of waits, whose number this
+// divides (us, one group / here: 128 x 768 x 3072 27 / 13.6, 128 x 768 x 768 8.5 / 7.0, 128 x 2304 x 768 9.0 / 8.0, 264 x 3072 x 768 12.0 / 10.9).
+template <int BM, int BN, int WM, int WN, int KG, int DA, int SB, typename Epi>
+__global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(const GemmArgs g, const Epi epi) {
+  constexpr int NW = WM * WN, NT = NW * kWave, ROWS = NT / 8;  // of a group; a thread loads 16 bytes of A, eight threads a row
   constexpr int PASSES = BM / ROWS, B_LOADS = BN / 8 / NW;
   constexpr int RB = BM / WM / 16, CB = BN / WN / 16;    // 16 x 16 blocks per wavefront
   constexpr int A_STAGE = BM * kRowBytes, B_STAGE = BN * kRowBytes, B_BASE = kSplitStagesA * A_STAGE;
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
   static_assert((DA == 2 || DA == 4) && SB >= 4 && (SB - 3) * (PASSES + B_LOADS) + 2 * PASSES + DA * PASSES < 64, "vmcnt is a six-bit counter");
   using Acc = floatx4;
 
-  extern __shared__ __align__(16) char smem[];
+  extern __shared__ __align__(16) char lds[];
 
   const int tiles = g.tiles_m * g.tiles_n, total = tiles * g.slices;  // (as in gemm_ring_kernel)
   const bool remap = total >= kXcdRemapMinTiles;
@@ -57,7 +60,9 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
   int tile_m, tile_n;
   tile_coords(logical, g.tiles_m, g.tiles_n, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  char* const smem = lds + group * split_lds_bytes<BM, BN, SB>();
+  const int tid = threadIdx.x - group * NT, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm0 = (wave / WN) * (BM / WM), wn0 = (wave % WN) * (BN / WN);
   const int lrow = lane & 15, lgrp = lane >> 4;
   int kdim = g.k, z_epi = 0;
@@ -68,7 +73,9 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
     k_lo = (uint32_t)lo * (uint32_t)sizeof(float);
     z_epi = slice;
   }
-  const int ksteps = kdim / BK;
+  // a group's share: `ksteps` steps of K, of which the last group's may be short (a step past its `valid` ones reads zeros)
+  const int ksteps = (kdim / BK + KG - 1) / KG, valid = KG > 1 ? max(min(kdim / BK - group * ksteps, ksteps), 0) : ksteps;
+  if constexpr (KG > 1) k_lo += (uint32_t)(group * ksteps) * kRowBytes;
 
   // ---- loads (rows past the edge repeat the last one; steps past the last read zeros)
   const int sub = tid >> 3, kq = tid & 7;
@@ -92,11 +99,11 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
   lds_char* lds0 = reinterpret_cast<lds_char*>(reinterpret_cast<uintptr_t>(smem));
   const int a_size = (int)((int64_t)g.m * lda_bytes), b_size = (int)((int64_t)g.n * ldb_bytes);
   auto request_a = [&](int p, int step, floatx4& dst) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.a), 0, step < ksteps ? a_size : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.a), 0, step < valid ? a_size : 0, 0x00020000);
     dst = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff_a[p], k_lo + step * kRowBytes, 0));
   };
   auto request_b = [&](int i, int step, int at) __attribute__((always_inline)) {
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.b_split), 0, step < ksteps ? b_size : 0, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g.b_split), 0, step < valid ? b_size : 0, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, lds0 + at + (wave * B_LOADS + i) * 1024, 16, voff_b[i], k_lo + step * kRowBytes, 0, 0);
   };
 #else
@@ -237,8 +244,9 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
       for (int p = 0; p < PASSES + B_PASSES; ++p) {
         const int row = (p < PASSES ? p : p - PASSES) * ROWS + sub;
         const char* src = p < PASSES ? g.a + (int64_t)min(m0 + row, g.m - 1) * lda_bytes : g.b + (int64_t)min(n0 + row, g.n - 1) * ldb_bytes;
-        *reinterpret_cast<Chunk*>(smem + (p < PASSES ? 0 : B_BASE) + row * kRowBytes + ((kq ^ split_swizzle(sub)) << 4)) =
-            *reinterpret_cast<const Chunk*>(src + k_lo + s * kRowBytes + kq * 16);
+        floatx4 x = *reinterpret_cast<const floatx4*>(src + (s < valid ? k_lo + s * kRowBytes : 0u) + kq * 16);
+        if (s >= valid) x = floatx4{0.f, 0.f, 0.f, 0.f};
+        *reinterpret_cast<floatx4*>(smem + (p < PASSES ? 0 : B_BASE) + row * kRowBytes + ((kq ^ split_swizzle(sub)) << 4)) = x;
       }
       __syncthreads();
 #pragma unroll
@@ -298,18 +306,48 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
     // (every stage has been read, and the loads past the last step are waited for: the first words of LDS hold the wavefronts' answers)
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
-    int* const answers = reinterpret_cast<int*>(smem);
+    int* const answers = reinterpret_cast<int*>(lds);
     const bool any = __ballot(outside) != 0;
-    if (lane == 0) answers[wave] = any;
+    if (lane == 0) answers[group * NW + wave] = any;
     __syncthreads();
     int again = 0;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) again |= answers[w];
+    for (int w = 0; w < KG * NW; ++w) again |= answers[w];
     if (__builtin_amdgcn_readfirstlane(again) != 0) fp32_loop(swap_tag);
   };
 
-  auto read = [&](int i, int j, int e) __attribute__((always_inline)) {
+  auto sum = [&](int i, int j, int e) __attribute__((always_inline)) {
     return __builtin_fmaf(acc_read(cross[i][j][e]), 1.f / kSplitScale, acc_read(acc[i][j][e]));
+  };
+  // the groups' sums meet: those of the others pass through LDS, lane by lane
+  floatx4 other[KG > 1 ? RB : 1][KG > 1 ? CB : 1];
+  auto read = [&](int i, int j, int e) __attribute__((always_inline)) {
+    if constexpr (KG > 1) return sum(i, j, e) + other[i][j][e];
+    else return sum(i, j, e);
+  };
+  auto meet = [&]() __attribute__((always_inline)) {
+    if constexpr (KG > 1) {
+      floatx4* const at = reinterpret_cast<floatx4*>(lds) + wave * (RB * CB * kWave) + lane;
+      constexpr int PER_GROUP = NW * RB * CB * kWave;
+      __syncthreads();  // (the wavefronts' answers have been read)
+      if (group != 0) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+          for (int j = 0; j < CB; ++j) at[(group - 1) * PER_GROUP + (i * CB + j) * kWave] = floatx4{sum(i, j, 0), sum(i, j, 1), sum(i, j, 2), sum(i, j, 3)};
+      }
+      __syncthreads();
+      if (group != 0) return false;
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          other[i][j] = at[(i * CB + j) * kWave];
+#pragma unroll
+          for (int o = 1; o < KG - 1; ++o) other[i][j] += at[o * PER_GROUP + (i * CB + j) * kWave];
+        }
+    }
+    return true;
   };
   auto unit_chunk = [&](int p) __attribute__((always_inline)) { return 2 * (2 * p + (lgrp & 1)) + (lgrp >> 1); };
   bool swap = true;
@@ -319,12 +357,14 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
     ColumnQuads<float, CB, false> quads;
     quads.load(epi.bias_ptr(), nullptr, n0 + wn0, g.n, lgrp, g.b);
     k_loop(std::true_type{});
+    if (!meet()) return;
     store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax, read);
   } else {
     if constexpr (HasColumnPass<Epi>::value) {
       float bj[CB];
       load_bias_columns_stride<CB, 16>(epi, n0 + wn0 + lrow, g.n, bj);
       k_loop(std::false_type{});
+      if (!meet()) return;
 #pragma unroll
       for (int j = 0; j < CB; ++j) {
         const int n = n0 + wn0 + j * 16 + lrow;
@@ -357,23 +397,23 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_split_kernel(const Ge
   }
 }
 
-template <int BM, int BN, int WM, int WN, int DA, int SB, typename Epi>
+template <int BM, int BN, int WM, int WN, int KG, int DA, int SB, typename Epi>
 int launch_split(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
-  constexpr int LDS = split_lds_bytes<BM, BN, SB>();
+  constexpr int LDS = KG * split_lds_bytes<BM, BN, SB>();
   static_assert(LDS <= kLdsPerCu, "tile does not fit in LDS");
-  if (describe_only("dma", WM * WN, BM, BN, slices)) return 0;
+  if (describe_only("dma", KG * WM * WN, BM, BN, slices)) return 0;
   g.tiles_m = (g.m + BM - 1) / BM;
   g.tiles_n = (g.n + BN - 1) / BN;
   g.slices = slices;
   const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n * slices;
   TTMI_REQUIRE(tiles < (1ll << 30), "GEMM grid too large");
   const unsigned grid_x = tiles >= kXcdRemapMinTiles ? (unsigned)(ceil_div(tiles, kNumXcd) * kNumXcd) : (unsigned)tiles;
-  auto kern = gemm_split_kernel<BM, BN, WM, WN, DA, SB, Epi>;
+  auto kern = gemm_split_kernel<BM, BN, WM, WN, KG, DA, SB, Epi>;
   if (LDS > 64 * 1024) {
     const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
     if (rc != 0) return rc;
   }
-  hipLaunchKernelGGL(kern, dim3(grid_x), dim3(WM * WN * kWave), LDS, s, g, epi);
+  hipLaunchKernelGGL(kern, dim3(grid_x), dim3(KG * WM * WN * kWave), LDS, s, g, epi);
   return launch_status("gemm_split_kernel");
 }
 
