@@ -335,6 +335,16 @@ TTMI_API int ttmi_fused_attention(const void* q, const void* k, const void* v, c
                                   const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq,
                                   int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype, void* stream);
 
+/* ttmi_fused_attention, the same bits in `out`, whose launch may also read `count` ranges of device memory (whole words:
+ * 4-byte aligned, a multiple of 4 bytes) and drop what it read: weights of the products that follow on the stream, which then
+ * come out of the last-level cache.  Worth it for weights that are in no cache, as those of a model that is larger than the cache.
+ * `ahead`, `ahead_bytes`: HOST arrays.  A launch that fills the chip by itself reads nothing. */
+#define TTMI_MAX_AHEAD 4
+TTMI_API int ttmi_fused_attention_ahead(const void* q, const void* k, const void* v, const float* mask, void* out,
+                                        const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq,
+                                        int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype,
+                                        const void* const* ahead, const int64_t* ahead_bytes, int64_t count, void* stream);
+
 /* Attention that returns its probabilities, for head_dim 64: P = softmax(scale * Q K^T + mask), out = P V with
  * K = [k_past | k] and V = [v_past | v] along the sequence.  q is [B,h,F,64]; k_past, v_past [B,h,past,64] (NULL with
  * past = 0), k, v [B,h,keys-past,64]; `mask` is an additive fp32 [B,keys], or [B,F,keys] with mask_per_query, or NULL;

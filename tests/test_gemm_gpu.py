@@ -1170,6 +1170,34 @@ def test_packed_attention_of_many_sequences(ttmi, dt, B, h, longest):
 
 
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("B,S,v_transposed,packed", [(1, 100, True, False), (1, 20, True, False), (2, 200, False, False), (22, 130, True, False),
+                                                     (2, 60, True, True)])
+def test_attention_that_reads_ahead(ttmi, dt, B, S, v_transposed, packed):
+    """The same bits with ranges to read ahead, on forms that read them and forms that do not (a full chip, a packed batch, fp32 with V
+    row-major); ranges of nothing, of one word, ragged, and larger than a round of the reading workgroups.  What is no whole word is refused."""
+    import ctypes
+    rng = np.random.default_rng(S)
+    h, d = 12, 64
+    Q, K, V = (dev(rng.standard_normal((B, h, S, d), np.float32), dt) for _ in range(3))
+    V, pitch = _v_operand(host(V), dt, v_transposed)
+    cu = torch.arange(B + 1, dtype=torch.int32, device="cuda") * S
+    ranges = [torch.ones(n, dtype=torch.int32, device="cuda") for n in (1, 1, 300001, 8 << 20)]
+    data = (ctypes.c_void_p * 4)(*[r.data_ptr() for r in ranges])
+
+    def run(sizes):
+        out = torch.full((B * S, h * d), 9.0, dtype=Q.dtype, device="cuda")
+        rc = ttmi.ttmi_fused_attention_ahead(ptr(Q), ptr(K), ptr(V), None, ptr(out), ptr(cu) if packed else None, B, h, S, d, pitch,
+                                             0.125, TTMI_DTYPES[dt], data, (ctypes.c_int64 * 4)(*sizes), len(sizes), stream())
+        return rc, out
+
+    (rc, want), (rc2, got) = run([]), run([0, 4, 4 * 300001, 32 << 20])
+    ok(rc)
+    ok(rc2)
+    assert torch.equal(got, want) and bool(torch.isfinite(want.float()).all())
+    assert run([4, 2])[0] != 0 and run([-4])[0] != 0
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("M,h,steps", [(1, 1, 1), (16, 1, 16), (17, 12, 12), (33, 3, 17), (8, 12, 24), (31, 4, 32), (40, 2, 33)])
 def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps):
     """LayerNorm on the rows' way into the form for few rows (and, past its sizes, in a launch of its own): one and two steps of K

@@ -900,3 +900,18 @@ def test_feed_forward_blocks(tt, oracle, dtype, is_trans_weight):
     assert got.dtype == dtype and max_abs(f(got), oracle.distill_ffn(*args)) < tol
     with pytest.raises(RuntimeError, match="model_dim"):
         pw(torch.zeros(1, 2, H + 8, device="cuda", dtype=dtype), is_trans_weight=is_trans_weight)
+
+
+@pytest.mark.parametrize("dtype,layers", [(torch.float32, 5), (torch.float16, 9)])
+def test_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
+    """Weights of more than the last-level cache holds are read ahead in the layer loop: the same bits as layer by layer, on the first
+    pass (which lays the weights out) and the second, at sizes where they are read ahead and where not."""
+    from transformers import BertConfig, BertModel
+    torch.manual_seed(0)
+    cfg = BertConfig(vocab_size=10, hidden_size=1024, num_hidden_layers=layers, num_attention_heads=16, intermediate_size=4096)
+    encoder = tt.BertEncoder.from_torch(BertModel(cfg).to("cuda", dtype).eval().encoder)
+    for batch, seq in [(1, 40), (1, 40), (1, 32), (2, 200)]:
+        x = torch.randn(batch, seq, 1024, device="cuda", dtype=dtype)
+        one_call = encoder(x, return_type=tt.ReturnType.TORCH)[0]
+        by_layer = encoder(x, output_hidden_states=True, return_type=tt.ReturnType.TORCH)[0]
+        assert torch.equal(one_call, by_layer) and bool(torch.isfinite(one_call.float()).all())

@@ -153,7 +153,13 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
                                                                  const T* __restrict__ v, const float* __restrict__ mask,
                                                                  T* __restrict__ out, const int32_t* __restrict__ cu,
                                                                  int heads, int seq, int v_pitch, float scale_log2e,
-                                                                 float inv_scale) {
+                                                                 float inv_scale, const Ahead ahead) {
+  if constexpr (!PACKED) {
+    if ((int)blockIdx.y >= ahead.rows) {
+      touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
+      return;
+    }
+  }
   // one LDS block: [2 x K tile | 2 x V^T tile | 2 x mask]; the front is reused for the output tile
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
   constexpr int kBQ = NW * 32;    // queries per workgroup
@@ -321,12 +327,13 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
 
 // attention_split.hip: the keys of a head split over the wavefronts of a workgroup
 int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s);
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s);
 
-// absmax / slots_written: see ttmi_fused_attention_absmax; both null for the plain entry point
+// absmax / slots_written: see ttmi_fused_attention_absmax; ahead: see ttmi_fused_attention_ahead; null for the plain entry point
 static int fused_attention_impl(const void* q, const void* k, const void* v, const float* mask, void* out,
                                 const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
-                                int64_t v_seq_pitch, float scale, int dtype, float* absmax, int* slots_written, void* stream) {
+                                int64_t v_seq_pitch, float scale, int dtype, float* absmax, int* slots_written, const Ahead* ahead,
+                                void* stream) {
   TTMI_REQUIRE(q && k && v && out, "null tensor");
   TTMI_REQUIRE(head_dim == kD, "fused attention is built for head_dim 64");
   TTMI_REQUIRE(dtype == TTMI_F16 || dtype == TTMI_BF16 || dtype == TTMI_F32, "fused attention is built for fp16 / bf16 / fp32");
@@ -372,7 +379,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   if (split && cu_seqlens == nullptr && v_seq_pitch > 0) {
     const bool leave_maxima = absmax != nullptr && dtype == TTMI_F32 && split_wgs <= TTMI_ABSMAX_SLOTS;
     const int rc = split_attention(q, k, v, mask, out, batch, heads, seq, v_seq_pitch, scale, dtype,
-                                   leave_maxima ? absmax : nullptr, (hipStream_t)stream);
+                                   leave_maxima ? absmax : nullptr, ahead, cus, (hipStream_t)stream);
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;
   }
@@ -383,6 +390,13 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
+  Ahead read_ahead{};
+  if (dtype != TTMI_F32 && cu_seqlens == nullptr) {
+    const unsigned more = ahead_rows(ahead, (int64_t)grid.x * grid.y, grid.x, cus);
+    if (more > 0) read_ahead = *ahead;
+    read_ahead.rows = (int)grid.y;
+    grid.y += more;
+  }
   if (dtype == TTMI_F32) {
     // the per-workgroup maxima: dense fp32 batches whose workgroups fit the slots
     const bool leave_maxima = absmax != nullptr && cu_seqlens == nullptr && (int64_t)grid.x * grid.y <= TTMI_ABSMAX_SLOTS;
@@ -393,7 +407,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }
 #define TTMI_FA_LAUNCH(T, PACKED, VT, NW)                                                                              \
   hipLaunchKernelGGL((fused_attention_kernel<T, PACKED, VT, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, \
-                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale)
+                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale, read_ahead)
 #define TTMI_FA_WAVES(T, PACKED, VT)                  \
   do {                                                \
     if (nw == 8) TTMI_FA_LAUNCH(T, PACKED, VT, 8);    \
@@ -424,7 +438,7 @@ int ttmi_fused_attention(const void* q, const void* k, const void* v, const floa
                          const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
                          int64_t v_seq_pitch, float scale, int dtype, void* stream) {
   return fused_attention_impl(q, k, v, mask, out, cu_seqlens, batch, heads, seq, head_dim, v_seq_pitch, scale, dtype, nullptr,
-                              nullptr, stream);
+                              nullptr, nullptr, stream);
 }
 
 int ttmi_fused_attention_absmax(const void* q, const void* k, const void* v, const float* mask, void* out,
@@ -434,7 +448,23 @@ int ttmi_fused_attention_absmax(const void* q, const void* k, const void* v, con
   TTMI_REQUIRE(absmax_slots && slots_written, "null absmax arguments");
   *slots_written = 0;
   return fused_attention_impl(q, k, v, mask, out, cu_seqlens, batch, heads, seq, head_dim, v_seq_pitch, scale, dtype,
-                              absmax_slots, slots_written, stream);
+                              absmax_slots, slots_written, nullptr, stream);
+}
+
+int ttmi_fused_attention_ahead(const void* q, const void* k, const void* v, const float* mask, void* out,
+                               const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
+                               int64_t v_seq_pitch, float scale, int dtype, const void* const* ahead, const int64_t* ahead_bytes,
+                               int64_t count, void* stream) {
+  TTMI_REQUIRE(count >= 0 && count <= TTMI_MAX_AHEAD && (count == 0 || (ahead && ahead_bytes)), "bad list of ranges to read ahead");
+  Ahead ranges{};
+  for (int64_t i = 0; i < count; ++i) {
+    TTMI_REQUIRE(ahead_bytes[i] >= 0 && (ahead_bytes[i] == 0 || ahead[i] != nullptr), "bad range to read ahead");
+    TTMI_REQUIRE((reinterpret_cast<uintptr_t>(ahead[i]) & 3) == 0 && (ahead_bytes[i] & 3) == 0, "a range to read ahead is whole words");
+    ranges.data[i] = static_cast<const char*>(ahead[i]);
+    ranges.bytes[i] = ahead_bytes[i];
+  }
+  return fused_attention_impl(q, k, v, mask, out, cu_seqlens, batch, heads, seq, head_dim, v_seq_pitch, scale, dtype, nullptr,
+                              nullptr, count > 0 ? &ranges : nullptr, stream);
 }
 
 }  // extern "C"

@@ -2,6 +2,7 @@
 // of 16-bit probabilities, and masks and scores far from zero.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -19,6 +20,41 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4), may_alias));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2), may_alias));
 
 constexpr int kD = 64;  // head dim
+
+// Weights that the following products read, brought from HBM into the last-level cache (256 MB, in front of the memory) by
+// workgroups of their own behind the `rows` grid rows that compute: attention over few sequences leaves most of the chip and nearly
+// all of the memory's bandwidth idle, and a product over few rows cannot hide the latency of HBM (128 x 2304 x 768 in fp32 halves 10.4
+// us with cold weights, 8.2 with weights in that cache).
+struct Ahead {
+  const char* data[TTMI_MAX_AHEAD];
+  int64_t bytes[TTMI_MAX_AHEAD];
+  int rows;
+};
+// One word of every 64 bytes, eight of them on the way per thread: 208 workgroups of 256 threads take 3.3 us for 9.4 MB, launch
+// included (whole lines 3.4, a word per 128 bytes 3.9).
+__device__ __forceinline__ void touch_ahead(const Ahead& ahead, int workgroup, int workgroups) {
+  constexpr int kLine = 64, kFlying = 8;
+  const int64_t first = ((int64_t)workgroup * blockDim.x + threadIdx.x) * kLine, stride = (int64_t)workgroups * blockDim.x * kLine;
+#pragma unroll 1
+  for (int r = 0; r < TTMI_MAX_AHEAD; ++r) {
+    const char* const data = ahead.data[r];
+    const int64_t bytes = ahead.bytes[r];
+#pragma unroll 1
+    for (int64_t at = first; at < bytes; at += kFlying * stride) {
+      uint32_t word[kFlying];
+#pragma unroll
+      for (int j = 0; j < kFlying; ++j) word[j] = *reinterpret_cast<const uint32_t*>(data + (at + j * stride < bytes ? at + j * stride : at));
+#pragma unroll
+      for (int j = 0; j < kFlying; ++j) asm volatile("" : : "v"(word[j]));
+    }
+  }
+}
+// Grid rows that `workgroups` in rows of `width` leave room for: a workgroup per idle CU, and half as many as CUs at least (reading
+// ahead is waiting for memory, it shares a CU well).  None where the attention itself fills the chip.
+inline unsigned ahead_rows(const Ahead* ahead, int64_t workgroups, int64_t width, int64_t cus) {
+  if (ahead == nullptr || workgroups > cus) return 0;
+  return (unsigned)ceil_div(std::max(cus - workgroups, cus / 2), width);
+}
 
 // D = A B + C over one 16-byte piece of both operands: eight K indices per half-wavefront in one instruction (16-bit types), or
 // four, one per instruction (fp32)

@@ -23,7 +23,7 @@ template <typename T, int NW>
 __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                   const T* __restrict__ v, const float* __restrict__ mask,
                                                                   T* __restrict__ out, int heads, int seq, int v_pitch, float scale_log2e, float inv_scale,
-                                                                  float* __restrict__ absmax) {
+                                                                  float* __restrict__ absmax, const Ahead ahead) {
   constexpr int KPC = 16 / (int)sizeof(T);   // elements per 16-byte piece
   constexpr int PIECES = kD / KPC / 2;       // pieces of a row per lane: 4 (16-bit), 8 (fp32)
   constexpr int VPIECES = 4 * (int)sizeof(T) / 2;  // pieces of V per lane and block: two halves of d, 32 keys
@@ -32,6 +32,10 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   __shared__ float stat[2][NW][kQ];  // m and l of every wavefront's share
   __shared__ float red[NW];
 
+  if ((int)blockIdx.y >= ahead.rows) {
+    touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int bh = blockIdx.y, b = bh / heads, head = bh - b * heads;
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     amax = group_max<kWave>(amax);
     if (lane == 0) red[wave] = amax;
     __syncthreads();
-    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), wgs = (int)(gridDim.x * gridDim.y);
+    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), wgs = (int)gridDim.x * ahead.rows;
     if (tid == 0) {
       float mx = red[0];
 #pragma unroll
@@ -248,13 +252,16 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 
 template <typename T>
 int launch(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-           int64_t seq, int64_t v_pitch, float scale, float* absmax, hipStream_t s) {
-  const dim3 grid((unsigned)ceil_div(seq, kQ), (unsigned)(batch * heads));
+           int64_t seq, int64_t v_pitch, float scale, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s) {
+  const unsigned width = (unsigned)ceil_div(seq, kQ), rows = (unsigned)(batch * heads);
+  const dim3 grid(width, rows + ahead_rows(ahead, (int64_t)width * rows, width, cus));
+  Ahead read_ahead = grid.y > rows ? *ahead : Ahead{};
+  read_ahead.rows = (int)rows;
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   // eight wavefronts where four would each have more than two blocks of keys
 #define TTMI_SPLIT_ATTENTION(NW)                                                                                              \
   hipLaunchKernelGGL((split_attention_kernel<T, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
-                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax)
+                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax, read_ahead)
   if (seq > 4 * 2 * kKeys) TTMI_SPLIT_ATTENTION(8);
   else TTMI_SPLIT_ATTENTION(4);
 #undef TTMI_SPLIT_ATTENTION
@@ -265,10 +272,10 @@ int launch(const void* q, const void* k, const void* v, const float* mask, void*
 
 // Arguments were checked by ttmi_fused_attention; absmax (fp32) needs seq / 32 * batch * heads workgroups to fit the slots.
 int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, hipStream_t s) {
-  if (dtype == TTMI_F16) return launch<f16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, s);
-  if (dtype == TTMI_BF16) return launch<bf16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, s);
-  return launch<float>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, absmax, s);
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s) {
+  if (dtype == TTMI_F16) return launch<f16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, cus, s);
+  if (dtype == TTMI_BF16) return launch<bf16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, cus, s);
+  return launch<float>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, absmax, ahead, cus, s);
 }
 
 }  // namespace ttmi

@@ -30,8 +30,9 @@ BERTLayer::BERTLayer(WeightMap* w, const std::string& p, int64_t n_heads) {
                                        Take(w, p + "output.LayerNorm.weight"), Take(w, p + "output.LayerNorm.bias")));
 }
 
-void BERTLayer::operator()(Tensor& hidden, Tensor& mask, Tensor* attention_out, Tensor* intermediate_out, Tensor* output) const {
-  (*attention_)(hidden, mask, attention_out);
+void BERTLayer::operator()(Tensor& hidden, Tensor& mask, Tensor* attention_out, Tensor* intermediate_out, Tensor* output,
+                           const std::vector<layers::WeightRange>& ahead) const {
+  (*attention_)(hidden, mask, attention_out, nullptr, false, ahead);
   (*intermediate_)(*attention_out, intermediate_out);
   (*output_)(*intermediate_out, *attention_out, output);
 }
@@ -63,7 +64,10 @@ struct BertModel::Impl {
     Tensor ext(nullptr);
     layers::PrepareBertMasks()(ids, mask, seq_type, position_ids, &ext);
     (*embedding_)(ids, *position_ids, *seq_type, hidden);
-    for (auto& layer : encoders_) layer(*hidden, ext, &att_out_, &intermediate_out_, hidden);
+    std::vector<layers::BertSubLayers> subs;
+    for (auto& layer : encoders_) subs.push_back({layer.attention_.get(), layer.intermediate_.get(), layer.output_.get()});
+    const auto ahead = layers::WeightsAhead(subs, *hidden);
+    for (size_t i = 0; i < encoders_.size(); ++i) encoders_[i](*hidden, ext, &att_out_, &intermediate_out_, hidden, ahead[i]);
   }
 
   std::unique_ptr<layers::BERTEmbedding> embedding_;

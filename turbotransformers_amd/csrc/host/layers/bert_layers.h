@@ -49,6 +49,7 @@ class BertIntermediate {
   void EnforceShapeAndType() const;
   // output = gelu(input * W + b)   (bert_intermediate.cpp:32-50)
   void operator()(const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
+  WeightRange weight() const { return packed_.Range(dense_weight_); }
 
  private:
   core::Tensor dense_weight_, dense_bias_;
@@ -65,6 +66,7 @@ class BertOutput {
   void EnforceShapeAndType() const;
   // output = LN(hidden_states * W + b + input_tensor)   (bert_output.cpp:29-55)
   void operator()(const core::Tensor& hidden_states, const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
+  WeightRange weight() const { return packed_.Range(dense_weight_); }
 
  private:
   core::Tensor dense_weight_, dense_bias_, layer_norm_weight_, layer_norm_bias_;

@@ -1,5 +1,6 @@
 #include "layers/multi_headed_attention.h"
 
+#include <algorithm>
 #include <cmath>
 
 #include "core/device_context.h"
@@ -66,7 +67,7 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
                                          Tensor* att_score, int64_t batch, int64_t seq, int64_t key_seq, const Tensor& k,
                                          const Tensor& v, const std::vector<int64_t>* seq_list, bool fused_core, int64_t v_pitch,
                                          bool post_layernorm, bool post_add_input, bool is_trans_weight,
-                                         const CacheGrowth* grow) const {
+                                         const CacheGrowth* grow, const std::vector<WeightRange>& ahead) const {
   const int dt = kernels::DeviceDType(query_tensor);
   const DLDeviceType dev = query_tensor.device_type();
   const int dev_id = query_tensor.device_id();
@@ -87,8 +88,12 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
     TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
     const int32_t* cu = nullptr;
     if (seq_list != nullptr) cu = DeviceContext::GetInstance().GetSeqPlan(*seq_list).cu_seqlens;
-    TT_DEVICE_CALL(ttmi_fused_attention(q_.raw(), k.raw(), v.raw(), mask, ctx_.mutable_raw(), cu, batch, heads, seq, d,
-                                        v_pitch, scaler, dt, Stream()));
+    const void* ahead_data[TTMI_MAX_AHEAD];
+    int64_t ahead_bytes[TTMI_MAX_AHEAD];
+    const size_t ranges = std::min(ahead.size(), (size_t)TTMI_MAX_AHEAD);
+    for (size_t i = 0; i < ranges; ++i) ahead_data[i] = ahead[i].data, ahead_bytes[i] = ahead[i].bytes;
+    TT_DEVICE_CALL(ttmi_fused_attention_ahead(q_.raw(), k.raw(), v.raw(), mask, ctx_.mutable_raw(), cu, batch, heads, seq, d,
+                                              v_pitch, scaler, dt, ahead_data, ahead_bytes, (int64_t)ranges, Stream()));
   } else {
   Tensor* score = att_score != nullptr ? att_score : &score_scratch_;
   // score is [B,h,F,T]: F = query positions, T = key positions (they differ for context attention
@@ -179,11 +184,11 @@ static void StoreInCache(std::unordered_map<std::string, Tensor*>& cache, const 
                   (size_t)src.numel() * src.element_size());
 }
 
-void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,
-                                      const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
-                                      Tensor* att_score, std::unordered_map<std::string, Tensor*> layer_cache,
-                                      bool pre_layernorm, bool post_layernorm, bool post_add_input,
-                                      bool is_trans_weight) const {
+void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,
+                                   const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
+                                   Tensor* att_score, std::unordered_map<std::string, Tensor*> layer_cache,
+                                   bool pre_layernorm, bool post_layernorm, bool post_add_input, bool is_trans_weight,
+                                   const std::vector<WeightRange>& ahead) const {
   std::lock_guard<std::mutex> g(mutex_);
   const bool is_self = attn_type == "self";
   TT_ENFORCE(is_self || attn_type == "context", "attn_type should be context or self.");
@@ -361,7 +366,7 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
   TT_ENFORCE_EQ(fused_core ? seq : growing ? v_cache.shape(2) : v_used->shape(2), key_seq, "keys and values differ in length");
 
   AttentionTail(query_tensor, attention_mask, output, att_score, batch, seq, key_seq, *k_used, *v_used, nullptr, fused_core, v_pitch,
-                post_layernorm, post_add_input, is_trans_weight, growing ? &growth : nullptr);
+                post_layernorm, post_add_input, is_trans_weight, growing ? &growth : nullptr, ahead);
   if (growing) {
     move_to_cache("self_keys", k_cache);
     move_to_cache("self_values", v_cache);
@@ -369,12 +374,29 @@ void MultiHeadedAttention::operator()(const Tensor& key_tensor, const Tensor& va
 }
 
 void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attention_mask, Tensor* output, Tensor* attn,
-                               bool is_trans_weight) const {
+                               bool is_trans_weight, const std::vector<WeightRange>& ahead) const {
   // bert_attention.cpp:29-47: self attention, post-LayerNorm, no extra residual
   std::unordered_map<std::string, Tensor*> dummy{};
-  MultiHeadedAttention::operator()(input_tensor, input_tensor, input_tensor, attention_mask, "self", output, attn, dummy,
-                                   false /* pre_layernorm */, true /* post_layernorm */, false /* post_add_input */,
-                                   is_trans_weight);
+  Forward(input_tensor, input_tensor, input_tensor, attention_mask, "self", output, attn, dummy, false /* pre_layernorm */,
+          true /* post_layernorm */, false /* post_add_input */, is_trans_weight, ahead);
+}
+
+std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<BertSubLayers>& layers, const Tensor& hidden) {
+  std::vector<std::vector<WeightRange>> ahead(layers.size());
+  if (hidden.numel() <= 32 * hidden.shape(-1)) return ahead;
+  int64_t bytes = 0;
+  for (size_t i = 0; i < layers.size(); ++i) {
+    for (const WeightRange& r : {layers[i].attention->dense_weight(), layers[i].intermediate->weight(), layers[i].output->weight()}) {
+      ahead[i].push_back(r);
+      bytes += r.bytes;
+    }
+    const WeightRange qkv = layers[i].attention->qkv_weight();
+    bytes += qkv.bytes;
+    if (i > 0) ahead[i - 1].push_back(qkv);
+  }
+  constexpr int64_t kStays = 200ll << 20;
+  if (bytes <= kStays) ahead.assign(layers.size(), {});
+  return ahead;
 }
 
 void MultiHeadedAttentionSmartBatch::operator()(const Tensor& key_tensor, const Tensor& value_tensor,

@@ -36,6 +36,14 @@ WeightRef PackedWeight::Get(const core::Tensor& w, bool is_trans_weight) const {
   return ref;
 }
 
+WeightRange PackedWeight::Range(const core::Tensor& w) const {
+  std::lock_guard<std::mutex> lock(mutex_);
+  if (source_ != w.raw() || packed_.is_null()) return {};
+  const int64_t bytes = w.numel() * (int64_t)w.element_size();
+  // (the halves of an fp32 weight lie behind its values, which are read for tiles outside their window only)
+  return {static_cast<const char*>(packed_.raw()) + (dtype_ == TTMI_F32_PACKED ? bytes : 0), bytes};
+}
+
 WeightRef PackedWeight::GetPair(const core::Tensor& w, const core::Tensor& v) const {
   TT_ENFORCE(w.n_dim() == 2 && v.n_dim() == 2 && w.shape(0) == v.shape(0) && w.shape(1) == v.shape(1), "a pair of weights has one shape");
   TT_ENFORCE(core::SameDataType(w.dtype(), v.dtype()), "a pair of weights has one element type");

@@ -21,12 +21,20 @@ struct WeightRef {
   int DTypeFor(int input) const { return input == TTMI_F32 && dtype == TTMI_F32_PACKED ? TTMI_F32_PACKED : input; }
 };
 
+// The bytes of a weight that a product reads.
+struct WeightRange {
+  const void* data = nullptr;
+  int64_t bytes = 0;
+};
+
 class PackedWeight {
  public:
   // W as [N, K]; `w` is [K, N] when !is_trans_weight, [N, K] (used as it is) otherwise.
   WeightRef Get(const core::Tensor& w, bool is_trans_weight) const;
   // [w; v] as [2 N, K] for two weights [K, N] that are applied to the same rows.
   WeightRef GetPair(const core::Tensor& w, const core::Tensor& v) const;
+  // What products of `w` [K, N] read; empty before the first Get.
+  WeightRange Range(const core::Tensor& w) const;
   // Output width N of `w` under the given layout.
   static int64_t OutDim(const core::Tensor& w, bool is_trans_weight) { return is_trans_weight ? w.shape(0) : w.shape(1); }
   static int64_t InDim(const core::Tensor& w, bool is_trans_weight) { return is_trans_weight ? w.shape(1) : w.shape(0); }

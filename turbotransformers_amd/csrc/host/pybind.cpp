@@ -125,7 +125,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
         return new layers::BertAttention(std::move(qkv_w), std::move(qkv_b), std::move(dense_w), std::move(dense_b),
                                          std::move(ln_w), std::move(ln_b), heads);
       }))
-      .def("__call__", &layers::BertAttention::operator(), py::arg("input_tensor"), py::arg("attention_mask"),
+      .def("__call__", py::overload_cast<const Tensor&, const Tensor&, Tensor*, Tensor*, bool>(&layers::BertAttention::operator(), py::const_), py::arg("input_tensor"), py::arg("attention_mask"),
            py::arg("output"), py::arg("attn") = nullptr, py::arg("is_trans_weight") = false);
 
   py::class_<layers::MultiHeadedAttention>(m, "MultiHeadedAttention")
@@ -272,26 +272,22 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
   // three temporaries and a stream query each: at batch 1 x seq 128 the interpreter, not the GPU, set the pace).
   // `layer_list` is a sequence of (BertAttention, BertIntermediate, BertOutput).  No counterpart in the reference.
   m.def("run_bert_layers", [](const py::sequence& layer_list, const Tensor& hidden, const Tensor& mask, Tensor* out) {
-    struct Sub {
-      const layers::BertAttention* attention;
-      const layers::BertIntermediate* intermediate;
-      const layers::BertOutput* output;
-    };
-    std::vector<Sub> subs;
+    std::vector<layers::BertSubLayers> subs;
     subs.reserve(py::len(layer_list));
     for (const py::handle& item : layer_list) {
       const py::tuple t = py::cast<py::tuple>(item);
       TT_ENFORCE_EQ(py::len(t), (size_t)3, "each layer is (attention, intermediate, output)");
-      subs.push_back(Sub{&py::cast<const layers::BertAttention&>(t[0]), &py::cast<const layers::BertIntermediate&>(t[1]),
+      subs.push_back({&py::cast<const layers::BertAttention&>(t[0]), &py::cast<const layers::BertIntermediate&>(t[1]),
                          &py::cast<const layers::BertOutput&>(t[2])});
     }
     TT_ENFORCE(!subs.empty() && out != nullptr, "run_bert_layers needs layers and an output tensor");
     Tensor attention_out(nullptr), intermediate_out(nullptr), even(nullptr), odd(nullptr);
     const Tensor* current = &hidden;
+    const auto ahead = layers::WeightsAhead(subs, hidden);
     for (size_t i = 0; i < subs.size(); ++i) {
       // the last layer writes the caller's tensor; before it two buffers alternate (a layer never writes what it reads)
       Tensor* target = (i + 1 == subs.size()) ? out : (i % 2 == 0 ? &even : &odd);
-      (*subs[i].attention)(*current, mask, &attention_out, nullptr, false);
+      (*subs[i].attention)(*current, mask, &attention_out, nullptr, false, ahead[i]);
       (*subs[i].intermediate)(attention_out, &intermediate_out);
       (*subs[i].output)(intermediate_out, attention_out, target);
       current = target;
