@@ -345,6 +345,21 @@ TTMI_API int ttmi_fused_attention_ahead(const void* q, const void* k, const void
                                         int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype,
                                         const void* const* ahead, const int64_t* ahead_bytes, int64_t count, void* stream);
 
+/* ttmi_fused_attention of a dense fp16 / bf16 batch with V transposed, and behind it the output projection, as one launch for few
+ * rows: partial[head] = context of that head, rounded to the type, times w's 64 columns of the head.  w is [N,K], N = K = h*64;
+ * partial fp32 [h, B*S, h*64], whose sum over the heads is the projection (ttmi_add_slices_layer_norm takes it).  The context
+ * itself is not written.  ahead, ahead_bytes, count: as in ttmi_fused_attention_ahead. */
+TTMI_API int ttmi_attention_projection(const void* q, const void* k, const void* v, const float* mask, const void* w,
+                                       float* partial, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
+                                       int64_t v_seq_pitch, float scale, int dtype, const void* const* ahead,
+                                       const int64_t* ahead_bytes, int64_t count, void* stream);
+/* out[m,n] = LN(sum of `count` fp32 slices [m,n] + bias + residual): the second half of ttmi_gemm_bias_layer_norm, whose rules hold
+ * for residual / residual_f32 / out_f32.  n <= 4096, a multiple of 4; slices and fp32 rows 16-byte aligned, rows of `dtype` aligned
+ * to four elements. */
+TTMI_API int ttmi_add_slices_layer_norm(const float* slices, int64_t count, void* out, const void* residual,
+                                        const float* residual_f32, const void* bias, const void* gamma, const void* beta,
+                                        float* out_f32, int64_t m, int64_t n, float eps, int dtype, void* stream);
+
 /* Attention that returns its probabilities, for head_dim 64: P = softmax(scale * Q K^T + mask), out = P V with
  * K = [k_past | k] and V = [v_past | v] along the sequence.  q is [B,h,F,64]; k_past, v_past [B,h,past,64] (NULL with
  * past = 0), k, v [B,h,keys-past,64]; `mask` is an additive fp32 [B,keys], or [B,F,keys] with mask_per_query, or NULL;

@@ -1197,6 +1197,54 @@ def test_attention_that_reads_ahead(ttmi, dt, B, S, v_transposed, packed):
     assert run([4, 2])[0] != 0 and run([-4])[0] != 0
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("B,h,S", [(1, 1, 1), (1, 12, 10), (3, 3, 32), (1, 5, 33), (2, 12, 60), (1, 16, 300)])
+def test_attention_with_its_projection(ttmi, dt, B, h, S):
+    """Attention and the output projection in one launch, a slice per head, against fp64; one and several blocks of queries and keys, a
+    last group of columns with idle wavefronts, four and eight wavefronts.  The slices' sum through the LayerNorm behind them, with
+    either residual, against ttmi_gemm_bias_layer_norm; more slices than one round of loads.  Ranges read ahead change nothing."""
+    import ctypes
+    rng = np.random.default_rng(B * S + h)
+    d, H, M = 64, 64 * h, B * S
+    Q, K, V = (rng.standard_normal((B, h, S, d), np.float32) for _ in range(3))
+    W = (rng.standard_normal((H, H)) / np.sqrt(H)).astype(np.float32)
+    mask = np.where(rng.random((B, S)) < 0.3, -1e4, 0).astype(np.float32)
+    mask[:, 0] = 0
+    dV, pitch = _v_operand(V, dt, True)
+    dQ, dK, dW, dmask = dev(Q, dt), dev(K, dt), dev(W, dt), dev(mask)
+    buffer = torch.full((h * M + 8, H), 9.0, device="cuda")
+    packed = buffer[:h * M].view(h, M, H)
+    words = torch.ones(1000, dtype=torch.int32, device="cuda")
+    for ranges in (0, 1):
+        ok(ttmi.ttmi_attention_projection(ptr(dQ), ptr(dK), ptr(dV), ptr(dmask), ptr(dW), ptr(packed), B, h, S, d, pitch, 0.125, TTMI_DTYPES[dt],
+                                          (ctypes.c_void_p * 1)(words.data_ptr()), (ctypes.c_int64 * 1)(4000), ranges, stream()))
+        first = packed.clone() if ranges == 0 else first
+        assert torch.equal(first, packed) and bool((buffer[h * M:] == 9.0).all())
+    q, k, v, w = (rounded(x, dt).astype(np.float64) for x in (Q, K, V, W))
+    p = np.exp(q @ k.transpose(0, 1, 3, 2) * 0.125 + mask[:, None, None, :])
+    ctx = ((p / p.sum(-1, keepdims=True)) @ v).transpose(0, 2, 1, 3).reshape(M, h, d)
+    want = np.stack([ctx[:, i] @ w[:, i * d:(i + 1) * d].T for i in range(h)])
+    # (probabilities and context are rounded to the type, both sums of products of size 1 / sqrt(H))
+    assert max_abs(host(packed), want) <= GEMM_TOL[dt] * 2
+    # the LayerNorm over the slices' sum: the same as over the rounded context's product, but for the order of the sums
+    R, bias, gamma, beta = (rng.standard_normal(n).astype(np.float32) for n in ((M, H), H, H, H))
+    dR, db, dg, dbeta = dev(R, dt), dev(bias, dt), dev(gamma, dt), dev(beta, dt)
+    r32 = dev(R)
+    for residual, residual32 in ((dR, None), (None, r32)):
+        out, out2 = torch.empty_like(dR), torch.empty_like(dR)
+        o32, o322 = torch.empty_like(r32), torch.empty_like(r32)
+        pp = lambda t: None if t is None else ptr(t)
+        ok(ttmi.ttmi_add_slices_layer_norm(ptr(packed), h, ptr(out), pp(residual), pp(residual32), ptr(db), ptr(dg), ptr(dbeta),
+                                           ptr(o32) if residual32 is not None else None, M, H, ctypes.c_float(1e-12), TTMI_DTYPES[dt], stream()))
+        x = want.sum(0) + rounded(bias, dt) + (R if residual is None else rounded(R, dt))
+        ref = (x - x.mean(1, keepdims=True)) / x.std(1, keepdims=True) * rounded(gamma, dt) + rounded(beta, dt)
+        assert max_abs(host(out), ref) <= GEMM_TOL[dt] * 6
+        if residual32 is not None:
+            assert max_abs(host(o32), ref) <= GEMM_TOL[dt] * 6
+    assert ttmi.ttmi_add_slices_layer_norm(ptr(packed), 0, ptr(out), None, ptr(r32), ptr(db), ptr(dg), ptr(dbeta), ptr(o32), M, H,
+                                           ctypes.c_float(1e-12), TTMI_DTYPES[dt], stream()) != 0
+
+
 @pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("M,h,steps", [(1, 1, 1), (16, 1, 16), (17, 12, 12), (33, 3, 17), (8, 12, 24), (31, 4, 32), (40, 2, 33)])
 def test_layer_norm_in_front_of_a_few_row_product(ttmi, oracle, dt, M, h, steps):

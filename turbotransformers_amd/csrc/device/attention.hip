@@ -154,11 +154,9 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
                                                                  T* __restrict__ out, const int32_t* __restrict__ cu,
                                                                  int heads, int seq, int v_pitch, float scale_log2e,
                                                                  float inv_scale, const Ahead ahead) {
-  if constexpr (!PACKED) {
-    if ((int)blockIdx.y >= ahead.rows) {
-      touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
-      return;
-    }
+  if ((int)blockIdx.y >= ahead.rows) {
+    touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
+    return;
   }
   // one LDS block: [2 x K tile | 2 x V^T tile | 2 x mask]; the front is reused for the output tile
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
@@ -179,7 +177,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   const int major = (PACKED ? blockIdx.x : blockIdx.y) / heads, head = (PACKED ? blockIdx.x : blockIdx.y) - major * heads;
   const int block = PACKED ? major : blockIdx.x;
   int b = PACKED ? blockIdx.y : major;
-  if (PACKED && seq > kOrderMinLength && gridDim.x * gridDim.y > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, gridDim.y, b, seq));
+  if (PACKED && seq > kOrderMinLength && gridDim.x * ahead.rows > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, ahead.rows, b, seq));
   const int bh = b * heads + head;
   const int q0 = block * kBQ + wave * 32;
 
@@ -327,7 +325,7 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
 
 // attention_split.hip: the keys of a head split over the wavefronts of a workgroup
 int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s);
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, hipStream_t s);
 
 // absmax / slots_written: see ttmi_fused_attention_absmax; ahead: see ttmi_fused_attention_ahead; null for the plain entry point
 static int fused_attention_impl(const void* q, const void* k, const void* v, const float* mask, void* out,
@@ -349,12 +347,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   // 64 x 512: 77 against 81).  Four win where the sequence fits them (up to 128 tokens), where two blocks of 256
   // queries stand against three of 128 (257..384 tokens; 64 x 300: 44 against 49 us), and where even their workgroups
   // are fewer than the compute units (4 x 512 tokens: 12.4 against 13.7 us).
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
+  const int cus = compute_units();
   const bool fits_four = seq <= 128 || 8 * ceil_div(seq, 256) >= 5 * ceil_div(seq, 128);
   int nw = (fits_four || ceil_div(seq, 128) * batch * heads < (int64_t)cus) ? 4 : 8;
   // fp32 in halves: splitting K and V on their way into LDS is half of a short sequence's work, and eight wavefronts share it even
@@ -379,7 +372,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   if (split && cu_seqlens == nullptr && v_seq_pitch > 0) {
     const bool leave_maxima = absmax != nullptr && dtype == TTMI_F32 && split_wgs <= TTMI_ABSMAX_SLOTS;
     const int rc = split_attention(q, k, v, mask, out, batch, heads, seq, v_seq_pitch, scale, dtype,
-                                   leave_maxima ? absmax : nullptr, ahead, cus, (hipStream_t)stream);
+                                   leave_maxima ? absmax : nullptr, ahead, (hipStream_t)stream);
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;
   }
@@ -391,8 +384,8 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
   Ahead read_ahead{};
-  if (dtype != TTMI_F32 && cu_seqlens == nullptr) {
-    const unsigned more = ahead_rows(ahead, (int64_t)grid.x * grid.y, grid.x, cus);
+  if (dtype != TTMI_F32) {
+    const unsigned more = ahead_rows(ahead, (int64_t)grid.x * grid.y, grid.x, (int64_t)cus * (16 / nw));
     if (more > 0) read_ahead = *ahead;
     read_ahead.rows = (int)grid.y;
     grid.y += more;
@@ -455,16 +448,11 @@ int ttmi_fused_attention_ahead(const void* q, const void* k, const void* v, cons
                                const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq, int64_t head_dim,
                                int64_t v_seq_pitch, float scale, int dtype, const void* const* ahead, const int64_t* ahead_bytes,
                                int64_t count, void* stream) {
-  TTMI_REQUIRE(count >= 0 && count <= TTMI_MAX_AHEAD && (count == 0 || (ahead && ahead_bytes)), "bad list of ranges to read ahead");
   Ahead ranges{};
-  for (int64_t i = 0; i < count; ++i) {
-    TTMI_REQUIRE(ahead_bytes[i] >= 0 && (ahead_bytes[i] == 0 || ahead[i] != nullptr), "bad range to read ahead");
-    TTMI_REQUIRE((reinterpret_cast<uintptr_t>(ahead[i]) & 3) == 0 && (ahead_bytes[i] & 3) == 0, "a range to read ahead is whole words");
-    ranges.data[i] = static_cast<const char*>(ahead[i]);
-    ranges.bytes[i] = ahead_bytes[i];
-  }
+  const int rc = ahead_ranges(ahead, ahead_bytes, count, &ranges);
+  if (rc != 0) return rc;
   return fused_attention_impl(q, k, v, mask, out, cu_seqlens, batch, heads, seq, head_dim, v_seq_pitch, scale, dtype, nullptr,
-                              nullptr, count > 0 ? &ranges : nullptr, stream);
+                              nullptr, &ranges, stream);
 }
 
 }  // extern "C"

@@ -28,8 +28,19 @@ constexpr int kD = 64;  // head dim
 struct Ahead {
   const char* data[TTMI_MAX_AHEAD];
   int64_t bytes[TTMI_MAX_AHEAD];
-  int rows;
+  int ranges, rows;
 };
+inline int ahead_ranges(const void* const* data, const int64_t* bytes, int64_t count, Ahead* out) {
+  TTMI_REQUIRE(count >= 0 && count <= TTMI_MAX_AHEAD && (count == 0 || (data && bytes)), "bad list of ranges to read ahead");
+  for (int64_t i = 0; i < count; ++i) {
+    TTMI_REQUIRE(bytes[i] >= 0 && (bytes[i] == 0 || data[i] != nullptr), "bad range to read ahead");
+    TTMI_REQUIRE((reinterpret_cast<uintptr_t>(data[i]) & 3) == 0 && (bytes[i] & 3) == 0, "a range to read ahead is whole words");
+    out->data[i] = static_cast<const char*>(data[i]);
+    out->bytes[i] = bytes[i];
+  }
+  out->ranges = (int)count;
+  return 0;
+}
 // One word of every 64 bytes, eight of them on the way per thread: 208 workgroups of 256 threads take 3.3 us for 9.4 MB, launch
 // included (whole lines 3.4, a word per 128 bytes 3.9).
 __device__ __forceinline__ void touch_ahead(const Ahead& ahead, int workgroup, int workgroups) {
@@ -49,10 +60,12 @@ __device__ __forceinline__ void touch_ahead(const Ahead& ahead, int workgroup, i
     }
   }
 }
-// Grid rows that `workgroups` in rows of `width` leave room for: a workgroup per idle CU, and half as many as CUs at least (reading
-// ahead is waiting for memory, it shares a CU well).  None where the attention itself fills the chip.
-inline unsigned ahead_rows(const Ahead* ahead, int64_t workgroups, int64_t width, int64_t cus) {
-  if (ahead == nullptr || workgroups > cus) return 0;
+// Grid rows for reading ahead behind `workgroups` of them in rows of `width`, of which `slots` fit the chip at a time: a workgroup
+// per idle CU, and half as many as CUs at least (reading ahead is waiting for memory, it shares a CU well).  None where the
+// attention takes several rounds.
+inline unsigned ahead_rows(const Ahead* ahead, int64_t workgroups, int64_t width, int64_t slots) {
+  const int64_t cus = compute_units();
+  if (ahead == nullptr || ahead->ranges == 0 || workgroups > slots) return 0;
   return (unsigned)ceil_div(std::max(cus - workgroups, cus / 2), width);
 }
 

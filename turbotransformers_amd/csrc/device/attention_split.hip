@@ -11,6 +11,12 @@
 // with the weights 2^(m_w - max m).
 // One sequence, 12 heads, us per launch before / after: fp16 387 tokens 10.6 / 7.0, fp32 128 tokens 12.7 / 6.3 (1.5 of each
 // is the launch, 1 the first loads; fp32 then runs 64 matrix instructions of 64 cycles in a chain per block of keys).
+//
+// With the output projection (PROJECT): up to some dozens of rows that product is a launch of its own for a few microseconds of
+// waiting.  A workgroup here has the context of 32 queries of one head in its hands, and its wavefronts multiply it by the head's 64
+// columns of w, whose loads were sent in front of the attention: an fp32 slice per head, added up by the kernel that
+// normalises.  128 columns a workgroup (NW = 4; blockIdx.z), each computing the attention again: 72 workgroups for 10 rows of 12 heads
+// are 5.2 us, the two launches they replace 4.3 and 4.0.
 #include "attention_common.h"
 
 namespace ttmi {
@@ -18,12 +24,19 @@ namespace {
 
 constexpr int kQ = 32, kKeys = 32;  // queries per workgroup, keys per block
 
+// The output projection behind the core (PROJECT): the rows of w (and columns of the product) that the workgroups of one blockIdx.z take.
+template <typename T>
+struct Projection {
+  const T* w;        // [n, n], n = heads * 64
+  float* partial;    // [heads, batch * seq, n]
+};
+
 // V is [B,h,d,v_pitch]
-template <typename T, int NW>
+template <typename T, int NW, bool PROJECT>
 __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                   const T* __restrict__ v, const float* __restrict__ mask,
                                                                   T* __restrict__ out, int heads, int seq, int v_pitch, float scale_log2e, float inv_scale,
-                                                                  float* __restrict__ absmax, const Ahead ahead) {
+                                                                  float* __restrict__ absmax, const Ahead ahead, const Projection<T> proj) {
   constexpr int KPC = 16 / (int)sizeof(T);   // elements per 16-byte piece
   constexpr int PIECES = kD / KPC / 2;       // pieces of a row per lane: 4 (16-bit), 8 (fp32)
   constexpr int VPIECES = 4 * (int)sizeof(T) / 2;  // pieces of V per lane and block: two halves of d, 32 keys
@@ -31,9 +44,11 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   __shared__ __align__(16) float part[NW][kQ][PITCH];
   __shared__ float stat[2][NW][kQ];  // m and l of every wavefront's share
   __shared__ float red[NW];
+  __shared__ __align__(16) T ctx[PROJECT ? kQ : 1][kD + 8];
 
   if ((int)blockIdx.y >= ahead.rows) {
-    touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
+    const int width = (int)(gridDim.x * gridDim.z);
+    touch_ahead(ahead, (int)(blockIdx.y - ahead.rows) * width + (int)(blockIdx.z * gridDim.x + blockIdx.x), (int)(gridDim.y - ahead.rows) * width);
     return;
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -44,6 +59,15 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   const T* kb = k + (int64_t)bh * seq * kD;
   const T* vb = v + (int64_t)bh * kD * v_pitch;
   const float* mb = mask != nullptr ? mask + (int64_t)b * seq : nullptr;
+
+  // the wavefront's 32 columns of the projection; its weights arrive during the attention
+  const int hidden = heads * kD, col0 = PROJECT ? (blockIdx.z * NW + wave) * 32 : 0;
+  u32x4 wf[PROJECT ? 4 : 1];
+  if constexpr (PROJECT) {
+    const T* row = proj.w + (int64_t)min(col0 + lrow, hidden - 1) * hidden + head * kD + lhalf * 8;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) wf[kk] = *reinterpret_cast<const u32x4*>(row + kk * 16);
+  }
 
   u32x4 qf[PIECES];
   {
@@ -216,6 +240,26 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     }
   }
   const float inv = 1.0f / l;
+  if constexpr (PROJECT) {
+    // the head's context, rounded as it is where it is stored, times its 64 columns of w: lane = query, four columns a register quad
+    Vec<T, EPT> r;
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) r.v[e] = from_float<T>(o[e] * inv);
+    store_vec<T, EPT>(&ctx[qi][d0], r);
+    __syncthreads();
+    floatx16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) acc = mma32<T>(wf[kk], *reinterpret_cast<const u32x4*>(&ctx[lrow][kk * 16 + lhalf * 8]), acc);
+    if (q0 + lrow < seq && col0 < hidden) {
+      const int64_t tokens = (int64_t)(ahead.rows / heads) * seq;  // (ahead.rows: batch * heads)
+      float* dst = proj.partial + (head * tokens + (int64_t)b * seq + q0 + lrow) * hidden + col0 + 4 * lhalf;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) *reinterpret_cast<floatx4*>(dst + 8 * g) = floatx4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    }
+    return;
+  }
   float amax = 0.f;
   if (q0 + qi < seq) {
     T* dst = out + ((int64_t)b * seq + q0 + qi) * (heads * kD) + head * kD + d0;
@@ -252,30 +296,74 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 
 template <typename T>
 int launch(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-           int64_t seq, int64_t v_pitch, float scale, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s) {
+           int64_t seq, int64_t v_pitch, float scale, float* absmax, const Ahead* ahead, hipStream_t s) {
   const unsigned width = (unsigned)ceil_div(seq, kQ), rows = (unsigned)(batch * heads);
-  const dim3 grid(width, rows + ahead_rows(ahead, (int64_t)width * rows, width, cus));
+  const dim3 grid(width, rows + ahead_rows(ahead, (int64_t)width * rows, width, 2 * compute_units()));
   Ahead read_ahead = grid.y > rows ? *ahead : Ahead{};
   read_ahead.rows = (int)rows;
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   // eight wavefronts where four would each have more than two blocks of keys
 #define TTMI_SPLIT_ATTENTION(NW)                                                                                              \
-  hipLaunchKernelGGL((split_attention_kernel<T, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
-                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax, read_ahead)
+  hipLaunchKernelGGL((split_attention_kernel<T, NW, false>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
+                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax, read_ahead, Projection<T>{})
   if (seq > 4 * 2 * kKeys) TTMI_SPLIT_ATTENTION(8);
   else TTMI_SPLIT_ATTENTION(4);
 #undef TTMI_SPLIT_ATTENTION
   return launch_status("split_attention_kernel");
 }
 
+template <typename T>
+int launch_projection(const void* q, const void* k, const void* v, const float* mask, const void* w, float* partial, int64_t batch,
+                      int64_t heads, int64_t seq, int64_t v_pitch, float scale, const Ahead& ahead, hipStream_t s) {
+  const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
+  auto launch = [&](auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    const unsigned width = (unsigned)ceil_div(seq, kQ), rows = (unsigned)(batch * heads), groups = (unsigned)ceil_div(heads * kD, NW * 32);
+    Ahead read_ahead = ahead;
+    read_ahead.rows = (int)rows;
+    const unsigned more = ahead_rows(&ahead, (int64_t)width * groups * rows, (int64_t)width * groups, 2 * compute_units());
+    hipLaunchKernelGGL((split_attention_kernel<T, NW, true>), dim3(width, rows + more, groups), dim3(NW * 64), 0, s, (const T*)q, (const T*)k,
+                       (const T*)v, mask, (T*)nullptr, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, (float*)nullptr, read_ahead,
+                       Projection<T>{(const T*)w, partial});
+  };
+  if (seq > 4 * 2 * kKeys) launch(std::integral_constant<int, 8>{});
+  else launch(std::integral_constant<int, 4>{});
+  return launch_status("attention_projection_kernel");
+}
+
 }  // namespace
 
 // Arguments were checked by ttmi_fused_attention; absmax (fp32) needs seq / 32 * batch * heads workgroups to fit the slots.
 int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
-                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, int64_t cus, hipStream_t s) {
-  if (dtype == TTMI_F16) return launch<f16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, cus, s);
-  if (dtype == TTMI_BF16) return launch<bf16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, cus, s);
-  return launch<float>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, absmax, ahead, cus, s);
+                    int64_t seq, int64_t v_pitch, float scale, int dtype, float* absmax, const Ahead* ahead, hipStream_t s) {
+  if (dtype == TTMI_F16) return launch<f16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, s);
+  if (dtype == TTMI_BF16) return launch<bf16>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, nullptr, ahead, s);
+  return launch<float>(q, k, v, mask, out, batch, heads, seq, v_pitch, scale, absmax, ahead, s);
 }
 
 }  // namespace ttmi
+
+using namespace ttmi;
+
+extern "C" {
+
+int ttmi_attention_projection(const void* q, const void* k, const void* v, const float* mask, const void* w, float* partial,
+                              int64_t batch, int64_t heads, int64_t seq, int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype,
+                              const void* const* ahead, const int64_t* ahead_bytes, int64_t count, void* stream) {
+  TTMI_REQUIRE(q && k && v && w && partial, "null tensor");
+  TTMI_REQUIRE(head_dim == kD, "the attention projection is built for head_dim 64");
+  TTMI_REQUIRE(dtype == TTMI_F16 || dtype == TTMI_BF16, "the attention projection is built for fp16 / bf16");
+  TTMI_REQUIRE(batch > 0 && heads > 0 && seq > 0 && batch * heads < 65536 && heads < 65536 && seq < (1 << 24), "bad shape");
+  TTMI_REQUIRE(v_seq_pitch >= seq && v_seq_pitch % 8 == 0 && v_seq_pitch < (1 << 24), "v_seq_pitch must be a multiple of 8 that is >= seq");
+  TTMI_REQUIRE(scale > 0.f, "scale must be positive");
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
+                         reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(partial);
+  TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
+  Ahead ranges{};
+  const int rc = ahead_ranges(ahead, ahead_bytes, count, &ranges);
+  if (rc != 0) return rc;
+  if (dtype == TTMI_F16) return launch_projection<f16>(q, k, v, mask, w, partial, batch, heads, seq, v_seq_pitch, scale, ranges, (hipStream_t)stream);
+  return launch_projection<bf16>(q, k, v, mask, w, partial, batch, heads, seq, v_seq_pitch, scale, ranges, (hipStream_t)stream);
+}
+
+}  // extern "C"

@@ -19,6 +19,10 @@ template <typename T>
 int gemm_norm_fused_typed(const GemmArgs& g, const void* gamma, const void* beta, float eps, void* c, int64_t ldc, int epilogue,
                           const ttmi_epilogue_args* args, hipStream_t s);
 template <typename T>
+int add_slices_layer_norm_typed(const float* slices, int64_t count, void* out, const void* residual, const float* residual_f32,
+                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n, float eps,
+                                hipStream_t s);
+template <typename T>
 int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* out, const void* residual, const float* residual_f32,
                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
                                int64_t k, float eps, int dtype, hipStream_t s);
@@ -219,6 +223,19 @@ int ttmi_gemm_bias_layer_norm(const void* a, const void* w, void* out, const voi
                               const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
                               int64_t k, float eps, int dtype, void* stream) {
   return gemm_bias_layer_norm_impl(a, w, out, residual, residual_f32, bias, gamma, beta, out_f32, m, n, k, eps, dtype, stream);
+}
+
+int ttmi_add_slices_layer_norm(const float* slices, int64_t count, void* out, const void* residual, const float* residual_f32,
+                               const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n,
+                               float eps, int dtype, void* stream) {
+  TTMI_REQUIRE(slices && out && bias && gamma && beta, "null tensor");
+  TTMI_REQUIRE((residual_f32 != nullptr) == (out_f32 != nullptr), "residual_f32 and out_f32 go together");
+  TTMI_REQUIRE(residual != nullptr || residual_f32 != nullptr, "a residual is required");
+  TTMI_REQUIRE(count > 0 && count < (1 << 16) && m >= 0 && m < (1ll << 31) && n >= 0 && n <= 4096 && n % 4 == 0, "dimension out of range");
+  if (m == 0 || n == 0) return 0;
+  TTMI_DISPATCH_FLOAT(dtype, T, return add_slices_layer_norm_typed<T>(slices, count, out, residual, residual_f32, bias, gamma, beta, out_f32,
+                                                                      m, n, eps, (hipStream_t)stream));
+  return 0;
 }
 
 int ttmi_gemm_bias_layer_norm_static(const void* a, const void* w, void* out, const void* residual,

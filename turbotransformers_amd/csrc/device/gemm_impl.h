@@ -1001,7 +1001,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
 // registers (ITERS float4 per thread), and writes LN(x) -- one launch and one pass over the row
 // instead of a reduce kernel, a 16-bit round trip and a LayerNorm kernel.  Needs n % 4 == 0,
 // n <= 1024 * ITERS and rows of every operand aligned to four elements.   mean / variance as in layer_norm.cpp:144-163 of the reference.
-template <typename T, int ITERS>
+template <typename T, int ITERS, int AT_ONCE>
 __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const float* __restrict__ ws, int splits, int m, int n,
                                                                       const T* __restrict__ bias, const T* residual,
                                                                       const float* residual32, const T* __restrict__ gamma,
@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const flo
   float x[ITERS][4];
   float sum = 0.f, sumsq = 0.f;
   // A row is a few KB: the kernel is a chain of waits, so everything the row needs is requested before the first use
-  // (gamma and beta in front of the reduction, the slices four at a time).
+  // (gamma and beta in front of the reduction, the slices AT_ONCE at a time).
   Vec<T, 4> gm[ITERS], bt[ITERS];
 #pragma unroll
   for (int it = 0; it < ITERS; ++it) {
@@ -1029,13 +1029,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const flo
       bt[it] = load_vec<T, 4>(beta + col);
       const float* p = ws + (int64_t)row * n + col;
       int sidx = 0;
-      for (; sidx + 4 <= splits; sidx += 4) {
-        float4 v[4];
+      auto add = [&](auto count) __attribute__((always_inline)) {
+        constexpr int N = decltype(count)::value;
+        float4 v[N];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const float4*>(p + (sidx + u) * mn);
+        for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const float4*>(p + (sidx + u) * mn);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) x[it][0] += v[u].x, x[it][1] += v[u].y, x[it][2] += v[u].z, x[it][3] += v[u].w;
-      }
+        for (int u = 0; u < N; ++u) x[it][0] += v[u].x, x[it][1] += v[u].y, x[it][2] += v[u].z, x[it][3] += v[u].w;
+        sidx += N;
+      };
+      if constexpr (AT_ONCE > 4)
+        while (sidx + AT_ONCE <= splits) add(std::integral_constant<int, AT_ONCE>{});
+      while (sidx + 4 <= splits) add(std::integral_constant<int, 4>{});
       for (; sidx < splits; ++sidx) {
         const float4 v = *reinterpret_cast<const float4*>(p + sidx * mn);
         x[it][0] += v.x; x[it][1] += v.y; x[it][2] += v.z; x[it][3] += v.w;
@@ -1397,16 +1402,6 @@ inline int launch_config(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-
-inline int compute_units() {
-  static int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return cus;
-}
 
 template <typename T, int BM, int BN, int WM, int WN, typename Epi, int NS = 2>
 inline int launch_fast(GemmArgs g, const Epi& epi, int batch, hipStream_t s) {

@@ -140,6 +140,36 @@ inline bool fp32_product_expected(int64_t m, int64_t n, int64_t k) {
   return (k >= 512 && tiles(64) <= cus / 4) || (k >= 1024 && tiles(128) <= cus / 2) || (k >= 2048 && tiles(256) <= cus / 2);
 }
 
+template <typename T>
+void launch_reduce_layer_norm(const float* ws, int slices, int64_t m, int64_t n, const void* bias, const void* residual,
+                              const float* residual_f32, const void* gamma, const void* beta, void* out, float* out_f32, float eps,
+                              hipStream_t s) {
+  auto launch = [&](auto iters, auto at_once) {
+    hipLaunchKernelGGL((splitk_reduce_layer_norm_kernel<T, decltype(iters)::value, decltype(at_once)::value>), dim3((unsigned)m), dim3(256), 0, s, ws, slices,
+                       (int)m, (int)n, (const T*)bias, (const T*)residual, residual_f32, (const T*)gamma, (const T*)beta, (T*)out,
+                       out_f32, eps);
+  };
+  // (a forward of 1 x 10 fp16 tokens, whose attention leaves a slice per head: 306 us with four slices on the way at a time, 297 with
+  // twelve; 20 x 100 tokens, two slices of 2000 rows, are 1 % slower on the kernel that has registers for twelve)
+  constexpr std::integral_constant<int, 4> four{};
+  if (n <= 1024 && slices >= 12) launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 12>{});
+  else if (n <= 1024) launch(std::integral_constant<int, 1>{}, four);
+  else if (n <= 2048) launch(std::integral_constant<int, 2>{}, four);
+  else launch(std::integral_constant<int, 4>{}, four);
+}
+
+// The slices of a product + AddBiasLayerNorm; the rows were checked by the caller.
+template <typename T>
+int add_slices_layer_norm_typed(const float* slices, int64_t count, void* out, const void* residual, const float* residual_f32,
+                                const void* bias, const void* gamma, const void* beta, float* out_f32, int64_t m, int64_t n, float eps,
+                                hipStream_t s) {
+  const uintptr_t rows = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(gamma) |
+                         reinterpret_cast<uintptr_t>(beta) | reinterpret_cast<uintptr_t>(residual);
+  TTMI_REQUIRE(rows % (4 * sizeof(T)) == 0 && aligned16(slices) && aligned16(residual_f32) && aligned16(out_f32), "rows must be aligned to four elements");
+  launch_reduce_layer_norm<T>(slices, (int)count, m, n, bias, residual, residual_f32, gamma, beta, out, out_f32, eps, s);
+  return launch_status("add_slices_layer_norm");
+}
+
 // Product + AddBiasLayerNorm.
 template <typename T>
 int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* out, const void* residual, const float* residual_f32,
@@ -159,14 +189,7 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* 
   g.inner = 1;
   if (packed) use_packed_weights(g);
   auto reduce = [&](const float* ws, int slices, bool, hipStream_t st) {
-    auto launch = [&](auto iters) {
-      hipLaunchKernelGGL((splitk_reduce_layer_norm_kernel<T, decltype(iters)::value>), dim3((unsigned)m), dim3(256), 0, st, ws,
-                         slices, (int)m, (int)n, (const T*)bias, (const T*)residual, residual_f32, (const T*)gamma,
-                         (const T*)beta, (T*)out, out_f32, eps);
-    };
-    if (n <= 1024) launch(std::integral_constant<int, 1>{});
-    else if (n <= 2048) launch(std::integral_constant<int, 2>{});
-    else launch(std::integral_constant<int, 4>{});
+    launch_reduce_layer_norm<T>(ws, slices, m, n, bias, residual, residual_f32, gamma, beta, out, out_f32, eps, st);
   };
   if constexpr (sizeof(T) == 2) {
     int slices = rows_ok ? w4_splitk_slices<T>(g, aligned) : 0;
@@ -231,6 +254,8 @@ int gemm_bias_layer_norm_typed(const void* a, const void* w, bool packed, void* 
                                         const ttmi_epilogue_args*, hipStream_t);                                              \
   template int gemm_bias_layer_norm_typed<T>(const void*, const void*, bool, void*, const void*, const float*, const void*,         \
                                              const void*, const void*, float*, int64_t, int64_t, int64_t, float, int,         \
-                                             hipStream_t);
+                                             hipStream_t);                                                                    \
+  template int add_slices_layer_norm_typed<T>(const float*, int64_t, void*, const void*, const float*, const void*, const void*, \
+                                              const void*, float*, int64_t, int64_t, float, hipStream_t);
 
 }  // namespace ttmi

@@ -261,19 +261,18 @@ void AddBiasLayerNormResidual(const Tensor& input_tensor, const Tensor& bias_ten
                                                      DeviceDType(*out_tensor), Stream()));
 }
 
-void GemmAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& residual, const Tensor& bias_tensor,
-                          const Tensor& gamma_tensor, const Tensor& beta_tensor, Tensor* out_tensor, float eps) {
+// The checks of a product followed by AddBiasLayerNorm, and the residual stream it takes: launch(residual, residual32, out32)
+template <typename Launch>
+static void WithResidual(int64_t m, int64_t n, const Tensor& residual, const Tensor& bias_tensor, const Tensor& gamma_tensor,
+                         const Tensor& beta_tensor, Tensor* out_tensor, const Launch& launch) {
   RequireGpu(*out_tensor, "AddBiasLayerNorm");
-  const int64_t k = in.shape(-1), m = in.numel() / k;
   TT_ENFORCE_EQ(n, gamma_tensor.shape(0), "AddBiasLayerNorm input_tensor.shape(-1) should be the same as gamma_tensor.shape(0)");
   TT_ENFORCE_EQ(n, beta_tensor.shape(0), "AddBiasLayerNorm input_tensor.shape(-1) should be the same as beta_tensor.shape(0)");
   TT_ENFORCE_EQ(n, bias_tensor.shape(0), "AddBiasLayerNorm input_tensor.shape(-1) should be the same as bias_tensor.shape(0)");
   TT_ENFORCE_EQ(residual.numel(), m * n, "The shape of the input_tensor and out_tensor is not equal.");
   TT_ENFORCE_EQ(out_tensor->numel(), m * n, "The shape of the input_tensor and out_tensor is not equal.");
-  const int dt = w_nk.DTypeFor(DeviceDType(*out_tensor));
   if (!KeepsFp32Residual(*out_tensor)) {
-    TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk.data, out_tensor->mutable_raw(), residual.raw(), nullptr, bias_tensor.raw(),
-                                             gamma_tensor.raw(), beta_tensor.raw(), nullptr, m, n, k, eps, dt, Stream()));
+    launch(residual.raw(), nullptr, nullptr);
     return;
   }
   Tensor converted(nullptr);
@@ -285,10 +284,25 @@ void GemmAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, co
     TT_DEVICE_CALL(ttmi_convert(residual.raw(), DeviceDType(residual), p, TTMI_F32, m * n, Stream()));
     residual32 = p;
   }
-  Tensor* out32 = out_tensor->EnsureShadow();
-  TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk.data, out_tensor->mutable_raw(), nullptr, residual32, bias_tensor.raw(),
-                                           gamma_tensor.raw(), beta_tensor.raw(), out32->mutableData<float>(), m, n, k, eps, dt,
-                                           Stream()));
+  launch(nullptr, residual32, out_tensor->EnsureShadow()->mutableData<float>());
+}
+
+void GemmAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& residual, const Tensor& bias_tensor,
+                          const Tensor& gamma_tensor, const Tensor& beta_tensor, Tensor* out_tensor, float eps) {
+  const int64_t k = in.shape(-1), m = in.numel() / k;
+  WithResidual(m, n, residual, bias_tensor, gamma_tensor, beta_tensor, out_tensor, [&](const void* r, const float* r32, float* out32) {
+    TT_DEVICE_CALL(ttmi_gemm_bias_layer_norm(in.raw(), w_nk.data, out_tensor->mutable_raw(), r, r32, bias_tensor.raw(), gamma_tensor.raw(),
+                                             beta_tensor.raw(), out32, m, n, k, eps, w_nk.DTypeFor(DeviceDType(*out_tensor)), Stream()));
+  });
+}
+
+void AddSlicesLayerNorm(const Tensor& slices, const Tensor& residual, const Tensor& bias_tensor, const Tensor& gamma_tensor,
+                        const Tensor& beta_tensor, Tensor* out_tensor, float eps) {
+  const int64_t m = slices.shape(1), n = slices.shape(2);
+  WithResidual(m, n, residual, bias_tensor, gamma_tensor, beta_tensor, out_tensor, [&](const void* r, const float* r32, float* out32) {
+    TT_DEVICE_CALL(ttmi_add_slices_layer_norm(slices.data<float>(), slices.shape(0), out_tensor->mutable_raw(), r, r32, bias_tensor.raw(),
+                                              gamma_tensor.raw(), beta_tensor.raw(), out32, m, n, eps, DeviceDType(*out_tensor), Stream()));
+  });
 }
 
 template <typename T, ActivationType ActType>

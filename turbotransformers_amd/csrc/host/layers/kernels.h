@@ -98,6 +98,9 @@ bool KeepsFp32Residual(const core::Tensor& t);  // true for bfloat16 tensors
 void GemmAddBiasLayerNorm(const core::Tensor& in, const WeightRef& w_nk, int64_t n, const core::Tensor& residual,
                           const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor, const core::Tensor& beta_tensor,
                           core::Tensor* out_tensor, float eps = 1e-12f);
+// The same of a product that exists as fp32 slices [count, m, n].
+void AddSlicesLayerNorm(const core::Tensor& slices, const core::Tensor& residual, const core::Tensor& bias_tensor,
+                        const core::Tensor& gamma_tensor, const core::Tensor& beta_tensor, core::Tensor* out_tensor, float eps = 1e-12f);
 
 // ---- fused forms used by the layers (no counterpart in the reference's kernel API) --------
 int DeviceDType(const core::Tensor& t);  // ttmi_dtype of a floating tensor, throws otherwise

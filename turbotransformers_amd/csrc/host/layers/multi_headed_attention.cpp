@@ -60,6 +60,16 @@ bool MultiHeadedAttention::UseProbsCore(int64_t head_dim, int64_t keys, std::ini
   return head_dim == 64 && keys > 0 && keys <= TTMI_PROBS_MAX_KEYS && aligned;
 }
 
+bool MultiHeadedAttention::UseProjectingCore(const Tensor& query_tensor, const WeightRef& wo, int64_t tokens, int64_t v_pitch, int dtype) const {
+  // us per forward of fp16 base, separate / projecting: 1 x 10 tokens 332 / 306, 1 x 32 343 / 311, 2 x 20 366 / 348, 1 x 64 368 / 352, 4 x
+  // 16 369 / 360, 1 x 100 437 / 444, 8 x 16 422 / 468: a product per head is as many fp32 slices, which more rows make the larger part.
+  constexpr int64_t kMostRows = 64;
+  bool aligned = true;
+  for (const void* p : {query_tensor.raw(), wo.data, dense_bias_.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw()})
+    aligned = aligned && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  return (dtype == TTMI_F16 || dtype == TTMI_BF16) && v_pitch > 0 && tokens <= kMostRows && query_tensor.shape(-1) <= 4096 && aligned;
+}
+
 static int64_t RoundUp8(int64_t n) { return (n + 7) / 8 * 8; }
 
 // score -> softmax -> P V -> merge heads -> output projection -> bias (+input) (+LayerNorm)
@@ -74,8 +84,24 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   const int64_t hidden = query_tensor.shape(-1), heads = num_attention_heads_, d = hidden / heads;
   const int64_t tokens = query_tensor.numel() / hidden;
 
-  ctx_.ReshapeAs(query_tensor.dtype(), {tokens, hidden}, dev, dev_id, "batch_gemm4/Reshape");
   const float scaler = 1.0f / std::sqrt(static_cast<float>(d));
+  const WeightRef wo = dense_packed_.Get(dense_weight_, is_trans_weight);
+  const void* ahead_data[TTMI_MAX_AHEAD];
+  int64_t ahead_bytes[TTMI_MAX_AHEAD];
+  const size_t ranges = std::min(ahead.size(), (size_t)TTMI_MAX_AHEAD);
+  for (size_t i = 0; i < ranges; ++i) ahead_data[i] = ahead[i].data, ahead_bytes[i] = ahead[i].bytes;
+  if (fused_core && seq_list == nullptr && post_layernorm && !post_add_input && UseProjectingCore(query_tensor, wo, tokens, v_pitch, dt)) {
+    if (!attention_mask.is_null()) TT_ENFORCE_EQ(attention_mask.numel(), batch * seq, "attention mask has the wrong size");
+    TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
+    float* partial = partial_.Reshape<float>({heads, tokens, hidden}, dev, dev_id, "gemm5/slices/Reshape");
+    TT_DEVICE_CALL(ttmi_attention_projection(q_.raw(), k.raw(), v.raw(), attention_mask.is_null() ? nullptr : attention_mask.data<float>(),
+                                             wo.data, partial, batch, heads, seq, d, v_pitch, scaler, dt, ahead_data,
+                                             ahead_bytes, (int64_t)ranges, Stream()));
+    output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
+    kernels::AddSlicesLayerNorm(partial_, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
+    return;
+  }
+  ctx_.ReshapeAs(query_tensor.dtype(), {tokens, hidden}, dev, dev_id, "batch_gemm4/Reshape");
 
   // Nobody asked for the probabilities: run the whole core as one kernel; the [B,h,S,S] scores
   // never reach HBM.
@@ -88,10 +114,6 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
     TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
     const int32_t* cu = nullptr;
     if (seq_list != nullptr) cu = DeviceContext::GetInstance().GetSeqPlan(*seq_list).cu_seqlens;
-    const void* ahead_data[TTMI_MAX_AHEAD];
-    int64_t ahead_bytes[TTMI_MAX_AHEAD];
-    const size_t ranges = std::min(ahead.size(), (size_t)TTMI_MAX_AHEAD);
-    for (size_t i = 0; i < ranges; ++i) ahead_data[i] = ahead[i].data, ahead_bytes[i] = ahead[i].bytes;
     TT_DEVICE_CALL(ttmi_fused_attention_ahead(q_.raw(), k.raw(), v.raw(), mask, ctx_.mutable_raw(), cu, batch, heads, seq, d,
                                               v_pitch, scaler, dt, ahead_data, ahead_bytes, (int64_t)ranges, Stream()));
   } else {
@@ -139,7 +161,6 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   }  // unfused core
 
   output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
-  const WeightRef wo = dense_packed_.Get(dense_weight_, is_trans_weight);
   if (!post_add_input && post_layernorm) {
     // gemm5 then AddBiasLayerNorm(query, bias, gamma, beta, out), eps 1e-12 (:359-371)
     kernels::GemmAddBiasLayerNorm(ctx_, wo, hidden, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);

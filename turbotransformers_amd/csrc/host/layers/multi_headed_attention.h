@@ -87,6 +87,9 @@ class MultiHeadedAttention {
   // The one-kernel core that also returns the probabilities (head size 64, up to TTMI_PROBS_MAX_KEYS keys).
   bool UseProbsCore(int64_t head_dim, int64_t keys, std::initializer_list<const core::Tensor*> tensors) const;
 
+  // Attention core and output projection as one launch, the heads' parts of it added up by the LayerNorm behind.
+  bool UseProjectingCore(const core::Tensor& query_tensor, const WeightRef& wo, int64_t tokens, int64_t v_pitch, int dtype) const;
+
   // Everything after q/k/v exist, shared by the dense and the smart-batch layers.
   // `fused_core`: the one-kernel attention core runs; `v_pitch` > 0: v holds V transposed, [B,h,d,v_pitch].
   // `seq` query positions against `key_seq` key positions held in k / v ([B,h,key_seq,d]); with `grow` the first of them
@@ -104,7 +107,7 @@ class MultiHeadedAttention {
 
   PackedWeight qkv_packed_, dense_packed_, q_packed_, k_packed_, v_packed_, kv_packed_;
   // Per-call intermediates, reused across calls (Reshape keeps a buffer that is large enough).
-  mutable core::Tensor q_, k_, v_, k_grown_, v_grown_, kv_bias_, ctx_, score_scratch_, ln_query_;
+  mutable core::Tensor q_, k_, v_, k_grown_, v_grown_, kv_bias_, ctx_, partial_, score_scratch_, ln_query_;
   mutable std::mutex mutex_;  // the layer keeps per-call state, like the reference (…attention.cpp:32,272)
 };
 
