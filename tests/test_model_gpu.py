@@ -915,3 +915,31 @@ def test_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
         one_call = encoder(x, return_type=tt.ReturnType.TORCH)[0]
         by_layer = encoder(x, output_hidden_states=True, return_type=tt.ReturnType.TORCH)[0]
         assert torch.equal(one_call, by_layer) and bool(torch.isfinite(one_call.float()).all())
+
+
+@pytest.mark.parametrize("kind", ["bert", "smart batch", "int8"])
+def test_layers_of_an_encoder_share_their_scratch(tt, kind):
+    """The layers of an encoder hold the tensors of a call in one place: the same bits as layers that share nothing, for batches that
+    grow and shrink, and the memory that a longer batch adds is that of one layer, not of all."""
+    from turbotransformers_amd import cxx
+    model, cfg = _hf_bert(6, seed=3, hidden_size=256, num_attention_heads=4, intermediate_size=1024, vocab_size=10)
+    layer_type, encoder_type = {"bert": (tt.BertLayer, tt.BertEncoder), "smart batch": (tt.BertLayerSmartBatch, tt.BertEncoderSmartBatch),
+                                "int8": (tt.QBertLayer, tt.QBertEncoder)}[kind]
+    encoder = encoder_type([layer_type.from_torch(l) for l in model.encoder.layer])
+    alone = [layer_type.from_torch(l) for l in model.encoder.layer]
+    torch_type = tt.ReturnType.TORCH
+    for lens in ([37, 20], [300, 255], [9, 64]):
+        args = (lens, ) if kind == "smart batch" else ()
+        shape = (1, sum(lens)) if kind == "smart batch" else (2, max(lens))
+        x = torch.randn(*shape, 256, device="cuda", generator=torch.Generator("cuda").manual_seed(lens[0]))
+        before = cxx.allocator_stats()["bytes_live"]
+        got = encoder(x, *args, return_type=torch_type)[0].clone()
+        torch.cuda.synchronize()
+        grown = cxx.allocator_stats()["bytes_live"] - before
+        if lens[0] == 300:  # six layers of their own hold at least q, k, v and the context each; one of them also the scores of its chain
+            assert grown < 6 * 4 * x.numel() * 4
+        want = x
+        for layer in alone:
+            want = layer(want, *args, return_type=torch_type)[0]
+        assert torch.equal(got, want)
+

@@ -55,7 +55,10 @@ struct BertModel::Impl {
                                                Take(&weights, e + "position_embeddings.weight"),
                                                Take(&weights, e + "token_type_embeddings.weight"),
                                                Take(&weights, e + "LayerNorm.weight"), Take(&weights, e + "LayerNorm.bias")));
-    for (size_t i = 0; i < n_layers; ++i) encoders_.emplace_back(&weights, "encoder.layer." + std::to_string(i) + ".", n_heads);
+    for (size_t i = 0; i < n_layers; ++i) {
+      encoders_.emplace_back(&weights, "encoder.layer." + std::to_string(i) + ".", n_heads);
+      encoders_[i].attention_->ShareScratch(*encoders_[0].attention_);
+    }
     if (weights.count("pooler.dense.weight"))
       pooler_.reset(new layers::BertPooler(Take(&weights, "pooler.dense.weight"), Take(&weights, "pooler.dense.bias")));
   }

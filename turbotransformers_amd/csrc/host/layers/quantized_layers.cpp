@@ -42,13 +42,13 @@ void QuantizedLinear::Prepare() const {
   prepared_ = true;
 }
 
-const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor) const {
+const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor, Tensor* quantised) const {
   kernels::RequireGpu(input_tensor, "QuantizedLinear");
   Prepare();
   const int64_t k = weight_.shape(0);
   TT_ENFORCE_EQ(input_tensor.shape(-1), k, "input width and weight rows differ");
   const int64_t m = input_tensor.numel() / k;
-  int8_t* qx = q_input_.Reshape<int8_t>({m, k}, input_tensor.device_type(), input_tensor.device_id(), "QuantizedLinear/q_input");
+  int8_t* qx = quantised->Reshape<int8_t>({m, k}, input_tensor.device_type(), input_tensor.device_id(), "QuantizedLinear/q_input");
   if (input_tensor.absmax() != nullptr) {
     // the kernel that produced the input left its per-workgroup maxima: one launch instead of two
     TT_DEVICE_CALL(ttmi_quantize_rows_i8_from_absmax(input_tensor.data<float>(), qx, act_scale_.mutableData<float>(),
@@ -60,7 +60,9 @@ const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor) const {
 }
 
 void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tensor) const {
-  const int8_t* qx = QuantizeInput(input_tensor);
+  const std::shared_ptr<Scratch> scratch = std::atomic_load(&scratch_);
+  std::lock_guard<std::mutex> lock(scratch->mutex);
+  const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;
   std::vector<int64_t> shape;
   for (size_t i = 0; i + 1 < input_tensor.n_dim(); ++i) shape.push_back(input_tensor.shape((int)i));
@@ -85,7 +87,9 @@ void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tens
 void QuantizedLinear::ProjectToHeads(const Tensor& input_tensor, const Tensor& bias, int64_t seq, int64_t heads, Tensor* q,
                                      Tensor* k_out, Tensor* v) const {
   TT_ENFORCE(bias_.is_null() && act_ < 0, "ProjectToHeads takes the bias as an argument");
-  const int8_t* qx = QuantizeInput(input_tensor);
+  const std::shared_ptr<Scratch> scratch = std::atomic_load(&scratch_);
+  std::lock_guard<std::mutex> lock(scratch->mutex);
+  const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;
   TT_ENFORCE_EQ(bias.numel(), n, "bias and weight shape mismatch");
   TT_ENFORCE(n % (3 * heads) == 0 && q->numel() == m * (n / 3), "q,k,v must be shaped [B, heads, S, d]");
@@ -97,17 +101,18 @@ void QuantizedLinear::ProjectToHeads(const Tensor& input_tensor, const Tensor& b
 void QuantizedBertAttention::operator()(const Tensor& input_tensor, const Tensor& attention_mask, Tensor* output,
                                         Tensor* attn) const {
   std::lock_guard<std::mutex> g(mutex_);
+  std::lock_guard<std::mutex> use(scratch_->mutex);
   kernels::RequireGpu(input_tensor, "QuantizedBertAttention");
   TT_ENFORCE_EQ(input_tensor.n_dim(), (size_t)3, "input should be [batch, seq, hidden]");
   const int64_t B = input_tensor.shape(0), S = input_tensor.shape(1), H = input_tensor.shape(2), d = H / heads_;
   const DLDeviceType dev = input_tensor.device_type();
   const int id = input_tensor.device_id();
   // QKV projection (int8) with bias and head split in its store; then the reference's unfused fp32 chain
-  q_.Reshape<float>({B, heads_, S, d}, dev, id, "self/q/Reshape");
-  k_.Reshape<float>({B, heads_, S, d}, dev, id, "self/k/Reshape");
-  v_.Reshape<float>({B, heads_, S, d}, dev, id, "self/v/Reshape");
-  qkv_.ProjectToHeads(input_tensor, qkv_bias_, S, heads_, &q_, &k_, &v_);
-  merged_.Reshape<float>({B, S, H}, dev, id, "batch_gemm4/Reshape");
+  scratch_->q.Reshape<float>({B, heads_, S, d}, dev, id, "self/q/Reshape");
+  scratch_->k.Reshape<float>({B, heads_, S, d}, dev, id, "self/k/Reshape");
+  scratch_->v.Reshape<float>({B, heads_, S, d}, dev, id, "self/v/Reshape");
+  qkv_.ProjectToHeads(input_tensor, qkv_bias_, S, heads_, &scratch_->q, &scratch_->k, &scratch_->v);
+  scratch_->merged.Reshape<float>({B, S, H}, dev, id, "batch_gemm4/Reshape");
   if (MultiHeadedAttention::UseFusedCore(attention_mask, attn, d, TTMI_F32, B, S, heads_)) {
     // nobody asked for the probabilities: the fp32 one-kernel attention (row-major V) in place of the four launches
     const float* mask = nullptr;
@@ -116,24 +121,24 @@ void QuantizedBertAttention::operator()(const Tensor& input_tensor, const Tensor
       mask = attention_mask.data<float>();
     }
     // the kernel leaves the maxima of the context with the tensor: the output projection quantises it in one launch
-    void* merged = merged_.mutable_raw();
-    float* slots = merged_.EnsureAbsmax()->mutableData<float>();
+    void* merged = scratch_->merged.mutable_raw();
+    float* slots = scratch_->merged.EnsureAbsmax()->mutableData<float>();
     int written = 0;
-    TT_DEVICE_CALL(ttmi_fused_attention_absmax(q_.raw(), k_.raw(), v_.raw(), mask, merged, nullptr, B, heads_, S, d, 0,
+    TT_DEVICE_CALL(ttmi_fused_attention_absmax(scratch_->q.raw(), scratch_->k.raw(), scratch_->v.raw(), mask, merged, nullptr, B, heads_, S, d, 0,
                                                1.0f / std::sqrt((float)d), TTMI_F32, slots, &written, Stream()));
-    if (written == 0) merged_.DropAbsmax();
-    dense_(merged_, output);
+    if (written == 0) scratch_->merged.DropAbsmax();
+    dense_(scratch_->merged, output);
     kernels::AddBiasLayerNormWithAbsmax(input_tensor, dense_bias_, ln_weight_, ln_bias_, output, 1e-12f);
     return;
   }
-  Tensor* score = attn != nullptr ? attn : &score_scratch_;
+  Tensor* score = attn != nullptr ? attn : &scratch_->score;
   score->Reshape<float>({B, heads_, S, S}, dev, id, "batch_gemm3/Reshape");
-  kernels::BatchMatMul(q_, false, k_, true, 1.0f / std::sqrt((float)d), score, 0.f);
+  kernels::BatchMatMul(scratch_->q, false, scratch_->k, true, 1.0f / std::sqrt((float)d), score, 0.f);
   kernels::ApplyMaskAndSoftmax(score, attention_mask, 1.0f);
-  ctx_.Reshape<float>({B, heads_, S, d}, dev, id, "ApplyMaskAndSoftmax/Reshape");
-  kernels::BatchMatMul(*score, false, v_, false, 1.0f, &ctx_, 0.f);
-  kernels::TransposeForScore(&merged_, ctx_);
-  dense_(merged_, output);
+  scratch_->ctx.Reshape<float>({B, heads_, S, d}, dev, id, "ApplyMaskAndSoftmax/Reshape");
+  kernels::BatchMatMul(*score, false, scratch_->v, false, 1.0f, &scratch_->ctx, 0.f);
+  kernels::TransposeForScore(&scratch_->merged, scratch_->ctx);
+  dense_(scratch_->merged, output);
   kernels::AddBiasLayerNormWithAbsmax(input_tensor, dense_bias_, ln_weight_, ln_bias_, output, 1e-12f);
 }
 

@@ -11,6 +11,7 @@
 // that every Linear of the layer is int8.
 #pragma once
 
+#include <memory>
 #include <mutex>
 #include <string>
 
@@ -32,15 +33,22 @@ class QuantizedLinear {
   // SplitAddBiasTransposeForScore of the attention in one kernel.  q,k,v are already shaped.
   void ProjectToHeads(const core::Tensor& input_tensor, const core::Tensor& bias, int64_t seq, int64_t heads, core::Tensor* q,
                       core::Tensor* k, core::Tensor* v) const;
+  // As MultiHeadedAttention::ShareScratch, for the quantised inputs.
+  void ShareScratch(const QuantizedLinear& other) { std::atomic_store(&scratch_, std::atomic_load(&other.scratch_)); }
   int64_t in_features() const { return weight_.shape(0); }
   int64_t out_features() const { return weight_.shape(1); }
 
  private:
   void Prepare() const;
-  const int8_t* QuantizeInput(const core::Tensor& input_tensor) const;  // -> q_input_, scale in act_scale_
+  const int8_t* QuantizeInput(const core::Tensor& input_tensor, core::Tensor* quantised) const;  // its scale in act_scale_
   core::Tensor weight_, bias_;
   int act_ = -1;  // ttmi_act; -1 = none
-  mutable core::Tensor q_weight_, w_scales_, q_input_, act_scale_;
+  struct Scratch {
+    core::Tensor q_input;
+    std::mutex mutex;  // from the launch that writes the quantised input to the one that reads it
+  };
+  mutable core::Tensor q_weight_, w_scales_, act_scale_;
+  std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
   mutable bool prepared_ = false;
   mutable std::mutex prepare_mutex_;  // the one-time weight quantisation; calls on one object are otherwise not concurrent
 };
@@ -55,12 +63,29 @@ class QuantizedBertAttention {
   // Same contract as BertAttention::operator() for fp32 tensors.
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output,
                   core::Tensor* attn = nullptr) const;
+  // As MultiHeadedAttention::ShareScratch.
+  void ShareScratch(const QuantizedBertAttention& other) {
+    if (&other == this) return;
+    std::shared_ptr<Scratch> shared;
+    {
+      std::lock_guard<std::mutex> lock(other.mutex_);
+      shared = other.scratch_;
+    }
+    std::lock_guard<std::mutex> lock(mutex_);
+    scratch_ = std::move(shared);
+    qkv_.ShareScratch(other.qkv_);
+    dense_.ShareScratch(other.qkv_);
+  }
 
  private:
   QuantizedLinear qkv_, dense_;
   core::Tensor qkv_bias_, dense_bias_, ln_weight_, ln_bias_;
   int64_t heads_;
-  mutable core::Tensor q_, k_, v_, ctx_, merged_, score_scratch_;
+  struct Scratch {
+    core::Tensor q, k, v, ctx, merged, score;
+    std::mutex mutex;
+  };
+  std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
   mutable std::mutex mutex_;
 };
 

@@ -126,7 +126,9 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                                          std::move(ln_w), std::move(ln_b), heads);
       }))
       .def("__call__", py::overload_cast<const Tensor&, const Tensor&, Tensor*, Tensor*, bool>(&layers::BertAttention::operator(), py::const_), py::arg("input_tensor"), py::arg("attention_mask"),
-           py::arg("output"), py::arg("attn") = nullptr, py::arg("is_trans_weight") = false);
+           py::arg("output"), py::arg("attn") = nullptr, py::arg("is_trans_weight") = false)
+      .def("share_scratch", [](layers::BertAttention& self, const layers::BertAttention& other) { self.ShareScratch(other); },
+           "Hold the tensors of a call where `other` holds its own: for layers that run one after the other.");
 
   py::class_<layers::MultiHeadedAttention>(m, "MultiHeadedAttention")
       .def(py::init([](Tensor& kw, Tensor& kb, Tensor& vw, Tensor& vb, Tensor& qw, Tensor& qb, Tensor& dw, Tensor& db,
@@ -157,7 +159,8 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                                                           std::move(qkvw), std::move(qkvb), std::move(gamma), std::move(beta),
                                                           heads);
       }))
-      .def("__call__", &layers::MultiHeadedAttentionSmartBatch::operator());
+      .def("__call__", &layers::MultiHeadedAttentionSmartBatch::operator())
+      .def("share_scratch", [](layers::MultiHeadedAttentionSmartBatch& self, const layers::MultiHeadedAttentionSmartBatch& other) { self.ShareScratch(other); });
 
   py::class_<layers::BertIntermediate>(m, "BertIntermediate")
       .def(py::init([](Tensor& w, Tensor& b) { return new layers::BertIntermediate(std::move(w), std::move(b)); }))
@@ -219,7 +222,8 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
       .def(py::init([](Tensor& w, Tensor& bias, const std::string& activation) {
         return new layers::QuantizedLinear(std::move(w), std::move(bias), activation);
       }))
-      .def("__call__", &layers::QuantizedLinear::operator());
+      .def("__call__", &layers::QuantizedLinear::operator())
+      .def("share_scratch", [](layers::QuantizedLinear& self, const layers::QuantizedLinear& other) { self.ShareScratch(other); });
 
   py::class_<layers::QuantizedBertAttention>(m, "QuantizedBertAttention")
       .def(py::init([](Tensor& qkv_w, Tensor& qkv_b, Tensor& dense_w, Tensor& dense_b, Tensor& ln_w, Tensor& ln_b, int heads) {
@@ -227,7 +231,8 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                                                   std::move(ln_w), std::move(ln_b), heads);
       }))
       .def("__call__", &layers::QuantizedBertAttention::operator(), py::arg("input_tensor"), py::arg("attention_mask"),
-           py::arg("output"), py::arg("attn") = nullptr);
+           py::arg("output"), py::arg("attn") = nullptr)
+      .def("share_scratch", [](layers::QuantizedBertAttention& self, const layers::QuantizedBertAttention& other) { self.ShareScratch(other); });
 
   m.def("build_smart_pad_mask",
         [](const std::vector<int64_t>& lens, Tensor* out) {

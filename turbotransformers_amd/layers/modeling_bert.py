@@ -13,7 +13,7 @@ import torch
 
 from .. import cxx
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, to_param_dict_convert_tt,
+from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, share_scratch, to_param_dict, to_param_dict_convert_tt,
                     try_convert, use_current_stream, weight_in_out)
 
 __all__ = ['BertEmbeddings', 'BertIntermediate', 'BertOutput', 'BertAttention', 'BertLayer', 'BertEncoder',
@@ -163,6 +163,7 @@ class BertLayer:
 class BertEncoder:
     def __init__(self, layer: Sequence[BertLayer]):
         self.layer = layer
+        share_scratch(l.attention for l in layer if isinstance(l, BertLayer))
 
     def __call__(self, hidden_states: AnyTensor, attention_mask: Optional[AnyTensor] = None,
                  head_mask: Optional[AnyTensor] = None, output_attentions: Optional[bool] = False,

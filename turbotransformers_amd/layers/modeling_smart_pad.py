@@ -16,8 +16,8 @@ from .. import cxx
 from .modeling_bert import (BertEmbeddings, BertIntermediate, BertOutput, BertPooler, PoolingMap, PoolingType,
                             SequencePool, _require_gpu)
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, try_convert, use_current_stream,
-                    weight_in_out)
+from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, share_scratch, try_convert,
+                    use_current_stream, weight_in_out)
 
 __all__ = ['MultiHeadedAttentionSmartBatch', 'BertLayerSmartBatch', 'BertEncoderSmartBatch',
            'BertModelNoPoolerSmartBatch', 'BertModelSmartBatch']
@@ -114,6 +114,7 @@ class BertLayerSmartBatch:
 class BertEncoderSmartBatch:
     def __init__(self, layer: Sequence[BertLayerSmartBatch]):
         self.layer = layer
+        share_scratch(l.attention for l in layer if isinstance(l, BertLayerSmartBatch))
 
     def __call__(self, hidden_states: AnyTensor, query_seq_len_list: Sequence[int],
                  attention_mask: Optional[AnyTensor] = None, head_mask: Optional[AnyTensor] = None,

@@ -15,7 +15,7 @@ import torch
 from .. import cxx
 from .modeling_bert import BertAttention, BertEmbeddings, BertPooler, PoolingMap, PoolingType, SequencePool, _require_gpu
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import convert2tt_tensor, create_empty_if_none, to_param_dict, try_convert, use_current_stream, weight_in_out
+from .utils import convert2tt_tensor, create_empty_if_none, share_scratch, to_param_dict, try_convert, use_current_stream, weight_in_out
 
 __all__ = ['QBertIntermediate', 'QBertOutput', 'QBertAttention', 'QBertLayer', 'QBertEncoder', 'QBertModel']
 
@@ -103,6 +103,9 @@ class QBertLayer:
 class QBertEncoder:
     def __init__(self, layers):
         self.layer = layers
+        plain = [l for l in layers if isinstance(l, QBertLayer)]
+        share_scratch(l.attention for l in plain)
+        share_scratch(part.linear for l in plain for part in (l.intermediate, l.output) if hasattr(part, 'linear'))
 
     def __call__(self, hidden_states, attention_mask=None, head_mask=None, output_attentions=False,
                  output_hidden_states=False, return_type: Optional[ReturnType] = None):
