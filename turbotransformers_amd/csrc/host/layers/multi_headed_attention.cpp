@@ -417,7 +417,8 @@ std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<BertSubLaye
     if (i > 0) ahead[i - 1].push_back(qkv);
   }
   constexpr int64_t kStays = 200ll << 20;
-  if (bytes <= kStays) ahead.assign(layers.size(), {});
+  const int64_t tensors = 16 * hidden.numel() * (int64_t)hidden.element_size();
+  if (bytes + tensors <= kStays) ahead.assign(layers.size(), {});
   return ahead;
 }
 
