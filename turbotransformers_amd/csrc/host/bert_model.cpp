@@ -67,7 +67,7 @@ struct BertModel::Impl {
     Tensor ext(nullptr);
     layers::PrepareBertMasks()(ids, mask, seq_type, position_ids, &ext);
     (*embedding_)(ids, *position_ids, *seq_type, hidden);
-    std::vector<layers::BertSubLayers> subs;
+    std::vector<layers::EncoderLayer<layers::BertAttention>> subs;
     for (auto& layer : encoders_) subs.push_back({layer.attention_.get(), layer.intermediate_.get(), layer.output_.get()});
     const auto ahead = layers::WeightsAhead(subs, *hidden);
     for (size_t i = 0; i < encoders_.size(); ++i) encoders_[i](*hidden, ext, &att_out_, &intermediate_out_, hidden, ahead[i]);

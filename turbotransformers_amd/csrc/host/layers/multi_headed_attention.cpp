@@ -403,32 +403,17 @@ void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attenti
           true /* post_layernorm */, false /* post_add_input */, is_trans_weight, ahead);
 }
 
-std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<BertSubLayers>& layers, const Tensor& hidden) {
-  std::vector<std::vector<WeightRange>> ahead(layers.size());
-  if (hidden.numel() <= 32 * hidden.shape(-1)) return ahead;
-  int64_t bytes = 0;
-  for (size_t i = 0; i < layers.size(); ++i) {
-    for (const WeightRange& r : {layers[i].attention->dense_weight(), layers[i].intermediate->weight(), layers[i].output->weight()}) {
-      ahead[i].push_back(r);
-      bytes += r.bytes;
-    }
-    const WeightRange qkv = layers[i].attention->qkv_weight();
-    bytes += qkv.bytes;
-    if (i > 0) ahead[i - 1].push_back(qkv);
-  }
+bool WeightsLeaveCache(int64_t bytes, const Tensor& hidden) {
   constexpr int64_t kStays = 200ll << 20;
   const int64_t tensors = 16 * hidden.numel() * (int64_t)hidden.element_size();
-  if (bytes + tensors <= kStays) ahead.assign(layers.size(), {});
-  return ahead;
+  return hidden.numel() > 32 * hidden.shape(-1) && bytes + tensors > kStays;
 }
 
-void MultiHeadedAttentionSmartBatch::operator()(const Tensor& key_tensor, const Tensor& value_tensor,
-                                                const Tensor& query_tensor, const Tensor& attention_mask,
-                                                const std::string& attn_type, Tensor* output, Tensor* att_score,
-                                                std::unordered_map<std::string, Tensor*> layer_cache,
-                                                const std::vector<int64_t>& query_seq_len_list,
-                                                const std::vector<int64_t>& key_seq_len_list, bool pre_layernorm,
-                                                bool post_layernorm, bool post_add_input, bool is_trans_weight) const {
+void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,
+                                             const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
+                                             Tensor* att_score, const std::unordered_map<std::string, Tensor*>& layer_cache,
+                                             const std::vector<int64_t>& query_seq_len_list, bool pre_layernorm, bool post_layernorm,
+                                             bool post_add_input, bool is_trans_weight, const std::vector<WeightRange>& ahead) const {
   std::lock_guard<std::mutex> g(mutex_);
   std::lock_guard<std::mutex> use(scratch_->mutex);
   TT_ENFORCE(attn_type == "self", "only attn_type \"self\" is built (\"context\" belongs to the decoder path)");
@@ -441,7 +426,6 @@ void MultiHeadedAttentionSmartBatch::operator()(const Tensor& key_tensor, const 
   MultiHeadedAttention::EnforceShapeAndType();
   (void)key_tensor;
   (void)value_tensor;
-  (void)key_seq_len_list;
 
   auto plan = DeviceContext::GetInstance().GetSeqPlan(query_seq_len_list);
   TT_ENFORCE_EQ(query_tensor.shape(1), plan.total, "The query_tensor shape 1 should be the sum of seq_len_list.");
@@ -483,7 +467,7 @@ void MultiHeadedAttentionSmartBatch::operator()(const Tensor& key_tensor, const 
                                  TTMI_EPI_QKV_SPLIT_PAD, &args, wqkv.DTypeFor(dt), Stream()));
 
   AttentionTail(query_tensor, attention_mask, output, att_score, batch, max_seq, max_seq, scratch_->k, scratch_->v, &query_seq_len_list, fused_core, 0,
-                post_layernorm, post_add_input, is_trans_weight);
+                post_layernorm, post_add_input, is_trans_weight, nullptr, ahead);
 }
 
 }  // namespace layers

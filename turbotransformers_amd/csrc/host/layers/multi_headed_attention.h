@@ -73,6 +73,9 @@ class MultiHeadedAttention {
   static bool UseFusedCore(const core::Tensor& attention_mask, const core::Tensor* att_score, int64_t head_dim, int dtype,
                            int64_t batch = 0, int64_t seq = 0, int64_t heads = 0, bool v_transposed = false);
 
+  WeightRange qkv_weight() const { return qkv_packed_.Range(qkv_weight_); }
+  WeightRange dense_weight() const { return dense_packed_.Range(dense_weight_); }
+
   // The layers of a stack run one after the other: they may share what they hold during a call.  With buffers of its own each layer of
   // an encoder writes and reads 4 x rows x hidden values in memory that the last-level cache (256 MB) has seen a whole pass ago, and
   // pushes the weights out of it: us per forward, own / shared, base: fp16 20 x 100 tokens 932 / 886, 12 x 64 592 / 527, int8 20 x 128
@@ -149,24 +152,7 @@ class BertAttention : public MultiHeadedAttention {
   }
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output, core::Tensor* attn,
                   bool is_trans_weight, const std::vector<WeightRange>& ahead) const;
-  WeightRange qkv_weight() const { return qkv_packed_.Range(qkv_weight_); }
-  WeightRange dense_weight() const { return dense_packed_.Range(dense_weight_); }
 };
-
-// One layer of an encoder.
-struct BertSubLayers {
-  const BertAttention* attention;
-  const BertIntermediate* intermediate;
-  const BertOutput* output;
-};
-// What the attention core of each layer may read ahead: the layer's other weights and the next layer's first one.  Nothing
-// for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
-// with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call
-// (Q, K, V, context, four of hidden states, the intermediate one, two fp32 slices of a product: 16 x rows x hidden) take their part of
-// the cache.  us per forward without / with, fp16 base (170 MB): 1 x 387 tokens 478 / 532 and 4 x 128 471 / 493 (180 MB in all), 12 x 64
-// 527 / 539 (189 MB), 20 x 100 888 / 853 (220 MB), 8 x 256 897 / 843, 40 x 128 1573 / 1518.
-// Nor for fp32 products of up to 32 rows, which take the fp32 weights as they are, all of a workgroup's share at once.
-std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<BertSubLayers>& layers, const core::Tensor& hidden);
 
 class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
  public:
@@ -179,8 +165,54 @@ class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
                   core::Tensor* att_score, std::unordered_map<std::string, core::Tensor*> layer_cache,
                   const std::vector<int64_t>& query_seq_len_list, const std::vector<int64_t>& key_seq_len_list,
                   bool pre_layernorm = false, bool post_layernorm = false, bool post_add_input = false,
-                  bool is_trans_weight = false) const;
+                  bool is_trans_weight = false) const {
+    Forward(key_tensor, value_tensor, query_tensor, attention_mask, attn_type, output, att_score, layer_cache, query_seq_len_list,
+            pre_layernorm, post_layernorm, post_add_input, is_trans_weight, {});
+  }
+  // self attention, post-LayerNorm, no extra residual, as a layer of an encoder
+  void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output,
+                  const std::vector<int64_t>& seq_len_list, const std::vector<WeightRange>& ahead) const {
+    Forward(input_tensor, input_tensor, input_tensor, attention_mask, "self", output, nullptr, {}, seq_len_list, false, true, false, false,
+            ahead);
+  }
+
+ private:
+  void Forward(const core::Tensor& key_tensor, const core::Tensor& value_tensor, const core::Tensor& query_tensor,
+               const core::Tensor& attention_mask, const std::string& attn_type, core::Tensor* output, core::Tensor* att_score,
+               const std::unordered_map<std::string, core::Tensor*>& layer_cache, const std::vector<int64_t>& query_seq_len_list,
+               bool pre_layernorm, bool post_layernorm, bool post_add_input, bool is_trans_weight,
+               const std::vector<WeightRange>& ahead) const;
 };
+
+// One layer of an encoder.
+template <typename Attention>
+struct EncoderLayer {
+  const Attention* attention;
+  const BertIntermediate* intermediate;
+  const BertOutput* output;
+};
+// What the attention core of each layer may read ahead: the layer's other weights and the next layer's first one.  Nothing
+// for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
+// with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call
+// (Q, K, V, context, four of hidden states, the intermediate one, two fp32 slices of a product: 16 x rows x hidden) take their part of
+// the cache.  us per forward without / with, fp16 base (170 MB): 1 x 387 tokens 478 / 532 and 4 x 128 471 / 493 (180 MB in all), 12 x 64
+// 527 / 539 (189 MB), 20 x 100 888 / 853 (220 MB), 8 x 256 897 / 843, 40 x 128 1573 / 1518.
+// Nor for fp32 products of up to 32 rows, which take the fp32 weights as they are, all of a workgroup's share at once.
+bool WeightsLeaveCache(int64_t bytes, const core::Tensor& hidden);
+template <typename Attention>
+std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<EncoderLayer<Attention>>& layers, const core::Tensor& hidden) {
+  std::vector<std::vector<WeightRange>> ahead(layers.size());
+  int64_t bytes = 0;
+  for (size_t i = 0; i < layers.size(); ++i) {
+    ahead[i] = {layers[i].attention->dense_weight(), layers[i].intermediate->weight(), layers[i].output->weight()};
+    const WeightRange qkv = layers[i].attention->qkv_weight();
+    for (const WeightRange& r : ahead[i]) bytes += r.bytes;
+    bytes += qkv.bytes;
+    if (i > 0) ahead[i - 1].push_back(qkv);
+  }
+  if (!WeightsLeaveCache(bytes, hidden)) ahead.assign(layers.size(), {});
+  return ahead;
+}
 
 }  // namespace layers
 }  // namespace turbo_transformers

@@ -159,7 +159,14 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                                                           std::move(qkvw), std::move(qkvb), std::move(gamma), std::move(beta),
                                                           heads);
       }))
-      .def("__call__", &layers::MultiHeadedAttentionSmartBatch::operator())
+      .def("__call__",
+           [](const layers::MultiHeadedAttentionSmartBatch& self, const Tensor& key, const Tensor& value, const Tensor& query, const Tensor& mask,
+              const std::string& attn_type, Tensor* output, Tensor* att_score, std::unordered_map<std::string, Tensor*> layer_cache,
+              const std::vector<int64_t>& query_lens, const std::vector<int64_t>& key_lens, bool pre_layernorm, bool post_layernorm,
+              bool post_add_input, bool is_trans_weight) {
+             self(key, value, query, mask, attn_type, output, att_score, std::move(layer_cache), query_lens, key_lens, pre_layernorm,
+                  post_layernorm, post_add_input, is_trans_weight);
+           })
       .def("share_scratch", [](layers::MultiHeadedAttentionSmartBatch& self, const layers::MultiHeadedAttentionSmartBatch& other) { self.ShareScratch(other); });
 
   py::class_<layers::BertIntermediate>(m, "BertIntermediate")
@@ -277,7 +284,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
   // three temporaries and a stream query each: at batch 1 x seq 128 the interpreter, not the GPU, set the pace).
   // `layer_list` is a sequence of (BertAttention, BertIntermediate, BertOutput).  No counterpart in the reference.
   m.def("run_bert_layers", [](const py::sequence& layer_list, const Tensor& hidden, const Tensor& mask, Tensor* out) {
-    std::vector<layers::BertSubLayers> subs;
+    std::vector<layers::EncoderLayer<layers::BertAttention>> subs;
     subs.reserve(py::len(layer_list));
     for (const py::handle& item : layer_list) {
       const py::tuple t = py::cast<py::tuple>(item);
@@ -293,6 +300,29 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
       // the last layer writes the caller's tensor; before it two buffers alternate (a layer never writes what it reads)
       Tensor* target = (i + 1 == subs.size()) ? out : (i % 2 == 0 ? &even : &odd);
       (*subs[i].attention)(*current, mask, &attention_out, nullptr, false, ahead[i]);
+      (*subs[i].intermediate)(attention_out, &intermediate_out);
+      (*subs[i].output)(intermediate_out, attention_out, target);
+      current = target;
+    }
+  });
+
+  // The same for a packed batch: `layer_list` is a sequence of (MultiHeadedAttentionSmartBatch, BertIntermediate, BertOutput).
+  m.def("run_smart_batch_layers", [](const py::sequence& layer_list, const Tensor& hidden, const Tensor& mask,
+                                     const std::vector<int64_t>& lens, Tensor* out) {
+    std::vector<layers::EncoderLayer<layers::MultiHeadedAttentionSmartBatch>> subs;
+    for (const py::handle& item : layer_list) {
+      const py::tuple t = py::cast<py::tuple>(item);
+      TT_ENFORCE_EQ(py::len(t), (size_t)3, "each layer is (attention, intermediate, output)");
+      subs.push_back({&py::cast<const layers::MultiHeadedAttentionSmartBatch&>(t[0]), &py::cast<const layers::BertIntermediate&>(t[1]),
+                      &py::cast<const layers::BertOutput&>(t[2])});
+    }
+    TT_ENFORCE(!subs.empty() && out != nullptr, "run_smart_batch_layers needs layers and an output tensor");
+    Tensor attention_out(nullptr), intermediate_out(nullptr), even(nullptr), odd(nullptr);
+    const Tensor* current = &hidden;
+    const auto ahead = layers::WeightsAhead(subs, hidden);
+    for (size_t i = 0; i < subs.size(); ++i) {
+      Tensor* target = (i + 1 == subs.size()) ? out : (i % 2 == 0 ? &even : &odd);
+      (*subs[i].attention)(*current, mask, &attention_out, lens, ahead[i]);
       (*subs[i].intermediate)(attention_out, &intermediate_out);
       (*subs[i].output)(intermediate_out, attention_out, target);
       current = target;

@@ -123,6 +123,13 @@ class BertEncoderSmartBatch:
         all_hidden_states, all_attentions = (), ()
         hidden_states = try_convert(hidden_states)
         attention_mask = try_convert(attention_mask)
+        if attention_mask is not None and not output_attentions and not output_hidden_states and self._plain_layers():
+            # nothing but the last hidden state is asked for: the layer loop runs inside the extension
+            use_current_stream()
+            last = cxx.Tensor.create_empty()
+            cxx.run_smart_batch_layers([(l.attention, l.intermediate, l.output) for l in self.layer], hidden_states, attention_mask,
+                                       [int(x) for x in query_seq_len_list], last)
+            return (convert_returns_as_type(last, return_type), )
         for layer in self.layer:
             layer_outputs = layer(hidden_states, query_seq_len_list, attention_mask,
                                   output_attentions=output_attentions, return_type=ReturnType.turbo_transformers)
@@ -137,6 +144,12 @@ class BertEncoderSmartBatch:
         if output_attentions:
             outputs = outputs + (all_attentions, )
         return outputs
+
+    def _plain_layers(self):
+        """Whether every layer is a BertLayerSmartBatch built from the three stock sub-layers (then the C++ loop may run them)."""
+        return len(self.layer) > 0 and all(
+            type(l) is BertLayerSmartBatch and type(l.attention) is MultiHeadedAttentionSmartBatch
+            and type(l.intermediate) is BertIntermediate and type(l.output) is BertOutput for l in self.layer)
 
     @staticmethod
     def from_torch(encoder):
