@@ -1198,6 +1198,27 @@ def test_attention_that_reads_ahead(ttmi, dt, B, S, v_transposed, packed):
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("B,h", [(3, 2), (45, 2), (60, 12)])
+@pytest.mark.parametrize("S", [9, 34, 36, 37, 39])
+def test_transposed_v_of_sequences_off_the_grid(ttmi, dt, B, h, S):
+    """Groups of eight and of four rows of the QKV product that two sequences share, divided at every place: V^T holds what a row-major V
+    does, and its pad columns nothing."""
+    import ctypes
+    rng = np.random.default_rng(S)
+    H, pitch, M = 64 * h, (S + 7) // 8 * 8 + 8, B * S
+    dA, dW = dev(rng.standard_normal((M, H), np.float32), dt), dev((rng.standard_normal((3 * H, H)) / np.sqrt(H)).astype(np.float32), dt)
+    db = dev(rng.standard_normal(3 * H).astype(np.float32), dt)
+    q, k, v = (torch.empty((B, h, S, 64), dtype=dA.dtype, device="cuda") for _ in range(3))
+    vt = torch.full((B, h, 64, pitch), 7.0, dtype=dA.dtype, device="cuda")
+    for out, v_pitch in ((v, 0), (vt, pitch)):
+        args = _epi(bias=db, q=q, k=k, v=out, seq=S, heads=h, head_dim=64, v_seq_pitch=v_pitch)
+        ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(dW), None, M, 3 * H, H, H, H, 3 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+    # (values of size 2, summed in the same or another order and rounded once)
+    assert max_abs(host(vt[..., :S]), host(v.transpose(2, 3))) <= GEMM_TOL[dt]
+    assert bool((vt[..., S:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("B,h,S", [(1, 1, 1), (1, 12, 10), (3, 3, 32), (1, 5, 33), (2, 12, 60), (1, 16, 300)])
 def test_attention_with_its_projection(ttmi, dt, B, h, S):
     """Attention and the output projection in one launch, a slice per head, against fp64; one and several blocks of queries and keys, a
