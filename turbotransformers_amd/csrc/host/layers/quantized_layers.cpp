@@ -24,9 +24,10 @@ QuantizedLinear::QuantizedLinear(core::Tensor weight, core::Tensor bias, const s
   else TT_ENFORCE(activation.empty(), "unknown activation %s", activation.c_str());
 }
 
-void QuantizedLinear::Prepare() const {
+std::shared_ptr<QuantizedLinear::Scratch> QuantizedLinear::Prepare(int64_t values) const {
   std::lock_guard<std::mutex> lock(prepare_mutex_);
-  if (prepared_) return;
+  const std::shared_ptr<Scratch>& scratch = values <= kOwnValues ? own_ : scratch_;
+  if (prepared_) return scratch;
   kernels::RequireGpu(weight_, "QuantizedLinear");
   TT_ENFORCE_EQ(weight_.n_dim(), (size_t)2, "weight must be [in, out]");
   const int64_t k = weight_.shape(0), n = weight_.shape(1);
@@ -40,11 +41,11 @@ void QuantizedLinear::Prepare() const {
   TT_DEVICE_CALL(ttmi_quantize_weight_rows_i8(t, q, s, n, k, Stream()));
   act_scale_.Reshape<float>({TTMI_QUANT_SCALE_FLOATS}, dev, id, "QuantizedLinear/act_scale");
   prepared_ = true;
+  return scratch;
 }
 
 const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor, Tensor* quantised) const {
   kernels::RequireGpu(input_tensor, "QuantizedLinear");
-  Prepare();
   const int64_t k = weight_.shape(0);
   TT_ENFORCE_EQ(input_tensor.shape(-1), k, "input width and weight rows differ");
   const int64_t m = input_tensor.numel() / k;
@@ -60,7 +61,7 @@ const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor, Tensor*
 }
 
 void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tensor) const {
-  const std::shared_ptr<Scratch> scratch = std::atomic_load(&scratch_);
+  const std::shared_ptr<Scratch> scratch = Prepare(input_tensor.numel());
   std::lock_guard<std::mutex> lock(scratch->mutex);
   const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;
@@ -87,7 +88,7 @@ void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tens
 void QuantizedLinear::ProjectToHeads(const Tensor& input_tensor, const Tensor& bias, int64_t seq, int64_t heads, Tensor* q,
                                      Tensor* k_out, Tensor* v) const {
   TT_ENFORCE(bias_.is_null() && act_ < 0, "ProjectToHeads takes the bias as an argument");
-  const std::shared_ptr<Scratch> scratch = std::atomic_load(&scratch_);
+  const std::shared_ptr<Scratch> scratch = Prepare(input_tensor.numel());
   std::lock_guard<std::mutex> lock(scratch->mutex);
   const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;

@@ -33,13 +33,21 @@ class QuantizedLinear {
   // SplitAddBiasTransposeForScore of the attention in one kernel.  q,k,v are already shaped.
   void ProjectToHeads(const core::Tensor& input_tensor, const core::Tensor& bias, int64_t seq, int64_t heads, core::Tensor* q,
                       core::Tensor* k, core::Tensor* v) const;
-  // As MultiHeadedAttention::ShareScratch, for the quantised inputs.
-  void ShareScratch(const QuantizedLinear& other) { std::atomic_store(&scratch_, std::atomic_load(&other.scratch_)); }
+  // As MultiHeadedAttention::ShareScratch, for the quantised inputs; between the same Linear of different layers.
+  void ShareScratch(const QuantizedLinear& other) {
+    if (&other == this) return;
+    std::shared_ptr<Scratch> shared;
+    {
+      std::lock_guard<std::mutex> lock(other.prepare_mutex_);
+      shared = other.scratch_;
+    }
+    std::lock_guard<std::mutex> lock(prepare_mutex_);
+    scratch_ = std::move(shared);
+  }
   int64_t in_features() const { return weight_.shape(0); }
   int64_t out_features() const { return weight_.shape(1); }
 
  private:
-  void Prepare() const;
   const int8_t* QuantizeInput(const core::Tensor& input_tensor, core::Tensor* quantised) const;  // its scale in act_scale_
   core::Tensor weight_, bias_;
   int act_ = -1;  // ttmi_act; -1 = none
@@ -47,10 +55,15 @@ class QuantizedLinear {
     core::Tensor q_input;
     std::mutex mutex;  // from the launch that writes the quantised input to the one that reads it
   };
+  // Up to a megabyte of quantised input a layer keeps a buffer of its own: a quantising launch of 77 rows into one that products of
+  // other layers have read is 3.8 instead of 3.3 us.
+  static constexpr int64_t kOwnValues = 1 << 20;
+  std::shared_ptr<Scratch> Prepare(int64_t values) const;
+  std::shared_ptr<Scratch> own_ = std::make_shared<Scratch>();
   mutable core::Tensor q_weight_, w_scales_, act_scale_;
   std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
   mutable bool prepared_ = false;
-  mutable std::mutex prepare_mutex_;  // the one-time weight quantisation; calls on one object are otherwise not concurrent
+  mutable std::mutex prepare_mutex_;  // scratch_, and the one-time weight quantisation; calls on one object are otherwise not concurrent
 };
 
 class QuantizedBertAttention {
@@ -74,7 +87,7 @@ class QuantizedBertAttention {
     std::lock_guard<std::mutex> lock(mutex_);
     scratch_ = std::move(shared);
     qkv_.ShareScratch(other.qkv_);
-    dense_.ShareScratch(other.qkv_);
+    dense_.ShareScratch(other.dense_);
   }
 
  private:

@@ -105,7 +105,8 @@ class QBertEncoder:
         self.layer = layers
         plain = [l for l in layers if isinstance(l, QBertLayer)]
         share_scratch(l.attention for l in plain)
-        share_scratch(part.linear for l in plain for part in (l.intermediate, l.output) if hasattr(part, 'linear'))
+        share_scratch(l.intermediate.linear for l in plain)
+        share_scratch(l.output.linear for l in plain)
 
     def __call__(self, hidden_states, attention_mask=None, head_mask=None, output_attentions=False,
                  output_hidden_states=False, return_type: Optional[ReturnType] = None):
