@@ -1386,6 +1386,35 @@ def test_fused_attention_fp32_outside_the_window(ttmi, what, v_transposed, packe
     assert bool(((got - want).abs() <= bound * column + 1e-30)[finite].all())
 
 
+@pytest.mark.parametrize("a,b", [(1e-8, 1e-8), (1e-6, 1e-6), (1e-8, 1.0), (1.0, 1e-7), (1e-15, 1e-15), (1e-3, 1e-3), (0.3, 0.3), (30.0, 30.0), (300.0, 1 / 300)])
+@pytest.mark.parametrize("v_transposed,packed", [(True, False), (False, True), (True, True)])
+def test_fused_attention_fp32_of_any_scale(ttmi, v_transposed, packed, a, b):
+    """|q| of size a, |k| of size b and the scale that brings the scores to size 1: no further from 64 bits than the fp32 instruction,
+    which a dense batch with row-major V runs on."""
+    B, h, S, d = 2, 3, 150, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    Q, K, V = (torch.randn(B, h, S, d, generator=g, device="cuda") for _ in range(3))
+    Q, K, scale, pitch = Q * a, K * b, 0.125 / (a * b), 152
+    v = V
+    if v_transposed:
+        v = torch.full((B, h, d, pitch), float("nan"), device="cuda")
+        v[..., :S] = V.transpose(2, 3)
+    cu = torch.tensor([0, S, 2 * S], dtype=torch.int32, device="cuda") if packed else None
+
+    def run(v, v_pitch, cu):
+        out = torch.full((B * S, h * d), 9.0, device="cuda")
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", 4))
+        ok(ttmi.ttmi_fused_attention(ptr(Q), ptr(K), ptr(v), None, ptr(out), ptr(cu), B, h, S, d, v_pitch, scale, capi.F32, stream()))
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+        return out.view(B, S, h, d).permute(0, 2, 1, 3).double()
+
+    want = _attention64(Q, K, V, None, float(np.float32(scale)))
+    got, fp32 = run(v, pitch if v_transposed else 0, cu), run(V, 0, None)
+    # as in test_fused_attention_fp32_in_halves
+    assert float((got - want).abs().max()) <= 2.0**-16 * float(want.abs().max())
+    assert float((got - want).norm()) <= float((fp32 - want).norm())
+
+
 def _packed(ttmi, W):
     """fp32 weights [N, K] as ttmi_split_weights lays them out."""
     N, K = W.shape

@@ -13,8 +13,8 @@
 // Both products run on v_mfma_f32_32x32x16_f16, three instructions for one, with Q, K, V and the probabilities split in fp16 halves
 // (split_f32.h): K and V once per workgroup on their way into LDS, the others in registers.  A sub-tile is 24 instructions of 32
 // cycles where the fp32 instruction needs 64 of 64, and what bounds the kernel is then the arithmetic around them.  Scores
-// have an absolute error, so Q and K only need an upper limit; a column of V has the window of split_f32.h.  A workgroup that
-// meets a value outside starts again on v_mfma_f32_32x32x2_f32: there an instruction takes K index 0 from lanes 0-31 and K index 1
+// have an absolute error, so Q and K only need an upper limit, which depends on the scale (score_limit); a column of V has the window
+// of split_f32.h.  A workgroup that meets a value outside starts again on v_mfma_f32_32x32x2_f32: there an instruction takes K index 0 from lanes 0-31 and K index 1
 // from lanes 32-63, and accumulator register 4g+i of a lane in half h is key 8g + 4h + i, so keys (8g+i, 8g+4+i) are paired in
 // instruction (g, i), A is the 16-byte chunk (2g+h) of a V^T row, and the head dimension is paired the same way.
 // us per launch, 12 heads, fp32 instruction / halves: 20 x 100 tokens 13.6 / 10.0, 8 x 256 23.4 / 16.9, 20 x 300 74 / 43, 20 x 512 148 / 72;
@@ -47,6 +47,12 @@ __device__ __forceinline__ int tile_off(int row, int chunk) { return row * kRow 
 __device__ __forceinline__ int vt_chunk(int c) { return 2 * (c >> 2) + (c & 1); }
 __device__ __forceinline__ int vt_half(int c) { return (c >> 1) & 1; }
 
+// The absolute values of Q and K have to stay below this for the halves to hold the scores.  What the halves leave of a product is
+// 3 * 2^-22 max(|q|, 2^-14) max(|k|, 2^-14) at most (split_f32.h): besides 3 * 2^-22 of the sum of |q k|, which the fp32 instruction leaves
+// as well, that is 64 * 3 * 2^-36 of the largest |q| or |k|, times the scale in an exponent: 2^-20 below this limit.  Of scales above 2^22 even
+// values below 2^-14 would leave more.
+inline float score_limit(float scale) { return scale <= 0x1p22f ? std::min(kSplitLargest, 256.f / scale) : 0.f; }
+
 template <int NW>
 constexpr int lds_bytes() {
   constexpr int tiles = 4 * kBKV * kRow + 2 * kBKV * 4, outb = NW * 32 * (kD + 4) * 4;
@@ -59,7 +65,7 @@ constexpr int lds_bytes() {
 template <int NW, bool VT, bool SPLIT>
 __device__ __forceinline__ bool attend(char* const smem, const float* __restrict__ qb, const float* __restrict__ kb, const float* __restrict__ vb,
                                        const float* __restrict__ mask, int q0, int kv_len, int v_pitch, float scale_log2e, float inv_scale,
-                                       floatx16 (&ot)[2], float& l_run) {
+                                       float qk_limit, floatx16 (&ot)[2], float& l_run) {
   constexpr int kPieces = 1024 / (NW * 64);  // 16-byte pieces of a K (V^T) tile per thread: 64 rows of 16
   constexpr int kTile = kBKV * kRow;         // 16 KB
   const int tid = threadIdx.x, lane = tid & 63;
@@ -69,7 +75,7 @@ __device__ __forceinline__ bool attend(char* const smem, const float* __restrict
   // Q fragments: B operand of the first product.  fp32: chunk 2kk+lhalf of the lane's query row; halves: eight values of the
   // head dimension, hi and lo.
   u32x4 qf[8];
-  float largest = 0.f;  // of Q and K: only their upper limit counts, since a score's error is absolute
+  float largest = 0.f;  // of Q and K
   {
     const int qi = q0 + lrow;
 #pragma unroll
@@ -312,7 +318,7 @@ __device__ __forceinline__ bool attend(char* const smem, const float* __restrict
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int e = 0; e < 16; ++e) ot[t][e] = __builtin_fmaf(oc[t][e], 1.f / kSplitScale, ot[t][e]);
-    bool outside = largest >= kSplitLargest;
+    bool outside = largest >= qk_limit;
     if constexpr (VT) {
 #pragma unroll
       for (int p = 0; p < kPieces; ++p) outside = outside || split_outside(group_max<16>(v_largest[p]));
@@ -336,7 +342,7 @@ template <int NW, bool VT, bool PACKED, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void fused_attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ mask,
     float* __restrict__ out, const int32_t* __restrict__ cu, int heads, int seq, int v_pitch, float scale_log2e,
-    float inv_scale, float* __restrict__ absmax) {
+    float inv_scale, float qk_limit, float* __restrict__ absmax) {
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
   constexpr int kBQ = NW * 32;  // queries per workgroup
   // dynamic LDS (lds_bytes<NW>(), more than the 64 KB a kernel gets without asking):
@@ -368,8 +374,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   floatx16 ot[2];
   float l_run;
   bool again = true;
-  if constexpr (SPLIT) again = attend<NW, VT, true>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, ot, l_run);
-  if (again) attend<NW, VT, false>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, ot, l_run);
+  if constexpr (SPLIT) again = attend<NW, VT, true>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, qk_limit, ot, l_run);
+  if (again) attend<NW, VT, false>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, qk_limit, ot, l_run);
 
   // normalise and write: ot[t][4g+i] = O[query lrow][d = 32t + 8g + 4*lhalf + i]
   const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
@@ -426,7 +432,7 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
     TTMI_REQUIRE((int64_t)grid.x * grid.y < (1ll << 31), "attention grid too large");
     grid = dim3((unsigned)(grid.x * heads), (unsigned)batch);
   }
-  const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
+  const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale, qk_limit = score_limit(scale);
   // more than 64 KB of dynamic LDS: the limit is raised once per kernel and device
   auto launch = [&](auto kern, int threads, int lds) -> int {
     static std::mutex mu;
@@ -442,7 +448,7 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
       }
     }
     hipLaunchKernelGGL(kern, grid, dim3(threads), lds, s, q, k, v, mask, out, cu, (int)heads, (int)seq, (int)v_seq_pitch, sl2,
-                       inv_scale, absmax);
+                       inv_scale, qk_limit, absmax);
     return 0;
   };
   const bool vt = v_seq_pitch > 0, packed = cu != nullptr;
