@@ -1525,3 +1525,66 @@ def test_packed_weights_outside_the_window(ttmi, M, N, K):
     finite = torch.isfinite(want)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got[~finite & ~torch.isnan(want)], want[~finite & ~torch.isnan(want)])
     assert bool(((got - want).abs() <= bound)[finite].all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 8, 32), (100, 776, 96), (129, 2304, 544), (129, 2304, 768), (264, 768, 3072), (387, 3072, 768), (1000, 1536, 160), (1999, 768, 768),
+                                   (2000, 3072, 128), (2500, 2304, 768)])
+def test_packed_weights_outside_the_window_beside_others(ttmi, M, N, K):
+    """What a row of either operand holds changes no other row's results, whatever tile they share: rows and columns outside the window
+    are right to fp32 accuracy, and all others keep their bits."""
+    import ctypes
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A, W = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 0.02
+
+    def run(A, W):
+        C = torch.full((M, N), 7.0, device="cuda")
+        ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, W)), ptr(C), M, N, K, K, K, N, capi.EPI_F32_OUT, ctypes.byref(_epi()), capi.F32_PACKED, stream()))
+        return C
+
+    alone = run(A, W)
+    rows, cols = torch.zeros(M, dtype=torch.bool, device="cuda"), torch.zeros(N, dtype=torch.bool, device="cuda")
+    rows[torch.tensor([0, 17, M // 2, M - 1])] = True
+    cols[torch.tensor([1, 2, 5, N - 2])] = True
+    A2, W2 = A.clone(), W.clone()
+    A2[rows] *= torch.tensor([1e-9, 1e5, 1e-6, 1e4], device="cuda")[:, None]
+    W2[cols] *= torch.tensor([1e-38, 1e30, 1e-7, 1e8], device="cuda")[:, None]  # (the first are subnormal)
+    got = run(A2, W2)
+    other = ~rows[:, None] & ~cols[None, :]
+    assert torch.equal(got[other], alone[other])
+    want = A2.double() @ W2.double().T
+    bound = (A2.double().abs() @ W2.double().abs().T) * (K + 8) * 2.0**-24 + 1e-37
+    assert bool(((got.double() - want).abs() <= bound)[~other].all())
+    A2[17, 3], W2[5, 1] = float("inf"), float("nan")
+    assert torch.equal(run(A2, W2)[other], alone[other])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,h", [(1, 37, 16), (7, 130, 12), (2, 387, 16), (20, 100, 12)])
+def test_packed_weights_head_split_outside_the_window(ttmi, B, S, h):
+    """The same through the head split and the column pass of a transposed V."""
+    import ctypes
+    d, H = 64, h * 64
+    g = torch.Generator(device="cuda").manual_seed(S + h)
+    A, W, bias = torch.randn(B * S, H, generator=g, device="cuda"), torch.randn(3 * H, H, generator=g, device="cuda") * 0.02, torch.randn(3 * H, generator=g, device="cuda")
+    pitch = (S + 7) // 8 * 8
+
+    def run(A, W):
+        q, k = (torch.empty(B, h, S, d, device="cuda") for _ in range(2))
+        v = torch.zeros(B, h, d, pitch, device="cuda")
+        args = _epi(bias=bias, q=q, k=k, v=v, seq=S, heads=h, head_dim=d, v_seq_pitch=pitch)
+        ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, W)), None, B * S, 3 * H, H, H, H, 3 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args), capi.F32_PACKED, stream()))
+        return torch.stack([q, k, v[..., :S].transpose(2, 3)]).permute(1, 3, 0, 2, 4).reshape(B * S, 3 * H)
+
+    alone = run(A, W)
+    A2, W2 = A.clone(), W.clone()
+    A2[11] *= 1e-8
+    A2[B * S - 1] *= 1e5
+    W2[H + 7] *= 1e-6
+    W2[3 * H - 3] *= 1e-6
+    got, other = run(A2, W2), torch.ones(B * S, 3 * H, dtype=torch.bool, device="cuda")
+    other[11] = other[B * S - 1] = other[:, H + 7] = other[:, 3 * H - 3] = False
+    assert torch.equal(got[other], alone[other])
+    want = A2.double() @ W2.double().T + bias.double()
+    bound = (A2.double().abs() @ W2.double().abs().T + bias.double().abs()) * (H + 8) * 2.0**-24
+    assert bool(((got.double() - want).abs() <= bound)[~other].all())

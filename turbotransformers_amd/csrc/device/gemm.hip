@@ -63,8 +63,9 @@ static int packed_operand(int* dtype, int64_t k, int64_t ldb, bool* packed) {
   return 0;
 }
 
-// The halves of packed weights (split_f32.h) behind their fp32 rows, and per row whether its largest value is outside the window
-// in which they hold it.  Once per weight: one workgroup per row, 16 bytes of it per thread and turn.
+// The halves of packed weights (split_f32.h) behind their fp32 rows, and a flag per row: the power of two that its halves were scaled by,
+// 0 for rows in the window, kSplitOutside for rows with an infinity.  Once per weight: one workgroup per row, 16 bytes of it per
+// thread and turn.
 static __global__ __launch_bounds__(256) void split_weights_kernel(float* __restrict__ packed, int n, int k) {
   __shared__ float part[256 / kWave];
   const int row = blockIdx.x;
@@ -73,18 +74,24 @@ static __global__ __launch_bounds__(256) void split_weights_kernel(float* __rest
   float largest = 0.f;
   for (int col = threadIdx.x * 4; col < k; col += 1024) {
     const float4 x = *reinterpret_cast<const float4*>(src + col);
-    const uint2 hi = make_uint2(split_hi(x.x, x.y), split_hi(x.z, x.w));
-    char* group = dst + (col / TTMI_PACKED_WEIGHT_K) * (TTMI_PACKED_WEIGHT_K * 4) + (col % TTMI_PACKED_WEIGHT_K) * 2;
-    *reinterpret_cast<uint2*>(group) = hi;
-    *reinterpret_cast<uint2*>(group + TTMI_PACKED_WEIGHT_K * 2) = make_uint2(split_lo(hi.x, x.x, x.y), split_lo(hi.y, x.z, x.w));
     split_max(largest, x.x, x.y);
     split_max(largest, x.z, x.w);
   }
   largest = group_max<kWave>(largest);
   if (threadIdx.x % kWave == 0) part[threadIdx.x / kWave] = largest;
   __syncthreads();
-  if (threadIdx.x == 0)
-    reinterpret_cast<int*>(packed + 2 * (int64_t)n * k)[row] = split_outside(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+  largest = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  const int flag = !split_outside(largest) ? 0 : largest == __builtin_inff() ? kSplitOutside : 1 - __builtin_amdgcn_frexp_expf(largest);
+  const int scale = flag == kSplitOutside ? 0 : flag;  // (the row's largest value comes to between 1 and 2)
+  for (int col = threadIdx.x * 4; col < k; col += 1024) {
+    float4 x = *reinterpret_cast<const float4*>(src + col);
+    x = make_float4(__builtin_ldexpf(x.x, scale), __builtin_ldexpf(x.y, scale), __builtin_ldexpf(x.z, scale), __builtin_ldexpf(x.w, scale));
+    const uint2 hi = make_uint2(split_hi(x.x, x.y), split_hi(x.z, x.w));
+    char* group = dst + (col / TTMI_PACKED_WEIGHT_K) * (TTMI_PACKED_WEIGHT_K * 4) + (col % TTMI_PACKED_WEIGHT_K) * 2;
+    *reinterpret_cast<uint2*>(group) = hi;
+    *reinterpret_cast<uint2*>(group + TTMI_PACKED_WEIGHT_K * 2) = make_uint2(split_lo(hi.x, x.x, x.y), split_lo(hi.y, x.z, x.w));
+  }
+  if (threadIdx.x == 0) reinterpret_cast<int*>(packed + 2 * (int64_t)n * k)[row] = flag;
 }
 
 static int gemm_bias_layer_norm_impl(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,

@@ -142,11 +142,11 @@ struct GemmArgs {
   int split_col, split_tiles;
   // fp32 products with packed weights (gemm_split.h): b is their fp32 part, these the halves and the per-row flags; else null
   const char* b_split;
-  const int* b_outside;
+  const int* b_flags;
 };
 inline void use_packed_weights(GemmArgs& g) {
   g.b_split = g.b + (int64_t)g.n * g.k * 4;
-  g.b_outside = reinterpret_cast<const int*>(g.b + (int64_t)g.n * g.k * 8);
+  g.b_flags = reinterpret_cast<const int*>(g.b + (int64_t)g.n * g.k * 8);
 }
 
 // ------------------------------------------------------------------------ epilogues -----
@@ -418,7 +418,8 @@ struct EpiQkvSplit {
     const uint32_t w = div_hidden.div(n);
     const uint32_t rem = n - w * hidden;
     const uint32_t head = div_dim.div(rem);
-    T* base = (w == 0) ? q : (w == 1 ? k : v);
+    T *const to_q = q, *const to_k = k, *const to_v = v;  // (read in a branch, they would be indexed in scratch memory)
+    T* const base = (w == 0) ? to_q : (w == 1 ? to_k : to_v);
     return base + (int64_t)head * seq * dim + (rem - head * dim);
   }
   __device__ __forceinline__ int64_t row_part(int m) const {

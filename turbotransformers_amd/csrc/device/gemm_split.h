@@ -92,8 +92,8 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
   float largest[PASSES];
 #pragma unroll
   for (int p = 0; p < PASSES; ++p) largest[p] = 0.f;
-  bool outside = false;  // B's rows: the packed weights say so
-  for (int r = tid; r < BN; r += NT) outside = outside || g.b_outside[min(n0 + r, g.n - 1)] != 0;
+  static_assert(BN <= NT && KG * NW * (int)sizeof(int) <= 256, "a column per thread, an answer per wavefront");
+  const int column_flag_here = tid < BN ? g.b_flags[min(n0 + tid, g.n - 1)] : 0;
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef __attribute__((address_space(3))) char lds_char;
   lds_char* lds0 = reinterpret_cast<lds_char*>(reinterpret_cast<uintptr_t>(smem));
@@ -232,42 +232,85 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
       }
     asm volatile("s_nop 7");  // (the matrix instructions are inline asm: no hazard is seen between them and the zeroing)
   };
-  // The tile with the fp32 instruction, from operands in fp32: seldom, and not in a hurry.
-  auto fp32_loop = [&](auto swap_tag) __attribute__((always_inline)) {
-    constexpr int B_PASSES = BN / ROWS;
-    static_assert(BN % ROWS == 0, "a pass loads rows of one operand");
-    clear();
+  floatx4 value[RB][CB];  // what the tile's (and group's) K steps add up to
+  auto sum = [&](int i, int j, int e) __attribute__((always_inline)) {
+    return __builtin_fmaf(acc_read(cross[i][j][e]), 1.f / kSplitScale, acc_read(acc[i][j][e]));
+  };
+  // What the main loop leaves to do where a row or a column of the tile is outside the window (split_f32.h): columns are scaled back, and
+  // rows of A, like columns with an infinity, are formed again with the fp32 instruction, from operands in fp32: the 16 x 16 blocks that
+  // one crosses, of which its elements are taken.  Every other element keeps its bits, whatever shares its tile.  Each wavefront for
+  // itself, straight from global memory: seldom, and in few registers.  us per launch, nothing / one row / every 32nd row of A / every
+  // 32nd column outside, and all of it on the fp32 tiles: 128 x 2304 x 768 8 / 19 / 19 / 8, 9.6; 2000 x 3072 x 768 31 / 64 / 103 / 32, 72;
+  // 10240 x 768 x 3072 144 / 242 / 554 / 147, 332.
+  constexpr int TOPS = 256, FLAGS = TOPS + KG * BM * 4, EXACT = FLAGS + BN * 4;  // behind the wavefronts' answers
+  static_assert(EXACT + KG * BM * BN * 4 <= KG * split_lds_bytes<BM, BN, SB>(), "a tile in fp32 beside what is known about its rows");
+  float* const tops = reinterpret_cast<float*>(lds + TOPS);             // the largest value of each row in each group's part of K
+  int* const column_flags = reinterpret_cast<int*>(lds + FLAGS);       // of the columns: split_f32.h
+  auto fp32_blocks = [&](auto swap_tag) __attribute__((always_inline)) {
+    constexpr bool SWAP = decltype(swap_tag)::value;
+    constexpr int PER_ROW = SWAP ? 1 : 4, PER_COL = SWAP ? 4 : 1;  // a lane holds a row's four columns of a block, or the other way round
+    static_assert(RB * PER_ROW <= 32, "a bit per row of a lane");
+    floatx4* const exact_at = reinterpret_cast<floatx4*>(lds + EXACT) + (group * NW + wave) * (RB * CB * kWave) + lane;
+    auto row_outside = [&](int i, int e) __attribute__((always_inline)) {
+      const int row = wm0 + i * 16 + (SWAP ? lrow : lgrp * 4 + e);
+      float top = tops[row];
+#pragma unroll
+      for (int o = 1; o < KG; ++o) top = fmaxf(top, tops[o * BM + row]);
+      return split_outside(top);
+    };
+    auto column_flag = [&](int j, int e) __attribute__((always_inline)) { return column_flags[wn0 + j * 16 + (SWAP ? lgrp * 4 + e : lrow)]; };
+    uint32_t row_bits = 0, row_blocks = 0, col_blocks = 0;  // of this lane; of the wavefront's blocks
+#pragma unroll
+    for (int q = 0; q < RB * PER_ROW; ++q) {
+      const bool out = row_outside(q / PER_ROW, q % PER_ROW);
+      row_bits |= (uint32_t)out << q;
+      row_blocks |= (uint32_t)(__ballot(out) != 0) << (q / PER_ROW);
+    }
+#pragma unroll
+    for (int q = 0; q < CB * PER_COL; ++q) {
+      const bool out = column_flag(q / PER_COL, q % PER_COL) == kSplitOutside;
+      col_blocks |= (uint32_t)(__ballot(out) != 0) << (q / PER_COL);
+    }
 #pragma unroll 1
-    for (int s = 0; s < ksteps; ++s) {
-      __syncthreads();
+    for (int i = 0; i < RB; ++i) {
+      const uint32_t blocks = (row_blocks >> i & 1) != 0 ? ~0u : col_blocks;
+      if (blocks == 0) continue;
+      floatx4 exact[CB];
+#pragma unroll
+      for (int j = 0; j < CB; ++j) exact[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const char* const a = g.a + k_lo + (size_t)min(m0 + wm0 + i * 16 + lrow, g.m - 1) * lda_bytes + lgrp * 16;
+      const char* const b = g.b + k_lo + lgrp * 16;
 #pragma unroll 1
-      for (int p = 0; p < PASSES + B_PASSES; ++p) {
-        const int row = (p < PASSES ? p : p - PASSES) * ROWS + sub;
-        const char* src = p < PASSES ? g.a + (int64_t)min(m0 + row, g.m - 1) * lda_bytes : g.b + (int64_t)min(n0 + row, g.n - 1) * ldb_bytes;
-        floatx4 x = *reinterpret_cast<const floatx4*>(src + (s < valid ? k_lo + s * kRowBytes : 0u) + kq * 16);
-        if (s >= valid) x = floatx4{0.f, 0.f, 0.f, 0.f};
-        *reinterpret_cast<floatx4*>(smem + (p < PASSES ? 0 : B_BASE) + row * kRowBytes + ((kq ^ split_swizzle(sub)) << 4)) = x;
+      for (int at = 0; at < valid * kRowBytes; at += 64) {  // a lane's four values of K of sixteen
+        const floatx4 fa = *reinterpret_cast<const floatx4*>(a + at);
+        floatx4 fb[CB];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) fb[j] = *reinterpret_cast<const floatx4*>(b + (uint32_t)min(n0 + wn0 + j * 16 + lrow, g.n - 1) * ldb_bytes + at);
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+          if ((blocks >> j & 1) == 0) continue;
+#pragma unroll
+          for (int part = 0; part < 4; ++part)
+            exact[j] = SWAP ? __builtin_amdgcn_mfma_f32_16x16x4f32(fb[j][part], fa[part], exact[j], 0, 0, 0)
+                            : __builtin_amdgcn_mfma_f32_16x16x4f32(fa[part], fb[j][part], exact[j], 0, 0, 0);
+        }
       }
-      __syncthreads();
 #pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        Chunk fa[RB], fb[CB];
+      for (int j = 0; j < CB; ++j) exact_at[(i * CB + j) * kWave] = exact[j];
+    }
 #pragma unroll
-        for (int i = 0; i < RB; ++i) fa[i] = *reinterpret_cast<const Chunk*>(smem + (((get_a - lds_base) ^ (half * 64)) + i * (16 * kRowBytes)));
+    for (int i = 0; i < RB; ++i) {
 #pragma unroll
-        for (int j = 0; j < CB; ++j) fb[j] = *reinterpret_cast<const Chunk*>(smem + (((get_b - lds_base) ^ (half * 64)) + j * (16 * kRowBytes)));
+      for (int j = 0; j < CB; ++j) {
+        const floatx4 exact = exact_at[(i * CB + j) * kWave];  // (its lane's own: nothing is waited for; unspecified where no element is taken)
 #pragma unroll
-        for (int part = 0; part < 4; ++part)
-#pragma unroll
-          for (int i = 0; i < RB; ++i)
-#pragma unroll
-            for (int j = 0; j < CB; ++j) {
-              if constexpr (decltype(swap_tag)::value) RingMma<float>::run(fb[j], fa[i], acc[i][j], part);
-              else RingMma<float>::run(fa[i], fb[j], acc[i][j], part);
-            }
+        for (int e = 0; e < 4; ++e) {
+          const int flag = column_flag(j, SWAP ? e : 0);
+          const bool out = ((row_bits >> (SWAP ? i : i * 4 + e) & 1) != 0) | (flag == kSplitOutside);
+          value[i][j][e] = out ? exact[e] : __builtin_ldexpf(value[i][j][e], -flag);
+        }
       }
     }
-    asm volatile("s_nop 15\n\ts_nop 15");
   };
   auto k_loop = [&](auto swap_tag) __attribute__((always_inline)) {
     clear();
@@ -301,11 +344,18 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
       for (int s = 0; turn(template_int<0>{}, s) && turn(template_int<1>{}, s + 1) && turn(template_int<2>{}, s + 2) && turn(template_int<3>{}, s + 3); s += 4) {}
     }
     asm volatile("s_nop 15\n\ts_nop 15");
-#pragma unroll
-    for (int p = 0; p < PASSES; ++p) outside = outside || split_outside(group_max<8>(largest[p]));
-    // (every stage has been read, and the loads past the last step are waited for: the first words of LDS hold the wavefronts' answers)
+    bool outside = column_flag_here != 0;
+    // (every stage has been read, and the loads past the last step are waited for: the front of LDS holds the wavefronts' answers
+    // and what they are about)
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PASSES; ++p) {
+      const float top = group_max<8>(largest[p]);
+      outside = outside || split_outside(top);
+      if (kq == 0) tops[group * BM + p * ROWS + sub] = top;
+    }
+    if (group == 0 && tid < BN) column_flags[tid] = column_flag_here;
     int* const answers = reinterpret_cast<int*>(lds);
     const bool any = __ballot(outside) != 0;
     if (lane == 0) answers[group * NW + wave] = any;
@@ -313,17 +363,18 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
     int again = 0;
 #pragma unroll
     for (int w = 0; w < KG * NW; ++w) again |= answers[w];
-    if (__builtin_amdgcn_readfirstlane(again) != 0) fp32_loop(swap_tag);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) value[i][j] = floatx4{sum(i, j, 0), sum(i, j, 1), sum(i, j, 2), sum(i, j, 3)};
+    if (__builtin_amdgcn_readfirstlane(again) != 0) fp32_blocks(swap_tag);
   };
 
-  auto sum = [&](int i, int j, int e) __attribute__((always_inline)) {
-    return __builtin_fmaf(acc_read(cross[i][j][e]), 1.f / kSplitScale, acc_read(acc[i][j][e]));
-  };
   // the groups' sums meet: those of the others pass through LDS, lane by lane
   floatx4 other[KG > 1 ? RB : 1][KG > 1 ? CB : 1];
   auto read = [&](int i, int j, int e) __attribute__((always_inline)) {
-    if constexpr (KG > 1) return sum(i, j, e) + other[i][j][e];
-    else return sum(i, j, e);
+    if constexpr (KG > 1) return value[i][j][e] + other[i][j][e];
+    else return value[i][j][e];
   };
   auto meet = [&]() __attribute__((always_inline)) {
     if constexpr (KG > 1) {
@@ -334,7 +385,7 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
-          for (int j = 0; j < CB; ++j) at[(group - 1) * PER_GROUP + (i * CB + j) * kWave] = floatx4{sum(i, j, 0), sum(i, j, 1), sum(i, j, 2), sum(i, j, 3)};
+          for (int j = 0; j < CB; ++j) at[(group - 1) * PER_GROUP + (i * CB + j) * kWave] = value[i][j];
       }
       __syncthreads();
       if (group != 0) return false;

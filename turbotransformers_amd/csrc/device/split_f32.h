@@ -14,10 +14,12 @@
 namespace ttmi {
 
 // The window of a row's largest absolute value in which the halves hold a product to fp32 accuracy.  Above, lo could
-// overflow; below, the subnormal step of lo, 2^-24 / 2^16, comes near 2^-24 of the row's largest value.  A tile one of whose
-// rows is outside (and not all zero) is computed again with the fp32 instruction, infinities included.
+// overflow; below, the subnormal step of lo, 2^-24 / 2^16, comes near 2^-24 of the row's largest value.  Rows of a weight that are outside
+// (and not all zero) are scaled by a power of two on their way into the halves, which their flag holds; rows with an infinity and rows of
+// the other operand that are outside are formed again with the fp32 instruction.
 constexpr float kSplitScale = 65536.f, kSplitLargest = 2048.f, kSplitSmallest = 0x1p-13f;
-__device__ __forceinline__ bool split_outside(float largest) { return !(largest == 0.f || (largest >= kSplitSmallest && largest < kSplitLargest)); }
+constexpr int kSplitOutside = 1 << 30;  // beside the powers of two that rows of packed weights are scaled by
+__device__ __forceinline__ bool split_outside(float largest) { return (largest != 0.f) & !((largest >= kSplitSmallest) & (largest < kSplitLargest)); }
 
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
