@@ -1415,6 +1415,39 @@ def test_fused_attention_fp32_of_any_scale(ttmi, v_transposed, packed, a, b):
     assert float((got - want).norm()) <= float((fp32 - want).norm())
 
 
+@pytest.mark.parametrize("waves", [-1, 4, 8])
+@pytest.mark.parametrize("form", ["V transposed", "packed", "packed, V transposed"])
+@pytest.mark.parametrize("keys", [1, 2, 7, 16, 31, 32, 33])
+def test_fused_attention_fp32_of_few_keys(ttmi, waves, form, keys):
+    """Sums of a few products are hardly rounded: no further from 64 bits than the fp32 instruction, which a dense batch with row-major V
+    runs on, whether the scores are small or not; beside a long sequence of a packed batch too."""
+    B, h, d, packed = 40, 3, 64, "packed" in form
+    lens = [keys] * B + ([150] if packed else [])
+    S, pitch = max(lens), (max(lens) + 7) // 8 * 8
+    g = torch.Generator(device="cuda").manual_seed(keys)
+    for size in (0.3, 1.0):
+        Q, K, V = (torch.randn(len(lens), h, S, d, generator=g, device="cuda") for _ in range(3))
+        Q, K = Q * size, K * size
+        Vt = torch.full((len(lens), h, d, pitch), float("nan"), device="cuda")
+        Vt[..., :S] = V.transpose(2, 3)
+        cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda") if packed else None
+
+        def run(Q, K, v, B, S, v_pitch, cu, waves):
+            out = torch.full((sum(lens) if cu is not None else B * S, h * d), 9.0, device="cuda")
+            ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", waves))
+            ok(ttmi.ttmi_fused_attention(ptr(Q), ptr(K), ptr(v), None, ptr(out), ptr(cu), B, h, S, d, v_pitch, 0.125, capi.F32, stream()))
+            ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+            return out[:40 * keys].view(40, keys, h, d).permute(0, 2, 1, 3).double()
+
+        few = [x[:40, :, :keys].contiguous() for x in (Q, K, V)]
+        want = _attention64(*few, None)
+        got = run(Q, K, V if form == "packed" else Vt, len(lens), S, 0 if form == "packed" else pitch, cu, waves)
+        fp32 = run(*few, 40, keys, 0, None, 4)
+        error, before = float((got - want).norm()), float((fp32 - want).norm())
+        # (the split over the wavefronts of a workgroup adds the shares in another order: as many roundings, not the same ones)
+        assert error <= before * 1.02, (error, before)
+
+
 def _packed(ttmi, W):
     """fp32 weights [N, K] as ttmi_split_weights lays them out."""
     N, K = W.shape

@@ -47,6 +47,13 @@ __device__ __forceinline__ int tile_off(int row, int chunk) { return row * kRow 
 __device__ __forceinline__ int vt_chunk(int c) { return 2 * (c >> 2) + (c & 1); }
 __device__ __forceinline__ int vt_half(int c) { return (c >> 1) & 1; }
 
+// Up to this many keys the fp32 instruction it is: sums of so few products are hardly rounded, and what the halves leave of the operands is
+// more.  Error against 64 bits, relative to the result (2-norms), scores of size 0.1, fp32 instruction / halves: 1 key 0 / 4.4e-8, 4 keys 6.6e-8 /
+// 8.4e-8, 16 keys 9.5e-8 / 9.7e-8, 32 keys 1.2e-7 / 1.1e-7; scores of size 1, 1 key 0.9e-8 / 4.5e-8, 4 keys 1.1e-7 / 1.1e-7, 32 keys 2.4e-7 / 1.6e-7.
+// It is no slower there: us per launch, 12 heads, halves / fp32 instruction on one sub-tile: 20 sequences of 10 tokens 6.3 / 5.8, of 30 6.7 /
+// 6.2, 32 of 5 to 30 9.4 / 6.5.  (A form of its own for them: 31 of 20 and one of 300 tokens 18.9 here, 20.2 so.)
+constexpr int kFewKeys = 32;
+
 // The absolute values of Q and K have to stay below this for the halves to hold the scores.  What the halves leave of a product is
 // 3 * 2^-22 max(|q|, 2^-14) max(|k|, 2^-14) at most (split_f32.h): besides 3 * 2^-22 of the sum of |q k|, which the fp32 instruction leaves
 // as well, that is 64 * 3 * 2^-36 of the largest |q| or |k|, times the scale in an exponent: 2^-20 below this limit.  Of scales above 2^22 even
@@ -201,6 +208,7 @@ __device__ __forceinline__ bool attend(char* const smem, const float* __restrict
     const float* mk = reinterpret_cast<const float*>(smem + 4 * kTile) + STAGE * kBKV;
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {  // two 32-key sub-tiles
+      if (!SPLIT && sub == 1 && kv_len <= kFewKeys) break;
       const int sk = sub * 32;
       // st[4g+i] = score of (key sk + 8g + 4*lhalf + i, query lrow), seeded with mask/scale
       floatx16 st;
@@ -374,7 +382,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
   floatx16 ot[2];
   float l_run;
   bool again = true;
-  if constexpr (SPLIT) again = attend<NW, VT, true>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, qk_limit, ot, l_run);
+  if constexpr (SPLIT)
+    if (kv_len > kFewKeys) again = attend<NW, VT, true>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, qk_limit, ot, l_run);
   if (again) attend<NW, VT, false>(smem, qb, kb, vb, mb, q0, kv_len, v_pitch, scale_log2e, inv_scale, qk_limit, ot, l_run);
 
   // normalise and write: ot[t][4g+i] = O[query lrow][d = 32t + 8g + 4*lhalf + i]
