@@ -330,7 +330,9 @@ TTMI_API int ttmi_gemm_batched_heads(const void* a, const void* b, void* c, int6
  * read (pad rows need not be zero) and `out` is packed [sum(len), h*64]
  * (…smart_batch.cpp:368-392).  `v_seq_pitch` = 0: v is [B,h,S,64]; > 0: v is stored transposed,
  * [B,h,64,v_seq_pitch] with v_seq_pitch a multiple of 8 and >= S, the layout the QKV_SPLIT
- * epilogues write when asked to (the faster path: tiles of V^T are copied, not scattered). */
+ * epilogues write when asked to (the faster path: tiles of V^T are copied, not scattered).
+ * fp32 of more than 32 keys, unless v is [B,h,S,64] of a dense batch, may be formed as with TTMI_F32_PACKED (below): scores to within 2^-20
+ * besides 3 * 2^-22 of scale * sum |q k|, probabilities and values as the operands there. */
 TTMI_API int ttmi_fused_attention(const void* q, const void* k, const void* v, const float* mask, void* out,
                                   const int32_t* cu_seqlens, int64_t batch, int64_t heads, int64_t seq,
                                   int64_t head_dim, int64_t v_seq_pitch, float scale, int dtype, void* stream);
@@ -395,8 +397,12 @@ typedef struct ttmi_epilogue_args {
  * floats (k a multiple of TTMI_PACKED_WEIGHT_K), written by the caller, and behind them what ttmi_split_weights computes from
  * them, TTMI_PACKED_WEIGHT_FLOATS(n, k) floats in all, 16-byte aligned.  ttmi_gemm_fused, ttmi_layer_norm_gemm_fused,
  * ttmi_gemm_bias_layer_norm[_static] and ttmi_gemm_describe take them as their weight with dtype TTMI_F32_PACKED (ldb = k);
- * everything else about such a call is as with TTMI_F32.  Infinities, NaNs and rows of any magnitude are allowed: what the halves
- * do not hold is computed from the fp32 rows.  No counterpart in the reference (cuBLAS takes its weights as they are). */
+ * everything else about such a call is as with TTMI_F32.  Infinities, NaNs and rows of any magnitude are allowed, and what a row
+ * holds changes no other row's results.  Accuracy: a product a b of two values other than zero enters the sums to within
+ * 3 * 2^-22 max(|a|, 2^-14) max(|b|, 2^-14).  Rows of w whose largest value is below 2^-13 or from 2^11 on are scaled by a power of two first,
+ * such rows of the other operand (or of a part of K, where K is cut) multiplied in fp32.  Over random operands the sums are nearer to
+ * 64 bits than with TTMI_F32; a single value may lose its last bit, and one far below the largest of its row more.  Callers who need
+ * every bit of the operands pass TTMI_F32.  No counterpart in the reference (cuBLAS takes its weights as they are). */
 #define TTMI_PACKED_WEIGHT_K 32
 #define TTMI_PACKED_WEIGHT_FLOATS(n, k) (2 * (n) * (k) + (n))
 TTMI_API int ttmi_split_weights(void* packed, int64_t n, int64_t k, void* stream);

@@ -1621,3 +1621,96 @@ def test_packed_weights_head_split_outside_the_window(ttmi, B, S, h):
     want = A2.double() @ W2.double().T + bias.double()
     bound = (A2.double().abs() @ W2.double().abs().T + bias.double().abs()) * (H + 8) * 2.0**-24
     assert bool(((got.double() - want).abs() <= bound)[~other].all())
+
+
+def _held(x):
+    """The size at which the halves hold a value: as if none but zero were smaller than 2^-14."""
+    return torch.where(x == 0, 0.0, x.double().abs().clamp(min=2.0**-14))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [100, 2000])
+@pytest.mark.parametrize("rest", [1e-2, 1e-4, 1e-6, 1e-7, 1e-10, 1e-13])
+@pytest.mark.parametrize("operand", ["A", "W"])
+def test_packed_weights_small_values_beside_large(ttmi, M, rest, operand):
+    """Rows whose largest value is in the window while the others are not, the large one beside a zero: 3 * 2^-22 max(|a|, 2^-14)
+    max(|b|, 2^-14) of each product, and the rounding of the sums as in _split_error_bound."""
+    import ctypes
+    N, K = 776, 416
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A, W = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda") * 0.02
+    small, other = (A, W) if operand == "A" else (W, A)
+    small *= rest / (1.0 if operand == "A" else 0.02)
+    small[:, 7], other[:, 7] = 1000.0, 0.0
+    C = torch.empty(M, N, device="cuda")
+    ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, W)), ptr(C), M, N, K, K, K, N, capi.EPI_F32_OUT, ctypes.byref(_epi()), capi.F32_PACKED, stream()))
+    want, absolute = A.double() @ W.double().T, A.double().abs() @ W.double().abs().T
+    bound = 3 * 2.0**-22 * (_held(A) @ _held(W).T) + absolute * (K / 32 + 8) * 2.0**-23
+    assert bool(((C.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [96, 768])
+def test_packed_weights_hold_single_values(ttmi, K):
+    """A unit matrix as the weight: values come out to within 2^-22 max(|x|, 2^-14), of any magnitude (rows outside the window as they are)."""
+    import ctypes
+    M = 500
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A = torch.randn(M, K, generator=g, device="cuda") * 2.0**torch.randint(-40, 9, (M, K), generator=g, device="cuda")
+    A[::50] *= 2.0**-30
+    A[::70] *= 2.0**20
+    C = torch.empty(M, K, device="cuda")
+    ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(_packed(ttmi, torch.eye(K, device="cuda"))), ptr(C), M, K, K, K, K, K, capi.EPI_F32_OUT, ctypes.byref(_epi()),
+                            capi.F32_PACKED, stream()))
+    largest = A.abs().amax(1, keepdim=True)
+    outside = (largest < 2.0**-13) | (largest >= 2.0**11)
+    assert 5 < int(outside.sum()) < 50
+    # (a row that is cut along K has parts that may be outside by themselves: then they are exact)
+    assert bool(((C.double() - A.double()).abs() <= torch.where(outside, 0.0, 2.0**-22 * _held(A))).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [32, 64])
+@pytest.mark.parametrize("M", [40, 500, 2000])
+def test_packed_weights_of_short_sums(ttmi, M, K):
+    """Sums of a few products too are no further from 64 bits than the fp32 instruction leaves them."""
+    import ctypes
+    N = 768
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    for make in (lambda *s: torch.randn(s, generator=g, device="cuda"), lambda *s: torch.rand(s, generator=g, device="cuda"),
+                 lambda *s: torch.nn.functional.gelu(torch.randn(s, generator=g, device="cuda"))):
+        A, W = make(M, K), make(N, K) * 0.02
+        want, error = A.double() @ W.double().T, []
+        for weight, dt in ((_packed(ttmi, W), capi.F32_PACKED), (W, capi.F32)):
+            C = torch.empty(M, N, device="cuda")
+            ok(ttmi.ttmi_gemm_fused(ptr(A), ptr(weight), ptr(C), M, N, K, K, K, N, capi.EPI_F32_OUT, ctypes.byref(_epi()), dt, stream()))
+            error.append(float((C.double() - want).norm()))
+        assert error[0] <= error[1], (error, K)
+
+
+@pytest.mark.parametrize("v_transposed,packed", [(True, False), (False, True)])
+@pytest.mark.parametrize("rest", [1e-2, 1e-4, 1e-6, 1e-9])
+def test_fused_attention_fp32_large_values_at_masked_keys(ttmi, v_transposed, packed, rest):
+    """Columns of V whose largest value sits at a masked key, the others far below: 3 * 2^-22 of each probability times max(|v|, 2^-14), a
+    probability counting 2^-14 of the row's largest at least (and not more than 1), beside what the scores leave."""
+    B, h, S, d = 2, 3, 150, 64
+    g = torch.Generator(device="cuda").manual_seed(7)
+    Q, K, V = (torch.randn(B, h, S, d, generator=g, device="cuda") for _ in range(3))
+    V *= rest
+    V[:, :, 70:80] = 1000.0
+    mask = torch.zeros(B, S, device="cuda")
+    mask[:, 70:80] = -1e9
+    pitch, v = 152, V
+    if v_transposed:
+        v = torch.full((B, h, d, pitch), float("nan"), device="cuda")
+        v[..., :S] = V.transpose(2, 3)
+    cu = torch.tensor([0, S, 2 * S], dtype=torch.int32, device="cuda") if packed else None
+    out = torch.full((B * S, h * d), 9.0, device="cuda")
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", 4))
+    ok(ttmi.ttmi_fused_attention(ptr(Q), ptr(K), ptr(v), ptr(mask), ptr(out), ptr(cu), B, h, S, d, pitch if v_transposed else 0, 0.125, capi.F32, stream()))
+    ok(ttmi.ttmi_set_kernel_switch(b"TTMI_ATTENTION_WAVES", -1))
+    got = out.view(B, S, h, d).permute(0, 2, 1, 3).double()
+    P = torch.softmax(Q.double() @ K.double().transpose(2, 3) * 0.125 + mask.double()[:, None, None, :], -1)
+    P2 = torch.where(P == 0, 0.0, P + 2.0**-14 * P.amax(-1, keepdim=True))
+    bound = 2.0**-16 * (P @ V.double().abs()) + 3 * 2.0**-22 * (P2 @ _held(V))
+    assert bool(((got - P @ V.double()).abs() <= bound).all())

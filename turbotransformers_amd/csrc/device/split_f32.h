@@ -1,12 +1,18 @@
 // fp32 products on the 16-bit matrix instructions of gfx950: a value is split in two halves of 11 bits,
 //
-//   x = (hi + lo / 2^16) (1 + 2^-22),  hi = fp16(x),  lo = fp16((x - hi) * 2^16)
-//   a b = hi_a hi_b + (hi_a lo_b + lo_a hi_b) / 2^16          (what lo_a lo_b would add is below 2^-22 a b)
+//   x = hi + lo / 2^16,  hi = fp16(x),  lo = fp16((x - hi) * 2^16),  to within 2^-22 max(|x|, 2^-14)
+//   a b = hi_a hi_b + (hi_a lo_b + lo_a hi_b) / 2^16,  to within 3 * 2^-22 max(|a|, 2^-14) max(|b|, 2^-14); a zero stays one
 //
-// and the sums of the two kinds of products are kept apart.  v_mfma_f32_16x16x4_f32 takes 32 cycles for an eighth of the
-// products that v_mfma_f32_16x16x32_f16 does in 16: three of the latter are 5.3 times as fast.
-// Error against 64 bits, relative to the result (2-norms), fp32 instruction / split, activations N(0,1), weights N(0, 0.02^2): K = 768
-// 5.0e-7 / 2.0e-7, K = 3072 1.0e-6 / 3.6e-7: the long sums are rounded 32 products at a time instead of four.
+// and the sums of the two kinds of products are kept apart (split and scaling as in Ootomo and Yokota, "Recovering single precision
+// accuracy from Tensor Cores while surpassing the FP32 theoretical peak performance", 2022).  v_mfma_f32_16x16x4_f32 takes 32 cycles for
+// an eighth of the products that v_mfma_f32_16x16x32_f16 does in 16: three of the latter are 5.3 times as fast.
+//
+// What that means for accuracy.  A quarter of the 24-bit values lose their last bit, and lo_a lo_b is dropped; the sums are rounded
+// 32 products at a time instead of four.  Error against 64 bits, relative to the result (2-norms), fp32 instruction / split, activations
+// N(0,1), weights N(0, 0.02^2): K = 32 1.02e-7 / 0.92e-7, K = 96 1.8e-7 / 1.0e-7, K = 768 5.0e-7 / 2.0e-7, K = 3072 1.0e-6 / 2.0e-7; GELU of
+// N(0,1) or values of one sign the same or better.  It is not nearer where a result hangs on one product (a weight that is a unit matrix gives a
+// quarter of its inputs back with another last bit), or on elements below 2^-14 beside larger ones whose products vanish: those are
+// held to 2^-36 instead of 24 bits.
 #pragma once
 
 #include "common.h"
