@@ -88,6 +88,38 @@ def test_bert_attention_vs_huggingface(tt, B, S):
     assert len(got2) == 1 and max_abs(host(got2[0]), host(got[0])) < 1e-5
 
 
+@pytest.mark.parametrize("heads,B,S", [(12, 1, 64), (12, 6, 10), (12, 64, 1), (16, 2, 33), (16, 2, 20), (18, 1, 8), (64, 1, 64)])
+def test_bert_attention_of_few_rows(tt, heads, B, S):
+    """Few rows on both sides of the line up to which the heads' products with the output weight go with the attention; many heads take
+    no memory for a product per head (64 MiB of fp32 at 64 heads)."""
+    import turbo_transformers.turbo_transformers_cxx as cxx
+    H = heads * 64
+    g = torch.Generator(device="cuda").manual_seed(heads + S)
+    rand = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    wqkv, bqkv, wo, bo = (rand(H, 3 * H) * H**-0.5).half(), (rand(3 * H) * 0.1).half(), (rand(H, H) * H**-0.5).half(), (rand(H) * 0.1).half()
+    gamma, beta = (1 + 0.1 * rand(H)).half(), (0.1 * rand(H)).half()
+    t = lambda x: cxx.Tensor.from_dlpack(torch.utils.dlpack.to_dlpack(x))
+    attention = cxx.BertAttention(*[t(x) for x in (wqkv, bqkv, wo, bo, gamma, beta)], heads)
+
+    def run(x):
+        out = cxx.Tensor.create_empty()
+        attention(t(x), cxx.Tensor.create_empty(), out)
+        torch.cuda.synchronize()
+        return torch.utils.dlpack.from_dlpack(out.to_dlpack())
+
+    run(rand(1, 128, H).half())  # lays the weights out, and the tensors of a longer call
+    x = rand(B, S, H).half()
+    before = torch.cuda.mem_get_info()[0]
+    got = run(x)
+    if heads > 16:
+        assert before - torch.cuda.mem_get_info()[0] < 16 << 20
+    q, k, v = (x.double() @ wqkv.double() + bqkv.double()).view(B, S, 3, heads, 64).permute(2, 0, 3, 1, 4)
+    ctx = (torch.softmax(q @ k.transpose(2, 3).contiguous() / 8, -1) @ v).transpose(1, 2).reshape(B, S, H)
+    want = torch.nn.functional.layer_norm(ctx @ wo.double() + bo.double() + x.double(), (H, ), gamma.double(), beta.double(), 1e-12)
+    # the output's own rounding (2^-11 of up to 5), and of Q, K, V and the context, each averaged over 64 and more products, as much again
+    assert float((got.double() - want).abs().max()) <= 1e-2
+
+
 def test_bert_layer_vs_oracle_and_huggingface(tt, oracle):
     model, cfg = _hf_bert(1, seed=3)
     layer = model.encoder.layer[0]

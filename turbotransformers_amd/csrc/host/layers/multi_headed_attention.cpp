@@ -60,14 +60,25 @@ bool MultiHeadedAttention::UseProbsCore(int64_t head_dim, int64_t keys, std::ini
   return head_dim == 64 && keys > 0 && keys <= TTMI_PROBS_MAX_KEYS && aligned;
 }
 
-bool MultiHeadedAttention::UseProjectingCore(const Tensor& query_tensor, const WeightRef& wo, int64_t tokens, int64_t v_pitch, int dtype) const {
+bool MultiHeadedAttention::UseProjectingCore(const Tensor& query_tensor, const WeightRef& wo, int64_t batch, int64_t seq, int64_t v_pitch, int dtype) const {
   // us per forward of fp16 base, separate / projecting: 1 x 10 tokens 332 / 306, 1 x 32 343 / 311, 2 x 20 366 / 348, 1 x 64 368 / 352, 4 x
-  // 16 369 / 360, 1 x 100 437 / 444, 8 x 16 422 / 468: a product per head is as many fp32 slices, which more rows make the larger part.
-  constexpr int64_t kMostRows = 64;
+  // 16 369 / 360, 1 x 100 437 / 444, 8 x 16 422 / 468.
+  // A workgroup takes 32 queries of a head and 128 columns, and computes their attention again for each 128: beyond the two that
+  // fit a CU at a time it is more work than the product, and from one per CU on the fp32 slices, one a head, have to be small.
+  // Attention to LayerNorm, separate / projecting, weights from HBM, heads x batch x tokens (workgroups): 4 x 64 x 1 (512) 9.1 / 7.4,
+  // 8 x 16 x 4 (512) 9.6 / 8.2, 12 x 6 x 10 (432) 10.4 / 9.9, 12 x 8 x 4 (576) 10.1 / 11.7, 12 x 64 x 1 (4608) 11.2 / 36.7; 14 x 1 x 64 (196) 10.7 /
+  // 10.5, 16 x 2 x 20 (256) 11.2 / 9.9, 14 x 3 x 21 (294, 3.2 MB of slices) 11.1 / 11.4, 16 x 2 x 33 (512, 4.3 MB) 11.6 / 12.3.
+  // Beyond 1024 columns the kernel that sums takes several turns for a row: 20 x 1 x 32 13.0 / 12.3, 24 x 1 x 8 12.0 / 13.3, 32 x 1 x 64 12.8 / 25.3,
+  // 64 x 1 x 64 20.8 / 78.9.
+  constexpr int64_t kMostRows = 64, kMostColumns = 1024, kSmallSlices = 600 * 1000;
+  const int64_t tokens = batch * seq, hidden = query_tensor.shape(-1), heads = num_attention_heads_;
+  const int64_t workgroups = (seq + 31) / 32 * batch * heads * ((hidden + 127) / 128), cus = DeviceContext::GetInstance().compute_units();
+  const bool wins = tokens <= kMostRows && hidden <= kMostColumns &&
+                    (workgroups <= cus || (workgroups <= 2 * cus && heads * tokens * hidden <= kSmallSlices));
   bool aligned = true;
   for (const void* p : {query_tensor.raw(), wo.data, dense_bias_.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw()})
     aligned = aligned && reinterpret_cast<uintptr_t>(p) % 16 == 0;
-  return (dtype == TTMI_F16 || dtype == TTMI_BF16) && v_pitch > 0 && tokens <= kMostRows && query_tensor.shape(-1) <= 4096 && aligned;
+  return (dtype == TTMI_F16 || dtype == TTMI_BF16) && v_pitch > 0 && wins && aligned;
 }
 
 static int64_t RoundUp8(int64_t n) { return (n + 7) / 8 * 8; }
@@ -90,7 +101,7 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   int64_t ahead_bytes[TTMI_MAX_AHEAD];
   const size_t ranges = std::min(ahead.size(), (size_t)TTMI_MAX_AHEAD);
   for (size_t i = 0; i < ranges; ++i) ahead_data[i] = ahead[i].data, ahead_bytes[i] = ahead[i].bytes;
-  if (fused_core && seq_list == nullptr && post_layernorm && !post_add_input && UseProjectingCore(query_tensor, wo, tokens, v_pitch, dt)) {
+  if (fused_core && seq_list == nullptr && post_layernorm && !post_add_input && UseProjectingCore(query_tensor, wo, batch, seq, v_pitch, dt)) {
     if (!attention_mask.is_null()) TT_ENFORCE_EQ(attention_mask.numel(), batch * seq, "attention mask has the wrong size");
     TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
     float* partial = scratch_->partial.Reshape<float>({heads, tokens, hidden}, dev, dev_id, "gemm5/slices/Reshape");

@@ -107,7 +107,7 @@ class MultiHeadedAttention {
   bool UseProbsCore(int64_t head_dim, int64_t keys, std::initializer_list<const core::Tensor*> tensors) const;
 
   // Attention core and output projection as one launch, the heads' parts of it added up by the LayerNorm behind.
-  bool UseProjectingCore(const core::Tensor& query_tensor, const WeightRef& wo, int64_t tokens, int64_t v_pitch, int dtype) const;
+  bool UseProjectingCore(const core::Tensor& query_tensor, const WeightRef& wo, int64_t batch, int64_t seq, int64_t v_pitch, int dtype) const;
 
   // Everything after q/k/v exist, shared by the dense and the smart-batch layers.
   // `fused_core`: the one-kernel attention core runs; `v_pitch` > 0: v holds V transposed, [B,h,d,v_pitch].
