@@ -149,11 +149,17 @@ void launch_reduce_layer_norm(const float* ws, int slices, int64_t m, int64_t n,
                        (int)m, (int)n, (const T*)bias, (const T*)residual, residual_f32, (const T*)gamma, (const T*)beta, (T*)out,
                        out_f32, eps);
   };
-  // (a forward of 1 x 10 fp16 tokens, whose attention leaves a slice per head: 306 us with four slices on the way at a time, 297 with
-  // twelve; 20 x 100 tokens, two slices of 2000 rows, are 1 % slower on the kernel that has registers for twelve)
+  // How many slices are on their way at a time: a chain of waits again, but registers that more rows would miss.  Up to 64 rows, where
+  // the attention leaves a slice per head, us for both launches with four / eight / twelve / sixteen at a time, 32 tokens: 6 slices 7.7 / 7.8 / 7.8 /
+  // 7.8, 8 7.6 / 7.4 / 7.7 / 7.7, 11 8.6 / 8.4 / 8.7 / 8.7, 12 8.2 / 8.1 / 7.9 / 8.3, 15 9.7 / 9.7 / 9.5 / 9.8, 16 8.8 / 8.4 / 8.7 / 8.5; 24 and 32 slices
+  // alone 3.0 / 2.8 / 2.9 / 3.3 and 3.3 / 3.1 / 3.3 / 3.3.  384 rows, 8 slices 2.6 / 2.8 / 2.8 / 2.8; 20 x 100 tokens, two slices of 2000 rows, a
+  // forward 1 % slower with twelve.
   constexpr std::integral_constant<int, 4> four{};
-  if (n <= 1024 && slices >= 12) launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 12>{});
-  else if (n <= 1024) launch(std::integral_constant<int, 1>{}, four);
+  constexpr std::integral_constant<int, 1> row{};
+  const bool twelve = slices >= 12 && (slices < 16 || m > 64);
+  if (n <= 1024 && twelve) launch(row, std::integral_constant<int, 12>{});
+  else if (n <= 1024 && slices >= 8 && m <= 64) launch(row, std::integral_constant<int, 8>{});
+  else if (n <= 1024) launch(row, four);
   else if (n <= 2048) launch(std::integral_constant<int, 2>{}, four);
   else launch(std::integral_constant<int, 4>{}, four);
 }
