@@ -50,6 +50,7 @@ class BertIntermediate {
   // output = gelu(input * W + b)   (bert_intermediate.cpp:32-50)
   void operator()(const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
   WeightRange weight() const { return packed_.Range(dense_weight_); }
+  int64_t out_features() const { return dense_weight_.shape(1); }
 
  private:
   core::Tensor dense_weight_, dense_bias_;

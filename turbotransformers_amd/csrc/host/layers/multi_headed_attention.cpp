@@ -414,10 +414,11 @@ void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attenti
           true /* post_layernorm */, false /* post_add_input */, is_trans_weight, ahead);
 }
 
-bool WeightsLeaveCache(int64_t bytes, const Tensor& hidden) {
+bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const Tensor& hidden) {
   constexpr int64_t kStays = 200ll << 20;
-  const int64_t tensors = 16 * hidden.numel() * (int64_t)hidden.element_size();
-  return hidden.numel() > 32 * hidden.shape(-1) && bytes + tensors > kStays;
+  const int64_t width = hidden.shape(-1), rows = width > 0 ? hidden.numel() / width : 0;
+  const int64_t tensors = rows * (12 * width + ffn) * (int64_t)hidden.element_size();
+  return rows > 32 && bytes + tensors > kStays;
 }
 
 void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,

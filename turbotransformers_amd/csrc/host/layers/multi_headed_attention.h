@@ -17,6 +17,7 @@
 //   AddBiasLayerNorm(out, input) in place                             (AddBiasLayerNorm)
 #pragma once
 
+#include <algorithm>
 #include <initializer_list>
 #include <memory>
 #include <mutex>
@@ -194,23 +195,27 @@ struct EncoderLayer {
 // What the attention core of each layer may read ahead: the layer's other weights and the next layer's first one.  Nothing
 // for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
 // with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call
-// (Q, K, V, context, four of hidden states, the intermediate one, two fp32 slices of a product: 16 x rows x hidden) take their part of
-// the cache.  us per forward without / with, fp16 base (170 MB): 1 x 387 tokens 478 / 532 and 4 x 128 471 / 493 (180 MB in all), 12 x 64
-// 527 / 539 (189 MB), 20 x 100 888 / 853 (220 MB), 8 x 256 897 / 843, 40 x 128 1573 / 1518.
+// (Q, K, V, context, four of hidden states, two fp32 slices of a product and the intermediate one: rows x (12 x hidden + ffn)) take their
+// part of the cache.  us per forward without / with, fp16 base (170 MB): 1 x 387 tokens 478 / 532 and 4 x 128 471 / 493 (180 MB in all), 12 x 64
+// 527 / 539 (189 MB), 20 x 100 888 / 853 (220 MB), 8 x 256 897 / 843, 40 x 128 1573 / 1518.  The line holds for other widths (MB in
+// all): 5 layers of 1280 / ffn 5120 1 x 128 221 / 224 (192), 4 x 128 328 / 310 (207), 20 x 100 681 / 655 (265), though 12 x 64 373 / 382 (217); 16 of
+// 768 / 1536 4 x 128 591 / 622 (154), 20 x 100 918 / 916 (185); 9 of 768 / 6144 1 x 128 373 / 365 (205), 12 x 64 558 / 522 (223); 32 of 512 /
+// 2048 1 x 128 926 / 946 (194), 4 x 128 1071 / 1051 (200), 8 x 256 1569 / 1525 (224).
 // Nor for fp32 products of up to 32 rows, which take the fp32 weights as they are, all of a workgroup's share at once.
-bool WeightsLeaveCache(int64_t bytes, const core::Tensor& hidden);
+bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const core::Tensor& hidden);
 template <typename Attention>
 std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<EncoderLayer<Attention>>& layers, const core::Tensor& hidden) {
   std::vector<std::vector<WeightRange>> ahead(layers.size());
-  int64_t bytes = 0;
+  int64_t bytes = 0, ffn = 0;
   for (size_t i = 0; i < layers.size(); ++i) {
     ahead[i] = {layers[i].attention->dense_weight(), layers[i].intermediate->weight(), layers[i].output->weight()};
     const WeightRange qkv = layers[i].attention->qkv_weight();
     for (const WeightRange& r : ahead[i]) bytes += r.bytes;
     bytes += qkv.bytes;
+    ffn = std::max(ffn, layers[i].intermediate->out_features());
     if (i > 0) ahead[i - 1].push_back(qkv);
   }
-  if (!WeightsLeaveCache(bytes, hidden)) ahead.assign(layers.size(), {});
+  if (!WeightsLeaveCache(bytes, ffn, hidden)) ahead.assign(layers.size(), {});
   return ahead;
 }
 
