@@ -279,6 +279,47 @@ def test_forward_replays_from_a_hip_graph(tt, dtype, B, S):
         assert torch.equal(captured, want), "replay %d" % step
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, "int8"])
+def test_graphs_of_two_attention_layers_replay_side_by_side(tt, dtype):
+    """The layers of an encoder lend each other the tensors of a call while the encoder runs; a layer that is called by itself has its
+    own, so graphs of two of them write nothing in common and may be replayed on two streams."""
+    model, cfg = _hf_bert(2, seed=4)
+    if dtype == "int8":
+        tmodel = tt.QBertModel.from_torch(model)
+    else:
+        tmodel = tt.BertModel.from_torch(model.to(dtype), torch.device("cuda:0"), "turbo")
+    x_type = torch.float32 if dtype == "int8" else dtype
+    B, S = 16, 128
+    g = torch.Generator().manual_seed(3)
+    tmodel(torch.randint(0, cfg.vocab_size, (B, S), generator=g).cuda())
+    layers = [l.attention for l in (tmodel if dtype == "int8" else tmodel.bertmodel_nopooler).encoder.layer]
+    inputs = [torch.randn(B, S, cfg.hidden_size, generator=g).to(x_type).cuda() for _ in layers]
+    graphs, outputs, streams = [], [], [torch.cuda.Stream() for _ in layers]
+    for layer, x, side in zip(layers, inputs, streams):
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(2):
+                layer(x)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            outputs.append(layer(x)[0])
+        graphs.append(graph)
+    for step in range(5):
+        fresh = [torch.randn(B, S, cfg.hidden_size, generator=g).to(x_type).cuda() for _ in layers]
+        want = [layer(x)[0].clone() for layer, x in zip(layers, fresh)]
+        for x, f in zip(inputs, fresh):
+            x.copy_(f)
+        torch.cuda.synchronize()
+        for _ in range(5):
+            for graph, side in zip(graphs, streams):
+                with torch.cuda.stream(side):
+                    graph.replay()
+        torch.cuda.synchronize()
+        for got, w in zip(outputs, want):
+            assert torch.equal(got, w), "step %d" % step
+
+
 @pytest.mark.parametrize("lens", [[4, 1], [9, 7, 13], [10, 19, 20], [50, 3, 17, 31, 8]])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_smart_batch_equals_per_request_dense(tt, lens, dtype):

@@ -31,8 +31,8 @@ BERTLayer::BERTLayer(WeightMap* w, const std::string& p, int64_t n_heads) {
 }
 
 void BERTLayer::operator()(Tensor& hidden, Tensor& mask, Tensor* attention_out, Tensor* intermediate_out, Tensor* output,
-                           const std::vector<layers::WeightRange>& ahead) const {
-  (*attention_)(hidden, mask, attention_out, nullptr, false, ahead);
+                           const std::vector<layers::WeightRange>& ahead, const layers::BertAttention* lender) const {
+  (*attention_)(hidden, mask, attention_out, nullptr, false, ahead, lender);
   (*intermediate_)(*attention_out, intermediate_out);
   (*output_)(*intermediate_out, *attention_out, output);
 }
@@ -57,7 +57,6 @@ struct BertModel::Impl {
                                                Take(&weights, e + "LayerNorm.weight"), Take(&weights, e + "LayerNorm.bias")));
     for (size_t i = 0; i < n_layers; ++i) {
       encoders_.emplace_back(&weights, "encoder.layer." + std::to_string(i) + ".", n_heads);
-      encoders_[i].attention_->ShareScratch(*encoders_[0].attention_);
     }
     if (weights.count("pooler.dense.weight"))
       pooler_.reset(new layers::BertPooler(Take(&weights, "pooler.dense.weight"), Take(&weights, "pooler.dense.bias")));
@@ -70,7 +69,7 @@ struct BertModel::Impl {
     std::vector<layers::EncoderLayer<layers::BertAttention>> subs;
     for (auto& layer : encoders_) subs.push_back({layer.attention_.get(), layer.intermediate_.get(), layer.output_.get()});
     const auto ahead = layers::WeightsAhead(subs, *hidden);
-    for (size_t i = 0; i < encoders_.size(); ++i) encoders_[i](*hidden, ext, &att_out_, &intermediate_out_, hidden, ahead[i]);
+    for (size_t i = 0; i < encoders_.size(); ++i) encoders_[i](*hidden, ext, &att_out_, &intermediate_out_, hidden, ahead[i], encoders_[0].attention_.get());
   }
 
   std::unique_ptr<layers::BERTEmbedding> embedding_;

@@ -29,7 +29,8 @@ struct BERTLayer {
   BERTLayer(WeightMap* weights, const std::string& prefix, int64_t n_heads);
 
   void operator()(core::Tensor& hidden, core::Tensor& mask, core::Tensor* attention_out, core::Tensor* intermediate_out,
-                  core::Tensor* output, const std::vector<layers::WeightRange>& ahead = {}) const;
+                  core::Tensor* output, const std::vector<layers::WeightRange>& ahead = {},
+                  const layers::BertAttention* lender = nullptr) const;
 
   std::unique_ptr<layers::BertAttention> attention_;
   std::unique_ptr<layers::BertIntermediate> intermediate_;

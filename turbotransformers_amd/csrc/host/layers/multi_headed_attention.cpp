@@ -84,7 +84,7 @@ bool MultiHeadedAttention::UseProjectingCore(const Tensor& query_tensor, const W
 static int64_t RoundUp8(int64_t n) { return (n + 7) / 8 * 8; }
 
 // score -> softmax -> P V -> merge heads -> output projection -> bias (+input) (+LayerNorm)
-void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tensor& attention_mask, Tensor* output,
+void MultiHeadedAttention::AttentionTail(Scratch& scratch, const Tensor& query_tensor, const Tensor& attention_mask, Tensor* output,
                                          Tensor* att_score, int64_t batch, int64_t seq, int64_t key_seq, const Tensor& k,
                                          const Tensor& v, const std::vector<int64_t>* seq_list, bool fused_core, int64_t v_pitch,
                                          bool post_layernorm, bool post_add_input, bool is_trans_weight,
@@ -104,15 +104,15 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   if (fused_core && seq_list == nullptr && post_layernorm && !post_add_input && UseProjectingCore(query_tensor, wo, batch, seq, v_pitch, dt)) {
     if (!attention_mask.is_null()) TT_ENFORCE_EQ(attention_mask.numel(), batch * seq, "attention mask has the wrong size");
     TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
-    float* partial = scratch_->partial.Reshape<float>({heads, tokens, hidden}, dev, dev_id, "gemm5/slices/Reshape");
-    TT_DEVICE_CALL(ttmi_attention_projection(scratch_->q.raw(), k.raw(), v.raw(), attention_mask.is_null() ? nullptr : attention_mask.data<float>(),
+    float* partial = scratch.partial.Reshape<float>({heads, tokens, hidden}, dev, dev_id, "gemm5/slices/Reshape");
+    TT_DEVICE_CALL(ttmi_attention_projection(scratch.q.raw(), k.raw(), v.raw(), attention_mask.is_null() ? nullptr : attention_mask.data<float>(),
                                              wo.data, partial, batch, heads, seq, d, v_pitch, scaler, dt, ahead_data,
                                              ahead_bytes, (int64_t)ranges, Stream()));
     output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
-    kernels::AddSlicesLayerNorm(scratch_->partial, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
+    kernels::AddSlicesLayerNorm(scratch.partial, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
     return;
   }
-  scratch_->ctx.ReshapeAs(query_tensor.dtype(), {tokens, hidden}, dev, dev_id, "batch_gemm4/Reshape");
+  scratch.ctx.ReshapeAs(query_tensor.dtype(), {tokens, hidden}, dev, dev_id, "batch_gemm4/Reshape");
 
   // Nobody asked for the probabilities: run the whole core as one kernel; the [B,h,S,S] scores
   // never reach HBM.
@@ -125,10 +125,10 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
     TT_ENFORCE_EQ(seq, key_seq, "the fused core is for self attention without a key/value cache");
     const int32_t* cu = nullptr;
     if (seq_list != nullptr) cu = DeviceContext::GetInstance().GetSeqPlan(*seq_list).cu_seqlens;
-    TT_DEVICE_CALL(ttmi_fused_attention_ahead(scratch_->q.raw(), k.raw(), v.raw(), mask, scratch_->ctx.mutable_raw(), cu, batch, heads, seq, d,
+    TT_DEVICE_CALL(ttmi_fused_attention_ahead(scratch.q.raw(), k.raw(), v.raw(), mask, scratch.ctx.mutable_raw(), cu, batch, heads, seq, d,
                                               v_pitch, scaler, dt, ahead_data, ahead_bytes, (int64_t)ranges, Stream()));
   } else {
-  Tensor* score = att_score != nullptr ? att_score : &scratch_->score;
+  Tensor* score = att_score != nullptr ? att_score : &scratch.score;
   // score is [B,h,F,T]: F = query positions, T = key positions (they differ for context attention
   // and when a key/value cache has been prepended)
   const int64_t F = seq, T = key_seq;
@@ -146,27 +146,27 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
       TT_ENFORCE_EQ(attention_mask.numel(), per_query ? batch * F * T : batch * T, "attention mask has the wrong size");
     }
     TT_DEVICE_CALL(ttmi_attention_with_probs(
-        scratch_->q.raw(), grow ? grow->k_past->raw() : nullptr, grow ? grow->v_past->raw() : nullptr, grow ? grow->k_past->shape(2) : 0,
+        scratch.q.raw(), grow ? grow->k_past->raw() : nullptr, grow ? grow->v_past->raw() : nullptr, grow ? grow->k_past->shape(2) : 0,
         k.raw(), v.raw(), grow ? grow->k_grown->mutable_raw() : nullptr, grow ? grow->v_grown->mutable_raw() : nullptr, mask,
-        per_query ? 1 : 0, score->mutable_raw(), scratch_->ctx.mutable_raw(), batch, heads, F, T, d, scaler, dt, Stream()));
+        per_query ? 1 : 0, score->mutable_raw(), scratch.ctx.mutable_raw(), batch, heads, F, T, d, scaler, dt, Stream()));
   } else {
   // batch_gemm3: score[b,h] = scaler * q[b,h] k[b,h]^T   (multi_headed_attention.cpp:328-330)
-  TT_DEVICE_CALL(ttmi_gemm_strided_batched(scratch_->q.raw(), k.raw(), score->mutable_raw(), F, T, d, d, d, T, F * d, T * d, F * T,
+  TT_DEVICE_CALL(ttmi_gemm_strided_batched(scratch.q.raw(), k.raw(), score->mutable_raw(), F, T, d, d, d, T, F * d, T * d, F * T,
                                            batch * heads, 1, scaler, 0.f, dt, Stream()));
   kernels::ApplyMaskAndSoftmax(score, attention_mask, 1.0f);
 
   if (seq_list == nullptr) {
     // batch_gemm4 with the [B,h,F,d] -> [B,F,h,d] transpose folded into the store (:345-354)
-    TT_DEVICE_CALL(ttmi_gemm_batched_heads(score->raw(), v.raw(), scratch_->ctx.mutable_raw(), F, d, T, T, d, hidden, heads,
+    TT_DEVICE_CALL(ttmi_gemm_batched_heads(score->raw(), v.raw(), scratch.ctx.mutable_raw(), F, d, T, T, d, hidden, heads,
                                            heads * F * T, F * T, heads * T * d, T * d, F * hidden, d, batch, 0, 1.f, 0.f, dt,
                                            Stream()));
   } else {
     // padded P V, then drop the pad rows while merging heads (…smart_batch.cpp:385-392)
-    Tensor& padded = scratch_->ln_query;  // free at this point of the call
+    Tensor& padded = scratch.ln_query;  // free at this point of the call
     padded.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "ApplyMaskAndSoftmax/Reshape");
     TT_DEVICE_CALL(ttmi_gemm_strided_batched(score->raw(), v.raw(), padded.mutable_raw(), seq, d, seq, seq, d, d, seq * seq,
                                              seq * d, seq * d, batch * heads, 0, 1.f, 0.f, dt, Stream()));
-    kernels::TransposeForScorePad(&scratch_->ctx, padded, *seq_list);
+    kernels::TransposeForScorePad(&scratch.ctx, padded, *seq_list);
   }
   }  // chain
   }  // unfused core
@@ -174,12 +174,12 @@ void MultiHeadedAttention::AttentionTail(const Tensor& query_tensor, const Tenso
   output->ReshapeAs(query_tensor.dtype(), {query_tensor.shape(0), query_tensor.shape(1), hidden}, dev, dev_id, "gemm5/Reshape");
   if (!post_add_input && post_layernorm) {
     // gemm5 then AddBiasLayerNorm(query, bias, gamma, beta, out), eps 1e-12 (:359-371)
-    kernels::GemmAddBiasLayerNorm(scratch_->ctx, wo, hidden, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
+    kernels::GemmAddBiasLayerNorm(scratch.ctx, wo, hidden, query_tensor, dense_bias_, layernorm_gamma_, layernorm_beta_, output, 1e-12f);
   } else {
     ttmi_epilogue_args args{};
     args.bias = dense_bias_.raw();
     args.residual = post_add_input ? query_tensor.raw() : nullptr;
-    TT_DEVICE_CALL(ttmi_gemm_fused(scratch_->ctx.raw(), wo.data, output->mutable_raw(), tokens, hidden, hidden, hidden, hidden, hidden,
+    TT_DEVICE_CALL(ttmi_gemm_fused(scratch.ctx.raw(), wo.data, output->mutable_raw(), tokens, hidden, hidden, hidden, hidden, hidden,
                                    post_add_input ? TTMI_EPI_BIAS_RESIDUAL : TTMI_EPI_BIAS, &args, wo.DTypeFor(dt), Stream()));
   }
 }
@@ -220,9 +220,10 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
                                    const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
                                    Tensor* att_score, std::unordered_map<std::string, Tensor*> layer_cache,
                                    bool pre_layernorm, bool post_layernorm, bool post_add_input, bool is_trans_weight,
-                                   const std::vector<WeightRange>& ahead) const {
+                                   const std::vector<WeightRange>& ahead, const MultiHeadedAttention& lender) const {
   std::lock_guard<std::mutex> g(mutex_);
-  std::lock_guard<std::mutex> use(scratch_->mutex);
+  Scratch& scratch = lender.scratch_;
+  std::lock_guard<std::mutex> use(scratch.mutex);
   const bool is_self = attn_type == "self";
   TT_ENFORCE(is_self || attn_type == "context", "attn_type should be context or self.");
   TT_ENFORCE_EQ(query_tensor.n_dim(), (size_t)3, "The query_tensors should be a matrix with shape [batch_size, query_seq_len, hidden_size].");
@@ -250,7 +251,7 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
   // a projection of the query, with LayerNorm in front where asked for (:66-80, :190-199 -- eps is 1e-6 there)
   auto project_query = [&](const WeightRef& packed_w, int64_t n, const ttmi_epilogue_args& args) {
     if (pre_layernorm) {
-      kernels::LayerNormGemm(query_tensor, layernorm_gamma_, layernorm_beta_, 1e-6f, &scratch_->ln_query, packed_w, nullptr, n,
+      kernels::LayerNormGemm(query_tensor, layernorm_gamma_, layernorm_beta_, 1e-6f, &scratch.ln_query, packed_w, nullptr, n,
                              TTMI_EPI_QKV_SPLIT, args);
     } else {
       TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), packed_w.data, nullptr, batch * seq, n, hidden, hidden, hidden, n,
@@ -258,8 +259,8 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
     }
   };
 
-  const Tensor* k_used = &scratch_->k;
-  const Tensor* v_used = &scratch_->v;
+  const Tensor* k_used = &scratch.k;
+  const Tensor* v_used = &scratch.v;
   int64_t v_pitch = 0;
   bool fused_core = false;
   // What a call adds to the layer cache is computed into fresh tensors and moved there: no copy.
@@ -283,24 +284,24 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
     const bool fused_self = layer_cache.empty() && UseFusedCore(attention_mask, att_score, d, dt, batch, seq, heads, true);
     if (fused_self) v_pitch = RoundUp8(seq);
     fused_core = fused_self;
-    scratch_->q.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/q/Reshape");
+    scratch.q.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/q/Reshape");
     const bool past_k = CacheHas(layer_cache, "self_keys"), past_v = CacheHas(layer_cache, "self_values");
-    Tensor* k_new = &scratch_->k;  // where the projection puts keys and values
-    Tensor* v_new = &scratch_->v;
+    Tensor* k_new = &scratch.k;  // where the projection puts keys and values
+    Tensor* v_new = &scratch.v;
     if (!layer_cache.empty() && !past_k && !past_v) {
       k_cache = fresh(seq, "self/self_key/Reshape");
       v_cache = fresh(seq, "self/self_value/Reshape");
       k_new = &k_cache;
       v_new = &v_cache;
     } else {
-    scratch_->k.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/k/Reshape");
-    if (v_pitch > 0) scratch_->v.ReshapeAs(query_tensor.dtype(), {batch, heads, d, v_pitch}, dev, dev_id, "self/v/Reshape");
-    else scratch_->v.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/v/Reshape");
+    scratch.k.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/k/Reshape");
+    if (v_pitch > 0) scratch.v.ReshapeAs(query_tensor.dtype(), {batch, heads, d, v_pitch}, dev, dev_id, "self/v/Reshape");
+    else scratch.v.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "self/v/Reshape");
     }
     // gemm012_fused + SplitAddBiasTransposeForScore in one launch (:199-203)
     ttmi_epilogue_args args{};
     args.bias = qkv_bias_.raw();
-    args.q = scratch_->q.mutable_raw();
+    args.q = scratch.q.mutable_raw();
     args.k = k_new->mutable_raw();
     args.v = v_new->mutable_raw();
     args.seq = seq;
@@ -329,20 +330,20 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
       v_cache = fresh(total, "self/self_value/Reshape");
       growth = CacheGrowth{layer_cache.at("self_keys"), layer_cache.at("self_values"), &k_cache, &v_cache};
     } else {
-      prepend("self_keys", &scratch_->k, &scratch_->k_grown, "self/keys/Concat");
-      prepend("self_values", &scratch_->v, &scratch_->v_grown, "self/values/Concat");
+      prepend("self_keys", &scratch.k, &scratch.k_grown, "self/keys/Concat");
+      prepend("self_values", &scratch.v, &scratch.v_grown, "self/values/Concat");
     }
-    if (!layer_cache.empty() && k_used == &scratch_->k && growth.k_grown == nullptr) {
-      StoreInCache(layer_cache, "self_keys", scratch_->k, "self/self_key/Reshape");
-      StoreInCache(layer_cache, "self_values", scratch_->v, "self/self_value/Reshape");
+    if (!layer_cache.empty() && k_used == &scratch.k && growth.k_grown == nullptr) {
+      StoreInCache(layer_cache, "self_keys", scratch.k, "self/self_key/Reshape");
+      StoreInCache(layer_cache, "self_values", scratch.v, "self/self_value/Reshape");
     }
   } else {
     TT_ENFORCE(!q_weight_.is_null() && !k_weight_.is_null() && !v_weight_.is_null() && !q_bias_.is_null() && !k_bias_.is_null() &&
                    !v_bias_.is_null(), "context attention needs the separate q/k/v weights and biases");
-    scratch_->q.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "context/AddBiasTransposeForScore/q_out2/Reshape");
+    scratch.q.ReshapeAs(query_tensor.dtype(), {batch, heads, seq, d}, dev, dev_id, "context/AddBiasTransposeForScore/q_out2/Reshape");
     ttmi_epilogue_args args{};
     args.bias = q_bias_.raw();
-    args.q = scratch_->q.mutable_raw();
+    args.q = scratch.q.mutable_raw();
     args.seq = seq;
     args.heads = heads;
     args.head_dim = d;
@@ -362,7 +363,7 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
       TT_ENFORCE(core::SameDataType(key_tensor.dtype(), query_tensor.dtype()) && core::SameDataType(value_tensor.dtype(), query_tensor.dtype()),
                  "key, value and query must share one element type");
       const bool keep = !layer_cache.empty();  // :128-150
-      Tensor *k_out = keep ? &k_cache : &scratch_->k, *v_out = keep ? &v_cache : &scratch_->v;
+      Tensor *k_out = keep ? &k_cache : &scratch.k, *v_out = keep ? &v_cache : &scratch.v;
       // Keys and values are usually projections of the same memory: then one product against both weights, whose tiles fill the
       // last round of workgroups better than two launches do (fp32 800 x 768: 2 x 16.3 us, together 23.3 and 2 for the bias, which is
       // joined on each call because it is read where the caller keeps it).
@@ -372,10 +373,10 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
         const int64_t len = key_tensor.shape(1);
         k_out->ReshapeAs(query_tensor.dtype(), {batch, heads, len, d}, dev, dev_id, "context/keys/AddBiasTransposeForScore/Reshape");
         v_out->ReshapeAs(query_tensor.dtype(), {batch, heads, len, d}, dev, dev_id, "context/values/AddBiasTransposeForScore/Reshape");
-        scratch_->kv_bias.ReshapeAs(query_tensor.dtype(), {2 * hidden}, dev, dev_id, "context/kv_bias/Reshape");
-        TT_DEVICE_CALL(ttmi_concat(k_bias_.raw(), v_bias_.raw(), scratch_->kv_bias.mutable_raw(), 1, hidden, hidden, dt, Stream()));
+        scratch.kv_bias.ReshapeAs(query_tensor.dtype(), {2 * hidden}, dev, dev_id, "context/kv_bias/Reshape");
+        TT_DEVICE_CALL(ttmi_concat(k_bias_.raw(), v_bias_.raw(), scratch.kv_bias.mutable_raw(), 1, hidden, hidden, dt, Stream()));
         ttmi_epilogue_args kv{};
-        kv.bias = scratch_->kv_bias.raw();
+        kv.bias = scratch.kv_bias.raw();
         kv.q = k_out->mutable_raw();
         kv.k = v_out->mutable_raw();
         kv.seq = len;
@@ -398,7 +399,7 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
   const int64_t key_seq = fused_core ? seq : growing ? k_cache.shape(2) : k_used->shape(2);
   TT_ENFORCE_EQ(fused_core ? seq : growing ? v_cache.shape(2) : v_used->shape(2), key_seq, "keys and values differ in length");
 
-  AttentionTail(query_tensor, attention_mask, output, att_score, batch, seq, key_seq, *k_used, *v_used, nullptr, fused_core, v_pitch,
+  AttentionTail(scratch, query_tensor, attention_mask, output, att_score, batch, seq, key_seq, *k_used, *v_used, nullptr, fused_core, v_pitch,
                 post_layernorm, post_add_input, is_trans_weight, growing ? &growth : nullptr, ahead);
   if (growing) {
     move_to_cache("self_keys", k_cache);
@@ -407,11 +408,12 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
 }
 
 void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attention_mask, Tensor* output, Tensor* attn,
-                               bool is_trans_weight, const std::vector<WeightRange>& ahead) const {
+                               bool is_trans_weight, const std::vector<WeightRange>& ahead, const BertAttention* lender) const {
   // bert_attention.cpp:29-47: self attention, post-LayerNorm, no extra residual
   std::unordered_map<std::string, Tensor*> dummy{};
   Forward(input_tensor, input_tensor, input_tensor, attention_mask, "self", output, attn, dummy, false /* pre_layernorm */,
-          true /* post_layernorm */, false /* post_add_input */, is_trans_weight, ahead);
+          true /* post_layernorm */, false /* post_add_input */, is_trans_weight, ahead,
+          lender != nullptr ? *lender : *this);
 }
 
 bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const Tensor& hidden) {
@@ -425,9 +427,11 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
                                              const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
                                              Tensor* att_score, const std::unordered_map<std::string, Tensor*>& layer_cache,
                                              const std::vector<int64_t>& query_seq_len_list, bool pre_layernorm, bool post_layernorm,
-                                             bool post_add_input, bool is_trans_weight, const std::vector<WeightRange>& ahead) const {
+                                             bool post_add_input, bool is_trans_weight, const std::vector<WeightRange>& ahead,
+                                             const MultiHeadedAttentionSmartBatch& lender) const {
   std::lock_guard<std::mutex> g(mutex_);
-  std::lock_guard<std::mutex> use(scratch_->mutex);
+  Scratch& scratch = lender.scratch_;
+  std::lock_guard<std::mutex> use(scratch.mutex);
   TT_ENFORCE(attn_type == "self", "only attn_type \"self\" is built (\"context\" belongs to the decoder path)");
   TT_ENFORCE(layer_cache.empty(), "layer_cache belongs to the decoder path and is not built");
   TT_ENFORCE(!pre_layernorm, "pre_layernorm is not built for the smart-batch layer");
@@ -456,7 +460,7 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
   // and that costs the QKV GEMM more than the scatter costs the attention kernel (20 requests, 6275 tokens:
   // 2.50 against 2.39 ms per forward).
   const bool fused_core = UseFusedCore(attention_mask, att_score, d, dt, batch, max_seq, heads);
-  Tensor* qkv[3] = {&scratch_->q, &scratch_->k, &scratch_->v};
+  Tensor* qkv[3] = {&scratch.q, &scratch.k, &scratch.v};
   const char* names[3] = {"self/q/Reshape", "self/k/Reshape", "self/v/Reshape"};
   for (int i = 0; i < 3; ++i) {
     qkv[i]->ReshapeAs(query_tensor.dtype(), {batch, heads, max_seq, d}, dev, dev_id, names[i]);
@@ -466,9 +470,9 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
   }
   ttmi_epilogue_args args{};
   args.bias = qkv_bias_.raw();
-  args.q = scratch_->q.mutable_raw();
-  args.k = scratch_->k.mutable_raw();
-  args.v = scratch_->v.mutable_raw();
+  args.q = scratch.q.mutable_raw();
+  args.k = scratch.k.mutable_raw();
+  args.v = scratch.v.mutable_raw();
   args.seq = max_seq;
   args.heads = heads;
   args.head_dim = d;
@@ -478,7 +482,7 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
   TT_DEVICE_CALL(ttmi_gemm_fused(query_tensor.raw(), wqkv.data, nullptr, plan.total, 3 * hidden, hidden, hidden, hidden, 3 * hidden,
                                  TTMI_EPI_QKV_SPLIT_PAD, &args, wqkv.DTypeFor(dt), Stream()));
 
-  AttentionTail(query_tensor, attention_mask, output, att_score, batch, max_seq, max_seq, scratch_->k, scratch_->v, &query_seq_len_list, fused_core, 0,
+  AttentionTail(scratch, query_tensor, attention_mask, output, att_score, batch, max_seq, max_seq, scratch.k, scratch.v, &query_seq_len_list, fused_core, 0,
                 post_layernorm, post_add_input, is_trans_weight, nullptr, ahead);
 }
 

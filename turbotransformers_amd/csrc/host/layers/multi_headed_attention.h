@@ -19,7 +19,6 @@
 
 #include <algorithm>
 #include <initializer_list>
-#include <memory>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -64,7 +63,7 @@ class MultiHeadedAttention {
                   bool pre_layernorm = false, bool post_layernorm = false, bool post_add_input = false,
                   bool is_trans_weight = false) const {
     Forward(key_tensor, value_tensor, query_tensor, attention_mask, attn_type, output, att_score, std::move(layer_cache), pre_layernorm,
-            post_layernorm, post_add_input, is_trans_weight, {});
+            post_layernorm, post_add_input, is_trans_weight, {}, *this);
   }
 
   // The whole attention core runs as one kernel when nobody asks for the probabilities
@@ -77,27 +76,22 @@ class MultiHeadedAttention {
   WeightRange qkv_weight() const { return qkv_packed_.Range(qkv_weight_); }
   WeightRange dense_weight() const { return dense_packed_.Range(dense_weight_); }
 
-  // The layers of a stack run one after the other: they may share what they hold during a call.  With buffers of its own each layer of
-  // an encoder writes and reads 4 x rows x hidden values in memory that the last-level cache (256 MB) has seen a whole pass ago, and
-  // pushes the weights out of it: us per forward, own / shared, base: fp16 20 x 100 tokens 932 / 886, 12 x 64 592 / 527, int8 20 x 128
-  // 1356 / 1223.
-  void ShareScratch(const MultiHeadedAttention& other) {
-    if (&other == this) return;
-    std::shared_ptr<Scratch> shared;
-    {
-      std::lock_guard<std::mutex> lock(other.mutex_);
-      shared = other.scratch_;
-    }
-    std::lock_guard<std::mutex> lock(mutex_);
-    scratch_ = std::move(shared);
-  }
-
  protected:
   // operator(); `ahead`: what the layer and the following ones read after the attention core (WeightsAhead).
+  // `lender`: whose tensors hold Q, K, V, the context ... during the call: those of this layer, or of another one of the stack that
+  // runs.  With its own each layer of an encoder writes and reads 4 x rows x hidden values in memory that the last-level cache (256 MB) has
+  // seen a whole pass ago, and pushes the weights out of it: us per forward, own / of one layer, base: fp16 20 x 100 tokens 932 / 886, 12 x 64
+  // 592 / 527, int8 20 x 128 1356 / 1223.  A layer that is called by itself has its own.
   void Forward(const core::Tensor& key_tensor, const core::Tensor& value_tensor, const core::Tensor& query_tensor,
                const core::Tensor& attention_mask, const std::string& attn_type, core::Tensor* output, core::Tensor* att_score,
                std::unordered_map<std::string, core::Tensor*> layer_cache, bool pre_layernorm, bool post_layernorm,
-               bool post_add_input, bool is_trans_weight, const std::vector<WeightRange>& ahead) const;
+               bool post_add_input, bool is_trans_weight, const std::vector<WeightRange>& ahead, const MultiHeadedAttention& lender) const;
+
+  // Per-call intermediates, reused across calls (Reshape keeps a buffer that is large enough).
+  struct Scratch {
+    core::Tensor q, k, v, k_grown, v_grown, kv_bias, ctx, partial, score, ln_query;
+    std::mutex mutex;  // from a call's first launch that writes here to its last that reads; all launches are on one stream
+  };
 
   // A key/value cache that the attention core extends: [past | new] along the sequence into the grown tensors.
   struct CacheGrowth {
@@ -114,7 +108,7 @@ class MultiHeadedAttention {
   // `fused_core`: the one-kernel attention core runs; `v_pitch` > 0: v holds V transposed, [B,h,d,v_pitch].
   // `seq` query positions against `key_seq` key positions held in k / v ([B,h,key_seq,d]); with `grow` the first of them
   // are in its past tensors instead, and k / v hold the rest.
-  void AttentionTail(const core::Tensor& query_tensor, const core::Tensor& attention_mask, core::Tensor* output,
+  void AttentionTail(Scratch& scratch, const core::Tensor& query_tensor, const core::Tensor& attention_mask, core::Tensor* output,
                      core::Tensor* att_score, int64_t batch, int64_t seq, int64_t key_seq, const core::Tensor& k,
                      const core::Tensor& v, const std::vector<int64_t>* seq_list, bool fused_core, int64_t v_pitch,
                      bool post_layernorm, bool post_add_input, bool is_trans_weight, const CacheGrowth* grow = nullptr,
@@ -126,12 +120,7 @@ class MultiHeadedAttention {
   int64_t num_attention_heads_;
 
   PackedWeight qkv_packed_, dense_packed_, q_packed_, k_packed_, v_packed_, kv_packed_;
-  // Per-call intermediates, reused across calls (Reshape keeps a buffer that is large enough) and by layers that share them.
-  struct Scratch {
-    core::Tensor q, k, v, k_grown, v_grown, kv_bias, ctx, partial, score, ln_query;
-    std::mutex mutex;  // from a call's first launch that writes here to its last that reads; all launches are on one stream
-  };
-  mutable std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
+  mutable Scratch scratch_;
   mutable std::mutex mutex_;  // the layer keeps per-call state, like the reference (…attention.cpp:32,272)
 };
 
@@ -152,7 +141,7 @@ class BertAttention : public MultiHeadedAttention {
     (*this)(input_tensor, attention_mask, output, attn, is_trans_weight, {});
   }
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output, core::Tensor* attn,
-                  bool is_trans_weight, const std::vector<WeightRange>& ahead) const;
+                  bool is_trans_weight, const std::vector<WeightRange>& ahead, const BertAttention* lender = nullptr) const;
 };
 
 class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
@@ -168,13 +157,14 @@ class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
                   bool pre_layernorm = false, bool post_layernorm = false, bool post_add_input = false,
                   bool is_trans_weight = false) const {
     Forward(key_tensor, value_tensor, query_tensor, attention_mask, attn_type, output, att_score, layer_cache, query_seq_len_list,
-            pre_layernorm, post_layernorm, post_add_input, is_trans_weight, {});
+            pre_layernorm, post_layernorm, post_add_input, is_trans_weight, {}, *this);
   }
   // self attention, post-LayerNorm, no extra residual, as a layer of an encoder
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output,
-                  const std::vector<int64_t>& seq_len_list, const std::vector<WeightRange>& ahead) const {
+                  const std::vector<int64_t>& seq_len_list, const std::vector<WeightRange>& ahead,
+                  const MultiHeadedAttentionSmartBatch& lender) const {
     Forward(input_tensor, input_tensor, input_tensor, attention_mask, "self", output, nullptr, {}, seq_len_list, false, true, false, false,
-            ahead);
+            ahead, lender);
   }
 
  private:
@@ -182,7 +172,7 @@ class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
                const core::Tensor& attention_mask, const std::string& attn_type, core::Tensor* output, core::Tensor* att_score,
                const std::unordered_map<std::string, core::Tensor*>& layer_cache, const std::vector<int64_t>& query_seq_len_list,
                bool pre_layernorm, bool post_layernorm, bool post_add_input, bool is_trans_weight,
-               const std::vector<WeightRange>& ahead) const;
+               const std::vector<WeightRange>& ahead, const MultiHeadedAttentionSmartBatch& lender) const;
 };
 
 // One layer of an encoder.

@@ -24,10 +24,9 @@ QuantizedLinear::QuantizedLinear(core::Tensor weight, core::Tensor bias, const s
   else TT_ENFORCE(activation.empty(), "unknown activation %s", activation.c_str());
 }
 
-std::shared_ptr<QuantizedLinear::Scratch> QuantizedLinear::Prepare(int64_t values) const {
+void QuantizedLinear::Prepare() const {
   std::lock_guard<std::mutex> lock(prepare_mutex_);
-  const std::shared_ptr<Scratch>& scratch = values <= kOwnValues ? own_ : scratch_;
-  if (prepared_) return scratch;
+  if (prepared_) return;
   kernels::RequireGpu(weight_, "QuantizedLinear");
   TT_ENFORCE_EQ(weight_.n_dim(), (size_t)2, "weight must be [in, out]");
   const int64_t k = weight_.shape(0), n = weight_.shape(1);
@@ -41,7 +40,6 @@ std::shared_ptr<QuantizedLinear::Scratch> QuantizedLinear::Prepare(int64_t value
   TT_DEVICE_CALL(ttmi_quantize_weight_rows_i8(t, q, s, n, k, Stream()));
   act_scale_.Reshape<float>({TTMI_QUANT_SCALE_FLOATS}, dev, id, "QuantizedLinear/act_scale");
   prepared_ = true;
-  return scratch;
 }
 
 const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor, Tensor* quantised) const {
@@ -60,10 +58,11 @@ const int8_t* QuantizedLinear::QuantizeInput(const Tensor& input_tensor, Tensor*
   return qx;
 }
 
-void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tensor) const {
-  const std::shared_ptr<Scratch> scratch = Prepare(input_tensor.numel());
-  std::lock_guard<std::mutex> lock(scratch->mutex);
-  const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
+void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tensor, const QuantizedLinear* lender) const {
+  Prepare();
+  Scratch& scratch = ScratchFor(input_tensor.numel(), lender);
+  std::lock_guard<std::mutex> lock(scratch.mutex);
+  const int8_t* qx = QuantizeInput(input_tensor, &scratch.q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;
   std::vector<int64_t> shape;
   for (size_t i = 0; i + 1 < input_tensor.n_dim(); ++i) shape.push_back(input_tensor.shape((int)i));
@@ -86,11 +85,12 @@ void QuantizedLinear::operator()(const Tensor& input_tensor, Tensor* output_tens
 }
 
 void QuantizedLinear::ProjectToHeads(const Tensor& input_tensor, const Tensor& bias, int64_t seq, int64_t heads, Tensor* q,
-                                     Tensor* k_out, Tensor* v) const {
+                                     Tensor* k_out, Tensor* v, const QuantizedLinear* lender) const {
   TT_ENFORCE(bias_.is_null() && act_ < 0, "ProjectToHeads takes the bias as an argument");
-  const std::shared_ptr<Scratch> scratch = Prepare(input_tensor.numel());
-  std::lock_guard<std::mutex> lock(scratch->mutex);
-  const int8_t* qx = QuantizeInput(input_tensor, &scratch->q_input);
+  Prepare();
+  Scratch& scratch = ScratchFor(input_tensor.numel(), lender);
+  std::lock_guard<std::mutex> lock(scratch.mutex);
+  const int8_t* qx = QuantizeInput(input_tensor, &scratch.q_input);
   const int64_t k = weight_.shape(0), n = weight_.shape(1), m = input_tensor.numel() / k;
   TT_ENFORCE_EQ(bias.numel(), n, "bias and weight shape mismatch");
   TT_ENFORCE(n % (3 * heads) == 0 && q->numel() == m * (n / 3), "q,k,v must be shaped [B, heads, S, d]");
@@ -100,20 +100,22 @@ void QuantizedLinear::ProjectToHeads(const Tensor& input_tensor, const Tensor& b
 }
 
 void QuantizedBertAttention::operator()(const Tensor& input_tensor, const Tensor& attention_mask, Tensor* output,
-                                        Tensor* attn) const {
+                                        Tensor* attn, const QuantizedBertAttention* lender) const {
   std::lock_guard<std::mutex> g(mutex_);
-  std::lock_guard<std::mutex> use(scratch_->mutex);
+  Scratch& scratch = lender != nullptr ? lender->scratch_ : scratch_;
+  const QuantizedLinear *qkv_lender = lender != nullptr ? &lender->qkv_ : nullptr, *dense_lender = lender != nullptr ? &lender->dense_ : nullptr;
+  std::lock_guard<std::mutex> use(scratch.mutex);
   kernels::RequireGpu(input_tensor, "QuantizedBertAttention");
   TT_ENFORCE_EQ(input_tensor.n_dim(), (size_t)3, "input should be [batch, seq, hidden]");
   const int64_t B = input_tensor.shape(0), S = input_tensor.shape(1), H = input_tensor.shape(2), d = H / heads_;
   const DLDeviceType dev = input_tensor.device_type();
   const int id = input_tensor.device_id();
   // QKV projection (int8) with bias and head split in its store; then the reference's unfused fp32 chain
-  scratch_->q.Reshape<float>({B, heads_, S, d}, dev, id, "self/q/Reshape");
-  scratch_->k.Reshape<float>({B, heads_, S, d}, dev, id, "self/k/Reshape");
-  scratch_->v.Reshape<float>({B, heads_, S, d}, dev, id, "self/v/Reshape");
-  qkv_.ProjectToHeads(input_tensor, qkv_bias_, S, heads_, &scratch_->q, &scratch_->k, &scratch_->v);
-  scratch_->merged.Reshape<float>({B, S, H}, dev, id, "batch_gemm4/Reshape");
+  scratch.q.Reshape<float>({B, heads_, S, d}, dev, id, "self/q/Reshape");
+  scratch.k.Reshape<float>({B, heads_, S, d}, dev, id, "self/k/Reshape");
+  scratch.v.Reshape<float>({B, heads_, S, d}, dev, id, "self/v/Reshape");
+  qkv_.ProjectToHeads(input_tensor, qkv_bias_, S, heads_, &scratch.q, &scratch.k, &scratch.v, qkv_lender);
+  scratch.merged.Reshape<float>({B, S, H}, dev, id, "batch_gemm4/Reshape");
   if (MultiHeadedAttention::UseFusedCore(attention_mask, attn, d, TTMI_F32, B, S, heads_)) {
     // nobody asked for the probabilities: the fp32 one-kernel attention (row-major V) in place of the four launches
     const float* mask = nullptr;
@@ -122,24 +124,24 @@ void QuantizedBertAttention::operator()(const Tensor& input_tensor, const Tensor
       mask = attention_mask.data<float>();
     }
     // the kernel leaves the maxima of the context with the tensor: the output projection quantises it in one launch
-    void* merged = scratch_->merged.mutable_raw();
-    float* slots = scratch_->merged.EnsureAbsmax()->mutableData<float>();
+    void* merged = scratch.merged.mutable_raw();
+    float* slots = scratch.merged.EnsureAbsmax()->mutableData<float>();
     int written = 0;
-    TT_DEVICE_CALL(ttmi_fused_attention_absmax(scratch_->q.raw(), scratch_->k.raw(), scratch_->v.raw(), mask, merged, nullptr, B, heads_, S, d, 0,
+    TT_DEVICE_CALL(ttmi_fused_attention_absmax(scratch.q.raw(), scratch.k.raw(), scratch.v.raw(), mask, merged, nullptr, B, heads_, S, d, 0,
                                                1.0f / std::sqrt((float)d), TTMI_F32, slots, &written, Stream()));
-    if (written == 0) scratch_->merged.DropAbsmax();
-    dense_(scratch_->merged, output);
+    if (written == 0) scratch.merged.DropAbsmax();
+    dense_(scratch.merged, output, dense_lender);
     kernels::AddBiasLayerNormWithAbsmax(input_tensor, dense_bias_, ln_weight_, ln_bias_, output, 1e-12f);
     return;
   }
-  Tensor* score = attn != nullptr ? attn : &scratch_->score;
+  Tensor* score = attn != nullptr ? attn : &scratch.score;
   score->Reshape<float>({B, heads_, S, S}, dev, id, "batch_gemm3/Reshape");
-  kernels::BatchMatMul(scratch_->q, false, scratch_->k, true, 1.0f / std::sqrt((float)d), score, 0.f);
+  kernels::BatchMatMul(scratch.q, false, scratch.k, true, 1.0f / std::sqrt((float)d), score, 0.f);
   kernels::ApplyMaskAndSoftmax(score, attention_mask, 1.0f);
-  scratch_->ctx.Reshape<float>({B, heads_, S, d}, dev, id, "ApplyMaskAndSoftmax/Reshape");
-  kernels::BatchMatMul(*score, false, scratch_->v, false, 1.0f, &scratch_->ctx, 0.f);
-  kernels::TransposeForScore(&scratch_->merged, scratch_->ctx);
-  dense_(scratch_->merged, output);
+  scratch.ctx.Reshape<float>({B, heads_, S, d}, dev, id, "ApplyMaskAndSoftmax/Reshape");
+  kernels::BatchMatMul(*score, false, scratch.v, false, 1.0f, &scratch.ctx, 0.f);
+  kernels::TransposeForScore(&scratch.merged, scratch.ctx);
+  dense_(scratch.merged, output, dense_lender);
   kernels::AddBiasLayerNormWithAbsmax(input_tensor, dense_bias_, ln_weight_, ln_bias_, output, 1e-12f);
 }
 

@@ -11,7 +11,6 @@
 // that every Linear of the layer is int8.
 #pragma once
 
-#include <memory>
 #include <mutex>
 #include <string>
 
@@ -28,22 +27,12 @@ class QuantizedLinear {
   // dequantises the product: Linear + FusedAddBiasGELU of QBertIntermediate as one call.
   QuantizedLinear(core::Tensor weight, core::Tensor bias, const std::string& activation);
   // output[tokens, out] (fp32) = act(dequant(q(input) * q(weight)^T) + bias)
-  void operator()(const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
+  // `lender`: whose tensor holds the quantised input, as in MultiHeadedAttention::Forward (null: this layer's; and so up to kOwnValues).
+  void operator()(const core::Tensor& input_tensor, core::Tensor* output_tensor, const QuantizedLinear* lender = nullptr) const;
   // A [hidden, 3*hidden] projection written as q,k,v[B, heads, S, d] = split(dequant(...) + bias): the Linear and
   // SplitAddBiasTransposeForScore of the attention in one kernel.  q,k,v are already shaped.
   void ProjectToHeads(const core::Tensor& input_tensor, const core::Tensor& bias, int64_t seq, int64_t heads, core::Tensor* q,
-                      core::Tensor* k, core::Tensor* v) const;
-  // As MultiHeadedAttention::ShareScratch, for the quantised inputs; between the same Linear of different layers.
-  void ShareScratch(const QuantizedLinear& other) {
-    if (&other == this) return;
-    std::shared_ptr<Scratch> shared;
-    {
-      std::lock_guard<std::mutex> lock(other.prepare_mutex_);
-      shared = other.scratch_;
-    }
-    std::lock_guard<std::mutex> lock(prepare_mutex_);
-    scratch_ = std::move(shared);
-  }
+                      core::Tensor* k, core::Tensor* v, const QuantizedLinear* lender = nullptr) const;
   int64_t in_features() const { return weight_.shape(0); }
   int64_t out_features() const { return weight_.shape(1); }
 
@@ -58,12 +47,12 @@ class QuantizedLinear {
   // Up to a megabyte of quantised input a layer keeps a buffer of its own: a quantising launch of 77 rows into one that products of
   // other layers have read is 3.8 instead of 3.3 us.
   static constexpr int64_t kOwnValues = 1 << 20;
-  std::shared_ptr<Scratch> Prepare(int64_t values) const;
-  std::shared_ptr<Scratch> own_ = std::make_shared<Scratch>();
+  void Prepare() const;
+  Scratch& ScratchFor(int64_t values, const QuantizedLinear* lender) const { return lender == nullptr || values <= kOwnValues ? scratch_ : lender->scratch_; }
   mutable core::Tensor q_weight_, w_scales_, act_scale_;
-  std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
+  mutable Scratch scratch_;
   mutable bool prepared_ = false;
-  mutable std::mutex prepare_mutex_;  // scratch_, and the one-time weight quantisation; calls on one object are otherwise not concurrent
+  mutable std::mutex prepare_mutex_;  // the one-time weight quantisation; calls on one object are otherwise not concurrent
 };
 
 class QuantizedBertAttention {
@@ -73,22 +62,9 @@ class QuantizedBertAttention {
       : qkv_(std::move(qkv_weight)), dense_(std::move(dense_weight)), qkv_bias_(std::move(qkv_bias)),
         dense_bias_(std::move(dense_bias)), ln_weight_(std::move(layer_norm_weight)), ln_bias_(std::move(layer_norm_bias)),
         heads_(num_attention_heads) {}
-  // Same contract as BertAttention::operator() for fp32 tensors.
+  // Same contract as BertAttention::operator() for fp32 tensors; `lender` as in MultiHeadedAttention::Forward (null: this layer).
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output,
-                  core::Tensor* attn = nullptr) const;
-  // As MultiHeadedAttention::ShareScratch.
-  void ShareScratch(const QuantizedBertAttention& other) {
-    if (&other == this) return;
-    std::shared_ptr<Scratch> shared;
-    {
-      std::lock_guard<std::mutex> lock(other.mutex_);
-      shared = other.scratch_;
-    }
-    std::lock_guard<std::mutex> lock(mutex_);
-    scratch_ = std::move(shared);
-    qkv_.ShareScratch(other.qkv_);
-    dense_.ShareScratch(other.dense_);
-  }
+                  core::Tensor* attn = nullptr, const QuantizedBertAttention* lender = nullptr) const;
 
  private:
   QuantizedLinear qkv_, dense_;
@@ -98,7 +74,7 @@ class QuantizedBertAttention {
     core::Tensor q, k, v, ctx, merged, score;
     std::mutex mutex;
   };
-  std::shared_ptr<Scratch> scratch_ = std::make_shared<Scratch>();
+  mutable Scratch scratch_;
   mutable std::mutex mutex_;
 };
 

@@ -125,10 +125,11 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
         return new layers::BertAttention(std::move(qkv_w), std::move(qkv_b), std::move(dense_w), std::move(dense_b),
                                          std::move(ln_w), std::move(ln_b), heads);
       }))
-      .def("__call__", py::overload_cast<const Tensor&, const Tensor&, Tensor*, Tensor*, bool>(&layers::BertAttention::operator(), py::const_), py::arg("input_tensor"), py::arg("attention_mask"),
-           py::arg("output"), py::arg("attn") = nullptr, py::arg("is_trans_weight") = false)
-      .def("share_scratch", [](layers::BertAttention& self, const layers::BertAttention& other) { self.ShareScratch(other); },
-           "Hold the tensors of a call where `other` holds its own: for layers that run one after the other.");
+      .def("__call__",
+           [](const layers::BertAttention& self, const Tensor& input, const Tensor& mask, Tensor* output, Tensor* attn, bool is_trans_weight,
+              const layers::BertAttention* lender) { self(input, mask, output, attn, is_trans_weight, {}, lender); },
+           py::arg("input_tensor"), py::arg("attention_mask"), py::arg("output"), py::arg("attn") = nullptr,
+           py::arg("is_trans_weight") = false, py::arg("lender") = nullptr);
 
   py::class_<layers::MultiHeadedAttention>(m, "MultiHeadedAttention")
       .def(py::init([](Tensor& kw, Tensor& kb, Tensor& vw, Tensor& vb, Tensor& qw, Tensor& qb, Tensor& dw, Tensor& db,
@@ -166,8 +167,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
               bool post_add_input, bool is_trans_weight) {
              self(key, value, query, mask, attn_type, output, att_score, std::move(layer_cache), query_lens, key_lens, pre_layernorm,
                   post_layernorm, post_add_input, is_trans_weight);
-           })
-      .def("share_scratch", [](layers::MultiHeadedAttentionSmartBatch& self, const layers::MultiHeadedAttentionSmartBatch& other) { self.ShareScratch(other); });
+           });
 
   py::class_<layers::BertIntermediate>(m, "BertIntermediate")
       .def(py::init([](Tensor& w, Tensor& b) { return new layers::BertIntermediate(std::move(w), std::move(b)); }))
@@ -229,8 +229,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
       .def(py::init([](Tensor& w, Tensor& bias, const std::string& activation) {
         return new layers::QuantizedLinear(std::move(w), std::move(bias), activation);
       }))
-      .def("__call__", &layers::QuantizedLinear::operator())
-      .def("share_scratch", [](layers::QuantizedLinear& self, const layers::QuantizedLinear& other) { self.ShareScratch(other); });
+      .def("__call__", &layers::QuantizedLinear::operator(), py::arg("input_tensor"), py::arg("output_tensor"), py::arg("lender") = nullptr);
 
   py::class_<layers::QuantizedBertAttention>(m, "QuantizedBertAttention")
       .def(py::init([](Tensor& qkv_w, Tensor& qkv_b, Tensor& dense_w, Tensor& dense_b, Tensor& ln_w, Tensor& ln_b, int heads) {
@@ -238,8 +237,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                                                   std::move(ln_w), std::move(ln_b), heads);
       }))
       .def("__call__", &layers::QuantizedBertAttention::operator(), py::arg("input_tensor"), py::arg("attention_mask"),
-           py::arg("output"), py::arg("attn") = nullptr)
-      .def("share_scratch", [](layers::QuantizedBertAttention& self, const layers::QuantizedBertAttention& other) { self.ShareScratch(other); });
+           py::arg("output"), py::arg("attn") = nullptr, py::arg("lender") = nullptr);
 
   m.def("build_smart_pad_mask",
         [](const std::vector<int64_t>& lens, Tensor* out) {
@@ -299,7 +297,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
     for (size_t i = 0; i < subs.size(); ++i) {
       // the last layer writes the caller's tensor; before it two buffers alternate (a layer never writes what it reads)
       Tensor* target = (i + 1 == subs.size()) ? out : (i % 2 == 0 ? &even : &odd);
-      (*subs[i].attention)(*current, mask, &attention_out, nullptr, false, ahead[i]);
+      (*subs[i].attention)(*current, mask, &attention_out, nullptr, false, ahead[i], subs[0].attention);
       (*subs[i].intermediate)(attention_out, &intermediate_out);
       (*subs[i].output)(intermediate_out, attention_out, target);
       current = target;
@@ -322,7 +320,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
     const auto ahead = layers::WeightsAhead(subs, hidden);
     for (size_t i = 0; i < subs.size(); ++i) {
       Tensor* target = (i + 1 == subs.size()) ? out : (i % 2 == 0 ? &even : &odd);
-      (*subs[i].attention)(*current, mask, &attention_out, lens, ahead[i]);
+      (*subs[i].attention)(*current, mask, &attention_out, lens, ahead[i], *subs[0].attention);
       (*subs[i].intermediate)(attention_out, &intermediate_out);
       (*subs[i].output)(intermediate_out, attention_out, target);
       current = target;

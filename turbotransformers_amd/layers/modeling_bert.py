@@ -13,7 +13,7 @@ import torch
 
 from .. import cxx
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, share_scratch, to_param_dict, to_param_dict_convert_tt,
+from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, to_param_dict_convert_tt,
                     try_convert, use_current_stream, weight_in_out)
 
 __all__ = ['BertEmbeddings', 'BertIntermediate', 'BertOutput', 'BertAttention', 'BertLayer', 'BertEncoder',
@@ -91,15 +91,16 @@ class BertOutput(cxx.BertOutput):
 class BertAttention(cxx.BertAttention):
     def __call__(self, input_tensor: AnyTensor, attention_mask: Optional[AnyTensor] = None,
                  head_mask: Optional[AnyTensor] = None, output_attentions: Optional[bool] = False,
-                 return_type: Optional[ReturnType] = None, is_trans_weight: Optional[bool] = False):
-        """-> (context_layer,) or (context_layer, attention_probs)."""
+                 return_type: Optional[ReturnType] = None, is_trans_weight: Optional[bool] = False, lender=None):
+        """-> (context_layer,) or (context_layer, attention_probs).  `lender`: another layer of the stack that runs, which holds the
+        tensors of the call."""
         assert head_mask is None
         use_current_stream()
         context_layer = cxx.Tensor.create_empty()
         # the probabilities [B,h,S,S] are only materialised as an output when asked for
         attn_probs = cxx.Tensor.create_empty() if output_attentions else None
         super().__call__(try_convert(input_tensor), try_convert(create_empty_if_none(attention_mask)), context_layer,
-                         attn_probs, bool(is_trans_weight))
+                         attn_probs, bool(is_trans_weight), lender)
         out = (convert_returns_as_type(context_layer, return_type), )
         if output_attentions:
             out = out + (convert_returns_as_type(attn_probs, ReturnType.turbo_transformers), )
@@ -163,7 +164,6 @@ class BertLayer:
 class BertEncoder:
     def __init__(self, layer: Sequence[BertLayer]):
         self.layer = layer
-        share_scratch(l.attention for l in layer if isinstance(l, BertLayer))
 
     def __call__(self, hidden_states: AnyTensor, attention_mask: Optional[AnyTensor] = None,
                  head_mask: Optional[AnyTensor] = None, output_attentions: Optional[bool] = False,

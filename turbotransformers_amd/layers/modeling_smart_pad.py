@@ -16,8 +16,8 @@ from .. import cxx
 from .modeling_bert import (BertEmbeddings, BertIntermediate, BertOutput, BertPooler, PoolingMap, PoolingType,
                             SequencePool, _require_gpu)
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, share_scratch, try_convert,
-                    use_current_stream, weight_in_out)
+from .utils import (AnyTensor, convert2tt_tensor, create_empty_if_none, to_param_dict, try_convert, use_current_stream,
+                    weight_in_out)
 
 __all__ = ['MultiHeadedAttentionSmartBatch', 'BertLayerSmartBatch', 'BertEncoderSmartBatch',
            'BertModelNoPoolerSmartBatch', 'BertModelSmartBatch']
@@ -114,7 +114,6 @@ class BertLayerSmartBatch:
 class BertEncoderSmartBatch:
     def __init__(self, layer: Sequence[BertLayerSmartBatch]):
         self.layer = layer
-        share_scratch(l.attention for l in layer if isinstance(l, BertLayerSmartBatch))
 
     def __call__(self, hidden_states: AnyTensor, query_seq_len_list: Sequence[int],
                  attention_mask: Optional[AnyTensor] = None, head_mask: Optional[AnyTensor] = None,
@@ -123,12 +122,13 @@ class BertEncoderSmartBatch:
         all_hidden_states, all_attentions = (), ()
         hidden_states = try_convert(hidden_states)
         attention_mask = try_convert(attention_mask)
-        if attention_mask is not None and not output_attentions and not output_hidden_states and self._plain_layers():
+        if not output_attentions and not output_hidden_states and self._plain_layers():
             # nothing but the last hidden state is asked for: the layer loop runs inside the extension
             use_current_stream()
+            lens = [int(x) for x in query_seq_len_list]
+            mask = attention_mask if attention_mask is not None else smart_pad_mask(lens)  # (what each layer would make for itself)
             last = cxx.Tensor.create_empty()
-            cxx.run_smart_batch_layers([(l.attention, l.intermediate, l.output) for l in self.layer], hidden_states, attention_mask,
-                                       [int(x) for x in query_seq_len_list], last)
+            cxx.run_smart_batch_layers([(l.attention, l.intermediate, l.output) for l in self.layer], hidden_states, mask, lens, last)
             return (convert_returns_as_type(last, return_type), )
         for layer in self.layer:
             layer_outputs = layer(hidden_states, query_seq_len_list, attention_mask,

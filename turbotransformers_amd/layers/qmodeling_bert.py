@@ -15,7 +15,7 @@ import torch
 from .. import cxx
 from .modeling_bert import BertAttention, BertEmbeddings, BertPooler, PoolingMap, PoolingType, SequencePool, _require_gpu
 from .return_type import ReturnType, convert_returns_as_type
-from .utils import convert2tt_tensor, create_empty_if_none, share_scratch, to_param_dict, try_convert, use_current_stream, weight_in_out
+from .utils import convert2tt_tensor, create_empty_if_none, to_param_dict, try_convert, use_current_stream, weight_in_out
 
 __all__ = ['QBertIntermediate', 'QBertOutput', 'QBertAttention', 'QBertLayer', 'QBertEncoder', 'QBertModel']
 
@@ -27,10 +27,10 @@ class QBertIntermediate:
         self.linear = cxx.QuantizedLinear(convert2tt_tensor(weight_in_out(p['dense.weight'])),
                                           convert2tt_tensor(p['dense.bias']), "gelu")
 
-    def __call__(self, input_tensor, return_type: Optional[ReturnType] = None):
+    def __call__(self, input_tensor, return_type: Optional[ReturnType] = None, lender=None):
         use_current_stream()
         out = cxx.Tensor.create_empty()
-        self.linear(try_convert(input_tensor), out)
+        self.linear(try_convert(input_tensor), out, lender.linear if lender is not None else None)
         return convert_returns_as_type(out, return_type)
 
     @staticmethod
@@ -46,10 +46,10 @@ class QBertOutput:
                                                               convert2tt_tensor(p['LayerNorm.weight']),
                                                               convert2tt_tensor(p['LayerNorm.bias']))
 
-    def __call__(self, intermediate_output, attention_output, return_type: Optional[ReturnType] = None):
+    def __call__(self, intermediate_output, attention_output, return_type: Optional[ReturnType] = None, lender=None):
         use_current_stream()
         out = cxx.Tensor.create_empty()
-        self.linear(try_convert(intermediate_output), out)
+        self.linear(try_convert(intermediate_output), out, lender.linear if lender is not None else None)
         self.turbo_bias_layernorm(try_convert(attention_output), out)
         return convert_returns_as_type(out, return_type)
 
@@ -60,12 +60,12 @@ class QBertOutput:
 
 class QBertAttention(cxx.QuantizedBertAttention):
     def __call__(self, input_tensor, attention_mask=None, output_attentions=False,
-                 return_type: Optional[ReturnType] = None):
+                 return_type: Optional[ReturnType] = None, lender=None):
         use_current_stream()
         context_layer = cxx.Tensor.create_empty()
         attn_probs = cxx.Tensor.create_empty() if output_attentions else None
         super().__call__(try_convert(input_tensor), try_convert(create_empty_if_none(attention_mask)), context_layer,
-                         attn_probs)
+                         attn_probs, lender)
         out = (convert_returns_as_type(context_layer, return_type), )
         if output_attentions:
             out = out + (convert_returns_as_type(attn_probs, ReturnType.turbo_transformers), )
@@ -87,12 +87,14 @@ class QBertLayer:
         self.output = QBertOutput.from_torch(bert_layer.output)
 
     def __call__(self, hidden_states, attention_mask=None, head_mask=None, output_attentions=False,
-                 return_type: Optional[ReturnType] = None):
+                 return_type: Optional[ReturnType] = None, lender=None):
+        """`lender`: another layer of the stack that runs, which holds the tensors of the call."""
+        lent = lambda part: {} if lender is None else {'lender': getattr(lender, part)}
         attn_out = self.attention(hidden_states, attention_mask, output_attentions=output_attentions,
-                                  return_type=ReturnType.turbo_transformers)
+                                  return_type=ReturnType.turbo_transformers, **lent('attention'))
         attention_output = attn_out[0]
-        intermediate_output = self.intermediate(attention_output, return_type=ReturnType.turbo_transformers)
-        layer_output = self.output(intermediate_output, attention_output, return_type=return_type)
+        intermediate_output = self.intermediate(attention_output, return_type=ReturnType.turbo_transformers, **lent('intermediate'))
+        layer_output = self.output(intermediate_output, attention_output, return_type=return_type, **lent('output'))
         return (layer_output, ) + attn_out[1:]
 
     @staticmethod
@@ -103,10 +105,6 @@ class QBertLayer:
 class QBertEncoder:
     def __init__(self, layers):
         self.layer = layers
-        plain = [l for l in layers if isinstance(l, QBertLayer)]
-        share_scratch(l.attention for l in plain)
-        share_scratch(l.intermediate.linear for l in plain)
-        share_scratch(l.output.linear for l in plain)
 
     def __call__(self, hidden_states, attention_mask=None, head_mask=None, output_attentions=False,
                  output_hidden_states=False, return_type: Optional[ReturnType] = None):
@@ -117,7 +115,7 @@ class QBertEncoder:
             if output_hidden_states:
                 all_hidden_states = all_hidden_states + (hidden_states, )
             layer_outputs = layer(hidden_states, attention_mask, output_attentions=output_attentions,
-                                  return_type=ReturnType.turbo_transformers)
+                                  return_type=ReturnType.turbo_transformers, **self._lent(layer))
             hidden_states = layer_outputs[0]
             if output_attentions:
                 all_attentions = all_attentions + (layer_outputs[1], )
@@ -127,6 +125,16 @@ class QBertEncoder:
         if output_attentions:
             outputs = outputs + (all_attentions, )
         return outputs
+
+    def _lent(self, layer):
+        """The layers run one after the other, on the tensors of the first: those built from the stock sub-layers, as the first is."""
+        first = self.layer[0]
+        if (type(layer) is QBertLayer and type(first) is QBertLayer and type(layer.attention) is type(first.attention)
+                and type(layer.attention) in (QBertAttention, BertAttention)
+                and type(layer.intermediate) is type(first.intermediate) is QBertIntermediate
+                and type(layer.output) is type(first.output) is QBertOutput):
+            return {'lender': first}
+        return {}
 
     @staticmethod
     def from_torch(encoder, quantize_attention: bool = True):

@@ -59,11 +59,3 @@ def use_current_stream():
 def weight_in_out(linear_weight: torch.Tensor) -> torch.Tensor:
     """nn.Linear keeps [out, in]; the layer classes take [in, out] (y = x W)."""
     return torch.clone(torch.t(linear_weight.detach()).contiguous())
-
-
-def share_scratch(parts):
-    """Let the parts of a stack that run one after the other hold the tensors of a call in one place."""
-    parts = list(parts)
-    for part in parts[1:]:
-        if type(part) is type(parts[0]) and hasattr(part, 'share_scratch'):
-            part.share_scratch(parts[0])
