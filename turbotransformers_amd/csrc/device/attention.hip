@@ -148,16 +148,14 @@ __device__ __forceinline__ void store_context(char* stage_base, int wave, int la
   }
 }
 
-template <typename T, bool PACKED, bool VT, int NW>
+// READS: Ahead or NothingAhead
+template <typename T, bool PACKED, bool VT, int NW, typename READS>
 __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                  const T* __restrict__ v, const float* __restrict__ mask,
                                                                  T* __restrict__ out, const int32_t* __restrict__ cu,
                                                                  int heads, int seq, int v_pitch, float scale_log2e,
-                                                                 float inv_scale, const Ahead ahead) {
-  if ((int)blockIdx.y >= ahead.rows) {
-    touch_ahead(ahead, (int)((blockIdx.y - ahead.rows) * gridDim.x + blockIdx.x), (int)((gridDim.y - ahead.rows) * gridDim.x));
-    return;
-  }
+                                                                 float inv_scale, const READS ahead) {
+  if (has_read_ahead(ahead)) return;
   // one LDS block: [2 x K tile | 2 x V^T tile | 2 x mask]; the front is reused for the output tile
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
   constexpr int kBQ = NW * 32;    // queries per workgroup
@@ -177,7 +175,8 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   const int major = (PACKED ? blockIdx.x : blockIdx.y) / heads, head = (PACKED ? blockIdx.x : blockIdx.y) - major * heads;
   const int block = PACKED ? major : blockIdx.x;
   int b = PACKED ? blockIdx.y : major;
-  if (PACKED && seq > kOrderMinLength && gridDim.x * ahead.rows > kOrderMinWorkgroups) b = __builtin_amdgcn_readfirstlane(longest_first(cu, ahead.rows, b, seq));
+  if (PACKED && seq > kOrderMinLength && gridDim.x * computing_rows(ahead) > kOrderMinWorkgroups)
+    b = __builtin_amdgcn_readfirstlane(longest_first(cu, computing_rows(ahead), b, seq));
   const int bh = b * heads + head;
   const int q0 = block * kBQ + wave * 32;
 
@@ -383,13 +382,6 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
-  Ahead read_ahead{};
-  if (dtype != TTMI_F32) {
-    const unsigned more = ahead_rows(ahead, (int64_t)grid.x * grid.y, grid.x, (int64_t)cus * (16 / nw));
-    if (more > 0) read_ahead = *ahead;
-    read_ahead.rows = (int)grid.y;
-    grid.y += more;
-  }
   if (dtype == TTMI_F32) {
     // the per-workgroup maxima: dense fp32 batches whose workgroups fit the slots
     const bool leave_maxima = absmax != nullptr && cu_seqlens == nullptr && (int64_t)grid.x * grid.y <= TTMI_ABSMAX_SLOTS;
@@ -398,9 +390,18 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;
   }
-#define TTMI_FA_LAUNCH(T, PACKED, VT, NW)                                                                              \
-  hipLaunchKernelGGL((fused_attention_kernel<T, PACKED, VT, NW>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, \
-                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale, read_ahead)
+  const unsigned more = ahead_rows(ahead, (int64_t)grid.x * grid.y, grid.x, (int64_t)cus * (16 / nw));
+  Ahead read_ahead = more > 0 ? *ahead : Ahead{};
+  read_ahead.rows = (int)grid.y;
+  grid.y += more;
+#define TTMI_FA_LAUNCH_READING(T, PACKED, VT, NW, READS, WHAT)                                                                \
+  hipLaunchKernelGGL((fused_attention_kernel<T, PACKED, VT, NW, READS>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, \
+                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale, WHAT)
+#define TTMI_FA_LAUNCH(T, PACKED, VT, NW)                                                      \
+  do {                                                                                         \
+    if (more > 0) TTMI_FA_LAUNCH_READING(T, PACKED, VT, NW, Ahead, read_ahead);                \
+    else TTMI_FA_LAUNCH_READING(T, PACKED, VT, NW, NothingAhead, NothingAhead{});              \
+  } while (0)
 #define TTMI_FA_WAVES(T, PACKED, VT)                  \
   do {                                                \
     if (nw == 8) TTMI_FA_LAUNCH(T, PACKED, VT, 8);    \
@@ -419,6 +420,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
 #undef TTMI_FA_LAYOUT
 #undef TTMI_FA_WAVES
 #undef TTMI_FA_LAUNCH
+#undef TTMI_FA_LAUNCH_READING
   return launch_status("fused_attention");
 }
 }  // namespace ttmi

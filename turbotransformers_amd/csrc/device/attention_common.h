@@ -69,6 +69,20 @@ inline unsigned ahead_rows(const Ahead* ahead, int64_t workgroups, int64_t width
   return (unsigned)ceil_div(std::max(cus - workgroups, cus / 2), width);
 }
 
+// A launch that reads nothing ahead is compiled without the list, whose arrival its workgroups would wait for at their start: us per
+// launch with / without, 12 heads, fp16, 1 x 10 tokens 3.84 / 3.72, 8 x 128 5.17 / 5.02, 8 x 256 7.54 / 7.44, 20 x 100 5.67 / 5.53.
+struct NothingAhead {};
+// The grid rows that compute; whether this workgroup is not one of them, and has read its share.
+__device__ __forceinline__ int computing_rows(const Ahead& ahead) { return ahead.rows; }
+__device__ __forceinline__ int computing_rows(const NothingAhead&) { return (int)gridDim.y; }
+__device__ __forceinline__ bool has_read_ahead(const Ahead& ahead) {
+  if ((int)blockIdx.y < ahead.rows) return false;
+  const int width = (int)(gridDim.x * gridDim.z);
+  touch_ahead(ahead, (int)(blockIdx.y - ahead.rows) * width + (int)(blockIdx.z * gridDim.x + blockIdx.x), (int)(gridDim.y - ahead.rows) * width);
+  return true;
+}
+__device__ __forceinline__ bool has_read_ahead(const NothingAhead&) { return false; }
+
 // D = A B + C over one 16-byte piece of both operands: eight K indices per half-wavefront in one instruction (16-bit types), or
 // four, one per instruction (fp32)
 template <typename T, typename Piece>

@@ -31,12 +31,12 @@ struct Projection {
   float* partial;    // [heads, batch * seq, n]
 };
 
-// V is [B,h,d,v_pitch]
-template <typename T, int NW, bool PROJECT>
+// V is [B,h,d,v_pitch]; READS: Ahead or NothingAhead
+template <typename T, int NW, bool PROJECT, typename READS>
 __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                                   const T* __restrict__ v, const float* __restrict__ mask,
                                                                   T* __restrict__ out, int heads, int seq, int v_pitch, float scale_log2e, float inv_scale,
-                                                                  float* __restrict__ absmax, const Ahead ahead, const Projection<T> proj) {
+                                                                  float* __restrict__ absmax, const READS ahead, const Projection<T> proj) {
   constexpr int KPC = 16 / (int)sizeof(T);   // elements per 16-byte piece
   constexpr int PIECES = kD / KPC / 2;       // pieces of a row per lane: 4 (16-bit), 8 (fp32)
   constexpr int VPIECES = 4 * (int)sizeof(T) / 2;  // pieces of V per lane and block: two halves of d, 32 keys
@@ -46,11 +46,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
   __shared__ float red[NW];
   __shared__ __align__(16) T ctx[PROJECT ? kQ : 1][kD + 8];
 
-  if ((int)blockIdx.y >= ahead.rows) {
-    const int width = (int)(gridDim.x * gridDim.z);
-    touch_ahead(ahead, (int)(blockIdx.y - ahead.rows) * width + (int)(blockIdx.z * gridDim.x + blockIdx.x), (int)(gridDim.y - ahead.rows) * width);
-    return;
-  }
+  if (has_read_ahead(ahead)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 31, lhalf = lane >> 5;
   const int bh = blockIdx.y, b = bh / heads, head = bh - b * heads;
@@ -253,7 +249,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) acc = mma32<T>(wf[kk], *reinterpret_cast<const u32x4*>(&ctx[lrow][kk * 16 + lhalf * 8]), acc);
     if (q0 + lrow < seq && col0 < hidden) {
-      const int64_t tokens = (int64_t)(ahead.rows / heads) * seq;  // (ahead.rows: batch * heads)
+      const int64_t tokens = (int64_t)(computing_rows(ahead) / heads) * seq;  // (the rows: batch * heads)
       float* dst = proj.partial + (head * tokens + (int64_t)b * seq + q0 + lrow) * hidden + col0 + 4 * lhalf;
 #pragma unroll
       for (int g = 0; g < 4; ++g) *reinterpret_cast<floatx4*>(dst + 8 * g) = floatx4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
@@ -282,7 +278,7 @@ __global__ __launch_bounds__(NW * 64) void split_attention_kernel(const T* __res
     amax = group_max<kWave>(amax);
     if (lane == 0) red[wave] = amax;
     __syncthreads();
-    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), wgs = (int)gridDim.x * ahead.rows;
+    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x), wgs = (int)gridDim.x * computing_rows(ahead);
     if (tid == 0) {
       float mx = red[0];
 #pragma unroll
@@ -298,17 +294,22 @@ template <typename T>
 int launch(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
            int64_t seq, int64_t v_pitch, float scale, float* absmax, const Ahead* ahead, hipStream_t s) {
   const unsigned width = (unsigned)ceil_div(seq, kQ), rows = (unsigned)(batch * heads);
-  const dim3 grid(width, rows + ahead_rows(ahead, (int64_t)width * rows, width, 2 * compute_units()));
-  Ahead read_ahead = grid.y > rows ? *ahead : Ahead{};
-  read_ahead.rows = (int)rows;
+  const unsigned more = ahead_rows(ahead, (int64_t)width * rows, width, 2 * compute_units());
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
+  auto launch_reading = [&](auto waves, const auto& reads) {
+    constexpr int NW = decltype(waves)::value;
+    hipLaunchKernelGGL((split_attention_kernel<T, NW, false, std::decay_t<decltype(reads)>>), dim3(width, rows + more), dim3(NW * 64), 0, s, (const T*)q,
+                       (const T*)k, (const T*)v, mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax, reads, Projection<T>{});
+  };
+  auto launch = [&](auto waves) {
+    if (more == 0) return launch_reading(waves, NothingAhead{});
+    Ahead read_ahead = *ahead;
+    read_ahead.rows = (int)rows;
+    launch_reading(waves, read_ahead);
+  };
   // eight wavefronts where four would each have more than two blocks of keys
-#define TTMI_SPLIT_ATTENTION(NW)                                                                                              \
-  hipLaunchKernelGGL((split_attention_kernel<T, NW, false>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, (const T*)v, \
-                     mask, (T*)out, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, absmax, read_ahead, Projection<T>{})
-  if (seq > 4 * 2 * kKeys) TTMI_SPLIT_ATTENTION(8);
-  else TTMI_SPLIT_ATTENTION(4);
-#undef TTMI_SPLIT_ATTENTION
+  if (seq > 4 * 2 * kKeys) launch(std::integral_constant<int, 8>{});
+  else launch(std::integral_constant<int, 4>{});
   return launch_status("split_attention_kernel");
 }
 
@@ -319,12 +320,16 @@ int launch_projection(const void* q, const void* k, const void* v, const float* 
   auto launch = [&](auto waves) {
     constexpr int NW = decltype(waves)::value;
     const unsigned width = (unsigned)ceil_div(seq, kQ), rows = (unsigned)(batch * heads), groups = (unsigned)ceil_div(heads * kD, NW * 32);
+    const unsigned more = ahead_rows(&ahead, (int64_t)width * groups * rows, (int64_t)width * groups, 2 * compute_units());
+    auto launch_reading = [&](const auto& reads) {
+      hipLaunchKernelGGL((split_attention_kernel<T, NW, true, std::decay_t<decltype(reads)>>), dim3(width, rows + more, groups), dim3(NW * 64), 0, s,
+                         (const T*)q, (const T*)k, (const T*)v, mask, (T*)nullptr, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale,
+                         (float*)nullptr, reads, Projection<T>{(const T*)w, partial});
+    };
+    if (more == 0) return launch_reading(NothingAhead{});
     Ahead read_ahead = ahead;
     read_ahead.rows = (int)rows;
-    const unsigned more = ahead_rows(&ahead, (int64_t)width * groups * rows, (int64_t)width * groups, 2 * compute_units());
-    hipLaunchKernelGGL((split_attention_kernel<T, NW, true>), dim3(width, rows + more, groups), dim3(NW * 64), 0, s, (const T*)q, (const T*)k,
-                       (const T*)v, mask, (T*)nullptr, (int)heads, (int)seq, (int)v_pitch, sl2, inv_scale, (float*)nullptr, read_ahead,
-                       Projection<T>{(const T*)w, partial});
+    launch_reading(read_ahead);
   };
   if (seq > 4 * 2 * kKeys) launch(std::integral_constant<int, 8>{});
   else launch(std::integral_constant<int, 4>{});
