@@ -1143,6 +1143,30 @@ def test_fused_attention_packed_batch(ttmi, oracle, attention_waves, dt, v_trans
     assert max_abs(host(out), want) <= GEMM_TOL[dt] * 2
 
 
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("v_transposed", [False, True])
+@pytest.mark.parametrize("lens", [[70, 5, 129, 33], [300, 5, 257, 256], [512] + [40, 100, 270] * 7])
+def test_fused_attention_packed_batch_has_the_same_bits_whatever_the_pad_rows_hold(ttmi, attention_waves, dt, v_transposed, lens):
+    rng = np.random.default_rng(18)
+    h, d = 3, 64
+    B, longest = len(lens), max(lens)
+    tensors = [rng.standard_normal((B, h, longest, d), np.float32) for _ in range(3)]
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    results = []
+    for pad in (0.0, 1.0, 30.0, np.inf, np.nan):
+        Q, K, V = (t.copy() for t in tensors)
+        for b, n in enumerate(lens):
+            for t in (Q, K, V):
+                t[b, :, n:] = t[b, :, n:] * pad if np.isfinite(pad) else pad
+        dV, pitch = _v_operand(V, dt, v_transposed)
+        out = torch.full((sum(lens), h * d), 9.0, dtype=dev(Q, dt).dtype, device="cuda")
+        dQ, dK = dev(Q, dt), dev(K, dt)
+        ok(ttmi.ttmi_fused_attention(ptr(dQ), ptr(dK), ptr(dV), None, ptr(out), ptr(cu), B, h, longest, d, pitch, 0.125, TTMI_DTYPES[dt], stream()))
+        torch.cuda.synchronize()
+        results.append(out)
+    assert bool(torch.isfinite(results[0].float()).all()) and all(torch.equal(r, results[0]) for r in results)
+
+
 @pytest.mark.parametrize("dt", ["f16", "f32"])
 @pytest.mark.parametrize("B,h,longest", [(64, 5, 140), (65, 4, 300), (130, 3, 129), (22, 12, 260), (90, 4, 128)])
 def test_packed_attention_of_many_sequences(ttmi, dt, B, h, longest):

@@ -192,13 +192,14 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   const T* kb = k + (int64_t)bh * seq * kD;
   const T* vb = v + (int64_t)bh * kD * (VT ? v_pitch : seq);
 
-  // Q fragments: B operand, lane = (query lrow, k-chunk by lhalf); 4 MFMA k-steps cover d = 64.
+  // Q fragments: B operand, lane = (query lrow, k-chunk by lhalf); 4 MFMA k-steps cover d = 64.  Rows past a packed sequence's end may be
+  // uninitialised memory: their scores would say when the wavefront's running maximum moves, and so how its other rows round.
   Chunk16 qf[4];
   {
     const int qi = q0 + lrow;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      if (qi < seq) qf[kk] = *reinterpret_cast<const Chunk16*>(qb + (int64_t)qi * kD + (2 * kk + lhalf) * 8);
+      if (qi < q_len) qf[kk] = *reinterpret_cast<const Chunk16*>(qb + (int64_t)qi * kD + (2 * kk + lhalf) * 8);
       else qf[kk] = Chunk16{{0u, 0u, 0u, 0u}};
     }
   }
