@@ -364,6 +364,30 @@ def test_smart_batch_attention_layer_vs_oracle(tt, oracle):
         assert max_abs(got_attn[b, :, :n], want_attn[b, :, :n]) < 1e-5
 
 
+@pytest.mark.parametrize("lens", [[129], [3, 200, 1], [512], [150, 140], [64] * 5 + [300]])
+def test_smart_batch_attention_of_few_long_requests(tt, oracle, lens):
+    """fp32, few requests of more than 128 tokens: the one-kernel attention against the CPU oracle, and without the memory that the scores
+    [B, h, max_len, max_len] of the chain take, which still runs where the probabilities are asked for."""
+    from turbotransformers_amd import cxx
+    model, cfg = _hf_bert(1, seed=78)
+    layer = model.encoder.layer[0]
+    mha = tt.MultiHeadedAttentionSmartBatch.from_torch(layer.attention)
+    heads, longest = cfg.num_attention_heads, max(lens)
+    x = torch.randn(1, sum(lens), cfg.hidden_size, generator=torch.Generator().manual_seed(3)).cuda()
+    run = lambda **kw: mha(x, x, x, lens, lens, attn_type="self", post_layernorm=True, **kw)
+    short = x[:, :128].contiguous()
+    mha(short, short, short, [128], [128], attn_type="self", post_layernorm=True, need_attn=False)  # lays the weights out
+    before = cxx.allocator_stats()["bytes_live"]
+    out = run(need_attn=False)[0]
+    # padded Q, K and V, the packed context and result; the scores would be twice a padded tensor at 129 tokens, more beyond
+    assert cxx.allocator_stats()["bytes_live"] - before < 6 * len(lens) * longest * cfg.hidden_size * 4
+    w = {k: v.detach().cpu().numpy() for k, v in layer.named_parameters()}
+    mask = np.where(np.arange(longest)[None, :] < np.array(lens)[:, None], 0.0, -1e9).astype(np.float32).reshape(len(lens), 1, longest)
+    want, _ = oracle.smart_attention(host(x), mask, oracle_layer_weights(w), lens, heads)
+    assert max_abs(host(out), want) < 1e-4
+    assert max_abs(host(run()[0]), want) < 1e-4
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 def test_albert_model_vs_huggingface(tt, dtype):
     from transformers import AlbertConfig, AlbertModel

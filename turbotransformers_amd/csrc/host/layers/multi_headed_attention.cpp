@@ -36,7 +36,7 @@ void BertAttention::EnforceShapeAndType() const {
 }
 
 bool MultiHeadedAttention::UseFusedCore(const Tensor& attention_mask, const Tensor* att_score, int64_t head_dim, int dtype,
-                                        int64_t batch, int64_t seq, int64_t heads, bool v_transposed) {
+                                        int64_t batch, int64_t seq, int64_t heads, bool in_halves) {
   bool mask_is_key_mask = true;
   if (!attention_mask.is_null()) {
     mask_is_key_mask = attention_mask.n_dim() == 2 || (attention_mask.n_dim() == 3 && attention_mask.shape(1) == 1) ||
@@ -44,12 +44,14 @@ bool MultiHeadedAttention::UseFusedCore(const Tensor& attention_mask, const Tens
   }
   bool dtype_ok = dtype == TTMI_F16 || dtype == TTMI_BF16;
   if (dtype == TTMI_F32 && batch > 0) {
-    // the fp32 kernel is bound by the matrix pipe: a wavefront's 32 queries cost 3.4 us per 64 keys.  It beats the
-    // three launches of the chain (18 us) when the sequence is short or when there are wavefronts for half the SIMDs
-    // (1024 on this chip).  (batch, seq: of the padded tensors when the batch is a packed one)
+    // On the fp32 instruction (a dense batch with V row-major) the kernel is bound by the matrix pipe: a wavefront's 32 queries cost 3.4 us
+    // per 64 keys.  It beats the three launches of the chain (18 us) when the sequence is short or when there are wavefronts for half
+    // the SIMDs (1024 on this chip).
     const int64_t wave_blocks = batch * heads * ((seq + 31) / 32);
-    // With V transposed, few long sequences take the form that splits the keys (1 x 512: 18 against 34 us).
-    dtype_ok = v_transposed || seq <= 128 || wave_blocks >= 512;
+    // In fp16 halves it takes half of that and always wins: dense with V transposed few long sequences have the form that splits the keys
+    // (1 x 512: 18 against 34 us); packed, us per forward of base, chain / kernel: 1 x 200 tokens 910 / 760, 1 x 512 1332 / 1136, 150 and
+    // 140 992 / 791, 4 x 130 1253 / 1014, 300, 20 and 10 1210 / 921, 3 x 350 1949 / 1384, 8 x 160 1690 / 1342.
+    dtype_ok = in_halves || seq <= 128 || wave_blocks >= 512;
   }
   return att_score == nullptr && head_dim == 64 && dtype_ok && mask_is_key_mask;
 }
@@ -459,7 +461,7 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
   // V stays row-major here: the transposed store needs the row map and a division per group of eight packed rows,
   // and that costs the QKV GEMM more than the scatter costs the attention kernel (20 requests, 6275 tokens:
   // 2.50 against 2.39 ms per forward).
-  const bool fused_core = UseFusedCore(attention_mask, att_score, d, dt, batch, max_seq, heads);
+  const bool fused_core = UseFusedCore(attention_mask, att_score, d, dt, batch, max_seq, heads, true);
   Tensor* qkv[3] = {&scratch.q, &scratch.k, &scratch.v};
   const char* names[3] = {"self/q/Reshape", "self/k/Reshape", "self/v/Reshape"};
   for (int i = 0; i < 3; ++i) {

@@ -68,10 +68,10 @@ class MultiHeadedAttention {
 
   // The whole attention core runs as one kernel when nobody asks for the probabilities
   // (head size 64, additive key mask broadcast over the query rows).
-  // batch, seq, heads: the shape of a dense batch (fp32 takes the fused kernel only for those, and only where it pays:
-  // everywhere if the caller keeps V transposed)
+  // batch, seq, heads: the shape of the batch (fp32 takes the fused kernel only where it pays: everywhere if `in_halves`, which it runs
+  // in on a packed batch or one whose V the caller keeps transposed)
   static bool UseFusedCore(const core::Tensor& attention_mask, const core::Tensor* att_score, int64_t head_dim, int dtype,
-                           int64_t batch = 0, int64_t seq = 0, int64_t heads = 0, bool v_transposed = false);
+                           int64_t batch = 0, int64_t seq = 0, int64_t heads = 0, bool in_halves = false);
 
   WeightRange qkv_weight() const { return qkv_packed_.Range(qkv_weight_); }
   WeightRange dense_weight() const { return dense_packed_.Range(dense_weight_); }
