@@ -1197,8 +1197,7 @@ def test_packed_attention_of_many_sequences(ttmi, dt, B, h, longest):
 @pytest.mark.parametrize("B,S,v_transposed,packed", [(1, 100, True, False), (1, 20, True, False), (2, 200, False, False), (22, 130, True, False),
                                                      (2, 60, True, True)])
 def test_attention_that_reads_ahead(ttmi, dt, B, S, v_transposed, packed):
-    """The same bits with ranges to read ahead, on forms that read them and forms that do not (a full chip, a packed batch, fp32 with V
-    row-major); ranges of nothing, of one word, ragged, and larger than a round of the reading workgroups.  What is no whole word is refused."""
+    """The same bits with ranges to read ahead, on forms that read them and forms that do not (fp32 with V row-major, fp32 packed); ranges of nothing, of one word, ragged, and larger than a round of the reading workgroups.  What is no whole word is refused."""
     import ctypes
     rng = np.random.default_rng(S)
     h, d = 12, 64
@@ -1219,6 +1218,35 @@ def test_attention_that_reads_ahead(ttmi, dt, B, S, v_transposed, packed):
     ok(rc2)
     assert torch.equal(got, want) and bool(torch.isfinite(want.float()).all())
     assert run([4, 2])[0] != 0 and run([-4])[0] != 0
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("B,longest,packed,v_transposed", [(20, 500, True, False), (20, 500, True, True), (3, 300, True, False), (64, 500, True, False),
+                                                           (64, 130, False, True), (64, 130, False, False)])
+def test_attention_that_reads_ahead_beside_many_workgroups(ttmi, dt, B, longest, packed, v_transposed):
+    """The same where the workgroups nearly fill the chip: ragged packed batches of more than 256 (whose sequences the kernel orders by
+    their lengths, for which it has to know the rows that only read), and, of 64 sequences, more than the chip holds at a time, which
+    read nothing.  NaN in the ranges and behind the sequences reaches no result."""
+    import ctypes
+    rng = np.random.default_rng(B + longest)
+    h, d = 12, 64
+    lens = [longest] + rng.integers(5, longest, B - 1).tolist() if packed else [longest] * B
+    cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+    Q, K, V = (rng.standard_normal((B, h, longest, d), np.float32) for _ in range(3))
+    for b, n in enumerate(lens):
+        Q[b, :, n:], K[b, :, n:], V[b, :, n:] = np.nan, np.nan, np.nan
+    Q, K, (V, pitch) = dev(Q, dt), dev(K, dt), _v_operand(V, dt, v_transposed)
+    ranges = [torch.full((n, ), float("nan"), device="cuda") for n in (300001, 4 << 20)]
+    data = (ctypes.c_void_p * 2)(*[r.data_ptr() for r in ranges])
+
+    def run(sizes):
+        out = torch.full((sum(lens) + 1, h * d), 9.0, dtype=Q.dtype, device="cuda")
+        ok(ttmi.ttmi_fused_attention_ahead(ptr(Q), ptr(K), ptr(V), None, ptr(out), ptr(cu) if packed else None, B, h, longest, d, pitch,
+                                           0.125, TTMI_DTYPES[dt], data, (ctypes.c_int64 * 2)(*sizes), len(sizes), stream()))
+        return out
+
+    want, got = run([]), run([4 * 300001, 16 << 20])
+    assert torch.equal(got, want) and bool(torch.isfinite(want.float()).all()) and bool((want[-1] == 9.0).all())
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])

@@ -1014,6 +1014,23 @@ def test_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
         assert torch.equal(one_call, by_layer) and bool(torch.isfinite(one_call.float()).all())
 
 
+@pytest.mark.parametrize("dtype,layers", [(torch.float32, 3), (torch.float16, 9), (torch.bfloat16, 9)])
+def test_packed_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
+    """The same for packed batches, each twice: few requests, twenty of 5 to 500 tokens (which start with the longest, and leave room to read
+    ahead), as many as take several rounds (which do not read)."""
+    from transformers import BertConfig, BertModel
+    torch.manual_seed(0)
+    cfg = BertConfig(vocab_size=10, hidden_size=1024, num_hidden_layers=layers, num_attention_heads=16, intermediate_size=4096)
+    encoder = tt.BertEncoderSmartBatch.from_torch(BertModel(cfg).to("cuda", dtype).eval().encoder)
+    rng = np.random.default_rng(20)
+    for lens in ([40], [17, 150], [500, 5] + rng.integers(5, 500, 14).tolist(), [300] + rng.integers(5, 200, 39).tolist()):
+        x = torch.randn(1, sum(lens), 1024, device="cuda", dtype=dtype)
+        by_layer = encoder(x, lens, output_hidden_states=True, return_type=tt.ReturnType.TORCH)[0].clone()
+        for _ in range(2):
+            one_call = encoder(x, lens, return_type=tt.ReturnType.TORCH)[0]
+            assert torch.equal(one_call, by_layer) and bool(torch.isfinite(one_call.float()).all())
+
+
 @pytest.mark.parametrize("kind", ["bert", "smart batch", "int8"])
 def test_layers_of_an_encoder_share_their_scratch(tt, kind):
     """The layers of an encoder hold the tensors of a call in one place: the same bits as layers that share nothing, for batches that
