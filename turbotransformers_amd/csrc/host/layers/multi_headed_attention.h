@@ -191,7 +191,9 @@ struct EncoderLayer {
 // all): 5 layers of 1280 / ffn 5120 1 x 128 221 / 224 (192), 4 x 128 328 / 310 (207), 20 x 100 681 / 655 (265), though 12 x 64 373 / 382 (217); 16 of
 // 768 / 1536 4 x 128 591 / 622 (154), 20 x 100 918 / 916 (185); 9 of 768 / 6144 1 x 128 373 / 365 (205), 12 x 64 558 / 522 (223); 32 of 512 /
 // 2048 1 x 128 926 / 946 (194), 4 x 128 1071 / 1051 (200), 8 x 256 1569 / 1525 (224).
-// Nor for fp32 products of up to 32 rows, which take the fp32 weights as they are, all of a workgroup's share at once.
+// Nor for up to 32 rows: those products request all of a workgroup's share of the weights at once (fp32 the fp32 weights as they are), so
+// reading ahead is no sooner, and the attention launch waits for it.  us per forward of large bf16 (600 MB), without / with: 1 x 8 tokens 666 /
+// 711, 1 x 10 677 / 713, 1 x 20 728 / 748, 1 x 32 715 / 726, 2 x 16 719 / 750, 3 x 10 751 / 854, 8 x 4 809 / 811, 32 x 1 822 / 821; fp16 the same.
 bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const core::Tensor& hidden);
 template <typename Attention>
 std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<EncoderLayer<Attention>>& layers, const core::Tensor& hidden) {
