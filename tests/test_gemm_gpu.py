@@ -1766,3 +1766,67 @@ def test_fused_attention_fp32_large_values_at_masked_keys(ttmi, v_transposed, pa
     P2 = torch.where(P == 0, 0.0, P + 2.0**-14 * P.amax(-1, keepdim=True))
     bound = 2.0**-16 * (P @ V.double().abs()) + 3 * 2.0**-22 * (P2 @ _held(V))
     assert bool(((got - P @ V.double()).abs() <= bound).all())
+
+
+def _guarded(rows, cols, dtype):
+    """A matrix with eight rows behind it that nothing may write."""
+    whole = torch.full((rows + 8, cols), 7.0, dtype=dtype, device="cuda")
+    return whole, whole[:rows]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("N,K", [(3072, 128), (776, 256)])
+@pytest.mark.parametrize("beside", [-1, 0, 1])
+def test_products_on_both_sides_of_the_write_through_line(ttmi, dt, N, K, beside):
+    """From 2 MiB of output on a launch writes its stores through L2; the row counts around that line, the last ones of a ragged tile, into a
+    matrix with guard rows."""
+    import ctypes
+    M = -(-(2 << 20) // (N * torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size())) + beside
+    rng = np.random.default_rng(M)
+    A, W, bias = rng.standard_normal((M, K), np.float32), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    dA, dW, db = dev(A, dt), dev(W, dt), dev(bias, dt)
+    want = np.maximum(rounded(A, dt).astype(np.float64) @ rounded(W, dt).T.astype(np.float64) + rounded(bias, dt), 0)
+    weights = [(dW, TTMI_DTYPES[dt])] + ([(_packed(ttmi, dW), capi.F32_PACKED)] if dt == "f32" else [])
+    for w, kind in weights:
+        whole, C = _guarded(M, N, dA.dtype)
+        ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(w), ptr(C), M, N, K, K, K, N, capi.EPI_BIAS_ACT, ctypes.byref(_epi(bias=db, act=capi.ACT_RELU)), kind, stream()))
+        # values of size up to 8, rounded once; fp32: sums of 256 products
+        assert max_abs(host(C), want) <= 2 * GEMM_TOL[dt]
+        assert bool((whole[M:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("beside", [-1, 0, 1])
+def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, beside):
+    """AddBiasLayerNorm by itself and behind a product, row counts around 2 MiB of output."""
+    n, K = 776, 128
+    m = -(-(2 << 20) // (n * torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size())) + beside
+    rng = np.random.default_rng(m)
+    x, res, bias, gamma, beta = (rng.standard_normal(s).astype(np.float32) for s in ((m, n), (m, n), (n,), (n,), (n,)))
+    A, W = rng.standard_normal((m, K), np.float32), (rng.standard_normal((n, K)) / np.sqrt(K)).astype(np.float32)
+    residual = res if shadow else rounded(res, dt)
+
+    def want(base):
+        s = base + residual + rounded(bias, dt).astype(np.float64)
+        return rounded(beta, dt) + rounded(gamma, dt) * (s - s.mean(1, keepdims=True)) / np.sqrt(s.var(1, keepdims=True) + 1e-12)
+
+    d = [ptr(dev(v, dt)) for v in (bias, gamma, beta)]
+    r16, r32 = ptr(dev(res, dt)), ptr(dev(res)) if shadow else None
+    tol = {"f32": 1e-4, "f16": 2e-2, "bf16": 1.2e-1}[dt]  # values of size up to 16, rounded once; in front of it the product may be
+    whole, out = _guarded(m, n, TORCH_DTYPES[dt])
+    out.copy_(dev(x, dt))
+    whole32, out32 = _guarded(m, n, torch.float32)
+    if shadow:
+        ok(ttmi.ttmi_add_bias_layer_norm_residual32(ptr(out), r32, *d, ptr(out32), m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+    else:
+        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), r16, *d, m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+    assert max_abs(host(out), want(rounded(x, dt).astype(np.float64))) <= tol
+    behind, out2 = _guarded(m, n, TORCH_DTYPES[dt])
+    ok(ttmi.ttmi_gemm_bias_layer_norm(ptr(dev(A, dt)), ptr(dev(W, dt)), ptr(out2), None if shadow else r16, r32, *d, ptr(out32) if shadow else None, m, n, K, 1e-12,
+                                      TTMI_DTYPES[dt], stream()))
+    assert max_abs(host(out2), want(rounded(A, dt).astype(np.float64) @ rounded(W, dt).T.astype(np.float64))) <= tol
+    for w in (whole, whole32, behind):
+        assert bool((w[m:] == 7.0).all())

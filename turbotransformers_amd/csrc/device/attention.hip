@@ -123,7 +123,7 @@ __device__ __forceinline__ void attention_tile(const char* kt, const char* vt, c
 // that it leaves as 128-byte rows.  out_head: first element of the head's columns in row 0 of this sequence.
 template <typename T>
 __device__ __forceinline__ void store_context(char* stage_base, int wave, int lane, const floatx16 (&ot)[2], float l_run,
-                                              T* out_head, int row_pitch, int q0, int q_end) {
+                                              T* out_head, int row_pitch, int q0, int q_end, bool through) {
   const int lrow = lane & 31, lhalf = lane >> 5;
   const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
   const float inv = 1.0f / l_tot;
@@ -143,7 +143,9 @@ __device__ __forceinline__ void store_context(char* stage_base, int wave, int la
     const int qi = q0 + r;
     if (qi < q_end) {
       const Chunk16 x = *reinterpret_cast<const Chunk16*>(stage_o + r * (kD + 8) + cchunk * 8);
-      *reinterpret_cast<Chunk16*>(out_head + (int64_t)qi * row_pitch + cchunk * 8) = x;
+      T* const to = out_head + (int64_t)qi * row_pitch + cchunk * 8;
+      if (through) store_through(to, x);
+      else *reinterpret_cast<Chunk16*>(to) = x;
     }
   }
 }
@@ -154,7 +156,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
                                                                  const T* __restrict__ v, const float* __restrict__ mask,
                                                                  T* __restrict__ out, const int32_t* __restrict__ cu,
                                                                  int heads, int seq, int v_pitch, float scale_log2e,
-                                                                 float inv_scale, const READS ahead) {
+                                                                 float inv_scale, bool through, const READS ahead) {
   if (has_read_ahead(ahead)) return;
   // one LDS block: [2 x K tile | 2 x V^T tile | 2 x mask]; the front is reused for the output tile
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
@@ -312,7 +314,7 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
   }
 
   store_context<T>(smem, wave, lane, ot, l_run, out + (int64_t)out_row0 * (heads * kD) + head * kD, heads * kD, q0,
-                   min(q_len, seq));
+                   min(q_len, seq), through);
 }
 
 }  // namespace ttmi
@@ -320,8 +322,8 @@ __global__ __launch_bounds__(NW * 64, 16 / NW) void fused_attention_kernel(const
 namespace ttmi {
 // attention_f32.hip: the fp32 form
 int fused_attention_f32(const float* q, const float* k, const float* v, const float* mask, float* out, const int32_t* cu,
-                        int64_t batch, int64_t heads, int64_t seq, int64_t v_seq_pitch, float scale, int nw, float* absmax,
-                        hipStream_t s);
+                        int64_t batch, int64_t heads, int64_t seq, int64_t v_seq_pitch, float scale, int nw, bool through,
+                        float* absmax, hipStream_t s);
 
 // attention_split.hip: the keys of a head split over the wavefronts of a workgroup
 int split_attention(const void* q, const void* k, const void* v, const float* mask, void* out, int64_t batch, int64_t heads,
@@ -383,11 +385,13 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
+  // (a packed batch: taken as half of the padded one)
+  const bool through = writes_through(batch * heads * seq * kD * (int64_t)dtype_size(dtype) / (cu_seqlens != nullptr ? 2 : 1));
   if (dtype == TTMI_F32) {
     // the per-workgroup maxima: dense fp32 batches whose workgroups fit the slots
     const bool leave_maxima = absmax != nullptr && cu_seqlens == nullptr && (int64_t)grid.x * grid.y <= TTMI_ABSMAX_SLOTS;
     const int rc = fused_attention_f32((const float*)q, (const float*)k, (const float*)v, mask, (float*)out, cu_seqlens, batch,
-                                       heads, seq, v_seq_pitch, scale, nw, leave_maxima ? absmax : nullptr, s);
+                                       heads, seq, v_seq_pitch, scale, nw, through, leave_maxima ? absmax : nullptr, s);
     if (rc == 0 && leave_maxima && slots_written != nullptr) *slots_written = TTMI_ABSMAX_SLOTS;
     return rc;
   }
@@ -397,7 +401,7 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   grid.y += more;
 #define TTMI_FA_LAUNCH_READING(T, PACKED, VT, NW, READS, WHAT)                                                                \
   hipLaunchKernelGGL((fused_attention_kernel<T, PACKED, VT, NW, READS>), grid, dim3(NW * 64), 0, s, (const T*)q, (const T*)k, \
-                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale, WHAT)
+                     (const T*)v, mask, (T*)out, cu_seqlens, (int)heads, (int)seq, (int)v_seq_pitch, sl2, inv_scale, through, WHAT)
 #define TTMI_FA_LAUNCH(T, PACKED, VT, NW)                                                      \
   do {                                                                                         \
     if (more > 0) TTMI_FA_LAUNCH_READING(T, PACKED, VT, NW, Ahead, read_ahead);                \

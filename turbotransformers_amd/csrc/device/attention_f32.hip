@@ -350,7 +350,7 @@ template <int NW, bool VT, bool PACKED, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void fused_attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ mask,
     float* __restrict__ out, const int32_t* __restrict__ cu, int heads, int seq, int v_pitch, float scale_log2e,
-    float inv_scale, float qk_limit, float* __restrict__ absmax) {
+    float inv_scale, float qk_limit, bool through, float* __restrict__ absmax) {
   static_assert(NW == 4 || NW == 8, "four or eight wavefronts");
   constexpr int kBQ = NW * 32;  // queries per workgroup
   // dynamic LDS (lds_bytes<NW>(), more than the 64 KB a kernel gets without asking):
@@ -406,7 +406,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int qi = q0 + r;
     if (qi < q_len) {
       const floatx4 x = *reinterpret_cast<const floatx4*>(stage_o + r * (kD + 4) + cchunk * 4);
-      *reinterpret_cast<floatx4*>(out + ((int64_t)out_row0 + qi) * hd + head * kD + cchunk * 4) = x;
+      float* const to = out + ((int64_t)out_row0 + qi) * hd + head * kD + cchunk * 4;
+      if (through) store_through(to, x);
+      else *reinterpret_cast<floatx4*>(to) = x;
       amax = fmaxf(fmaxf(amax, fmaxf(fabsf(x[0]), fabsf(x[1]))), fmaxf(fabsf(x[2]), fabsf(x[3])));
     }
   }
@@ -434,8 +436,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 
 // Launch; arguments were checked by ttmi_fused_attention.
 int fused_attention_f32(const float* q, const float* k, const float* v, const float* mask, float* out, const int32_t* cu,
-                        int64_t batch, int64_t heads, int64_t seq, int64_t v_seq_pitch, float scale, int nw, float* absmax,
-                        hipStream_t s) {
+                        int64_t batch, int64_t heads, int64_t seq, int64_t v_seq_pitch, float scale, int nw, bool through,
+                        float* absmax, hipStream_t s) {
   dim3 grid((unsigned)ceil_div(seq, nw * 32), (unsigned)(batch * heads));
   if (cu != nullptr) {  // blocks and heads in one row, see the kernel
     TTMI_REQUIRE((int64_t)grid.x * grid.y < (1ll << 31), "attention grid too large");
@@ -457,7 +459,7 @@ int fused_attention_f32(const float* q, const float* k, const float* v, const fl
       }
     }
     hipLaunchKernelGGL(kern, grid, dim3(threads), lds, s, q, k, v, mask, out, cu, (int)heads, (int)seq, (int)v_seq_pitch, sl2,
-                       inv_scale, qk_limit, absmax);
+                       inv_scale, qk_limit, through, absmax);
     return 0;
   };
   const bool vt = v_seq_pitch > 0, packed = cu != nullptr;

@@ -77,6 +77,30 @@ __device__ __forceinline__ void store_vec_unaligned(T* p, const Vec<T, N>& x) {
   reinterpret_cast<UnalignedVec<T, N>*>(p)->x = x;
 }
 
+// ---- stores that do not wait in L2 ---------------------------------------------------------
+// What a launch has stored lies in the L2s (4 MB each) until it ends, and the next launch starts when all of it has been written
+// back: behind a product that stores 12 MB 3.5 us after its last wavefront, 2.2 if the stores went through L2 at once, while other
+// wavefronts still computed.  A store that goes through takes longer (the stores of a 128 x 192 tile 2.0 -> 2.4 us, of a 64 x 96 one
+// 1.1 -> 1.8), so few bytes stay: us a forward of base, never / from 0.5, 1.5, 4.5 MB of a launch on: fp16 1 x 387 tokens 477 / 471, 479, 482;
+// 8 x 128 600 / 583, 585, 590; 8 x 256 829 / 783, 783, 791; fp32 1 x 128 555 / 547, 549, 560; 3 x 128 802 / 778, 780, 784; decoder prefix 8 x 33
+// fp32 667 / 670, 663, 665.  20 x 100 fp16 853 / 814 from 1.5 MB on, 64 x 512 7283 / 7220, 20 packed requests 1875 / 1793.
+// Rows of a transposed V stay wherever they are not whole cache lines: 40 x 100 tokens 1384 / 1465 with them.
+constexpr int64_t kWriteThroughBytes = 2ll << 20;
+inline bool writes_through(int64_t bytes) { return bytes >= kWriteThroughBytes; }
+// An 8- or 16-byte store, aligned to the element.  The compiler does not count it, which makes its waits longer than they need to
+// be, never shorter.  (The no-op: it does not know either that the next instruction must not overwrite the stored registers.)
+template <typename V>
+__device__ __forceinline__ void store_through(void* p, const V& x) {
+  static_assert(sizeof(V) == 16 || sizeof(V) == 8 || sizeof(V) == 4, "one store");
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef uint32_t Quad __attribute__((ext_vector_type(4)));
+  typedef uint32_t Pair __attribute__((ext_vector_type(2)));
+  if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(__builtin_bit_cast(Quad, x)) : "memory");
+  else if constexpr (sizeof(V) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(__builtin_bit_cast(Pair, x)) : "memory");
+  else asm volatile("global_store_dword %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(__builtin_bit_cast(uint32_t, x)) : "memory");
+#endif
+}
+
 // ---- wave64 reductions over groups of G lanes (G power of two, 4 <= G <= 64) ------------
 // Partners come through data-parallel-primitive moves and the row swaps, a few cycles each, where a __shfl_xor is a trip
 // through the LDS unit (~100 cycles, six in a chain: the larger part of a LayerNorm over a few rows).  The order is that

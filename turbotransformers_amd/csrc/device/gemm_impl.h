@@ -137,6 +137,7 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int k_chunk;  // split-K: blockIdx.y owns K range [y*k_chunk, (y+1)*k_chunk) and z passed to the epilogue is y; 0 = whole K
   int slices;   // split-K on the ring kernel: workgroups cover slices x tiles
+  bool write_through;  // 16-byte stores of the output, see writes_through()
   // One-wavefront-per-SIMD kernel only: a column at which a new run of tiles starts (0 = none).  Tile columns
   // [0, split_tiles) cover [0, split_col), the last of them ragged; the tiles after them start at split_col again.
   int split_col, split_tiles;
@@ -1034,7 +1035,8 @@ template <typename T, int ITERS, int AT_ONCE>
 __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const float* __restrict__ ws, int splits, int m, int n,
                                                                       const T* __restrict__ bias, const T* residual,
                                                                       const float* residual32, const T* __restrict__ gamma,
-                                                                      const T* __restrict__ beta, T* out, float* out32, float eps) {
+                                                                      const T* __restrict__ beta, T* out, float* out32, float eps,
+                                                                      bool through) {
   __shared__ float red[2][4];
   const int row = blockIdx.x;
   const int64_t mn = (int64_t)m * n;
@@ -1110,10 +1112,17 @@ __global__ __launch_bounds__(256) void splitk_reduce_layer_norm_kernel(const flo
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         y[j] = to_float(bt[it].v[j]) + to_float(gm[it].v[j]) * rstd * (x[it][j] - mean);
+        asm volatile("" : "+v"(y[j]));  // out is the rounding of the fp32 value, not of the exact multiply-add
         o.v[j] = from_float<T>(y[j]);
       }
-      store_vec<T, 4>(out + (int64_t)row * n + col, o);
-      if (out32 != nullptr) *reinterpret_cast<float4*>(out32 + (int64_t)row * n + col) = make_float4(y[0], y[1], y[2], y[3]);
+      if (through) store_through(out + (int64_t)row * n + col, o);
+      else store_vec<T, 4>(out + (int64_t)row * n + col, o);
+      if (out32 != nullptr) {
+        const float4 whole = make_float4(y[0], y[1], y[2], y[3]);
+        float4* const to = reinterpret_cast<float4*>(out32 + (int64_t)row * n + col);
+        if (through) store_through(to, whole);
+        else *to = whole;
+      }
     }
   }
 }

@@ -144,10 +144,10 @@ struct ColumnQuads {
     }
   }
 };
-// read(i, j, e): element e of the lane's part of block (i, j).
+// read(i, j, e): element e of the lane's part of block (i, j).  through: see writes_through().
 template <int RB, int CB, typename Epi, typename Quads, typename Read>
 __device__ __forceinline__ void store_rows32(const GemmArgs& g, const Epi& epi, const Quads& quads, int z_epi, int m_first, int n_first, int lrow, int lgrp,
-                                             float& amax, const Read& read) {
+                                             float& amax, bool through, const Read& read) {
   using Dest = RingDest<Epi>;
   using Elem = typename Dest::Elem;
   float act_scale = 0.f;
@@ -183,10 +183,25 @@ __device__ __forceinline__ void store_rows32(const GemmArgs& g, const Epi& epi, 
 #pragma unroll
           for (int e = 0; e < 4; ++e) out.v[e] += res.v[e];
         }
-        store_vec<Elem, 4>(col + row_at[i], out);
+        if (through) store_through(col + row_at[i], out);
+        else store_vec<Elem, 4>(col + row_at[i], out);
       }
     }
   }
+}
+
+// Tiles of 32 rows are for launches that store little: they are compiled without the question.  So are those of int8, which come in
+// two forms: its products are short (4 x 128 tokens, the head split in 128 x 64 tiles 7.5 us with the question, 7.2 without).
+enum class Stores { kAsk, kStay, kThrough };
+template <typename Epi>
+constexpr Stores default_stores(int tile_rows) { return tile_rows > 32 && !Dequantises<Epi>::value ? Stores::kAsk : Stores::kStay; }
+// The stores of a launch of whole output tiles: written through where they are many.
+template <typename Epi>
+inline bool stores_through(const GemmArgs& g) {
+  const int64_t bytes = (int64_t)g.m * g.n * g.slices * (int64_t)sizeof(typename RingDest<Epi>::Elem);
+  // a short int8 product is stores for the most part: 4 x 128 tokens 787 / 803 us with its 4.7 and 6.3 MB written through, 20 x 128 (7.9 MB
+  // and more) 1224 / 1179
+  return Dequantises<Epi>::value ? bytes >= (7ll << 20) : writes_through(bytes);
 }
 
 template <int BM, int BN, int NS>
@@ -197,7 +212,7 @@ constexpr int ring_lds_bytes() { return NS * (BM + BN) * kRowBytes; }
 // K step s: multiply its first half while its second half is read and the rest of step s - 1 + NS is requested; wait until
 // step s + 1 has landed (the NS - 2 younger steps stay in flight) and everyone has read step s; multiply the second half
 // while the first half of step s + 1 is read and the first loads of step s + NS go into the stage just freed.
-template <typename T, int BM, int BN, int WM, int WN, int NS, typename Epi>
+template <typename T, int BM, int BN, int WM, int WN, int NS, typename Epi, Stores STORES>
 __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const GemmArgs g, const Epi epi) {
   constexpr int NW = WM * WN;
   constexpr int RB = BM / WM / 16, CB = BN / WN / 16;  // 16 x 16 blocks per wavefront
@@ -377,6 +392,7 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
   };
 
   float amax = 0.f;
+  const bool through = STORES == Stores::kThrough || (STORES == Stores::kAsk && g.write_through);
   bool swap = true;
   if constexpr (HasColumnPass<Epi>::value) swap = !(epi.column_pass() && n0 + wn0 >= epi.first_column_of_pass());
   using Dest = RingDest<Epi>;
@@ -387,7 +403,7 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
       if constexpr (Dequantises<Epi>::value) w_scale = epi.w_scale;
       quads.load(bias, w_scale, n0 + wn0, g.n, lgrp, g.b);
       k_loop(std::true_type{});
-      store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax,
+      store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax, through,
                            [&](int i, int j, int e) __attribute__((always_inline)) { return acc_read(acc[i][j][e]); });
     } else {
 #pragma unroll
@@ -430,7 +446,11 @@ __global__ __launch_bounds__(WM * WN * kWave, 1) void gemm_ring_kernel(const Gem
 #pragma unroll
               for (int e = 0; e < 8; ++e) fin[e] += res[e];
             }
-            store_row8(col_at[p] + row_at[i], fin);
+            Vec<typename Dest::Elem, 8> rounded;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) rounded.v[e] = from_float<typename Dest::Elem>(fin[e]);
+            if (through) store_through(col_at[p] + row_at[i], rounded);
+            else store_vec(col_at[p] + row_at[i], rounded);
           }
         }
       }
@@ -486,13 +506,18 @@ inline int launch_ring(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
   TTMI_REQUIRE(tiles < (1ll << 30), "GEMM grid too large");
   const unsigned grid_x = tiles >= kXcdRemapMinTiles ? (unsigned)(ceil_div(tiles, kNumXcd) * kNumXcd) : (unsigned)tiles;
   if (!absmax_grid_ok(epi, grid_x, 1)) return launch_ring<T, BM, BN, WM, WN, NS>(g, without_absmax(epi), slices, s);
-  auto kern = gemm_ring_kernel<T, BM, BN, WM, WN, NS, Epi>;
-  if (LDS > 64 * 1024) {
-    const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
-    if (rc != 0) return rc;
-  }
-  hipLaunchKernelGGL(kern, dim3(grid_x), dim3(WM * WN * kWave), LDS, s, g, epi);
-  return launch_status("gemm_ring_kernel");
+  g.write_through = stores_through<Epi>(g);
+  auto launch = [&](auto kern) -> int {
+    if (LDS > 64 * 1024) {
+      const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
+      if (rc != 0) return rc;
+    }
+    hipLaunchKernelGGL(kern, dim3(grid_x), dim3(WM * WN * kWave), LDS, s, g, epi);
+    return launch_status("gemm_ring_kernel");
+  };
+  if constexpr (Dequantises<Epi>::value)
+    if (g.write_through) return launch(gemm_ring_kernel<T, BM, BN, WM, WN, NS, Epi, Stores::kThrough>);
+  return launch(gemm_ring_kernel<T, BM, BN, WM, WN, NS, Epi, default_stores<Epi>(BM)>);
 }
 
 // ------------------------------------------------------------------------ selection -----

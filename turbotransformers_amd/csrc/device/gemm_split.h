@@ -409,7 +409,7 @@ __global__ __launch_bounds__(KG * WM * WN * kWave, 1) void gemm_split_kernel(con
     quads.load(epi.bias_ptr(), nullptr, n0 + wn0, g.n, lgrp, g.b);
     k_loop(std::true_type{});
     if (!meet()) return;
-    store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax, read);
+    store_rows32<RB, CB>(g, epi, quads, z_epi, m0 + wm0, n0 + wn0, lrow, lgrp, amax, default_stores<Epi>(BM) == Stores::kAsk && g.write_through, read);
   } else {
     if constexpr (HasColumnPass<Epi>::value) {
       float bj[CB];
@@ -464,6 +464,7 @@ int launch_split(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
     const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
     if (rc != 0) return rc;
   }
+  g.write_through = stores_through<Epi>(g);
   hipLaunchKernelGGL(kern, dim3(grid_x), dim3(KG * WM * WN * kWave), LDS, s, g, epi);
   return launch_status("gemm_split_kernel");
 }

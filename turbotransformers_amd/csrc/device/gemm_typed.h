@@ -147,7 +147,7 @@ void launch_reduce_layer_norm(const float* ws, int slices, int64_t m, int64_t n,
   auto launch = [&](auto iters, auto at_once) {
     hipLaunchKernelGGL((splitk_reduce_layer_norm_kernel<T, decltype(iters)::value, decltype(at_once)::value>), dim3((unsigned)m), dim3(256), 0, s, ws, slices,
                        (int)m, (int)n, (const T*)bias, (const T*)residual, residual_f32, (const T*)gamma, (const T*)beta, (T*)out,
-                       out_f32, eps);
+                       out_f32, eps, writes_through(m * n * (int64_t)(sizeof(T) + (out_f32 != nullptr ? sizeof(float) : 0))));
   };
   // How many slices are on their way at a time: a chain of waits again, but registers that more rows would miss.  Up to 64 rows, where
   // the attention leaves a slice per head, us for both launches with four / eight / twelve / sixteen at a time, 32 tokens: 6 slices 7.7 / 7.8 / 7.8 /

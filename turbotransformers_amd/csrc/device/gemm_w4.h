@@ -366,8 +366,14 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
   // the output matrix of a linear epilogue (the resource ends at row M; the stores are predicated on the row as well)
   const uint32_t ldc_bytes = (uint32_t)LinearDest<Epi>::ldc(epi) * (uint32_t)sizeof(T);
   const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(LinearDest<Epi>::base(epi), 0, (int)min((int64_t)g.m * ldc_bytes, (int64_t)0x7fffffff), 0x00020000);
+  constexpr int kThrough = 16;  // cache policy: sc1, as in store_through()
   auto store_c = [&](Quad x, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
-    __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, 0);
+    if (g.write_through) __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, kThrough);
+    else __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, 0);
+  };
+  auto store_16 = [&](T* p, Quad x) __attribute__((always_inline)) {  // (aligned to the element)
+    if (g.write_through) store_through(p, x);
+    else store_vec_unaligned<T, 8>(p, __builtin_bit_cast(Vec<T, 8>, x));
   };
   // direct stores of the head split: one resource per destination tensor, each [B, heads, S, d] = M x hidden elements
   // (the launcher checks that this is below 2 GiB and that 16 consecutive rows share a sequence)
@@ -375,7 +381,8 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
     if constexpr (DIRECT && HasColumnPass<Epi>::value) {
       T* base = which == 0 ? epi.q : (which == 1 ? epi.k : epi.v);
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)((int64_t)g.m * epi.hidden * (int64_t)sizeof(T)), 0x00020000);
-      __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, 0);
+      if (g.write_through) __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, kThrough);
+      else __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, 0);
     }
   };
 #else
@@ -383,6 +390,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
   auto dma_issue_one = [&](int) {};
   const uint32_t ldc_bytes = 0;
   auto store_c = [&](Quad, uint32_t, uint32_t) {};
+  auto store_16 = [&](T*, Quad) {};
 #endif
   auto dma_issue = [&](auto lo_tag, auto hi_tag) __attribute__((always_inline)) {
     constexpr int LO = decltype(lo_tag)::value, HI = decltype(hi_tag)::value;
@@ -764,8 +772,14 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
               const int ncol = n0 + wn0 + unit_chunk(v) * 8;
               if ((whole_rows || m < m_lim) && (whole_width || ncol < n_lim)) {
                 float* dst = epi.c + ((int64_t)slice * g.m + m) * epi.ldc + ncol;
-                *reinterpret_cast<floatx4*>(dst) = floatx4{out[0], out[1], out[2], out[3]};
-                *reinterpret_cast<floatx4*>(dst + 4) = floatx4{out[4], out[5], out[6], out[7]};
+                const floatx4 lo{out[0], out[1], out[2], out[3]}, hi{out[4], out[5], out[6], out[7]};
+                if (g.write_through) {
+                  store_through(dst, lo);
+                  store_through(dst + 4, hi);
+                } else {
+                  *reinterpret_cast<floatx4*>(dst) = lo;
+                  *reinterpret_cast<floatx4*>(dst + 4) = hi;
+                }
               }
               packed[v] = Quad{0, 0, 0, 0};
             } else {
@@ -817,7 +831,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
             for (int pass = 0; pass < PASSES; ++pass) {
               const int m = row0 + st_row[pass];
               if ((whole_rows || m < m_lim) && (whole_width || n0 + wn0 + st_col[pass] < n_lim))
-                *reinterpret_cast<Quad*>(col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m))) = landed[pass];
+                store_16(col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m)), landed[pass]);
             }
           }
         }
@@ -897,7 +911,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
               const int ncol = n0 + wn0 + j * 32 + p * 8 + rd_col;
               T* dst = vt_base + (int64_t)(j * 32 + p * 8) * epi.v_pitch + row_off;
               if (rows_whole) {
-                if (ncol < n_lim) *reinterpret_cast<Quad*>(dst) = vt_landed[p];
+                if (ncol < n_lim) store_16(dst, vt_landed[p]);
               } else if (in_sequence) {
                 if (ncol < n_lim) store_vec_unaligned<T, 8>(dst, __builtin_bit_cast(Vec<T, 8>, vt_landed[p]));
               } else if (m < m_lim && ncol < n_lim) {
@@ -993,6 +1007,7 @@ inline int launch_w4(GemmArgs g, const Epi& epi, hipStream_t s, int split_col = 
   auto kern = gemm_w4_kernel<T, BN, kW4Block, Epi, AS, DIRECT>;
   const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
   if (rc != 0) return rc;
+  g.write_through = writes_through((int64_t)g.m * g.n * slices * (StoresF32<Epi>::value ? 4 : (int)sizeof(T)));
   hipLaunchKernelGGL(kern, dim3(grid), dim3(kW4Threads), LDS, s, g, epi);
   return launch_status("gemm_w4_kernel");
 }
