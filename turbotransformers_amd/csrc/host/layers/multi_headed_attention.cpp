@@ -419,7 +419,7 @@ void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attenti
 }
 
 bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const Tensor& hidden) {
-  constexpr int64_t kStays = 200ll << 20;
+  constexpr int64_t kStays = 195 * 1000 * 1000;
   const int64_t width = hidden.shape(-1), rows = width > 0 ? hidden.numel() / width : 0;
   const int64_t tensors = rows * (12 * width + ffn) * (int64_t)hidden.element_size();
   return rows > 32 && bytes + tensors > kStays;

@@ -186,11 +186,11 @@ struct EncoderLayer {
 // for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
 // with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call
 // (Q, K, V, context, four of hidden states, two fp32 slices of a product and the intermediate one: rows x (12 x hidden + ffn)) take their
-// part of the cache.  us per forward without / with, fp16 base (170 MB): 1 x 387 tokens 478 / 532 and 4 x 128 471 / 493 (180 MB in all), 12 x 64
-// 527 / 539 (189 MB), 20 x 100 888 / 853 (220 MB), 8 x 256 897 / 843, 40 x 128 1573 / 1518.  The line holds for other widths (MB in
-// all): 5 layers of 1280 / ffn 5120 1 x 128 221 / 224 (192), 4 x 128 328 / 310 (207), 20 x 100 681 / 655 (265), though 12 x 64 373 / 382 (217); 16 of
-// 768 / 1536 4 x 128 591 / 622 (154), 20 x 100 918 / 916 (185); 9 of 768 / 6144 1 x 128 373 / 365 (205), 12 x 64 558 / 522 (223); 32 of 512 /
-// 2048 1 x 128 926 / 946 (194), 4 x 128 1071 / 1051 (200), 8 x 256 1569 / 1525 (224).
+// part of the cache.  The line is 195 MB of both: us per forward without / with, fp16 base (170 MB), 1 x 387 tokens 475 / 542, 4 x 128 463 / 489
+// (182 MB in all), 6 x 128 536 / 532 (189), 8 x 128 587 / 581 (195), 9 x 128 657 / 613 (198), 11 x 128 770 / 681, 3 x 512 861 / 768, and from 208
+// MB on, where the line was, 20 x 100 888 / 853, 40 x 128 1573 / 1518.  It holds for other widths: 5 layers of 1280 / ffn 5120 1 x 128 221 /
+// 224 (192), 4 x 128 328 / 310 (207), 20 x 100 681 / 655 (265), though 12 x 64 373 / 382 (217); 16 of 768 / 1536 4 x 128 591 / 622 (154), 20 x 100 918 / 916 (185); 9 of 768 / 6144
+// 1 x 128 373 / 365 (205), 12 x 64 558 / 522 (223); 32 of 512 / 2048 1 x 128 926 / 946 (194), 4 x 128 1071 / 1051 (200), 8 x 256 1569 / 1525 (224).
 // Nor for up to 32 rows: those products request all of a workgroup's share of the weights at once (fp32 the fp32 weights as they are), so
 // reading ahead is no sooner, and the attention launch waits for it.  us per forward of large bf16 (600 MB), without / with: 1 x 8 tokens 666 /
 // 711, 1 x 10 677 / 713, 1 x 20 728 / 748, 1 x 32 715 / 726, 2 x 16 719 / 750, 3 x 10 751 / 854, 8 x 4 809 / 811, 32 x 1 822 / 821; fp16 the same.
