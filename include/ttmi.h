@@ -421,6 +421,11 @@ TTMI_API int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, i
                              int64_t lda, int64_t ldb, int64_t ldc, int epilogue,
                              const ttmi_epilogue_args* args, int dtype, void* stream);
 
+/* act(a w^T + bias), a [m,k], w [n,k], c [m,n] contiguous: ttmi_gemm_fused with BIAS_ACT, on the kernel that is fastest for the size.
+ * (For GELU over 65 to 128 rows ttmi_gemm_fused keeps the forms that ttmi_gemm_describe names for it.) */
+TTMI_API int ttmi_gemm_bias_act(const void* a, const void* w, const void* bias, void* c, int64_t m, int64_t n, int64_t k, int act,
+                                int dtype, void* stream);
+
 /* ttmi_gemm_fused on LayerNorm(x): x [m,k], w [n,k] and normed [m,k] are contiguous.  One launch for a few rows with the
  * QKV_SPLIT and the BIAS_ACT (ReLU) epilogue; otherwise ttmi_layer_norm_from into `normed` (scratch of the caller, which must
  * not overlap x) and the product from there.  What `normed` holds afterwards is unspecified.

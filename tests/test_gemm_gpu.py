@@ -1830,3 +1830,21 @@ def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, be
     assert max_abs(host(out2), want(rounded(A, dt).astype(np.float64) @ rounded(W, dt).T.astype(np.float64))) <= tol
     for w in (whole, whole32, behind):
         assert bool((w[m:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("M", [1, 64, 65, 97, 128, 129])
+@pytest.mark.parametrize("N,K", [(3072, 768), (776, 96), (130, 64)])
+def test_gemm_bias_act_has_no_named_form(ttmi, dt, M, N, K):
+    """The layers' product with bias and activation, around the rows for which ttmi_gemm_fused keeps the form that ttmi_gemm_describe names."""
+    rng = np.random.default_rng(M + N)
+    A, W, bias = rng.standard_normal((M, K), np.float32), (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    dA, dW, db = dev(A, dt), dev(W, dt), dev(bias, dt)
+    x = torch.from_numpy(rounded(A, dt)).double() @ torch.from_numpy(rounded(W, dt)).double().T + torch.from_numpy(rounded(bias, dt)).double()
+    want = torch.nn.functional.gelu(x, approximate="tanh").numpy()
+    for w, kind in [(dW, TTMI_DTYPES[dt])] + ([(_packed(ttmi, dW), capi.F32_PACKED)] if dt == "f32" else []):
+        whole, C = _guarded(M, N, dA.dtype)
+        ok(ttmi.ttmi_gemm_bias_act(ptr(dA), ptr(w), ptr(db), ptr(C), M, N, K, capi.ACT_GELU, kind, stream()))
+        assert max_abs(host(C), want) <= 2 * GEMM_TOL[dt]  # values of size up to 8, rounded once
+        assert bool((whole[M:] == 7.0).all())

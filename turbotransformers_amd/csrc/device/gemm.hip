@@ -152,9 +152,9 @@ int ttmi_gemm_batched_heads(const void* a, const void* b, void* c, int64_t m, in
   return 0;
 }
 
-int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda,
-                    int64_t ldb, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, int dtype,
-                    void* stream) {
+static int gemm_fused_impl(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda,
+                           int64_t ldb, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, int dtype, bool any_form,
+                           void* stream) {
   TTMI_REQUIRE(a && b && args, "null argument");
   TTMI_REQUIRE(m < (1ll << 31) && n < (1ll << 31) && k < (1ll << 31), "dimension too large");
   TTMI_REQUIRE(lda >= k && ldb >= k, "leading dimension too small");
@@ -167,9 +167,24 @@ int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, int64_t n,
   g.m = (int)m; g.n = (int)n; g.k = (int)k;
   g.lda = lda; g.ldb = ldb;
   g.inner = 1;
+  g.any_form = any_form;
   if (packed) use_packed_weights(g);
   TTMI_DISPATCH_FLOAT(dtype, T, return gemm_fused_typed<T>(g, c, ldc, epilogue, args, (hipStream_t)stream, nullptr));
   return 0;
+}
+
+int ttmi_gemm_fused(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda,
+                    int64_t ldb, int64_t ldc, int epilogue, const ttmi_epilogue_args* args, int dtype,
+                    void* stream) {
+  return gemm_fused_impl(a, b, c, m, n, k, lda, ldb, ldc, epilogue, args, dtype, false, stream);
+}
+
+int ttmi_gemm_bias_act(const void* a, const void* w, const void* bias, void* c, int64_t m, int64_t n, int64_t k, int act, int dtype,
+                       void* stream) {
+  ttmi_epilogue_args args{};
+  args.bias = bias;
+  args.act = act;
+  return gemm_fused_impl(a, w, c, m, n, k, k, k, n, TTMI_EPI_BIAS_ACT, &args, dtype, true, stream);
 }
 
 int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const void* beta, float eps, void* normed, const void* w, void* c,

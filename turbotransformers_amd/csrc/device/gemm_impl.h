@@ -138,6 +138,7 @@ struct GemmArgs {
   int k_chunk;  // split-K: blockIdx.y owns K range [y*k_chunk, (y+1)*k_chunk) and z passed to the epilogue is y; 0 = whole K
   int slices;   // split-K on the ring kernel: workgroups cover slices x tiles
   bool write_through;  // 16-byte stores of the output, see writes_through()
+  bool any_form;       // no form that callers know by its name is kept (ttmi_gemm_bias_act)
   // One-wavefront-per-SIMD kernel only: a column at which a new run of tiles starts (0 = none).  Tile columns
   // [0, split_tiles) cover [0, split_col), the last of them ragged; the tiles after them start at split_col again.
   int split_col, split_tiles;

@@ -30,9 +30,10 @@ struct RingKernel {
   // tiles).  Neither is the fastest since the ring tiles.  us, kept / ring: fp32 128 x 3072 x 768 14.8 / 9.5, 128 x 4096 x
   // 1024 16.7 / 11.9, 128 x 2048 x 512 9.5 / 7.2; fp16 128 x 3072 x 768 8.4 / 5.0, 72 x 3072 x 768 8.3 / 5.1.  Outside these
   // lines they would cost up to four times the ring's time (fp16 128 x 16384 x 4096 114 / 30, fp32 128 x 8192 x 512 18.1 / 11.4).
+  // ttmi_gemm_bias_act, which the layers call, has no such form: us a forward of fp16 base, as ttmi_gemm_fused / so: 1 x 70 tokens 416 / 369, 1 x 128 424 / 378.
   static bool keeps_named_form(const GemmArgs& g) {
     const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T)), tiles = ceil_div(g.m, 64) * ceil_div(g.n, 64);
-    return g.m > 64 && g.m <= 128 && (sizeof(T) == 4 ? ksteps >= 8 && tiles <= 128 : ksteps < 16 && tiles > 64);
+    return !g.any_form && g.m > 64 && g.m <= 128 && (sizeof(T) == 4 ? ksteps >= 8 && tiles <= 128 : ksteps < 16 && tiles > 64);
   }
   static RingPlan plan(const GemmArgs& g, const Epi& epi) {
     // a cut needs an epilogue that the reduction kernel can apply to rows of eight columns

@@ -50,11 +50,8 @@ void BERTEmbedding::operator()(const Tensor& input_ids, const Tensor& position_i
 // ------------------------------------------------------------------------------ FFN -----
 static void GemmBiasAct(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& bias, int act, Tensor* out) {
   const int64_t k = in.shape(-1), m = in.numel() / k;
-  ttmi_epilogue_args args{};
-  args.bias = bias.raw();
-  args.act = act;
-  TT_DEVICE_CALL(ttmi_gemm_fused(in.raw(), w_nk.data, out->mutable_raw(), m, n, k, k, k, n, TTMI_EPI_BIAS_ACT, &args,
-                                 w_nk.DTypeFor(kernels::DeviceDType(in)), Stream()));
+  TT_DEVICE_CALL(ttmi_gemm_bias_act(in.raw(), w_nk.data, bias.raw(), out->mutable_raw(), m, n, k, act,
+                                    w_nk.DTypeFor(kernels::DeviceDType(in)), Stream()));
 }
 
 static void GemmThenAddBiasLayerNorm(const Tensor& in, const WeightRef& w_nk, int64_t n, const Tensor& bias, const Tensor& residual,
