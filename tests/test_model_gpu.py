@@ -917,6 +917,59 @@ def test_multi_headed_attention_context_memory_cache(tt, oracle):
     assert np.isfinite(host(out2)).all()
 
 
+@pytest.mark.parametrize("form", ["plain", "strided", "graded", "tt tensors", "no mask", "user dict"])
+@pytest.mark.parametrize("attn_type", ["self", "context"])
+def test_attention_calls_handled_by_the_extension(tt, form, attn_type):
+    """A call whose results go to torch is handled by the extension, one that brings its own output by the Python wrapper: the same bits,
+    the same cache, whatever the arguments are; what is no tensor is left to the wrapper."""
+    import collections
+    from turbotransformers_amd.layers.utils import convert2tt_tensor
+    B, F, T, H, h = 2, 3, (3 if attn_type == "self" else 5), 256, 4
+    _, _, layer = _make_mha(tt, h, H, seed=5)
+    g = torch.Generator().manual_seed(3)
+    query = torch.randn(B, F, H, generator=g).cuda()
+    memory = query if attn_type == "self" else torch.randn(B, T, H, generator=g).cuda()
+    mask = (torch.rand(B, 1, T + (2 if attn_type == "self" else 0), generator=g) < 0.3).float().cuda() * -1e9
+    past = {k: torch.randn(B, h, 2, H // h, generator=g).cuda() for k in ("self_keys", "self_values")}
+
+    def run(**kw):
+        q, m, k = query, memory, mask
+        if form == "strided":
+            q = torch.stack([query, query], 2)[:, :, 1]
+            m = q if attn_type == "self" else torch.cat([memory, memory], 2)[:, :, :H]
+            k = torch.cat([mask, mask], 2)[:, :, :mask.shape[2]]
+        elif form == "graded":
+            q = query.clone().requires_grad_()
+            m = q if attn_type == "self" else memory.clone().requires_grad_()
+        elif form == "tt tensors":
+            q = convert2tt_tensor(query.clone())
+            m = q if attn_type == "self" else convert2tt_tensor(memory.clone())
+        elif form == "no mask":
+            k = None
+        cache = dict({k2: v.clone() for k2, v in past.items()}, memory_keys=None, memory_values=None)
+        if form == "user dict":
+            cache = collections.OrderedDict(cache)
+        out, attn = layer(m, m, q, mask=k, layer_cache=cache, attn_type=attn_type, pre_layernorm=True, post_add_input=True, **kw)
+        return out, attn, cache
+
+    one, other = run(), run(output=tt.cxx.Tensor.create_empty(), attn=tt.cxx.Tensor.create_empty())
+    assert torch.equal(one[0], other[0]) and torch.equal(one[1], other[1])
+    for name in ("self_keys", "self_values", "memory_keys", "memory_values"):
+        a, b = one[2][name], other[2][name]
+        assert (a is None and b is None) or torch.equal(a, b), name
+    assert one[2]["self_keys"].shape[2] == (5 if attn_type == "self" else 2)
+    for bad in (dict(attn_type=None), dict(attn_type="both"), dict(attn_type=attn_type, layer_cache={"self_keys": torch.zeros(B, h + 1, 2, H // h).cuda()}),
+                dict(attn_type=attn_type, mask="mask")):
+        errors = []
+        for kw in ({}, dict(output=tt.cxx.Tensor.create_empty())):
+            with pytest.raises(Exception) as e:
+                layer(memory, memory, query, **dict(dict(mask=None, layer_cache=None), **bad), **kw)
+            errors.append(type(e.value))
+        assert errors[0] is errors[1], bad
+    with pytest.raises(TypeError):
+        layer(None, memory, query, mask=None, attn_type=attn_type)
+
+
 @pytest.mark.parametrize("T", [1, 9, 130])
 def test_multi_headed_attention_one_memory_for_keys_and_values(tt, T):
     """Keys and values of the same tensor take one product, of two tensors two: the same cache and output, also after the bias

@@ -33,6 +33,121 @@ static void DLPackCapsuleDestructor(PyObject* data) {
   }
 }
 
+static std::unique_ptr<Tensor> FromCapsule(const py::object& capsule) {
+  auto* tensor = static_cast<DLManagedTensor*>(PyCapsule_GetPointer(capsule.ptr(), "dltensor"));
+  if (tensor == nullptr) throw py::error_already_set();
+  TT_ENFORCE(tensor->dl_tensor.strides == nullptr || tensor->dl_tensor.ndim == 0 ||
+                 [&] {
+                   int64_t expect = 1;
+                   for (int i = tensor->dl_tensor.ndim - 1; i >= 0; --i) {
+                     if (tensor->dl_tensor.shape[i] != 1 && tensor->dl_tensor.strides[i] != expect) return false;
+                     expect *= tensor->dl_tensor.shape[i];
+                   }
+                   return true;
+                 }(),
+             "from_dlpack: tensor must be contiguous");
+  PyCapsule_SetName(capsule.ptr(), "used_tensor");
+  return std::make_unique<Tensor>(tensor);
+}
+
+// What the calls below need of torch, handed over once when the package is imported (this module is built without torch's headers).
+struct TorchBridge {
+  PyObject *tensor_type = nullptr, *to_capsule = nullptr, *from_capsule = nullptr;
+  PyObject *requires_grad = nullptr, *detach = nullptr, *is_contiguous = nullptr, *contiguous = nullptr;  // attribute names
+};
+static TorchBridge torch_bridge;
+
+static py::object Owned(PyObject* o) {
+  if (o == nullptr) throw py::error_already_set();
+  return py::reinterpret_steal<py::object>(o);
+}
+
+// A Python argument as a tensor: a Tensor itself, an alias of a torch tensor, an empty one for None.
+struct TensorArg {
+  Tensor* tensor = nullptr;
+  std::unique_ptr<Tensor> own;
+  // false: neither (the caller leaves such arguments to the Python wrappers)
+  bool Take(const py::handle& obj, bool none_is_empty) {
+    if (obj.is_none()) {
+      if (!none_is_empty) return false;
+      own = std::make_unique<Tensor>(nullptr);
+    } else if (py::isinstance<Tensor>(obj)) {
+      tensor = obj.cast<Tensor*>();
+      return true;
+    } else {
+      const TorchBridge& b = torch_bridge;
+      if (b.tensor_type == nullptr || PyObject_IsInstance(obj.ptr(), b.tensor_type) != 1) {
+        PyErr_Clear();
+        return false;
+      }
+      py::object t = py::reinterpret_borrow<py::object>(obj);
+      if (Owned(PyObject_CallMethodObjArgs(t.ptr(), b.is_contiguous, nullptr)).ptr() != Py_True)
+        t = Owned(PyObject_CallMethodObjArgs(t.ptr(), b.contiguous, nullptr));
+      if (Owned(PyObject_GetAttr(t.ptr(), b.requires_grad)).ptr() != Py_False)
+        t = Owned(PyObject_CallMethodObjArgs(t.ptr(), b.detach, nullptr));
+      own = FromCapsule(Owned(PyObject_CallFunctionObjArgs(b.to_capsule, t.ptr(), nullptr)));
+    }
+    tensor = own.get();
+    return true;
+  }
+};
+
+static py::object ToTorch(Tensor& tensor) {
+  const py::capsule capsule(tensor.ToDLPack(), "dltensor", DLPackCapsuleDestructor);
+  return Owned(PyObject_CallFunctionObjArgs(torch_bridge.from_capsule, capsule.ptr(), nullptr));
+}
+
+// MultiHeadedAttention.__call__ of the Python package for arguments that are torch tensors, Tensors or None and results that go to
+// torch: the conversions and the cache dict are handled here instead of in the interpreter.  None where an argument is anything else;
+// nothing has happened then.  A step of six decoder layers is 49 launches and 18 such calls; 8 x 1 tokens, 40 cached,
+// fp16, its host time bounds it: 300 us with the wrappers' conversions, 257 so.
+static py::object CallMultiHeadedAttention(const layers::MultiHeadedAttention& self, const py::object& key, const py::object& value,
+                                           const py::object& query, const py::object& mask, const py::object& layer_cache,
+                                           const py::object& attn_type, bool pre_layernorm, bool post_layernorm, bool post_add_input,
+                                           bool is_trans_weight) {
+  const bool has_cache = !layer_cache.is_none();
+  if (!PyUnicode_Check(attn_type.ptr()) || (has_cache && !PyDict_CheckExact(layer_cache.ptr()))) return py::none();
+  const std::string type = attn_type.cast<std::string>();
+  TensorArg q, k, v, m;
+  if (!q.Take(query, false) || (!key.is(query) && !k.Take(key, false)) || (!value.is(key) && !v.Take(value, false)) || !m.Take(mask, true))
+    return py::none();
+  Tensor* const key_tensor = key.is(query) ? q.tensor : k.tensor;
+  Tensor* const value_tensor = value.is(key) ? key_tensor : v.tensor;
+  std::vector<std::pair<py::object, TensorArg>> entries;
+  std::unordered_map<std::string, Tensor*> cache;
+  if (has_cache) {
+    const py::dict dict = py::reinterpret_borrow<py::dict>(layer_cache);
+    entries.reserve(dict.size());
+    for (const auto& item : dict) {
+      if (!PyUnicode_Check(item.first.ptr())) return py::none();
+      entries.emplace_back(py::reinterpret_borrow<py::object>(item.first), TensorArg{});
+      if (!entries.back().second.Take(item.second, true)) return py::none();
+      cache[item.first.cast<std::string>()] = entries.back().second.tensor;
+    }
+  }
+  Tensor output(nullptr), attn(nullptr);
+  self(*key_tensor, *value_tensor, *q.tensor, *m.tensor, type, &output, &attn, std::move(cache), pre_layernorm, post_layernorm, post_add_input,
+       is_trans_weight);
+  const bool context = type.find("context") != std::string::npos, own = type.find("self") != std::string::npos;
+  for (auto& entry : entries) {
+    const std::string name = entry.first.cast<std::string>();
+    if ((context && name.find("memory") != std::string::npos) || (own && name.find("self") != std::string::npos))
+      if (PyDict_SetItem(layer_cache.ptr(), entry.first.ptr(), ToTorch(*entry.second.tensor).ptr()) != 0) throw py::error_already_set();
+  }
+  py::object out = ToTorch(output);
+  return py::make_tuple(std::move(out), ToTorch(attn));
+}
+
+// The same for the feed-forward blocks.
+template <typename FeedForward>
+static py::object CallFeedForward(const FeedForward& self, const py::object& input, bool is_trans_weight) {
+  TensorArg in;
+  if (!in.Take(input, false)) return py::none();
+  Tensor output(nullptr);
+  self(*in.tensor, &output, is_trans_weight);
+  return ToTorch(output);
+}
+
 template <typename T>
 static Tensor NpArray2Tensor(py::array_t<T, py::array::c_style | py::array::forcecast> array, const std::string& dev_name) {
   if (array.ndim() == 0) throw std::runtime_error("nparray2tensor: numpy array shall not be empty!");
@@ -82,22 +197,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
 
   py::class_<Tensor>(m, "Tensor")
       .def_static("from_dlpack",
-                  [](py::capsule capsule) -> std::unique_ptr<Tensor> {
-                    auto* tensor = static_cast<DLManagedTensor*>(PyCapsule_GetPointer(capsule.ptr(), "dltensor"));
-                    if (tensor == nullptr) throw py::error_already_set();
-                    TT_ENFORCE(tensor->dl_tensor.strides == nullptr || tensor->dl_tensor.ndim == 0 ||
-                                   [&] {
-                                     int64_t expect = 1;
-                                     for (int i = tensor->dl_tensor.ndim - 1; i >= 0; --i) {
-                                       if (tensor->dl_tensor.shape[i] != 1 && tensor->dl_tensor.strides[i] != expect) return false;
-                                       expect *= tensor->dl_tensor.shape[i];
-                                     }
-                                     return true;
-                                   }(),
-                               "from_dlpack: tensor must be contiguous");
-                    PyCapsule_SetName(capsule.ptr(), "used_tensor");
-                    return std::make_unique<Tensor>(tensor);
-                  })
+                  [](py::capsule capsule) { return FromCapsule(capsule); })
       .def("to_dlpack",
            [](Tensor& tensor) -> py::capsule {
              auto* dlpack = tensor.ToDLPack();
@@ -326,6 +426,21 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
       current = target;
     }
   });
+
+  m.def("bind_torch", [](const py::object& tensor_type, const py::object& to_capsule, const py::object& from_capsule) {
+    TorchBridge b;
+    b.tensor_type = tensor_type.inc_ref().ptr();  // (kept for the process, as torch itself is)
+    b.to_capsule = to_capsule.inc_ref().ptr();
+    b.from_capsule = from_capsule.inc_ref().ptr();
+    b.requires_grad = PyUnicode_InternFromString("requires_grad");
+    b.detach = PyUnicode_InternFromString("detach");
+    b.is_contiguous = PyUnicode_InternFromString("is_contiguous");
+    b.contiguous = PyUnicode_InternFromString("contiguous");
+    torch_bridge = b;
+  });
+  m.def("call_multi_headed_attention", &CallMultiHeadedAttention);
+  m.def("call_feed_forward", &CallFeedForward<layers::PositionwiseFeedForward>);
+  m.def("call_feed_forward", &CallFeedForward<layers::DistrillFFN>);
 
   m.def("set_stream", [](uintptr_t s) { core::DeviceContext::GetInstance().set_stream(reinterpret_cast<void*>(s)); },
         "Enqueue all following kernels on this hipStream_t (pass torch.cuda.current_stream().cuda_stream).");

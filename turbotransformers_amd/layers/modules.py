@@ -28,6 +28,11 @@ class MultiHeadedAttention(cxx.MultiHeadedAttention):
         [B,1,T] or [B,F,T].  `layer_cache` is updated in place with torch tensors, like the reference:
         the memory_* entries after a "context" call, the self_* entries after a "self" call."""
         use_current_stream()
+        if output is None and attn is None and (return_type is None or return_type is ReturnType.TORCH):
+            done = cxx.call_multi_headed_attention(self, key_tensor, value_tensor, query_tensor, mask, layer_cache, attn_type, pre_layernorm,
+                                                   post_layernorm, post_add_input, is_trans_weight)
+            if done is not None:
+                return done
         output = create_empty_if_none(output)
         attn = create_empty_if_none(attn)
         cache = {}
@@ -88,6 +93,10 @@ class _FeedForward:
     def __call__(self, input_tensor: AnyTensor, return_type: Optional[ReturnType] = None, is_trans_weight: bool = False,
                  output: Optional[cxx.Tensor] = None):
         use_current_stream()
+        if output is None and (return_type is None or return_type is ReturnType.TORCH):
+            done = cxx.call_feed_forward(self, input_tensor, is_trans_weight)
+            if done is not None:
+                return done
         output = create_empty_if_none(output)
         super().__call__(try_convert(input_tensor), output, is_trans_weight)
         return convert_returns_as_type(output, return_type)

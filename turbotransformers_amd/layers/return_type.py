@@ -11,6 +11,7 @@ __all__ = ['ReturnType', 'convert_returns_as_type']
 
 
 _capsule_to_torch = getattr(torch._C, '_from_dlpack', dlpack.from_dlpack)  # a capsule needs no protocol negotiation
+cxx.bind_torch(torch.Tensor, dlpack.to_dlpack, _capsule_to_torch)
 
 
 class ReturnType(enum.Enum):
