@@ -1798,6 +1798,26 @@ def test_products_on_both_sides_of_the_write_through_line(ttmi, dt, N, K, beside
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("beside", [0, 1])
+def test_products_on_both_sides_of_the_line_where_stores_stay_again(ttmi, dt, beside):
+    """Outputs of 144 MiB (16-bit, the 256-row tiles) and 90 MiB (fp32, the split ring) are the largest that are written through."""
+    import ctypes
+    N, K = 3072, 128
+    M = ((90 << 20) // (4 * N) if dt == "f32" else (144 << 20) // (2 * N)) + beside
+    torch.manual_seed(M)
+    A, W, bias = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda") / K**0.5, torch.randn(N, device="cuda")
+    dA, dW, db = (x.to(TORCH_DTYPES[dt]) for x in (A, W, bias))
+    want = (dA.double() @ dW.double().t() + db.double()).relu_()
+    w, kind = (_packed(ttmi, dW), capi.F32_PACKED) if dt == "f32" else (dW, TTMI_DTYPES[dt])
+    whole, C = _guarded(M, N, dA.dtype)
+    ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(w), ptr(C), M, N, K, K, K, N, capi.EPI_BIAS_ACT, ctypes.byref(_epi(bias=db, act=capi.ACT_RELU)), kind, stream()))
+    # values of size up to 8, rounded once; fp32: sums of 128 products
+    assert float((C.double() - want).abs().max()) <= 2 * GEMM_TOL[dt]
+    assert bool((whole[M:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("shadow", [False, True])
 @pytest.mark.parametrize("beside", [-1, 0, 1])
 def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, beside):

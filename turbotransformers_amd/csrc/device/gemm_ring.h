@@ -201,7 +201,9 @@ inline bool stores_through(const GemmArgs& g) {
   const int64_t bytes = (int64_t)g.m * g.n * g.slices * (int64_t)sizeof(typename RingDest<Epi>::Elem);
   // a short int8 product is stores for the most part: 4 x 128 tokens 787 / 803 us with its 4.7 and 6.3 MB written through, 20 x 128 (7.9 MB
   // and more) 1224 / 1179
-  return Dequantises<Epi>::value ? bytes >= (7ll << 20) : writes_through(bytes);
+  // The products of many rounds of tiles stay: 24576 x 1024 x 4096 in bf16, 101 MB of fp32, 196 us / 206 through
+  constexpr int64_t kMostThrough = 90ll << 20;
+  return bytes <= kMostThrough && (Dequantises<Epi>::value ? bytes >= (7ll << 20) : writes_through(bytes));
 }
 
 template <int BM, int BN, int NS>

@@ -250,7 +250,7 @@ constexpr int w4_lds_bytes() {
 // between them, so a store instruction writes sixteen 64-byte segments instead of four 256-byte ones, and the LDS
 // round trip and its waits are gone.  The launcher uses it for the 256-wide tile (measured 1 % faster on the whole
 // BERT-base forward there, level at 192 wide), where the freed LDS also makes room for the third A stage.
-template <typename T, int BN, int MF, typename Epi, int AS = 2, bool DIRECT = false>
+template <typename T, int BN, int MF, typename Epi, int AS = 2, bool DIRECT = false, bool THROUGH = false>
 __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, const Epi epi) {
   static_assert(!DIRECT || ((LinearDest<Epi>::value || HasColumnPass<Epi>::value) && MF == 16),
                 "direct stores: row-major 16-bit outputs or the head split, 16-wide blocks");
@@ -366,14 +366,9 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
   // the output matrix of a linear epilogue (the resource ends at row M; the stores are predicated on the row as well)
   const uint32_t ldc_bytes = (uint32_t)LinearDest<Epi>::ldc(epi) * (uint32_t)sizeof(T);
   const __amdgpu_buffer_rsrc_t rsrc_c = __builtin_amdgcn_make_buffer_rsrc(LinearDest<Epi>::base(epi), 0, (int)min((int64_t)g.m * ldc_bytes, (int64_t)0x7fffffff), 0x00020000);
-  constexpr int kThrough = 16;  // cache policy: sc1, as in store_through()
+  constexpr int kCachePolicy = THROUGH ? 16 : 0;  // sc1, as in store_through()
   auto store_c = [&](Quad x, uint32_t voff, uint32_t soff) __attribute__((always_inline)) {
-    if (g.write_through) __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, kThrough);
-    else __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, 0);
-  };
-  auto store_16 = [&](T* p, Quad x) __attribute__((always_inline)) {  // (aligned to the element)
-    if (g.write_through) store_through(p, x);
-    else store_vec_unaligned<T, 8>(p, __builtin_bit_cast(Vec<T, 8>, x));
+    __builtin_amdgcn_raw_buffer_store_b128(x, rsrc_c, (int)voff, (int)soff, kCachePolicy);
   };
   // direct stores of the head split: one resource per destination tensor, each [B, heads, S, d] = M x hidden elements
   // (the launcher checks that this is below 2 GiB and that 16 consecutive rows share a sequence)
@@ -381,8 +376,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
     if constexpr (DIRECT && HasColumnPass<Epi>::value) {
       T* base = which == 0 ? epi.q : (which == 1 ? epi.k : epi.v);
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)((int64_t)g.m * epi.hidden * (int64_t)sizeof(T)), 0x00020000);
-      if (g.write_through) __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, kThrough);
-      else __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(x, rsrc, (int)voff, (int)soff, kCachePolicy);
     }
   };
 #else
@@ -390,7 +384,6 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
   auto dma_issue_one = [&](int) {};
   const uint32_t ldc_bytes = 0;
   auto store_c = [&](Quad, uint32_t, uint32_t) {};
-  auto store_16 = [&](T*, Quad) {};
 #endif
   auto dma_issue = [&](auto lo_tag, auto hi_tag) __attribute__((always_inline)) {
     constexpr int LO = decltype(lo_tag)::value, HI = decltype(hi_tag)::value;
@@ -772,14 +765,8 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
               const int ncol = n0 + wn0 + unit_chunk(v) * 8;
               if ((whole_rows || m < m_lim) && (whole_width || ncol < n_lim)) {
                 float* dst = epi.c + ((int64_t)slice * g.m + m) * epi.ldc + ncol;
-                const floatx4 lo{out[0], out[1], out[2], out[3]}, hi{out[4], out[5], out[6], out[7]};
-                if (g.write_through) {
-                  store_through(dst, lo);
-                  store_through(dst + 4, hi);
-                } else {
-                  *reinterpret_cast<floatx4*>(dst) = lo;
-                  *reinterpret_cast<floatx4*>(dst + 4) = hi;
-                }
+                *reinterpret_cast<floatx4*>(dst) = floatx4{out[0], out[1], out[2], out[3]};
+                *reinterpret_cast<floatx4*>(dst + 4) = floatx4{out[4], out[5], out[6], out[7]};
               }
               packed[v] = Quad{0, 0, 0, 0};
             } else {
@@ -831,7 +818,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
             for (int pass = 0; pass < PASSES; ++pass) {
               const int m = row0 + st_row[pass];
               if ((whole_rows || m < m_lim) && (whole_width || n0 + wn0 + st_col[pass] < n_lim))
-                store_16(col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m)), landed[pass]);
+                *reinterpret_cast<Quad*>(col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m))) = landed[pass];
             }
           }
         }
@@ -911,7 +898,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
               const int ncol = n0 + wn0 + j * 32 + p * 8 + rd_col;
               T* dst = vt_base + (int64_t)(j * 32 + p * 8) * epi.v_pitch + row_off;
               if (rows_whole) {
-                if (ncol < n_lim) store_16(dst, vt_landed[p]);
+                if (ncol < n_lim) *reinterpret_cast<Quad*>(dst) = vt_landed[p];
               } else if (in_sequence) {
                 if (ncol < n_lim) store_vec_unaligned<T, 8>(dst, __builtin_bit_cast(Vec<T, 8>, vt_landed[p]));
               } else if (m < m_lim && ncol < n_lim) {
@@ -1004,12 +991,24 @@ inline int launch_w4(GemmArgs g, const Epi& epi, hipStream_t s, int split_col = 
   TTMI_REQUIRE(tiles < (1ll << 30), "GEMM grid too large");
   // one persistent workgroup per CU (the LDS allows no second one), a multiple of the XCD count
   const unsigned grid = (unsigned)(std::min<int64_t>(ceil_div(tiles, kNumXcd), std::max(1, compute_units() / kNumXcd)) * kNumXcd);
-  auto kern = gemm_w4_kernel<T, BN, kW4Block, Epi, AS, DIRECT>;
-  const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
-  if (rc != 0) return rc;
-  g.write_through = writes_through((int64_t)g.m * g.n * slices * (StoresF32<Epi>::value ? 4 : (int)sizeof(T)));
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(kW4Threads), LDS, s, g, epi);
-  return launch_status("gemm_w4_kernel");
+  auto launch = [&](auto kern) -> int {
+    const int rc = allow_large_lds(reinterpret_cast<const void*>(kern), LDS);
+    if (rc != 0) return rc;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kW4Threads), LDS, s, g, epi);
+    return launch_status("gemm_w4_kernel");
+  };
+  // 16-bit outputs go through L2 (two forms: the question at each store costs what it gains) unless they are more than the last-level
+  // cache takes beside the operands.  us a forward, all stay / all through: fp16 base 30 x 200 tokens 1785 / 1765, 50 x 141 2060 / 2008, 16 x 512
+  // 2303 / 2243, 48 x 512 (151 MB of intermediate values) 6067 / 5916, 64 x 512 (201 MB) 7054 / 7060; large bf16 24 x 200 4611 / 4544, 32 x 512 (134 MB)
+  // 12520 / 12438, 48 x 512 (201 MB) 19493 / 19600, 64 x 512 (268 MB) 23950 / 24600.  The head split, whose transposed V stays, comes to its end
+  // sooner: 24576 x 3072 x 1024 (151 MB) 161 / 170 us a launch.  fp32 outputs, stored 16 bytes of every 32 at a time, stay: 32768 x 1024 x 4096
+  // 142 / 187 us.
+  constexpr int64_t kMostThrough = HasColumnPass<Epi>::value ? 120ll << 20 : 144ll << 20;
+  if constexpr (!StoresF32<Epi>::value) {
+    const int64_t bytes = (int64_t)g.m * g.n * (int64_t)sizeof(T);
+    if (writes_through(bytes) && bytes <= kMostThrough) return launch(gemm_w4_kernel<T, BN, kW4Block, Epi, AS, DIRECT, true>);
+  }
+  return launch(gemm_w4_kernel<T, BN, kW4Block, Epi, AS, DIRECT>);
 }
 
 // The 256 x 192 tile against the tile configurations of the 8-wavefront kernels: the same cost model, with the
