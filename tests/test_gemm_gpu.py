@@ -840,6 +840,21 @@ def test_quantisation_rounds_as_the_division_does(ttmi, exponent):
         assert np.array_equal(host(q), want)
 
 
+@pytest.mark.parametrize("beside", [-3, 0, 5])
+@pytest.mark.parametrize("x_off,q_off", [(0, 0), (0, 4), (1, 0), (0, 1)])
+def test_quantisation_on_both_sides_of_the_write_through_line(ttmi, oracle, beside, x_off, q_off):
+    """From 2 MiB of output on its stores go through L2: counts around that, tensors that start off the vector alignment, guard bytes behind."""
+    n = (2 << 20) + beside
+    whole_x = torch.from_numpy(np.random.default_rng(n).standard_normal(n + 8).astype(np.float32)).cuda()
+    x = whole_x[x_off:x_off + n]
+    whole_q = torch.full((n + 32, ), 99, dtype=torch.int8, device="cuda")
+    q, scale = whole_q[q_off:q_off + n], torch.full((capi.QUANT_SCALE_FLOATS, ), float("nan"), device="cuda")
+    ok(ttmi.ttmi_quantize_rows_i8(ptr(x), ptr(q), ptr(scale), 1, n, stream()))
+    want, want_scale = oracle.quantize_tensor_i8(host(x).reshape(1, n))
+    assert np.array_equal(host(q), want.reshape(-1)) and host(scale)[0] == np.float32(want_scale)
+    assert bool((whole_q[:q_off] == 99).all()) and bool((whole_q[q_off + n:] == 99).all())
+
+
 def test_int8_linear_pipeline(ttmi, oracle):
     """quantize -> int8 GEMM -> dequant+bias, against the oracle's statement of the same scheme."""
     rng = np.random.default_rng(3)
