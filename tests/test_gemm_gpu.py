@@ -855,6 +855,20 @@ def test_quantisation_on_both_sides_of_the_write_through_line(ttmi, oracle, besi
     assert bool((whole_q[:q_off] == 99).all()) and bool((whole_q[q_off + n:] == 99).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [512 * 1024, 512 * 1024 + 1, 512 * 1024 + 2044, 512 * 1024 + 2048, 513 * 1024 + 1027, (2 << 20) - 2045])
+@pytest.mark.parametrize("x_off", [0, 1])
+def test_quantisation_with_two_loads_a_lane(ttmi, oracle, n, x_off):
+    """From 512 Ki to 2 Mi values a workgroup takes 2048 of them: counts next to the line and to whole workgroups, guard bytes behind."""
+    x = torch.from_numpy(np.random.default_rng(n).standard_normal(n + 8).astype(np.float32)).cuda()[x_off:x_off + n]
+    whole_q = torch.full((n + 32, ), 99, dtype=torch.int8, device="cuda")
+    scale = torch.full((capi.QUANT_SCALE_FLOATS, ), float("nan"), device="cuda")
+    ok(ttmi.ttmi_quantize_rows_i8(ptr(x), ptr(whole_q), ptr(scale), 1, n, stream()))
+    want, want_scale = oracle.quantize_tensor_i8(host(x).reshape(1, n))
+    assert np.array_equal(host(whole_q[:n]), want.reshape(-1)) and host(scale)[0] == np.float32(want_scale)
+    assert bool((whole_q[n:] == 99).all())
+
+
 def test_int8_linear_pipeline(ttmi, oracle):
     """quantize -> int8 GEMM -> dequant+bias, against the oracle's statement of the same scheme."""
     rng = np.random.default_rng(3)

@@ -57,8 +57,11 @@ __device__ __forceinline__ int quantize_one(float x, float scale, float inv_scal
 // partial: `partials` per-workgroup maxima of |x|, written by absmax_kernel (then scale_dev + 2) or by the kernel
 // that produced x.
 // A workgroup quantises VECS * 1024 elements.  Bound by the traffic of x, and for a few MB by its waits: the elements are
-// requested before the maxima are reduced (2560 x 768: 4.1 -> 3.4 us).  Four 16-byte loads per lane where there is more work
-// than one round of workgroups (2560 x 3072: 8.4 -> 7.2 us), one below that, where the lane's own chain counts.
+// requested before the maxima are reduced (2560 x 768: 4.1 -> 3.4 us).  Four 16-byte loads per lane from 2 MiB of values on
+// (2560 x 3072: 8.4 us with one, 7.2), two from 512 Ki to there, where four leave a second round of workgroups half empty, one
+// below that, where the lane's own chain counts.  us a forward of base, passes of 512 Ki to 2 Mi values with four / one / two: 1 x 200 tokens
+// 824 / 815 / 814, 4 x 128 774 / 777 / 773, 10 x 100 889 / 874 / 873, 16 x 100 1002 / 1001 / 986, 13 x 160 1291 / 1306 / 1289, 20 x 128 1159 / 1181 /
+// 1154; two for the passes of 2 MiB and more as well: 20 x 128 1179.
 template <int VECS, bool THROUGH = false>
 __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__ x, int8_t* __restrict__ q,
                                                        float* __restrict__ scale_dev, const float* __restrict__ partial,
@@ -104,7 +107,7 @@ static int launch_quantize(const float* x, int8_t* q, float* scale_dev, const fl
   else if (ceil_div(n, 1024) <= 512)
     hipLaunchKernelGGL(quantize_kernel<1>, dim3((unsigned)ceil_div(n, 1024)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
   else
-    hipLaunchKernelGGL(quantize_kernel<4>, dim3((unsigned)ceil_div(n, 4096)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
+    hipLaunchKernelGGL(quantize_kernel<2>, dim3((unsigned)ceil_div(n, 2048)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
   return launch_status("quantize_kernel");
 }
 
