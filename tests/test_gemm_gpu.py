@@ -1883,6 +1883,27 @@ def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, be
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("n,rows_a_group", [(768, None), (64, 16), (1024, 4)])
+def test_layer_norm_of_few_rows_takes_one_wavefront_a_workgroup(ttmi, dt, n, rows_a_group):
+    """Row counts on both sides of 255 workgroups of four wavefronts, and ones that leave a wavefront partly idle."""
+    per = rows_a_group or (4 if dt == "f32" else 8)
+    rng = np.random.default_rng(n)
+    for m in (1, 3, 2 * per + 1, 255 * per - 1, 255 * per, 255 * per + 1):
+        x, res = rng.standard_normal((m, n), np.float32), rng.standard_normal((m, n), np.float32)
+        bias, gamma, beta = (rng.standard_normal(n).astype(np.float32) for _ in range(3))
+        whole, out = _guarded(m, n, TORCH_DTYPES[dt])
+        out.copy_(dev(x, dt))
+        held = [dev(v, dt) for v in (res, bias, gamma, beta)]
+        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), *[ptr(v) for v in held], m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+        s = rounded(x, dt).astype(np.float64) + rounded(res, dt) + rounded(bias, dt)
+        want = rounded(beta, dt) + rounded(gamma, dt) * (s - s.mean(1, keepdims=True)) / np.sqrt(s.var(1, keepdims=True) + 1e-12)
+        # values of size up to 16, rounded once
+        assert max_abs(host(out), want) <= {"f32": 1e-4, "f16": 2e-2, "bf16": 1.2e-1}[dt]
+        assert bool((whole[m:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
 @pytest.mark.parametrize("M", [1, 64, 65, 97, 128, 129])
 @pytest.mark.parametrize("N,K", [(3072, 768), (776, 96), (130, 64)])
 def test_gemm_bias_act_has_no_named_form(ttmi, dt, M, N, K):

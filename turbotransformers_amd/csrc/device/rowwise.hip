@@ -3,13 +3,15 @@
 // Layout idea shared by both: a row is owned by a group of G lanes of one wavefront
 // (G = 8..64); every lane keeps ITERS 16-byte vectors of the row in registers, so the row
 // is read from HBM once and written once, and the two reductions are wave64 shuffles with
-// no LDS and no block barrier.  A block is 256 threads = 4 wavefronts = 256/G rows.
+// no LDS and no block barrier.  A block is 256 threads = 4 wavefronts = 256/G rows
+// (LayerNorm over few rows: one wavefront).
 // Rows too long for the register budget go to a block-per-row fallback.
 #include "common.h"
 
 namespace ttmi {
 
 constexpr int kBlock = 256;
+constexpr int kCus = 256;  // compute units
 
 // --------------------------------------------------------------------------- LayerNorm --
 // x = out (+ input + bias); mean = sum(x)/n; var = sum(x*x)/n - mean^2;
@@ -23,13 +25,13 @@ constexpr int kBlock = 256;
 // absmax (optional): TTMI_ABSMAX_SLOTS floats; workgroup b writes max|result| of its rows to slot b and workgroup 0
 // zeroes the slots past the grid (the launcher passes it only when the grid fits), so that the dynamic quantisation
 // of the next Linear's input finds its scale without a pass of its own.
-template <typename T, int VEC, int G, int ITERS, bool ADD, int RES32, bool THROUGH>
-__global__ __launch_bounds__(kBlock) void layer_norm_rows(T* __restrict__ out, const T* __restrict__ input,
+template <typename T, int VEC, int G, int ITERS, bool ADD, int RES32, bool THROUGH, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void layer_norm_rows(T* __restrict__ out, const T* __restrict__ input,
                                                           const T* __restrict__ bias,
                                                           const T* __restrict__ gamma,
                                                           const T* __restrict__ beta, int64_t m, int n,
                                                           float eps, const float* res32, float* out32, float* absmax) {
-  constexpr int ROWS = kBlock / G;
+  constexpr int ROWS = BLOCK / G;
   const int lane = threadIdx.x % G;
   const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / G;
   const bool row_ok = row < m;
@@ -108,18 +110,18 @@ __global__ __launch_bounds__(kBlock) void layer_norm_rows(T* __restrict__ out, c
     }
   }
   if (absmax != nullptr) {
-    __shared__ float red[kBlock / kWave];
+    __shared__ float red[BLOCK / kWave];
     amax = group_max<kWave>(amax);
     if (threadIdx.x % kWave == 0) red[threadIdx.x / kWave] = amax;
     __syncthreads();
     if (threadIdx.x == 0) {
       float mx = 0.f;
 #pragma unroll
-      for (int w = 0; w < kBlock / kWave; ++w) mx = fmaxf(mx, red[w]);
+      for (int w = 0; w < BLOCK / kWave; ++w) mx = fmaxf(mx, red[w]);
       absmax[blockIdx.x] = mx;
     }
     if (blockIdx.x == 0)
-      for (int i = (int)gridDim.x + (int)threadIdx.x; i < TTMI_ABSMAX_SLOTS; i += kBlock) absmax[i] = 0.f;
+      for (int i = (int)gridDim.x + (int)threadIdx.x; i < TTMI_ABSMAX_SLOTS; i += BLOCK) absmax[i] = 0.f;
   }
 }
 
@@ -175,15 +177,24 @@ template <typename T, int VEC, int G, int ITERS, bool ADD, int RES32>
 static int launch_ln_rows(T* out, const T* input, const T* bias, const T* gamma, const T* beta, int64_t m,
                           int n, float eps, const float* res32, float* out32, hipStream_t s, float* absmax, int* slots_written) {
   constexpr int ROWS = kBlock / G;
-  const int64_t grid = ceil_div(m, ROWS);
+  int64_t grid = ceil_div(m, ROWS);
   if (grid > TTMI_ABSMAX_SLOTS) absmax = nullptr;  // more workgroups than slots: the caller finds the maximum itself
   if (slots_written != nullptr) *slots_written = absmax != nullptr ? TTMI_ABSMAX_SLOTS : 0;
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlock), 0, s, out, input, bias, gamma, beta, m, n, eps, res32, out32, absmax);
+  auto launch = [&](auto kern, int block = kBlock) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(block), 0, s, out, input, bias, gamma, beta, m, n, eps, res32, out32, absmax);
   };
+  const bool through = sizeof(T) * VEC == 16 && writes_through(m * n * (int64_t)sizeof(T));
+  // Fewer workgroups than CUs: one wavefront each, so that more CUs take part; the lanes of a row are the same ones.  us a forward, four / one:
+  // decoder prefix 8 x 33 tokens in fp32 (66 / 264 workgroups) 659 / 656, fp16 1 x 387 (49 / 194) 473.3 / 471.5.  (A maximum is one slot
+  // per workgroup of four.)
+  if (absmax == nullptr && !through && grid < kCus) {
+    grid = ceil_div(m, kWave / G);
+    launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, false, kWave>, kWave);
+    return launch_status("layer_norm_rows");
+  }
   // (a form of its own: few rows do without the question, int8 2 x 100 tokens 710 / 700 us)
-  if (sizeof(T) * VEC == 16 && writes_through(m * n * (int64_t)sizeof(T))) launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, true>);
-  else launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, false>);
+  if (through) launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, true, kBlock>);
+  else launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, false, kBlock>);
   return launch_status("layer_norm_rows");
 }
 
