@@ -390,3 +390,30 @@ def test_picking_a_tile_costs_less_than_a_microsecond():
 
     for m, n, k, dt in ((128, 768, 3072, capi.F32), (896, 768, 3072, capi.F32), (8, 768, 3072, capi.F16), (128, 768, 3072, capi.F16)):
         assert best_us(m, n, k, dt, capi.EPI_BIAS) < best_us(m, n, k, dt, capi.EPI_NONE) + 0.8, (m, n, k, dt)
+
+
+def test_kernel_forms_that_write_through_contain_such_stores(tmp_path):
+    """The large tiles are compiled twice, with output stores that stay in L2 and with ones that go through it (the sc1 bit of a
+    store): each form has the stores of its name, whatever epilogue it is for."""
+    import re
+    import shutil
+    objdump = shutil.which("llvm-objdump", path=os.pathsep.join([os.environ.get("PATH", ""), "/opt/rocm/llvm/bin"]))
+    if objdump is None:
+        pytest.skip("no llvm-objdump")
+    os.symlink(capi.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    stores = {}
+    for bundle in sorted(tmp_path.glob("lib.so.*gfx950")):
+        if b"gemm_w4_kernel" not in bundle.read_bytes():
+            continue
+        text = subprocess.run([objdump, "-d", "-C", bundle], check=True, capture_output=True, text=True).stdout
+        for name, body in re.findall(r"^[0-9a-f]+ <(void ttmi::gemm_w4_kernel<.*)>:\n((?:.+\n)+)", text, flags=re.M):
+            found = re.findall(r"\b(?:buffer|global|flat)_store_dwordx4\b.*", body)
+            stores[name] = (len(found), sum(" sc1" in s for s in found))
+    assert len(stores) >= 40
+    for name, (count, through) in stores.items():
+        assert count > 0, name
+        if re.search(r", true>\(", name):  # the last parameter
+            assert through > 0, name
+        else:
+            assert through == 0, name

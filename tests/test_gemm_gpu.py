@@ -1918,3 +1918,52 @@ def test_gemm_bias_act_has_no_named_form(ttmi, dt, M, N, K):
         ok(ttmi.ttmi_gemm_bias_act(ptr(dA), ptr(w), ptr(db), ptr(C), M, N, K, capi.ACT_GELU, kind, stream()))
         assert max_abs(host(C), want) <= 2 * GEMM_TOL[dt]  # values of size up to 8, rounded once
         assert bool((whole[M:] == 7.0).all())
+
+
+def _guarded_heads(B, h, S, d, dtype):
+    """A head-split tensor with eight sequences' worth of one head behind it that nothing may write."""
+    whole = torch.full((B * h * S * d + 8 * S * d, ), 7.0, dtype=dtype, device="cuda")
+    return whole, whole[:B * h * S * d].view(B, h, S, d)
+
+
+@pytest.mark.parametrize("dt,forced", [("f32", False), ("f16", False), ("f16", True), ("bf16", False), ("bf16", True)])
+@pytest.mark.parametrize("v_transposed", [False, True])
+@pytest.mark.parametrize("S", [100, 112, 75])
+@pytest.mark.parametrize("mib", [2, 120])
+def test_head_split_on_both_sides_of_the_write_through_lines(ttmi, dt, forced, v_transposed, S, mib):
+    """From 2 MiB of output on the head split writes Q, K and a row-major V through L2, up to 120 MiB on the large tiles (90 MiB in fp32, which
+    two sequence counts on each side of the other types' line are past): by direct stores where sequences are multiples of 16 and from
+    the strips where not, on tiles of the launcher's choice and on the large ones."""
+    import ctypes
+    h, d = 2, 64
+    H = h * d
+    element = torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size()
+    below = (mib << 20) // (3 * H * element * S)
+    torch.manual_seed(S)
+    if forced:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_LARGE_TILE", 1))
+    try:
+        for B in (below, below + 1):
+            M = B * S
+            A, W, bias = torch.randn(M, H, device="cuda"), torch.randn(3 * H, H, device="cuda") / H**0.5, torch.randn(3 * H, device="cuda")
+            dA, dW, db = (x.to(TORCH_DTYPES[dt]) for x in (A, W, bias))
+            want = (dA.double() @ dW.double().t() + db.double()).view(B, S, 3, h, d).permute(2, 0, 3, 1, 4)
+            pitch = (S + 7) // 8 * 8 + 8 if v_transposed else 0
+            for w, kind in [(dW, TTMI_DTYPES[dt])] + ([(_packed(ttmi, dW), capi.F32_PACKED)] if dt == "f32" else []):
+                held = [_guarded_heads(B, h, S, d, dA.dtype) for _ in range(3)]
+                (_, q), (_, k), (_, v) = held
+                if v_transposed:
+                    whole_v = torch.full((B * h * d * pitch + 8 * pitch, ), 7.0, dtype=dA.dtype, device="cuda")
+                    v = whole_v[:B * h * d * pitch].view(B, h, d, pitch)
+                args = _epi(bias=db, q=q, k=k, v=v, seq=S, heads=h, head_dim=d, v_seq_pitch=pitch)
+                ok(ttmi.ttmi_gemm_fused(ptr(dA), ptr(w), None, M, 3 * H, H, H, H, 3 * H, capi.EPI_QKV_SPLIT, ctypes.byref(args), kind, stream()))
+                if v_transposed:
+                    assert bool((v[..., S:] == 7.0).all()) and bool((whole_v[v.numel():] == 7.0).all())
+                    v = v[..., :S].transpose(2, 3)
+                for got, exact in zip((q, k, v), want):
+                    # values of size up to 8, rounded once; fp32: sums of 128 products
+                    assert float((got.double() - exact).abs().max()) <= 2 * GEMM_TOL[dt]
+                for whole, part in held:
+                    assert bool((whole[part.numel():] == 7.0).all())
+    finally:
+        ok(ttmi.ttmi_set_kernel_switch(b"TTMI_LARGE_TILE", -1))

@@ -255,6 +255,7 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
   static_assert(!DIRECT || ((LinearDest<Epi>::value || HasColumnPass<Epi>::value) && MF == 16),
                 "direct stores: row-major 16-bit outputs or the head split, 16-wide blocks");
   static_assert(sizeof(T) == 2, "16-bit operands");
+  static_assert(!(THROUGH && StoresF32<Epi>::value), "fp32 outputs have no form that writes through");
   static_assert(MF == 32 || MF == 16, "block sizes of the matrix instructions");
   static_assert(AS == 2 || (AS == 3 && MF == 16 && !HasColumnPass<Epi>::value), "three A stages: 16-wide blocks, row-major epilogues");
   constexpr int BM = 256;
@@ -817,8 +818,11 @@ __global__ __launch_bounds__(kW4Threads) void gemm_w4_kernel(const GemmArgs g, c
 #pragma unroll
             for (int pass = 0; pass < PASSES; ++pass) {
               const int m = row0 + st_row[pass];
-              if ((whole_rows || m < m_lim) && (whole_width || n0 + wn0 + st_col[pass] < n_lim))
-                *reinterpret_cast<Quad*>(col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m))) = landed[pass];
+              if ((whole_rows || m < m_lim) && (whole_width || n0 + wn0 + st_col[pass] < n_lim)) {
+                T* const to = col_ptr[pass] + (block_in_one_sequence ? block_part : epi.row_part(m));
+                if constexpr (THROUGH) store_through(to, landed[pass]);
+                else *reinterpret_cast<Quad*>(to) = landed[pass];
+              }
             }
           }
         }
@@ -999,10 +1003,12 @@ inline int launch_w4(GemmArgs g, const Epi& epi, hipStream_t s, int split_col = 
   };
   // 16-bit outputs go through L2 (two forms: the question at each store costs what it gains) unless they are more than the last-level
   // cache takes beside the operands.  us a forward, all stay / all through: fp16 base 30 x 200 tokens 1785 / 1765, 50 x 141 2060 / 2008, 16 x 512
-  // 2303 / 2243, 48 x 512 (151 MB of intermediate values) 6067 / 5916, 64 x 512 (201 MB) 7054 / 7060; large bf16 24 x 200 4611 / 4544, 32 x 512 (134 MB)
-  // 12520 / 12438, 48 x 512 (201 MB) 19493 / 19600, 64 x 512 (268 MB) 23950 / 24600.  The head split, whose transposed V stays, comes to its end
-  // sooner: 24576 x 3072 x 1024 (151 MB) 161 / 170 us a launch.  fp32 outputs, stored 16 bytes of every 32 at a time, stay: 32768 x 1024 x 4096
-  // 142 / 187 us.
+  // 2303 / 2243, 48 x 512 (151 MB of intermediate values) 6067 / 5916, 52 to 64 x 512 (164 to 201 MB) level; large bf16 24 x 200 4611 / 4544, 32 x 512
+  // (134 MB) 12520 / 12438, 48 x 512 (201 MB) 19493 / 19600, 64 x 512 (268 MB) 23950 / 24600.  Of the head split Q, K and a row-major V go, by direct
+  // stores or from the strips (sequences off the 16-grid, us with those of the strips staying / going: fp16 base 50 x 141 1978 / 1961, 30 x 200 1731 /
+  // 1719, 64 x 100 1874 / 1859, 40 x 100 level; large bf16 24 x 200 4533 / 4519, 32 x 200 5748 / 5709); a transposed V stays, and the launch comes to
+  // its end sooner: 24576 x 3072 x 1024 (151 MB) 161 / 170 us.  fp32 outputs, stored 16 bytes of every 32 at a time, stay: 32768 x 1024 x
+  // 4096 142 / 187 us.
   constexpr int64_t kMostThrough = HasColumnPass<Epi>::value ? 120ll << 20 : 144ll << 20;
   if constexpr (!StoresF32<Epi>::value) {
     const int64_t bytes = (int64_t)g.m * g.n * (int64_t)sizeof(T);
