@@ -1967,3 +1967,48 @@ def test_head_split_on_both_sides_of_the_write_through_lines(ttmi, dt, forced, v
                     assert bool((whole[part.numel():] == 7.0).all())
     finally:
         ok(ttmi.ttmi_set_kernel_switch(b"TTMI_LARGE_TILE", -1))
+
+
+@pytest.mark.parametrize("beside", [-1, 0, 1])
+@pytest.mark.parametrize("N,K", [(768, 128), (520, 256), (64, 128)])
+@pytest.mark.parametrize("absmax", [False, True])
+def test_int8_products_on_both_sides_of_the_write_through_line(ttmi, N, K, beside, absmax):
+    """From 2 MiB of fp32 output on the dequantising stores go through L2: row counts around that line, guard rows, the bits of the product
+    and its dequantisation one after the other; with the maxima that the next quantisation takes."""
+    import ctypes
+    M = -(-(2 << 20) // (4 * N)) + beside
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a, b = (torch.randint(-127, 128, s, generator=g, device="cuda", dtype=torch.int8) for s in ((M, K), (N, K)))
+    sx, sw, bias = torch.tensor([0.0123, 0.0], device="cuda"), (torch.rand(N, generator=g, device="cuda") + 0.5) * 1e-3, torch.randn(N, generator=g, device="cuda")
+    acc, two_step = torch.empty((M, N), dtype=torch.int32, device="cuda"), torch.empty((M, N), device="cuda")
+    ok(ttmi.ttmi_gemm_i8(ptr(a), ptr(b), ptr(acc), M, N, K, K, K, N, stream()))
+    ok(ttmi.ttmi_dequant_bias(ptr(acc), ptr(sx), ptr(sw), ptr(bias), ptr(two_step), M, N, stream()))
+    whole, fused = _guarded(M, N, torch.float32)
+    if absmax:
+        slots, written = torch.full((capi.ABSMAX_SLOTS, ), float("nan"), device="cuda"), ctypes.c_int(-1)
+        ok(ttmi.ttmi_gemm_i8_dequant_absmax(ptr(a), ptr(b), ptr(fused), ptr(sx), ptr(sw), ptr(bias), -1, M, N, K, K, K, N, ptr(slots), ctypes.byref(written), stream()))
+        assert written.value == 0 or float(slots.max()) == float(two_step.abs().max())
+    else:
+        ok(ttmi.ttmi_gemm_i8_dequant(ptr(a), ptr(b), ptr(fused), ptr(sx), ptr(sw), ptr(bias), -1, M, N, K, K, K, N, stream()))
+    assert torch.equal(fused, two_step) and bool((whole[M:] == 7.0).all())
+
+
+@pytest.mark.parametrize("mib", [2, 12, 90])
+@pytest.mark.parametrize("S", [64, 75])
+def test_int8_head_split_on_both_sides_of_the_write_through_lines(ttmi, S, mib):
+    """The int8 head split writes through from 12 to 90 MiB of output: sequence counts around those lines and around 2 MiB, where other products begin."""
+    h, d = 2, 64
+    H = h * d
+    below = (mib << 20) // (3 * H * 4 * S)
+    for B in (below, below + 1):
+        M = B * S
+        g = torch.Generator(device="cuda").manual_seed(M)
+        a, b = (torch.randint(-127, 128, s, generator=g, device="cuda", dtype=torch.int8) for s in ((M, H), (3 * H, H)))
+        sx, sw, bias = torch.tensor([0.0123, 0.0], device="cuda"), (torch.rand(3 * H, generator=g, device="cuda") + 0.5) * 1e-3, torch.randn(3 * H, generator=g, device="cuda")
+        flat, two = torch.empty((M, 3 * H), device="cuda"), [torch.empty((B, h, S, d), device="cuda") for _ in range(3)]
+        ok(ttmi.ttmi_gemm_i8_dequant(ptr(a), ptr(b), ptr(flat), ptr(sx), ptr(sw), None, -1, M, 3 * H, H, H, H, 3 * H, stream()))
+        ok(ttmi.ttmi_split_add_bias_transpose_for_score(ptr(flat), ptr(bias), *[ptr(t) for t in two], B, S, h, d, TTMI_DTYPES["f32"], stream()))
+        held = [_guarded_heads(B, h, S, d, torch.float32) for _ in range(3)]
+        ok(ttmi.ttmi_gemm_i8_dequant_qkv_split(ptr(a), ptr(b), ptr(sx), ptr(sw), ptr(bias), *[ptr(t) for _, t in held], M, 3 * H, H, H, H, S, h, d, stream()))
+        for (whole, one), want in zip(held, two):
+            assert torch.equal(one, want) and bool((whole[one.numel():] == 7.0).all())

@@ -195,15 +195,19 @@ __device__ __forceinline__ void store_rows32(const GemmArgs& g, const Epi& epi, 
 enum class Stores { kAsk, kStay, kThrough };
 template <typename Epi>
 constexpr Stores default_stores(int tile_rows) { return tile_rows > 32 && !Dequantises<Epi>::value ? Stores::kAsk : Stores::kStay; }
-// The stores of a launch of whole output tiles: written through where they are many.
+// The stores of a launch of whole output tiles: written through where they are many.  The head split of int8, whose
+// tiles leave in pieces of a head's 256 bytes, only from 12 MiB on.  us a forward of int8, its stores staying / through, the other products' as
+// they are: base 4 x 128 tokens (4.5 MiB) 770 / 779, 5 x 128 (5.6) 785 / 790, 8 x 128 (9) 900 / 907, 10 x 128 (11.3)
+// 933 / 936, 12 x 128 (13.5) 1005 / 1000, 20 x 128 (22.5) 1223 / 1219; large 3 x 128 (4.5) 1725 / 1738, 6 x 128 (9) 2064 / 2067, 8 x 128 (12) 2163 /
+// 2152; 512 wide 6 x 128 (4.5) 1925 / 1957, 8 x 128 (6) 1986 / 2000, 12 x 128 (9) 2266 / 2269, 16 x 128 (12) 2366 / 2359.  Its other products from
+// 2 MiB on, as everywhere: base 4 x 128 (up to 6 MiB) 770 / 762, 6 x 128 848 / 831, 16 x 128 1126 / 1092, 20 x 100 1136 / 1102; large 4 x 128
+// 1838 / 1808; only 512 wide 4 x 128 (4 MiB) 1815 / 1819.
 template <typename Epi>
 inline bool stores_through(const GemmArgs& g) {
   const int64_t bytes = (int64_t)g.m * g.n * g.slices * (int64_t)sizeof(typename RingDest<Epi>::Elem);
-  // a short int8 product is stores for the most part: 4 x 128 tokens 787 / 803 us with its 4.7 and 6.3 MB written through, 20 x 128 (7.9 MB
-  // and more) 1224 / 1179
   // The products of many rounds of tiles stay: 24576 x 1024 x 4096 in bf16, 101 MB of fp32, 196 us / 206 through
-  constexpr int64_t kMostThrough = 90ll << 20;
-  return bytes <= kMostThrough && (Dequantises<Epi>::value ? bytes >= (7ll << 20) : writes_through(bytes));
+  constexpr int64_t kMostThrough = 90ll << 20, kInt8HeadsThrough = 12ll << 20;
+  return bytes <= kMostThrough && (std::is_same<Epi, EpiDequantQkvSplit>::value ? bytes >= kInt8HeadsThrough : writes_through(bytes));
 }
 
 template <int BM, int BN, int NS>
