@@ -2012,3 +2012,17 @@ def test_int8_head_split_on_both_sides_of_the_write_through_lines(ttmi, S, mib):
         ok(ttmi.ttmi_gemm_i8_dequant_qkv_split(ptr(a), ptr(b), ptr(sx), ptr(sw), ptr(bias), *[ptr(t) for _, t in held], M, 3 * H, H, H, H, S, h, d, stream()))
         for (whole, one), want in zip(held, two):
             assert torch.equal(one, want) and bool((whole[one.numel():] == 7.0).all())
+
+
+@pytest.mark.parametrize("rows", [12287, 12288, 12289])
+@pytest.mark.parametrize("k", [171, 192])
+def test_quantisation_on_both_sides_of_the_rows_that_write_through(ttmi, oracle, rows, k):
+    """Passes of 2 MiB and more write through L2 up to 12288 rows; ragged and whole workgroups, guard bytes behind."""
+    n = rows * k
+    x = torch.randn(n, generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    whole_q = torch.full((n + 32, ), 99, dtype=torch.int8, device="cuda")
+    scale = torch.full((capi.QUANT_SCALE_FLOATS, ), float("nan"), device="cuda")
+    ok(ttmi.ttmi_quantize_rows_i8(ptr(x), ptr(whole_q), ptr(scale), rows, k, stream()))
+    want, want_scale = oracle.quantize_tensor_i8(host(x).reshape(rows, k))
+    assert np.array_equal(host(whole_q[:n]), want.reshape(-1)) and host(scale)[0] == np.float32(want_scale)
+    assert bool((whole_q[n:] == 99).all())

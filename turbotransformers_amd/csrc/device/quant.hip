@@ -99,15 +99,21 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
   for (int64_t i = n4 * 4 + blockIdx.x * (int64_t)256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
     q[i] = (int8_t)quantize_one(x[i], scale, inv_scale);
 }
-static int launch_quantize(const float* x, int8_t* q, float* scale_dev, const float* partial, int partials, int64_t n, hipStream_t s) {
+// rows: tokens.  What is written through is the passes of up to 12288 tokens: us a forward, all passes staying / those of the intermediate
+// values through / all through: base 20 x 128 tokens (8 MB of them) 1167 / 1157 / 1157, 8 x 300 1578 / 1568 / 1568, 24 x 200 2641 / 2634 / 2634, 32 x 300 (29 MB)
+// 4624 / 4605 / 4606, 16 x 512 level, large 16 x 256 4678 / 4651 / 4651, 16 x 512 (34 MB) 11233 / 11211 / 11207; 32 x 512, inputs of 13 MB and
+// intermediate values of 50, 7732 all staying, 7767 the inputs through, 7790 all; 48 x 512 (19 and 75 MB) 11963, 12050, 12036; large 32 x 512
+// 21077, 21115, 21125.
+constexpr int64_t kMostRowsThrough = 12288;
+static int launch_quantize(const float* x, int8_t* q, float* scale_dev, const float* partial, int partials, int64_t rows, int64_t n, hipStream_t s) {
   TTMI_REQUIRE(n < (1ll << 42), "too many elements");
-  // (2560 x 3072 and 2400 x 3072 values: 20 x 128 tokens 1195 -> 1186 us a forward, 8 x 300 1611 -> 1601)
-  if (writes_through(n))
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(quantize_kernel<4, true>), dim3((unsigned)ceil_div(n, 4096)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
-  else if (ceil_div(n, 1024) <= 512)
-    hipLaunchKernelGGL(quantize_kernel<1>, dim3((unsigned)ceil_div(n, 1024)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
-  else
-    hipLaunchKernelGGL(quantize_kernel<2>, dim3((unsigned)ceil_div(n, 2048)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
+  auto launch = [&](auto kern, int vecs) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(n, vecs * 1024)), dim3(256), 0, s, x, q, scale_dev, partial, partials, n);
+  };
+  if (writes_through(n) && rows <= kMostRowsThrough) launch(quantize_kernel<4, true>, 4);
+  else if (writes_through(n)) launch(quantize_kernel<4>, 4);
+  else if (ceil_div(n, 1024) <= 512) launch(quantize_kernel<1>, 1);
+  else launch(quantize_kernel<2>, 2);
   return launch_status("quantize_kernel");
 }
 
@@ -175,7 +181,7 @@ int ttmi_quantize_rows_i8(const float* x, int8_t* q, float* scale_dev, int64_t m
   const int partials = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, 256 * 16), kMaxPartials));
   static_assert(kMaxPartials + 2 == TTMI_QUANT_SCALE_FLOATS, "scale_dev holds the scale, the maximum and the partial maxima");
   hipLaunchKernelGGL(absmax_kernel, dim3((unsigned)partials), dim3(256), 0, s, x, n, scale_dev + 2);
-  return launch_quantize(x, q, scale_dev, scale_dev + 2, partials, n, s);
+  return launch_quantize(x, q, scale_dev, scale_dev + 2, partials, m, n, s);
 }
 
 int ttmi_quantize_rows_i8_from_absmax(const float* x, int8_t* q, float* scale_dev, const float* absmax_slots, int64_t m,
@@ -183,7 +189,7 @@ int ttmi_quantize_rows_i8_from_absmax(const float* x, int8_t* q, float* scale_de
   TTMI_REQUIRE(x && q && scale_dev && absmax_slots, "null tensor");
   const int64_t n = m * k;
   if (n <= 0) return 0;
-  return launch_quantize(x, q, scale_dev, absmax_slots, TTMI_ABSMAX_SLOTS, n, (hipStream_t)stream);
+  return launch_quantize(x, q, scale_dev, absmax_slots, TTMI_ABSMAX_SLOTS, m, n, (hipStream_t)stream);
 }
 
 int ttmi_quantize_weight_rows_i8(const float* w, int8_t* q, float* scales, int64_t n, int64_t k, void* stream) {
