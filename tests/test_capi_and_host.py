@@ -417,3 +417,20 @@ def test_kernel_forms_that_write_through_contain_such_stores(tmp_path):
             assert through > 0, name
         else:
             assert through == 0, name
+
+
+@pytest.mark.parametrize("layers,width,ffn,element,lens,reads", [
+    # base: the tensors of some 1100 tokens push its weights out, those of one or a few sequences do not
+    (12, 768, 3072, 2, 512, False), (12, 768, 3072, 2, 1000, False), (12, 768, 3072, 2, 1152, True), (12, 768, 3072, 2, 1536, True), (12, 768, 3072, 2, 2000, True),
+    (13, 768, 3072, 2, 600, False), (13, 768, 3072, 2, 500, False), (13, 768, 3072, 2, 768, True), (14, 768, 3072, 2, 300, False), (17, 768, 1536, 2, 2048, True),
+    # weights of 176 to 201 MB whose tensors add up to less than 200 MiB: narrower and wider layers, fp32
+    (29, 512, 2048, 2, 1536, False), (32, 512, 2048, 2, 128, False), (7, 1024, 4096, 2, 768, False), (5, 1280, 5120, 2, 128, False), (5, 1280, 5120, 2, 256, False),
+    (4, 1280, 5120, 2, 1024, False), (6, 768, 3072, 4, 512, False), (6, 768, 3072, 4, 600, False), (14, 512, 2048, 4, 768, False),
+    # beyond: always, but for up to 32 rows
+    (24, 1024, 4096, 2, 33, True), (24, 1024, 4096, 2, 32, False), (12, 768, 3072, 4, 128, True), (5, 1280, 5120, 2, 768, True), (6, 768, 3072, 4, 1024, True)])
+def test_weights_are_read_ahead_where_they_leave_the_cache(layers, width, ffn, element, lens, reads):
+    """The attention of a layer reads the following weights ahead where that was measured to gain: each line's time with and without
+    stands at the rule."""
+    from turbotransformers_amd import cxx
+    weights = layers * (4 * width * width + 2 * width * ffn) * element
+    assert cxx.weights_leave_cache(weights, lens, width, ffn, element) is reads

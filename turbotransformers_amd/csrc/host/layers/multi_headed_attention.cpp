@@ -418,11 +418,12 @@ void BertAttention::operator()(const Tensor& input_tensor, const Tensor& attenti
           lender != nullptr ? *lender : *this);
 }
 
-bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const Tensor& hidden) {
-  constexpr int64_t kStays = 195 * 1000 * 1000;
-  const int64_t width = hidden.shape(-1), rows = width > 0 ? hidden.numel() / width : 0;
-  const int64_t tensors = rows * (12 * width + ffn) * (int64_t)hidden.element_size();
-  return rows > 32 && bytes + tensors > kStays;
+bool WeightsLeaveCache(int64_t bytes, int64_t rows, int64_t width, int64_t ffn, int64_t element_size) {
+  constexpr int64_t kMB = 1000 * 1000, kLeaves = 200ll << 20, kMayLeave = 195 * kMB;
+  if (rows <= 32) return false;
+  const int64_t tensors = rows * (12 * width + ffn) * element_size, layer = (4 * width * width + 2 * width * ffn) * element_size;
+  if (bytes + tensors > kLeaves) return true;
+  return bytes + tensors > kMayLeave && element_size == 2 && tensors > 18 * kMB && layer > 8 * kMB && layer < 22 * kMB;
 }
 
 void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,

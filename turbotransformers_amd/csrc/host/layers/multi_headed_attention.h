@@ -186,15 +186,19 @@ struct EncoderLayer {
 // for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
 // with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call
 // (Q, K, V, context, four of hidden states, two fp32 slices of a product and the intermediate one: rows x (12 x hidden + ffn)) take their
-// part of the cache.  The line is 195 MB of both: us per forward without / with, fp16 base (170 MB), 1 x 387 tokens 475 / 542, 4 x 128 463 / 489
-// (182 MB in all), 6 x 128 536 / 532 (189), 8 x 128 587 / 581 (195), 9 x 128 657 / 613 (198), 11 x 128 770 / 681, 3 x 512 861 / 768, and from 208
-// MB on, where the line was, 20 x 100 888 / 853, 40 x 128 1573 / 1518.  It holds for other widths: 5 layers of 1280 / ffn 5120 1 x 128 221 /
-// 224 (192), 4 x 128 328 / 310 (207), 20 x 100 681 / 655 (265), though 12 x 64 373 / 382 (217); 16 of 768 / 1536 4 x 128 591 / 622 (154), 20 x 100 918 / 916 (185); 9 of 768 / 6144
-// 1 x 128 373 / 365 (205), 12 x 64 558 / 522 (223); 32 of 512 / 2048 1 x 128 926 / 946 (194), 4 x 128 1071 / 1051 (200), 8 x 256 1569 / 1525 (224).
+// part of the cache.  From 200 MiB of both on they are read ahead: us per forward without / with, fp16 base (170 MB of weights), 20 x 100 tokens 848 /
+// 791, 40 x 128 1573 / 1518; large bf16 (604 MB), 1 x 128 928 / 880, 8 x 128 1601 / 1517.
+// Between 195 MB and there weights may leave the cache or not.  Of 640, 768 and 896 columns in 16 bits they do: fp16 base 9 x 128 (198 MB)
+// 663 / 629, 11 x 128 731 / 692, 3 x 512 843 / 791, bf16 12 x 128 835 / 734, 13 layers 6 x 128 (203 MB) 600 / 576, 17 of 768 / ffn 1536 16 x 128 1030 /
+// 933.  Of 512, 1024 and 1280 they do not, nor in fp32, and reading them costs what a layer holds (6, 25, 39 and from 13 MB): 29 layers of 512 12 x
+// 128 1219 / 1229, 7 of 1024 in fp16 6 x 128 426 / 444, 4 of 1280 8 x 128 328 / 342, 6 of 768 in fp32 4 x 128 404 / 428 and 2 x 300 468 / 503,
+// 14 of 512 in fp32 8 x 128 806 / 859.  Nor do they where the tensors are few: 13 layers of 768 in fp16 2 x 300 (15 MB of
+// them) 564 / 631, 1 x 500 (12 MB) 563 / 609, 14 1 x 300 526 / 556, 5 of 1280 1 x 128 207 / 222.  Below 195 MB in all: base 1 x
+// 387 (182 MB) 470 / 535, 4 x 128 457 / 481, 8 x 128 (195 MB) between 587 / 584 and 612 / 587 from process to process.
 // Nor for up to 32 rows: those products request all of a workgroup's share of the weights at once (fp32 the fp32 weights as they are), so
 // reading ahead is no sooner, and the attention launch waits for it.  us per forward of large bf16 (600 MB), without / with: 1 x 8 tokens 666 /
 // 711, 1 x 10 677 / 713, 1 x 20 728 / 748, 1 x 32 715 / 726, 2 x 16 719 / 750, 3 x 10 751 / 854, 8 x 4 809 / 811, 32 x 1 822 / 821; fp16 the same.
-bool WeightsLeaveCache(int64_t bytes, int64_t ffn, const core::Tensor& hidden);
+bool WeightsLeaveCache(int64_t bytes, int64_t rows, int64_t width, int64_t ffn, int64_t element_size);
 template <typename Attention>
 std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<EncoderLayer<Attention>>& layers, const core::Tensor& hidden) {
   std::vector<std::vector<WeightRange>> ahead(layers.size());
@@ -207,7 +211,8 @@ std::vector<std::vector<WeightRange>> WeightsAhead(const std::vector<EncoderLaye
     ffn = std::max(ffn, layers[i].intermediate->out_features());
     if (i > 0) ahead[i - 1].push_back(qkv);
   }
-  if (!WeightsLeaveCache(bytes, ffn, hidden)) ahead.assign(layers.size(), {});
+  const int64_t width = hidden.shape(-1), rows = width > 0 ? hidden.numel() / width : 0;
+  if (!WeightsLeaveCache(bytes, rows, width, ffn, (int64_t)hidden.element_size())) ahead.assign(layers.size(), {});
   return ahead;
 }
 

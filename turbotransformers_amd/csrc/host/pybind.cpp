@@ -460,6 +460,8 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
   m.def("allocator_schema", [] { return core::allocator::Allocator::GetInstance().schema(); });
   m.def("model_aware_chunks", [] { return core::allocator::Allocator::GetInstance().model_aware_chunks(); },
         "(number of chunks, total bytes) held by the model-aware plan");
+  m.def("weights_leave_cache", &layers::WeightsLeaveCache, py::arg("bytes"), py::arg("rows"), py::arg("width"), py::arg("ffn"), py::arg("element_size"),
+        "Whether the layers of an encoder read their weights ahead, for tests.");
   // The planner as plain functions, for tests: records are (name, start_op, end_op, size).
   using Rec = std::tuple<std::string, int64_t, int64_t, int64_t>;
   auto to_records = [](const std::vector<Rec>& in) {
