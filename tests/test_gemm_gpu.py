@@ -1845,60 +1845,90 @@ def test_products_on_both_sides_of_the_line_where_stores_stay_again(ttmi, dt, be
     assert bool((whole[M:] == 7.0).all())
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("dt", ALL_DTYPES)
-@pytest.mark.parametrize("shadow", [False, True])
-@pytest.mark.parametrize("beside", [-1, 0, 1])
-def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, beside):
-    """AddBiasLayerNorm by itself and behind a product, row counts around 2 MiB of output."""
-    n, K = 776, 128
-    m = -(-(2 << 20) // (n * torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size())) + beside
+def _layer_norm_operands(dt, m, n, shadow):
+    """-> residual (fp32 if `shadow`) and the three row vectors as the kernel sees them, want(base in 64 bits), the operands on the device."""
     rng = np.random.default_rng(m)
-    x, res, bias, gamma, beta = (rng.standard_normal(s).astype(np.float32) for s in ((m, n), (m, n), (n,), (n,), (n,)))
-    A, W = rng.standard_normal((m, K), np.float32), (rng.standard_normal((n, K)) / np.sqrt(K)).astype(np.float32)
+    res, bias, gamma, beta = (rng.standard_normal(s).astype(np.float32) for s in ((m, n), (n,), (n,), (n,)))
     residual = res if shadow else rounded(res, dt)
 
     def want(base):
         s = base + residual + rounded(bias, dt).astype(np.float64)
         return rounded(beta, dt) + rounded(gamma, dt) * (s - s.mean(1, keepdims=True)) / np.sqrt(s.var(1, keepdims=True) + 1e-12)
 
-    d = [ptr(dev(v, dt)) for v in (bias, gamma, beta)]
-    r16, r32 = ptr(dev(res, dt)), ptr(dev(res)) if shadow else None
-    tol = {"f32": 1e-4, "f16": 2e-2, "bf16": 1.2e-1}[dt]  # values of size up to 16, rounded once; in front of it the product may be
+    return rng, want, dev(res, dt), dev(res), [dev(v, dt) for v in (bias, gamma, beta)]
+
+
+LAYER_NORM_TOL = {"f32": 1e-4, "f16": 2e-2, "bf16": 1.2e-1}  # values of size up to 16, rounded once; in front of it the product may be
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("beside", [-1, 0, 1])
+@pytest.mark.parametrize("n", [776, 768, 1024])
+def test_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, beside, n):
+    """AddBiasLayerNorm by itself, row counts around 2 MiB of output, where it also leaves the workgroups of one wavefront."""
+    m = -(-(2 << 20) // (n * torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size())) + beside
+    rng, want, res, res32, row = _layer_norm_operands(dt, m, n, shadow)
+    x = rng.standard_normal((m, n)).astype(np.float32)
     whole, out = _guarded(m, n, TORCH_DTYPES[dt])
     out.copy_(dev(x, dt))
     whole32, out32 = _guarded(m, n, torch.float32)
     if shadow:
-        ok(ttmi.ttmi_add_bias_layer_norm_residual32(ptr(out), r32, *d, ptr(out32), m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+        ok(ttmi.ttmi_add_bias_layer_norm_residual32(ptr(out), ptr(res32), *[ptr(v) for v in row], ptr(out32), m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+        assert torch.equal(out, out32.to(out.dtype))
     else:
-        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), r16, *d, m, n, 1e-12, TTMI_DTYPES[dt], stream()))
-    assert max_abs(host(out), want(rounded(x, dt).astype(np.float64))) <= tol
-    behind, out2 = _guarded(m, n, TORCH_DTYPES[dt])
-    ok(ttmi.ttmi_gemm_bias_layer_norm(ptr(dev(A, dt)), ptr(dev(W, dt)), ptr(out2), None if shadow else r16, r32, *d, ptr(out32) if shadow else None, m, n, K, 1e-12,
-                                      TTMI_DTYPES[dt], stream()))
-    assert max_abs(host(out2), want(rounded(A, dt).astype(np.float64) @ rounded(W, dt).T.astype(np.float64))) <= tol
-    for w in (whole, whole32, behind):
+        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), ptr(res), *[ptr(v) for v in row], m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+    assert max_abs(host(out), want(rounded(x, dt).astype(np.float64))) <= LAYER_NORM_TOL[dt]
+    for w in (whole, whole32):
         assert bool((w[m:] == 7.0).all())
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", ALL_DTYPES)
-@pytest.mark.parametrize("n,rows_a_group", [(768, None), (64, 16), (1024, 4)])
-def test_layer_norm_of_few_rows_takes_one_wavefront_a_workgroup(ttmi, dt, n, rows_a_group):
-    """Row counts on both sides of 255 workgroups of four wavefronts, and ones that leave a wavefront partly idle."""
-    per = rows_a_group or (4 if dt == "f32" else 8)
-    rng = np.random.default_rng(n)
-    for m in (1, 3, 2 * per + 1, 255 * per - 1, 255 * per, 255 * per + 1):
-        x, res = rng.standard_normal((m, n), np.float32), rng.standard_normal((m, n), np.float32)
-        bias, gamma, beta = (rng.standard_normal(n).astype(np.float32) for _ in range(3))
+@pytest.mark.parametrize("shadow", [False, True])
+@pytest.mark.parametrize("beside", [-1, 0, 1])
+@pytest.mark.parametrize("n", [776, 260])
+def test_summing_layer_norm_on_both_sides_of_the_write_through_line(ttmi, dt, shadow, beside, n):
+    """The LayerNorm that sums the slices of a product with K of twice its columns and more: row counts around 2 MiB of what it stores, the
+    unrounded rows among it, of widths that leave its workgroups partly idle."""
+    K = 1664
+    stored = torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size() + (4 if shadow else 0)
+    m = -(-(2 << 20) // (n * stored)) + beside
+    rng, want, res, res32, row = _layer_norm_operands(dt, m, n, shadow)
+    A, W = rng.standard_normal((m, K), np.float32), (rng.standard_normal((n, K)) / np.sqrt(K)).astype(np.float32)
+    exact = want(rounded(A, dt).astype(np.float64) @ rounded(W, dt).T.astype(np.float64))
+    for w, kind in [(dev(W, dt), TTMI_DTYPES[dt])] + ([(_packed(ttmi, dev(W)), capi.F32_PACKED)] if dt == "f32" else []):
+        whole, out = _guarded(m, n, TORCH_DTYPES[dt])
+        whole32, out32 = _guarded(m, n, torch.float32)
+        ok(ttmi.ttmi_gemm_bias_layer_norm(ptr(dev(A, dt)), ptr(w), ptr(out), None if shadow else ptr(res), ptr(res32) if shadow else None, *[ptr(v) for v in row],
+                                          ptr(out32) if shadow else None, m, n, K, 1e-12, kind, stream()))
+        assert max_abs(host(out), exact) <= LAYER_NORM_TOL[dt]
+        if shadow:
+            assert torch.equal(out, out32.to(out.dtype))
+        for guarded in (whole, whole32):
+            assert bool((guarded[m:] == 7.0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("n", [64, 128, 256, 512, 1024])
+def test_layer_norm_of_few_rows_takes_one_wavefront_a_workgroup(ttmi, dt, n):
+    """Row counts on both sides of 255 workgroups of four wavefronts (of widths that store less than 2 MiB there), and ones that leave a wavefront
+    partly idle."""
+    element = torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size()
+    vectors = n * element // 16
+    per = 16 if vectors <= 16 else 8 if vectors <= 32 else 4  # rows of four wavefronts
+    if n * element > 2048:
+        per = None  # its 255 workgroups are past 2 MiB: the counts around that line are another test's
+    for m in (1, 3, 11) + ((2 * per + 1, 255 * per - 1, 255 * per, 255 * per + 1) if per else (300, )):
+        assert per is None or 255 * per * n * element < 2 << 20
+        rng, want, res, _, row = _layer_norm_operands(dt, m, n, False)
+        x = rng.standard_normal((m, n), np.float32)
         whole, out = _guarded(m, n, TORCH_DTYPES[dt])
         out.copy_(dev(x, dt))
-        held = [dev(v, dt) for v in (res, bias, gamma, beta)]
-        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), *[ptr(v) for v in held], m, n, 1e-12, TTMI_DTYPES[dt], stream()))
-        s = rounded(x, dt).astype(np.float64) + rounded(res, dt) + rounded(bias, dt)
-        want = rounded(beta, dt) + rounded(gamma, dt) * (s - s.mean(1, keepdims=True)) / np.sqrt(s.var(1, keepdims=True) + 1e-12)
-        # values of size up to 16, rounded once
-        assert max_abs(host(out), want) <= {"f32": 1e-4, "f16": 2e-2, "bf16": 1.2e-1}[dt]
+        ok(ttmi.ttmi_add_bias_layer_norm(ptr(out), ptr(res), *[ptr(v) for v in row], m, n, 1e-12, TTMI_DTYPES[dt], stream()))
+        assert max_abs(host(out), want(rounded(x, dt).astype(np.float64))) <= LAYER_NORM_TOL[dt]
         assert bool((whole[m:] == 7.0).all())
 
 

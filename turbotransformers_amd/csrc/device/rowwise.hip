@@ -11,7 +11,6 @@
 namespace ttmi {
 
 constexpr int kBlock = 256;
-constexpr int kCus = 256;  // compute units
 
 // --------------------------------------------------------------------------- LayerNorm --
 // x = out (+ input + bias); mean = sum(x)/n; var = sum(x*x)/n - mean^2;
@@ -183,11 +182,15 @@ static int launch_ln_rows(T* out, const T* input, const T* bias, const T* gamma,
   auto launch = [&](auto kern, int block = kBlock) {
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(block), 0, s, out, input, bias, gamma, beta, m, n, eps, res32, out32, absmax);
   };
-  const bool through = sizeof(T) * VEC == 16 && writes_through(m * n * (int64_t)sizeof(T));
+  static_assert(sizeof(T) * VEC == 16, "one store a vector");
+  // Without an upper line: fp16 base 128 x 512 tokens (100 MB a launch), the stores of LayerNorms staying / through 14244 / 14209 us a forward, fp32
+  // base 64 x 512 (100 MB) and 128 x 512 (201 MB) level.  out32 stays, and its bytes do not count: large bf16 with it through as well 20 x 100
+  // tokens 2123 / 2149, 20 x 128 2587 / 2620, 16 x 256 3631 / 3696, 64 x 512 24065 / 24922; with `out` staying too, 4 x 128 to 64 x 512, 1.000 to 1.004 times the time.
+  const bool through = writes_through(m * n * (int64_t)sizeof(T));
   // Fewer workgroups than CUs: one wavefront each, so that more CUs take part; the lanes of a row are the same ones.  us a forward, four / one:
   // decoder prefix 8 x 33 tokens in fp32 (66 / 264 workgroups) 659 / 656, fp16 1 x 387 (49 / 194) 473.3 / 471.5.  (A maximum is one slot
   // per workgroup of four.)
-  if (absmax == nullptr && !through && grid < kCus) {
+  if (absmax == nullptr && !through && grid < compute_units()) {
     grid = ceil_div(m, kWave / G);
     launch(layer_norm_rows<T, VEC, G, ITERS, ADD, RES32, false, kWave>, kWave);
     return launch_status("layer_norm_rows");
