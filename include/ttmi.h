@@ -446,6 +446,8 @@ TTMI_API int ttmi_layer_norm_gemm_fused(const void* x, const void* gamma, const 
  * `args` supplies seq / heads / head_dim / v_seq_pitch (and batch); pointers in it are ignored. */
 TTMI_API int ttmi_gemm_describe(int64_t m, int64_t n, int64_t k, int epilogue, const ttmi_epilogue_args* args, int dtype,
                                 char* out, size_t capacity);
+/* The same for ttmi_gemm_bias_act, the layers' product with bias and activation, which does not always run what ttmi_gemm_fused does. */
+TTMI_API int ttmi_gemm_bias_act_describe(int64_t m, int64_t n, int64_t k, int act, int dtype, char* out, size_t capacity);
 
 
 /* Measurement aid, never on a product path: a loop of nothing but matrix instructions on register operands, one

@@ -434,3 +434,35 @@ def test_weights_are_read_ahead_where_they_leave_the_cache(layers, width, ffn, e
     from turbotransformers_amd import cxx
     weights = layers * (4 * width * width + 2 * width * ffn) * element
     assert cxx.weights_leave_cache(weights, lens, width, ffn, element) is reads
+
+
+def test_the_layers_product_with_activation_has_no_named_form():
+    """ttmi_gemm_bias_act takes the ring tiles where ttmi_gemm_fused keeps the form that ttmi_gemm_describe names for GELU over 65 to 128
+    rows, and its own description says so; elsewhere the two run the same."""
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+    args = capi.EpilogueArgs()
+
+    def variants(m, n, k, act, dt):
+        args.act = act
+        capi.check(lib.ttmi_gemm_describe(m, n, k, capi.EPI_BIAS_ACT, ctypes.byref(args), dt, buf, 64))
+        fused = buf.value.decode()
+        capi.check(lib.ttmi_gemm_bias_act_describe(m, n, k, act, dt, buf, 64))
+        return fused, buf.value.decode()
+
+    for m in (65, 97, 128):
+        for dt in (capi.F16, capi.BF16):
+            assert variants(m, 3072, 768, capi.ACT_GELU, dt)[0] == "wave1w_32x32"
+            assert variants(m, 3072, 768, capi.ACT_GELU, dt)[1].startswith("dma")
+        assert "_splitk" in variants(m, 3072, 768, capi.ACT_GELU, capi.F32)[0]
+        one, other = variants(m, 3072, 768, capi.ACT_GELU, capi.F32)
+        assert other.startswith("dma") and "_splitk" not in other
+    for m in (1, 10, 64, 129, 2000, 32768):
+        for dt in (capi.F16, capi.BF16, capi.F32, capi.F32_PACKED):
+            for act in (capi.ACT_GELU, capi.ACT_RELU):
+                one, other = variants(m, 3072, 768, act, dt)
+                assert one == other, (m, dt, act)
+    one, other = variants(128, 3072, 768, capi.ACT_RELU, capi.F16)
+    assert one == other
+    assert lib.ttmi_gemm_bias_act_describe(128, 3072, 768, capi.ACT_GELU, capi.F16, buf, 4) != 0  # too small for the answer
+    assert lib.ttmi_gemm_bias_act_describe(128, 3072, 768, 99, capi.F16, buf, 64) != 0

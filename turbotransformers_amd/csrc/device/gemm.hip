@@ -117,6 +117,23 @@ static int gemm_bias_layer_norm_impl(const void* a, const void* w, void* out, co
 
 using namespace ttmi;
 
+// The name of what `launch`, a call that launches one product, would run.
+template <typename Launch>
+static int describe(char* out, size_t capacity, const Launch& launch) {
+  TTMI_REQUIRE(out != nullptr && capacity > 0, "no room for the answer");
+  std::string name;
+  struct Install {
+    explicit Install(std::string* p) { tl_describe = p; }
+    ~Install() { tl_describe = nullptr; }
+  } install(&name);
+  // operands that pass every alignment test; nothing dereferences them in a dry run
+  const int rc = launch(reinterpret_cast<void*>((uintptr_t)1 << 20));
+  if (rc != 0) return rc;
+  TTMI_REQUIRE(name.size() < capacity, "the answer does not fit");
+  std::memcpy(out, name.c_str(), name.size() + 1);
+  return 0;
+}
+
 extern "C" {
 
 int ttmi_gemm(const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldb,
@@ -219,26 +236,20 @@ int ttmi_split_weights(void* packed, int64_t n, int64_t k, void* stream) {
 
 int ttmi_gemm_describe(int64_t m, int64_t n, int64_t k, int epilogue, const ttmi_epilogue_args* args, int dtype, char* out,
                        size_t capacity) {
-  TTMI_REQUIRE(out != nullptr && capacity > 0, "no room for the answer");
-  // operands that pass every alignment test; nothing dereferences them in a dry run
-  void* fake = reinterpret_cast<void*>((uintptr_t)1 << 20);
-  ttmi_epilogue_args filled{};
-  if (args != nullptr) filled = *args;
-  filled.bias = fake;
-  filled.residual = fake;
-  filled.q = filled.k = filled.v = fake;
-  if (epilogue == TTMI_EPI_QKV_SPLIT_PAD) filled.token_rows = static_cast<const int32_t*>(fake);
-  std::string name;
-  struct Install {
-    explicit Install(std::string* p) { tl_describe = p; }
-    ~Install() { tl_describe = nullptr; }
-  } install(&name);
-  const int rc = epilogue == TTMI_EPI_NONE ? ttmi_gemm(fake, fake, fake, m, n, k, k, k, n, 1, 1.f, 0.f, dtype, nullptr)
-                                           : ttmi_gemm_fused(fake, fake, fake, m, n, k, k, k, n, epilogue, &filled, dtype, nullptr);
-  if (rc != 0) return rc;
-  TTMI_REQUIRE(name.size() < capacity, "the answer does not fit");
-  std::memcpy(out, name.c_str(), name.size() + 1);
-  return 0;
+  return describe(out, capacity, [&](void* fake) {
+    ttmi_epilogue_args filled{};
+    if (args != nullptr) filled = *args;
+    filled.bias = fake;
+    filled.residual = fake;
+    filled.q = filled.k = filled.v = fake;
+    if (epilogue == TTMI_EPI_QKV_SPLIT_PAD) filled.token_rows = static_cast<const int32_t*>(fake);
+    return epilogue == TTMI_EPI_NONE ? ttmi_gemm(fake, fake, fake, m, n, k, k, k, n, 1, 1.f, 0.f, dtype, nullptr)
+                                     : ttmi_gemm_fused(fake, fake, fake, m, n, k, k, k, n, epilogue, &filled, dtype, nullptr);
+  });
+}
+
+int ttmi_gemm_bias_act_describe(int64_t m, int64_t n, int64_t k, int act, int dtype, char* out, size_t capacity) {
+  return describe(out, capacity, [&](void* fake) { return ttmi_gemm_bias_act(fake, fake, fake, fake, m, n, k, act, dtype, nullptr); });
 }
 
 int ttmi_gemm_bias_layer_norm(const void* a, const void* w, void* out, const void* residual, const float* residual_f32,
