@@ -385,7 +385,8 @@ static int fused_attention_impl(const void* q, const void* k, const void* v, con
   }
   const float sl2 = scale * 1.4426950408889634f, inv_scale = 1.0f / scale;
   hipStream_t s = (hipStream_t)stream;
-  // (a packed batch: taken as half of the padded one)
+  // A packed batch: taken as half of the padded one.  No upper line: us a forward, staying / through, fp16 base 128 x 512 tokens (100 MB) 14225 /
+  // 14209, large bf16 32 x 512 (34 MB) 12212 / 12180, 64 x 512 (67 MB) 24097 / 24065, fp32 base 64 x 512 (100 MB) and 128 x 512 (201 MB) level.
   const bool through = writes_through(batch * heads * seq * kD * (int64_t)dtype_size(dtype) / (cu_seqlens != nullptr ? 2 : 1));
   if (dtype == TTMI_F32) {
     // the per-workgroup maxima: dense fp32 batches whose workgroups fit the slots

@@ -83,12 +83,13 @@ __device__ __forceinline__ void store_vec_unaligned(T* p, const Vec<T, N>& x) {
 // wavefronts still computed.  A store that goes through takes longer (the stores of a 128 x 192 tile 2.0 -> 2.4 us, of a 64 x 96 one
 // 1.1 -> 1.8), so few bytes stay: us a forward of base, never / from 0.5, 1.5, 4.5 MB of a launch on: fp16 1 x 387 tokens 477 / 471, 479, 482;
 // 8 x 128 600 / 583, 585, 590; 8 x 256 829 / 783, 783, 791; fp32 1 x 128 555 / 547, 549, 560; 3 x 128 802 / 778, 780, 784; decoder prefix 8 x 33
-// fp32 667 / 670, 663, 665.  20 x 100 fp16 853 / 814 from 1.5 MB on, 16 x 512 2429 / 2320, 20 packed requests 1875 / 1793.  Products of
-// 90 MB and more stay (gemm_ring.h, gemm_w4.h).
-// Rows of a transposed V stay wherever they are not whole cache lines: 40 x 100 tokens 1384 / 1465 with them.
+// fp32 667 / 670, 663, 665.  20 x 100 fp16 853 / 814 from 1.5 MB on, 16 x 512 2429 / 2320, 20 packed requests 1875 / 1793.
+// Upper lines: kMostThrough of the ring tiles (gemm_ring.h) and of the large ones (gemm_w4.h, whose fp32 outputs stay whatever their size),
+// kMostRowsThrough of the quantising passes (quant.hip).  LayerNorms and attention have none.
+// Rows of a transposed V stay, which at most lengths are no whole cache lines: 40 x 100 tokens 1384 / 1465 with them.
 constexpr int64_t kWriteThroughBytes = 2ll << 20;
 inline bool writes_through(int64_t bytes) { return bytes >= kWriteThroughBytes; }
-// An 8- or 16-byte store, aligned to the element.  The compiler does not count it, which makes its waits longer than they need to
+// A store of 4, 8 or 16 bytes, aligned to the element.  The compiler does not count it, which makes its waits longer than they need to
 // be, never shorter.  (The no-op: it does not know either that the next instruction must not overwrite the stored registers.)
 template <typename V>
 __device__ __forceinline__ void store_through(void* p, const V& x) {
