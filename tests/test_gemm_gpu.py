@@ -2056,3 +2056,33 @@ def test_quantisation_on_both_sides_of_the_rows_that_write_through(ttmi, oracle,
     want, want_scale = oracle.quantize_tensor_i8(host(x).reshape(rows, k))
     assert np.array_equal(host(whole_q[:n]), want.reshape(-1)) and host(scale)[0] == np.float32(want_scale)
     assert bool((whole_q[n:] == 99).all())
+
+
+@pytest.mark.parametrize("dt", ALL_DTYPES)
+@pytest.mark.parametrize("v_transposed", [False, True])
+@pytest.mark.parametrize("S", [128, 100, 300])
+@pytest.mark.parametrize("packed", [False, True])
+def test_fused_attention_on_both_sides_of_the_write_through_line(ttmi, dt, v_transposed, S, packed):
+    """From 2 MiB of context on (of packed batches half of the padded size) it is written through L2: sequence counts on both sides, each
+    sequence's own softmax in 64 bits, guard rows behind."""
+    h, d = 2, 64
+    element = torch.empty(0, dtype=TORCH_DTYPES[dt]).element_size()
+    at_line = -(-(2 << 20) * (2 if packed else 1) // (h * S * d * element))
+    rng = np.random.default_rng(S)
+    for B in (at_line - 1, at_line):
+        lens = [S] + [int(n) for n in rng.integers(1, S + 1, B - 1)] if packed else [S] * B
+        g = torch.Generator(device="cuda").manual_seed(B)
+        q, k, v = (torch.randn(B, h, S, d, generator=g, device="cuda").to(TORCH_DTYPES[dt]) for _ in range(3))
+        pitch, given = (S + 7) // 8 * 8, v
+        if v_transposed:
+            given = torch.full((B, h, d, pitch), float("nan"), dtype=v.dtype, device="cuda")
+            given[..., :S] = v.transpose(2, 3)
+        cu = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda") if packed else None
+        keys = (torch.arange(S, device="cuda")[None] < torch.tensor(lens, device="cuda")[:, None])
+        whole, out = _guarded(sum(lens), h * d, q.dtype)
+        ok(ttmi.ttmi_fused_attention(ptr(q), ptr(k), ptr(given), None, ptr(out), ptr(cu), B, h, S, d, pitch if v_transposed else 0, 0.125, TTMI_DTYPES[dt], stream()))
+        scores = (q.double() @ k.double().transpose(2, 3).contiguous() * 0.125).masked_fill(~keys[:, None, None, :], float("-inf"))
+        want = (torch.softmax(scores, -1) @ v.double()).transpose(1, 2).reshape(B * S, h * d)[keys.reshape(-1)]
+        # P is rounded to 16 bits before the second product
+        assert float((out.double() - want).abs().max()) <= (5e-5 if dt == "f32" else 2 * GEMM_TOL[dt])
+        assert bool((whole[sum(lens):] == 7.0).all())

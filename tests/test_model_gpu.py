@@ -917,9 +917,22 @@ def test_multi_headed_attention_context_memory_cache(tt, oracle):
     assert np.isfinite(host(out2)).all()
 
 
+def _spied(monkeypatch, module, name):
+    """-> a list that gets, for each call of module.name, whether it had a result."""
+    results, call = [], getattr(module, name)
+
+    def spy(*args):
+        result = call(*args)
+        results.append(result is not None)
+        return result
+
+    monkeypatch.setattr(module, name, spy)
+    return results
+
+
 @pytest.mark.parametrize("form", ["plain", "strided", "graded", "tt tensors", "no mask", "user dict"])
 @pytest.mark.parametrize("attn_type", ["self", "context"])
-def test_attention_calls_handled_by_the_extension(tt, form, attn_type):
+def test_attention_calls_handled_by_the_extension(tt, monkeypatch, form, attn_type):
     """A call whose results go to torch is handled by the extension, one that brings its own output by the Python wrapper: the same bits,
     the same cache, whatever the arguments are; what is no tensor is left to the wrapper."""
     import collections
@@ -952,7 +965,11 @@ def test_attention_calls_handled_by_the_extension(tt, form, attn_type):
         out, attn = layer(m, m, q, mask=k, layer_cache=cache, attn_type=attn_type, pre_layernorm=True, post_add_input=True, **kw)
         return out, attn, cache
 
-    one, other = run(), run(output=tt.cxx.Tensor.create_empty(), attn=tt.cxx.Tensor.create_empty())
+    handled = _spied(monkeypatch, tt.cxx, "call_multi_headed_attention")
+    one = run()
+    assert handled == [form != "user dict"]
+    other = run(output=tt.cxx.Tensor.create_empty(), attn=tt.cxx.Tensor.create_empty())
+    assert len(handled) == 1  # a call that brings its own output is the wrapper's
     assert torch.equal(one[0], other[0]) and torch.equal(one[1], other[1])
     for name in ("self_keys", "self_values", "memory_keys", "memory_values"):
         a, b = one[2][name], other[2][name]
@@ -1050,6 +1067,43 @@ def test_feed_forward_blocks(tt, oracle, dtype, is_trans_weight):
     assert got.dtype == dtype and max_abs(f(got), oracle.distill_ffn(*args)) < tol
     with pytest.raises(RuntimeError, match="model_dim"):
         pw(torch.zeros(1, 2, H + 8, device="cuda", dtype=dtype), is_trans_weight=is_trans_weight)
+
+
+@pytest.mark.parametrize("form", ["plain", "strided", "graded", "tt tensor", "one row", "half"])
+@pytest.mark.parametrize("block", ["PositionwiseFeedForward", "DistrillFFN"])
+def test_feed_forward_calls_handled_by_the_extension(tt, monkeypatch, form, block):
+    """The same of the feed-forward blocks: the bits of a call that brings its own output, which the wrapper handles; what is no tensor is
+    left to the wrapper and fails as it does there."""
+    from turbotransformers_amd.layers.utils import convert2tt_tensor
+    torch.manual_seed(13)
+    H, F = 256, 1024
+    dtype = torch.float16 if form == "half" else torch.float32
+    mod = _OnmtLikeFfn(H, F).cuda().to(dtype)
+    layer = tt.PositionwiseFeedForward.from_onmt(mod) if block == "PositionwiseFeedForward" else tt.DistrillFFN.from_torch(mod, mod.layer_norm)
+    x = torch.randn(1 if form == "one row" else 3, 1 if form == "one row" else 17, H, generator=torch.Generator().manual_seed(14)).cuda().to(dtype)
+
+    def given():
+        if form == "strided":
+            return torch.stack([x, x], 2)[:, :, 1]
+        if form == "graded":
+            return x.clone().requires_grad_()
+        return convert2tt_tensor(x.clone()) if form == "tt tensor" else x
+
+    handled = _spied(monkeypatch, tt.cxx, "call_feed_forward")
+    one = layer(given())
+    assert handled == [True] and isinstance(one, torch.Tensor) and one.dtype == dtype and not one.requires_grad
+    other = layer(given(), output=tt.cxx.Tensor.create_empty())
+    assert len(handled) == 1 and torch.equal(one, other) and one.shape == x.shape
+    host_copy = layer(given(), return_type=tt.ReturnType.NUMPY)
+    assert len(handled) == 1 and np.array_equal(host_copy, one.float().cpu().numpy())
+    for bad in (None, "x", [1.0]):
+        errors = []
+        for kw in ({}, dict(output=tt.cxx.Tensor.create_empty())):
+            with pytest.raises(Exception) as e:
+                layer(bad, **kw)
+            errors.append(type(e.value))
+        assert errors[0] is errors[1], bad
+    assert not any(handled[1:])
 
 
 @pytest.mark.parametrize("dtype,layers", [(torch.float32, 5), (torch.float16, 9)])
