@@ -186,7 +186,12 @@ static int launch_ln_rows(T* out, const T* input, const T* bias, const T* gamma,
   // Without an upper line: fp16 base 128 x 512 tokens (100 MB a launch), the stores of LayerNorms staying / through 14244 / 14209 us a forward, fp32
   // base 64 x 512 (100 MB) and 128 x 512 (201 MB) level.  out32 stays, and its bytes do not count: large bf16 with it through as well 20 x 100
   // tokens 2123 / 2149, 20 x 128 2587 / 2620, 16 x 256 3631 / 3696, 64 x 512 24065 / 24922; with `out` staying too, 4 x 128 to 64 x 512, 1.000 to 1.004 times the time.
-  const bool through = writes_through(m * n * (int64_t)sizeof(T));
+  // fp32 from 6 MB on, 16 bits from 2 MiB as everywhere.  us a forward, staying / through: int8 (fp32 activations) base 6 x 128 tokens (2.4 MB) 826 /
+  // 837, 8 x 128 867 / 879, 12 x 128 (4.7 MB) 979 / 985, 16 x 128 (6.3 MB) 1106 / 1107, 24 x 128 1548 / 1541, large 5 x 128 (2.6 MB) 1932 / 1965, 8 x 128
+  // (4.2 MB) 2094 / 2114; fp32 base 6 x 128 1083 / 1088, 8 x 128 1191 / 1193, 12 x 128 1416 / 1414, 20 x 100 (6.1 MB) 1665 / 1658; fp16 base 12 x 128
+  // (2.4 MB) 710 / 709, 16 x 128 815 / 804; large bf16 8 x 128 (2.1 MB) 1540 / 1536.
+  const int64_t bytes = m * n * (int64_t)sizeof(T);
+  const bool through = writes_through(bytes) && (sizeof(T) == 2 || bytes >= 6 * 1000 * 1000);
   // Fewer workgroups than CUs: one wavefront each, so that more CUs take part; the lanes of a row are the same ones.  us a forward, four / one:
   // decoder prefix 8 x 33 tokens in fp32 (66 / 264 workgroups) 659 / 656, fp16 1 x 387 (49 / 194) 473.3 / 471.5.  (A maximum is one slot
   // per workgroup of four.)
