@@ -85,7 +85,8 @@ __device__ __forceinline__ void store_vec_unaligned(T* p, const Vec<T, N>& x) {
 // 8 x 128 600 / 583, 585, 590; 8 x 256 829 / 783, 783, 791; fp32 1 x 128 555 / 547, 549, 560; 3 x 128 802 / 778, 780, 784; decoder prefix 8 x 33
 // fp32 667 / 670, 663, 665.  20 x 100 fp16 853 / 814 from 1.5 MB on, 16 x 512 2429 / 2320, 20 packed requests 1875 / 1793.
 // Upper lines: kMostThrough of the ring tiles (gemm_ring.h) and of the large ones (gemm_w4.h, whose fp32 outputs stay whatever their size),
-// kMostRowsThrough of the quantising passes (quant.hip).  LayerNorms and attention have none.
+// kMostRowsThrough of the quantising passes (quant.hip).  LayerNorms and attention have none.  Two begin later than at 2 MiB: the head split of
+// int8 (gemm_ring.h) and LayerNorms in fp32 (rowwise.hip).
 // Rows of a transposed V stay, which at most lengths are no whole cache lines: 40 x 100 tokens 1384 / 1465 with them.
 constexpr int64_t kWriteThroughBytes = 2ll << 20;
 inline bool writes_through(int64_t bytes) { return bytes >= kWriteThroughBytes; }
