@@ -1,0 +1,140 @@
+"""A stack of encoder layers over a few rows as one launch (ttmi_encoder_chain), against the same layers in 64 bits.
+
+Tolerance: a layer rounds its values to 16 bits at eight places (the row, Q, K, V, probabilities, context, the second row, the intermediate
+one), each by at most eps / 2 of an O(1) value, and every one reaches the output through a LayerNorm whose gain here is at most 2: sixteen halves of
+eps per layer and O(1) value, of which the largest of some thousand is within 4.
+"""
+import ctypes
+
+import pytest
+import torch
+
+from helpers import TORCH_DTYPES, TTMI_DTYPES, ok, ptr, stream
+
+pytestmark = pytest.mark.gpu
+EPS = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+
+class Stack:
+    def __init__(self, dt, layers, heads, ffn, seed=0):
+        gen = torch.Generator().manual_seed(seed)
+        self.dt, self.layers, self.heads, self.hidden, self.ffn = dt, layers, heads, heads * 64, ffn
+        h = self.hidden
+        rnd = lambda *shape: torch.randn(shape, generator=gen)
+        self.weights = []
+        for _ in range(layers):
+            w = [rnd(3 * h, h) / h ** 0.5, rnd(3 * h) * 0.1, rnd(h, h) / h ** 0.5, rnd(h) * 0.1, 1 + rnd(h) * 0.1, rnd(h) * 0.1,
+                 rnd(ffn, h) / h ** 0.5, rnd(ffn) * 0.1, rnd(h, ffn) / ffn ** 0.5, rnd(h) * 0.1, 1 + rnd(h) * 0.1, rnd(h) * 0.1]
+            self.weights.append([t.to(TORCH_DTYPES[dt]).cuda() for t in w])
+
+    def input(self, batch, seq, seed):
+        return torch.randn((batch, seq, self.hidden), generator=torch.Generator().manual_seed(seed)).to(TORCH_DTYPES[self.dt]).cuda()
+
+    def run(self, ttmi, x, mask=None, workgroups=0, patience=0):
+        batch, seq, h = x.shape
+        size = ctypes.c_int64()
+        ok(ttmi.ttmi_encoder_chain_workspace(self.layers, batch * seq, self.heads, h, self.ffn, TTMI_DTYPES[self.dt], ctypes.addressof(size)))
+        assert size.value > 0
+        out, space = torch.empty_like(x), torch.zeros(size.value, dtype=torch.uint8, device="cuda")
+        out32 = torch.empty(x.shape, device="cuda") if self.dt == "bf16" else None
+        pointers = (ctypes.c_void_p * (12 * self.layers))(*[w.data_ptr() for l in self.weights for w in l])
+        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(x), None, ptr(mask), ptr(out), ptr(out32), ptr(space), self.layers, batch, seq,
+                                   self.heads, h, self.ffn, 1e-12, TTMI_DTYPES[self.dt], workgroups, patience, stream()))
+        torch.cuda.synchronize()
+        if out32 is not None:
+            assert torch.equal(out, out32.to(out.dtype)) or not torch.isfinite(out).all()
+        return out
+
+    def exact(self, x, mask=None):
+        x = x.double().cpu()
+        batch, seq, h = x.shape
+        norm = lambda y, g, b: torch.nn.functional.layer_norm(y, (h,), g, b, 1e-12)
+        for layer in self.weights:
+            qkv_w, qkv_b, o_w, o_b, g1, b1, w1, c1, w2, c2, g2, b2 = (w.double().cpu() for w in layer)
+            q, k, v = (x @ qkv_w.T + qkv_b).view(batch, seq, 3, self.heads, 64).permute(2, 0, 3, 1, 4)
+            scores = q @ k.transpose(-1, -2) / 8
+            if mask is not None:
+                scores = scores + mask.double().cpu()[:, None, None, :]
+            ctx = (scores.softmax(-1) @ v).permute(0, 2, 1, 3).reshape(batch, seq, h)
+            x = norm(x + ctx @ o_w.T + o_b, g1, b1)
+            y = torch.nn.functional.gelu(x @ w1.T + c1, approximate="tanh")
+            x = norm(x + y @ w2.T + c2, g2, b2)
+        return x
+
+
+# one row, a row short of a block, full blocks, sequences that share it; heads and widths at both
+# ends of the range, an intermediate row that the wavefronts share unevenly
+SHAPES = [(1, 1), (1, 10), (1, 16), (4, 4), (16, 1), (3, 5), (1, 15)]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("layers,heads,ffn", [(2, 12, 3072), (2, 16, 4096), (1, 4, 256), (3, 5, 1088)])
+def test_a_stack_as_one_launch(ttmi, dt, layers, heads, ffn):
+    stack = Stack(dt, layers, heads, ffn)
+    for batch, seq in SHAPES:
+        x = stack.input(batch, seq, batch * 100 + seq)
+        mask = None
+        if seq > 2:
+            mask = torch.zeros((batch, seq))
+            mask[-1, seq // 2:] = -10000.0
+            mask = mask.cuda()
+        error = (stack.run(ttmi, x, mask).double().cpu() - stack.exact(x, mask)).abs().max().item()
+        assert error <= 4 * 8 * EPS[dt] * layers, (batch, seq, error)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("batch,seq", [(1, 10), (2, 8)])
+def test_any_number_of_workgroups_gives_the_same_bits(ttmi, dt, batch, seq):
+    """One workgroup does everything itself; few of them, with no patience, compute what they miss."""
+    stack = Stack(dt, 2, 12, 3072)
+    x = stack.input(batch, seq, 5)
+    want = stack.run(ttmi, x)
+    for workgroups, patience in [(1, 0), (7, 1), (100, 1), (0, 1)]:
+        assert torch.equal(stack.run(ttmi, x, None, workgroups, patience), want), (workgroups, patience)
+
+
+@pytest.mark.parametrize("batch,seq", [(3, 5), (2, 8)])
+def test_what_is_not_finite_stays_in_its_sequence(ttmi, batch, seq):
+    """Among it the NaN that marks a word nobody has written."""
+    stack = Stack("f16", 2, 12, 3072)
+    x = stack.input(batch, seq, 9)
+    want = stack.run(ttmi, x)
+    bad = x.clone()
+    bad[1].view(torch.int16)[:] = -1
+    got = stack.run(ttmi, bad)
+    assert torch.isnan(got[1]).all()
+    bad[1] = float("inf")
+    assert torch.isnan(stack.run(ttmi, bad)[1]).all()
+    for b in (b for b in range(batch) if b != 1):
+        assert torch.equal(got[b], want[b])
+    masked = torch.zeros((batch, seq), device="cuda")
+    masked[0] = torch.finfo(torch.float32).min  # a wholly masked sequence is the mean of its values, as a softmax has it
+    assert torch.isfinite(stack.run(ttmi, x, masked)).all()
+
+
+def test_replayed_from_a_graph(ttmi):
+    """The workspace is prepared on every replay."""
+    stack = Stack("f16", 2, 12, 3072)
+    x, other = stack.input(1, 10, 3), stack.input(1, 10, 4)
+    want = [stack.run(ttmi, x), stack.run(ttmi, other)]
+    size = ctypes.c_int64()
+    ok(ttmi.ttmi_encoder_chain_workspace(2, 10, 12, 768, 3072, TTMI_DTYPES["f16"], ctypes.addressof(size)))
+    out, space, given = torch.empty_like(x), torch.empty(size.value, dtype=torch.uint8, device="cuda"), x.clone()
+    pointers = (ctypes.c_void_p * 24)(*[w.data_ptr() for l in stack.weights for w in l])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(given), None, None, ptr(out), None, ptr(space), 2, 1, 10, 12, 768, 3072, 1e-12,
+                                   TTMI_DTYPES["f16"], 0, 0, stream()))
+    for turn in range(6):
+        given.copy_([x, other][turn % 2])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[turn % 2]), turn
+
+
+def test_what_is_not_built_has_no_workspace(ttmi):
+    size = ctypes.c_int64(7)
+    for args in [(2, 17, 12, 768, 3072, "f16"), (25, 8, 12, 768, 3072, "f16"), (2, 8, 12, 768, 3072, "f32"), (2, 8, 17, 1088, 3072, "f16"),
+                 (2, 8, 3, 192, 768, "f16"), (2, 8, 12, 1536, 3072, "f16"), (2, 8, 12, 768, 3104, "f16"), (2, 8, 12, 768, 4160, "f16")]:
+        ok(ttmi.ttmi_encoder_chain_workspace(*args[:5], TTMI_DTYPES[args[5]], ctypes.addressof(size)))
+        assert size.value == 0, args

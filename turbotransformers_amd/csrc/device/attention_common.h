@@ -134,14 +134,14 @@ __device__ __forceinline__ uint32_t load_mask(const float* mask) { return *reint
 // (error 2^-13; no row with an unmasked key comes near) the maximum is subtracted from the scores first, exactly.
 // The test is three instructions per 32 keys, 1 to 2 % of a launch: fp16 1 x 400 tokens 6.6 / 6.8, 32 packed requests 23.8 / 24.0,
 // fp32 16 x 512 146.1 / 146.6.  (Joined to the test for a maximum that moves it costs registers: 8 x 256 7.8 against 7.6.)
-template <typename Scores>
+template <int N = 16, typename Scores>
 __device__ __forceinline__ float relative_scores(Scores& st, float m_run, float scale_log2e) {
   const float neg_m = -m_run * scale_log2e;
   const bool far = fabsf(neg_m) > 0x1p12f;
   if (__builtin_expect(!__any(far), 1)) return neg_m;
   const float shift = far ? m_run : 0.f;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) st[e] -= shift;
+  for (int e = 0; e < N; ++e) st[e] -= shift;
   return far ? 0.f : neg_m;
 }
 

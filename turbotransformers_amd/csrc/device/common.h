@@ -35,7 +35,8 @@ int check_hip(hipError_t e, const char* what);
 
 inline int launch_status(const char* what) { return check_hip(hipGetLastError(), what); }
 
-int* async_error_flag();  // device-visible pinned int, 0 = ok
+int* async_error_flag();  // device-visible pinned int, 0 = ok, 1 = an embedding id out of range, or:
+constexpr int kRowsNeverCame = 2;
 
 // ---- kernel-selection switches ----------------------------------------------------------
 // Overrides of the launchers' own choices, for A/B timing and for tests of small and ragged shapes.  Each starts

@@ -1,0 +1,607 @@
+// A stack of encoder layers over up to 16 rows as ONE launch (16-bit types).
+//
+// With a handful of rows a layer is six dependent launches of 3.7 to 5.3 us each, of which nothing but the change from one to the next
+// is long: launch, first operands, drain.  Here workgroups of sixteen wavefronts stay, and what one step of the chain leaves for the next goes
+// through memory, past the L2s (an exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same
+// reads and writes 2.9, a barrier over the grid with counters 4 to 5).  Nobody waits at a barrier of the grid: the exchange
+// memory is filled with a word that no result has (kUnwritten: a NaN that every store here replaces by another NaN) and a reader asks
+// again until it has words of another value.  The weights and parameters of an item are requested in front of its rows and arrive while it waits for them.
+//
+// Steps of a layer, and items (16 or 32 columns each) of a step:
+//   0  LayerNorm of the previous layer's rows, QKV product                     3H/32 items
+//   1  attention of all heads (a wavefront each), output projection, residual  H/16
+//   2  LayerNorm, FFN1, GELU                                                   F/32
+//   3  FFN2, residual                                                          H/16
+// and the last LayerNorm.  Rows in front of a LayerNorm travel in fp32; each item normalises all of them for itself (the attention is
+// likewise computed by every item of step 1): a few hundred cycles instead of one more exchange.
+//
+// us per forward, layer by layer / as one launch: fp16 base 1 x 1 token 280 / 158, 1 x 10 305 / 190, 4 x 4 308 / 198; bf16 large 1 x 10
+// 674 / 492, 2 x 8 673 / 506.  What bounds a step of 3.2 to 4 us: the exchange 1.0 to 1.5 (a store to memory, and a load that finds it), the
+// LayerNorm of 16 rows on every CU 0.5 to 1.2 (vector instructions: 16 rows are four a SIMD), the product and the sum over the wavefronts 0.6.
+// Measured and no better: 16 columns an item (240 workgroups instead of 144) level; Q, K, V and the intermediate rows row by row instead
+// of in the order of the registers 10 rows 218 / 183, 16 251 / 194 (the launch alone).
+//
+// Progress does not depend on how many of the workgroups are resident.  Items are pure functions of the step before, and who executes an
+// item a second time writes the same bits.  A workgroup that has waited `patience` polls in vain (others hold the CUs, or the
+// grid is smaller than the items) executes the steps that it misses by itself, from the last one whose inputs it has seen, and
+// goes on; workgroups that start late find everything written.
+#include <mutex>
+#include <set>
+
+#include "attention_common.h"
+
+namespace ttmi {
+namespace {
+
+constexpr int kWaves = 16, kThreads = kWaves * kWave;
+constexpr int kRows = 16;                         // of a block of the matrix instruction: as many as a call may have
+constexpr int kColumns = 2;                       // blocks of 16 columns of an item of steps 0 and 2
+constexpr int kPitch = kColumns * 16 + 4;         // words of a row of a partial tile
+constexpr uint32_t kUnwritten = 0xffffffffu, kOtherNaN = 0xfffefffeu;
+constexpr int kThroughMemory = 17;                // cache policy sc0 | sc1: not from, and not into, the L2 of the XCD
+constexpr int kMostLayers = 24;
+constexpr int kMostTries = 4096;
+constexpr int kLdsMost = 80 * 1024;
+constexpr uint32_t kOutside = 0xffffff00u;        // an offset past every buffer: a load from there is zero
+
+struct ChainLayer {
+  const void *qkv_w, *qkv_b, *out_w, *out_b, *gamma1, *beta1, *ffn1_w, *ffn1_b, *ffn2_w, *ffn2_b, *gamma2, *beta2;
+};
+// Where a layer's results lie in its part of the exchange memory.
+struct Places {
+  uint32_t qk, vt, x0, sum1, mid, x1, sum2, end;
+};
+struct ChainArgs {
+  ChainLayer layer[kMostLayers];
+  const void* input;     // [rows, hidden]
+  const float* input32;  // the same unrounded, or null
+  const float* mask;     // [rows], additive, or null
+  void* out;
+  float* out32;
+  char* exchange;
+  uint32_t layer_bytes;  // of the exchange memory
+  Places at;
+  int layers, rows, seq, heads, hidden, ffn, patience;
+  float eps, scale_log2e, inv_scale;
+  int* error;
+};
+
+inline uint32_t up256(uint32_t n) { return (n + 255u) & ~255u; }
+inline Places places(int rows, int hidden, int ffn, int residual_size) {
+  Places p;
+  const uint32_t r = (uint32_t)rows, h = (uint32_t)hidden;
+  p.qk = 0;                                                  // Q, then K: [H / 8, kRows, 8]
+  p.vt = p.qk + 2 * h * kRows * 2;                           // V: [H, kRows]
+  p.x0 = p.vt + h * kRows * 2;                               // [H / 16, rows, 16] of the residual's type
+  p.sum1 = p.x0 + up256(r * h * (uint32_t)residual_size);    // [rows, H] fp32
+  p.mid = p.sum1 + up256(r * h * 4);                         // [F / 64, 2, 4, kRows, 8], see mid_offset
+  p.x1 = p.mid + (uint32_t)ffn * kRows * 2;
+  p.sum2 = p.x1 + up256(r * h * (uint32_t)residual_size);
+  p.end = p.sum2 + up256(r * h * 4);
+  return p;
+}
+
+__device__ __forceinline__ uint32_t storable(uint32_t word) { return word == kUnwritten ? kOtherNaN : word; }
+// The largest word so far: kUnwritten if one of them is.
+__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x4& x) { return max(max(max(m, x[0]), max(x[1], x[2])), x[3]); }
+__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x2& x) { return max(max(m, x[0]), x[1]); }
+
+template <typename T>
+__device__ __forceinline__ floatx4 mma16(const u32x4& a, const u32x4& b, floatx4 c) {
+  if constexpr (std::is_same<T, f16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ float low(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair & 0xffffu)); }
+template <typename T>
+__device__ __forceinline__ float high(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair >> 16)); }
+
+// Q, K, V and the rows of FFN2 lie as the wavefronts that read them hold them in registers, a load of one 64 consecutive pieces: what goes past
+// the L2 is paid by the line and the load.  In bytes, of an even column (a pair of rows of V):
+__device__ __forceinline__ uint32_t q_offset(int row, int col) { return (uint32_t)(((col >> 3) * kRows + row) * 8 + (col & 7)) * 2; }
+__device__ __forceinline__ uint32_t v_offset(int row, int col) { return (uint32_t)(col * kRows + row) * 2; }
+__device__ __forceinline__ uint32_t mid_offset(int row, int col) {
+  return (uint32_t)(((((col >> 6) * 2 + ((col >> 3) & 1)) * 4 + ((col >> 4) & 3)) * kRows + row) * 8 + (col & 7)) * 2;
+}
+
+// Whether one of the values is an infinity or a NaN.
+template <typename T, typename Words>
+__device__ __forceinline__ bool unbounded(const Words& x) {
+  constexpr uint32_t exponent = std::is_same<T, f16>::value ? 0x7c00u : 0x7f80u;
+  bool any = false;
+#pragma unroll
+  for (uint32_t w = 0; w < sizeof(Words) / 4; ++w) any = any | ((x[w] & exponent) == exponent) | ((x[w] >> 16 & exponent) == exponent);
+  return any;
+}
+// A pair of values of V, zero where its keys are not in [from, to).
+__device__ __forceinline__ uint32_t keys_within(uint32_t pair, int key, int from, int to) {
+  return (key >= from && key < to ? pair & 0xffffu : 0u) | (key + 1 >= from && key + 1 < to ? pair & 0xffff0000u : 0u);
+}
+
+// LDS: rows of the A operand (or, in step 1, the heads' contexts), then the partial tiles.
+__host__ __device__ inline int row_pitch(int hidden) { return hidden * 2 + 16; }  // bytes; four banks further per row
+constexpr int kContextPitch = (kD + 8) * 2;
+__host__ __device__ inline int rows_bytes(int hidden) {
+  const int rows = kRows * row_pitch(hidden), contexts = kWaves * kRows * kContextPitch;
+  return rows > contexts ? rows : contexts;
+}
+__host__ __device__ inline int lds_bytes(int hidden) { return rows_bytes(hidden) + kWaves * kRows * kPitch * 4; }
+
+// TURNS: turns of 256 columns that a row of the hidden state takes at most; PIECES: 128-byte pieces of a row of FFN2's weight
+// that a wavefront takes at most (of the other weights it is one).
+template <typename T, int TURNS, int PIECES>
+__global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr bool WIDE = std::is_same<T, bf16>::value;  // the residual stays in fp32
+  constexpr int RS = WIDE ? 4 : 2;
+  extern __shared__ __align__(16) char smem[];
+  __shared__ int missing;
+  __shared__ ChainLayer layers[kMostLayers];  // (where the arguments lie a first read takes as long as an exchange)
+  // The arguments are read, and what depends on the lane is computed, where an item needs it: kept over the loop they are a hundred registers.
+  typedef const __attribute__((address_space(4))) ChainArgs Arguments;
+  auto arguments = []() __attribute__((always_inline)) {
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return reinterpret_cast<Arguments*>(p);
+  };
+  const int G = gridDim.x, me = blockIdx.x;
+  auto items = [&](int step) __attribute__((always_inline)) {
+    const Arguments& a = *arguments();
+    return step == 4 * a.layers ? 1 : (step & 3) == 0 ? 3 * a.hidden / (16 * kColumns) : (step & 3) == 2 ? a.ffn / (16 * kColumns) : a.hidden / 16;
+  };
+  // The first item of a step for this workgroup.  Steps 1 and 3 are the last workgroups': others than those of steps 0 and 2 where the
+  // grid has as many, so that each has a step's time for its weights to arrive.
+  auto first_item = [&](int step) __attribute__((always_inline)) {
+    const int first = (step & 1) == 1 ? max(G - arguments()->hidden / 16, 0) : 0;
+    return me >= first ? me - first : me - first + G;
+  };
+  const int last_step = 4 * arguments()->layers;
+  auto advance = [&](int& s, int& i) __attribute__((always_inline)) {
+    i += G;
+    while (s <= last_step && i >= items(s)) {
+      ++s;
+      if (s <= last_step) i = first_item(s);
+    }
+  };
+
+  // The item at hand; while `solo` one of a step that others were to execute, on the way to (resume_step, resume_item).
+  int step = 0, item = first_item(0) - G;
+  advance(step, item);
+  if (step > last_step) return;
+  int seen = 0, resume_step = 0, resume_item = 0, tries = 0;
+  bool solo = false;
+  if (threadIdx.x == 0) missing = 0;
+  constexpr int WORDS = sizeof(ChainLayer) / 8;
+  if ((int)threadIdx.x < arguments()->layers * WORDS)
+    reinterpret_cast<uint64_t*>(layers)[threadIdx.x] = reinterpret_cast<const __attribute__((address_space(4))) uint64_t*>(&arguments()->layer)[threadIdx.x];
+  __syncthreads();
+  auto uniform = [](const void* const& p) __attribute__((always_inline)) -> const void* {
+    const uint64_t x = reinterpret_cast<const uint64_t&>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x), hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));  // (they return int)
+    return reinterpret_cast<const void*>((uint64_t)hi << 32 | lo);
+  };
+
+  for (;;) {
+    const Arguments& a = *arguments();
+    const auto& at = a.at;
+    const int H = a.hidden, F = a.ffn, rows = a.rows, patience = a.patience;
+    const int pitch = row_pitch(H);
+    float* const part = reinterpret_cast<float*>(smem + rows_bytes(H));
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 15, lgrp = lane >> 4;
+    const int l = step >> 2, ph = step & 3;
+    const uint32_t base = (uint32_t)l * a.layer_bytes;
+    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, a.layers * a.layer_bytes, 0x00020000);
+    auto load4 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(mem, offset, 0, kThroughMemory); };
+    auto load2 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x2)__builtin_amdgcn_raw_buffer_load_b64(mem, offset, 0, kThroughMemory); };
+    auto load1 = [&](uint32_t offset) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(mem, offset, 0, kThroughMemory); };
+    auto store1 = [&](uint32_t offset, uint32_t x) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b32(storable(x), mem, offset, 0, kThroughMemory); };
+    // Asks again until there is no unwritten word; `ask` returns the largest of those it has loaded.
+    bool late = false;
+    auto await = [&](auto&& ask) __attribute__((always_inline)) {
+      for (int polls = 0;; ++polls) {
+        asm volatile("" ::: "memory");
+        if (__builtin_amdgcn_ballot_w64(ask() == kUnwritten) == 0) break;
+        if (polls >= patience) {
+          late = true;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    };
+
+    // What the item needs besides its rows is requested in front of them: it arrives while the item waits.
+    const ChainLayer& y = layers[min(l, a.layers - 1)];
+    const int K = ph == 3 ? F : H, N = ph == 0 ? 3 * H : ph == 2 ? F : H;
+    const __amdgpu_buffer_rsrc_t weights =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(uniform(ph == 0 ? y.qkv_w : ph == 1 ? y.out_w : ph == 2 ? y.ffn1_w : y.ffn2_w)), 0, step == last_step ? 0 : N * K * 2, 0x00020000);
+    const int n0 = item * (ph & 1 ? 16 : 16 * kColumns);
+    const uint32_t w_row = (uint32_t)((n0 + lrow) * K + lgrp * 16) * 2;
+    // The thread's part of the output: two columns of a row, or two rows of a column of V; 128 threads for 16 x 16 values.
+    const int block = tid >> 7, at_tid = tid & 127;
+    const bool stores = step != last_step && block < (ph & 1 ? 1 : kColumns), transposed = ph == 0 && n0 >= 2 * H;
+    uint32_t bias = 0;
+    if (stores) {
+      const void* b = uniform(ph == 0 ? y.qkv_b : ph == 1 ? y.out_b : ph == 2 ? y.ffn1_b : y.ffn2_b);
+      if (transposed) bias = static_cast<const uint16_t*>(b)[n0 + block * 16 + lrow];
+      else bias = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(b) + n0 + block * 16 + 2 * (tid & 7));
+    }
+    floatx4 acc[kColumns];
+#pragma unroll
+    for (int c = 0; c < kColumns; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+    float res0 = 0.f, res1 = 0.f;  // the residual of the thread's two columns (steps 1 and 3)
+    const bool pairs_here = stores && (at_tid >> 3) < rows;
+
+    if ((ph & 1) == 0) {  // (the last step among them)
+      u32x4 wf[kColumns][2];
+      const uint32_t piece = wave < H / 64 ? w_row + wave * 128 : kOutside;
+#pragma unroll
+      for (int c = 0; c < kColumns; ++c)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) wf[c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, wave < H / 64 ? piece + (uint32_t)(c * 16 * H * 2 + s * 16) : kOutside, 0, 0);
+      if (step == 0) {
+        if (wave < rows)
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t) {
+            const int col = t * 256 + lane * 4;
+            if (col < H) *reinterpret_cast<u32x2*>(smem + wave * pitch + col * 2) = *reinterpret_cast<const u32x2*>(static_cast<const T*>(a.input) + wave * H + col);
+          }
+      } else {
+        u32x2 gm[TURNS], bt[TURNS];
+        {
+          const void* gamma = uniform(ph == 2 ? y.gamma1 : layers[l - 1].gamma2);
+          const void* beta = uniform(ph == 2 ? y.beta1 : layers[l - 1].beta2);
+          const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(gamma), 0, H * 2, 0x00020000);
+          const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(beta), 0, H * 2, 0x00020000);
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t) {
+            gm[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(g, t * 512 + lane * 8, 0, 0);
+            bt[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(b, t * 512 + lane * 8, 0, 0);
+          }
+        }
+        // rows and columns that do not exist are zeros
+        const uint32_t from = ph == 2 ? base + at.sum1 : base - a.layer_bytes + at.sum2;
+        const uint32_t keep = ph == 2 ? base + at.x1 : base + at.x0;
+        u32x4 raw[TURNS];
+        await([&]() __attribute__((always_inline)) {
+          uint32_t m = 0;
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t) {
+            const int col = t * 256 + lane * 4;
+            raw[t] = load4(wave < rows && col < H ? from + (uint32_t)(wave * H + col) * 4 : kOutside);
+          }
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t) m = largest(m, raw[t]);
+          return m;
+        });
+        if (late) {
+          missing = 1;
+        } else if (wave < rows) {
+          float sum = 0.f, sumsq = 0.f;
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float x = __builtin_bit_cast(float, (uint32_t)raw[t][e]);
+              sum += x;
+              sumsq += x * x;
+            }
+          sum = group_sum<kWave>(sum);
+          sumsq = group_sum<kWave>(sumsq);
+          const float mean = sum / (float)H;
+          const float var = fmaxf(sumsq / (float)H - mean * mean, 0.f);  // as in layer_norm_rows
+          const float rstd = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+          for (int t = 0; t < TURNS; ++t) {
+            const int col = t * 256 + lane * 4;
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float b = e & 1 ? high<T>(bt[t][e >> 1]) : low<T>(bt[t][e >> 1]), g = e & 1 ? high<T>(gm[t][e >> 1]) : low<T>(gm[t][e >> 1]);
+              v[e] = b + g * rstd * (__builtin_bit_cast(float, (uint32_t)raw[t][e]) - mean);
+              asm volatile("" : "+v"(v[e]));  // rounded once, from fp32
+            }
+            const u32x2 r = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+            if (col >= H) continue;
+            if (step == last_step) {
+              *reinterpret_cast<u32x2*>(static_cast<T*>(a.out) + wave * H + col) = r;
+              if (WIDE && a.out32 != nullptr) *reinterpret_cast<floatx4*>(a.out32 + wave * H + col) = floatx4{v[0], v[1], v[2], v[3]};
+              continue;
+            }
+            *reinterpret_cast<u32x2*>(smem + wave * pitch + col * 2) = r;
+            if (col / (16 * kColumns) == item) {
+              const uint32_t to = keep + (uint32_t)(((col >> 4) * rows + wave) * 16 + (col & 15)) * RS;
+              if constexpr (WIDE) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) store1(to + 4 * e, __builtin_bit_cast(uint32_t, v[e]));
+              } else {
+                store1(to, r[0]);
+                store1(to + 4, r[1]);
+              }
+            }
+          }
+        }
+      }
+      __syncthreads();
+      if (wave < H / 64) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const u32x4 x = *reinterpret_cast<const u32x4*>(smem + lrow * pitch + wave * 128 + lgrp * 32 + s * 16);
+#pragma unroll
+          for (int c = 0; c < kColumns; ++c) acc[c] = mma16<T>(x, wf[c][s], acc[c]);
+        }
+      }
+    } else {
+      // The residual, written a step before what the item waits for (the first layer's is the input).
+      const bool from_input = step == 1;
+      const int res_index = (tid >> 3) * H + item * 16 + 2 * (tid & 7);
+      const uint32_t res_at = pairs_here && !from_input ? (ph == 1 ? base + at.x0 : base + at.x1) + (uint32_t)(item * rows * 16 + 2 * tid) * RS : kOutside;
+      u32x2 res = {0u, 0u};
+      auto ask_residual = [&]() __attribute__((always_inline)) {
+        if constexpr (WIDE) res = load2(res_at);
+        else res[0] = load1(res_at);
+        return res;
+      };
+      if (ph == 1) {
+        const bool has = wave < a.heads;
+        u32x4 wf[2];
+        const uint32_t piece = has ? w_row + wave * 128 : kOutside;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) wf[s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, piece + s * 16, 0, 0);
+        char* const ctx = smem + wave * (kRows * kContextPitch);
+        // Scores transposed: lane = query, four keys a register quad, which is how the second product takes them if V^T comes in the same
+        // order (its other four keys of eight are zeros).  A query sees the keys of its own sequence.
+        u32x4 qf[2], kf[2];
+        u32x2 vf[4];
+        const uint32_t mask_bits = a.mask != nullptr ? load_mask(a.mask + min(lrow, rows - 1)) : 0u;
+        const int first = lrow / a.seq * a.seq, last = first + a.seq;
+        const bool has_row = has && lrow < rows;  // (the others are zeros)
+        const uint32_t q_at = base + at.qk + q_offset(lrow, wave * kD + lgrp * 8), k_at = q_at + (uint32_t)H * 32;
+        const uint32_t v_at = base + at.vt + v_offset(4 * lgrp, wave * kD + lrow);
+        await([&]() __attribute__((always_inline)) {
+          const u32x2 r = ask_residual();
+#pragma unroll
+          for (int s = 0; s < 2; ++s) {
+            qf[s] = load4(has_row ? q_at + s * 1024 : kOutside);
+            kf[s] = load4(has_row ? k_at + s * 1024 : kOutside);
+          }
+#pragma unroll
+          for (int t = 0; t < 4; ++t) vf[t] = load2(has ? v_at + t * 512 : kOutside);
+          uint32_t m = largest(0u, r);
+#pragma unroll
+          for (int s = 0; s < 2; ++s) m = largest(largest(m, qf[s]), kf[s]);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) m = largest(m, vf[t]);
+          return m;
+        });
+        if (has) {
+          floatx4 st = {0.f, 0.f, 0.f, 0.f};
+          const float mk = lrow < rows ? mask_in_scores(mask_bits, a.inv_scale) : -__builtin_inff();
+          st = __builtin_amdgcn_mfma_f32_16x16x4f32(lgrp == 0 ? mk : 0.f, 1.f, st, 0, 0, 0);
+#pragma unroll
+          for (int s = 0; s < 2; ++s) st = mma16<T>(kf[s], qf[s], st);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st[e] = 4 * lgrp + e >= first && 4 * lgrp + e < last ? st[e] : -__builtin_inff();
+          float mx = fmaxf(fmaxf(st[0], st[1]), fmaxf(st[2], st[3]));
+          const LanePair rows2 = swap_rows(mx);
+          mx = fmaxf(rows2.a, rows2.b);
+          const LanePair halves = swap_halves(mx);
+          const float m_run = fmaxf(-kFarthestScore, fmaxf(halves.a, halves.b));
+          const float neg_m = relative_scores<4>(st, m_run, a.scale_log2e);
+          u32x4 pf = {0u, 0u, 0u, 0u};
+          float sum = 0.f;
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            pf[w] = pack2<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w], a.scale_log2e, neg_m)),
+                             __builtin_amdgcn_exp2f(__builtin_fmaf(st[2 * w + 1], a.scale_log2e, neg_m)));
+            sum = add_pair<T>(pf[w], sum);
+          }
+          const LanePair sum2 = swap_rows(sum);
+          sum = sum2.a + sum2.b;
+          const LanePair sum4 = swap_halves(sum);
+          const float inv = 1.0f / (sum4.a + sum4.b);
+          // (0 * infinity: where V is not finite, one sequence at a time)
+          const bool apart = a.seq < rows && __builtin_amdgcn_ballot_w64(unbounded<T>(vf[0]) | unbounded<T>(vf[1]) | unbounded<T>(vf[2]) | unbounded<T>(vf[3])) != 0;
+#pragma unroll 1
+          for (int from = 0; from < (apart ? rows : 1); from += a.seq) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              u32x2 v = vf[t];
+              if (apart)
+#pragma unroll
+                for (int w = 0; w < 2; ++w) v[w] = keys_within(v[w], 4 * lgrp + 2 * w, from, from + a.seq);
+              const floatx4 ot = mma16<T>(u32x4{v[0], v[1], 0u, 0u}, pf, floatx4{0.f, 0.f, 0.f, 0.f});
+              if (!apart || first == from)
+                *reinterpret_cast<u32x2*>(ctx + lrow * kContextPitch + (t * 16 + 4 * lgrp) * 2) =
+                    u32x2{pack2<T>(ot[0] * inv, ot[1] * inv), pack2<T>(ot[2] * inv, ot[3] * inv)};
+            }
+          }
+#pragma unroll
+          for (int s = 0; s < 2; ++s) acc[0] = mma16<T>(*reinterpret_cast<const u32x4*>(ctx + lrow * kContextPitch + lgrp * 32 + s * 16), wf[s], acc[0]);
+        }
+      } else {
+        const int share = (F / 64 + kWaves - 1) / kWaves, first = wave * share, mine = min(F / 64 - first, share);
+        const int there = lrow < rows ? mine : 0;
+        const uint32_t row_at = base + at.mid + mid_offset(lrow, first * 64 + lgrp * 16);
+        u32x4 wf[2 * PIECES], af[2 * PIECES];
+#pragma unroll
+        for (int p = 0; p < 2 * PIECES; ++p)
+          wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (first + p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
+        await([&]() __attribute__((always_inline)) {
+          const u32x2 r = ask_residual();
+#pragma unroll
+          for (int p = 0; p < 2 * PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
+          uint32_t m = largest(0u, r);
+#pragma unroll
+          for (int p = 0; p < 2 * PIECES; ++p) m = largest(m, af[p]);
+          return m;
+        });
+#pragma unroll
+        for (int p = 0; p < 2 * PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
+      }
+      if (late) missing = 1;
+      if (from_input && pairs_here) {
+        if (WIDE && a.input32 != nullptr) res = *reinterpret_cast<const u32x2*>(a.input32 + res_index);
+        else res[0] = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(a.input) + res_index);
+      }
+      if (WIDE && (!from_input || a.input32 != nullptr)) {
+        res0 = __builtin_bit_cast(float, (uint32_t)res[0]);
+        res1 = __builtin_bit_cast(float, (uint32_t)res[1]);
+      } else {
+        res0 = low<T>(res[0]);
+        res1 = high<T>(res[0]);
+      }
+    }
+
+#pragma unroll
+    for (int c = 0; c < kColumns; ++c)
+      if (c == 0 || (ph & 1) == 0)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[(wave * kRows + lgrp * 4 + e) * kPitch + c * 16 + lrow] = acc[c][e];
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(missing) != 0) {  // set in front of the barrier: the same for all
+      __syncthreads();
+      if (tid == 0) missing = 0;
+      if (!solo && seen < step) {
+        solo = true;
+        resume_step = step, resume_item = item;
+        step = seen, item = 0;
+      } else if (++tries > kMostTries) {  // (not reached: what an item reads has been written, or is being written by a workgroup that runs)
+        if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
+        return;
+      }
+      __syncthreads();
+      continue;
+    }
+
+    if (stores) {
+      float v0 = 0.f, v1 = 0.f;
+      if (transposed) {  // V: two rows of a column
+        const int r = 2 * (at_tid >> 4);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          v0 += part[(w * kRows + r) * kPitch + block * 16 + lrow];
+          v1 += part[(w * kRows + r + 1) * kPitch + block * 16 + lrow];
+        }
+        const float b = low<T>(bias);
+        v0 = r < rows ? v0 + b : 0.f;
+        v1 = r + 1 < rows ? v1 + b : 0.f;
+        store1(base + at.vt + v_offset(r, n0 - 2 * H + block * 16 + lrow), pack2<T>(v0, v1));
+      } else if (pairs_here) {
+        const int r = at_tid >> 3, c = block * 16 + 2 * (tid & 7);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          const floatx2 p = *reinterpret_cast<const floatx2*>(part + (w * kRows + r) * kPitch + c);
+          v0 += p[0];
+          v1 += p[1];
+        }
+        v0 += low<T>(bias);
+        v1 += high<T>(bias);
+        if (ph == 0) {
+          store1(base + at.qk + q_offset(r, n0 + c), pack2<T>(v0, v1));
+        } else if (ph == 2) {
+          store1(base + at.mid + mid_offset(r, n0 + c), pack2<T>(gelu_tanh(v0), gelu_tanh(v1)));
+        } else {
+          const uint32_t to = base + (ph == 1 ? at.sum1 : at.sum2) + (uint32_t)(r * H + n0 + c) * 4;
+          store1(to, __builtin_bit_cast(uint32_t, v0 + res0));
+          store1(to + 4, __builtin_bit_cast(uint32_t, v1 + res1));
+        }
+      }
+    }
+    tries = 0;
+    if (!solo) {
+      seen = step;
+      advance(step, item);
+      if (step > last_step) return;
+    } else if (++item >= items(step)) {
+      item = 0;
+      if (++step == resume_step) item = resume_item, solo = false;
+    }
+    __syncthreads();  // the rows and partial tiles have been read
+  }
+#endif
+}
+
+__global__ void unwritten_kernel(u32x4* p, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
+}
+
+int64_t workspace_bytes(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype) {
+  const bool takes = (dtype == TTMI_F16 || dtype == TTMI_BF16) && layers >= 1 && layers <= kMostLayers && rows >= 1 && rows <= kRows && heads >= 1 &&
+                     heads >= 4 && heads <= kWaves && hidden == heads * kD && ffn >= 256 && ffn % 64 == 0 && ffn <= kWaves * 4 * 64;
+  if (!takes) return 0;
+  return layers * (int64_t)places((int)rows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end;
+}
+
+}  // namespace
+}  // namespace ttmi
+
+using namespace ttmi;
+
+extern "C" {
+
+int ttmi_encoder_chain_workspace(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype, int64_t* bytes) {
+  TTMI_REQUIRE(bytes != nullptr, "null result");
+  *bytes = workspace_bytes(layers, rows, heads, hidden, ffn, dtype);
+  return 0;
+}
+
+int ttmi_encoder_chain(const void* const* weights, const void* input, const float* input32, const float* mask, void* out, float* out32,
+                       void* workspace, int64_t layers, int64_t batch, int64_t seq, int64_t heads, int64_t hidden, int64_t ffn, float eps, int dtype,
+                       int workgroups, int patience, void* stream) {
+  TTMI_REQUIRE(weights && input && out && workspace, "null tensor");
+  TTMI_REQUIRE(batch > 0 && seq > 0 && batch <= kRows && seq <= kRows && workgroups >= 0 && patience >= 0, "bad shape");
+  const int64_t rows = batch * seq, bytes = workspace_bytes(layers, rows, heads, hidden, ffn, dtype);
+  TTMI_REQUIRE(bytes > 0, "this stack of layers is not run as one launch");
+  ChainArgs a{};
+  uintptr_t bits = reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(input32) | reinterpret_cast<uintptr_t>(out) |
+                   reinterpret_cast<uintptr_t>(out32) | reinterpret_cast<uintptr_t>(workspace);
+  for (int64_t l = 0; l < layers; ++l) {
+    const void* const* w = weights + l * 12;
+    for (int i = 0; i < 12; ++i) {
+      TTMI_REQUIRE(w[i] != nullptr, "null weight");
+      bits |= reinterpret_cast<uintptr_t>(w[i]);
+    }
+    a.layer[l] = {w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], w[10], w[11]};
+  }
+  TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
+  const int cus = compute_units();
+  a.input = input, a.input32 = input32, a.mask = mask, a.out = out, a.out32 = out32, a.exchange = static_cast<char*>(workspace);
+  a.layer_bytes = (uint32_t)(bytes / layers);
+  a.at = places((int)rows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2);
+  a.layers = (int)layers, a.rows = (int)rows, a.seq = (int)seq, a.heads = (int)heads, a.hidden = (int)hidden, a.ffn = (int)ffn;
+  a.patience = patience > 0 ? patience : 512;
+  a.eps = eps, a.scale_log2e = 0.125f * 1.4426950408889634f, a.inv_scale = 8.0f, a.error = async_error_flag();
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * cus)), dim3(256), 0, s, static_cast<u32x4*>(workspace),
+                     bytes / 16);
+  const int64_t widest = std::max(3 * hidden, ffn) / (16 * kColumns) + hidden / 16;
+  const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(widest, cus);
+  const int lds = lds_bytes((int)hidden);
+  // more than 64 KB of dynamic LDS: the limit is raised once per kernel and device
+  auto launch = [&](auto kernel) -> int {
+    static std::mutex mu;
+    static std::set<int> done;
+    int dev = 0;
+    TTMI_HIP(hipGetDevice(&dev));
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      if (done.count(dev) == 0) {
+        TTMI_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMost));
+        done.insert(dev);
+      }
+    }
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, s, a);
+    return launch_status("encoder_chain_kernel");
+  };
+  auto sized = [&](auto turns, auto pieces) -> int {
+    constexpr int TURNS = decltype(turns)::value, PIECES = decltype(pieces)::value;
+    return dtype == TTMI_F16 ? launch(encoder_chain_kernel<f16, TURNS, PIECES>) : launch(encoder_chain_kernel<bf16, TURNS, PIECES>);
+  };
+  if (hidden <= 3 * 256 && ffn <= kWaves * 3 * 64) return sized(std::integral_constant<int, 3>{}, std::integral_constant<int, 3>{});
+  return sized(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});
+}
+
+}  // extern "C"

@@ -226,7 +226,9 @@ int ttmi_event_elapsed_ms(void* start, void* stop, float* ms) {
 int ttmi_check_async(void) {
   int* flag = async_error_flag();
   if (flag && *flag != 0) {
+    const int what = *flag;
     *flag = 0;
+    if (what == kRowsNeverCame) return fail(TTMI_EDEVICE, "encoder chain: rows that it waited for never came");
     return fail(TTMI_EINDEX, "embedding id out of range");
   }
   return 0;

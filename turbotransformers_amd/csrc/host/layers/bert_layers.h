@@ -14,6 +14,7 @@
 #pragma once
 
 #include <string>
+#include <vector>
 
 #include "core/tensor.h"
 #include "layers/kernels.h"
@@ -47,10 +48,16 @@ class BertIntermediate {
     EnforceShapeAndType();
   }
   void EnforceShapeAndType() const;
+  DLDataType dtype() const { return dense_weight_.dtype(); }
   // output = gelu(input * W + b)   (bert_intermediate.cpp:32-50)
   void operator()(const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
   WeightRange weight() const { return packed_.Range(dense_weight_); }
   int64_t out_features() const { return dense_weight_.shape(1); }
+  int64_t in_features() const { return dense_weight_.shape(0); }
+  // weight [out,in], bias
+  void AppendParameters(std::vector<const void*>* to) const {
+    to->insert(to->end(), {packed_.Get(dense_weight_, false).data, dense_bias_.raw()});
+  }
 
  private:
   core::Tensor dense_weight_, dense_bias_;
@@ -68,6 +75,13 @@ class BertOutput {
   // output = LN(hidden_states * W + b + input_tensor)   (bert_output.cpp:29-55)
   void operator()(const core::Tensor& hidden_states, const core::Tensor& input_tensor, core::Tensor* output_tensor) const;
   WeightRange weight() const { return packed_.Range(dense_weight_); }
+  int64_t in_features() const { return dense_weight_.shape(0); }
+  int64_t out_features() const { return dense_weight_.shape(1); }
+  DLDataType dtype() const { return dense_weight_.dtype(); }
+  // weight [out,in], bias, LayerNorm gamma and beta
+  void AppendParameters(std::vector<const void*>* to) const {
+    to->insert(to->end(), {packed_.Get(dense_weight_, false).data, dense_bias_.raw(), layer_norm_weight_.raw(), layer_norm_bias_.raw()});
+  }
 
  private:
   core::Tensor dense_weight_, dense_bias_, layer_norm_weight_, layer_norm_bias_;

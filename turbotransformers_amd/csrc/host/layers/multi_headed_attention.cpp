@@ -489,5 +489,51 @@ void MultiHeadedAttentionSmartBatch::Forward(const Tensor& key_tensor, const Ten
                 post_layernorm, post_add_input, is_trans_weight, nullptr, ahead);
 }
 
+bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, const Tensor& hidden, const Tensor& mask, Tensor* out) {
+  if (layers.empty() || hidden.is_null() || !hidden.is_gpu() || hidden.n_dim() != 3) return false;
+  const BertAttention& first = *layers[0].attention;
+  const int64_t batch = hidden.shape(0), seq = hidden.shape(1), width = hidden.shape(2), rows = batch * seq;
+  const int64_t heads = first.heads(), ffn = layers[0].intermediate->out_features(), count = (int64_t)layers.size();
+  const int dt = core::ToDeviceDType(hidden.dtype());
+  if (batch < 1 || seq < 1 || first.hidden() != width) return false;
+  int64_t bytes = 0;
+  TT_DEVICE_CALL(ttmi_encoder_chain_workspace(count, rows, heads, width, ffn, dt, &bytes));
+  if (bytes <= 0) return false;
+  for (const auto& l : layers) {
+    const bool same = l.attention->heads() == heads && l.attention->hidden() == width && l.intermediate->in_features() == width &&
+                      l.intermediate->out_features() == ffn && l.output->in_features() == ffn && l.output->out_features() == width &&
+                      core::SameDataType(l.attention->dtype(), hidden.dtype()) && core::SameDataType(l.intermediate->dtype(), hidden.dtype()) &&
+                      core::SameDataType(l.output->dtype(), hidden.dtype());
+    if (!same) return false;
+  }
+  const float* additive = nullptr;
+  if (!mask.is_null()) {
+    if (!MultiHeadedAttention::UseFusedCore(mask, nullptr, width / heads, dt) || mask.numel() != rows) return false;
+    additive = mask.data<float>();
+  }
+  std::vector<const void*> parameters;
+  parameters.reserve(12 * layers.size());
+  for (const auto& l : layers) {
+    l.attention->AppendParameters(&parameters);
+    l.intermediate->AppendParameters(&parameters);
+    l.output->AppendParameters(&parameters);
+  }
+  const float* input32 = hidden.shadow() != nullptr ? hidden.shadow()->data<float>() : nullptr;
+  uintptr_t bits = reinterpret_cast<uintptr_t>(hidden.raw()) | reinterpret_cast<uintptr_t>(input32);
+  for (const void* p : parameters) bits |= reinterpret_cast<uintptr_t>(p);
+  if ((bits & 15) != 0) return false;
+  const DLDeviceType dev = hidden.device_type();
+  const int dev_id = hidden.device_id();
+  Tensor workspace(nullptr);
+  float* const space = workspace.Reshape<float>({bytes / 4}, dev, dev_id, "EncoderChain/workspace");
+  out->ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
+  void* const result = out->mutable_raw();
+  float* const result32 = kernels::KeepsFp32Residual(*out) ? out->EnsureShadow()->mutableData<float>() : nullptr;
+  if (reinterpret_cast<uintptr_t>(result) % 16 != 0 || result == hidden.raw()) return false;  // (a workgroup that starts late reads the input late)
+  TT_DEVICE_CALL(ttmi_encoder_chain(parameters.data(), hidden.raw(), input32, additive, result, result32, space, count, batch, seq, heads, width,
+                                    ffn, 1e-12f, dt, 0, 0, Stream()));
+  return true;
+}
+
 }  // namespace layers
 }  // namespace turbo_transformers

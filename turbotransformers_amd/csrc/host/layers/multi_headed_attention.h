@@ -142,6 +142,15 @@ class BertAttention : public MultiHeadedAttention {
   }
   void operator()(const core::Tensor& input_tensor, const core::Tensor& attention_mask, core::Tensor* output, core::Tensor* attn,
                   bool is_trans_weight, const std::vector<WeightRange>& ahead, const BertAttention* lender = nullptr) const;
+
+  int64_t heads() const { return num_attention_heads_; }
+  int64_t hidden() const { return dense_weight_.shape(0); }
+  DLDataType dtype() const { return dense_weight_.dtype(); }
+  // QKV weight [3H,H], bias, output weight [H,H], bias, LayerNorm gamma and beta
+  void AppendParameters(std::vector<const void*>* to) const {
+    to->insert(to->end(), {qkv_packed_.Get(qkv_weight_, false).data, qkv_bias_.raw(), dense_packed_.Get(dense_weight_, false).data,
+                           dense_bias_.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw()});
+  }
 };
 
 class MultiHeadedAttentionSmartBatch : public MultiHeadedAttention {
@@ -182,6 +191,13 @@ struct EncoderLayer {
   const BertIntermediate* intermediate;
   const BertOutput* output;
 };
+// The whole stack as one launch (ttmi_encoder_chain) for up to 16 rows in 16-bit types: a block of the matrix instruction, and one row for each
+// of a workgroup's sixteen wavefronts to normalise.  (A form of two blocks, us per forward layer by layer / as one launch: fp16 base 1 x 17 305 / 263, 1 x 32 304 / 277,
+// bf16 large 2 x 16 720 / 689: the gain goes as the rows do, and there a stack gives the bits that its layers give one by one.)  false: nothing was done.  `hidden` [batch,seq,H], `mask` additive
+// fp32 per key or empty.
+bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, const core::Tensor& hidden, const core::Tensor& mask,
+                     core::Tensor* out);
+
 // What the attention core of each layer may read ahead: the layer's other weights and the next layer's first one.  Nothing
 // for weights that stay in the last-level cache (256 MB) from one pass to the next: up to 200 MB of them products run as fast as
 // with one weight over and over, of 640 MB 128 x 2304 x 768 in fp32 halves takes 10.4 instead of 8.2 us.  The tensors of a call

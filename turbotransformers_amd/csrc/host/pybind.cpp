@@ -391,6 +391,7 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
                          &py::cast<const layers::BertOutput&>(t[2])});
     }
     TT_ENFORCE(!subs.empty() && out != nullptr, "run_bert_layers needs layers and an output tensor");
+    if (layers::RunEncoderChain(subs, hidden, mask, out)) return;
     Tensor attention_out(nullptr), intermediate_out(nullptr), even(nullptr), odd(nullptr);
     const Tensor* current = &hidden;
     const auto ahead = layers::WeightsAhead(subs, hidden);
