@@ -5,6 +5,8 @@ Inputs are scaled so outputs are O(1); fp32 must agree to 1e-4 (accumulation ord
 fp16 to 4e-3 and bf16 to 3e-2 max-abs (one storage rounding of an O(1..4) value); int8
 accumulators are compared bit-exactly against an integer brute force.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -2085,3 +2087,23 @@ def test_fused_attention_on_both_sides_of_the_write_through_line(ttmi, dt, v_tra
         # P is rounded to 16 bits before the second product
         assert float((out.double() - want).abs().max()) <= (5e-5 if dt == "f32" else 2 * GEMM_TOL[dt])
         assert bool((whole[sum(lens):] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("tile,m,n,k", [("160x64", 800, 3072, 768), ("160x64", 797, 3080, 768), ("160x128", 1600, 3072, 768),
+                                        ("160x128", 1589, 3064, 768), ("256x160", 6275, 3072, 768), ("256x160", 6145, 3048, 896)])
+def test_tiles_between_powers_of_two(ttmi, dt, tile, m, n, k):
+    """Whole tiles, and rows and columns that end inside one.  Against 64 bits: the result's own rounding (half of its last place), and 2^-12
+    of an O(1) value for sums of k products in fp32 and the GELU of them."""
+    name = ctypes.create_string_buffer(64)
+    ok(ttmi.ttmi_gemm_bias_act_describe(m, n, k, capi.ACT_GELU, TTMI_DTYPES[dt], name, 64))
+    assert tile in name.value.decode(), name.value
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    a, w, b = (torch.randn(shape, generator=gen, device="cuda").mul_(scale).to(TORCH_DTYPES[dt])
+               for shape, scale in [((m, k), 1.0), ((n, k), k ** -0.5), ((n,), 0.1)])
+    c = torch.full((m + 1, n), 7.0, device="cuda", dtype=TORCH_DTYPES[dt])
+    ok(ttmi.ttmi_gemm_bias_act(ptr(a), ptr(w), ptr(b), ptr(c), m, n, k, capi.ACT_GELU, TTMI_DTYPES[dt], stream()))
+    want = torch.nn.functional.gelu(a.double() @ w.double().T + b.double(), approximate="tanh")
+    half = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    assert bool(((c[:m].double() - want).abs() <= half * want.abs() + 2.0 ** -12).all())
+    assert bool((c[m] == 7.0).all())

@@ -534,9 +534,15 @@ inline int launch_ring(GemmArgs g, const Epi& epi, int slices, hipStream_t s) {
 // a workgroup that waits for its own latencies, `shared` one on a CU whose matrix pipe or operand path is full.  The
 // numbers are least-squares fits to launches of M = 72 ... 16384 rows by the four encoder products of hidden 768 and
 // 1024 (fp16, fp32, int8); over those the tile the model picks is 0.3 % (fp32: 2.5 %) slower than the best one.
+// Tiles of 160 rows or columns (16-bit) stand between those that powers of two give: where 128 x 192 are just too many for a round or
+// leave a quarter of the CUs idle.  us, the best tile without / with them: 6275 x 3072 x 768 40.8 / 35.1 (256 x 160), 6275 x 768 x 3072 29.9 /
+// 27.9, 3200 x 3072 x 768 23.0 / 20.5, 2560 x 4096 x 1024 27.4 / 24.7 (160 x 128), 800 x 3072 x 768 8.5 / 7.7 (160 x 64); a forward: base
+// fp16 49 x 128 tokens 1704 / 1612, 20 packed requests 1786 / 1704, 25 x 128 1005 / 993, 3 x 300 637 / 625, large bf16 20 x 128 2594 / 2520, 8 x 100 1478 / 1444.
+// (96 x 192, 160 x 192, 192 x 128, 192 x 192, 96 x 128, 192 x 96 and 128 x 160 as well: 0.1 % more over those launches.)
 struct RingTile {
   int bm, bn, wave_cols, resident;
   float first, again, lone, shared;
+  bool lone_block;  // a wavefront's 16-row blocks do not pair up: a column of V leaves by the four rows, not by eight
 };
 // X(BM, BN, WM, WN, stages, resident, first, again, lone, shared)
 #define TTMI_RING_TILES_16(X)                                \
@@ -544,10 +550,13 @@ struct RingTile {
   X(64, 64, 4, 2, 4, 2, 3.10f, 0.65f, 0.177f, 0.177f)        \
   X(64, 96, 4, 1, 4, 2, 3.27f, 1.15f, 0.188f, 0.212f)        \
   X(128, 64, 2, 2, 4, 1, 3.19f, 2.17f, 0.252f, 0.252f)       \
+  X(160, 64, 2, 2, 4, 1, 3.40f, 2.60f, 0.305f, 0.305f)       \
   X(128, 96, 4, 1, 3, 1, 3.58f, 2.66f, 0.325f, 0.326f)       \
   X(128, 128, 4, 2, 3, 1, 3.74f, 4.03f, 0.374f, 0.373f)      \
+  X(160, 128, 2, 2, 3, 1, 4.65f, 5.20f, 0.411f, 0.411f)      \
   X(128, 192, 4, 2, 3, 1, 4.88f, 6.69f, 0.464f, 0.461f)      \
-  X(256, 128, 4, 2, 3, 1, 5.36f, 8.33f, 0.576f, 0.571f)
+  X(256, 128, 4, 2, 3, 1, 5.36f, 8.33f, 0.576f, 0.571f)      \
+  X(256, 160, 4, 1, 3, 1, 7.10f, 9.60f, 0.661f, 0.661f)
 #define TTMI_RING_TILES_32(X)                                \
   X(32, 64, 2, 2, 4, 3, 3.40f, 0.11f, 0.215f, 0.263f)        \
   X(64, 64, 2, 2, 3, 3, 3.83f, 0.22f, 0.332f, 0.499f)        \
@@ -580,8 +589,8 @@ struct RingTile {
   X(128, 128, 4, 2, 1, 2, 4, 1, 5.71f, 9.31f, 0.573f, 0.573f)      \
   X(128, 192, 4, 2, 1, 2, 4, 1, 7.29f, 13.8f, 0.738f, 0.738f)
 
-#define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
-#define TTMI_SPLIT_ROW(BM, BN, WM, WN, KG, DA, SB, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S},
+#define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S, BM / WM / 16 > 1 && BM / WM / 16 % 2 != 0},
+#define TTMI_SPLIT_ROW(BM, BN, WM, WN, KG, DA, SB, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S, BM / WM / 16 > 1 && BM / WM / 16 % 2 != 0},
 template <size_t ELEM>
 struct RingTiles;
 template <>
@@ -606,10 +615,16 @@ enum class RingUse { kWhole, kSliced, kCut, kLayerNorm };  // never cut along K 
 struct RingPlan {
   int tile = -1, slices = 1;
   int64_t rounds = 0;  // workgroups per CU, rounded up
+  int tile_values = 0;
   double us = 1e300;
 };
 
-// column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V)
+// column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V), and its rows come in pairs of blocks (a
+// forward of fp16 base, without / with tiles of 160 rows there, 16 x 128 tokens 718 / 724 us, 20 x 100 733 / 736)
+// widest: the most columns of a wavefront; the head split has registers for 128
+constexpr int kRingWidest = 160, kRingWidestSplit = 128;
+template <typename Epi>
+constexpr int ring_widest() { return HasColumnPass<Epi>::value ? kRingWidestSplit : kRingWidest; }
 constexpr int kRingColumns = 32;  // the narrowest wavefront's: a limit that is no multiple of it suits no tile
 template <typename Tiles>
 constexpr bool ring_columns_ok() {
@@ -626,7 +641,7 @@ constexpr bool ring_columns_ok() {
 // Host time, ns, with a plain loop / so: fp32 128 x 768 x 3072 2070 / 260, fp16 8 x 768 x 3072 2310 / 190, 2000 x 768 x 3072
 // 730 / 110, whole 145 / 80.
 template <typename Tiles>
-inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit) {
+inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit, int widest) {
   static_assert(ring_columns_ok<Tiles>(), "kRingColumns");
   constexpr uint32_t kMostSlices = 16;
   constexpr uint64_t kMostTiles = 1u << 27;  // (launch_ring refuses such grids: 32-bit arithmetic suffices)
@@ -641,7 +656,7 @@ inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, 
   int index = 0;
   for (const RingTile& t : Tiles::k) {
     const int i = index++;
-    if (column_limit > 0 && column_limit % t.wave_cols != 0) continue;
+    if (t.wave_cols > widest || (column_limit > 0 && (column_limit % t.wave_cols != 0 || t.lone_block))) continue;
     const uint32_t tiles = (uint32_t)std::min<uint64_t>((uint64_t)((rows + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn), kMostTiles);
     const double least = t.first + steps * t.shared * (double)tiles / cus;
     uint32_t room = 0, q = 0;  // room: q workgroups on every CU
@@ -655,17 +670,17 @@ inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, 
       }
       if (use == RingUse::kCut && s == 1 && most > 1) continue;
       const double us = t.first + t.again * (q - 1.0) + share[s] * std::max<double>(t.lone * (q <= (uint32_t)t.resident ? 1 : (q + t.resident - 1) / t.resident), t.shared * q) + extra;
-      if (us < best.us) best = RingPlan{i, (int)s, q, us};
+      if (us < best.us) best = RingPlan{i, (int)s, q, t.bm * t.bn, us};
     }
   }
   return best;
 }
 template <typename T>
-inline RingPlan pick_ring(const GemmArgs& g, RingUse use, int64_t column_limit = 0) {
+inline RingPlan pick_ring(const GemmArgs& g, RingUse use, int64_t column_limit = 0, int widest = kRingWidest) {
   const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T));
   if constexpr (sizeof(T) == 4)
-    if (g.b_split != nullptr) return pick_tile_of<SplitTiles>(g.m, g.n, ksteps, use, column_limit);
-  return pick_tile_of<RingTiles<sizeof(T)>>(g.m, g.n, ksteps, use, column_limit);
+    if (g.b_split != nullptr) return pick_tile_of<SplitTiles>(g.m, g.n, ksteps, use, column_limit, widest);
+  return pick_tile_of<RingTiles<sizeof(T)>>(g.m, g.n, ksteps, use, column_limit, widest);
 }
 
 template <typename T>
@@ -690,7 +705,9 @@ inline int launch_ring_tile(int tile, const GemmArgs& g, const Epi& epi, int sli
     }
   }
 #define TTMI_RING_TRY(BM, BN, WM, WN, NS, R, F, A, L, S) \
-  if (tile == index++) return launch_ring<T, BM, BN, WM, WN, NS>(g, epi, slices, s);
+  if constexpr (BN / WN <= ring_widest<Epi>())           \
+    if (tile == index) return launch_ring<T, BM, BN, WM, WN, NS>(g, epi, slices, s); \
+  ++index;
   if constexpr (sizeof(T) == 2) { TTMI_RING_TILES_16(TTMI_RING_TRY) }
   if constexpr (sizeof(T) == 4) { TTMI_RING_TILES_32(TTMI_RING_TRY) }
   if constexpr (sizeof(T) == 1) { TTMI_RING_TILES_8(TTMI_RING_TRY) }
