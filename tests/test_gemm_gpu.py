@@ -2089,6 +2089,26 @@ def test_fused_attention_on_both_sides_of_the_write_through_line(ttmi, dt, v_tra
         assert bool((whole[sum(lens):] == 7.0).all())
 
 
+@pytest.mark.parametrize("B,S", [(20, 100), (17, 113)])
+def test_fp32_head_split_just_short_of_a_round(ttmi, B, S):
+    """96 x 192 tiles, rows that end inside one, V transposed.  An fp32 product to 3 * 2^-22 of its operands (at least 2^-14), 768 of them summed."""
+    h, d, k, m = 12, 64, 768, B * S
+    pitch = (S + 7) // 8 * 8
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    a, w, b = (torch.randn(shape, generator=gen, device="cuda").mul_(scale) for shape, scale in [((m, k), 1.0), ((3 * h * d, k), k ** -0.5), ((3 * h * d,), 0.1)])
+    q, kk = torch.empty(B, h, S, d, device="cuda"), torch.empty(B, h, S, d, device="cuda")
+    v = torch.full((B, h, d, pitch), 7.0, device="cuda")
+    args = capi.EpilogueArgs(bias=b.data_ptr(), q=q.data_ptr(), k=kk.data_ptr(), v=v.data_ptr(), seq=S, heads=h, head_dim=d, v_seq_pitch=pitch)
+    name = ctypes.create_string_buffer(64)
+    ok(ttmi.ttmi_gemm_describe(m, 3 * h * d, k, capi.EPI_QKV_SPLIT, ctypes.byref(args), capi.F32_PACKED, name, 64))
+    assert "96x192" in name.value.decode(), name.value
+    ok(ttmi.ttmi_gemm_fused(ptr(a), ptr(_packed(ttmi, w)), None, m, 3 * h * d, k, k, k, 3 * h * d, capi.EPI_QKV_SPLIT, ctypes.byref(args), capi.F32_PACKED, stream()))
+    want = (a.double() @ w.double().T + b.double()).view(B, S, 3, h, d).permute(2, 0, 3, 1, 4)
+    room = (a.abs().double() @ w.abs().double().T + b.abs().double()).view(B, S, 3, h, d).permute(2, 0, 3, 1, 4) * (3 * 2.0 ** -22 + 2.0 ** -20)
+    for got, i in [(q, 0), (kk, 1), (v[..., :S].transpose(2, 3), 2)]:
+        assert bool(((got.double() - want[i]).abs() <= room[i]).all()), i
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("tile,m,n,k", [("160x64", 800, 3072, 768), ("160x64", 797, 3080, 768), ("160x128", 1600, 3072, 768),
                                         ("160x128", 1589, 3064, 768), ("256x160", 6275, 3072, 768), ("256x160", 6145, 3048, 896)])

@@ -577,6 +577,10 @@ struct RingTile {
 
 // X(BM, BN, WM, WN, K groups, A steps in registers, B stages, resident, first, again, lone, shared): fp32 with packed weights
 // (gemm_split.h).  Fits of the same kind (M = 40 ... 10240, K = 256 ... 3072; the tile the model picks is 0.1 % slower than the best one).
+// 96 x 192 in twelve wavefronts is for a head split just short of a round of 128 x 192, whose stores the smaller tile takes better: 2000 x 2304 x 768
+// at 100 tokens 27.1 / 22.8 us, a forward of base fp32 20 x 100 1540 / 1512, 20 x 200 2717 / 2590.  (The other products gain in a loop, 1600 x 3072 x
+// 768 24.6 / 21.6, and lose in a forward, where the chip is at its power limit: 15 x 100 1420 / 1425, 12 x 128 1410 / 1414.  Four or six wavefronts 5 %
+// more; 96 x 128, 160 x 64, 160 x 128 and 128 x 160 win nowhere.)
 #define TTMI_SPLIT_TILES(X)                                        \
   X(32, 32, 2, 1, 4, 4, 5, 1, 4.80f, 3.23f, 0.100f, 0.100f)        \
   X(32, 64, 2, 2, 1, 4, 6, 2, 3.02f, 1.19f, 0.260f, 0.161f)        \
@@ -587,6 +591,7 @@ struct RingTile {
   X(64, 192, 4, 2, 1, 2, 4, 1, 4.96f, 7.32f, 0.508f, 0.509f)       \
   X(64, 256, 2, 4, 1, 2, 4, 1, 5.62f, 9.16f, 0.603f, 0.603f)       \
   X(128, 128, 4, 2, 1, 2, 4, 1, 5.71f, 9.31f, 0.573f, 0.573f)      \
+  X(96, 192, 6, 2, 1, 2, 4, 1, 6.60f, 7.50f, 0.620f, 0.620f)       \
   X(128, 192, 4, 2, 1, 2, 4, 1, 7.29f, 13.8f, 0.738f, 0.738f)
 
 #define TTMI_RING_ROW(BM, BN, WM, WN, NS, R, F, A, L, S) RingTile{BM, BN, BN / WN, R, F, A, L, S, BM / WM / 16 > 1 && BM / WM / 16 % 2 != 0},
@@ -621,10 +626,10 @@ struct RingPlan {
 
 // column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V), and its rows come in pairs of blocks (a
 // forward of fp16 base, without / with tiles of 160 rows there, 16 x 128 tokens 718 / 724 us, 20 x 100 733 / 736)
-// widest: the most columns of a wavefront; the head split has registers for 128
-constexpr int kRingWidest = 160, kRingWidestSplit = 128;
+// head_split: tiles of kHeadSplitRows rows are for it alone (below), and it has registers for kRingWidestSplit columns of a wavefront
+constexpr int kHeadSplitRows = 96, kRingWidestSplit = 128;
 template <typename Epi>
-constexpr int ring_widest() { return HasColumnPass<Epi>::value ? kRingWidestSplit : kRingWidest; }
+constexpr bool ring_takes(int rows, int wave_cols) { return HasColumnPass<Epi>::value ? wave_cols <= kRingWidestSplit : rows != kHeadSplitRows; }
 constexpr int kRingColumns = 32;  // the narrowest wavefront's: a limit that is no multiple of it suits no tile
 template <typename Tiles>
 constexpr bool ring_columns_ok() {
@@ -641,7 +646,7 @@ constexpr bool ring_columns_ok() {
 // Host time, ns, with a plain loop / so: fp32 128 x 768 x 3072 2070 / 260, fp16 8 x 768 x 3072 2310 / 190, 2000 x 768 x 3072
 // 730 / 110, whole 145 / 80.
 template <typename Tiles>
-inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit, int widest) {
+inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, int64_t column_limit, bool head_split) {
   static_assert(ring_columns_ok<Tiles>(), "kRingColumns");
   constexpr uint32_t kMostSlices = 16;
   constexpr uint64_t kMostTiles = 1u << 27;  // (launch_ring refuses such grids: 32-bit arithmetic suffices)
@@ -656,7 +661,8 @@ inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, 
   int index = 0;
   for (const RingTile& t : Tiles::k) {
     const int i = index++;
-    if (t.wave_cols > widest || (column_limit > 0 && (column_limit % t.wave_cols != 0 || t.lone_block))) continue;
+    if (head_split ? t.wave_cols > kRingWidestSplit : t.bm == kHeadSplitRows) continue;
+    if (column_limit > 0 && (column_limit % t.wave_cols != 0 || t.lone_block)) continue;
     const uint32_t tiles = (uint32_t)std::min<uint64_t>((uint64_t)((rows + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn), kMostTiles);
     const double least = t.first + steps * t.shared * (double)tiles / cus;
     uint32_t room = 0, q = 0;  // room: q workgroups on every CU
@@ -676,11 +682,11 @@ inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, 
   return best;
 }
 template <typename T>
-inline RingPlan pick_ring(const GemmArgs& g, RingUse use, int64_t column_limit = 0, int widest = kRingWidest) {
+inline RingPlan pick_ring(const GemmArgs& g, RingUse use, int64_t column_limit = 0, bool head_split = false) {
   const int64_t ksteps = g.k / (kRowBytes / (int)sizeof(T));
   if constexpr (sizeof(T) == 4)
-    if (g.b_split != nullptr) return pick_tile_of<SplitTiles>(g.m, g.n, ksteps, use, column_limit, widest);
-  return pick_tile_of<RingTiles<sizeof(T)>>(g.m, g.n, ksteps, use, column_limit, widest);
+    if (g.b_split != nullptr) return pick_tile_of<SplitTiles>(g.m, g.n, ksteps, use, column_limit, head_split);
+  return pick_tile_of<RingTiles<sizeof(T)>>(g.m, g.n, ksteps, use, column_limit, head_split);
 }
 
 template <typename T>
@@ -698,14 +704,16 @@ inline int launch_ring_tile(int tile, const GemmArgs& g, const Epi& epi, int sli
   if constexpr (sizeof(T) == 4) {
     if (g.b_split != nullptr) {
 #define TTMI_SPLIT_TRY(BM, BN, WM, WN, KG, DA, SB, R, F, A, L, S) \
-  if (tile == index++) return launch_split<BM, BN, WM, WN, KG, DA, SB>(g, epi, slices, s);
+  if constexpr (ring_takes<Epi>(BM, BN / WN))                     \
+    if (tile == index) return launch_split<BM, BN, WM, WN, KG, DA, SB>(g, epi, slices, s); \
+  ++index;
       TTMI_SPLIT_TILES(TTMI_SPLIT_TRY)
 #undef TTMI_SPLIT_TRY
       return fail(TTMI_EINVAL, "no such tile");
     }
   }
 #define TTMI_RING_TRY(BM, BN, WM, WN, NS, R, F, A, L, S) \
-  if constexpr (BN / WN <= ring_widest<Epi>())           \
+  if constexpr (ring_takes<Epi>(BM, BN / WN))            \
     if (tile == index) return launch_ring<T, BM, BN, WM, WN, NS>(g, epi, slices, s); \
   ++index;
   if constexpr (sizeof(T) == 2) { TTMI_RING_TILES_16(TTMI_RING_TRY) }

@@ -41,7 +41,7 @@ struct RingKernel {
     RingUse use = cut && column_limit(epi) == 0 ? RingUse::kSliced : RingUse::kWhole;
     if constexpr (IsGelu<Epi>::value && sizeof(T) == 4)
       if (g.b_split == nullptr && keeps_named_form(g)) use = RingUse::kCut;
-    return pick_ring<T>(g, use, column_limit(epi), ring_widest<Epi>());
+    return pick_ring<T>(g, use, column_limit(epi), HasColumnPass<Epi>::value);
   }
   static bool ok(const GemmArgs& g, const Epi& epi, int batch) {
     return batch == 1 && g.k_chunk == 0 && ring_operands_ok<T>(g) && epilogue_vec(epi) && column_limit(epi) % kRingColumns == 0;
