@@ -542,6 +542,32 @@ TTMI_API int ttmi_encoder_chain(const void* const* weights, const void* input, c
                                 float* out32, void* workspace, int64_t layers, int64_t batch, int64_t seq, int64_t heads,
                                 int64_t hidden, int64_t ffn, float eps, int dtype, int workgroups, int patience, void* stream);
 
+#define TTMI_CHAIN_MAX_ROWS 16
+/* A decoder layer's attention or feed-forward block as one launch: a token each of `rows` (up to TTMI_CHAIN_MAX_ROWS) sequences, fp16 or bf16, hidden a
+ * multiple of 64 up to 1024.  As the layers' own launches compute it:
+ * ttmi_decoder_attention     y = LN(x) w_in^T + b_in: rows of Q, K and V (k_out, v_out given: k_past and v_past [rows,heads,keys-1,64] are copied and
+ *                            y's key and value appended) or of Q alone (k_past and v_past [rows,heads,keys,64] are attended over);
+ *                            probs [rows,heads,keys] = softmax(scale q k^T + mask), mask additive fp32 [rows,keys] or null;
+ *                            out = x + (probs v) w_out^T + b_out.  hidden = 64 * heads, up to 512 keys.
+ * ttmi_decoder_feed_forward  out = x + relu(LN(x) w1^T + b1) w2^T + b2; inner a multiple of 64 up to 4096.
+ *   weights [out,in]; out must be another tensor than x
+ *   exchange   as many bytes as ttmi_decoder_chain_workspace says (heads = 0: feed-forward; inner: 3 * hidden or hidden for attention; 0: not
+ *              built), prepared once by ttmi_decoder_chain_prepare and used by one call after the other on one stream
+ *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed
+ *   workgroups, patience: as in ttmi_encoder_chain
+ * No counterpart in the reference. */
+TTMI_API int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, int64_t inner, int64_t keys, int dtype, int64_t* bytes);
+TTMI_API int ttmi_decoder_chain_prepare(void* exchange, int64_t bytes, void* stream);
+TTMI_API int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, float eps, const void* w_in, const void* b_in,
+                                    const void* w_out, const void* b_out, const void* k_past, const void* v_past, void* k_out, void* v_out,
+                                    const float* mask, void* probs, void* out, void* exchange, int turn, int64_t rows, int64_t heads,
+                                    int64_t hidden, int64_t keys, float scale, int dtype, int workgroups, int patience, void* stream);
+TTMI_API int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta, float eps, const void* w1, const void* b1,
+                                       const void* w2, const void* b2, void* out, void* exchange, int turn, int64_t rows, int64_t hidden,
+                                       int64_t inner, int dtype, int workgroups, int patience, void* stream);
+/* *capturing = 1 while calls on the stream are recorded into a graph. */
+TTMI_API int ttmi_stream_capturing(void* stream, int* capturing);
+
 #ifdef __cplusplus
 }
 #endif

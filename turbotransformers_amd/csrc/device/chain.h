@@ -1,0 +1,96 @@
+// What the kernels share that run several dependent steps of a few rows as one launch (encoder_chain.hip, decoder_chain.hip).
+//
+// What one step leaves for the next goes through memory, past the L2s.  The exchange memory is filled with a word that no result has
+// (kUnwritten: a NaN that every store here replaces by another one), and a reader asks again until it has words of another value.
+// An exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same reads and writes 2.9, a
+// barrier over the grid with counters 4 to 5.
+#pragma once
+
+#include "attention_common.h"
+
+namespace ttmi {
+
+constexpr int kChainWaves = 16, kChainThreads = kChainWaves * kWave;
+constexpr int kChainRows = TTMI_CHAIN_MAX_ROWS;    // of a block of the matrix instruction: as many as a call may have
+static_assert(kChainRows == 16 && kChainRows == kChainWaves, "a block of rows, and a row for each wavefront to normalise");
+constexpr int kChainColumns = 2;                   // blocks of 16 columns of an item of a step with LayerNorm in front
+constexpr int kChainPitch = kChainColumns * 16 + 4;  // words of a row of a partial tile
+constexpr uint32_t kUnwritten = 0xffffffffu, kOtherNaN = 0xfffefffeu;
+constexpr int kThroughMemory = 17;                 // cache policy sc0 | sc1: not from, and not into, the L2 of the XCD
+constexpr uint32_t kOutside = 0xffffff00u;         // an offset past every buffer: a load from there is zero
+constexpr int kChainPatience = 512;                // polls, of about a microsecond
+constexpr int kChainMostTries = 4096;
+
+__device__ __forceinline__ uint32_t storable(uint32_t word) { return word == kUnwritten ? kOtherNaN : word; }
+// The largest word so far: kUnwritten if one of them is.
+__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x4& x) { return max(max(max(m, x[0]), max(x[1], x[2])), x[3]); }
+__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x2& x) { return max(max(m, x[0]), x[1]); }
+
+template <typename T>
+__device__ __forceinline__ floatx4 mma16(const u32x4& a, const u32x4& b, floatx4 c) {
+  if constexpr (std::is_same<T, f16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+template <typename T>
+__device__ __forceinline__ float low(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair & 0xffffu)); }
+template <typename T>
+__device__ __forceinline__ float high(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair >> 16)); }
+
+// Rows that the next step multiplies as they are lie as its wavefronts hold them in registers, a load of one 64 consecutive pieces: what
+// goes past the L2 is paid by the line and the load.  [K / 64, 2, 4, kChainRows, 8], in bytes, of an even column:
+__device__ __forceinline__ uint32_t fragment_offset(int row, int col) {
+  return (uint32_t)(((((col >> 6) * 2 + ((col >> 3) & 1)) * 4 + ((col >> 4) & 3)) * kChainRows + row) * 8 + (col & 7)) * 2;
+}
+
+__host__ __device__ inline int chain_row_pitch(int hidden) { return hidden * 2 + 16; }  // bytes of an LDS row of the A operand; four banks further per row
+
+// A row in front of a product: x, four values of every 256 columns per lane (zeros past the row), becomes v = beta + gamma * (x - mean) / sqrt(var + eps).
+template <typename T, int TURNS>
+__device__ __forceinline__ void normalise_row(const float (&x)[TURNS][4], const u32x2 (&gamma)[TURNS], const u32x2 (&beta)[TURNS], int width, float eps,
+                                              float (&v)[TURNS][4]) {
+  float sum = 0.f, sumsq = 0.f;
+#pragma unroll
+  for (int t = 0; t < TURNS; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sum += x[t][e];
+      sumsq += x[t][e] * x[t][e];
+    }
+  sum = group_sum<kWave>(sum);
+  sumsq = group_sum<kWave>(sumsq);
+  const float mean = sum / (float)width;
+  const float var = fmaxf(sumsq / (float)width - mean * mean, 0.f);  // as in layer_norm_rows
+  const float rstd = 1.0f / sqrtf(var + eps);
+#pragma unroll
+  for (int t = 0; t < TURNS; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float b = e & 1 ? high<T>(beta[t][e >> 1]) : low<T>(beta[t][e >> 1]), g = e & 1 ? high<T>(gamma[t][e >> 1]) : low<T>(gamma[t][e >> 1]);
+      v[t][e] = b + g * rstd * (x[t][e] - mean);
+      asm volatile("" : "+v"(v[t][e]));  // rounded once, from fp32
+    }
+}
+
+// Two values of a tile that the wavefronts hold in parts: (row, column) and the one `step` words further.
+__device__ __forceinline__ floatx2 sum_parts(const float* part, int row, int column, int step) {
+  floatx2 v = {0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kChainWaves; ++w) {
+    const float* p = part + (w * kChainRows + row) * kChainPitch + column;
+    v[0] += p[0];
+    v[1] += p[step];
+  }
+  return v;
+}
+
+static __global__ void unwritten_kernel(u32x4* p, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
+}
+inline int launch_unwritten(void* p, int64_t bytes, hipStream_t s) {
+  hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * compute_units())), dim3(256), 0, s, static_cast<u32x4*>(p),
+                     bytes / 16);
+  return launch_status("unwritten_kernel");
+}
+
+}  // namespace ttmi

@@ -1,0 +1,510 @@
+// One decoder layer's attention (self attention over a growing cache, or attention over an encoder memory) or its feed-forward block as
+// ONE launch: a token each of up to 16 sequences, 16-bit types.
+//
+//   attention     0  LayerNorm, projection of Q (and K, V)                     N/32 items
+//                 1  attention, a query each: W wavefronts a head              batch * heads * W / 16
+//                 2  output projection, bias, residual                         H/16
+//   feed-forward  0  LayerNorm, W1, ReLU                                       F/32
+//                 1  W2, bias, residual                                        H/16
+//
+// Such a call was three launches (two), of 4.3 to 5.8 us each on the GPU and 3 on the host, of which nothing but the change from one to the next is
+// long.  The exchange between the steps is that of chain.h, with as many workgroups as there are items, so that every one has requested its
+// weights, or its keys and values, before it waits.  Progress does not depend on how many of them are resident, as in encoder_chain.hip: a workgroup that
+// has waited in vain executes all items of the steps in front of its own.
+//
+// us a step of six layers of base in fp16 (48 launches before, 18 now): 8 sequences, 41 and 100 keys, 236 / 184; 1 x 6 and 20 219 / 158, 4 x 201 and 30
+// 249 / 174, 16 x 41 and 100 248 / 214, 16 x 251 and 256 309 / 262.  What is left of a launch of 9 to 11: its start 0.5, arguments and first operands 1.5 to
+// 2.5, LayerNorm and product 1, an exchange 0.7 to 1.3 each, attention 1 (3.5 with 64 keys a wavefront), its parts' sum and the last product 1.5.
+// Measured and no better: the arguments held in registers (60 of the scalar ones spill) 11.4 / 12.5 a launch.
+//
+// The exchange memory is kept by the caller in two parts that take turns: a launch fills the part that the one before it has used.  Where launches are
+// recorded and replayed, in an order that nobody knows, they use a third part, which is filled in front of each.
+#include <mutex>
+#include <set>
+
+#include "chain.h"
+
+namespace ttmi {
+namespace {
+
+constexpr int kWaves = kChainWaves, kThreads = kChainThreads, kRows = kChainRows, kColumns = kChainColumns, kPitch = kChainPitch;
+constexpr int kMostHidden = 1024, kMostInner = 4096, kMostKeys = 512;
+constexpr int kTurns = kMostHidden / 256, kPieces = kMostInner / 64 / kWaves;
+constexpr int kLdsMost = 80 * 1024;
+
+enum Block { kFeedForward, kSelfAttention, kMemoryAttention };
+
+struct DecoderArgs {
+  const void *x, *gamma, *beta, *w_in, *b_in, *w_out, *b_out;  // x [rows, H]
+  const void *k_past, *v_past;                                 // [rows, heads, past, 64]
+  void *k_out, *v_out;                                         // [rows, heads, keys, 64], or null
+  const float* mask;                                           // [rows, keys], or null
+  void *probs, *out;                                           // [rows, heads, keys]; [rows, H]
+  char *exchange, *other;                                      // the part of this launch, the part to fill, or null
+  uint32_t bytes;                                              // of a part
+  int rows, heads, hidden, width, inner;                       // width: of step 0's product; inner: of the last one's rows
+  int past, keys, waves, patience;                             // waves: of a head
+  float eps, scale;
+  int* error;
+};
+
+// Exchange memory: step 0's rows ([rows, width]; in front of a product in fragment order), then the attention's in fragment order.
+__host__ __device__ inline uint32_t context_at(int width) { return (uint32_t)(kRows * width * 2); }
+
+template <typename T>
+__device__ __forceinline__ float dot8(const u32x4& a, const u32x4& b, float acc) {
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    acc = __builtin_fmaf(low<T>(a[w]), low<T>(b[w]), acc);
+    acc = __builtin_fmaf(high<T>(a[w]), high<T>(b[w]), acc);
+  }
+  return acc;
+}
+// Lanes that differ by 1, 2 and 4, and by 8, 16 and 32.
+template <typename Op>
+__device__ __forceinline__ float over_pieces(float v, Op op) {
+  v = op(v, dpp_move<0xB1>(v));
+  v = op(v, dpp_move<0x4E>(v));
+  return op(v, dpp_move<0x141>(v));  // (row_half_mirror: the quads agree)
+}
+template <typename Op>
+__device__ __forceinline__ float over_keys(float v, Op op) {
+  v = op(v, dpp_move<0x128>(v));  // row_ror:8
+  const LanePair rows = swap_rows(v);
+  v = op(rows.a, rows.b);
+  const LanePair halves = swap_halves(v);
+  return op(halves.a, halves.b);
+}
+
+// LOADS: keys of a lane of the attention
+template <typename T, Block BLOCK, int LOADS>
+__global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderArgs) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int STEPS = BLOCK == kFeedForward ? 2 : 3;
+  constexpr float kLog2e = 1.4426950408889634f;
+  extern __shared__ __align__(16) char smem[];
+  __shared__ int missing;
+  __shared__ float stat[2][kWaves];
+  // (as in encoder_chain.hip: what depends on the lane or the arguments is not kept over the loop)
+  typedef const __attribute__((address_space(4))) DecoderArgs Arguments;
+  auto arguments = []() __attribute__((always_inline)) {
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return reinterpret_cast<Arguments*>(p);
+  };
+  const int G = gridDim.x, me = blockIdx.x;
+  auto items = [&](int step) __attribute__((always_inline)) {
+    const Arguments& a = *arguments();
+    if (step == 0) return a.width / (16 * kColumns);
+    if (step == STEPS - 1) return a.hidden / 16;
+    return (a.rows * a.heads * a.waves + kWaves - 1) / kWaves;
+  };
+  // The steps' items one after the other over the workgroups.
+  auto first_item = [&](int step) __attribute__((always_inline)) {
+    int before = 0;
+    for (int s = 0; s < step; ++s) before += items(s);
+    before %= G;
+    return me >= before ? me - before : me - before + G;
+  };
+  auto advance = [&](int& s, int& i) __attribute__((always_inline)) {
+    i += G;
+    while (s < STEPS && i >= items(s)) {
+      ++s;
+      if (s < STEPS) i = first_item(s);
+    }
+  };
+  // All of the arguments are requested at once: where they lie a first read takes as long as an exchange.
+  {
+    const __attribute__((address_space(4))) uint32_t* words = reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(arguments());
+    uint32_t first[sizeof(DecoderArgs) / 64 + 1];
+#pragma unroll
+    for (uint32_t i = 0; i < sizeof(first) / 4; ++i) first[i] = words[min(i * 16, (uint32_t)sizeof(DecoderArgs) / 4 - 1)];
+#pragma unroll
+    for (uint32_t i = 0; i < sizeof(first) / 4; ++i) asm volatile("" : : "s"(first[i]));
+  }
+  // The workgroups that are done first fill the other part of the exchange memory.
+  auto leave = [&]() __attribute__((always_inline)) {
+    const Arguments& a = *arguments();
+    const int fillers = min(G, items(0));
+    if (a.other != nullptr && me < fillers)
+      for (uint32_t at = (uint32_t)(me * kThreads + (int)threadIdx.x) * 16; at < a.bytes; at += (uint32_t)(fillers * kThreads) * 16)
+        *reinterpret_cast<u32x4*>(a.other + at) = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
+  };
+
+  int step = 0, item = first_item(0) - G;
+  advance(step, item);
+  if (step >= STEPS) return;  // (not of those that fill)
+  int resume_step = 0, resume_item = 0, tries = 0;
+  bool solo = false;
+  if (threadIdx.x == 0) missing = 0;
+  __syncthreads();
+
+  for (;;) {
+    const Arguments& a = *arguments();
+    const int H = a.hidden, rows = a.rows, heads = a.heads, patience = a.patience;
+    float* const part = reinterpret_cast<float*>(smem + kRows * chain_row_pitch(H));
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 15, lgrp = lane >> 4;
+    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, a.bytes, 0x00020000);
+    auto load4 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(mem, offset, 0, kThroughMemory); };
+    auto store1 = [&](uint32_t offset, uint32_t x) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b32(storable(x), mem, offset, 0, kThroughMemory); };
+    // Asks again until there is no unwritten word; `ask` returns the largest of those it has loaded.
+    bool late = false;
+    auto await = [&](auto&& ask) __attribute__((always_inline)) {
+      for (int polls = 0;; ++polls) {
+        asm volatile("" ::: "memory");
+        if (__builtin_amdgcn_ballot_w64(ask() == kUnwritten) == 0) break;
+        if (polls >= patience) {
+          late = true;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    };
+    const bool product = step == 0 || step == STEPS - 1;
+    const int block = tid >> 7, at_tid = tid & 127, row = at_tid >> 3;
+    const int n0 = step == 0 ? item * 16 * kColumns : item * 16;
+    const bool stores = product && block < (step == 0 ? kColumns : 1) && row < rows;
+    const int column = n0 + block * 16 + 2 * (tid & 7);
+    uint32_t bias = 0, residual = 0;
+    if (stores) {
+      bias = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(step == 0 ? a.b_in : a.b_out) + column);
+      if (step != 0) residual = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(a.x) + row * H + column);
+    }
+    floatx4 acc[kColumns];
+#pragma unroll
+    for (int c = 0; c < kColumns; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    if (step == 0) {
+      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_in), 0, a.width * H * 2, 0x00020000);
+      const uint32_t w_row = (uint32_t)((n0 + lrow) * H + wave * 64 + lgrp * 16) * 2;
+      const int pitch = chain_row_pitch(H);
+      u32x4 wf[kColumns][2];
+      u32x2 raw[kTurns], gm[kTurns], bt[kTurns];
+      const __amdgpu_buffer_rsrc_t x = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, rows * H * 2, 0x00020000);
+      const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.gamma), 0, H * 2, 0x00020000);
+      const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.beta), 0, H * 2, 0x00020000);
+#pragma unroll
+      for (int t = 0; t < kTurns; ++t) {  // rows and columns that do not exist are zeros
+        const int col = t * 256 + lane * 4;
+        raw[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(x, wave < rows && col < H ? (uint32_t)(wave * H + col) * 2 : kOutside, 0, 0);
+        gm[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(g, (uint32_t)col * 2, 0, 0);
+        bt[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(b, (uint32_t)col * 2, 0, 0);
+      }
+#pragma unroll
+      for (int c = 0; c < kColumns; ++c)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          wf[c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, wave < H / 64 ? w_row + (uint32_t)(c * 16 * H * 2 + s * 16) : kOutside, 0, 0);
+      if (wave < rows) {
+        float v[kTurns][4], normed[kTurns][4];
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[t][e] = e & 1 ? high<T>(raw[t][e >> 1]) : low<T>(raw[t][e >> 1]);
+        normalise_row<T, kTurns>(v, gm, bt, H, a.eps, normed);
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t) {
+          const int col = t * 256 + lane * 4;
+          if (col < H) *reinterpret_cast<u32x2*>(smem + wave * pitch + col * 2) = u32x2{pack2<T>(normed[t][0], normed[t][1]), pack2<T>(normed[t][2], normed[t][3])};
+        }
+      }
+      __syncthreads();
+      if (wave < H / 64)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const u32x4 rows_here = *reinterpret_cast<const u32x4*>(smem + lrow * pitch + wave * 128 + lgrp * 32 + s * 16);
+#pragma unroll
+          for (int c = 0; c < kColumns; ++c) acc[c] = mma16<T>(rows_here, wf[c][s], acc[c]);
+        }
+    } else if (step == STEPS - 1) {
+      const int K = a.inner, share = (K / 64 + kWaves - 1) / kWaves, first = wave * share, mine = min(K / 64 - first, share), there = lrow < rows ? mine : 0;
+      constexpr int PIECES = BLOCK == kFeedForward ? kPieces : 1;
+      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_out), 0, H * K * 2, 0x00020000);
+      const uint32_t w_row = (uint32_t)((n0 + lrow) * K + first * 64 + lgrp * 16) * 2;
+      const uint32_t row_at = (BLOCK == kFeedForward ? 0u : context_at(a.width)) + fragment_offset(lrow, first * 64 + lgrp * 16);
+      u32x4 wf[2 * PIECES], af[2 * PIECES];
+#pragma unroll
+      for (int p = 0; p < 2 * PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
+      await([&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < 2 * PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
+        uint32_t m = 0;
+#pragma unroll
+        for (int p = 0; p < 2 * PIECES; ++p) m = largest(m, af[p]);
+        return m;
+      });
+      if (late) missing = 1;
+#pragma unroll
+      for (int p = 0; p < 2 * PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
+    } else {
+      // A wavefront takes 8 * LOADS keys of a head: a lane eight columns of every eighth key.
+      const int pair = item * (kWaves / a.waves) + wave / a.waves, share = wave % a.waves, key0 = share * (8 * LOADS) + (lane >> 3), piece = lane & 7;
+      const bool has = pair < rows * heads;
+      const int b = has ? pair / heads : 0, head = has ? pair - b * heads : 0, keys = a.keys, past = a.past;
+      const __amdgpu_buffer_rsrc_t kp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.k_past), 0, rows * heads * past * 128, 0x00020000);
+      const __amdgpu_buffer_rsrc_t vp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.v_past), 0, rows * heads * past * 128, 0x00020000);
+      u32x4 kf[LOADS], vf[LOADS];
+      float mk[LOADS];
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int key = key0 + i * 8;
+        const uint32_t at = has && key < past ? (uint32_t)((pair * past + key) * 128 + piece * 16) : kOutside;
+        kf[i] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(kp, at, 0, 0);
+        vf[i] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(vp, at, 0, 0);
+        mk[i] = a.mask != nullptr ? a.mask[b * keys + min(key, keys - 1)] : 0.f;
+      }
+      u32x4 qf, kn = {0u, 0u, 0u, 0u}, vn = {0u, 0u, 0u, 0u};
+      const uint32_t at = (uint32_t)(b * a.width + head * kD + piece * 8) * 2;
+      await([&]() __attribute__((always_inline)) {
+        qf = load4(has ? at : kOutside);
+        if constexpr (BLOCK == kSelfAttention) {
+          kn = load4(has ? at + (uint32_t)H * 2 : kOutside);
+          vn = load4(has ? at + (uint32_t)H * 4 : kOutside);
+        }
+        return largest(largest(largest(0u, qf), kn), vn);
+      });
+      if (late) missing = 1;
+      float s[LOADS], mx = -__builtin_inff();
+      auto larger = [](float x, float y) { return fmaxf(x, y); };
+      auto add = [](float x, float y) { return x + y; };
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int key = key0 + i * 8;
+        if constexpr (BLOCK == kSelfAttention) {
+          if (key == past) kf[i] = kn, vf[i] = vn;
+          if (!late && has && key < keys) {
+            const int64_t to = ((int64_t)pair * keys + key) * kD + piece * 8;
+            *reinterpret_cast<u32x4*>(static_cast<T*>(a.k_out) + to) = kf[i];
+            *reinterpret_cast<u32x4*>(static_cast<T*>(a.v_out) + to) = vf[i];
+          }
+        }
+        s[i] = __builtin_fmaf(over_pieces(dot8<T>(kf[i], qf, 0.f), add), a.scale, mk[i]);
+        if (key < keys) mx = fmaxf(mx, s[i]);
+      }
+      mx = over_keys(mx, larger);
+      if (lane == 0) stat[0][wave] = mx;
+      __syncthreads();
+      const int lead = wave - share;
+      for (int w = 0; w < a.waves; ++w) mx = fmaxf(mx, stat[0][lead + w]);
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        s[i] = key0 + i * 8 < keys ? __builtin_amdgcn_exp2f((s[i] - mx) * kLog2e) : 0.f;
+        sum += s[i];
+      }
+      sum = over_keys(sum, add);
+      if (lane == 0) stat[1][wave] = sum;
+      __syncthreads();
+      sum = 0.f;
+      for (int w = 0; w < a.waves; ++w) sum += stat[1][lead + w];
+      const float inv = 1.0f / sum;
+      float o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int key = key0 + i * 8;
+        const T p = from_float<T>(s[i] * inv);
+        if (!late && has && key < keys && piece == 0) static_cast<T*>(a.probs)[(int64_t)pair * keys + key] = p;
+        const float weight = to_float(p);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {  // (keys past the last are zeros)
+          o[2 * w] = __builtin_fmaf(weight, low<T>(vf[i][w]), o[2 * w]);
+          o[2 * w + 1] = __builtin_fmaf(weight, high<T>(vf[i][w]), o[2 * w + 1]);
+        }
+      }
+      // eight groups of lanes have a part each: two of a row of 16 lanes meet here, the rest in LDS
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] += dpp_move<0x128>(o[e]);
+      if ((lane & 8) == 0)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+          *reinterpret_cast<floatx4*>(part + (wave * 4 + lgrp) * kD + piece * 8 + e) = floatx4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+    }
+
+    if (product) {
+#pragma unroll
+      for (int c = 0; c < kColumns; ++c)
+        if (c == 0 || step == 0)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[(wave * kRows + lgrp * 4 + e) * kPitch + c * 16 + lrow] = acc[c][e];
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(missing) != 0) {  // set in front of the barrier: the same for all
+      __syncthreads();
+      if (tid == 0) missing = 0;
+      if (!solo && step > 0) {
+        solo = true;
+        resume_step = step, resume_item = item;
+        step = 0, item = 0;
+      } else if (++tries > kChainMostTries) {  // (not reached: what an item reads this workgroup has written)
+        if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
+        return;
+      }
+      __syncthreads();
+      continue;
+    }
+    if (stores) {
+      const floatx2 v = sum_parts(part, row, column - n0, 1);
+      float v0 = v[0] + low<T>(bias), v1 = v[1] + high<T>(bias);
+      if (step == STEPS - 1) {
+        *reinterpret_cast<uint32_t*>(static_cast<T*>(a.out) + row * H + column) = pack2<T>(v0 + low<T>(residual), v1 + high<T>(residual));
+      } else if constexpr (BLOCK == kFeedForward) {
+        store1(fragment_offset(row, column), pack2<T>(fmaxf(v0, 0.f), fmaxf(v1, 0.f)));
+      } else {
+        store1((uint32_t)(row * a.width + column) * 2, pack2<T>(v0, v1));
+      }
+    } else if (!product) {
+      // the context of the workgroup's heads, two columns a thread
+      const int mine = tid / (kD / 2), pair = item * (kWaves / a.waves) + mine, col = 2 * (tid % (kD / 2));
+      if (mine < kWaves / a.waves && pair < rows * heads) {
+        float v0 = 0.f, v1 = 0.f;
+#pragma unroll 4
+        for (int w = 0; w < 4 * a.waves; ++w) {
+          const floatx2 p = *reinterpret_cast<const floatx2*>(part + (mine * 4 * a.waves + w) * kD + col);
+          v0 += p[0];
+          v1 += p[1];
+        }
+        const int b = pair / heads;
+        store1(context_at(a.width) + fragment_offset(b, (pair - b * heads) * kD + col), pack2<T>(v0, v1));
+      }
+    }
+    tries = 0;
+    if (!solo) {
+      advance(step, item);
+      if (step >= STEPS) {
+        leave();
+        return;
+      }
+    } else if (++item >= items(step)) {
+      item = 0;
+      if (++step == resume_step) item = resume_item, solo = false;
+    }
+    __syncthreads();  // the rows and partial tiles have been read
+  }
+#endif
+}
+
+int64_t part_bytes(Block block, int64_t hidden, int64_t width) { return kRows * 2 * (width + (block == kFeedForward ? 0 : hidden)); }
+
+template <typename T, Block BLOCK, int LOADS>
+int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
+  a.waves = 1;
+  while (BLOCK != kFeedForward && a.waves * 8 * LOADS < a.keys) a.waves *= 2;
+  const int64_t middle = BLOCK == kFeedForward ? 0 : ceil_div((int64_t)a.rows * a.heads * a.waves, kWaves);
+  const int64_t all = a.width / (16 * kColumns) + middle + a.hidden / 16;
+  const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(all, compute_units());
+  const int lds = kRows * chain_row_pitch(a.hidden) + kWaves * kRows * kPitch * 4;
+  auto kernel = decoder_chain_kernel<T, BLOCK, LOADS>;
+  // more than 64 KB of dynamic LDS: the limit is raised once per kernel and device
+  static std::mutex mu;
+  static std::set<int> done;
+  int dev = 0;
+  TTMI_HIP(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (done.count(dev) == 0) {
+      TTMI_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsMost));
+      done.insert(dev);
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, s, a);
+  return launch_status("decoder_chain_kernel");
+}
+
+template <typename T, Block BLOCK>
+int launch(const DecoderArgs& a, int workgroups, hipStream_t s) {
+  // Few keys a wavefront: the sixteen of a workgroup share four SIMDs, and what the attention of 64 keys takes there is more than an exchange.
+  if constexpr (BLOCK != kFeedForward)
+    if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, 8>(a, workgroups, s);
+  return launch_sized<T, BLOCK, 2>(a, workgroups, s);
+}
+
+// Takes the part of the exchange memory whose turn it is.
+int take_part(DecoderArgs& a, void* exchange, int64_t bytes, int turn, hipStream_t s) {
+  TTMI_REQUIRE(turn >= 0 && turn <= 2, "turn is 0, 1 or 2");
+  a.bytes = (uint32_t)bytes;
+  a.exchange = static_cast<char*>(exchange) + turn * bytes;
+  a.other = turn == 2 ? nullptr : static_cast<char*>(exchange) + (1 - turn) * bytes;
+  return turn == 2 ? launch_unwritten(a.exchange, bytes, s) : 0;
+}
+
+bool takes(int64_t rows, int64_t hidden, int dtype) {
+  return (dtype == TTMI_F16 || dtype == TTMI_BF16) && rows >= 1 && rows <= kRows && hidden >= 64 && hidden % 64 == 0 && hidden <= kMostHidden;
+}
+
+}  // namespace
+}  // namespace ttmi
+
+using namespace ttmi;
+
+extern "C" {
+
+int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, int64_t inner, int64_t keys, int dtype, int64_t* bytes) {
+  TTMI_REQUIRE(bytes != nullptr, "null result");
+  *bytes = 0;
+  if (!takes(rows, hidden, dtype)) return 0;
+  if (heads > 0) {
+    if (hidden == heads * kD && keys >= 1 && keys <= kMostKeys && (inner == hidden || inner == 3 * hidden)) *bytes = 3 * part_bytes(kSelfAttention, hidden, inner);
+  } else if (inner >= 64 && inner % 64 == 0 && inner <= kMostInner) {
+    *bytes = 3 * part_bytes(kFeedForward, hidden, inner);
+  }
+  return 0;
+}
+
+int ttmi_decoder_chain_prepare(void* exchange, int64_t bytes, void* stream) {
+  TTMI_REQUIRE(exchange && bytes > 0 && bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(exchange) & 15) == 0, "exchange memory comes in whole, aligned 16 bytes");
+  return launch_unwritten(exchange, bytes, (hipStream_t)stream);
+}
+
+int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta, float eps, const void* w1, const void* b1, const void* w2, const void* b2,
+                              void* out, void* exchange, int turn, int64_t rows, int64_t hidden, int64_t inner, int dtype, int workgroups, int patience,
+                              void* stream) {
+  TTMI_REQUIRE(x && gamma && beta && w1 && b1 && w2 && b2 && out && exchange, "null tensor");
+  int64_t bytes = 0;
+  const int rc = ttmi_decoder_chain_workspace(rows, 0, hidden, inner, 0, dtype, &bytes);
+  if (rc != 0) return rc;
+  TTMI_REQUIRE(bytes > 0 && workgroups >= 0 && patience >= 0, "this block is not run as one launch");
+  uintptr_t bits = 0;
+  for (const void* p : {x, gamma, beta, w1, b1, w2, b2, (const void*)out, (const void*)exchange}) bits |= reinterpret_cast<uintptr_t>(p);
+  TTMI_REQUIRE((bits & 15) == 0 && x != out, "tensors must be 16-byte aligned, and out another one than x");
+  DecoderArgs a{};
+  a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w1, a.b_in = b1, a.w_out = w2, a.b_out = b2, a.out = out;
+  a.rows = (int)rows, a.hidden = (int)hidden, a.width = (int)inner, a.inner = (int)inner, a.eps = eps, a.heads = 1;
+  a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
+  const int part = take_part(a, exchange, bytes / 3, turn, (hipStream_t)stream);
+  if (part != 0) return part;
+  return dtype == TTMI_F16 ? launch<f16, kFeedForward>(a, workgroups, (hipStream_t)stream) : launch<bf16, kFeedForward>(a, workgroups, (hipStream_t)stream);
+}
+
+int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, float eps, const void* w_in, const void* b_in, const void* w_out,
+                           const void* b_out, const void* k_past, const void* v_past, void* k_out, void* v_out, const float* mask, void* probs, void* out,
+                           void* exchange, int turn, int64_t rows, int64_t heads, int64_t hidden, int64_t keys, float scale, int dtype, int workgroups,
+                           int patience, void* stream) {
+  TTMI_REQUIRE(x && gamma && beta && w_in && b_in && w_out && b_out && k_past && v_past && probs && out && exchange, "null tensor");
+  TTMI_REQUIRE((k_out == nullptr) == (v_out == nullptr), "the grown cache is both tensors or none");
+  const bool grows = k_out != nullptr;
+  const int64_t width = grows ? 3 * hidden : hidden, past = grows ? keys - 1 : keys;
+  int64_t bytes = 0;
+  const int rc = ttmi_decoder_chain_workspace(rows, heads, hidden, width, keys, dtype, &bytes);
+  if (rc != 0) return rc;
+  TTMI_REQUIRE(heads > 0 && bytes > 0 && past > 0 && workgroups >= 0 && patience >= 0, "this attention is not run as one launch");
+  uintptr_t bits = 0;
+  for (const void* p : {x, gamma, beta, w_in, b_in, w_out, b_out, k_past, v_past, (const void*)k_out, (const void*)v_out, (const void*)out, (const void*)exchange})
+    bits |= reinterpret_cast<uintptr_t>(p);
+  TTMI_REQUIRE((bits & 15) == 0 && x != out, "tensors must be 16-byte aligned, and out another one than x");
+  DecoderArgs a{};
+  a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w_in, a.b_in = b_in, a.w_out = w_out, a.b_out = b_out, a.out = out;
+  a.k_past = k_past, a.v_past = v_past, a.k_out = k_out, a.v_out = v_out, a.mask = mask, a.probs = probs;
+  a.rows = (int)rows, a.heads = (int)heads, a.hidden = (int)hidden, a.width = (int)width, a.inner = (int)hidden, a.eps = eps, a.scale = scale;
+  a.past = (int)past, a.keys = (int)keys;
+  a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
+  const int part = take_part(a, exchange, bytes / 3, turn, (hipStream_t)stream);
+  if (part != 0) return part;
+  if (grows) return dtype == TTMI_F16 ? launch<f16, kSelfAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kSelfAttention>(a, workgroups, (hipStream_t)stream);
+  return dtype == TTMI_F16 ? launch<f16, kMemoryAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kMemoryAttention>(a, workgroups, (hipStream_t)stream);
+}
+
+}  // extern "C"

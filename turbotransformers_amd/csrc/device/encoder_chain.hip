@@ -2,10 +2,7 @@
 //
 // With a handful of rows a layer is six dependent launches of 3.7 to 5.3 us each, of which nothing but the change from one to the next
 // is long: launch, first operands, drain.  Here workgroups of sixteen wavefronts stay, and what one step of the chain leaves for the next goes
-// through memory, past the L2s (an exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same
-// reads and writes 2.9, a barrier over the grid with counters 4 to 5).  Nobody waits at a barrier of the grid: the exchange
-// memory is filled with a word that no result has (kUnwritten: a NaN that every store here replaces by another NaN) and a reader asks
-// again until it has words of another value.  The weights and parameters of an item are requested in front of its rows and arrive while it waits for them.
+// through memory (chain.h).  The weights and parameters of an item are requested in front of its rows and arrive while it waits for them.
 //
 // Steps of a layer, and items (16 or 32 columns each) of a step:
 //   0  LayerNorm of the previous layer's rows, QKV product                     3H/32 items
@@ -28,21 +25,14 @@
 #include <mutex>
 #include <set>
 
-#include "attention_common.h"
+#include "chain.h"
 
 namespace ttmi {
 namespace {
 
-constexpr int kWaves = 16, kThreads = kWaves * kWave;
-constexpr int kRows = 16;                         // of a block of the matrix instruction: as many as a call may have
-constexpr int kColumns = 2;                       // blocks of 16 columns of an item of steps 0 and 2
-constexpr int kPitch = kColumns * 16 + 4;         // words of a row of a partial tile
-constexpr uint32_t kUnwritten = 0xffffffffu, kOtherNaN = 0xfffefffeu;
-constexpr int kThroughMemory = 17;                // cache policy sc0 | sc1: not from, and not into, the L2 of the XCD
+constexpr int kWaves = kChainWaves, kThreads = kChainThreads, kRows = kChainRows, kColumns = kChainColumns, kPitch = kChainPitch;
 constexpr int kMostLayers = 24;
-constexpr int kMostTries = 4096;
 constexpr int kLdsMost = 80 * 1024;
-constexpr uint32_t kOutside = 0xffffff00u;        // an offset past every buffer: a load from there is zero
 
 struct ChainLayer {
   const void *qkv_w, *qkv_b, *out_w, *out_b, *gamma1, *beta1, *ffn1_w, *ffn1_b, *ffn2_w, *ffn2_b, *gamma2, *beta2;
@@ -74,35 +64,16 @@ inline Places places(int rows, int hidden, int ffn, int residual_size) {
   p.vt = p.qk + 2 * h * kRows * 2;                           // V: [H, kRows]
   p.x0 = p.vt + h * kRows * 2;                               // [H / 16, rows, 16] of the residual's type
   p.sum1 = p.x0 + up256(r * h * (uint32_t)residual_size);    // [rows, H] fp32
-  p.mid = p.sum1 + up256(r * h * 4);                         // [F / 64, 2, 4, kRows, 8], see mid_offset
+  p.mid = p.sum1 + up256(r * h * 4);                         // [F / 64, 2, 4, kRows, 8], see fragment_offset
   p.x1 = p.mid + (uint32_t)ffn * kRows * 2;
   p.sum2 = p.x1 + up256(r * h * (uint32_t)residual_size);
   p.end = p.sum2 + up256(r * h * 4);
   return p;
 }
 
-__device__ __forceinline__ uint32_t storable(uint32_t word) { return word == kUnwritten ? kOtherNaN : word; }
-// The largest word so far: kUnwritten if one of them is.
-__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x4& x) { return max(max(max(m, x[0]), max(x[1], x[2])), x[3]); }
-__device__ __forceinline__ uint32_t largest(uint32_t m, const u32x2& x) { return max(max(m, x[0]), x[1]); }
-
-template <typename T>
-__device__ __forceinline__ floatx4 mma16(const u32x4& a, const u32x4& b, floatx4 c) {
-  if constexpr (std::is_same<T, f16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-template <typename T>
-__device__ __forceinline__ float low(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair & 0xffffu)); }
-template <typename T>
-__device__ __forceinline__ float high(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair >> 16)); }
-
-// Q, K, V and the rows of FFN2 lie as the wavefronts that read them hold them in registers, a load of one 64 consecutive pieces: what goes past
-// the L2 is paid by the line and the load.  In bytes, of an even column (a pair of rows of V):
+// Q, K and V lie as the wavefronts that read them hold them in registers (as fragment_offset does).  In bytes, of an even column (a pair of rows of V):
 __device__ __forceinline__ uint32_t q_offset(int row, int col) { return (uint32_t)(((col >> 3) * kRows + row) * 8 + (col & 7)) * 2; }
 __device__ __forceinline__ uint32_t v_offset(int row, int col) { return (uint32_t)(col * kRows + row) * 2; }
-__device__ __forceinline__ uint32_t mid_offset(int row, int col) {
-  return (uint32_t)(((((col >> 6) * 2 + ((col >> 3) & 1)) * 4 + ((col >> 4) & 3)) * kRows + row) * 8 + (col & 7)) * 2;
-}
 
 // Whether one of the values is an infinity or a NaN.
 template <typename T, typename Words>
@@ -119,10 +90,9 @@ __device__ __forceinline__ uint32_t keys_within(uint32_t pair, int key, int from
 }
 
 // LDS: rows of the A operand (or, in step 1, the heads' contexts), then the partial tiles.
-__host__ __device__ inline int row_pitch(int hidden) { return hidden * 2 + 16; }  // bytes; four banks further per row
 constexpr int kContextPitch = (kD + 8) * 2;
 __host__ __device__ inline int rows_bytes(int hidden) {
-  const int rows = kRows * row_pitch(hidden), contexts = kWaves * kRows * kContextPitch;
+  const int rows = kRows * chain_row_pitch(hidden), contexts = kWaves * kRows * kContextPitch;
   return rows > contexts ? rows : contexts;
 }
 __host__ __device__ inline int lds_bytes(int hidden) { return rows_bytes(hidden) + kWaves * kRows * kPitch * 4; }
@@ -185,7 +155,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     const Arguments& a = *arguments();
     const auto& at = a.at;
     const int H = a.hidden, F = a.ffn, rows = a.rows, patience = a.patience;
-    const int pitch = row_pitch(H);
+    const int pitch = chain_row_pitch(H);
     float* const part = reinterpret_cast<float*>(smem + rows_bytes(H));
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
@@ -278,30 +248,16 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
         if (late) {
           missing = 1;
         } else if (wave < rows) {
-          float sum = 0.f, sumsq = 0.f;
+          float x[TURNS][4], normed[TURNS][4];
 #pragma unroll
           for (int t = 0; t < TURNS; ++t)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float x = __builtin_bit_cast(float, (uint32_t)raw[t][e]);
-              sum += x;
-              sumsq += x * x;
-            }
-          sum = group_sum<kWave>(sum);
-          sumsq = group_sum<kWave>(sumsq);
-          const float mean = sum / (float)H;
-          const float var = fmaxf(sumsq / (float)H - mean * mean, 0.f);  // as in layer_norm_rows
-          const float rstd = 1.0f / sqrtf(var + a.eps);
+            for (int e = 0; e < 4; ++e) x[t][e] = __builtin_bit_cast(float, (uint32_t)raw[t][e]);
+          normalise_row<T, TURNS>(x, gm, bt, H, a.eps, normed);
 #pragma unroll
           for (int t = 0; t < TURNS; ++t) {
             const int col = t * 256 + lane * 4;
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float b = e & 1 ? high<T>(bt[t][e >> 1]) : low<T>(bt[t][e >> 1]), g = e & 1 ? high<T>(gm[t][e >> 1]) : low<T>(gm[t][e >> 1]);
-              v[e] = b + g * rstd * (__builtin_bit_cast(float, (uint32_t)raw[t][e]) - mean);
-              asm volatile("" : "+v"(v[e]));  // rounded once, from fp32
-            }
+            const float (&v)[4] = normed[t];
             const u32x2 r = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
             if (col >= H) continue;
             if (step == last_step) {
@@ -423,7 +379,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
       } else {
         const int share = (F / 64 + kWaves - 1) / kWaves, first = wave * share, mine = min(F / 64 - first, share);
         const int there = lrow < rows ? mine : 0;
-        const uint32_t row_at = base + at.mid + mid_offset(lrow, first * 64 + lgrp * 16);
+        const uint32_t row_at = base + at.mid + fragment_offset(lrow, first * 64 + lgrp * 16);
         u32x4 wf[2 * PIECES], af[2 * PIECES];
 #pragma unroll
         for (int p = 0; p < 2 * PIECES; ++p)
@@ -467,7 +423,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
         solo = true;
         resume_step = step, resume_item = item;
         step = seen, item = 0;
-      } else if (++tries > kMostTries) {  // (not reached: what an item reads has been written, or is being written by a workgroup that runs)
+      } else if (++tries > kChainMostTries) {  // (not reached: what an item reads has been written, or is being written by a workgroup that runs)
         if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
         return;
       }
@@ -476,32 +432,20 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     }
 
     if (stores) {
-      float v0 = 0.f, v1 = 0.f;
       if (transposed) {  // V: two rows of a column
         const int r = 2 * (at_tid >> 4);
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-          v0 += part[(w * kRows + r) * kPitch + block * 16 + lrow];
-          v1 += part[(w * kRows + r + 1) * kPitch + block * 16 + lrow];
-        }
+        const floatx2 v = sum_parts(part, r, block * 16 + lrow, kPitch);
         const float b = low<T>(bias);
-        v0 = r < rows ? v0 + b : 0.f;
-        v1 = r + 1 < rows ? v1 + b : 0.f;
+        const float v0 = r < rows ? v[0] + b : 0.f, v1 = r + 1 < rows ? v[1] + b : 0.f;
         store1(base + at.vt + v_offset(r, n0 - 2 * H + block * 16 + lrow), pack2<T>(v0, v1));
       } else if (pairs_here) {
         const int r = at_tid >> 3, c = block * 16 + 2 * (tid & 7);
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) {
-          const floatx2 p = *reinterpret_cast<const floatx2*>(part + (w * kRows + r) * kPitch + c);
-          v0 += p[0];
-          v1 += p[1];
-        }
-        v0 += low<T>(bias);
-        v1 += high<T>(bias);
+        const floatx2 v = sum_parts(part, r, c, 1);
+        const float v0 = v[0] + low<T>(bias), v1 = v[1] + high<T>(bias);
         if (ph == 0) {
           store1(base + at.qk + q_offset(r, n0 + c), pack2<T>(v0, v1));
         } else if (ph == 2) {
-          store1(base + at.mid + mid_offset(r, n0 + c), pack2<T>(gelu_tanh(v0), gelu_tanh(v1)));
+          store1(base + at.mid + fragment_offset(r, n0 + c), pack2<T>(gelu_tanh(v0), gelu_tanh(v1)));
         } else {
           const uint32_t to = base + (ph == 1 ? at.sum1 : at.sum2) + (uint32_t)(r * H + n0 + c) * 4;
           store1(to, __builtin_bit_cast(uint32_t, v0 + res0));
@@ -521,11 +465,6 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     __syncthreads();  // the rows and partial tiles have been read
   }
 #endif
-}
-
-__global__ void unwritten_kernel(u32x4* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
 }
 
 int64_t workspace_bytes(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype) {
@@ -572,11 +511,11 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
   a.layer_bytes = (uint32_t)(bytes / layers);
   a.at = places((int)rows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2);
   a.layers = (int)layers, a.rows = (int)rows, a.seq = (int)seq, a.heads = (int)heads, a.hidden = (int)hidden, a.ffn = (int)ffn;
-  a.patience = patience > 0 ? patience : 512;
+  a.patience = patience > 0 ? patience : kChainPatience;
   a.eps = eps, a.scale_log2e = 0.125f * 1.4426950408889634f, a.inv_scale = 8.0f, a.error = async_error_flag();
   hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * cus)), dim3(256), 0, s, static_cast<u32x4*>(workspace),
-                     bytes / 16);
+  const int rc = launch_unwritten(workspace, bytes, s);
+  if (rc != 0) return rc;
   const int64_t widest = std::max(3 * hidden, ffn) / (16 * kColumns) + hidden / 16;
   const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(widest, cus);
   const int lds = lds_bytes((int)hidden);

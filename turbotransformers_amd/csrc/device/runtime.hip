@@ -223,12 +223,20 @@ int ttmi_event_elapsed_ms(void* start, void* stop, float* ms) {
   return 0;
 }
 
+int ttmi_stream_capturing(void* stream, int* capturing) {
+  TTMI_REQUIRE(capturing != nullptr, "null result");
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) != hipSuccess) (void)hipGetLastError();  // (the null stream while another one captures)
+  *capturing = status == hipStreamCaptureStatusActive ? 1 : 0;
+  return 0;
+}
+
 int ttmi_check_async(void) {
   int* flag = async_error_flag();
   if (flag && *flag != 0) {
     const int what = *flag;
     *flag = 0;
-    if (what == kRowsNeverCame) return fail(TTMI_EDEVICE, "encoder chain: rows that it waited for never came");
+    if (what == kRowsNeverCame) return fail(TTMI_EDEVICE, "rows that a chain of steps waited for never came");
     return fail(TTMI_EINDEX, "embedding id out of range");
   }
   return 0;

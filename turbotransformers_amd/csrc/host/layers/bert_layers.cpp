@@ -155,8 +155,35 @@ static void CheckFfn(const Tensor& input, const Tensor& w1, const Tensor& b1, co
   TT_ENFORCE(core::SameDataType(input.dtype(), w1.dtype()), "input and weights must share one element type");
 }
 
+// A token each of a few sequences (ttmi_decoder_feed_forward); false: nothing was done.
+bool PositionwiseFeedForward::AsOneLaunch(const Tensor& input_tensor, Tensor* output, bool is_trans_weight) const {
+  const int64_t rows = input_tensor.shape(0) * input_tensor.shape(1), model_dim = input_tensor.shape(2);
+  const int dt = kernels::DeviceDType(input_tensor);
+  if (dt == TTMI_F32 || rows > TTMI_CHAIN_MAX_ROWS) return false;
+  const int64_t d_ff = PackedWeight::OutDim(dense_weight_1_, is_trans_weight);
+  int64_t bytes = 0;
+  TT_DEVICE_CALL(ttmi_decoder_chain_workspace(rows, 0, model_dim, d_ff, 0, dt, &bytes));
+  if (bytes == 0 || layer_norm_weight_.numel() != model_dim || layer_norm_bias_.numel() != model_dim) return false;
+  const void* w1 = packed1_.Get(dense_weight_1_, is_trans_weight).data;
+  const void* w2 = packed2_.Get(dense_weight_2_, is_trans_weight).data;
+  const DLDeviceType dev = input_tensor.device_type();
+  const int id = input_tensor.device_id();
+  output->ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/Reshape");
+  void* const out = output->mutable_raw();
+  uintptr_t bits = reinterpret_cast<uintptr_t>(out);
+  for (const void* p : {input_tensor.raw(), layer_norm_weight_.raw(), layer_norm_bias_.raw(), w1, dense_bias_1_.raw(), w2, dense_bias_2_.raw()})
+    bits |= reinterpret_cast<uintptr_t>(p);
+  if ((bits & 15) != 0 || out == input_tensor.raw()) return false;
+  exchange_.Use(bytes, dev, id, [&](void* memory, int turn) {
+    TT_DEVICE_CALL(ttmi_decoder_feed_forward(input_tensor.raw(), layer_norm_weight_.raw(), layer_norm_bias_.raw(), 1e-12f, w1, dense_bias_1_.raw(), w2,
+                                             dense_bias_2_.raw(), out, memory, turn, rows, model_dim, d_ff, dt, 0, 0, Stream()));
+  });
+  return true;
+}
+
 void PositionwiseFeedForward::operator()(const Tensor& input_tensor, Tensor* output, bool is_trans_weight) const {
   CheckFfn(input_tensor, dense_weight_1_, dense_bias_1_, dense_weight_2_, dense_bias_2_, is_trans_weight, "PositionwiseFeedForward");
+  if (AsOneLaunch(input_tensor, output, is_trans_weight)) return;
   const int64_t model_dim = input_tensor.shape(2), d_ff = PackedWeight::OutDim(dense_weight_1_, is_trans_weight);
   const int64_t m = input_tensor.numel() / model_dim;
   const DLDeviceType dev = input_tensor.device_type();

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "core/tensor.h"
+#include "layers/exchange_memory.h"
 #include "layers/kernels.h"
 #include "layers/packed_weight.h"
 
@@ -116,9 +117,11 @@ class PositionwiseFeedForward {
   void operator()(const core::Tensor& input_tensor, core::Tensor* output, bool is_trans_weight = false) const;
 
  private:
+  bool AsOneLaunch(const core::Tensor& input_tensor, core::Tensor* output, bool is_trans_weight) const;
   core::Tensor dense_weight_1_, dense_bias_1_, dense_weight_2_, dense_bias_2_, layer_norm_weight_, layer_norm_bias_;
   PackedWeight packed1_, packed2_;
   mutable core::Tensor normed_, hidden_;
+  mutable ExchangeMemory exchange_;
 };
 
 class DistrillFFN {

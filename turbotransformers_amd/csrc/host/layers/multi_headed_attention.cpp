@@ -218,6 +218,58 @@ static void StoreInCache(std::unordered_map<std::string, Tensor*>& cache, const 
                   (size_t)src.numel() * src.element_size());
 }
 
+bool MultiHeadedAttention::AsOneLaunch(const Tensor& query_tensor, const Tensor& attention_mask, bool is_self, Tensor* output, Tensor* att_score,
+                                       const std::unordered_map<std::string, Tensor*>& layer_cache, bool is_trans_weight) const {
+  const int dt = kernels::DeviceDType(query_tensor);
+  if (dt == TTMI_F32 || query_tensor.shape(0) > TTMI_CHAIN_MAX_ROWS || query_tensor.shape(1) != 1 || att_score == nullptr) return false;
+  const char *key_name = is_self ? "self_keys" : "memory_keys", *value_name = is_self ? "self_values" : "memory_values";
+  if (!CacheHas(layer_cache, key_name) || !CacheHas(layer_cache, value_name)) return false;
+  const Tensor &k_past = *layer_cache.at(key_name), &v_past = *layer_cache.at(value_name);
+  const int64_t batch = query_tensor.shape(0), hidden = query_tensor.shape(2), heads = num_attention_heads_, past = k_past.shape(2);
+  const int64_t keys = is_self ? past + 1 : past, width = is_self ? 3 * hidden : hidden;
+  if (past < 1 || v_past.shape(2) != past || layernorm_gamma_.numel() != hidden || layernorm_beta_.numel() != hidden) return false;
+  int64_t bytes = 0;
+  TT_DEVICE_CALL(ttmi_decoder_chain_workspace(batch, heads, hidden, width, keys, dt, &bytes));
+  if (bytes == 0) return false;
+  const float* mask = nullptr;
+  if (!attention_mask.is_null()) {
+    if (attention_mask.numel() != batch * keys) return false;
+    mask = attention_mask.data<float>();
+  }
+  if (is_self) MultiHeadedAttention::EnforceShapeAndType();
+  for (const Tensor* t : {&q_weight_, &k_weight_, &v_weight_, &q_bias_, &k_bias_, &v_bias_})
+    if (!is_self && t->is_null()) return false;
+  const Tensor &in_weight = is_self ? qkv_weight_ : q_weight_, &in_bias = is_self ? qkv_bias_ : q_bias_;
+  if (in_weight.numel() != width * hidden || in_bias.numel() != width) return false;
+  const void* w_in = (is_self ? qkv_packed_ : q_packed_).Get(in_weight, is_trans_weight).data;
+  const void* w_out = dense_packed_.Get(dense_weight_, is_trans_weight).data;
+  const DLDeviceType dev = query_tensor.device_type();
+  const int dev_id = query_tensor.device_id();
+  uintptr_t bits = 0;
+  for (const void* p : {query_tensor.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw(), w_in, in_bias.raw(), w_out, dense_bias_.raw(), k_past.raw(), v_past.raw()})
+    bits |= reinterpret_cast<uintptr_t>(p);
+  output->ReshapeAs(query_tensor.dtype(), {batch, 1, hidden}, dev, dev_id, "gemm5/Reshape");
+  void* const out = output->mutable_raw();
+  if (((bits | reinterpret_cast<uintptr_t>(out)) & 15) != 0 || out == query_tensor.raw()) return false;
+  att_score->ReshapeAs(query_tensor.dtype(), {batch, heads, 1, keys}, dev, dev_id, "batch_gemm3/Reshape");
+  Tensor k_grown(nullptr), v_grown(nullptr);
+  if (is_self) {
+    k_grown.ReshapeAs(query_tensor.dtype(), {batch, heads, keys, hidden / heads}, dev, dev_id, "self/self_key/Reshape");
+    v_grown.ReshapeAs(query_tensor.dtype(), {batch, heads, keys, hidden / heads}, dev, dev_id, "self/self_value/Reshape");
+  }
+  exchange_.Use(bytes, dev, dev_id, [&](void* memory, int turn) {
+    TT_DEVICE_CALL(ttmi_decoder_attention(query_tensor.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw(), 1e-6f, w_in, in_bias.raw(), w_out,
+                                          dense_bias_.raw(), k_past.raw(), v_past.raw(), is_self ? k_grown.mutable_raw() : nullptr,
+                                          is_self ? v_grown.mutable_raw() : nullptr, mask, att_score->mutable_raw(), out, memory, turn, batch, heads, hidden,
+                                          keys, 1.0f / std::sqrt(static_cast<float>(hidden / heads)), dt, 0, 0, Stream()));
+  });
+  if (is_self) {
+    *layer_cache.at(key_name) = std::move(k_grown);
+    *layer_cache.at(value_name) = std::move(v_grown);
+  }
+  return true;
+}
+
 void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value_tensor, const Tensor& query_tensor,
                                    const Tensor& attention_mask, const std::string& attn_type, Tensor* output,
                                    Tensor* att_score, std::unordered_map<std::string, Tensor*> layer_cache,
@@ -250,6 +302,7 @@ void MultiHeadedAttention::Forward(const Tensor& key_tensor, const Tensor& value
   }
 
   if (pre_layernorm) TT_ENFORCE(!layernorm_gamma_.is_null() && !layernorm_beta_.is_null(), "pre_layernorm needs LayerNorm parameters");
+  if (pre_layernorm && post_add_input && AsOneLaunch(query_tensor, attention_mask, is_self, output, att_score, layer_cache, is_trans_weight)) return;
   // a projection of the query, with LayerNorm in front where asked for (:66-80, :190-199 -- eps is 1e-6 there)
   auto project_query = [&](const WeightRef& packed_w, int64_t n, const ttmi_epilogue_args& args) {
     if (pre_layernorm) {

@@ -26,6 +26,7 @@
 
 #include "core/tensor.h"
 #include "layers/bert_layers.h"
+#include "layers/exchange_memory.h"
 #include "layers/packed_weight.h"
 
 namespace turbo_transformers {
@@ -101,6 +102,11 @@ class MultiHeadedAttention {
   // The one-kernel core that also returns the probabilities (head size 64, up to TTMI_PROBS_MAX_KEYS keys).
   bool UseProbsCore(int64_t head_dim, int64_t keys, std::initializer_list<const core::Tensor*> tensors) const;
 
+  // The whole call as one launch (ttmi_decoder_attention): a token each of a few sequences, over a growing cache or a projected memory, with
+  // LayerNorm in front and the input added behind; false: nothing was done.
+  bool AsOneLaunch(const core::Tensor& query_tensor, const core::Tensor& attention_mask, bool is_self, core::Tensor* output, core::Tensor* att_score,
+                   const std::unordered_map<std::string, core::Tensor*>& layer_cache, bool is_trans_weight) const;
+
   // Attention core and output projection as one launch, the heads' parts of it added up by the LayerNorm behind.
   bool UseProjectingCore(const core::Tensor& query_tensor, const WeightRef& wo, int64_t batch, int64_t seq, int64_t v_pitch, int dtype) const;
 
@@ -121,6 +127,7 @@ class MultiHeadedAttention {
 
   PackedWeight qkv_packed_, dense_packed_, q_packed_, k_packed_, v_packed_, kv_packed_;
   mutable Scratch scratch_;
+  mutable ExchangeMemory exchange_;
   mutable std::mutex mutex_;  // the layer keeps per-call state, like the reference (…attention.cpp:32,272)
 };
 
