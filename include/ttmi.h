@@ -524,13 +524,15 @@ TTMI_API int ttmi_gemm_i8_dequant_qkv_split(const int8_t* a, const int8_t* b, co
 TTMI_API int ttmi_dequant_bias(const int32_t* acc, const float* act_scale_dev, const float* w_scale,
                                const float* bias, float* out, int64_t m, int64_t n, void* stream);
 
-/* ttmi_encoder_chain: a stack of post-LayerNorm encoder layers over a few rows as one launch (plus one that prepares the workspace), fp16 or
+/* ttmi_encoder_chain: a stack of post-LayerNorm encoder layers over a few rows as one launch, fp16 or
  *   bf16: per layer out = LN(x + attention(x) ...), LN(... + gelu(x w1 + b1) w2 + b2), as the layers' own launches compute it.
  *   weights    HOST list of 12 device pointers per layer: qkv weight [3H,H] and bias, output weight [H,H] and bias, LayerNorm gamma and beta,
  *              FFN1 weight [F,H] and bias, FFN2 weight [H,F] and bias, LayerNorm gamma and beta (all weights [out,in])
  *   input      [batch,seq,H]; input32: the same before rounding (bf16: the residual is taken from it), or null
  *   mask       additive fp32 [batch,seq] per key, or null;  out [batch,seq,H];  out32: bf16, the unrounded result, or null
- *   workspace  as many bytes as ttmi_encoder_chain_workspace says, of device memory, 16-byte aligned; nothing in it outlives the call
+ *   exchange   as many bytes as ttmi_encoder_chain_workspace says, 16-byte aligned, prepared once by ttmi_chain_prepare and used by one call
+ *              after the other on one stream
+ *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed
  *   workgroups, patience: 0, or (tests) how many workgroups are launched and how often one asks for rows that are not there yet
  *              before it computes them itself; neither changes a bit of the result
  * ttmi_encoder_chain_workspace says 0 for what is not built: other types, more than 24 layers, more than 16 rows (batch * seq), head
@@ -538,8 +540,9 @@ TTMI_API int ttmi_dequant_bias(const int32_t* acc, const float* act_scale_dev, c
  * No counterpart in the reference. */
 TTMI_API int ttmi_encoder_chain_workspace(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype,
                                           int64_t* bytes);
+TTMI_API int ttmi_chain_prepare(void* exchange, int64_t bytes, void* stream);
 TTMI_API int ttmi_encoder_chain(const void* const* weights, const void* input, const float* input32, const float* mask, void* out,
-                                float* out32, void* workspace, int64_t layers, int64_t batch, int64_t seq, int64_t heads,
+                                float* out32, void* exchange, int turn, int64_t layers, int64_t batch, int64_t seq, int64_t heads,
                                 int64_t hidden, int64_t ffn, float eps, int dtype, int workgroups, int patience, void* stream);
 
 #define TTMI_CHAIN_MAX_ROWS 16
@@ -552,12 +555,11 @@ TTMI_API int ttmi_encoder_chain(const void* const* weights, const void* input, c
  * ttmi_decoder_feed_forward  out = x + relu(LN(x) w1^T + b1) w2^T + b2; inner a multiple of 64 up to 4096.
  *   weights [out,in]; out must be another tensor than x
  *   exchange   as many bytes as ttmi_decoder_chain_workspace says (heads = 0: feed-forward; inner: 3 * hidden or hidden for attention; 0: not
- *              built), prepared once by ttmi_decoder_chain_prepare and used by one call after the other on one stream
+ *              built), prepared once by ttmi_chain_prepare and used by one call after the other on one stream
  *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed
  *   workgroups, patience: as in ttmi_encoder_chain
  * No counterpart in the reference. */
 TTMI_API int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, int64_t inner, int64_t keys, int dtype, int64_t* bytes);
-TTMI_API int ttmi_decoder_chain_prepare(void* exchange, int64_t bytes, void* stream);
 TTMI_API int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, float eps, const void* w_in, const void* b_in,
                                     const void* w_out, const void* b_out, const void* k_past, const void* v_past, void* k_out, void* v_out,
                                     const float* mask, void* probs, void* out, void* exchange, int turn, int64_t rows, int64_t heads,

@@ -21,7 +21,7 @@ class Exchange:
         ok(ttmi.ttmi_decoder_chain_workspace(rows, heads, hidden, inner, keys, TTMI_DTYPES[dt], ctypes.addressof(size)))
         assert size.value > 0
         self.memory = torch.zeros(size.value, dtype=torch.uint8, device="cuda")
-        ok(ttmi.ttmi_decoder_chain_prepare(ptr(self.memory), size.value, stream()))
+        ok(ttmi.ttmi_chain_prepare(ptr(self.memory), size.value, stream()))
         self.turn = 0
 
     def next(self):

@@ -21,7 +21,7 @@ class Stack:
         self.dt, self.layers, self.heads, self.hidden, self.ffn = dt, layers, heads, heads * 64, ffn
         h = self.hidden
         rnd = lambda *shape: torch.randn(shape, generator=gen)
-        self.weights = []
+        self.weights, self.space, self.turn = [], None, 1
         for _ in range(layers):
             w = [rnd(3 * h, h) / h ** 0.5, rnd(3 * h) * 0.1, rnd(h, h) / h ** 0.5, rnd(h) * 0.1, 1 + rnd(h) * 0.1, rnd(h) * 0.1,
                  rnd(ffn, h) / h ** 0.5, rnd(ffn) * 0.1, rnd(h, ffn) / ffn ** 0.5, rnd(h) * 0.1, 1 + rnd(h) * 0.1, rnd(h) * 0.1]
@@ -30,15 +30,23 @@ class Stack:
     def input(self, batch, seq, seed):
         return torch.randn((batch, seq, self.hidden), generator=torch.Generator().manual_seed(seed)).to(TORCH_DTYPES[self.dt]).cuda()
 
+    def exchange(self, ttmi):
+        """The memory of calls of any number of rows, which take turns."""
+        size = ctypes.c_int64()
+        ok(ttmi.ttmi_encoder_chain_workspace(self.layers, 1, self.heads, self.hidden, self.ffn, TTMI_DTYPES[self.dt], ctypes.addressof(size)))
+        assert size.value > 0
+        if self.space is None:
+            self.space = torch.zeros(size.value, dtype=torch.uint8, device="cuda")
+            ok(ttmi.ttmi_chain_prepare(ptr(self.space), size.value, stream()))
+        self.turn = 1 - self.turn
+        return self.space
+
     def run(self, ttmi, x, mask=None, workgroups=0, patience=0):
         batch, seq, h = x.shape
-        size = ctypes.c_int64()
-        ok(ttmi.ttmi_encoder_chain_workspace(self.layers, batch * seq, self.heads, h, self.ffn, TTMI_DTYPES[self.dt], ctypes.addressof(size)))
-        assert size.value > 0
-        out, space = torch.empty_like(x), torch.zeros(size.value, dtype=torch.uint8, device="cuda")
+        space, out = self.exchange(ttmi), torch.empty_like(x)
         out32 = torch.empty(x.shape, device="cuda") if self.dt == "bf16" else None
         pointers = (ctypes.c_void_p * (12 * self.layers))(*[w.data_ptr() for l in self.weights for w in l])
-        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(x), None, ptr(mask), ptr(out), ptr(out32), ptr(space), self.layers, batch, seq,
+        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(x), None, ptr(mask), ptr(out), ptr(out32), ptr(space), self.turn, self.layers, batch, seq,
                                    self.heads, h, self.ffn, 1e-12, TTMI_DTYPES[self.dt], workgroups, patience, stream()))
         torch.cuda.synchronize()
         if out32 is not None:
@@ -113,23 +121,22 @@ def test_what_is_not_finite_stays_in_its_sequence(ttmi, batch, seq):
 
 
 def test_replayed_from_a_graph(ttmi):
-    """The workspace is prepared on every replay."""
+    """An odd number of calls, and calls of the owner of the exchange memory between the replays."""
     stack = Stack("f16", 2, 12, 3072)
     x, other = stack.input(1, 10, 3), stack.input(1, 10, 4)
     want = [stack.run(ttmi, x), stack.run(ttmi, other)]
-    size = ctypes.c_int64()
-    ok(ttmi.ttmi_encoder_chain_workspace(2, 10, 12, 768, 3072, TTMI_DTYPES["f16"], ctypes.addressof(size)))
-    out, space, given = torch.empty_like(x), torch.empty(size.value, dtype=torch.uint8, device="cuda"), x.clone()
+    out, space, given = torch.empty_like(x), stack.space, x.clone()
     pointers = (ctypes.c_void_p * 24)(*[w.data_ptr() for l in stack.weights for w in l])
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(given), None, None, ptr(out), None, ptr(space), 2, 1, 10, 12, 768, 3072, 1e-12,
+        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(given), None, None, ptr(out), None, ptr(space), 2, 2, 1, 10, 12, 768, 3072, 1e-12,
                                    TTMI_DTYPES["f16"], 0, 0, stream()))
     for turn in range(6):
         given.copy_([x, other][turn % 2])
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want[turn % 2]), turn
+        assert torch.equal(stack.run(ttmi, other), want[1])
 
 
 def test_what_is_not_built_has_no_workspace(ttmi):

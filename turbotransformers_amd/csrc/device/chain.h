@@ -2,6 +2,8 @@
 //
 // What one step leaves for the next goes through memory, past the L2s.  The exchange memory is filled with a word that no result has
 // (kUnwritten: a NaN that every store here replaces by another one), and a reader asks again until it has words of another value.
+// The exchange memory is kept by the caller in two parts that take turns: a launch fills the part that the one before it has used.  Where launches are
+// recorded and replayed, in an order that nobody knows, they use a third part, which is filled in front of each.
 // An exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same reads and writes 2.9, a
 // barrier over the grid with counters 4 to 5.
 #pragma once
@@ -91,6 +93,18 @@ inline int launch_unwritten(void* p, int64_t bytes, hipStream_t s) {
   hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * compute_units())), dim3(256), 0, s, static_cast<u32x4*>(p),
                      bytes / 16);
   return launch_status("unwritten_kernel");
+}
+// The part of a launch, and the one that it fills for the next.
+inline int take_part(void* exchange, int64_t bytes, int turn, char** mine, char** other, hipStream_t s) {
+  TTMI_REQUIRE(turn >= 0 && turn <= 2, "turn is 0, 1 or 2");
+  *mine = static_cast<char*>(exchange) + turn * bytes;
+  *other = turn == 2 ? nullptr : static_cast<char*>(exchange) + (1 - turn) * bytes;
+  return turn == 2 ? launch_unwritten(*mine, bytes, s) : 0;
+}
+// Workgroup `rank` of `count` fills its share.
+__device__ __forceinline__ void fill_unwritten(char* p, uint32_t bytes, int rank, int count) {
+  for (uint32_t at = (uint32_t)(rank * kChainThreads + (int)threadIdx.x) * 16; at < bytes; at += (uint32_t)(count * kChainThreads) * 16)
+    *reinterpret_cast<u32x4*>(p + at) = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
 }
 
 }  // namespace ttmi

@@ -16,9 +16,6 @@
 // 249 / 174, 16 x 41 and 100 248 / 214, 16 x 251 and 256 309 / 262.  What is left of a launch of 9 to 11: its start 0.5, arguments and first operands 1.5 to
 // 2.5, LayerNorm and product 1, an exchange 0.7 to 1.3 each, attention 1 (3.5 with 64 keys a wavefront), its parts' sum and the last product 1.5.
 // Measured and no better: the arguments held in registers (60 of the scalar ones spill) 11.4 / 12.5 a launch.
-//
-// The exchange memory is kept by the caller in two parts that take turns: a launch fills the part that the one before it has used.  Where launches are
-// recorded and replayed, in an order that nobody knows, they use a third part, which is filled in front of each.
 #include <mutex>
 #include <set>
 
@@ -126,9 +123,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
   auto leave = [&]() __attribute__((always_inline)) {
     const Arguments& a = *arguments();
     const int fillers = min(G, items(0));
-    if (a.other != nullptr && me < fillers)
-      for (uint32_t at = (uint32_t)(me * kThreads + (int)threadIdx.x) * 16; at < a.bytes; at += (uint32_t)(fillers * kThreads) * 16)
-        *reinterpret_cast<u32x4*>(a.other + at) = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
+    if (a.other != nullptr && me < fillers) fill_unwritten(a.other, a.bytes, me, fillers);
   };
 
   int step = 0, item = first_item(0) - G;
@@ -422,15 +417,6 @@ int launch(const DecoderArgs& a, int workgroups, hipStream_t s) {
   return launch_sized<T, BLOCK, 2>(a, workgroups, s);
 }
 
-// Takes the part of the exchange memory whose turn it is.
-int take_part(DecoderArgs& a, void* exchange, int64_t bytes, int turn, hipStream_t s) {
-  TTMI_REQUIRE(turn >= 0 && turn <= 2, "turn is 0, 1 or 2");
-  a.bytes = (uint32_t)bytes;
-  a.exchange = static_cast<char*>(exchange) + turn * bytes;
-  a.other = turn == 2 ? nullptr : static_cast<char*>(exchange) + (1 - turn) * bytes;
-  return turn == 2 ? launch_unwritten(a.exchange, bytes, s) : 0;
-}
-
 bool takes(int64_t rows, int64_t hidden, int dtype) {
   return (dtype == TTMI_F16 || dtype == TTMI_BF16) && rows >= 1 && rows <= kRows && hidden >= 64 && hidden % 64 == 0 && hidden <= kMostHidden;
 }
@@ -454,7 +440,7 @@ int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, in
   return 0;
 }
 
-int ttmi_decoder_chain_prepare(void* exchange, int64_t bytes, void* stream) {
+int ttmi_chain_prepare(void* exchange, int64_t bytes, void* stream) {
   TTMI_REQUIRE(exchange && bytes > 0 && bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(exchange) & 15) == 0, "exchange memory comes in whole, aligned 16 bytes");
   return launch_unwritten(exchange, bytes, (hipStream_t)stream);
 }
@@ -474,7 +460,8 @@ int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta
   a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w1, a.b_in = b1, a.w_out = w2, a.b_out = b2, a.out = out;
   a.rows = (int)rows, a.hidden = (int)hidden, a.width = (int)inner, a.inner = (int)inner, a.eps = eps, a.heads = 1;
   a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
-  const int part = take_part(a, exchange, bytes / 3, turn, (hipStream_t)stream);
+  a.bytes = (uint32_t)(bytes / 3);
+  const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
   if (part != 0) return part;
   return dtype == TTMI_F16 ? launch<f16, kFeedForward>(a, workgroups, (hipStream_t)stream) : launch<bf16, kFeedForward>(a, workgroups, (hipStream_t)stream);
 }
@@ -501,7 +488,8 @@ int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, f
   a.rows = (int)rows, a.heads = (int)heads, a.hidden = (int)hidden, a.width = (int)width, a.inner = (int)hidden, a.eps = eps, a.scale = scale;
   a.past = (int)past, a.keys = (int)keys;
   a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
-  const int part = take_part(a, exchange, bytes / 3, turn, (hipStream_t)stream);
+  a.bytes = (uint32_t)(bytes / 3);
+  const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
   if (part != 0) return part;
   if (grows) return dtype == TTMI_F16 ? launch<f16, kSelfAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kSelfAttention>(a, workgroups, (hipStream_t)stream);
   return dtype == TTMI_F16 ? launch<f16, kMemoryAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kMemoryAttention>(a, workgroups, (hipStream_t)stream);

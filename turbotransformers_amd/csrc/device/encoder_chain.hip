@@ -12,8 +12,8 @@
 // and the last LayerNorm.  Rows in front of a LayerNorm travel in fp32; each item normalises all of them for itself (the attention is
 // likewise computed by every item of step 1): a few hundred cycles instead of one more exchange.
 //
-// us per forward, layer by layer / as one launch: fp16 base 1 x 1 token 280 / 158, 1 x 10 305 / 190, 4 x 4 308 / 198; bf16 large 1 x 10
-// 674 / 492, 2 x 8 673 / 506.  What bounds a step of 3.2 to 4 us: the exchange 1.0 to 1.5 (a store to memory, and a load that finds it), the
+// us per forward, layer by layer / as one launch: fp16 base 1 x 1 token 280 / 157, 1 x 8 291 / 176, 4 x 4 308 / 199; bf16 large 1 x 8
+// 661 / 461, 1 x 16 675 / 511 (the exchange memory filled by a launch of its own in front: 160, 179, 201, 464, 515).  What bounds a step of 3.2 to 4 us: the exchange 1.0 to 1.5 (a store to memory, and a load that finds it), the
 // LayerNorm of 16 rows on every CU 0.5 to 1.2 (vector instructions: 16 rows are four a SIMD), the product and the sum over the wavefronts 0.6.
 // Measured and no better: 16 columns an item (240 workgroups instead of 144) level; Q, K, V and the intermediate rows row by row instead
 // of in the order of the registers 10 rows 218 / 183, 16 251 / 194 (the launch alone).
@@ -48,7 +48,7 @@ struct ChainArgs {
   const float* mask;     // [rows], additive, or null
   void* out;
   float* out32;
-  char* exchange;
+  char *exchange, *other;  // the part of this launch, the part to fill, or null
   uint32_t layer_bytes;  // of the exchange memory
   Places at;
   int layers, rows, seq, heads, hidden, ffn, patience;
@@ -135,6 +135,10 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
   };
 
   // The item at hand; while `solo` one of a step that others were to execute, on the way to (resume_step, resume_item).
+  {
+    const Arguments& a = *arguments();
+    if (a.other != nullptr) fill_unwritten(a.other, (uint32_t)a.layers * a.layer_bytes, me, G);
+  }
   int step = 0, item = first_item(0) - G;
   advance(step, item);
   if (step > last_step) return;
@@ -471,7 +475,7 @@ int64_t workspace_bytes(int64_t layers, int64_t rows, int64_t heads, int64_t hid
   const bool takes = (dtype == TTMI_F16 || dtype == TTMI_BF16) && layers >= 1 && layers <= kMostLayers && rows >= 1 && rows <= kRows && heads >= 1 &&
                      heads >= 4 && heads <= kWaves && hidden == heads * kD && ffn >= 256 && ffn % 64 == 0 && ffn <= kWaves * 4 * 64;
   if (!takes) return 0;
-  return layers * (int64_t)places((int)rows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end;
+  return 3 * layers * (int64_t)places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end;  // (of all rows: calls of any number of them take turns)
 }
 
 }  // namespace
@@ -488,15 +492,15 @@ int ttmi_encoder_chain_workspace(int64_t layers, int64_t rows, int64_t heads, in
 }
 
 int ttmi_encoder_chain(const void* const* weights, const void* input, const float* input32, const float* mask, void* out, float* out32,
-                       void* workspace, int64_t layers, int64_t batch, int64_t seq, int64_t heads, int64_t hidden, int64_t ffn, float eps, int dtype,
+                       void* exchange, int turn, int64_t layers, int64_t batch, int64_t seq, int64_t heads, int64_t hidden, int64_t ffn, float eps, int dtype,
                        int workgroups, int patience, void* stream) {
-  TTMI_REQUIRE(weights && input && out && workspace, "null tensor");
+  TTMI_REQUIRE(weights && input && out && exchange, "null tensor");
   TTMI_REQUIRE(batch > 0 && seq > 0 && batch <= kRows && seq <= kRows && workgroups >= 0 && patience >= 0, "bad shape");
   const int64_t rows = batch * seq, bytes = workspace_bytes(layers, rows, heads, hidden, ffn, dtype);
   TTMI_REQUIRE(bytes > 0, "this stack of layers is not run as one launch");
   ChainArgs a{};
   uintptr_t bits = reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(input32) | reinterpret_cast<uintptr_t>(out) |
-                   reinterpret_cast<uintptr_t>(out32) | reinterpret_cast<uintptr_t>(workspace);
+                   reinterpret_cast<uintptr_t>(out32) | reinterpret_cast<uintptr_t>(exchange);
   for (int64_t l = 0; l < layers; ++l) {
     const void* const* w = weights + l * 12;
     for (int i = 0; i < 12; ++i) {
@@ -507,14 +511,14 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
   }
   TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
   const int cus = compute_units();
-  a.input = input, a.input32 = input32, a.mask = mask, a.out = out, a.out32 = out32, a.exchange = static_cast<char*>(workspace);
-  a.layer_bytes = (uint32_t)(bytes / layers);
-  a.at = places((int)rows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2);
+  a.input = input, a.input32 = input32, a.mask = mask, a.out = out, a.out32 = out32;
+  a.layer_bytes = (uint32_t)(bytes / 3 / layers);
+  a.at = places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2);
   a.layers = (int)layers, a.rows = (int)rows, a.seq = (int)seq, a.heads = (int)heads, a.hidden = (int)hidden, a.ffn = (int)ffn;
   a.patience = patience > 0 ? patience : kChainPatience;
   a.eps = eps, a.scale_log2e = 0.125f * 1.4426950408889634f, a.inv_scale = 8.0f, a.error = async_error_flag();
   hipStream_t s = (hipStream_t)stream;
-  const int rc = launch_unwritten(workspace, bytes, s);
+  const int rc = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, s);
   if (rc != 0) return rc;
   const int64_t widest = std::max(3 * hidden, ffn) / (16 * kColumns) + hidden / 16;
   const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(widest, cus);

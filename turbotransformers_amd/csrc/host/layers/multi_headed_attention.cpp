@@ -577,14 +577,14 @@ bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, con
   if ((bits & 15) != 0) return false;
   const DLDeviceType dev = hidden.device_type();
   const int dev_id = hidden.device_id();
-  Tensor workspace(nullptr);
-  float* const space = workspace.Reshape<float>({bytes / 4}, dev, dev_id, "EncoderChain/workspace");
   out->ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
   void* const result = out->mutable_raw();
   float* const result32 = kernels::KeepsFp32Residual(*out) ? out->EnsureShadow()->mutableData<float>() : nullptr;
   if (reinterpret_cast<uintptr_t>(result) % 16 != 0 || result == hidden.raw()) return false;  // (a workgroup that starts late reads the input late)
-  TT_DEVICE_CALL(ttmi_encoder_chain(parameters.data(), hidden.raw(), input32, additive, result, result32, space, count, batch, seq, heads, width,
-                                    ffn, 1e-12f, dt, 0, 0, Stream()));
+  first.exchange().Use(bytes, dev, dev_id, [&](void* memory, int turn) {
+    TT_DEVICE_CALL(ttmi_encoder_chain(parameters.data(), hidden.raw(), input32, additive, result, result32, memory, turn, count, batch, seq, heads, width,
+                                      ffn, 1e-12f, dt, 0, 0, Stream()));
+  });
   return true;
 }
 

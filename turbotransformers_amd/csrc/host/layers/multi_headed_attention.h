@@ -151,6 +151,7 @@ class BertAttention : public MultiHeadedAttention {
                   bool is_trans_weight, const std::vector<WeightRange>& ahead, const BertAttention* lender = nullptr) const;
 
   int64_t heads() const { return num_attention_heads_; }
+  ExchangeMemory& exchange() const { return exchange_; }  // of the encoder whose first layer this is
   int64_t hidden() const { return dense_weight_.shape(0); }
   DLDataType dtype() const { return dense_weight_.dtype(); }
   // QKV weight [3H,H], bias, output weight [H,H], bias, LayerNorm gamma and beta
