@@ -546,13 +546,13 @@ TTMI_API int ttmi_encoder_chain(const void* const* weights, const void* input, c
                                 int64_t hidden, int64_t ffn, float eps, int dtype, int workgroups, int patience, void* stream);
 
 #define TTMI_CHAIN_MAX_ROWS 16
-/* A decoder layer's attention or feed-forward block as one launch: a token each of `rows` (up to TTMI_CHAIN_MAX_ROWS) sequences, fp16 or bf16, hidden a
- * multiple of 64 up to 1024.  As the layers' own launches compute it:
+/* A decoder layer's attention or feed-forward block as one launch: a token each of `rows` (up to TTMI_CHAIN_MAX_ROWS) sequences, fp32, fp16 or bf16, hidden
+ * a multiple of 64 up to 1024.  As the layers' own launches compute it:
  * ttmi_decoder_attention     y = LN(x) w_in^T + b_in: rows of Q, K and V (k_out, v_out given: k_past and v_past [rows,heads,keys-1,64] are copied and
  *                            y's key and value appended) or of Q alone (k_past and v_past [rows,heads,keys,64] are attended over);
  *                            probs [rows,heads,keys] = softmax(scale q k^T + mask), mask additive fp32 [rows,keys] or null;
  *                            out = x + (probs v) w_out^T + b_out.  hidden = 64 * heads, up to 512 keys.
- * ttmi_decoder_feed_forward  out = x + relu(LN(x) w1^T + b1) w2^T + b2; inner a multiple of 64 up to 4096.
+ * ttmi_decoder_feed_forward  out = x + relu(LN(x) w1^T + b1) w2^T + b2; inner a multiple of 64 up to 4096 (fp32: 3072).
  *   weights [out,in]; out must be another tensor than x
  *   exchange   as many bytes as ttmi_decoder_chain_workspace says (heads = 0: feed-forward; inner: 3 * hidden or hidden for attention; 0: not
  *              built), prepared once by ttmi_chain_prepare and used by one call after the other on one stream

@@ -28,9 +28,15 @@ __device__ __forceinline__ uint32_t storable(uint32_t word) { return word == kUn
 __device__ __forceinline__ uint32_t largest(uint32_t m, const u32x4& x) { return max(max(max(m, x[0]), max(x[1], x[2])), x[3]); }
 __device__ __forceinline__ uint32_t largest(uint32_t m, const u32x2& x) { return max(max(m, x[0]), x[1]); }
 
+// 16 bytes of a row of either operand: eight 16-bit values, or four of fp32 with an instruction for each.
 template <typename T>
 __device__ __forceinline__ floatx4 mma16(const u32x4& a, const u32x4& b, floatx4 c) {
-  if constexpr (std::is_same<T, f16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
+  if constexpr (std::is_same<T, float>::value) {
+    const floatx4 x = __builtin_bit_cast(floatx4, a), y = __builtin_bit_cast(floatx4, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], y[j], c, 0, 0, 0);
+    return c;
+  } else if constexpr (std::is_same<T, f16>::value) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c, 0, 0, 0);
   else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 template <typename T>
@@ -38,17 +44,34 @@ __device__ __forceinline__ float low(uint32_t pair) { return (float)__builtin_bi
 template <typename T>
 __device__ __forceinline__ float high(uint32_t pair) { return (float)__builtin_bit_cast(T, (uint16_t)(pair >> 16)); }
 
+// Four values of a row.
+template <typename T>
+using Four = typename std::conditional<sizeof(T) == 4, u32x4, u32x2>::type;
+template <typename T>
+__device__ __forceinline__ float of_four(const Four<T>& x, int e) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, (uint32_t)x[e]);
+  else return e & 1 ? high<T>(x[e >> 1]) : low<T>(x[e >> 1]);
+}
+template <typename T>
+__device__ __forceinline__ Four<T> to_four(const float (&v)[4]) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(u32x4, floatx4{v[0], v[1], v[2], v[3]});
+  else return u32x2{pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3])};
+}
+
 // Rows that the next step multiplies as they are lie as its wavefronts hold them in registers, a load of one 64 consecutive pieces: what
-// goes past the L2 is paid by the line and the load.  [K / 64, 2, 4, kChainRows, 8], in bytes, of an even column:
+// goes past the L2 is paid by the line and the load.  [K / 64, 2, 4, kChainRows, 8], of fp32 [K / 32, 2, 4, kChainRows, 4];
+// in bytes, of an even column:
+template <typename T>
 __device__ __forceinline__ uint32_t fragment_offset(int row, int col) {
+  if constexpr (sizeof(T) == 4) return (uint32_t)(((((col >> 5) * 2 + ((col >> 2) & 1)) * 4 + ((col >> 3) & 3)) * kChainRows + row) * 4 + (col & 3)) * 4;
   return (uint32_t)(((((col >> 6) * 2 + ((col >> 3) & 1)) * 4 + ((col >> 4) & 3)) * kChainRows + row) * 8 + (col & 7)) * 2;
 }
 
-__host__ __device__ inline int chain_row_pitch(int hidden) { return hidden * 2 + 16; }  // bytes of an LDS row of the A operand; four banks further per row
+__host__ __device__ inline int chain_row_pitch(int hidden, int element = 2) { return hidden * element + 16; }  // bytes of an LDS row of the A operand; four banks further per row
 
 // A row in front of a product: x, four values of every 256 columns per lane (zeros past the row), becomes v = beta + gamma * (x - mean) / sqrt(var + eps).
 template <typename T, int TURNS>
-__device__ __forceinline__ void normalise_row(const float (&x)[TURNS][4], const u32x2 (&gamma)[TURNS], const u32x2 (&beta)[TURNS], int width, float eps,
+__device__ __forceinline__ void normalise_row(const float (&x)[TURNS][4], const Four<T> (&gamma)[TURNS], const Four<T> (&beta)[TURNS], int width, float eps,
                                               float (&v)[TURNS][4]) {
   float sum = 0.f, sumsq = 0.f;
 #pragma unroll
@@ -67,8 +90,7 @@ __device__ __forceinline__ void normalise_row(const float (&x)[TURNS][4], const 
   for (int t = 0; t < TURNS; ++t)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float b = e & 1 ? high<T>(beta[t][e >> 1]) : low<T>(beta[t][e >> 1]), g = e & 1 ? high<T>(gamma[t][e >> 1]) : low<T>(gamma[t][e >> 1]);
-      v[t][e] = b + g * rstd * (x[t][e] - mean);
+      v[t][e] = of_four<T>(beta[t], e) + of_four<T>(gamma[t], e) * rstd * (x[t][e] - mean);
       asm volatile("" : "+v"(v[t][e]));  // rounded once, from fp32
     }
 }

@@ -1,5 +1,5 @@
 // One decoder layer's attention (self attention over a growing cache, or attention over an encoder memory) or its feed-forward block as
-// ONE launch: a token each of up to 16 sequences, 16-bit types.
+// ONE launch: a token each of up to 16 sequences.
 //
 //   attention     0  LayerNorm, projection of Q (and K, V)                     N/32 items
 //                 1  attention, a query each: W wavefronts a head              batch * heads * W / 16
@@ -15,6 +15,10 @@
 // us a step of six layers of base in fp16 (48 launches before, 18 now): 8 sequences, 41 and 100 keys, 236 / 184; 1 x 6 and 20 219 / 158, 4 x 201 and 30
 // 249 / 174, 16 x 41 and 100 248 / 214, 16 x 251 and 256 309 / 262.  What is left of a launch of 9 to 11: its start 0.5, arguments and first operands 1.5 to
 // 2.5, LayerNorm and product 1, an exchange 0.7 to 1.3 each, attention 1 (3.5 with 64 keys a wavefront), its parts' sum and the last product 1.5.
+// fp32 multiplies in fp32 (four instructions where 16 bits take one, the weights as they are, not their halves) and reads and exchanges twice the bytes:
+// 8 sequences, 40 and 100 keys, 319 / 273; 1 x 5 and 20 286 / 225, 4 x 200 and 30 356 / 254, 16 x 40 and 100 357 / 319, 16 x 250 and 256 453 / 395.  Its
+// error against 64 bits, rms after six layers, is what it was with the split products: 3.6 to 4.4e-7 / 3.6 to 4.4e-7 (attention's 1.1e-9 to 2.5e-8, 2 to 17%
+// less now).  Rows of 4096 products would not fit its registers: the feed-forward block goes to 3072 there.
 // Measured and no better: the arguments held in registers (60 of the scalar ones spill) 11.4 / 12.5 a launch.
 #include <mutex>
 #include <set>
@@ -26,8 +30,9 @@ namespace {
 
 constexpr int kWaves = kChainWaves, kThreads = kChainThreads, kRows = kChainRows, kColumns = kChainColumns, kPitch = kChainPitch;
 constexpr int kMostHidden = 1024, kMostInner = 4096, kMostKeys = 512;
-constexpr int kTurns = kMostHidden / 256, kPieces = kMostInner / 64 / kWaves;
-constexpr int kLdsMost = 80 * 1024;
+constexpr int kMostInner32 = 3072;  // fp32
+constexpr int kTurns = kMostHidden / 256;
+constexpr int kLdsMost = 112 * 1024;
 
 enum Block { kFeedForward, kSelfAttention, kMemoryAttention };
 
@@ -46,16 +51,23 @@ struct DecoderArgs {
 };
 
 // Exchange memory: step 0's rows ([rows, width]; in front of a product in fragment order), then the attention's in fragment order.
-__host__ __device__ inline uint32_t context_at(int width) { return (uint32_t)(kRows * width * 2); }
+__host__ __device__ inline uint32_t context_at(int width, int element) { return (uint32_t)(kRows * width * element); }
 
+// Eight columns of a row, and column e of them.
 template <typename T>
-__device__ __forceinline__ float dot8(const u32x4& a, const u32x4& b, float acc) {
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    acc = __builtin_fmaf(low<T>(a[w]), low<T>(b[w]), acc);
-    acc = __builtin_fmaf(high<T>(a[w]), high<T>(b[w]), acc);
+struct Eight {
+  u32x4 q[sizeof(T) / 2];
+  __device__ __forceinline__ float at(int e) const {
+    if constexpr (sizeof(T) == 4) return __builtin_bit_cast(float, (uint32_t)q[e >> 2][e & 3]);
+    else return e & 1 ? high<T>(q[0][e >> 1]) : low<T>(q[0][e >> 1]);
   }
-  return acc;
+};
+template <typename T>
+__device__ __forceinline__ float dot8(const Eight<T>& a, const Eight<T>& b) {
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum = __builtin_fmaf(a.at(e), b.at(e), sum);
+  return sum;
 }
 // Lanes that differ by 1, 2 and 4, and by 8, 16 and 32.
 template <typename Op>
@@ -78,6 +90,9 @@ template <typename T, Block BLOCK, int LOADS>
 __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderArgs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int STEPS = BLOCK == kFeedForward ? 2 : 3;
+  constexpr int E = sizeof(T), PIECE = 128 / E;                                     // a piece: 128 bytes of a row
+  constexpr int PIECES = kMostHidden / PIECE / kWaves;                              // of a row of H, that a wavefront takes at most
+  constexpr int OUT_PIECES = BLOCK != kFeedForward ? PIECES : (E == 4 ? kMostInner32 : kMostInner) / PIECE / kWaves;
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __align__(16) char smem[];
   __shared__ int missing;
@@ -137,13 +152,31 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
   for (;;) {
     const Arguments& a = *arguments();
     const int H = a.hidden, rows = a.rows, heads = a.heads, patience = a.patience;
-    float* const part = reinterpret_cast<float*>(smem + kRows * chain_row_pitch(H));
+    float* const part = reinterpret_cast<float*>(smem + kRows * chain_row_pitch(H, E));
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 15, lgrp = lane >> 4;
     const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, a.bytes, 0x00020000);
     auto load4 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(mem, offset, 0, kThroughMemory); };
     auto store1 = [&](uint32_t offset, uint32_t x) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b32(storable(x), mem, offset, 0, kThroughMemory); };
+    auto store_pair = [&](uint32_t offset, float v0, float v1) __attribute__((always_inline)) {
+      if constexpr (E == 4) {
+        store1(offset, __builtin_bit_cast(uint32_t, v0));
+        store1(offset + 4, __builtin_bit_cast(uint32_t, v1));
+      } else {
+        store1(offset, pack2<T>(v0, v1));
+      }
+    };
+    // two values of a row
+    typedef typename std::conditional<E == 4, u32x2, uint32_t>::type Two;
+    auto first_of = [](const Two& x) __attribute__((always_inline)) {
+      if constexpr (E == 4) return __builtin_bit_cast(float, (uint32_t)x[0]);
+      else return low<T>(x);
+    };
+    auto second_of = [](const Two& x) __attribute__((always_inline)) {
+      if constexpr (E == 4) return __builtin_bit_cast(float, (uint32_t)x[1]);
+      else return high<T>(x);
+    };
     // Asks again until there is no unwritten word; `ask` returns the largest of those it has loaded.
     bool late = false;
     auto await = [&](auto&& ask) __attribute__((always_inline)) {
@@ -162,103 +195,123 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     const int n0 = step == 0 ? item * 16 * kColumns : item * 16;
     const bool stores = product && block < (step == 0 ? kColumns : 1) && row < rows;
     const int column = n0 + block * 16 + 2 * (tid & 7);
-    uint32_t bias = 0, residual = 0;
+    Two bias = {}, residual = {};
     if (stores) {
-      bias = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(step == 0 ? a.b_in : a.b_out) + column);
-      if (step != 0) residual = *reinterpret_cast<const uint32_t*>(static_cast<const T*>(a.x) + row * H + column);
+      bias = *reinterpret_cast<const Two*>(static_cast<const T*>(step == 0 ? a.b_in : a.b_out) + column);
+      if (step != 0) residual = *reinterpret_cast<const Two*>(static_cast<const T*>(a.x) + row * H + column);
     }
     floatx4 acc[kColumns];
 #pragma unroll
     for (int c = 0; c < kColumns; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     if (step == 0) {
-      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_in), 0, a.width * H * 2, 0x00020000);
-      const uint32_t w_row = (uint32_t)((n0 + lrow) * H + wave * 64 + lgrp * 16) * 2;
-      const int pitch = chain_row_pitch(H);
-      u32x4 wf[kColumns][2];
-      u32x2 raw[kTurns], gm[kTurns], bt[kTurns];
-      const __amdgpu_buffer_rsrc_t x = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, rows * H * 2, 0x00020000);
-      const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.gamma), 0, H * 2, 0x00020000);
-      const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.beta), 0, H * 2, 0x00020000);
+      const int pieces = H / PIECE, share = (pieces + kWaves - 1) / kWaves, mine = min(pieces - wave * share, share);
+      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_in), 0, a.width * H * E, 0x00020000);
+      const uint32_t w_row = (uint32_t)((n0 + lrow) * H * E + wave * share * 128 + lgrp * 32);
+      const int pitch = chain_row_pitch(H, E);
+      u32x4 wf[PIECES][kColumns][2];
+      Four<T> raw[kTurns], gm[kTurns], bt[kTurns];
+      const __amdgpu_buffer_rsrc_t x = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, rows * H * E, 0x00020000);
+      const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.gamma), 0, H * E, 0x00020000);
+      const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.beta), 0, H * E, 0x00020000);
+      auto four = [&](const __amdgpu_buffer_rsrc_t& from, uint32_t at) __attribute__((always_inline)) {
+        if constexpr (E == 4) return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0);
+        else return (u32x2)__builtin_amdgcn_raw_buffer_load_b64(from, at, 0, 0);
+      };
 #pragma unroll
       for (int t = 0; t < kTurns; ++t) {  // rows and columns that do not exist are zeros
         const int col = t * 256 + lane * 4;
-        raw[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(x, wave < rows && col < H ? (uint32_t)(wave * H + col) * 2 : kOutside, 0, 0);
-        gm[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(g, (uint32_t)col * 2, 0, 0);
-        bt[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(b, (uint32_t)col * 2, 0, 0);
+        raw[t] = four(x, wave < rows && col < H ? (uint32_t)((wave * H + col) * E) : kOutside);
+        gm[t] = four(g, (uint32_t)(col * E));
+        bt[t] = four(b, (uint32_t)(col * E));
       }
 #pragma unroll
-      for (int c = 0; c < kColumns; ++c)
+      for (int p = 0; p < PIECES; ++p)
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
-          wf[c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, wave < H / 64 ? w_row + (uint32_t)(c * 16 * H * 2 + s * 16) : kOutside, 0, 0);
+        for (int c = 0; c < kColumns; ++c)
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+            wf[p][c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p < mine ? w_row + (uint32_t)(c * 16 * H * E + p * 128 + s * 16) : kOutside, 0, 0);
       if (wave < rows) {
         float v[kTurns][4], normed[kTurns][4];
 #pragma unroll
         for (int t = 0; t < kTurns; ++t)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[t][e] = e & 1 ? high<T>(raw[t][e >> 1]) : low<T>(raw[t][e >> 1]);
+          for (int e = 0; e < 4; ++e) v[t][e] = of_four<T>(raw[t], e);
         normalise_row<T, kTurns>(v, gm, bt, H, a.eps, normed);
 #pragma unroll
         for (int t = 0; t < kTurns; ++t) {
           const int col = t * 256 + lane * 4;
-          if (col < H) *reinterpret_cast<u32x2*>(smem + wave * pitch + col * 2) = u32x2{pack2<T>(normed[t][0], normed[t][1]), pack2<T>(normed[t][2], normed[t][3])};
+          if (col < H) *reinterpret_cast<Four<T>*>(smem + wave * pitch + col * E) = to_four<T>(normed[t]);
         }
       }
       __syncthreads();
-      if (wave < H / 64)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          const u32x4 rows_here = *reinterpret_cast<const u32x4*>(smem + lrow * pitch + wave * 128 + lgrp * 32 + s * 16);
+      for (int p = 0; p < PIECES; ++p)
+        if (p < mine)
 #pragma unroll
-          for (int c = 0; c < kColumns; ++c) acc[c] = mma16<T>(rows_here, wf[c][s], acc[c]);
-        }
+          for (int s = 0; s < 2; ++s) {
+            const u32x4 rows_here = *reinterpret_cast<const u32x4*>(smem + lrow * pitch + (wave * share + p) * 128 + lgrp * 32 + s * 16);
+#pragma unroll
+            for (int c = 0; c < kColumns; ++c) acc[c] = mma16<T>(rows_here, wf[p][c][s], acc[c]);
+          }
     } else if (step == STEPS - 1) {
-      const int K = a.inner, share = (K / 64 + kWaves - 1) / kWaves, first = wave * share, mine = min(K / 64 - first, share), there = lrow < rows ? mine : 0;
-      constexpr int PIECES = BLOCK == kFeedForward ? kPieces : 1;
-      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_out), 0, H * K * 2, 0x00020000);
-      const uint32_t w_row = (uint32_t)((n0 + lrow) * K + first * 64 + lgrp * 16) * 2;
-      const uint32_t row_at = (BLOCK == kFeedForward ? 0u : context_at(a.width)) + fragment_offset(lrow, first * 64 + lgrp * 16);
-      u32x4 wf[2 * PIECES], af[2 * PIECES];
+      const int K = a.inner, share = (K / PIECE + kWaves - 1) / kWaves, first = wave * share, mine = min(K / PIECE - first, share), there = lrow < rows ? mine : 0;
+      const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_out), 0, H * K * E, 0x00020000);
+      const uint32_t w_row = (uint32_t)((n0 + lrow) * K * E + first * 128 + lgrp * 32);
+      const uint32_t row_at = (BLOCK == kFeedForward ? 0u : context_at(a.width, E)) + fragment_offset<T>(lrow, first * PIECE + lgrp * (PIECE / 4));
+      u32x4 wf[2 * OUT_PIECES], af[2 * OUT_PIECES];
 #pragma unroll
-      for (int p = 0; p < 2 * PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
+      for (int p = 0; p < 2 * OUT_PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
       await([&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < 2 * PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
+        for (int p = 0; p < 2 * OUT_PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
         uint32_t m = 0;
 #pragma unroll
-        for (int p = 0; p < 2 * PIECES; ++p) m = largest(m, af[p]);
+        for (int p = 0; p < 2 * OUT_PIECES; ++p) m = largest(m, af[p]);
         return m;
       });
       if (late) missing = 1;
 #pragma unroll
-      for (int p = 0; p < 2 * PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
+      for (int p = 0; p < 2 * OUT_PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
     } else {
       // A wavefront takes 8 * LOADS keys of a head: a lane eight columns of every eighth key.
       const int pair = item * (kWaves / a.waves) + wave / a.waves, share = wave % a.waves, key0 = share * (8 * LOADS) + (lane >> 3), piece = lane & 7;
       const bool has = pair < rows * heads;
       const int b = has ? pair / heads : 0, head = has ? pair - b * heads : 0, keys = a.keys, past = a.past;
-      const __amdgpu_buffer_rsrc_t kp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.k_past), 0, rows * heads * past * 128, 0x00020000);
-      const __amdgpu_buffer_rsrc_t vp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.v_past), 0, rows * heads * past * 128, 0x00020000);
-      u32x4 kf[LOADS], vf[LOADS];
+      const __amdgpu_buffer_rsrc_t kp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.k_past), 0, rows * heads * past * kD * E, 0x00020000);
+      const __amdgpu_buffer_rsrc_t vp = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.v_past), 0, rows * heads * past * kD * E, 0x00020000);
+      Eight<T> kf[LOADS], vf[LOADS];
       float mk[LOADS];
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         const int key = key0 + i * 8;
-        const uint32_t at = has && key < past ? (uint32_t)((pair * past + key) * 128 + piece * 16) : kOutside;
-        kf[i] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(kp, at, 0, 0);
-        vf[i] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(vp, at, 0, 0);
+        const uint32_t at = (uint32_t)((pair * past + key) * (kD * E) + piece * (8 * E));
+#pragma unroll
+        for (int h = 0; h < E / 2; ++h) {
+          kf[i].q[h] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(kp, has && key < past ? at + h * 16 : kOutside, 0, 0);
+          vf[i].q[h] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(vp, has && key < past ? at + h * 16 : kOutside, 0, 0);
+        }
         mk[i] = a.mask != nullptr ? a.mask[b * keys + min(key, keys - 1)] : 0.f;
       }
-      u32x4 qf, kn = {0u, 0u, 0u, 0u}, vn = {0u, 0u, 0u, 0u};
-      const uint32_t at = (uint32_t)(b * a.width + head * kD + piece * 8) * 2;
+      Eight<T> qf, kn, vn;
+      const uint32_t at = (uint32_t)((b * a.width + head * kD + piece * 8) * E), row_bytes = (uint32_t)(H * E);
       await([&]() __attribute__((always_inline)) {
-        qf = load4(has ? at : kOutside);
-        if constexpr (BLOCK == kSelfAttention) {
-          kn = load4(has ? at + (uint32_t)H * 2 : kOutside);
-          vn = load4(has ? at + (uint32_t)H * 4 : kOutside);
+        uint32_t m = 0;
+#pragma unroll
+        for (int h = 0; h < E / 2; ++h) {
+          qf.q[h] = load4(has ? at + h * 16 : kOutside);
+          if constexpr (BLOCK == kSelfAttention) {
+            kn.q[h] = load4(has ? at + row_bytes + h * 16 : kOutside);
+            vn.q[h] = load4(has ? at + 2 * row_bytes + h * 16 : kOutside);
+          }
         }
-        return largest(largest(largest(0u, qf), kn), vn);
+#pragma unroll
+        for (int h = 0; h < E / 2; ++h) {
+          m = largest(m, qf.q[h]);
+          if constexpr (BLOCK == kSelfAttention) m = largest(largest(m, kn.q[h]), vn.q[h]);
+        }
+        return m;
       });
       if (late) missing = 1;
       float s[LOADS], mx = -__builtin_inff();
@@ -271,11 +324,14 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
           if (key == past) kf[i] = kn, vf[i] = vn;
           if (!late && has && key < keys) {
             const int64_t to = ((int64_t)pair * keys + key) * kD + piece * 8;
-            *reinterpret_cast<u32x4*>(static_cast<T*>(a.k_out) + to) = kf[i];
-            *reinterpret_cast<u32x4*>(static_cast<T*>(a.v_out) + to) = vf[i];
+#pragma unroll
+            for (int h = 0; h < E / 2; ++h) {
+              *reinterpret_cast<u32x4*>(static_cast<T*>(a.k_out) + to + h * (16 / E)) = kf[i].q[h];
+              *reinterpret_cast<u32x4*>(static_cast<T*>(a.v_out) + to + h * (16 / E)) = vf[i].q[h];
+            }
           }
         }
-        s[i] = __builtin_fmaf(over_pieces(dot8<T>(kf[i], qf, 0.f), add), a.scale, mk[i]);
+        s[i] = __builtin_fmaf(over_pieces(dot8<T>(kf[i], qf), add), a.scale, mk[i]);
         if (key < keys) mx = fmaxf(mx, s[i]);
       }
       mx = over_keys(mx, larger);
@@ -305,10 +361,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
         if (!late && has && key < keys && piece == 0) static_cast<T*>(a.probs)[(int64_t)pair * keys + key] = p;
         const float weight = to_float(p);
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {  // (keys past the last are zeros)
-          o[2 * w] = __builtin_fmaf(weight, low<T>(vf[i][w]), o[2 * w]);
-          o[2 * w + 1] = __builtin_fmaf(weight, high<T>(vf[i][w]), o[2 * w + 1]);
-        }
+        for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(weight, vf[i].at(e), o[e]);  // (keys past the last are zeros)
       }
       // eight groups of lanes have a part each: two of a row of 16 lanes meet here, the rest in LDS
 #pragma unroll
@@ -343,13 +396,16 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     }
     if (stores) {
       const floatx2 v = sum_parts(part, row, column - n0, 1);
-      float v0 = v[0] + low<T>(bias), v1 = v[1] + high<T>(bias);
+      const float v0 = v[0] + first_of(bias), v1 = v[1] + second_of(bias);
       if (step == STEPS - 1) {
-        *reinterpret_cast<uint32_t*>(static_cast<T*>(a.out) + row * H + column) = pack2<T>(v0 + low<T>(residual), v1 + high<T>(residual));
+        Vec<T, 2> r;
+        r.v[0] = from_float<T>(v0 + first_of(residual));
+        r.v[1] = from_float<T>(v1 + second_of(residual));
+        store_vec<T, 2>(static_cast<T*>(a.out) + row * H + column, r);
       } else if constexpr (BLOCK == kFeedForward) {
-        store1(fragment_offset(row, column), pack2<T>(fmaxf(v0, 0.f), fmaxf(v1, 0.f)));
+        store_pair(fragment_offset<T>(row, column), fmaxf(v0, 0.f), fmaxf(v1, 0.f));
       } else {
-        store1((uint32_t)(row * a.width + column) * 2, pack2<T>(v0, v1));
+        store_pair((uint32_t)((row * a.width + column) * E), v0, v1);
       }
     } else if (!product) {
       // the context of the workgroup's heads, two columns a thread
@@ -363,7 +419,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
           v1 += p[1];
         }
         const int b = pair / heads;
-        store1(context_at(a.width) + fragment_offset(b, (pair - b * heads) * kD + col), pack2<T>(v0, v1));
+        store_pair(context_at(a.width, E) + fragment_offset<T>(b, (pair - b * heads) * kD + col), v0, v1);
       }
     }
     tries = 0;
@@ -382,7 +438,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
 #endif
 }
 
-int64_t part_bytes(Block block, int64_t hidden, int64_t width) { return kRows * 2 * (width + (block == kFeedForward ? 0 : hidden)); }
+int64_t part_bytes(Block block, int64_t hidden, int64_t width, int64_t element) { return kRows * element * (width + (block == kFeedForward ? 0 : hidden)); }
 
 template <typename T, Block BLOCK, int LOADS>
 int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
@@ -391,7 +447,7 @@ int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
   const int64_t middle = BLOCK == kFeedForward ? 0 : ceil_div((int64_t)a.rows * a.heads * a.waves, kWaves);
   const int64_t all = a.width / (16 * kColumns) + middle + a.hidden / 16;
   const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(all, compute_units());
-  const int lds = kRows * chain_row_pitch(a.hidden) + kWaves * kRows * kPitch * 4;
+  const int lds = kRows * chain_row_pitch(a.hidden, sizeof(T)) + kWaves * kRows * kPitch * 4;
   auto kernel = decoder_chain_kernel<T, BLOCK, LOADS>;
   // more than 64 KB of dynamic LDS: the limit is raised once per kernel and device
   static std::mutex mu;
@@ -413,12 +469,12 @@ template <typename T, Block BLOCK>
 int launch(const DecoderArgs& a, int workgroups, hipStream_t s) {
   // Few keys a wavefront: the sixteen of a workgroup share four SIMDs, and what the attention of 64 keys takes there is more than an exchange.
   if constexpr (BLOCK != kFeedForward)
-    if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, 8>(a, workgroups, s);
+    if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, sizeof(T) == 4 ? 4 : 8>(a, workgroups, s);  // (fp32: 64 keys do not fit the registers)
   return launch_sized<T, BLOCK, 2>(a, workgroups, s);
 }
 
 bool takes(int64_t rows, int64_t hidden, int dtype) {
-  return (dtype == TTMI_F16 || dtype == TTMI_BF16) && rows >= 1 && rows <= kRows && hidden >= 64 && hidden % 64 == 0 && hidden <= kMostHidden;
+  return (dtype == TTMI_F32 || dtype == TTMI_F16 || dtype == TTMI_BF16) && rows >= 1 && rows <= kRows && hidden >= 64 && hidden % 64 == 0 && hidden <= kMostHidden;
 }
 
 }  // namespace
@@ -433,9 +489,9 @@ int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, in
   *bytes = 0;
   if (!takes(rows, hidden, dtype)) return 0;
   if (heads > 0) {
-    if (hidden == heads * kD && keys >= 1 && keys <= kMostKeys && (inner == hidden || inner == 3 * hidden)) *bytes = 3 * part_bytes(kSelfAttention, hidden, inner);
-  } else if (inner >= 64 && inner % 64 == 0 && inner <= kMostInner) {
-    *bytes = 3 * part_bytes(kFeedForward, hidden, inner);
+    if (hidden == heads * kD && keys >= 1 && keys <= kMostKeys && (inner == hidden || inner == 3 * hidden)) *bytes = 3 * part_bytes(kSelfAttention, hidden, inner, (int64_t)dtype_size(dtype));
+  } else if (inner >= 64 && inner % 64 == 0 && inner <= (dtype == TTMI_F32 ? kMostInner32 : kMostInner)) {
+    *bytes = 3 * part_bytes(kFeedForward, hidden, inner, (int64_t)dtype_size(dtype));
   }
   return 0;
 }
@@ -463,7 +519,8 @@ int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta
   a.bytes = (uint32_t)(bytes / 3);
   const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
   if (part != 0) return part;
-  return dtype == TTMI_F16 ? launch<f16, kFeedForward>(a, workgroups, (hipStream_t)stream) : launch<bf16, kFeedForward>(a, workgroups, (hipStream_t)stream);
+  TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kFeedForward>(a, workgroups, (hipStream_t)stream)));
+  return 0;
 }
 
 int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, float eps, const void* w_in, const void* b_in, const void* w_out,
@@ -491,8 +548,12 @@ int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, f
   a.bytes = (uint32_t)(bytes / 3);
   const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
   if (part != 0) return part;
-  if (grows) return dtype == TTMI_F16 ? launch<f16, kSelfAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kSelfAttention>(a, workgroups, (hipStream_t)stream);
-  return dtype == TTMI_F16 ? launch<f16, kMemoryAttention>(a, workgroups, (hipStream_t)stream) : launch<bf16, kMemoryAttention>(a, workgroups, (hipStream_t)stream);
+  if (grows) {
+    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kSelfAttention>(a, workgroups, (hipStream_t)stream)));
+  } else {
+    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kMemoryAttention>(a, workgroups, (hipStream_t)stream)));
+  }
+  return 0;
 }
 
 }  // extern "C"

@@ -383,7 +383,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
       } else {
         const int share = (F / 64 + kWaves - 1) / kWaves, first = wave * share, mine = min(F / 64 - first, share);
         const int there = lrow < rows ? mine : 0;
-        const uint32_t row_at = base + at.mid + fragment_offset(lrow, first * 64 + lgrp * 16);
+        const uint32_t row_at = base + at.mid + fragment_offset<T>(lrow, first * 64 + lgrp * 16);
         u32x4 wf[2 * PIECES], af[2 * PIECES];
 #pragma unroll
         for (int p = 0; p < 2 * PIECES; ++p)
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
         if (ph == 0) {
           store1(base + at.qk + q_offset(r, n0 + c), pack2<T>(v0, v1));
         } else if (ph == 2) {
-          store1(base + at.mid + fragment_offset(r, n0 + c), pack2<T>(gelu_tanh(v0), gelu_tanh(v1)));
+          store1(base + at.mid + fragment_offset<T>(r, n0 + c), pack2<T>(gelu_tanh(v0), gelu_tanh(v1)));
         } else {
           const uint32_t to = base + (ph == 1 ? at.sum1 : at.sum2) + (uint32_t)(r * H + n0 + c) * 4;
           store1(to, __builtin_bit_cast(uint32_t, v0 + res0));

@@ -159,7 +159,7 @@ static void CheckFfn(const Tensor& input, const Tensor& w1, const Tensor& b1, co
 bool PositionwiseFeedForward::AsOneLaunch(const Tensor& input_tensor, Tensor* output, bool is_trans_weight) const {
   const int64_t rows = input_tensor.shape(0) * input_tensor.shape(1), model_dim = input_tensor.shape(2);
   const int dt = kernels::DeviceDType(input_tensor);
-  if (dt == TTMI_F32 || rows > TTMI_CHAIN_MAX_ROWS) return false;
+  if (rows > TTMI_CHAIN_MAX_ROWS) return false;
   const int64_t d_ff = PackedWeight::OutDim(dense_weight_1_, is_trans_weight);
   int64_t bytes = 0;
   TT_DEVICE_CALL(ttmi_decoder_chain_workspace(rows, 0, model_dim, d_ff, 0, dt, &bytes));

@@ -221,7 +221,7 @@ static void StoreInCache(std::unordered_map<std::string, Tensor*>& cache, const 
 bool MultiHeadedAttention::AsOneLaunch(const Tensor& query_tensor, const Tensor& attention_mask, bool is_self, Tensor* output, Tensor* att_score,
                                        const std::unordered_map<std::string, Tensor*>& layer_cache, bool is_trans_weight) const {
   const int dt = kernels::DeviceDType(query_tensor);
-  if (dt == TTMI_F32 || query_tensor.shape(0) > TTMI_CHAIN_MAX_ROWS || query_tensor.shape(1) != 1 || att_score == nullptr) return false;
+  if (query_tensor.shape(0) > TTMI_CHAIN_MAX_ROWS || query_tensor.shape(1) != 1 || att_score == nullptr) return false;
   const char *key_name = is_self ? "self_keys" : "memory_keys", *value_name = is_self ? "self_values" : "memory_values";
   if (!CacheHas(layer_cache, key_name) || !CacheHas(layer_cache, value_name)) return false;
   const Tensor &k_past = *layer_cache.at(key_name), &v_past = *layer_cache.at(value_name);
