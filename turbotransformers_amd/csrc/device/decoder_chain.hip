@@ -12,13 +12,20 @@
 // weights, or its keys and values, before it waits.  Progress does not depend on how many of them are resident, as in encoder_chain.hip: a workgroup that
 // has waited in vain executes all items of the steps in front of its own.
 //
-// us a step of six layers of base in fp16 (48 launches before, 18 now): 8 sequences, 41 and 100 keys, 236 / 184; 1 x 6 and 20 219 / 158, 4 x 201 and 30
-// 249 / 174, 16 x 41 and 100 248 / 214, 16 x 251 and 256 309 / 262.  What is left of a launch of 9 to 11: its start 0.5, arguments and first operands 1.5 to
-// 2.5, LayerNorm and product 1, an exchange 0.7 to 1.3 each, attention 1 (3.5 with 64 keys a wavefront), its parts' sum and the last product 1.5.
-// fp32 multiplies in fp32 (four instructions where 16 bits take one, the weights as they are, not their halves) and reads and exchanges twice the bytes:
-// 8 sequences, 40 and 100 keys, 319 / 273; 1 x 5 and 20 286 / 225, 4 x 200 and 30 356 / 254, 16 x 40 and 100 357 / 319, 16 x 250 and 256 453 / 395.  Its
-// error against 64 bits, rms after six layers, is what it was with the split products: 3.6 to 4.4e-7 / 3.6 to 4.4e-7 (attention's 1.1e-9 to 2.5e-8, 2 to 17%
-// less now).  Rows of 4096 products would not fit its registers: the feed-forward block goes to 3072 there.
+// us a step of six layers of base (48 launches before, 18 now), by sequences and keys of the two attentions:
+//              1 x 6, 20    4 x 201, 30    8 x 41, 100    16 x 41, 100    16 x 251, 256
+//   fp16       255 / 151    250 / 169      240 / 179      250 / 213       308 / 262
+//   fp32       286 / 229    357 / 257      328 / 278      356 / 317       454 / 395
+// What is left of a launch of 8 to 12 in fp16: its start 0.5, arguments and first operands 1.5 to 2.5, LayerNorm and product 1, an exchange 0.7 to 1.3 each,
+// attention 1 (3.5 with 64 keys a wavefront), its parts' sum and the last product 1.5.  A load of 16 bytes a lane takes the CU 16 cycles whatever it reads: what
+// is asked for, in which order, and by how many wavefronts decides.  The weights first, the rows and parameters of the LayerNorm after them and
+// together, nothing by wavefronts without a share: 8 sequences 188 / 178, 4 180 / 169, 1 159 / 151, 16 218 / 214; fp32 level to 1%.
+// fp32 multiplies in fp32 (four instructions where 16 bits take one, the weights as they are, not their halves) and reads and exchanges twice the bytes.  Its
+// error against 64 bits, rms after six layers, was 3.64 to 4.44e-7 with the split products and is 3.61 to 4.41e-7, that of the probabilities 11% less.
+// Rows of 4096 products would not fit its registers: the feed-forward block goes to 3072 there.
+// Measured and no better: a wavefront normalises the columns that it multiplies, of all rows (parameters read once a CU, no rows in LDS, but 12 loads more
+// a wavefront): fp32 8 sequences 274 / 302, fp16 8 188 / 196, 16 x 251 262 / 258; rows and parameters requested in front of the weights: fp32 274 / 281 to
+// 286, 1 x 6 226 / 242 to 245.
 // Measured and no better: the arguments held in registers (60 of the scalar ones spill) 11.4 / 12.5 a launch.
 #include <mutex>
 #include <set>
@@ -85,14 +92,14 @@ __device__ __forceinline__ float over_keys(float v, Op op) {
   return op(halves.a, halves.b);
 }
 
-// LOADS: keys of a lane of the attention
+// LOADS: keys of a lane of the attention; pieces of a wavefront of the feed-forward block's last product
 template <typename T, Block BLOCK, int LOADS>
 __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderArgs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int STEPS = BLOCK == kFeedForward ? 2 : 3;
   constexpr int E = sizeof(T), PIECE = 128 / E;                                     // a piece: 128 bytes of a row
   constexpr int PIECES = kMostHidden / PIECE / kWaves;                              // of a row of H, that a wavefront takes at most
-  constexpr int OUT_PIECES = BLOCK != kFeedForward ? PIECES : (E == 4 ? kMostInner32 : kMostInner) / PIECE / kWaves;
+  constexpr int OUT_PIECES = BLOCK != kFeedForward ? PIECES : LOADS;          // of a row in front of the last product
   constexpr float kLog2e = 1.4426950408889634f;
   extern __shared__ __align__(16) char smem[];
   __shared__ int missing;
@@ -210,7 +217,6 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
       const uint32_t w_row = (uint32_t)((n0 + lrow) * H * E + wave * share * 128 + lgrp * 32);
       const int pitch = chain_row_pitch(H, E);
       u32x4 wf[PIECES][kColumns][2];
-      Four<T> raw[kTurns], gm[kTurns], bt[kTurns];
       const __amdgpu_buffer_rsrc_t x = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.x), 0, rows * H * E, 0x00020000);
       const __amdgpu_buffer_rsrc_t g = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.gamma), 0, H * E, 0x00020000);
       const __amdgpu_buffer_rsrc_t b = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.beta), 0, H * E, 0x00020000);
@@ -219,20 +225,24 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
         else return (u32x2)__builtin_amdgcn_raw_buffer_load_b64(from, at, 0, 0);
       };
 #pragma unroll
-      for (int t = 0; t < kTurns; ++t) {  // rows and columns that do not exist are zeros
-        const int col = t * 256 + lane * 4;
-        raw[t] = four(x, wave < rows && col < H ? (uint32_t)((wave * H + col) * E) : kOutside);
-        gm[t] = four(g, (uint32_t)(col * E));
-        bt[t] = four(b, (uint32_t)(col * E));
-      }
-#pragma unroll
       for (int p = 0; p < PIECES; ++p)
 #pragma unroll
         for (int c = 0; c < kColumns; ++c)
 #pragma unroll
           for (int s = 0; s < 2; ++s)
             wf[p][c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p < mine ? w_row + (uint32_t)(c * 16 * H * E + p * 128 + s * 16) : kOutside, 0, 0);
+      // Requested in this order and here, not where they are used: the weights come from the furthest.
+      asm volatile("" ::: "memory");
       if (wave < rows) {
+        Four<T> raw[kTurns], gm[kTurns], bt[kTurns];
+#pragma unroll
+        for (int t = 0; t < kTurns; ++t) {  // columns that do not exist are zeros
+          const int col = t * 256 + lane * 4;
+          raw[t] = four(x, col < H ? (uint32_t)((wave * H + col) * E) : kOutside);
+          gm[t] = four(g, (uint32_t)(col * E));
+          bt[t] = four(b, (uint32_t)(col * E));
+        }
+        asm volatile("" ::: "memory");
         float v[kTurns][4], normed[kTurns][4];
 #pragma unroll
         for (int t = 0; t < kTurns; ++t)
@@ -261,20 +271,22 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
       const uint32_t w_row = (uint32_t)((n0 + lrow) * K * E + first * 128 + lgrp * 32);
       const uint32_t row_at = (BLOCK == kFeedForward ? 0u : context_at(a.width, E)) + fragment_offset<T>(lrow, first * PIECE + lgrp * (PIECE / 4));
       u32x4 wf[2 * OUT_PIECES], af[2 * OUT_PIECES];
+      if (BLOCK == kFeedForward || mine > 0) {  // (the same for the wavefront; all of them have a share of the many rows of W2)
 #pragma unroll
-      for (int p = 0; p < 2 * OUT_PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
-      await([&]() __attribute__((always_inline)) {
+        for (int p = 0; p < 2 * OUT_PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
+        await([&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < 2 * OUT_PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
-        uint32_t m = 0;
+          for (int p = 0; p < 2 * OUT_PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
+          uint32_t m = 0;
 #pragma unroll
-        for (int p = 0; p < 2 * OUT_PIECES; ++p) m = largest(m, af[p]);
-        return m;
-      });
-      if (late) missing = 1;
+          for (int p = 0; p < 2 * OUT_PIECES; ++p) m = largest(m, af[p]);
+          return m;
+        });
+        if (late) missing = 1;
 #pragma unroll
-      for (int p = 0; p < 2 * OUT_PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
-    } else {
+        for (int p = 0; p < 2 * OUT_PIECES; ++p) acc[0] = mma16<T>(af[p], wf[p], acc[0]);
+      }
+    } else if constexpr (BLOCK != kFeedForward) {
       // A wavefront takes 8 * LOADS keys of a head: a lane eight columns of every eighth key.
       const int pair = item * (kWaves / a.waves) + wave / a.waves, share = wave % a.waves, key0 = share * (8 * LOADS) + (lane >> 3), piece = lane & 7;
       const bool has = pair < rows * heads;
@@ -470,7 +482,13 @@ int launch(const DecoderArgs& a, int workgroups, hipStream_t s) {
   // Few keys a wavefront: the sixteen of a workgroup share four SIMDs, and what the attention of 64 keys takes there is more than an exchange.
   if constexpr (BLOCK != kFeedForward)
     if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, sizeof(T) == 4 ? 4 : 8>(a, workgroups, s);  // (fp32: 64 keys do not fit the registers)
-  return launch_sized<T, BLOCK, 2>(a, workgroups, s);
+  if constexpr (BLOCK == kFeedForward) {
+    constexpr int kPieces = 3072 * (int)sizeof(T) / 128 / kWaves;
+    if (a.inner > 3072) return launch_sized<T, BLOCK, sizeof(T) == 4 ? kPieces : 4>(a, workgroups, s);  // (fp32: refused)
+    return launch_sized<T, BLOCK, kPieces>(a, workgroups, s);
+  } else {
+    return launch_sized<T, BLOCK, 2>(a, workgroups, s);
+  }
 }
 
 bool takes(int64_t rows, int64_t hidden, int dtype) {
