@@ -12,9 +12,11 @@
 // and the last LayerNorm.  Rows in front of a LayerNorm travel in fp32; each item normalises all of them for itself (the attention is
 // likewise computed by every item of step 1): a few hundred cycles instead of one more exchange.
 //
-// us per forward, layer by layer / as one launch: fp16 base 1 x 1 token 280 / 157, 1 x 8 291 / 176, 4 x 4 308 / 199; bf16 large 1 x 8
-// 661 / 461, 1 x 16 675 / 511 (the exchange memory filled by a launch of its own in front: 160, 179, 201, 464, 515).  What bounds a step of 3.2 to 4 us: the exchange 1.0 to 1.5 (a store to memory, and a load that finds it), the
-// LayerNorm of 16 rows on every CU 0.5 to 1.2 (vector instructions: 16 rows are four a SIMD), the product and the sum over the wavefronts 0.6.
+// us per forward, layer by layer / as one launch: fp16 base 1 x 1 token 280 / 156, 1 x 8 291 / 175, 1 x 10 297 / 188, 4 x 4 308 / 198; bf16 large 1 x 8
+// 661 / 420, 1 x 16 675 / 485 (the exchange memory filled by a launch of its own in front: 3 to 5 more; every wavefront asking for rows and parameters,
+// also those that have no row: large 461 and 511, base level).  What bounds a step of 3.2 to 4 us: the exchange 1.0 to 1.5 (a store to memory, and a load
+// that finds it), the LayerNorm of 16 rows on every CU 0.5 to 1.2 (vector instructions: 16 rows are four a SIMD), the product and the sum over the
+// wavefronts 0.6.
 // Measured and no better: 16 columns an item (240 workgroups instead of 144) level; Q, K, V and the intermediate rows row by row instead
 // of in the order of the registers 10 rows 218 / 183, 16 251 / 194 (the launch alone).
 //
@@ -209,11 +211,17 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
 
     if ((ph & 1) == 0) {  // (the last step among them)
       u32x4 wf[kColumns][2];
-      const uint32_t piece = wave < H / 64 ? w_row + wave * 128 : kOutside;
+      // Beyond 768 columns (nearly) all wavefronts have a share: a branch instead of a choice of addresses, large 1 x 8 445 / 420, 1 x 16 509 / 485; with twelve
+      // of sixteen base 1 x 10 187.9 / 189.5.
+      constexpr bool BRANCH = TURNS > 3;
+      if (!BRANCH || wave < H / 64) {
+        const uint32_t piece = BRANCH || wave < H / 64 ? w_row + wave * 128 : kOutside;
 #pragma unroll
-      for (int c = 0; c < kColumns; ++c)
+        for (int c = 0; c < kColumns; ++c)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) wf[c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, wave < H / 64 ? piece + (uint32_t)(c * 16 * H * 2 + s * 16) : kOutside, 0, 0);
+          for (int s = 0; s < 2; ++s)
+            wf[c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, BRANCH || wave < H / 64 ? piece + (uint32_t)(c * 16 * H * 2 + s * 16) : kOutside, 0, 0);
+      }
       if (step == 0) {
         if (wave < rows)
 #pragma unroll
@@ -221,7 +229,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
             const int col = t * 256 + lane * 4;
             if (col < H) *reinterpret_cast<u32x2*>(smem + wave * pitch + col * 2) = *reinterpret_cast<const u32x2*>(static_cast<const T*>(a.input) + wave * H + col);
           }
-      } else {
+      } else if (wave < rows) {
         u32x2 gm[TURNS], bt[TURNS];
         {
           const void* gamma = uniform(ph == 2 ? y.gamma1 : layers[l - 1].gamma2);
@@ -234,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
             bt[t] = (u32x2)__builtin_amdgcn_raw_buffer_load_b64(b, t * 512 + lane * 8, 0, 0);
           }
         }
-        // rows and columns that do not exist are zeros
+        // columns that do not exist are zeros
         const uint32_t from = ph == 2 ? base + at.sum1 : base - a.layer_bytes + at.sum2;
         const uint32_t keep = ph == 2 ? base + at.x1 : base + at.x0;
         u32x4 raw[TURNS];
@@ -243,7 +251,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
 #pragma unroll
           for (int t = 0; t < TURNS; ++t) {
             const int col = t * 256 + lane * 4;
-            raw[t] = load4(wave < rows && col < H ? from + (uint32_t)(wave * H + col) * 4 : kOutside);
+            raw[t] = load4(col < H ? from + (uint32_t)(wave * H + col) * 4 : kOutside);
           }
 #pragma unroll
           for (int t = 0; t < TURNS; ++t) m = largest(m, raw[t]);
@@ -251,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
         });
         if (late) {
           missing = 1;
-        } else if (wave < rows) {
+        } else {
           float x[TURNS][4], normed[TURNS][4];
 #pragma unroll
           for (int t = 0; t < TURNS; ++t)
