@@ -145,3 +145,34 @@ def test_what_is_not_built_has_no_workspace(ttmi):
                  (2, 8, 3, 192, 768, "f16"), (2, 8, 12, 1536, 3072, "f16"), (2, 8, 12, 768, 3104, "f16"), (2, 8, 12, 768, 4160, "f16")]:
         ok(ttmi.ttmi_encoder_chain_workspace(*args[:5], TTMI_DTYPES[args[5]], ctypes.addressof(size)))
         assert size.value == 0, args
+
+
+def test_a_recorded_stack_leaves_another_number_of_its_layers_alone():
+    """Two stacks with the same first layer have exchange memory of two sizes: replays of the one between calls of the other."""
+    import turbo_transformers as tt
+    from test_model_gpu import _hf_bert
+
+    model, cfg = _hf_bert(3, seed=11)
+    encoder = tt.BertModel.from_torch(model.half(), torch.device("cuda:0"), "turbo").bertmodel_nopooler.encoder
+    gen = torch.Generator().manual_seed(2)
+    long, short = [torch.randn(1, 10, cfg.hidden_size, generator=gen).half().cuda() for _ in range(2)]
+    layers = list(encoder.layer)
+
+    def run(count, x):
+        encoder.layer = layers[:count]
+        return encoder(x)[0]
+
+    want = [run(3, long).clone(), run(2, short).clone()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run(2, short)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = run(2, short)
+    for _ in range(4):
+        assert torch.equal(run(3, long), want[0])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, want[1])

@@ -1,7 +1,10 @@
 // The memory through which the steps of a call that runs as one launch pass their rows (ttmi_encoder_chain, ttmi_decoder_attention,
-// ttmi_decoder_feed_forward): its parts take turns from call to call of the layer that holds it, and go with it.
+// ttmi_decoder_feed_forward): its parts take turns from call to call of the layer that holds it, and go with it.  Calls of another size have
+// memory of their own, so that a recorded call, replayed between them, writes nothing that they count on, and its memory stays where it is.  (The sizes
+// do not depend on the rows: there is one, but for encoders of another number of layers.)
 #pragma once
 
+#include <list>
 #include <mutex>
 
 #include "core/device_context.h"
@@ -18,25 +21,37 @@ class ExchangeMemory {
   void Use(int64_t bytes, DLDeviceType device, int device_id, const Launch& launch) {
     std::lock_guard<std::mutex> lock(mutex_);
     void* const stream = core::DeviceContext::GetInstance().stream();
-    float* const memory = memory_.Reshape<float>({bytes / 4}, device, device_id, "chain/exchange");
+    Memory* m = nullptr;
+    for (Memory& known : memory_)
+      if (known.bytes == bytes && known.device_id == device_id) m = &known;
+    if (m == nullptr) {
+      memory_.emplace_back();
+      m = &memory_.back();
+      m->bytes = bytes, m->device_id = device_id;
+    }
+    float* const memory = m->words.Reshape<float>({bytes / 4}, device, device_id, "chain/exchange");
     int capturing = 0;
     TT_DEVICE_CALL(ttmi_stream_capturing(stream, &capturing));
     if (capturing) {  // replayed in an order that is not known here
       launch(memory, 2);
       return;
     }
-    if (prepared_ != bytes) TT_DEVICE_CALL(ttmi_chain_prepare(memory, bytes, stream));
-    prepared_ = 0;  // (until the call is queued)
-    launch(memory, turn_);
-    turn_ = 1 - turn_;
-    prepared_ = bytes;
+    if (!m->prepared) TT_DEVICE_CALL(ttmi_chain_prepare(memory, bytes, stream));
+    m->prepared = false;  // (until the call is queued)
+    launch(memory, m->turn);
+    m->turn = 1 - m->turn;
+    m->prepared = true;
   }
 
  private:
+  struct Memory {
+    core::Tensor words{nullptr};
+    int64_t bytes = 0;
+    int device_id = 0, turn = 0;
+    bool prepared = false;
+  };
   std::mutex mutex_;
-  core::Tensor memory_{nullptr};
-  int64_t prepared_ = 0;  // bytes
-  int turn_ = 0;
+  std::list<Memory> memory_;
 };
 
 }  // namespace layers
