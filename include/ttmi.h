@@ -536,7 +536,7 @@ TTMI_API int ttmi_dequant_bias(const int32_t* acc, const float* act_scale_dev, c
  *   workgroups, patience: 0, or (tests) how many workgroups are launched and how often one asks for rows that are not there yet
  *              before it computes them itself; neither changes a bit of the result
  * ttmi_encoder_chain_workspace says 0 for what is not built: other types, more than 24 layers, more than 16 rows (batch * seq), head
- *   sizes other than 64, fewer than 4 or more than 16 heads, F no multiple of 64 or outside 256 to 4096.
+ *   sizes other than 64, fewer than 4 or more than 16 heads, F no multiple of 64 or outside H to 4096.
  * No counterpart in the reference. */
 TTMI_API int ttmi_encoder_chain_workspace(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype,
                                           int64_t* bytes);

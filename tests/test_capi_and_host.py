@@ -466,3 +466,15 @@ def test_the_layers_product_with_activation_has_no_named_form():
     assert one == other
     assert lib.ttmi_gemm_bias_act_describe(128, 3072, 768, capi.ACT_GELU, capi.F16, buf, 4) != 0  # too small for the answer
     assert lib.ttmi_gemm_bias_act_describe(128, 3072, 768, 99, capi.F16, buf, 64) != 0
+
+
+def test_encoder_stacks_as_one_launch_have_inner_rows_as_wide_as_the_hidden_ones():
+    """The items of a step write the residual of the columns of their own number: with fewer items than column blocks some would
+    never be written."""
+    lib = capi.load()
+    size = ctypes.c_int64(7)
+    for heads, ffn, built in [(12, 768, True), (12, 704, False), (12, 512, False), (12, 256, False), (16, 1024, True), (16, 960, False), (4, 256, True),
+                              (4, 192, False), (12, 4096, True)]:
+        for dtype in (capi.F16, capi.BF16):
+            capi.check(lib.ttmi_encoder_chain_workspace(2, 8, heads, heads * 64, ffn, dtype, ctypes.addressof(size)))
+            assert (size.value > 0) == built, (heads, ffn)

@@ -480,8 +480,9 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
 }
 
 int64_t workspace_bytes(int64_t layers, int64_t rows, int64_t heads, int64_t hidden, int64_t ffn, int dtype) {
-  const bool takes = (dtype == TTMI_F16 || dtype == TTMI_BF16) && layers >= 1 && layers <= kMostLayers && rows >= 1 && rows <= kRows && heads >= 1 &&
-                     heads >= 4 && heads <= kWaves && hidden == heads * kD && ffn >= 256 && ffn % 64 == 0 && ffn <= kWaves * 4 * 64;
+  // ffn >= hidden: the items of step 2 are those that write x1, each the columns of its own number, which has to reach all of them.
+  const bool takes = (dtype == TTMI_F16 || dtype == TTMI_BF16) && layers >= 1 && layers <= kMostLayers && rows >= 1 && rows <= kRows && heads >= 4 &&
+                     heads <= kWaves && hidden == heads * kD && ffn >= hidden && ffn % 64 == 0 && ffn <= kWaves * 4 * 64;
   if (!takes) return 0;
   return 3 * layers * (int64_t)places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end;  // (of all rows: calls of any number of them take turns)
 }
