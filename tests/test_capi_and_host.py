@@ -478,3 +478,99 @@ def test_encoder_stacks_as_one_launch_have_inner_rows_as_wide_as_the_hidden_ones
         for dtype in (capi.F16, capi.BF16):
             capi.check(lib.ttmi_encoder_chain_workspace(2, 8, heads, heads * 64, ffn, dtype, ctypes.addressof(size)))
             assert (size.value > 0) == built, (heads, ffn)
+
+
+_WALK = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "chain_walk.h"
+// Workgroups of a chain, one round of waiting or one item a turn, in a random order; `resident` of them run at a time.  An item reads what the items of
+// the step before have written, which arrives up to three turns later; one of them (lost_step, lost_item) reads something that nobody writes.
+int main(int argc, char** argv) {
+  const int workgroups = atoi(argv[1]), resident = atoi(argv[2]), resumes = atoi(argv[3]), lost_step = atoi(argv[4]), lost_item = atoi(argv[5]);
+  srand(atoi(argv[6]));
+  const std::vector<int> counts = {5, 2, 7, 2, 5, 2, 7, 2, 1};
+  const int steps = (int)counts.size();
+  std::vector<std::vector<long>> written(steps);
+  for (int s = 0; s < steps; ++s) written[s].assign(counts[s], -1);
+  struct Workgroup {
+    ttmi::ChainWalk walk;
+    int seen = 0;
+    bool over = false, gave_up = false;
+  };
+  std::vector<Workgroup> all(workgroups);
+  auto items = [&](int s) { return counts[s]; };
+  long turns = 0;
+  int started = 0, over = 0, gave_up = 0;
+  std::vector<int> running;
+  while (over < workgroups) {
+    while ((int)running.size() < resident && started < workgroups) {
+      const int me = started++;
+      Workgroup& w = all[me];
+      auto first_item = [&](int s) { return (me + s) % workgroups; };
+      w.walk.item = me - workgroups;
+      w.walk.forward(workgroups, steps, items, first_item);
+      if (w.walk.step >= steps) ++over;
+      else running.push_back(me);
+    }
+    if (running.empty()) continue;
+    const int at = rand() % (int)running.size(), me = running[at];
+    Workgroup& w = all[me];
+    auto first_item = [&](int s) { return (me + s) % workgroups; };
+    const int s = w.walk.step;
+    bool there = !(s == lost_step && w.walk.item == lost_item);
+    for (int i = 0; s > 0 && i < counts[s - 1]; ++i) there = there && written[s - 1][i] >= 0 && written[s - 1][i] <= turns;
+    bool ends = false;
+    if (there) {
+      if (written[s][w.walk.item] < 0) written[s][w.walk.item] = turns + rand() % 4;
+      if (!w.walk.solo()) w.seen = s;
+      w.walk.executed(workgroups, steps, items, first_item);
+      ends = w.walk.step >= steps;
+    } else if (!w.walk.late(resumes ? w.seen : 0)) {
+      ends = true, ++gave_up;
+    }
+    if (ends) running.erase(running.begin() + at), ++over;
+    if (++turns > 20L * 1000 * 1000) return 3;
+  }
+  bool complete = true;
+  for (const auto& step : written)
+    for (long x : step) complete = complete && x >= 0;
+  printf("%d %d\n", gave_up, (int)complete);
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def walk(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("walk")
+    source, program = folder / "walk.cpp", folder / "walk"
+    source.write_text(_WALK)
+    device = os.path.join(os.path.dirname(capi.HEADER), "..", "turbotransformers_amd", "csrc", "device")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", device, str(source), "-o", str(program)], check=True)
+
+    def run(*args):
+        done = subprocess.run([str(program)] + [str(a) for a in args], capture_output=True, text=True, timeout=100)
+        assert done.returncode == 0, (args, done.returncode)  # (3: it would not have ended)
+        return [int(x) for x in done.stdout.split()]
+
+    return run
+
+
+@pytest.mark.parametrize("workgroups,resident", [(1, 1), (3, 1), (7, 2), (7, 7), (12, 5)])
+@pytest.mark.parametrize("resumes", [0, 1])
+def test_a_chain_of_steps_ends_whoever_is_resident(walk, workgroups, resident, resumes):
+    """Workgroups that wait in vain compute what they miss: nobody gives up, and everything is written.  resumes: from the last step whose inputs
+    were seen (encoder layers) or from the first (a decoder's blocks)."""
+    for seed in range(20):
+        assert walk(workgroups, resident, resumes, -1, -1, seed) == [0, 1]
+
+
+@pytest.mark.parametrize("workgroups,resident", [(1, 1), (3, 1), (7, 2), (7, 7), (12, 5)])
+@pytest.mark.parametrize("resumes", [0, 1])
+@pytest.mark.parametrize("lost", [(0, 3), (3, 1), (6, 6), (8, 0)])
+def test_a_chain_whose_item_reads_what_nobody_writes_ends_too(walk, workgroups, resident, resumes, lost):
+    """A mistake in a shape or a rule is an error, not a launch that never ends."""
+    gave_up, complete = walk(workgroups, resident, resumes, *lost, 1)
+    assert gave_up > 0 and not complete

@@ -9,6 +9,7 @@
 #pragma once
 
 #include "attention_common.h"
+#include "chain_walk.h"
 
 namespace ttmi {
 
@@ -21,7 +22,6 @@ constexpr uint32_t kUnwritten = 0xffffffffu, kOtherNaN = 0xfffefffeu;
 constexpr int kThroughMemory = 17;                 // cache policy sc0 | sc1: not from, and not into, the L2 of the XCD
 constexpr uint32_t kOutside = 0xffffff00u;         // an offset past every buffer: a load from there is zero
 constexpr int kChainPatience = 512;                // polls, of about a microsecond
-constexpr int kChainMostTries = 4096;
 
 __device__ __forceinline__ uint32_t storable(uint32_t word) { return word == kUnwritten ? kOtherNaN : word; }
 // The largest word so far: kUnwritten if one of them is.

@@ -125,13 +125,6 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     before %= G;
     return me >= before ? me - before : me - before + G;
   };
-  auto advance = [&](int& s, int& i) __attribute__((always_inline)) {
-    i += G;
-    while (s < STEPS && i >= items(s)) {
-      ++s;
-      if (s < STEPS) i = first_item(s);
-    }
-  };
   // All of the arguments are requested at once: where they lie a first read takes as long as an exchange.
   {
     const __attribute__((address_space(4))) uint32_t* words = reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(arguments());
@@ -148,16 +141,16 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     if (a.other != nullptr && me < fillers) fill_unwritten(a.other, a.bytes, me, fillers);
   };
 
-  int step = 0, item = first_item(0) - G;
-  advance(step, item);
-  if (step >= STEPS) return;  // (not of those that fill)
-  int resume_step = 0, resume_item = 0, tries = 0;
-  bool solo = false;
+  ChainWalk walk;
+  walk.item = first_item(0) - G;
+  walk.forward(G, STEPS, items, first_item);
+  if (walk.step >= STEPS) return;  // (not of those that fill)
   if (threadIdx.x == 0) missing = 0;
   __syncthreads();
 
   for (;;) {
     const Arguments& a = *arguments();
+    const int step = walk.step, item = walk.item;
     const int H = a.hidden, rows = a.rows, heads = a.heads, patience = a.patience;
     float* const part = reinterpret_cast<float*>(smem + kRows * chain_row_pitch(H, E));
     int tid = threadIdx.x;
@@ -395,12 +388,9 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     if (__builtin_amdgcn_readfirstlane(missing) != 0) {  // set in front of the barrier: the same for all
       __syncthreads();
       if (tid == 0) missing = 0;
-      if (!solo && step > 0) {
-        solo = true;
-        resume_step = step, resume_item = item;
-        step = 0, item = 0;
-      } else if (++tries > kChainMostTries) {  // (not reached: what an item reads this workgroup has written)
+      if (!walk.late(0)) {  // (not reached while every item's inputs are some item's outputs)
         if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
+        leave();
         return;
       }
       __syncthreads();
@@ -434,16 +424,10 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
         store_pair(context_at(a.width, E) + fragment_offset<T>(b, (pair - b * heads) * kD + col), v0, v1);
       }
     }
-    tries = 0;
-    if (!solo) {
-      advance(step, item);
-      if (step >= STEPS) {
-        leave();
-        return;
-      }
-    } else if (++item >= items(step)) {
-      item = 0;
-      if (++step == resume_step) item = resume_item, solo = false;
+    walk.executed(G, STEPS, items, first_item);
+    if (walk.step >= STEPS) {
+      leave();
+      return;
     }
     __syncthreads();  // the rows and partial tiles have been read
   }

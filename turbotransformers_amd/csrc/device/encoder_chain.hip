@@ -23,7 +23,7 @@
 // Progress does not depend on how many of the workgroups are resident.  Items are pure functions of the step before, and who executes an
 // item a second time writes the same bits.  A workgroup that has waited `patience` polls in vain (others hold the CUs, or the
 // grid is smaller than the items) executes the steps that it misses by itself, from the last one whose inputs it has seen, and
-// goes on; workgroups that start late find everything written.
+// goes on; workgroups that start late find everything written.  That ends whatever an item waits for (chain_walk.h): where nobody writes it, in an error.
 #include <mutex>
 #include <set>
 
@@ -128,24 +128,16 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     return me >= first ? me - first : me - first + G;
   };
   const int last_step = 4 * arguments()->layers;
-  auto advance = [&](int& s, int& i) __attribute__((always_inline)) {
-    i += G;
-    while (s <= last_step && i >= items(s)) {
-      ++s;
-      if (s <= last_step) i = first_item(s);
-    }
-  };
 
-  // The item at hand; while `solo` one of a step that others were to execute, on the way to (resume_step, resume_item).
   {
     const Arguments& a = *arguments();
     if (a.other != nullptr) fill_unwritten(a.other, (uint32_t)a.layers * a.layer_bytes, me, G);
   }
-  int step = 0, item = first_item(0) - G;
-  advance(step, item);
-  if (step > last_step) return;
-  int seen = 0, resume_step = 0, resume_item = 0, tries = 0;
-  bool solo = false;
+  ChainWalk walk;
+  walk.item = first_item(0) - G;
+  walk.forward(G, last_step + 1, items, first_item);
+  if (walk.step > last_step) return;
+  int seen = 0;  // the last step whose inputs the workgroup has seen
   if (threadIdx.x == 0) missing = 0;
   constexpr int WORDS = sizeof(ChainLayer) / 8;
   if ((int)threadIdx.x < arguments()->layers * WORDS)
@@ -159,6 +151,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
 
   for (;;) {
     const Arguments& a = *arguments();
+    const int step = walk.step, item = walk.item;
     const auto& at = a.at;
     const int H = a.hidden, F = a.ffn, rows = a.rows, patience = a.patience;
     const int pitch = chain_row_pitch(H);
@@ -431,11 +424,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     if (__builtin_amdgcn_readfirstlane(missing) != 0) {  // set in front of the barrier: the same for all
       __syncthreads();
       if (tid == 0) missing = 0;
-      if (!solo && seen < step) {
-        solo = true;
-        resume_step = step, resume_item = item;
-        step = seen, item = 0;
-      } else if (++tries > kChainMostTries) {  // (not reached: what an item reads has been written, or is being written by a workgroup that runs)
+      if (!walk.late(seen)) {  // (not reached while every item's inputs are some item's outputs)
         if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
         return;
       }
@@ -465,15 +454,9 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
         }
       }
     }
-    tries = 0;
-    if (!solo) {
-      seen = step;
-      advance(step, item);
-      if (step > last_step) return;
-    } else if (++item >= items(step)) {
-      item = 0;
-      if (++step == resume_step) item = resume_item, solo = false;
-    }
+    if (!walk.solo()) seen = step;
+    walk.executed(G, last_step + 1, items, first_item);
+    if (walk.step > last_step) return;
     __syncthreads();  // the rows and partial tiles have been read
   }
 #endif
