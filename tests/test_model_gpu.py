@@ -1121,6 +1121,57 @@ def test_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
         assert torch.equal(one_call, by_layer) and bool(torch.isfinite(one_call.float()).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("batch,seq", [(1, 1), (1, 10), (3, 5), (2, 8), (1, 16), (1, 17), (2, 16), (1, 33)])
+def test_a_stack_has_the_bits_of_its_layers(tt, dtype, batch, seq):
+    """Asked for in one call, with all hidden states, layer by layer, and in place."""
+    model, cfg = _hf_bert(3, seed=7)
+    encoder = tt.BertEncoder.from_torch(model.to(dtype).encoder)
+    turbo = tt.ReturnType.turbo_transformers
+    x = torch.randn(batch, seq, cfg.hidden_size, generator=torch.Generator().manual_seed(seq)).cuda().to(dtype)
+    mask = torch.zeros(batch, 1, 1, seq, device="cuda")
+    mask[-1, ..., (seq + 1) // 2:] = -10000.0
+    want = encoder(x, mask)[0].clone()
+    assert bool(torch.isfinite(want.float()).all())
+    last, states = encoder(x, mask, output_hidden_states=True)
+    assert torch.equal(last, want) and len(states) == 3
+    one = x
+    for layer in encoder.layer:
+        one = layer(one, mask, return_type=turbo)[0]
+    assert torch.equal(torch.utils.dlpack.from_dlpack(one.to_dlpack()), want)
+    from turbotransformers_amd.layers.utils import convert2tt_tensor
+    same = convert2tt_tensor(x.clone())
+    tt.cxx.run_bert_layers([(l.attention, l.intermediate, l.output) for l in encoder.layer], same, convert2tt_tensor(mask), same)
+    assert torch.equal(torch.utils.dlpack.from_dlpack(same.to_dlpack()), want)
+
+
+@pytest.mark.parametrize("shape", [(1, 10), (2, 8), (1, 17)])
+def test_a_short_forward_has_the_same_bits_in_a_plan_and_in_cxx(tt, tmp_path, shape):
+    """Few rows in fp16: where the activations have planned places (the layers' input and output the same one), and from the C++ model."""
+    from turbotransformers_amd.convert_huggingface_bert_to_npz import bert_to_npz_arrays
+    model, cfg = _hf_bert(3, seed=5)
+    model = model.half()
+    path = str(tmp_path / "bert.npz")
+    np.savez(path, **{name: value.astype(np.float16) for name, value in bert_to_npz_arrays(model).items()})
+    cxx_model = tt.cxx.CxxBertModel(path, cfg.num_hidden_layers, cfg.num_attention_heads)
+    tmodel = tt.BertModel.from_torch(model, torch.device("cuda:0"), "turbo")
+    ids = torch.randint(0, cfg.vocab_size, shape, generator=torch.Generator().manual_seed(3)).cuda()
+    want = [t.clone() for t in tmodel(ids)[:2]]
+    out = tt.cxx.Tensor.create_empty()
+    from turbotransformers_amd.layers.utils import convert2tt_tensor
+    cxx_model.encode(convert2tt_tensor(ids), out)
+    assert torch.equal(torch.utils.dlpack.from_dlpack(out.to_dlpack()), want[0])
+    try:
+        tt.reset_allocator_schema("model-aware")
+        tt.bert_opt_mem_allocate_api(ids.shape[0], ids.shape[1], cfg.num_attention_heads, cfg.hidden_size, cfg.num_hidden_layers, "GPU")
+        for _ in range(2):
+            got = tmodel(ids)[:2]
+            torch.cuda.synchronize()
+            assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    finally:
+        tt.reset_allocator_schema("naive")
+
+
 @pytest.mark.parametrize("dtype,layers", [(torch.float32, 3), (torch.float16, 9), (torch.bfloat16, 9)])
 def test_packed_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
     """The same for packed batches, each twice: few requests, twenty of 5 to 500 tokens (which start with the longest, and leave room to read

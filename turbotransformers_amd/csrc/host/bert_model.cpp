@@ -68,6 +68,7 @@ struct BertModel::Impl {
     (*embedding_)(ids, *position_ids, *seq_type, hidden);
     std::vector<layers::EncoderLayer<layers::BertAttention>> subs;
     for (auto& layer : encoders_) subs.push_back({layer.attention_.get(), layer.intermediate_.get(), layer.output_.get()});
+    if (layers::RunEncoderChain(subs, *hidden, ext, hidden)) return;  // (the bits of run_bert_layers, for few rows too)
     const auto ahead = layers::WeightsAhead(subs, *hidden);
     for (size_t i = 0; i < encoders_.size(); ++i) encoders_[i](*hidden, ext, &att_out_, &intermediate_out_, hidden, ahead[i], encoders_[0].attention_.get());
   }

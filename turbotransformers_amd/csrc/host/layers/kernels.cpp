@@ -232,6 +232,11 @@ void AddBiasLayerNormWithAbsmax(const Tensor& input_tensor, const Tensor& bias_t
   if (written == 0) out_tensor->DropAbsmax();
 }
 
+bool Overlap(const Tensor& a, const Tensor& b) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a.raw()), y = reinterpret_cast<uintptr_t>(b.raw());
+  return x < y + (uintptr_t)b.numel() * b.element_size() && y < x + (uintptr_t)a.numel() * a.element_size();
+}
+
 bool KeepsFp32Residual(const Tensor& t) { return core::ToDeviceDType(t.dtype()) == TTMI_BF16; }
 
 void AddBiasLayerNormResidual(const Tensor& input_tensor, const Tensor& bias_tensor, const Tensor& gamma_tensor,

@@ -577,14 +577,22 @@ bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, con
   if ((bits & 15) != 0) return false;
   const DLDeviceType dev = hidden.device_type();
   const int dev_id = hidden.device_id();
-  out->ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
-  void* const result = out->mutable_raw();
-  float* const result32 = kernels::KeepsFp32Residual(*out) ? out->EnsureShadow()->mutableData<float>() : nullptr;
-  if (reinterpret_cast<uintptr_t>(result) % 16 != 0 || result == hidden.raw()) return false;  // (a workgroup that starts late reads the input late)
+  // A workgroup that starts late reads the input late: where the result would lie over it (the same tensor, or one place in a plan for both) it gets
+  // memory of its own, so that a call has the bits that it has elsewhere.
+  Tensor apart(nullptr);
+  Tensor* target = out;
+  if (out == &hidden) target = &apart;
+  else out->ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
+  if (target == out && kernels::Overlap(*out, hidden)) target = &apart;
+  if (target == &apart) apart.ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "chain/out");
+  void* const result = target->mutable_raw();
+  float* const result32 = kernels::KeepsFp32Residual(*target) ? target->EnsureShadow()->mutableData<float>() : nullptr;
+  if (reinterpret_cast<uintptr_t>(result) % 16 != 0) return false;
   first.exchange().Use(bytes, dev, dev_id, [&](void* memory, int turn) {
     TT_DEVICE_CALL(ttmi_encoder_chain(parameters.data(), hidden.raw(), input32, additive, result, result32, memory, turn, count, batch, seq, heads, width,
                                       ffn, 1e-12f, dt, 0, 0, Stream()));
   });
+  if (target == &apart) *out = std::move(apart);
   return true;
 }
 

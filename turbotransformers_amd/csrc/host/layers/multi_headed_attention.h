@@ -200,9 +200,10 @@ struct EncoderLayer {
   const BertOutput* output;
 };
 // The whole stack as one launch (ttmi_encoder_chain) for up to 16 rows in 16-bit types: a block of the matrix instruction, and one row for each
-// of a workgroup's sixteen wavefronts to normalise.  (A form of two blocks, us per forward layer by layer / as one launch: fp16 base 1 x 17 305 / 263, 1 x 32 304 / 277,
-// bf16 large 2 x 16 720 / 689: the gain goes as the rows do, and there a stack gives the bits that its layers give one by one.)  false: nothing was done.  `hidden` [batch,seq,H], `mask` additive
-// fp32 per key or empty.
+// of a workgroup's sixteen wavefronts to normalise.  A stack has the bits of its layers run so one by one, whose sums differ from those of the
+// sub-layers' own launches: whoever runs whole layers comes here (a stack, a layer of it, the C++ model), so that a model's result does not depend on how it is
+// asked for.  (A form of two blocks, us per forward layer by layer / as one launch: fp16 base 1 x 17 305 / 263, 1 x 32 304 / 277, bf16 large 2 x 16 720 /
+// 689, is not built.)  false: nothing was done.  `hidden` [batch,seq,H], `mask` additive fp32 per key or empty; `out` may be `hidden` or lie over it.
 bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, const core::Tensor& hidden, const core::Tensor& mask,
                      core::Tensor* out);
 

@@ -133,15 +133,31 @@ class BertAttention(cxx.BertAttention):
             'output.LayerNorm.bias')), num_attention_heads)
 
 
+def _run_layers(layers, hidden_states, attention_mask):
+    """Layers built from the three stock sub-layers, one after the other inside the extension; -> the last hidden state."""
+    use_current_stream()
+    last = cxx.Tensor.create_empty()
+    cxx.run_bert_layers([(l.attention, l.intermediate, l.output) for l in layers], try_convert(hidden_states),
+                        try_convert(create_empty_if_none(attention_mask)), last)
+    return last
+
+
 class BertLayer:
     def __init__(self, attention: BertAttention, intermediate: BertIntermediate, output: BertOutput):
         self.attention = attention
         self.intermediate = intermediate
         self.output = output
 
+    def _plain(self):
+        """Whether the sub-layers are the three stock ones (then the extension may run the layer)."""
+        return type(self.attention) is BertAttention and type(self.intermediate) is BertIntermediate and type(self.output) is BertOutput
+
     def __call__(self, hidden_states: AnyTensor, attention_mask: Optional[AnyTensor] = None,
                  head_mask: Optional[AnyTensor] = None, output_attentions=False,
                  return_type: Optional[ReturnType] = None):
+        if not output_attentions and head_mask is None and self._plain():
+            # as a stack of one, so that layers called one by one give the bits of the stack
+            return (convert_returns_as_type(_run_layers([self], hidden_states, attention_mask), return_type), )
         attn_out = self.attention(hidden_states, attention_mask, head_mask, output_attentions=output_attentions,
                                   return_type=ReturnType.turbo_transformers)
         attention_output = attn_out[0]
@@ -173,11 +189,7 @@ class BertEncoder:
         attention_mask = try_convert(attention_mask)
         if not output_attentions and not output_hidden_states and self._plain_layers():
             # nothing but the last hidden state is asked for: the layer loop runs inside the extension
-            use_current_stream()
-            last = cxx.Tensor.create_empty()
-            cxx.run_bert_layers([(l.attention, l.intermediate, l.output) for l in self.layer], hidden_states,
-                                create_empty_if_none(attention_mask), last)
-            return (convert_returns_as_type(last, return_type), )
+            return (convert_returns_as_type(_run_layers(self.layer, hidden_states, attention_mask), return_type), )
         for layer in self.layer:
             layer_outputs = layer(hidden_states=hidden_states, attention_mask=attention_mask,
                                   output_attentions=output_attentions, return_type=ReturnType.turbo_transformers)
@@ -196,9 +208,7 @@ class BertEncoder:
 
     def _plain_layers(self):
         """Whether every layer is a BertLayer built from the three stock sub-layers (then the C++ loop may run them)."""
-        return len(self.layer) > 0 and all(
-            type(l) is BertLayer and type(l.attention) is BertAttention and type(l.intermediate) is BertIntermediate
-            and type(l.output) is BertOutput for l in self.layer)
+        return len(self.layer) > 0 and all(type(l) is BertLayer and l._plain() for l in self.layer)
 
     @staticmethod
     def from_torch(encoder):
