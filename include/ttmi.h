@@ -529,7 +529,8 @@ TTMI_API int ttmi_dequant_bias(const int32_t* acc, const float* act_scale_dev, c
  *   weights    HOST list of 12 device pointers per layer: qkv weight [3H,H] and bias, output weight [H,H] and bias, LayerNorm gamma and beta,
  *              FFN1 weight [F,H] and bias, FFN2 weight [H,F] and bias, LayerNorm gamma and beta (all weights [out,in])
  *   input      [batch,seq,H]; input32: the same before rounding (bf16: the residual is taken from it), or null
- *   mask       additive fp32 [batch,seq] per key, or null;  out [batch,seq,H];  out32: bf16, the unrounded result, or null
+ *   mask       additive fp32 [batch,seq] per key, or null;  out [batch,seq,H];  out32: bf16, the unrounded result, or null;
+ *              neither may share memory with input, input32, mask or the other
  *   exchange   as many bytes as ttmi_encoder_chain_workspace says, 16-byte aligned, prepared once by ttmi_chain_prepare and used by one call
  *              after the other on one stream
  *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed
@@ -553,7 +554,7 @@ TTMI_API int ttmi_encoder_chain(const void* const* weights, const void* input, c
  *                            probs [rows,heads,keys] = softmax(scale q k^T + mask), mask additive fp32 [rows,keys] or null;
  *                            out = x + (probs v) w_out^T + b_out.  hidden = 64 * heads, up to 512 keys.
  * ttmi_decoder_feed_forward  out = x + relu(LN(x) w1^T + b1) w2^T + b2; inner a multiple of 64 up to 4096 (fp32: 3072).
- *   weights [out,in]; out must be another tensor than x
+ *   weights [out,in]; results must share no memory with x, the cache, the mask or each other
  *   exchange   as many bytes as ttmi_decoder_chain_workspace says (heads = 0: feed-forward; inner: 3 * hidden or hidden for attention; 0: not
  *              built), prepared once by ttmi_chain_prepare and used by one call after the other on one stream
  *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed

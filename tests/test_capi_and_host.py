@@ -574,3 +574,57 @@ def test_a_chain_whose_item_reads_what_nobody_writes_ends_too(walk, workgroups, 
     """A mistake in a shape or a rule is an error, not a launch that never ends."""
     gave_up, complete = walk(workgroups, resident, resumes, *lost, 1)
     assert gave_up > 0 and not complete
+
+
+def _refused(rc):
+    return rc == -1 and b"must share no memory" in capi.load().ttmi_last_error()
+
+
+@pytest.mark.parametrize("dtype", [capi.F16, capi.BF16])
+def test_a_stack_as_one_launch_refuses_a_result_over_what_it_reads(dtype):
+    """Addresses only: the check stands in front of every device call.  A workgroup that starts late reads its input late."""
+    lib = capi.load()
+    rows, hidden = 10, 768
+    weights = (ctypes.c_void_p * 12)(*[0x10000 * (i + 1) for i in range(12)])
+    x, x32, mask, out, out32, memory = (0x40000000 + 0x100000 * i for i in range(6))
+    good = dict(x=x, x32=x32, mask=mask, out=out, out32=out32)
+
+    def call(**places):
+        p = dict(good, **places)
+        return lib.ttmi_encoder_chain(ctypes.addressof(weights), p["x"], p["x32"], p["mask"], p["out"], p["out32"], memory, 3, 1, 1, rows, 12, hidden, 3072, 1e-12,
+                                      dtype, 0, 0, None)
+
+    assert not _refused(call())  # (stopped by the turn, 3)
+    assert not _refused(call(out=x + rows * hidden * 2)) and not _refused(call(x32=None, mask=None, out32=None))
+    for places in (dict(out=x), dict(out=x + rows * hidden * 2 - 16), dict(out=x32 + 16), dict(out=mask), dict(out32=x), dict(out32=x32), dict(out32=mask - 16),
+                   dict(out32=out), dict(out32=out + rows * hidden * 2 - 16)):
+        assert _refused(call(**places)), places
+
+
+@pytest.mark.parametrize("grows", [True, False])
+def test_a_decoder_block_as_one_launch_refuses_results_over_what_it_reads_or_each_other(grows):
+    lib = capi.load()
+    rows, heads, hidden, keys = 8, 12, 768, 41
+    names = ["x", "gamma", "beta", "w_in", "b_in", "w_out", "b_out", "k_past", "v_past", "k_out", "v_out", "mask", "probs", "out"]
+    good = {n: 0x40000000 + 0x1000000 * i for i, n in enumerate(names)}
+    if not grows:
+        good.update(k_out=None, v_out=None)
+
+    def call(**places):
+        p = dict(good, **places)
+        return lib.ttmi_decoder_attention(p["x"], p["gamma"], p["beta"], 1e-6, p["w_in"], p["b_in"], p["w_out"], p["b_out"], p["k_past"], p["v_past"], p["k_out"],
+                                          p["v_out"], p["mask"], p["probs"], p["out"], 0x10000, 3, rows, heads, hidden, keys, 0.125, capi.F16, 0, 0, None)
+
+    assert not _refused(call()) and not _refused(call(mask=None))
+    places = [dict(out=good["x"]), dict(out=good["x"] + rows * hidden * 2 - 16), dict(out=good["probs"]), dict(probs=good["x"] + 16), dict(probs=good["mask"]),
+              dict(out=good["v_past"] + 16), dict(probs=good["k_past"])]
+    if grows:
+        places += [dict(k_out=good["k_past"]), dict(v_out=good["k_past"]), dict(k_out=good["v_out"]), dict(out=good["k_out"]), dict(probs=good["v_out"] + 2)]
+    for p in places:
+        assert _refused(call(**p)), p
+
+    def block(x, out):
+        return lib.ttmi_decoder_feed_forward(x, 0x20000, 0x30000, 1e-12, 0x1000000, 0x40000, 0x2000000, 0x50000, out, 0x10000, 3, rows, hidden, 3072, capi.F16, 0, 0,
+                                             None)
+
+    assert not _refused(block(0x60000, 0x80000)) and _refused(block(0x60000, 0x60000)) and _refused(block(0x60000, 0x60010))

@@ -1106,6 +1106,44 @@ def test_feed_forward_calls_handled_by_the_extension(tt, monkeypatch, form, bloc
     assert not any(handled[1:])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("how", ["plan", "in place"])
+def test_decoder_blocks_have_the_same_bits_where_results_lie_over_inputs(tt, dtype, how):
+    """A step's blocks in a plan that was made for an encoder, where results share places with what they are made of, and with
+    the result written to the input's tensor."""
+    B, heads, H, past = 8, 12, 768, 40
+    turbo, empty = tt.ReturnType.turbo_transformers, tt.cxx.Tensor.create_empty
+    from turbotransformers_amd.layers.utils import convert2tt_tensor
+    mha = [_make_mha(tt, heads, H, dtype=dtype, seed=s)[2] for s in (1, 2)]
+    ffn = tt.PositionwiseFeedForward.from_onmt(_OnmtLikeFfn(H, 3072).cuda().to(dtype))
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(B, 1, H, generator=gen).cuda().to(dtype)
+    keys, values = [torch.randn(B, heads, past, 64, generator=gen).cuda().to(dtype) for _ in range(2)]
+    to_torch = lambda t: torch.utils.dlpack.from_dlpack(t.to_dlpack()).clone()
+
+    def step(in_place):
+        cache = {"memory_keys": keys, "memory_values": values, "self_keys": keys, "self_values": values}
+        y, probs = convert2tt_tensor(x.clone()), []
+        for layer, kind in zip(mha, ("self", "context")):
+            out, p = layer(y, y, y, None, cache, kind, pre_layernorm=True, post_add_input=True, return_type=turbo, output=y if in_place else empty(), attn=empty())
+            probs.append(to_torch(p))
+            y = out
+        y = ffn(y, return_type=turbo, output=y if in_place else empty())
+        return [to_torch(y), cache["self_keys"].clone(), cache["self_values"].clone()] + probs
+
+    want = step(False)
+    if how == "in place":
+        got = step(True)
+    else:
+        try:
+            tt.reset_allocator_schema("model-aware")
+            tt.bert_opt_mem_allocate_api(B, past + 1, heads, H, 1, "GPU")
+            got = step(False)
+        finally:
+            tt.reset_allocator_schema("naive")
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("dtype,layers", [(torch.float32, 5), (torch.float16, 9)])
 def test_layer_loop_of_weights_beyond_the_cache(tt, dtype, layers):
     """Weights of more than the last-level cache holds are read ahead in the layer loop: the same bits as layer by layer, on the first

@@ -8,6 +8,8 @@
 // barrier over the grid with counters 4 to 5.
 #pragma once
 
+#include <initializer_list>
+
 #include "attention_common.h"
 #include "chain_walk.h"
 
@@ -115,6 +117,25 @@ inline int launch_unwritten(void* p, int64_t bytes, hipStream_t s) {
   hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * compute_units())), dim3(256), 0, s, static_cast<u32x4*>(p),
                      bytes / 16);
   return launch_status("unwritten_kernel");
+}
+// A result of a chain, or what it reads while results are written.
+struct Extent {
+  const void* at;
+  int64_t bytes;
+};
+// A workgroup that starts late reads late: whether no result shares a byte with what is read, or with another result.
+inline bool results_apart(std::initializer_list<Extent> results, std::initializer_list<Extent> reads) {
+  auto share = [](const Extent& a, const Extent& b) {
+    const uintptr_t x = reinterpret_cast<uintptr_t>(a.at), y = reinterpret_cast<uintptr_t>(b.at);
+    return x != 0 && y != 0 && x < y + (uintptr_t)b.bytes && y < x + (uintptr_t)a.bytes;
+  };
+  for (const Extent& r : results) {
+    for (const Extent& o : results)
+      if (&o != &r && share(r, o)) return false;
+    for (const Extent& o : reads)
+      if (share(r, o)) return false;
+  }
+  return true;
 }
 // The part of a launch, and the one that it fills for the next.
 inline int take_part(void* exchange, int64_t bytes, int turn, char** mine, char** other, hipStream_t s) {

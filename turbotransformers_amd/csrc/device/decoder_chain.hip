@@ -513,7 +513,9 @@ int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta
   TTMI_REQUIRE(bytes > 0 && workgroups >= 0 && patience >= 0, "this block is not run as one launch");
   uintptr_t bits = 0;
   for (const void* p : {x, gamma, beta, w1, b1, w2, b2, (const void*)out, (const void*)exchange}) bits |= reinterpret_cast<uintptr_t>(p);
-  TTMI_REQUIRE((bits & 15) == 0 && x != out, "tensors must be 16-byte aligned, and out another one than x");
+  TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
+  const int64_t e = (int64_t)dtype_size(dtype);
+  TTMI_REQUIRE(results_apart({{out, rows * hidden * e}}, {{x, rows * hidden * e}}), "out must share no memory with x");
   DecoderArgs a{};
   a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w1, a.b_in = b1, a.w_out = w2, a.b_out = b2, a.out = out;
   a.rows = (int)rows, a.hidden = (int)hidden, a.width = (int)inner, a.inner = (int)inner, a.eps = eps, a.heads = 1;
@@ -540,7 +542,11 @@ int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, f
   uintptr_t bits = 0;
   for (const void* p : {x, gamma, beta, w_in, b_in, w_out, b_out, k_past, v_past, (const void*)k_out, (const void*)v_out, (const void*)out, (const void*)exchange})
     bits |= reinterpret_cast<uintptr_t>(p);
-  TTMI_REQUIRE((bits & 15) == 0 && x != out, "tensors must be 16-byte aligned, and out another one than x");
+  TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
+  const int64_t e = (int64_t)dtype_size(dtype), values = rows * hidden * e;
+  TTMI_REQUIRE(results_apart({{out, values}, {probs, rows * heads * keys * e}, {k_out, values * keys}, {v_out, values * keys}},
+                             {{x, values}, {k_past, values * past}, {v_past, values * past}, {mask, rows * keys * 4}}),
+               "the results must share no memory with x, the cache, the mask or each other");
   DecoderArgs a{};
   a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w_in, a.b_in = b_in, a.w_out = w_out, a.b_out = b_out, a.out = out;
   a.k_past = k_past, a.v_past = v_past, a.k_out = k_out, a.v_out = v_out, a.mask = mask, a.probs = probs;

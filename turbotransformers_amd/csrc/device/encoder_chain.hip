@@ -502,6 +502,9 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
     a.layer[l] = {w[0], w[1], w[2], w[3], w[4], w[5], w[6], w[7], w[8], w[9], w[10], w[11]};
   }
   TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
+  const int64_t values = rows * hidden;
+  TTMI_REQUIRE(results_apart({{out, values * 2}, {out32, values * 4}}, {{input, values * 2}, {input32, values * 4}, {mask, rows * 4}}),
+               "out and out32 must share no memory with input, input32, mask or each other");
   const int cus = compute_units();
   a.input = input, a.input32 = input32, a.mask = mask, a.out = out, a.out32 = out32;
   a.layer_bytes = (uint32_t)(bytes / 3 / layers);

@@ -168,16 +168,20 @@ bool PositionwiseFeedForward::AsOneLaunch(const Tensor& input_tensor, Tensor* ou
   const void* w2 = packed2_.Get(dense_weight_2_, is_trans_weight).data;
   const DLDeviceType dev = input_tensor.device_type();
   const int id = input_tensor.device_id();
-  output->ReshapeAs(input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev, id, "FFN/Reshape");
-  void* const out = output->mutable_raw();
-  uintptr_t bits = reinterpret_cast<uintptr_t>(out);
+  uintptr_t bits = 0;
   for (const void* p : {input_tensor.raw(), layer_norm_weight_.raw(), layer_norm_bias_.raw(), w1, dense_bias_1_.raw(), w2, dense_bias_2_.raw()})
     bits |= reinterpret_cast<uintptr_t>(p);
-  if ((bits & 15) != 0 || out == input_tensor.raw()) return false;
+  if ((bits & 15) != 0) return false;
+  Tensor apart(nullptr);
+  Tensor* const target = kernels::ResultBeside(output, {&input_tensor}, &apart, input_tensor.dtype(), {input_tensor.shape(0), input_tensor.shape(1), model_dim}, dev,
+                                               id, "FFN/Reshape");
+  void* const out = target->mutable_raw();
+  if (reinterpret_cast<uintptr_t>(out) % 16 != 0) return false;
   exchange_.Use(bytes, dev, id, [&](void* memory, int turn) {
     TT_DEVICE_CALL(ttmi_decoder_feed_forward(input_tensor.raw(), layer_norm_weight_.raw(), layer_norm_bias_.raw(), 1e-12f, w1, dense_bias_1_.raw(), w2,
                                              dense_bias_2_.raw(), out, memory, turn, rows, model_dim, d_ff, dt, 0, 0, Stream()));
   });
+  if (target != output) *output = std::move(apart);
   return true;
 }
 

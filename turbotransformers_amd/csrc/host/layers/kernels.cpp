@@ -237,6 +237,19 @@ bool Overlap(const Tensor& a, const Tensor& b) {
   return x < y + (uintptr_t)b.numel() * b.element_size() && y < x + (uintptr_t)a.numel() * a.element_size();
 }
 
+Tensor* ResultBeside(Tensor* t, std::initializer_list<const Tensor*> others, Tensor* apart, DLDataType dtype, const std::vector<int64_t>& shape,
+                     DLDeviceType device_type, int device_id, const char* name) {
+  bool over = false;
+  for (const Tensor* o : others) over = over || o == t;
+  if (!over) {
+    t->ReshapeAs(dtype, shape, device_type, device_id, name);
+    for (const Tensor* o : others) over = over || (!o->is_null() && Overlap(*t, *o));
+  }
+  if (!over) return t;
+  apart->ReshapeAs(dtype, shape, device_type, device_id, "chain/result");
+  return apart;
+}
+
 bool KeepsFp32Residual(const Tensor& t) { return core::ToDeviceDType(t.dtype()) == TTMI_BF16; }
 
 void AddBiasLayerNormResidual(const Tensor& input_tensor, const Tensor& bias_tensor, const Tensor& gamma_tensor,

@@ -14,6 +14,7 @@
 //   kernels/seq_pool.h                     SeqPool
 #pragma once
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -93,6 +94,10 @@ void AddBiasLayerNormResidual(const core::Tensor& input_tensor, const core::Tens
 void AddBiasLayerNormWithAbsmax(const core::Tensor& input_tensor, const core::Tensor& bias_tensor, const core::Tensor& gamma_tensor,
                                 const core::Tensor& beta_tensor, core::Tensor* out_tensor, float eps);
 bool Overlap(const core::Tensor& a, const core::Tensor& b);  // whether the two share a byte
+// Shapes `t` for a result that is written while `others` are read or written; -> it, or where it would lie over one of them (the same tensor, or places of
+// one plan that were not meant to be live together) `apart`, in memory of its own, which the caller moves into `t` afterwards.
+core::Tensor* ResultBeside(core::Tensor* t, std::initializer_list<const core::Tensor*> others, core::Tensor* apart, DLDataType dtype,
+                           const std::vector<int64_t>& shape, DLDeviceType device_type, int device_id, const char* name);
 bool KeepsFp32Residual(const core::Tensor& t);  // true for bfloat16 tensors
 // out = AddBiasLayerNorm(in . w^T, residual) with the same treatment of the residual; `w_nk` is the
 // [n, k] weight on the device, `out_tensor` already has its [.., n] shape.

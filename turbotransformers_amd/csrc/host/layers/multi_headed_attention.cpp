@@ -248,10 +248,13 @@ bool MultiHeadedAttention::AsOneLaunch(const Tensor& query_tensor, const Tensor&
   uintptr_t bits = 0;
   for (const void* p : {query_tensor.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw(), w_in, in_bias.raw(), w_out, dense_bias_.raw(), k_past.raw(), v_past.raw()})
     bits |= reinterpret_cast<uintptr_t>(p);
-  output->ReshapeAs(query_tensor.dtype(), {batch, 1, hidden}, dev, dev_id, "gemm5/Reshape");
-  void* const out = output->mutable_raw();
-  if (((bits | reinterpret_cast<uintptr_t>(out)) & 15) != 0 || out == query_tensor.raw()) return false;
-  att_score->ReshapeAs(query_tensor.dtype(), {batch, heads, 1, keys}, dev, dev_id, "batch_gemm3/Reshape");
+  if ((bits & 15) != 0) return false;
+  Tensor out_apart(nullptr), probs_apart(nullptr);
+  Tensor* const out = kernels::ResultBeside(output, {&query_tensor, &attention_mask, &k_past, &v_past}, &out_apart, query_tensor.dtype(), {batch, 1, hidden},
+                                            dev, dev_id, "gemm5/Reshape");
+  Tensor* const probs = kernels::ResultBeside(att_score, {&query_tensor, &attention_mask, &k_past, &v_past, out}, &probs_apart, query_tensor.dtype(),
+                                              {batch, heads, 1, keys}, dev, dev_id, "batch_gemm3/Reshape");
+  if (reinterpret_cast<uintptr_t>(out->raw()) % 16 != 0) return false;
   Tensor k_grown(nullptr), v_grown(nullptr);
   if (is_self) {
     k_grown.ReshapeAs(query_tensor.dtype(), {batch, heads, keys, hidden / heads}, dev, dev_id, "self/self_key/Reshape");
@@ -260,9 +263,11 @@ bool MultiHeadedAttention::AsOneLaunch(const Tensor& query_tensor, const Tensor&
   exchange_.Use(bytes, dev, dev_id, [&](void* memory, int turn) {
     TT_DEVICE_CALL(ttmi_decoder_attention(query_tensor.raw(), layernorm_gamma_.raw(), layernorm_beta_.raw(), 1e-6f, w_in, in_bias.raw(), w_out,
                                           dense_bias_.raw(), k_past.raw(), v_past.raw(), is_self ? k_grown.mutable_raw() : nullptr,
-                                          is_self ? v_grown.mutable_raw() : nullptr, mask, att_score->mutable_raw(), out, memory, turn, batch, heads, hidden,
+                                          is_self ? v_grown.mutable_raw() : nullptr, mask, probs->mutable_raw(), out->mutable_raw(), memory, turn, batch, heads, hidden,
                                           keys, 1.0f / std::sqrt(static_cast<float>(hidden / heads)), dt, 0, 0, Stream()));
   });
+  if (out != output) *output = std::move(out_apart);
+  if (probs != att_score) *att_score = std::move(probs_apart);
   if (is_self) {
     *layer_cache.at(key_name) = std::move(k_grown);
     *layer_cache.at(value_name) = std::move(v_grown);
@@ -580,11 +585,7 @@ bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, con
   // A workgroup that starts late reads the input late: where the result would lie over it (the same tensor, or one place in a plan for both) it gets
   // memory of its own, so that a call has the bits that it has elsewhere.
   Tensor apart(nullptr);
-  Tensor* target = out;
-  if (out == &hidden) target = &apart;
-  else out->ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
-  if (target == out && kernels::Overlap(*out, hidden)) target = &apart;
-  if (target == &apart) apart.ReshapeAs(hidden.dtype(), {batch, seq, width}, dev, dev_id, "chain/out");
+  Tensor* const target = kernels::ResultBeside(out, {&hidden, &mask}, &apart, hidden.dtype(), {batch, seq, width}, dev, dev_id, "BERTEmbedding/Reshape");
   void* const result = target->mutable_raw();
   float* const result32 = kernels::KeepsFp32Residual(*target) ? target->EnsureShadow()->mutableData<float>() : nullptr;
   if (reinterpret_cast<uintptr_t>(result) % 16 != 0) return false;
@@ -592,7 +593,7 @@ bool RunEncoderChain(const std::vector<EncoderLayer<BertAttention>>& layers, con
     TT_DEVICE_CALL(ttmi_encoder_chain(parameters.data(), hidden.raw(), input32, additive, result, result32, memory, turn, count, batch, seq, heads, width,
                                       ffn, 1e-12f, dt, 0, 0, Stream()));
   });
-  if (target == &apart) *out = std::move(apart);
+  if (target != out) *out = std::move(apart);
   return true;
 }
 
