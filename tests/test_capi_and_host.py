@@ -628,3 +628,10 @@ def test_a_decoder_block_as_one_launch_refuses_results_over_what_it_reads_or_eac
                                              None)
 
     assert not _refused(block(0x60000, 0x80000)) and _refused(block(0x60000, 0x60000)) and _refused(block(0x60000, 0x60010))
+
+
+@pytest.mark.parametrize("hidden,inner,element,one", [(256, 1024, 2, True), (1024, 4096, 2, True), (64, 64, 2, True), (768, 3072, 4, True), (1024, 3072, 4, True),
+                                                      (1024, 2048, 4, False), (768, 768, 4, False), (512, 2048, 4, False), (256, 3072, 4, False), (64, 256, 4, False)])
+def test_feed_forward_blocks_run_as_one_launch_where_that_was_measured_to_gain(hidden, inner, element, one):
+    from turbotransformers_amd import cxx
+    assert cxx.feed_forward_runs_as_one_launch(hidden, inner, element) is one

@@ -22,7 +22,8 @@
 // together, nothing by wavefronts without a share: 8 sequences 188 / 178, 4 180 / 169, 1 159 / 151, 16 218 / 214; fp32 level to 1%.
 // fp32 multiplies in fp32 (four instructions where 16 bits take one, the weights as they are, not their halves) and reads and exchanges twice the bytes.  Its
 // error against 64 bits, rms after six layers, was 3.64 to 4.44e-7 with the split products and is 3.61 to 4.41e-7, that of the probabilities 11% less.
-// Rows of 4096 products would not fit its registers: the feed-forward block goes to 3072 there.
+// Rows of 4096 products would not fit its registers: the feed-forward block goes to 3072 there (128 of them, no scratch).  Where it pays stands at
+// FeedForwardRunsAsOneLaunch.
 // Measured and no better: a wavefront normalises the columns that it multiplies, of all rows (parameters read once a CU, no rows in LDS, but 12 loads more
 // a wavefront): fp32 8 sequences 274 / 302, fp16 8 188 / 196, 16 x 251 262 / 258; rows and parameters requested in front of the weights: fp32 274 / 281 to
 // 286, 1 x 6 226 / 242 to 245.

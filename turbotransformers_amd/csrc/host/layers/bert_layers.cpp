@@ -155,7 +155,9 @@ static void CheckFfn(const Tensor& input, const Tensor& w1, const Tensor& b1, co
   TT_ENFORCE(core::SameDataType(input.dtype(), w1.dtype()), "input and weights must share one element type");
 }
 
-// A token each of a few sequences (ttmi_decoder_feed_forward); false: nothing was done.
+bool FeedForwardRunsAsOneLaunch(int64_t hidden, int64_t inner, int64_t element_size) { return element_size == 2 || hidden * inner >= 768 * 3072; }
+
+// A few rows (ttmi_decoder_feed_forward); false: nothing was done.
 bool PositionwiseFeedForward::AsOneLaunch(const Tensor& input_tensor, Tensor* output, bool is_trans_weight) const {
   const int64_t rows = input_tensor.shape(0) * input_tensor.shape(1), model_dim = input_tensor.shape(2);
   const int dt = kernels::DeviceDType(input_tensor);
@@ -163,7 +165,7 @@ bool PositionwiseFeedForward::AsOneLaunch(const Tensor& input_tensor, Tensor* ou
   const int64_t d_ff = PackedWeight::OutDim(dense_weight_1_, is_trans_weight);
   int64_t bytes = 0;
   TT_DEVICE_CALL(ttmi_decoder_chain_workspace(rows, 0, model_dim, d_ff, 0, dt, &bytes));
-  if (bytes == 0 || layer_norm_weight_.numel() != model_dim || layer_norm_bias_.numel() != model_dim) return false;
+  if (bytes == 0 || !FeedForwardRunsAsOneLaunch(model_dim, d_ff, (int64_t)input_tensor.element_size()) || layer_norm_weight_.numel() != model_dim || layer_norm_bias_.numel() != model_dim) return false;
   const void* w1 = packed1_.Get(dense_weight_1_, is_trans_weight).data;
   const void* w2 = packed2_.Get(dense_weight_2_, is_trans_weight).data;
   const DLDeviceType dev = input_tensor.device_type();

@@ -104,6 +104,15 @@ class AlbertLayer {
   PackedWeight packed1_, packed2_;
 };
 
+// Whether the feed-forward block of a few rows runs as one launch (ttmi_decoder_feed_forward) where that is built.  In 16 bits always.  In fp32, where it
+// multiplies in fp32 instead of in halves, where the weights are large: what counts then is that they are requested in front of everything else.  us per
+// step of six decoder layers, two launches / one, 1 to 8 sequences of 40 keys: hidden x inner 768 x 3072 239 to 279 / 229 to 271, 1024 x 3072 262 to 314 / 256 to
+// 302; 16 sequences 311 / 310, 359 / 354; a first step of 4 and 16 tokens 358, 373 / 347, 372, 396, 419 / 384, 414.  Smaller ones lose: 256 x 1024 172 to 199 /
+// 175 to 205, 512 x 2048 201 to 229 / 206 to 236, 768 x 768 214 to 247 / 219 to 259; 1024 x 2048 gains up to 8 sequences, 248 to 295 / 244 to 290, and
+// loses from 16 rows on, 339 / 344, a first step 409 / 415.  (The block by itself, over and over, its weights in the cache, loses at 768 x 3072 too: six of 1, 8,
+// 16 rows 79, 80, 84 / 78, 84, 92.)
+bool FeedForwardRunsAsOneLaunch(int64_t hidden, int64_t inner, int64_t element_size);
+
 // Feed-forward blocks of the decoder / DistilBERT wrappers (positionwise_ffn.h:23-84).  Weights are
 // [in, out], or [out, in] when called with is_trans_weight.
 class PositionwiseFeedForward {

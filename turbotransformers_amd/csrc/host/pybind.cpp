@@ -463,6 +463,8 @@ PYBIND11_MODULE(turbo_transformers_cxx, m) {
         "(number of chunks, total bytes) held by the model-aware plan");
   m.def("weights_leave_cache", &layers::WeightsLeaveCache, py::arg("bytes"), py::arg("rows"), py::arg("width"), py::arg("ffn"), py::arg("element_size"),
         "Whether the layers of an encoder read their weights ahead, for tests.");
+  m.def("feed_forward_runs_as_one_launch", &layers::FeedForwardRunsAsOneLaunch, py::arg("hidden"), py::arg("inner"), py::arg("element_size"),
+        "Whether a decoder's feed-forward block of a few rows, where it is built as one launch, runs so, for tests.");
   // The planner as plain functions, for tests: records are (name, start_op, end_op, size).
   using Rec = std::tuple<std::string, int64_t, int64_t, int64_t>;
   auto to_records = [](const std::vector<Rec>& in) {
