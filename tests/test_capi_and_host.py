@@ -635,3 +635,14 @@ def test_a_decoder_block_as_one_launch_refuses_results_over_what_it_reads_or_eac
 def test_feed_forward_blocks_run_as_one_launch_where_that_was_measured_to_gain(hidden, inner, element, one):
     from turbotransformers_amd import cxx
     assert cxx.feed_forward_runs_as_one_launch(hidden, inner, element) is one
+
+
+@pytest.mark.parametrize("batch,seq,narrow", [(20, 100, True), (20, 200, True), (12, 460, True), (12, 500, True), (18, 464, False), (20, 440, False), (20, 480, False),
+                                              (24, 500, False), (32, 500, False), (20, 128, False), (16, 300, False)])
+def test_fp32_head_splits_take_the_tile_of_their_own_up_to_three_rounds(batch, seq, narrow):
+    """96 x 192 where 128 x 192 would leave a quarter of the compute units idle; beyond three rounds of workgroups that was measured to lose."""
+    lib = capi.load()
+    buf = ctypes.create_string_buffer(64)
+    args = capi.EpilogueArgs(bias=4096, q=4096, k=4096, v=4096, seq=seq, heads=12, head_dim=64, v_seq_pitch=(seq + 7) // 8 * 8)
+    capi.check(lib.ttmi_gemm_describe(batch * seq, 2304, 768, capi.EPI_QKV_SPLIT, ctypes.byref(args), capi.F32_PACKED, buf, 64))
+    assert ("96x192" in buf.value.decode()) == narrow, buf.value

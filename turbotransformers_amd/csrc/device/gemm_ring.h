@@ -626,8 +626,11 @@ struct RingPlan {
 
 // column_limit > 0: a wavefront's columns must not straddle it (the start of a transposed V), and its rows come in pairs of blocks (a
 // forward of fp16 base, without / with tiles of 160 rows there, 16 x 128 tokens 718 / 724 us, 20 x 100 733 / 736)
-// head_split: tiles of kHeadSplitRows rows are for it alone (below), and it has registers for kRingWidestSplit columns of a wavefront
-constexpr int kHeadSplitRows = 96, kRingWidestSplit = 128;
+// head_split: tiles of kHeadSplitRows rows are for it alone (above) and for up to kHeadSplitRounds workgroups a CU, and it has registers for kRingWidestSplit
+// columns of a wavefront.  Beyond, the launch is long enough that the chip runs at its power limit, which the model does not know: us per forward of base fp32,
+// without / with such tiles, 18 x 464 tokens 6019 / 6134, 20 x 440 6145 / 6259, 20 x 480 6445 / 6542, 24 x 500 8025 / 8088, 32 x 500 9872 / 10214; up to three
+// rounds 19 x 100 1529 / 1495, 20 x 200 2746 / 2628, 12 x 460 4229 / 4036, 12 x 500 4334 / 4199.
+constexpr int kHeadSplitRows = 96, kHeadSplitRounds = 3, kRingWidestSplit = 128;
 template <typename Epi>
 constexpr bool ring_takes(int rows, int wave_cols) { return HasColumnPass<Epi>::value ? wave_cols <= kRingWidestSplit : rows != kHeadSplitRows; }
 constexpr int kRingColumns = 32;  // the narrowest wavefront's: a limit that is no multiple of it suits no tile
@@ -664,6 +667,7 @@ inline RingPlan pick_tile_of(int64_t m, int64_t n, int64_t ksteps, RingUse use, 
     if (head_split ? t.wave_cols > kRingWidestSplit : t.bm == kHeadSplitRows) continue;
     if (column_limit > 0 && (column_limit % t.wave_cols != 0 || t.lone_block)) continue;
     const uint32_t tiles = (uint32_t)std::min<uint64_t>((uint64_t)((rows + t.bm - 1) / t.bm) * ((cols + t.bn - 1) / t.bn), kMostTiles);
+    if (t.bm == kHeadSplitRows && tiles > kHeadSplitRounds * cus) continue;
     const double least = t.first + steps * t.shared * (double)tiles / cus;
     uint32_t room = 0, q = 0;  // room: q workgroups on every CU
     for (uint32_t s = 1; s <= most; ++s) {
