@@ -533,7 +533,7 @@ TTMI_API int ttmi_dequant_bias(const int32_t* acc, const float* act_scale_dev, c
  *              neither may share memory with input, input32, mask or the other
  *   exchange   as many bytes as ttmi_encoder_chain_workspace says, 16-byte aligned, prepared once by ttmi_chain_prepare and used by one call
  *              after the other on one stream
- *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed
+ *   turn       0, 1, 0, 1, ... from call to call; 2: a call that may be recorded and replayed (in any order and number, between the others too)
  *   workgroups, patience: 0, or (tests) how many workgroups are launched and how often one asks for rows that are not there yet
  *              before it computes them itself; neither changes a bit of the result
  * ttmi_encoder_chain_workspace says 0 for what is not built: other types, more than 24 layers, more than 16 rows (batch * seq), head

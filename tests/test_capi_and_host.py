@@ -558,6 +558,33 @@ def walk(tmp_path_factory):
     return run
 
 
+def test_workgroups_of_a_launch_add_up_to_one_unit(tmp_path):
+    """Whoever has not added its share yet, of any number of workgroups, finds as many whole units as at the launch's start; at its end there is
+    one more, also where 32 bits overflow."""
+    (tmp_path / "share.cpp").write_text(r"""
+#include <initializer_list>
+#include "chain_walk.h"
+int main() {
+  using namespace ttmi;
+  for (uint32_t g = 1; g <= (uint32_t)kChainMostWorkgroups; g = g < 600 ? g + 1 : g * 2 - g / 3)
+    for (uint32_t start : {0u, 5 * kLaunchUnit, 0u - kLaunchUnit}) {
+      uint32_t count = start;
+      for (uint32_t r = 0; r < g; ++r) {
+        if (count / kLaunchUnit != start / kLaunchUnit || launch_share(r, g) == 0) return 1;
+        count += launch_share(r, g);
+      }
+      if (count != start + kLaunchUnit) return 2;
+    }
+  uint32_t sum = 0;
+  for (int r = 0; r < kChainMostWorkgroups; ++r) sum += launch_share(r, kChainMostWorkgroups);
+  return sum == kLaunchUnit ? 0 : 3;
+}
+""")
+    device = os.path.join(os.path.dirname(capi.HEADER), "..", "turbotransformers_amd", "csrc", "device")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", device, str(tmp_path / "share.cpp"), "-o", str(tmp_path / "share")], check=True)
+    assert subprocess.run([str(tmp_path / "share")], timeout=60).returncode == 0
+
+
 @pytest.mark.parametrize("workgroups,resident", [(1, 1), (3, 1), (7, 2), (7, 7), (12, 5)])
 @pytest.mark.parametrize("resumes", [0, 1])
 def test_a_chain_of_steps_ends_whoever_is_resident(walk, workgroups, resident, resumes):

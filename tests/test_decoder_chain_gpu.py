@@ -170,3 +170,73 @@ def test_what_is_not_built_has_no_workspace(ttmi):
                  (8, 12, 768, 1536, 40, "f16"), (8, 0, 768, 4160, 0, "f16"), (8, 0, 800, 3072, 0, "f16"), (8, 0, 1088, 3072, 0, "f16"), (8, 0, 768, 3136, 0, "f32")]:
         ok(ttmi.ttmi_decoder_chain_workspace(*args[:5], TTMI_DTYPES[args[5]], ctypes.addressof(size)))
         assert size.value == 0, args
+
+
+def _layer(seed=0, hidden=768, inner=3072):
+    import turbo_transformers as tt
+    from test_model_gpu import _OnmtLikeFfn
+
+    torch.manual_seed(seed)
+    return tt.PositionwiseFeedForward.from_onmt(_OnmtLikeFfn(hidden, inner).cuda().half())
+
+
+def _recorded(side, call):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = call()
+    return graph, out
+
+
+@pytest.mark.parametrize("rows", [1, 8, 16])
+def test_recorded_calls_of_a_layer_are_replayed_in_any_order(rows):
+    """Graphs of one and of two calls of one layer, between its own calls: each launch finds the part of the exchange memory whose turn it is."""
+    layer = _layer()
+    gen = torch.Generator().manual_seed(rows)
+    xs = [torch.randn(rows, 1, 768, generator=gen).half().cuda() for _ in range(3)]
+    want = [layer(x).clone() for x in xs]
+    twice = layer(layer(xs[2])).clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        kept = [layer(xs[0]) for _ in range(8)]  # (results that the recorded calls find room in)
+    side.synchronize()
+    del kept
+    one, out_one = _recorded(side, lambda: layer(xs[0]))
+    other, out_other = _recorded(side, lambda: layer(xs[1]))
+    two, out_two = _recorded(side, lambda: layer(layer(xs[2])))
+    for order in ("1", "22", "121", "2", "3", "1331", "23", "3221", "111"):
+        for o in (out_one, out_other, out_two):
+            o.fill_(7.0)
+        for kind in order:
+            {"1": one, "2": other, "3": two}[kind].replay()
+        torch.cuda.synchronize()
+        for kind, out, exact in (("1", out_one, want[0]), ("2", out_other, want[1]), ("3", out_two, twice)):
+            assert kind not in order or torch.equal(out, exact), order
+        assert torch.equal(layer(xs[1]), want[1])
+
+
+def test_a_call_that_is_recorded_before_any_is_made():
+    """The exchange memory, where another layer's was before, is prepared by the graph itself."""
+    given_back = _layer(1)
+    x = torch.randn(8, 1, 768, generator=torch.Generator().manual_seed(5)).half().cuda()
+    given_back(x)
+    layer = _layer(2)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        layer(torch.randn(20, 1, 768, device="cuda").half())  # two launches: lays the weights out
+        kept = [given_back(x) for _ in range(4)]
+        side.synchronize()
+    del given_back, kept
+    graph, out = _recorded(side, lambda: layer(x))
+    other, out_other = _recorded(side, lambda: layer(x))
+    seen = []
+    for g, o in ((graph, out), (graph, out), (other, out_other), (graph, out), (other, out_other)):
+        o.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        seen.append(o.clone())
+    want = layer(x)
+    assert all(torch.equal(o, want) for o in seen)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(layer(x), want)

@@ -194,3 +194,35 @@ def test_layers_with_inner_rows_narrower_than_the_hidden_ones(dt, inner):
     with torch.no_grad():
         want = model.float().cpu().double().encoder(x.double().cpu(), attention_mask=None)[0]
     assert (got.double().cpu() - want).abs().max().item() <= 2 * 4 * 8 * EPS[dt]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+def test_recorded_stacks_are_replayed_in_any_order(dt):
+    """One call of three layers and three of one layer each, recorded, between calls of their owner."""
+    import turbo_transformers as tt
+    from test_model_gpu import _hf_bert
+
+    model, cfg = _hf_bert(3, seed=12)
+    encoder = tt.BertEncoder.from_torch(model.to(TORCH_DTYPES[dt]).encoder)
+    gen = torch.Generator().manual_seed(6)
+    x, y = [torch.randn(1, 10, cfg.hidden_size, generator=gen).to(TORCH_DTYPES[dt]).cuda() for _ in range(2)]
+    want = [encoder(x)[0].clone(), encoder(y)[0].clone()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        kept = [(encoder(x), encoder(x, output_hidden_states=True)) for _ in range(4)]  # (results that the recorded calls find room in)
+    side.synchronize()
+    del kept
+    graphs = []
+    for call in (lambda: encoder(x)[0], lambda: encoder(y, output_hidden_states=True)[0]):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = call()
+        graphs.append((graph, out))
+    for order in ((0, ), (1, ), (0, 1, 1), (1, 0), (0, 0, 0), (1, 1)):
+        for k in order:
+            graphs[k][1].fill_(7.0)
+            graphs[k][0].replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(graphs[k][1], want[k]) for k in order), order
+        assert torch.equal(encoder(y)[0], want[1]) and torch.equal(encoder(x, output_hidden_states=True)[0], want[0])

@@ -2,8 +2,11 @@
 //
 // What one step leaves for the next goes through memory, past the L2s.  The exchange memory is filled with a word that no result has
 // (kUnwritten: a NaN that every store here replaces by another one), and a reader asks again until it has words of another value.
-// The exchange memory is kept by the caller in two parts that take turns: a launch fills the part that the one before it has used.  Where launches are
-// recorded and replayed, in an order that nobody knows, they use a third part, which is filled in front of each.
+// The exchange memory is kept by the caller in parts that take turns: a launch fills the part that the one before it has used.  Where launches are
+// recorded and replayed, in an order that nobody knows, the host cannot tell whose turn it is: they have two parts of their own and count themselves behind
+// those (count_launch).  us per recorded step of six decoder layers of base, three launches a layer each filling its part by a launch in front / so, and the 48
+// launches that they replace: fp16 1 x 6 keys 183 / 168, 220; 8 x 41 214 / 198, 231; 16 x 41 248 / 232, 236; 16 x 201 273 / 255, 262; fp32 8 x 41 306 / 286, 308;
+// 16 x 41 345 / 319, 331; an encoder layer of base by itself, 10 rows, 27.5 / 23.7, 27.
 // An exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same reads and writes 2.9, a
 // barrier over the grid with counters 4 to 5.
 #pragma once
@@ -109,14 +112,20 @@ __device__ __forceinline__ floatx2 sum_parts(const float* part, int row, int col
   return v;
 }
 
-static __global__ void unwritten_kernel(u32x4* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten};
+constexpr int kCountBytes = 256;  // behind the parts: the recorded launches so far, and nothing else in its line
+inline int64_t exchange_bytes(int64_t part) { return 4 * part + kCountBytes; }
+inline int64_t part_of_exchange(int64_t bytes) { return (bytes - kCountBytes) / 4; }
+
+static __global__ void prepare_exchange_kernel(u32x4* p, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const uint32_t word = i < n - kCountBytes / 16 ? kUnwritten : 0u;
+    p[i] = u32x4{word, word, word, word};
+  }
 }
-inline int launch_unwritten(void* p, int64_t bytes, hipStream_t s) {
-  hipLaunchKernelGGL(unwritten_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * compute_units())), dim3(256), 0, s, static_cast<u32x4*>(p),
-                     bytes / 16);
-  return launch_status("unwritten_kernel");
+inline int launch_prepare_exchange(void* p, int64_t bytes, hipStream_t s) {
+  hipLaunchKernelGGL(prepare_exchange_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(bytes / 16, 256), 2 * compute_units())), dim3(256), 0, s,
+                     static_cast<u32x4*>(p), bytes / 16);
+  return launch_status("prepare_exchange_kernel");
 }
 // A result of a chain, or what it reads while results are written.
 struct Extent {
@@ -137,12 +146,26 @@ inline bool results_apart(std::initializer_list<Extent> results, std::initialize
   }
   return true;
 }
-// The part of a launch, and the one that it fills for the next.
-inline int take_part(void* exchange, int64_t bytes, int turn, char** mine, char** other, hipStream_t s) {
+// The part of a launch, the one that it fills for the next (null: it works out both by itself), and where recorded launches are counted.
+struct Turn {
+  char *mine, *other;
+  uint32_t* count;
+};
+inline int take_turn(void* exchange, int64_t part, int turn, Turn* to) {
   TTMI_REQUIRE(turn >= 0 && turn <= 2, "turn is 0, 1 or 2");
-  *mine = static_cast<char*>(exchange) + turn * bytes;
-  *other = turn == 2 ? nullptr : static_cast<char*>(exchange) + (1 - turn) * bytes;
-  return turn == 2 ? launch_unwritten(*mine, bytes, s) : 0;
+  char* const at = static_cast<char*>(exchange);
+  *to = turn == 2 ? Turn{at + 2 * part, nullptr, reinterpret_cast<uint32_t*>(at + 4 * part)} : Turn{at + turn * part, at + (1 - turn) * part, nullptr};
+  return 0;
+}
+
+// Recorded launches are counted (chain_walk.h).  Of the count the whole units are the same for all workgroups of a launch: every other launch has the second
+// part.  One thread of a workgroup asks, in a first step behind the weights: all wavefronts at one address are a queue (a recorded step of hidden 1024, inner 3072,
+// 16 sequences of 200 keys: one thread 264 us, each wavefront once 269, for each of its items 367).
+__device__ __forceinline__ uint32_t launches_so_far(const uint32_t* count) { return __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ uint32_t part_offset(uint32_t launches, uint32_t part) { return (0u - (launches / kLaunchUnit & 1u)) & part; }
+// At a workgroup's end; a thread of it that has asked has its answer by then.
+__device__ __forceinline__ void count_launch(uint32_t* count, int rank, int workgroups) {
+  if (threadIdx.x == 0) (void)__hip_atomic_fetch_add(count, launch_share((uint32_t)rank, (uint32_t)workgroups), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Workgroup `rank` of `count` fills its share.
 __device__ __forceinline__ void fill_unwritten(char* p, uint32_t bytes, int rank, int count) {

@@ -8,6 +8,8 @@
 // rounds for each of its items.
 #pragma once
 
+#include <cstdint>
+
 #if defined(__HIP__)
 #define TTMI_WALK __host__ __device__ __forceinline__
 #else
@@ -17,6 +19,12 @@
 namespace ttmi {
 
 constexpr int kChainMostTries = 4096;
+
+// Launches whose order the host does not know are counted in memory, in units that the workgroups of each add up between them, one share when each ends.
+// While one has not ended a unit is not full, so that whoever reads the count, however late it started, finds the same number of whole units.
+constexpr uint32_t kLaunchUnit = 1u << 16;
+constexpr int kChainMostWorkgroups = 1 << 15;  // (a share of at least one, in 32 bits)
+TTMI_WALK uint32_t launch_share(uint32_t rank, uint32_t workgroups) { return (rank + 1) * kLaunchUnit / workgroups - rank * kLaunchUnit / workgroups; }
 
 struct ChainWalk {
   int step = 0, item = 0;                // the item at hand

@@ -50,7 +50,8 @@ struct DecoderArgs {
   void *k_out, *v_out;                                         // [rows, heads, keys, 64], or null
   const float* mask;                                           // [rows, keys], or null
   void *probs, *out;                                           // [rows, heads, keys]; [rows, H]
-  char *exchange, *other;                                      // the part of this launch, the part to fill, or null
+  char *exchange, *other;                                      // the part of this launch, the part to fill (recorded: the first of the two)
+  uint32_t* count;                                             // of recorded launches
   uint32_t bytes;                                              // of a part
   int rows, heads, hidden, width, inner;                       // width: of step 0's product; inner: of the last one's rows
   int past, keys, waves, patience;                             // waves: of a head
@@ -93,8 +94,9 @@ __device__ __forceinline__ float over_keys(float v, Op op) {
   return op(halves.a, halves.b);
 }
 
-// LOADS: keys of a lane of the attention; pieces of a wavefront of the feed-forward block's last product
-template <typename T, Block BLOCK, int LOADS>
+// LOADS: keys of a lane of the attention; pieces of a wavefront of the feed-forward block's last product.  RECORDED: the launch finds its part of the
+// exchange memory by itself.
+template <typename T, Block BLOCK, int LOADS, bool RECORDED>
 __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderArgs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int STEPS = BLOCK == kFeedForward ? 2 : 3;
@@ -135,18 +137,27 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
 #pragma unroll
     for (uint32_t i = 0; i < sizeof(first) / 4; ++i) asm volatile("" : : "s"(first[i]));
   }
+  __shared__ uint32_t launches;  // recorded: so far
+  auto shift = [&]() __attribute__((always_inline)) { return RECORDED ? part_offset(__builtin_amdgcn_readfirstlane(launches), arguments()->bytes) : 0u; };
   // The workgroups that are done first fill the other part of the exchange memory.
   auto leave = [&]() __attribute__((always_inline)) {
     const Arguments& a = *arguments();
     const int fillers = min(G, items(0));
-    if (a.other != nullptr && me < fillers) fill_unwritten(a.other, a.bytes, me, fillers);
+    if (me < fillers) fill_unwritten(RECORDED ? a.exchange + (a.bytes - shift()) : a.other, a.bytes, me, fillers);
+    if constexpr (RECORDED) count_launch(a.count, me, G);
   };
 
   ChainWalk walk;
   walk.item = first_item(0) - G;
   walk.forward(G, STEPS, items, first_item);
-  if (walk.step >= STEPS) return;  // (not of those that fill)
-  if (threadIdx.x == 0) missing = 0;
+  if (walk.step >= STEPS) {
+    leave();
+    return;
+  }
+  if (threadIdx.x == 0) {
+    missing = 0;
+    if (RECORDED && walk.step != 0) launches = launches_so_far(arguments()->count);
+  }
   __syncthreads();
 
   for (;;) {
@@ -157,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 15, lgrp = lane >> 4;
-    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, a.bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, RECORDED ? 2 * a.bytes : a.bytes, 0x00020000);
     auto load4 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(mem, offset, 0, kThroughMemory); };
     auto store1 = [&](uint32_t offset, uint32_t x) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b32(storable(x), mem, offset, 0, kThroughMemory); };
     auto store_pair = [&](uint32_t offset, float v0, float v1) __attribute__((always_inline)) {
@@ -227,6 +238,8 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
             wf[p][c][s] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p < mine ? w_row + (uint32_t)(c * 16 * H * E + p * 128 + s * 16) : kOutside, 0, 0);
       // Requested in this order and here, not where they are used: the weights come from the furthest.
       asm volatile("" ::: "memory");
+      uint32_t so_far = 0;
+      if (RECORDED && tid == 0) so_far = launches_so_far(a.count);
       if (wave < rows) {
         Four<T> raw[kTurns], gm[kTurns], bt[kTurns];
 #pragma unroll
@@ -249,6 +262,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
           if (col < H) *reinterpret_cast<Four<T>*>(smem + wave * pitch + col * E) = to_four<T>(normed[t]);
         }
       }
+      if (RECORDED && tid == 0) launches = so_far;
       __syncthreads();
 #pragma unroll
       for (int p = 0; p < PIECES; ++p)
@@ -263,11 +277,11 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
       const int K = a.inner, share = (K / PIECE + kWaves - 1) / kWaves, first = wave * share, mine = min(K / PIECE - first, share), there = lrow < rows ? mine : 0;
       const __amdgpu_buffer_rsrc_t weights = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(a.w_out), 0, H * K * E, 0x00020000);
       const uint32_t w_row = (uint32_t)((n0 + lrow) * K * E + first * 128 + lgrp * 32);
-      const uint32_t row_at = (BLOCK == kFeedForward ? 0u : context_at(a.width, E)) + fragment_offset<T>(lrow, first * PIECE + lgrp * (PIECE / 4));
       u32x4 wf[2 * OUT_PIECES], af[2 * OUT_PIECES];
       if (BLOCK == kFeedForward || mine > 0) {  // (the same for the wavefront; all of them have a share of the many rows of W2)
 #pragma unroll
         for (int p = 0; p < 2 * OUT_PIECES; ++p) wf[p] = (u32x4)__builtin_amdgcn_raw_buffer_load_b128(weights, p / 2 < mine ? w_row + (p / 2) * 128 + (p & 1) * 16 : kOutside, 0, 0);
+        const uint32_t row_at = shift() + (BLOCK == kFeedForward ? 0u : context_at(a.width, E)) + fragment_offset<T>(lrow, first * PIECE + lgrp * (PIECE / 4));
         await([&]() __attribute__((always_inline)) {
 #pragma unroll
           for (int p = 0; p < 2 * OUT_PIECES; ++p) af[p] = load4(p / 2 < there ? row_at + p * (kRows * 64) : kOutside);
@@ -301,7 +315,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
         mk[i] = a.mask != nullptr ? a.mask[b * keys + min(key, keys - 1)] : 0.f;
       }
       Eight<T> qf, kn, vn;
-      const uint32_t at = (uint32_t)((b * a.width + head * kD + piece * 8) * E), row_bytes = (uint32_t)(H * E);
+      const uint32_t at = shift() + (uint32_t)((b * a.width + head * kD + piece * 8) * E), row_bytes = (uint32_t)(H * E);
       await([&]() __attribute__((always_inline)) {
         uint32_t m = 0;
 #pragma unroll
@@ -406,9 +420,9 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
         r.v[1] = from_float<T>(v1 + second_of(residual));
         store_vec<T, 2>(static_cast<T*>(a.out) + row * H + column, r);
       } else if constexpr (BLOCK == kFeedForward) {
-        store_pair(fragment_offset<T>(row, column), fmaxf(v0, 0.f), fmaxf(v1, 0.f));
+        store_pair(shift() + fragment_offset<T>(row, column), fmaxf(v0, 0.f), fmaxf(v1, 0.f));
       } else {
-        store_pair((uint32_t)((row * a.width + column) * E), v0, v1);
+        store_pair(shift() + (uint32_t)((row * a.width + column) * E), v0, v1);
       }
     } else if (!product) {
       // the context of the workgroup's heads, two columns a thread
@@ -422,7 +436,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
           v1 += p[1];
         }
         const int b = pair / heads;
-        store_pair(context_at(a.width, E) + fragment_offset<T>(b, (pair - b * heads) * kD + col), v0, v1);
+        store_pair(shift() + context_at(a.width, E) + fragment_offset<T>(b, (pair - b * heads) * kD + col), v0, v1);
       }
     }
     walk.executed(G, STEPS, items, first_item);
@@ -437,7 +451,7 @@ __global__ __launch_bounds__(kThreads) void decoder_chain_kernel(const DecoderAr
 
 int64_t part_bytes(Block block, int64_t hidden, int64_t width, int64_t element) { return kRows * element * (width + (block == kFeedForward ? 0 : hidden)); }
 
-template <typename T, Block BLOCK, int LOADS>
+template <typename T, Block BLOCK, int LOADS, bool RECORDED>
 int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
   a.waves = 1;
   while (BLOCK != kFeedForward && a.waves * 8 * LOADS < a.keys) a.waves *= 2;
@@ -445,7 +459,7 @@ int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
   const int64_t all = a.width / (16 * kColumns) + middle + a.hidden / 16;
   const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(all, compute_units());
   const int lds = kRows * chain_row_pitch(a.hidden, sizeof(T)) + kWaves * kRows * kPitch * 4;
-  auto kernel = decoder_chain_kernel<T, BLOCK, LOADS>;
+  auto kernel = decoder_chain_kernel<T, BLOCK, LOADS, RECORDED>;
   // more than 64 KB of dynamic LDS: the limit is raised once per kernel and device
   static std::mutex mu;
   static std::set<int> done;
@@ -462,18 +476,27 @@ int launch_sized(DecoderArgs a, int workgroups, hipStream_t s) {
   return launch_status("decoder_chain_kernel");
 }
 
-template <typename T, Block BLOCK>
-int launch(const DecoderArgs& a, int workgroups, hipStream_t s) {
+template <typename T, Block BLOCK, bool RECORDED>
+int launch_for(const DecoderArgs& a, int workgroups, hipStream_t s) {
   // Few keys a wavefront: the sixteen of a workgroup share four SIMDs, and what the attention of 64 keys takes there is more than an exchange.
   if constexpr (BLOCK != kFeedForward)
-    if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, sizeof(T) == 4 ? 4 : 8>(a, workgroups, s);  // (fp32: 64 keys do not fit the registers)
+    if (a.keys > 16 * kWaves) return launch_sized<T, BLOCK, sizeof(T) == 4 ? 4 : 8, RECORDED>(a, workgroups, s);  // (fp32: 64 keys do not fit the registers)
   if constexpr (BLOCK == kFeedForward) {
     constexpr int kPieces = 3072 * (int)sizeof(T) / 128 / kWaves;
-    if (a.inner > 3072) return launch_sized<T, BLOCK, sizeof(T) == 4 ? kPieces : 4>(a, workgroups, s);  // (fp32: refused)
-    return launch_sized<T, BLOCK, kPieces>(a, workgroups, s);
+    if (a.inner > 3072) return launch_sized<T, BLOCK, sizeof(T) == 4 ? kPieces : 4, RECORDED>(a, workgroups, s);  // (fp32: refused)
+    return launch_sized<T, BLOCK, kPieces, RECORDED>(a, workgroups, s);
   } else {
-    return launch_sized<T, BLOCK, 2>(a, workgroups, s);
+    return launch_sized<T, BLOCK, 2, RECORDED>(a, workgroups, s);
   }
+}
+
+template <typename T, Block BLOCK>
+int launch(DecoderArgs a, void* exchange, int turn, int workgroups, hipStream_t s) {
+  Turn t;
+  const int rc = take_turn(exchange, a.bytes, turn, &t);
+  if (rc != 0) return rc;
+  a.exchange = t.mine, a.other = t.other, a.count = t.count;
+  return t.count != nullptr ? launch_for<T, BLOCK, true>(a, workgroups, s) : launch_for<T, BLOCK, false>(a, workgroups, s);
 }
 
 bool takes(int64_t rows, int64_t hidden, int dtype) {
@@ -492,16 +515,17 @@ int ttmi_decoder_chain_workspace(int64_t rows, int64_t heads, int64_t hidden, in
   *bytes = 0;
   if (!takes(rows, hidden, dtype)) return 0;
   if (heads > 0) {
-    if (hidden == heads * kD && keys >= 1 && keys <= kMostKeys && (inner == hidden || inner == 3 * hidden)) *bytes = 3 * part_bytes(kSelfAttention, hidden, inner, (int64_t)dtype_size(dtype));
+    if (hidden == heads * kD && keys >= 1 && keys <= kMostKeys && (inner == hidden || inner == 3 * hidden)) *bytes = exchange_bytes(part_bytes(kSelfAttention, hidden, inner, (int64_t)dtype_size(dtype)));
   } else if (inner >= 64 && inner % 64 == 0 && inner <= (dtype == TTMI_F32 ? kMostInner32 : kMostInner)) {
-    *bytes = 3 * part_bytes(kFeedForward, hidden, inner, (int64_t)dtype_size(dtype));
+    *bytes = exchange_bytes(part_bytes(kFeedForward, hidden, inner, (int64_t)dtype_size(dtype)));
   }
   return 0;
 }
 
 int ttmi_chain_prepare(void* exchange, int64_t bytes, void* stream) {
-  TTMI_REQUIRE(exchange && bytes > 0 && bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(exchange) & 15) == 0, "exchange memory comes in whole, aligned 16 bytes");
-  return launch_unwritten(exchange, bytes, (hipStream_t)stream);
+  TTMI_REQUIRE(exchange && bytes > kCountBytes && bytes % 16 == 0 && (reinterpret_cast<uintptr_t>(exchange) & 15) == 0,
+               "exchange memory comes in whole, aligned 16 bytes");
+  return launch_prepare_exchange(exchange, bytes, (hipStream_t)stream);
 }
 
 int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta, float eps, const void* w1, const void* b1, const void* w2, const void* b2,
@@ -511,7 +535,7 @@ int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta
   int64_t bytes = 0;
   const int rc = ttmi_decoder_chain_workspace(rows, 0, hidden, inner, 0, dtype, &bytes);
   if (rc != 0) return rc;
-  TTMI_REQUIRE(bytes > 0 && workgroups >= 0 && patience >= 0, "this block is not run as one launch");
+  TTMI_REQUIRE(bytes > 0 && workgroups >= 0 && workgroups <= kChainMostWorkgroups && patience >= 0, "this block is not run as one launch");
   uintptr_t bits = 0;
   for (const void* p : {x, gamma, beta, w1, b1, w2, b2, (const void*)out, (const void*)exchange}) bits |= reinterpret_cast<uintptr_t>(p);
   TTMI_REQUIRE((bits & 15) == 0, "tensors must be 16-byte aligned");
@@ -521,10 +545,8 @@ int ttmi_decoder_feed_forward(const void* x, const void* gamma, const void* beta
   a.x = x, a.gamma = gamma, a.beta = beta, a.w_in = w1, a.b_in = b1, a.w_out = w2, a.b_out = b2, a.out = out;
   a.rows = (int)rows, a.hidden = (int)hidden, a.width = (int)inner, a.inner = (int)inner, a.eps = eps, a.heads = 1;
   a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
-  a.bytes = (uint32_t)(bytes / 3);
-  const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
-  if (part != 0) return part;
-  TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kFeedForward>(a, workgroups, (hipStream_t)stream)));
+  a.bytes = (uint32_t)part_of_exchange(bytes);
+  TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kFeedForward>(a, exchange, turn, workgroups, (hipStream_t)stream)));
   return 0;
 }
 
@@ -539,7 +561,7 @@ int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, f
   int64_t bytes = 0;
   const int rc = ttmi_decoder_chain_workspace(rows, heads, hidden, width, keys, dtype, &bytes);
   if (rc != 0) return rc;
-  TTMI_REQUIRE(heads > 0 && bytes > 0 && past > 0 && workgroups >= 0 && patience >= 0, "this attention is not run as one launch");
+  TTMI_REQUIRE(heads > 0 && bytes > 0 && past > 0 && workgroups >= 0 && workgroups <= kChainMostWorkgroups && patience >= 0, "this attention is not run as one launch");
   uintptr_t bits = 0;
   for (const void* p : {x, gamma, beta, w_in, b_in, w_out, b_out, k_past, v_past, (const void*)k_out, (const void*)v_out, (const void*)out, (const void*)exchange})
     bits |= reinterpret_cast<uintptr_t>(p);
@@ -554,13 +576,11 @@ int ttmi_decoder_attention(const void* x, const void* gamma, const void* beta, f
   a.rows = (int)rows, a.heads = (int)heads, a.hidden = (int)hidden, a.width = (int)width, a.inner = (int)hidden, a.eps = eps, a.scale = scale;
   a.past = (int)past, a.keys = (int)keys;
   a.patience = patience > 0 ? patience : kChainPatience, a.error = async_error_flag();
-  a.bytes = (uint32_t)(bytes / 3);
-  const int part = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, (hipStream_t)stream);
-  if (part != 0) return part;
+  a.bytes = (uint32_t)part_of_exchange(bytes);
   if (grows) {
-    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kSelfAttention>(a, workgroups, (hipStream_t)stream)));
+    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kSelfAttention>(a, exchange, turn, workgroups, (hipStream_t)stream)));
   } else {
-    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kMemoryAttention>(a, workgroups, (hipStream_t)stream)));
+    TTMI_DISPATCH_FLOAT(dtype, T, return (launch<T, kMemoryAttention>(a, exchange, turn, workgroups, (hipStream_t)stream)));
   }
   return 0;
 }

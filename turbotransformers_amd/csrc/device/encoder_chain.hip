@@ -50,7 +50,8 @@ struct ChainArgs {
   const float* mask;     // [rows], additive, or null
   void* out;
   float* out32;
-  char *exchange, *other;  // the part of this launch, the part to fill, or null
+  char *exchange, *other;  // the part of this launch, the part to fill (recorded: the first of the two)
+  uint32_t* count;         // of recorded launches
   uint32_t layer_bytes;  // of the exchange memory
   Places at;
   int layers, rows, seq, heads, hidden, ffn, patience;
@@ -100,8 +101,8 @@ __host__ __device__ inline int rows_bytes(int hidden) {
 __host__ __device__ inline int lds_bytes(int hidden) { return rows_bytes(hidden) + kWaves * kRows * kPitch * 4; }
 
 // TURNS: turns of 256 columns that a row of the hidden state takes at most; PIECES: 128-byte pieces of a row of FFN2's weight
-// that a wavefront takes at most (of the other weights it is one).
-template <typename T, int TURNS, int PIECES>
+// that a wavefront takes at most (of the other weights it is one).  RECORDED: the launch finds its part of the exchange memory by itself.
+template <typename T, int TURNS, int PIECES, bool RECORDED>
 __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr bool WIDE = std::is_same<T, bf16>::value;  // the residual stays in fp32
@@ -129,20 +130,35 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
   };
   const int last_step = 4 * arguments()->layers;
 
-  {
-    const Arguments& a = *arguments();
-    if (a.other != nullptr) fill_unwritten(a.other, (uint32_t)a.layers * a.layer_bytes, me, G);
-  }
+  __shared__ uint32_t launches;  // recorded: so far
+  uint32_t shift = 0;
+  if constexpr (!RECORDED) fill_unwritten(arguments()->other, (uint32_t)arguments()->layers * arguments()->layer_bytes, me, G);
+  auto leave = [&]() __attribute__((always_inline)) {
+    if constexpr (RECORDED) {
+      const Arguments& a = *arguments();
+      const uint32_t part = (uint32_t)a.layers * a.layer_bytes;
+      const int fillers = min(G, items(0));  // (they know the part)
+      if (me < fillers) fill_unwritten(a.exchange + (part - shift), part, me, fillers);
+      count_launch(a.count, me, G);
+    }
+  };
   ChainWalk walk;
   walk.item = first_item(0) - G;
   walk.forward(G, last_step + 1, items, first_item);
-  if (walk.step > last_step) return;
+  if (walk.step > last_step) {
+    leave();
+    return;
+  }
   int seen = 0;  // the last step whose inputs the workgroup has seen
-  if (threadIdx.x == 0) missing = 0;
+  if (threadIdx.x == 0) {
+    missing = 0;
+    if (RECORDED) launches = launches_so_far(arguments()->count);
+  }
   constexpr int WORDS = sizeof(ChainLayer) / 8;
   if ((int)threadIdx.x < arguments()->layers * WORDS)
     reinterpret_cast<uint64_t*>(layers)[threadIdx.x] = reinterpret_cast<const __attribute__((address_space(4))) uint64_t*>(&arguments()->layer)[threadIdx.x];
   __syncthreads();
+  if constexpr (RECORDED) shift = part_offset(__builtin_amdgcn_readfirstlane(launches), (uint32_t)arguments()->layers * arguments()->layer_bytes);
   auto uniform = [](const void* const& p) __attribute__((always_inline)) -> const void* {
     const uint64_t x = reinterpret_cast<const uint64_t&>(p);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x), hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));  // (they return int)
@@ -160,8 +176,8 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     asm volatile("" : "+v"(tid));
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lrow = lane & 15, lgrp = lane >> 4;
     const int l = step >> 2, ph = step & 3;
-    const uint32_t base = (uint32_t)l * a.layer_bytes;
-    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, a.layers * a.layer_bytes, 0x00020000);
+    const uint32_t base = (uint32_t)l * a.layer_bytes + shift;
+    const __amdgpu_buffer_rsrc_t mem = __builtin_amdgcn_make_buffer_rsrc(a.exchange, 0, (RECORDED ? 2 : 1) * a.layers * a.layer_bytes, 0x00020000);
     auto load4 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x4)__builtin_amdgcn_raw_buffer_load_b128(mem, offset, 0, kThroughMemory); };
     auto load2 = [&](uint32_t offset) __attribute__((always_inline)) { return (u32x2)__builtin_amdgcn_raw_buffer_load_b64(mem, offset, 0, kThroughMemory); };
     auto load1 = [&](uint32_t offset) __attribute__((always_inline)) { return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(mem, offset, 0, kThroughMemory); };
@@ -426,6 +442,7 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
       if (tid == 0) missing = 0;
       if (!walk.late(seen)) {  // (not reached while every item's inputs are some item's outputs)
         if (tid == 0 && a.error != nullptr) *a.error = kRowsNeverCame;
+        leave();
         return;
       }
       __syncthreads();
@@ -456,7 +473,10 @@ __global__ __launch_bounds__(kThreads) void encoder_chain_kernel(const ChainArgs
     }
     if (!walk.solo()) seen = step;
     walk.executed(G, last_step + 1, items, first_item);
-    if (walk.step > last_step) return;
+    if (walk.step > last_step) {
+      leave();
+      return;
+    }
     __syncthreads();  // the rows and partial tiles have been read
   }
 #endif
@@ -467,7 +487,7 @@ int64_t workspace_bytes(int64_t layers, int64_t rows, int64_t heads, int64_t hid
   const bool takes = (dtype == TTMI_F16 || dtype == TTMI_BF16) && layers >= 1 && layers <= kMostLayers && rows >= 1 && rows <= kRows && heads >= 4 &&
                      heads <= kWaves && hidden == heads * kD && ffn >= hidden && ffn % 64 == 0 && ffn <= kWaves * 4 * 64;
   if (!takes) return 0;
-  return 3 * layers * (int64_t)places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end;  // (of all rows: calls of any number of them take turns)
+  return exchange_bytes(layers * (int64_t)places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2).end);  // (of all rows: calls of any number of them take turns)
 }
 
 }  // namespace
@@ -487,7 +507,7 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
                        void* exchange, int turn, int64_t layers, int64_t batch, int64_t seq, int64_t heads, int64_t hidden, int64_t ffn, float eps, int dtype,
                        int workgroups, int patience, void* stream) {
   TTMI_REQUIRE(weights && input && out && exchange, "null tensor");
-  TTMI_REQUIRE(batch > 0 && seq > 0 && batch <= kRows && seq <= kRows && workgroups >= 0 && patience >= 0, "bad shape");
+  TTMI_REQUIRE(batch > 0 && seq > 0 && batch <= kRows && seq <= kRows && workgroups >= 0 && workgroups <= kChainMostWorkgroups && patience >= 0, "bad shape");
   const int64_t rows = batch * seq, bytes = workspace_bytes(layers, rows, heads, hidden, ffn, dtype);
   TTMI_REQUIRE(bytes > 0, "this stack of layers is not run as one launch");
   ChainArgs a{};
@@ -507,14 +527,16 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
                "out and out32 must share no memory with input, input32, mask or each other");
   const int cus = compute_units();
   a.input = input, a.input32 = input32, a.mask = mask, a.out = out, a.out32 = out32;
-  a.layer_bytes = (uint32_t)(bytes / 3 / layers);
+  a.layer_bytes = (uint32_t)(part_of_exchange(bytes) / layers);
   a.at = places(kRows, (int)hidden, (int)ffn, dtype == TTMI_BF16 ? 4 : 2);
   a.layers = (int)layers, a.rows = (int)rows, a.seq = (int)seq, a.heads = (int)heads, a.hidden = (int)hidden, a.ffn = (int)ffn;
   a.patience = patience > 0 ? patience : kChainPatience;
   a.eps = eps, a.scale_log2e = 0.125f * 1.4426950408889634f, a.inv_scale = 8.0f, a.error = async_error_flag();
   hipStream_t s = (hipStream_t)stream;
-  const int rc = take_part(exchange, bytes / 3, turn, &a.exchange, &a.other, s);
+  Turn t;
+  const int rc = take_turn(exchange, part_of_exchange(bytes), turn, &t);
   if (rc != 0) return rc;
+  a.exchange = t.mine, a.other = t.other, a.count = t.count;
   const int64_t widest = std::max(3 * hidden, ffn) / (16 * kColumns) + hidden / 16;
   const unsigned grid = workgroups > 0 ? (unsigned)workgroups : (unsigned)std::min<int64_t>(widest, cus);
   const int lds = lds_bytes((int)hidden);
@@ -536,7 +558,8 @@ int ttmi_encoder_chain(const void* const* weights, const void* input, const floa
   };
   auto sized = [&](auto turns, auto pieces) -> int {
     constexpr int TURNS = decltype(turns)::value, PIECES = decltype(pieces)::value;
-    return dtype == TTMI_F16 ? launch(encoder_chain_kernel<f16, TURNS, PIECES>) : launch(encoder_chain_kernel<bf16, TURNS, PIECES>);
+    if (t.count != nullptr) return dtype == TTMI_F16 ? launch(encoder_chain_kernel<f16, TURNS, PIECES, true>) : launch(encoder_chain_kernel<bf16, TURNS, PIECES, true>);
+    return dtype == TTMI_F16 ? launch(encoder_chain_kernel<f16, TURNS, PIECES, false>) : launch(encoder_chain_kernel<bf16, TURNS, PIECES, false>);
   };
   if (hidden <= 3 * 256 && ffn <= kWaves * 3 * 64) return sized(std::integral_constant<int, 3>{}, std::integral_constant<int, 3>{});
   return sized(std::integral_constant<int, 4>{}, std::integral_constant<int, 4>{});

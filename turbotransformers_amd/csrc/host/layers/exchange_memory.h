@@ -1,7 +1,7 @@
 // The memory through which the steps of a call that runs as one launch pass their rows (ttmi_encoder_chain, ttmi_decoder_attention,
-// ttmi_decoder_feed_forward): its parts take turns from call to call of the layer that holds it, and go with it.  Calls of another size have
-// memory of their own, so that a recorded call, replayed between them, writes nothing that they count on, and its memory stays where it is.  (The sizes
-// do not depend on the rows: there is one, but for encoders of another number of layers.)
+// ttmi_decoder_feed_forward): two of its parts take turns from call to call of the layer that holds it, two from one recorded call to the next, and all of it goes
+// with the layer.  Calls of another size have memory of their own, so that a recorded call, replayed between them, writes nothing that they count on, and its
+// memory stays where it is.  (The sizes do not depend on the rows: there is one, but for encoders, which may be run by the stack and by the layer.)
 #pragma once
 
 #include <list>
@@ -32,7 +32,8 @@ class ExchangeMemory {
     float* const memory = m->words.Reshape<float>({bytes / 4}, device, device_id, "chain/exchange");
     int capturing = 0;
     TT_DEVICE_CALL(ttmi_stream_capturing(stream, &capturing));
-    if (capturing) {  // replayed in an order that is not known here
+    if (capturing) {  // replayed in an order that is not known here: such launches count themselves
+      if (!m->prepared) TT_DEVICE_CALL(ttmi_chain_prepare(memory, bytes, stream));  // (recorded too: each replay finds all parts as they should be)
       launch(memory, 2);
       return;
     }
