@@ -41,20 +41,22 @@ class Stack:
         self.turn = 1 - self.turn
         return self.space
 
-    def run(self, ttmi, x, mask=None, workgroups=0, patience=0):
+    def run(self, ttmi, x, mask=None, workgroups=0, patience=0, x32=None):
         batch, seq, h = x.shape
         space, out = self.exchange(ttmi), torch.empty_like(x)
-        out32 = torch.empty(x.shape, device="cuda") if self.dt == "bf16" else None
+        self.out32 = out32 = torch.empty(x.shape, device="cuda") if self.dt == "bf16" else None
         pointers = (ctypes.c_void_p * (12 * self.layers))(*[w.data_ptr() for l in self.weights for w in l])
-        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(x), None, ptr(mask), ptr(out), ptr(out32), ptr(space), self.turn, self.layers, batch, seq,
+        ok(ttmi.ttmi_encoder_chain(ctypes.addressof(pointers), ptr(x), ptr(x32), ptr(mask), ptr(out), ptr(out32), ptr(space), self.turn, self.layers, batch, seq,
                                    self.heads, h, self.ffn, 1e-12, TTMI_DTYPES[self.dt], workgroups, patience, stream()))
         torch.cuda.synchronize()
         if out32 is not None:
             assert torch.equal(out, out32.to(out.dtype)) or not torch.isfinite(out).all()
         return out
 
-    def exact(self, x, mask=None):
+    def exact(self, x, mask=None, residual=None, stored=lambda r: r):
+        """residual: what the first one is taken from; stored: what becomes of each of them before it is added."""
         x = x.double().cpu()
+        residual = x if residual is None else residual.double().cpu()
         batch, seq, h = x.shape
         norm = lambda y, g, b: torch.nn.functional.layer_norm(y, (h,), g, b, 1e-12)
         for layer in self.weights:
@@ -64,9 +66,9 @@ class Stack:
             if mask is not None:
                 scores = scores + mask.double().cpu()[:, None, None, :]
             ctx = (scores.softmax(-1) @ v).permute(0, 2, 1, 3).reshape(batch, seq, h)
-            x = norm(x + ctx @ o_w.T + o_b, g1, b1)
+            x = norm(stored(residual) + ctx @ o_w.T + o_b, g1, b1)
             y = torch.nn.functional.gelu(x @ w1.T + c1, approximate="tanh")
-            x = norm(x + y @ w2.T + c2, g2, b2)
+            residual = x = norm(stored(x) + y @ w2.T + c2, g2, b2)
         return x
 
 
@@ -88,6 +90,29 @@ def test_a_stack_as_one_launch(ttmi, dt, layers, heads, ffn):
             mask = mask.cuda()
         error = (stack.run(ttmi, x, mask).double().cpu() - stack.exact(x, mask)).abs().max().item()
         assert error <= 4 * 8 * EPS[dt] * layers, (batch, seq, error)
+
+
+@pytest.mark.parametrize("layers,heads,ffn", [(1, 12, 3072), (3, 12, 3072), (2, 16, 4096), (2, 5, 1088)])
+@pytest.mark.parametrize("batch,seq", [(1, 1), (3, 5), (1, 16)])
+@pytest.mark.parametrize("given", [True, False])
+def test_the_residual_of_bf16_stays_in_fp32(ttmi, layers, heads, ffn, batch, seq, given):
+    """From the input before it was rounded (where it is given) to the unrounded result.  What is added to a residual is small here, so that its eight
+    roundings to 16 bits per layer, of at most 2^-8 / 2 of an O(1) value each and a 32nd of that behind the projection, stay below a quarter of one rounding of
+    the residual itself: rms 2^-8 / 2 / sqrt(3) / 32 * sqrt(8) = 1.0e-4 per layer, and twice that is allowed.  The test shows that it would see a rounded one."""
+    stack = Stack("bf16", layers, heads, ffn)
+    for layer in stack.weights:
+        for w in (layer[2], layer[3], layer[8], layer[9]):
+            w.mul_(1.0 / 32)  # (exact)
+    x32 = torch.randn((batch, seq, stack.hidden), generator=torch.Generator().manual_seed(seq)).cuda()
+    x = x32.bfloat16()
+    out = stack.run(ttmi, x, x32=x32 if given else None)
+    want = stack.exact(x, residual=x32 if given else x)
+    rms = lambda t: t.double().cpu().pow(2).mean().sqrt().item()
+    bound = 2 * layers * 2.0 ** -8 / 2 / 3 ** 0.5 / 32 * 8 ** 0.5
+    rounded = stack.exact(x, residual=x32 if given else x, stored=lambda r: r.float().bfloat16().double())
+    assert rms(rounded - want) > 1.5 * bound
+    assert rms(stack.out32.double().cpu() - want) <= bound
+    assert torch.equal(out, stack.out32.bfloat16())
 
 
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
@@ -226,3 +251,26 @@ def test_recorded_stacks_are_replayed_in_any_order(dt):
         torch.cuda.synchronize()
         assert all(torch.equal(graphs[k][1], want[k]) for k in order), order
         assert torch.equal(encoder(y)[0], want[1]) and torch.equal(encoder(x, output_hidden_states=True)[0], want[0])
+
+
+@pytest.mark.parametrize("dt,layers,heads,ffn", [("f16", 12, 12, 3072), ("bf16", 12, 12, 3072), ("bf16", 24, 16, 4096), ("f16", 24, 16, 4096)])
+@pytest.mark.parametrize("batch,seq", [(1, 1), (1, 10), (3, 5), (2, 8)])
+def test_whole_models_of_a_few_rows(dt, layers, heads, ffn, batch, seq):
+    """BertModel with a padding mask, weights as the published models start from (N(0, 0.02)) with every bias and LayerNorm parameter perturbed, against the model in
+    64 bits on what is stored.  Each layer rounds its values at eight places to half of eps at most, of O(1) values, independently, and the LayerNorms pass that on
+    at a gain of about one: sqrt(8 * layers) eps / 2 / sqrt(3) rms."""
+    import turbo_transformers as tt
+    from test_model_gpu import _hf_bert
+
+    model, cfg = _hf_bert(layers, seed=layers, hidden_size=heads * 64, num_attention_heads=heads, intermediate_size=ffn, vocab_size=500)
+    model = model.to(TORCH_DTYPES[dt])
+    ids = torch.randint(0, cfg.vocab_size, (batch, seq), generator=torch.Generator().manual_seed(seq)).cuda()
+    keep = torch.ones(batch, seq, dtype=torch.int64)
+    keep[-1, (seq + 1) // 2:] = 0
+    hidden = tt.BertModel.from_torch(model, torch.device("cuda:0"), "turbo")(ids, attention_masks=keep.cuda())[0]
+    with torch.no_grad():
+        want = model.double()(input_ids=ids, attention_mask=keep.cuda()).last_hidden_state
+    rows = keep.bool().cuda()
+    error = (hidden.double() - want)[rows]
+    assert bool(torch.isfinite(hidden.float()).all())
+    assert error.pow(2).mean().sqrt().item() <= (8 * layers) ** 0.5 * EPS[dt] / 2 / 3 ** 0.5

@@ -2127,3 +2127,87 @@ def test_tiles_between_powers_of_two(ttmi, dt, tile, m, n, k):
     half = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
     assert bool(((c[:m].double() - want).abs() <= half * want.abs() + 2.0 ** -12).all())
     assert bool((c[m] == 7.0).all())
+
+
+def _tile_operands(m, n, k, dt):
+    gen = torch.Generator(device="cuda").manual_seed(m + n)
+    return [torch.randn(shape, generator=gen, device="cuda").mul_(scale).to(TORCH_DTYPES[dt]) for shape, scale in [((m, k), 1.0), ((n, k), k ** -0.5), ((n,), 0.1)]]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("fp32_out", [False, True])
+@pytest.mark.parametrize("tile,m,n,k", [("160x64", 2800, 768, 768), ("160x64", 2797, 776, 768), ("160x64", 2400, 1024, 4096), ("160x128", 6000, 768, 3072),
+                                        ("160x128", 5989, 760, 768), ("256x160", 11500, 768, 768), ("256x160", 11490, 776, 832)])
+def test_tiles_between_powers_of_two_store_products(ttmi, dt, fp32_out, tile, m, n, k):
+    """With a bias alone, in the operands' type and in fp32.  Against 64 bits: k products by sixteen at a time are k / 16 roundings of at most 2^-24 of the
+    sum of their magnitudes; then the result's own rounding, half of its last place."""
+    epilogue = capi.EPI_F32_OUT if fp32_out else capi.EPI_BIAS
+    a, w, b = _tile_operands(m, n, k, dt)
+    args = _epi(bias=b)
+    name = ctypes.create_string_buffer(64)
+    ok(ttmi.ttmi_gemm_describe(m, n, k, epilogue, ctypes.byref(args), TTMI_DTYPES[dt], name, 64))
+    assert tile in name.value.decode(), name.value
+    c = torch.full((m + 1, n), 7.0, device="cuda", dtype=torch.float32 if fp32_out else TORCH_DTYPES[dt])
+    ok(ttmi.ttmi_gemm_fused(ptr(a), ptr(w), ptr(c), m, n, k, k, k, n, epilogue, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+    want = a.double() @ w.double().T + b.double()
+    room = (a.abs().double() @ w.abs().double().T + b.abs().double()) * (k // 16 + 2) * 2.0 ** -24
+    if not fp32_out:
+        room += {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt] * want.abs()
+    assert bool(((c[:m].double() - want).abs() <= room).all())
+    assert bool((c[m] == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("tile,heads,lens", [("160x64", 12, [160] + [90] * 8 + [120]), ("160x64", 16, [200, 3, 97, 150, 50, 111, 89]),
+                                             ("160x128", 12, [200, 1, 7] + [100] * 17 + [95]), ("160x128", 16, [113] * 13 + [31])])
+def test_tiles_between_powers_of_two_split_the_heads_of_a_packed_batch(ttmi, dt, tile, heads, lens):
+    """Rows that end inside a tile, requests that begin and end inside one; what lies past a request's rows stays as it was.  Tolerance as above."""
+    d, B, S, total = 64, len(lens), max(lens), sum(lens)
+    h = heads * d
+    a, w, b = _tile_operands(total, 3 * h, h, dt)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    rows = torch.empty(total, dtype=torch.int32, device="cuda")
+    ok(ttmi.ttmi_build_token_rows(ptr(cu), B, S, total, ptr(rows), stream()))
+    q, k, v = (torch.full((B, heads, S, d), 7.0, dtype=a.dtype, device="cuda") for _ in range(3))
+    args = _epi(bias=b, q=q, k=k, v=v, seq=S, heads=heads, head_dim=d, token_rows=rows, batch=B)
+    name = ctypes.create_string_buffer(64)
+    ok(ttmi.ttmi_gemm_describe(total, 3 * h, h, capi.EPI_QKV_SPLIT_PAD, ctypes.byref(args), TTMI_DTYPES[dt], name, 64))
+    assert tile in name.value.decode(), name.value
+    ok(ttmi.ttmi_gemm_fused(ptr(a), ptr(w), None, total, 3 * h, h, h, h, 3 * h, capi.EPI_QKV_SPLIT_PAD, ctypes.byref(args), TTMI_DTYPES[dt], stream()))
+    want = a.double() @ w.double().T + b.double()
+    room = (a.abs().double() @ w.abs().double().T + b.abs().double()) * (h // 16 + 2) * 2.0 ** -24 + {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt] * want.abs()
+    want, room = (t.view(total, 3, heads, d) for t in (want, room))
+    at = 0
+    for i, n in enumerate(lens):
+        for part, got in enumerate((q, k, v)):
+            assert bool(((got[i, :, :n].double() - want[at:at + n, part].transpose(0, 1)).abs() <= room[at:at + n, part].transpose(0, 1)).all()), (i, part)
+            assert bool((got[i, :, n:] == 7.0).all())
+        at += n
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("fp32_residual", [False, True])
+@pytest.mark.parametrize("m,n,k", [(2400, 1024, 1024), (3000, 768, 3072), (6000, 768, 768), (6275, 768, 3072), (9001, 1024, 1024), (11490, 768, 768)])
+def test_projections_of_the_sizes_between_powers_of_two_with_layer_norm(ttmi, dt, fp32_residual, m, n, k):
+    """Products that a LayerNorm follows, whole and in slices, at the row counts that tiles of 160 rows and columns are for.  Against 64 bits: with the residual in
+    fp32 the sums' roundings alone, k / 16 + 20 of 2^-24 of the sum of magnitudes, through a LayerNorm that divides by no less than one; else the roundings of the
+    product and of the result to the stored type, half of the last place of values up to 6 each."""
+    a, w, b = _tile_operands(m, n, k, dt)
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    res = torch.randn(m, n, generator=gen, device="cuda")
+    gamma, beta = (torch.randn(n, generator=gen, device="cuda").mul_(0.1).add_(x).to(a.dtype) for x in (1.0, 0.0))
+    stored = res if fp32_residual else res.to(a.dtype)
+    out, out32 = torch.full((m + 1, n), 7.0, dtype=a.dtype, device="cuda"), torch.full((m + 1, n), 7.0, device="cuda") if fp32_residual else None
+    ok(ttmi.ttmi_gemm_bias_layer_norm(ptr(a), ptr(w), ptr(out), None if fp32_residual else ptr(stored), ptr(stored) if fp32_residual else None, ptr(b), ptr(gamma),
+                                      ptr(beta), ptr(out32), m, n, k, 1e-12, TTMI_DTYPES[dt], stream()))
+    x = a.double() @ w.double().T + b.double() + stored.double()
+    want = torch.nn.functional.layer_norm(x, (n, ), gamma.double(), beta.double(), 1e-12)
+    sums = float((a.abs().double() @ w.abs().double().T + b.abs().double() + stored.abs().double()).max()) * (k // 16 + 20) * 2.0 ** -24
+    gain = float(gamma.abs().max())
+    half = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}[dt]
+    if fp32_residual:
+        assert float((out32[:m].double() - want).abs().max()) <= 2 * gain * sums
+        assert torch.equal(out[:m], out32[:m].to(a.dtype)) and bool((out32[m] == 7.0).all())
+    else:
+        assert float((out[:m].double() - want).abs().max()) <= 2 * gain * (sums + 6 * half) + 6 * half
+    assert bool((out[m] == 7.0).all())
