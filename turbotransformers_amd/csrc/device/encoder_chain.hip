@@ -24,6 +24,9 @@
 // item a second time writes the same bits.  A workgroup that has waited `patience` polls in vain (others hold the CUs, or the
 // grid is smaller than the items) executes the steps that it misses by itself, from the last one whose inputs it has seen, and
 // goes on; workgroups that start late find everything written.  That ends whatever an item waits for (chain_walk.h): where nobody writes it, in an error.
+// Beside a busy stream that is worth more than it costs: one launch gets its CUs once where 76 get them each time anew.  us per forward of base, 1 x 10
+// tokens, layer by layer / as one launch, median beside torch's fp16 products on another stream of 1024^3: 330 / 220, 2048^3: 477 / 232, 4096^3: 5640 / 234,
+// 8192^3: 10200 / 1405 (one in thirty there takes 16.9 ms: it computes alone); a decoder step of 8 sequences, 40 keys 288 / 212, 390 / 255, 4880 / 1965, 10060 / 9890.
 #include <mutex>
 #include <set>
 
@@ -51,12 +54,12 @@ struct ChainArgs {
   void* out;
   float* out32;
   char *exchange, *other;  // the part of this launch, the part to fill (recorded: the first of the two)
-  uint32_t* count;         // of recorded launches
   uint32_t layer_bytes;  // of the exchange memory
   Places at;
   int layers, rows, seq, heads, hidden, ffn, patience;
   float eps, scale_log2e, inv_scale;
   int* error;
+  uint32_t* count;  // of recorded launches; last, so that eps stays in the line of 64 bytes that every workgroup has read by then (10 rows 188.2 / 190.4 us)
 };
 
 inline uint32_t up256(uint32_t n) { return (n + 255u) & ~255u; }
