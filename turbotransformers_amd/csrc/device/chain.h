@@ -7,7 +7,8 @@
 // those (count_launch).  us per recorded step of six decoder layers of base, three launches a layer each filling its part by a launch in front / so, and the 48
 // launches that they replace: fp16 1 x 6 keys 183 / 168, 220; 8 x 41 214 / 198, 231; 16 x 41 248 / 232, 236; 16 x 201 273 / 255, 262; fp32 8 x 41 306 / 286, 308;
 // 16 x 41 345 / 319, 331; an encoder layer of base by itself, 10 rows, 27.5 / 23.7, 27.
-// An exchange between 256 workgroups takes 1.3 to 1.6 us for 16 to 32 KB; a launch of its own with the same reads and writes 2.9, a
+// An exchange between 256 workgroups that each read all of it takes 1.3 to 1.6 us for 16 to 32 KB, measured by itself (in the chains, where fewer take
+// part or read a share, 0.7 to 1.5); a launch of its own with the same reads and writes 2.9, a
 // barrier over the grid with counters 4 to 5.
 #pragma once
 

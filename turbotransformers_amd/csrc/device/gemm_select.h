@@ -56,7 +56,7 @@ struct RingKernel {
       const int force = kernel_switch(kSwitchLargeTile);
       // More than one workgroup per CU: long enough a launch that the chip runs at its power limit, under which the small
       // tiles' extra LDS and L2 traffic costs clock (16384 x 1024 x 4096: 123 us against 106 although the unthrottled
-      // model has it 20 % ahead).  Less so the largest of them, while there are two rounds: 6275 x 3072 x 768 (GELU) in a forward of 20 packed
+      // model has it 20 % ahead).  Less so the largest of them, 256 x 160 in 16 bits alone, while there are two rounds: 6275 x 3072 x 768 (GELU) in a forward of 20 packed
       // requests 44 us on the large tiles, 37 in 256 x 160.
       const double margin = p.rounds > 1 ? (p.rounds == 2 && p.tile_values >= 256 * 160 ? 1.1 : 1.3) : 1.0;
       if (force != 0 && LargeTileKernel<T, Epi>::eligible(g, epi) && (force == 1 || LargeTileKernel<T, Epi>::us(g, epi) < margin * p.us))
